@@ -1,8 +1,9 @@
-// Paged-attention prefill on MFMA tiles for head sizes the 64/128 kernel does
-// not take: key size D and value size Dv independent, each a multiple of 8
-// and at most 128, bf16, gfx950.
+// Paged-attention prefill on MFMA tiles with the hybrid families' options: key
+// size D and value size Dv independent, each a multiple of 8 and at most 128,
+// bf16, gfx950.  D == Dv of 64 or 128 runs flash_prefill.h's kernel; the one
+// here takes every other pair.
 //
-// Same tiling as the fixed-size flash-prefill kernel: grid = (64-row query
+// Tiling: grid = (64-row query
 // tiles, q heads), 4 waves per workgroup, wave w owns rows [16w, 16w+16) and
 // walks the sequence's pages 32 keys at a time with
 // mfma_f32_16x16x32_bf16: S^T = K Q^T (so a lane ends up holding 8 scores of
@@ -27,6 +28,7 @@
 // entries, so a latent cache can pass its key rows as values.
 
 #include "elem_types.h"
+#include "flash_prefill.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -307,6 +309,54 @@ extern "C" int lig_paged_attention_prefill_tiles(
       !aligned16(v_cache) || num_q_heads % num_kv_heads != 0)
     return 1;
   if (ntiles <= 0) return 0;
+  flash_prefill::Args a{};
+  a.out = (uint16_t*)out;
+  a.q = (const uint16_t*)q;
+  a.q_stride = q_stride;
+  a.k_cache = (const uint16_t*)k_cache;
+  a.v_cache = (const uint16_t*)v_cache;
+  a.gate = (const uint16_t*)gate;
+  a.gate_stride = gate_stride;
+  a.sink = sink;
+  a.tile_seq = tile_seq;
+  a.tile_qstart = tile_qstart;
+  a.query_start_locs = query_start_locs;
+  a.context_lens = context_lens;
+  a.block_tables = block_tables;
+  a.score_bias = score_bias;
+  a.scale = scale;
+  a.temp_coef = temp_coef;
+  a.temp_every = temp_every;
+  a.temp_every_int = temp_every_int;
+  a.num_q_heads = num_q_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.v_row = v_row;
+  a.block_size = block_size;
+  a.block_shift = flash_prefill::shift_of(block_size);
+  a.max_blocks = max_blocks;
+  a.chunk = chunk;
+  a.window = window;
+  a.gate_per_head = gate_per_head;
+  a.softcap = softcap;
+  if (flash_prefill::serves(a, D, Dv)) {
+#define LAUNCH_FP(HD)                                                                      \
+  do {                                                                                     \
+    if (softcap > 0.f && sigmoid_weights)                                                  \
+      flash_prefill::launch_mode<HD, true, true, true>(a, ntiles, stream);                 \
+    else if (softcap > 0.f)                                                                \
+      flash_prefill::launch_mode<HD, true, false, true>(a, ntiles, stream);                \
+    else if (sigmoid_weights)                                                              \
+      flash_prefill::launch_mode<HD, false, true, true>(a, ntiles, stream);                \
+    else                                                                                   \
+      flash_prefill::launch_mode<HD, false, false, true>(a, ntiles, stream);               \
+  } while (0)
+    if (D == 64)
+      LAUNCH_FP(64);
+    else
+      LAUNCH_FP(128);
+#undef LAUNCH_FP
+    return 0;
+  }
   dim3 grid(ntiles, num_q_heads);
   dim3 block(256);
 #define LAUNCH_PT(DKP, DVP)                                                   \

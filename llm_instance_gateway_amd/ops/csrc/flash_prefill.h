@@ -1,0 +1,453 @@
+// Paged flash attention over prompt portions on MFMA tiles: bf16, key and
+// value heads of the same size 64 or 128, gfx950.  Shared by the Llama path
+// (torch extension) and the hybrid families' path (light library).
+//
+// What bounds it: at a few thousand keys the two contractions, 4 * D flops per
+// (row, key) pair and head.  The kernel this replaces gave a workgroup ONE
+// query head and 16 rows per wave, so every 16 rows of every head read the K
+// and V tile from LDS again, and its scores went through LDS between the two
+// products.  Here
+//   * a workgroup serves a tile of 64 query rows of GH heads of one key/value
+//     head, a wave RB = GH blocks of 16 rows of one of them, so an operand
+//     read from LDS feeds RB matrix instructions.  Two heads where that still
+//     gives every CU two workgroups, else one (see launch());
+//   * keys are dealt to the rows of the S^T = K Q^T tiles in the order in
+//     which a lane's scores ARE the operand of O^T += V^T P^T (rows g*4+i of
+//     two tiles hold keys g*8+i and g*8+4+i), so the weights never leave the
+//     registers, and row statistics are one scalar per lane for both products;
+//   * V is transposed while it is staged (byte permutes in registers), both
+//     tiles are XOR-swizzled so that the 16-byte operand reads of 8
+//     consecutive lanes cover all LDS banks;
+//   * the next 64 keys are loaded into registers while the current ones are
+//     used, LDS is double-buffered: one barrier per 64 keys;
+//   * the accumulators are only rescaled when a row's maximum grew, and masks
+//     are only evaluated on tiles that cross a row's visible range.
+// Measured, 32 query and 8 key/value heads of 128, before -> after: 4096 rows
+// on 4000 cached keys 3409 -> 495 us (119 -> 820 TFLOP/s); 20 prompts of 200
+// 130 -> 42 us; one of 202 20.6 -> 10.1 us; 8 of 1000 with a window of 512
+// 571 -> 114 us, with a soft cap 578 -> 137, with sigmoid weights 566 -> 110.
+// Four heads per workgroup and 64 rows per wave (all 512 registers, one wave
+// per SIMD) was slower everywhere: 781 us in the first of these.
+#pragma once
+
+#include "common.h"
+
+namespace flash_prefill {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int KT = 64;      // keys per tile
+constexpr int TQ = 64;      // query rows of a tile of the caller's tile list
+constexpr float LOG2E = 1.44269504088896340736f;
+
+struct Args {
+  uint16_t* out;            // [R, Hq * D]
+  const uint16_t* q;        // rows q_stride entries apart
+  long q_stride;
+  const uint16_t* k_cache;  // [blocks, Hkv, BS, D]
+  const uint16_t* v_cache;  // rows v_row entries apart
+  const uint16_t* gate;     // nullable
+  long gate_stride;
+  const float* sink;        // nullable, [Hq]
+  const int* tile_seq;
+  const int* tile_qstart;
+  const int* query_start_locs;
+  const int* context_lens;
+  const int* block_tables;
+  const float* score_bias;  // nullable, [Hq]
+  float scale;
+  float temp_coef, temp_every;
+  int temp_every_int;
+  int num_q_heads, num_kv_heads;
+  int v_row;
+  int block_size, block_shift;  // block_shift < 0: not a power of two
+  int max_blocks;
+  int chunk, window;
+  int gate_per_head;
+  float softcap;
+};
+
+// max over the four 16-lane groups, result in all of them
+LIG_DEVICE float max_over_groups(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t v = __builtin_bit_cast(uint32_t, y);
+  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+LIG_DEVICE uint32_t pack_bf16(float a, float b) {
+  return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+}
+
+// CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
+// sigmoid(score + bias) weights.  EXTRA: temperature, gate, sink, chunk and
+// window are looked at (the plain causal kernel leaves them out).
+template <int D, int GH, bool CAP, bool SIG, bool EXTRA>
+__global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
+  constexpr int RB = GH;       // blocks of 16 rows per wave
+
+  constexpr int KS = D / 32;   // matrix steps over the head size
+  constexpr int DB = D / 16;   // blocks of 16 output entries
+  constexpr int CH = D / 8;    // 16-byte chunks of a row
+  constexpr int TPT = KT * CH / 256;  // keys a thread stages: 4 (D = 128) or 2
+  static_assert(16 * RB * (4 / GH) == TQ, "a workgroup serves one query tile of each of its heads");
+
+  struct Shared {
+    uint16_t K[2][KT * D];
+    uint16_t VT[2][D * KT];
+  };
+  __shared__ Shared sm;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+
+  // grid.x runs over the head groups, so that with a multiple of 8 of them
+  // every XCD keeps to some heads' keys in its own L2; the tile list runs
+  // backwards, so that of one prompt the rows with the most keys start first
+  const int tile = gridDim.y - 1 - blockIdx.y;
+  const int s = a.tile_seq[tile];
+  const int qt = a.tile_qstart[tile];
+  const int lo = a.query_start_locs[s];
+  const int n = a.query_start_locs[s + 1] - lo;
+  if (qt >= n || n <= 0) return;
+  const int ctx = a.context_lens[s];
+  const int* bt = a.block_tables + (size_t)s * a.max_blocks;
+  const int group = a.num_q_heads / a.num_kv_heads;
+  const int per_kv = group / GH;
+  const int kvh = blockIdx.x / per_kv;
+  const int h = kvh * group + (blockIdx.x % per_kv) * GH + wave % GH;
+  const int row0 = qt + (wave / GH) * (16 * RB);  // first row of this wave in the portion
+
+  // ---- rows of this wave: row rb*16 + li belongs to this lane ---------------
+  bf16x8_t q_frag[RB][KS];
+  float c[RB];         // log2 units per unit of the raw score
+  int key_lo[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int r = row0 + rb * 16 + li;
+    const int rr = r < n ? r : n - 1;
+    const int qpos = ctx - n + rr;
+    float sc = a.scale;
+    key_lo[rb] = 0;
+    if (EXTRA) {
+      if (a.temp_coef != 0.f) {
+        const float m = a.temp_every_int > 0 ? (float)((qpos + 1) / a.temp_every_int)
+                                             : floorf((float)(qpos + 1) / a.temp_every);
+        sc *= 1.f + a.temp_coef * logf(m + 1.f);
+      }
+      if (a.chunk > 0) key_lo[rb] = (qpos / a.chunk) * a.chunk;
+      if (a.window > 0) key_lo[rb] = max(key_lo[rb], qpos - a.window + 1);
+    }
+    // a negative scale goes into the sign of the query, so that the largest
+    // raw score is the largest scaled one
+    const uint32_t flip = sc < 0.f ? 0x80008000u : 0u;
+    sc = fabsf(sc);
+    c[rb] = CAP ? sc / a.softcap : sc * LOG2E;
+    const uint16_t* qp = a.q + (size_t)(lo + rr) * a.q_stride + (size_t)h * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u32x4 raw = *reinterpret_cast<const u32x4*>(qp + ks * 32 + lg * 8);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) raw[e] ^= flip;
+      q_frag[rb][ks] = __builtin_bit_cast(bf16x8_t, raw);
+    }
+  }
+  const float bias = SIG && a.score_bias ? a.score_bias[h] : 0.f;
+  const float cap2 = CAP ? a.softcap * LOG2E : 0.f;
+
+  float m[RB], l[RB];
+  f32x4_t acc[RB][DB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    m[rb] = -INFINITY;
+    l[rb] = 0.f;
+    if (EXTRA && !SIG && a.sink) {
+      // a key with that unscaled score and no value; each lane sums its own keys, so
+      // only one of the four groups starts with it
+      m[rb] = a.sink[h] * LOG2E;
+      l[rb] = lg == 0 ? 1.f : 0.f;
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[rb][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // ---- walk ------------------------------------------------------------------
+  const int qpos0 = ctx - n + qt;
+  const int kv_end = min(ctx, qpos0 + TQ);
+  int kv_begin = 0;
+  if (EXTRA) {
+    if (a.chunk > 0) kv_begin = (qpos0 / a.chunk) * a.chunk;
+    if (a.window > 0) kv_begin = max(kv_begin, qpos0 - a.window + 1);
+    kv_begin = max(kv_begin, 0) & ~(KT - 1);
+  }
+  const int wave_first = ctx - n + row0;                                   // position of the wave's first row
+  const int wave_last_lo = __builtin_amdgcn_readlane(key_lo[RB - 1], 15);  // largest lower bound
+
+  // staging: this thread brings chunk `ch` of keys st*TPT .. +TPT
+  const int ch = tid % CH;
+  const int st = tid / CH;
+  const size_t kv_head_rows = (size_t)kvh * a.block_size;
+  const size_t block_rows = (size_t)a.num_kv_heads * a.block_size;
+  u32x4 kreg[TPT], vreg[TPT];
+
+  // keys past the end repeat the last one.  Where the block size is a multiple
+  // of 4 the TPT keys of a thread lie in one block (tiles start at multiples
+  // of 64), whose number is read one tile ahead
+  const bool one_block = (a.block_size & 3) == 0;
+  auto block_index = [&](int t) { return a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size; };
+  auto block_of = [&](int kv0) { return bt[block_index(min(kv0 + st * TPT, ctx - 1))]; };
+  auto fetch = [&](int kv0, int blk) {
+    int b0 = block_index(min(kv0 + st * TPT, ctx - 1)) * a.block_size;
+#pragma unroll
+    for (int i = 0; i < TPT; ++i) {
+      const int t = min(kv0 + st * TPT + i, ctx - 1);
+      if (!one_block) {
+        const int b = block_index(t);
+        blk = bt[b];
+        b0 = b * a.block_size;
+      }
+      const size_t row = (size_t)blk * block_rows + kv_head_rows + (t - b0);
+      kreg[i] = *reinterpret_cast<const u32x4*>(a.k_cache + row * D + ch * 8);
+      vreg[i] = *reinterpret_cast<const u32x4*>(a.v_cache + row * a.v_row + ch * 8);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < TPT; ++i) {
+      const int t = st * TPT + i;
+      const int f = (t & 3) | ((t >> 1) & 4);
+      *reinterpret_cast<u32x4*>(&sm.K[buf][t * D + ((ch ^ f) * 8)]) = kreg[i];
+    }
+    // entry e of key i -> row ch*8+e, key i; eight 16-byte units of 8 keys per row
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int d = ch * 8 + e;
+      const int unit = ((st * TPT) >> 3) ^ ((d ^ (d >> 3)) & 7);
+      uint16_t* p = &sm.VT[buf][d * KT + unit * 8 + ((st * TPT) & 7)];
+      const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+      if constexpr (TPT == 4) {
+        u32x2 w;
+        w[0] = __builtin_amdgcn_perm(vreg[1][e / 2], vreg[0][e / 2], sel);
+        w[1] = __builtin_amdgcn_perm(vreg[3][e / 2], vreg[2][e / 2], sel);
+        *reinterpret_cast<u32x2*>(p) = w;
+      } else {
+        *reinterpret_cast<uint32_t*>(p) = __builtin_amdgcn_perm(vreg[1][e / 2], vreg[0][e / 2], sel);
+      }
+    }
+  };
+
+  int blk_next = block_of(kv_begin);
+  fetch(kv_begin, blk_next);
+  blk_next = block_of(kv_begin + KT);
+  stage(0);
+  __syncthreads();
+
+  int buf = 0;
+  for (int kv0 = kv_begin; kv0 < kv_end; kv0 += KT, buf ^= 1) {
+    const bool more = kv0 + KT < kv_end;
+    if (more) {
+      fetch(kv0 + KT, blk_next);
+      blk_next = block_of(kv0 + 2 * KT);
+    }
+
+    // ---- S^T = K Q^T --------------------------------------------------------------
+    // s[rb][t2][x][i]: key kv0 + t2*32 + lg*8 + x*4 + i of row rb*16 + li
+    f32x4_t s4[RB][2][2];
+    {
+      // tile row li stands for key (li/4)*8 + li%4 (+4 in the second tile)
+      const int key_row = ((li >> 2) << 3) | (li & 3);
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const int t = t2 * 32 + key_row + x * 4;
+          const int f = (t & 3) | ((t >> 1) & 4);
+          bf16x8_t kf[KS];
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            kf[ks] = __builtin_bit_cast(
+                bf16x8_t, *reinterpret_cast<const u32x4*>(&sm.K[buf][t * D + (((ks * 4 + lg) ^ f) * 8)]));
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) {
+            s4[rb][t2][x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+              s4[rb][t2][x] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], q_frag[rb][ks], s4[rb][t2][x], 0, 0, 0);
+          }
+        }
+      }
+    }
+
+    // ---- weights -------------------------------------------------------------------
+    const bool masked = kv0 + KT - 1 > wave_first || kv0 < wave_last_lo;
+    bf16x8_t p_frag[RB][2];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      uint32_t dead = 0;  // bit per score of this lane
+      if (masked) {
+        const int qpos = ctx - n + row0 + rb * 16 + li;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int key = kv0 + (e >> 3) * 32 + lg * 8 + (e & 7);
+          if (key > qpos || key >= ctx || key < key_lo[rb]) {
+            dead |= 1u << e;
+            s4[rb][e >> 3][(e >> 2) & 1][e & 3] = -INFINITY;
+          }
+        }
+      }
+      float mx = -INFINITY;
+      if constexpr (!SIG) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s4[rb][e >> 3][(e >> 2) & 1][e & 3]);
+        mx = max_over_groups(mx);
+        if constexpr (CAP)
+          mx = mx == -INFINITY ? mx : cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
+                                                              1.f + __builtin_amdgcn_exp2f(mx * c[rb] * (2.f * LOG2E))));
+        else
+          mx = mx == -INFINITY ? mx : mx * c[rb];
+        if (__any(mx > m[rb])) {
+          const float m_new = fmaxf(m[rb], mx);
+          const float alpha = m[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[rb] - m_new);
+          m[rb] = m_new;
+          l[rb] *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[rb][db][i] *= alpha;
+        }
+      }
+      const float mm = m[rb] == -INFINITY ? 0.f : m[rb];
+      float p[16];
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float v = s4[rb][e >> 3][(e >> 2) & 1][e & 3];
+        float w;
+        if constexpr (CAP) {
+          // softcap * tanh(v * scale / softcap) in log2 units
+          const float b = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
+                                                  1.f + __builtin_amdgcn_exp2f(v * c[rb] * (2.f * LOG2E))));
+          if constexpr (SIG)
+            w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(b + bias * LOG2E)));
+          else
+            w = __builtin_amdgcn_exp2f(b - mm);
+        } else if constexpr (SIG) {
+          w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * c[rb] + bias * LOG2E)));
+        } else {
+          w = __builtin_amdgcn_exp2f(__builtin_fmaf(v, c[rb], -mm));
+        }
+        p[e] = w;
+      }
+      if (masked) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p[e] = (dead >> e) & 1 ? 0.f : p[e];
+      }
+      if constexpr (!SIG) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum += p[e];
+        l[rb] += sum;
+      }
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        u32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = pack_bf16(p[t2 * 8 + 2 * e], p[t2 * 8 + 2 * e + 1]);
+        p_frag[rb][t2] = __builtin_bit_cast(bf16x8_t, w);
+      }
+    }
+
+    // ---- O^T += V^T P^T --------------------------------------------------------------
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const int d = db * 16 + li;
+        const int unit = (t2 * 4 + lg) ^ ((d ^ (d >> 3)) & 7);
+        const bf16x8_t vf =
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(&sm.VT[buf][d * KT + unit * 8]));
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_frag[rb][t2], acc[rb][db], 0, 0, 0);
+      }
+    }
+
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  }
+
+  // ---- normalise, gate, store: this lane holds entries db*16 + lg*4 + i of its row ----
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int r = row0 + rb * 16 + li;
+    float f = 1.f;
+    if constexpr (!SIG) {
+      float t = l[rb];
+      t += __shfl_xor(t, 16, 64);
+      t += __shfl_xor(t, 32, 64);
+      f = t > 0.f ? 1.f / t : (t == 0.f ? 0.f : t);
+    }
+    if (r >= n) continue;
+    const uint16_t* gp = nullptr;
+    if (EXTRA && a.gate) {
+      gp = a.gate + (size_t)(lo + r) * a.gate_stride;
+      if (a.gate_per_head) {
+        f *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[h])));
+        gp = nullptr;
+      } else {
+        gp += (size_t)h * D;
+      }
+    }
+    uint16_t* op = a.out + ((size_t)(lo + r) * a.num_q_heads + h) * D;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      const int d = db * 16 + lg * 4;
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[i] = acc[rb][db][i] * f;
+        if (EXTRA && gp) o[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[d + i])));
+      }
+      u32x2 w;
+      w[0] = pack_bf16(o[0], o[1]);
+      w[1] = pack_bf16(o[2], o[3]);
+      *reinterpret_cast<u32x2*>(op + d) = w;
+    }
+  }
+}
+
+// What the kernel takes; callers without another kernel check it themselves.
+static inline bool serves(const Args& a, int D, int Dv) {
+  auto al = [](const void* p, unsigned to) { return (reinterpret_cast<uintptr_t>(p) & (to - 1)) == 0; };
+  return D == Dv && (D == 64 || D == 128) && a.q_stride % 8 == 0 && a.v_row % 8 == 0 && a.v_row >= D &&
+         al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
+}
+
+template <int D, bool CAP, bool SIG, bool EXTRA>
+static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
+  // Two heads per workgroup halve the reads of K and V; the line is where
+  // that leaves two workgroups for every CU (heads of 128, 32 over 8):
+  // 1280 workgroups 41.6 us against 47.8 with one head, 4096 rows on 4000 keys
+  // 495 against 680, but 96 workgroups 34 us against 25, 64 12.6 against 10.1
+  const int group = a.num_q_heads / a.num_kv_heads;
+  if (group % 2 == 0 && (long)ntiles * (a.num_q_heads / 2) >= 512)
+    hipLaunchKernelGGL((flash_prefill_kernel<D, 2, CAP, SIG, EXTRA>), dim3(a.num_q_heads / 2, ntiles), dim3(256), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((flash_prefill_kernel<D, 1, CAP, SIG, EXTRA>), dim3(a.num_q_heads, ntiles), dim3(256), 0,
+                       stream, a);
+}
+
+static inline int shift_of(int block_size) {
+  return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
+}
+
+}  // namespace flash_prefill

@@ -1,0 +1,131 @@
+"""The shared flash-prefill kernel at the sizes where its tiling can go wrong:
+portions around the 16-row blocks, 64-row tiles and 64-key tiles, block sizes
+that keep or split a thread's keys, group sizes that take one or two heads per
+workgroup, and the options' bounds.
+
+Tolerance: weights and results are rounded to bf16 once.  bf16 has 8 significant
+bits, so a rounding is off by at most half of 2^-7, that is 2^-8, and a result
+by at most 2^-7 of the weighted sum of |v|; sums are fp32 (1e-6 covers them)."""
+
+import pytest
+import torch
+
+from llm_instance_gateway_amd import ops
+from llm_instance_gateway_amd.ops import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+def _batch(segs, G, D, bs, H, seed):
+    """segs: (tokens after the step, tokens it brings) per sequence."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    need = [(c + bs - 1) // bs for c, _ in segs]
+    pool = sum(need) + 3
+    perm = torch.randperm(pool, generator=torch.Generator().manual_seed(seed))[: sum(need)].tolist()
+    tab, at = [], 0
+    for k in need:
+        tab.append(perm[at : at + k] + [0] * (max(need) - k))
+        at += k
+    T = sum(n for _, n in segs)
+    starts = [sum(n for _, n in segs[:i]) for i in range(len(segs) + 1)]
+    tiles = [(i, b) for i, (_, n) in enumerate(segs) for b in range(0, n, 64)]
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(BF)
+    return dict(
+        q=rnd(T, H * D), k=rnd(pool, G, bs, D), v=rnd(pool, G, bs, D), tab=i32(tab), starts=i32(starts),
+        ctx=i32([c for c, _ in segs]), ts=i32([a for a, _ in tiles]), tq=i32([b for _, b in tiles]),
+        tok_seq=i32([i for i, (_, n) in enumerate(segs) for _ in range(n)]),
+        pos=torch.tensor([p for c, n in segs for p in range(c - n, c)], device="cuda"), rnd=rnd,
+    )
+
+
+def _check(got, b, D, scale, H, **kw):
+    args = (b["k"].float(), b["v"].float(), b["tab"], b["tok_seq"], b["pos"], scale, H)
+    ref = torch_ref.paged_attention_general(b["q"].float(), *args, **kw)
+    mag = torch_ref.paged_attention_general(b["q"].float(), args[0], args[1].abs(), *args[2:], **kw)
+    assert torch.isfinite(got.float()).all()
+    assert ((got.float() - ref).abs() <= 2.0 ** -7 * mag.abs() + 1e-6).all()
+
+
+SEGS = [
+    [(1, 1)], [(16, 16), (17, 17)], [(63, 63), (64, 64), (65, 65)], [(65, 1), (128, 64), (129, 64), (200, 72)],
+    [(700, 130), (66, 2), (64, 5)],
+]
+
+
+@pytest.mark.parametrize("segs", SEGS, ids=range(len(SEGS)))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (128, 3, 1, 6), (64, 4, 4, 32), (64, 6, 1, 2)])
+def test_causal(segs, D, H, G, bs):
+    b = _batch(segs, G, D, bs, H, 7)
+    T = b["q"].shape[0]
+    got = ops.paged_attention_prefill(
+        b["q"].view(T, H, D), b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+        tile_qstart=b["tq"])
+    _check(got.view(T, -1), b, D, D ** -0.5, H)
+
+
+@pytest.mark.parametrize("D,H,G", [(128, 32, 8), (64, 32, 16)])
+def test_two_heads_per_workgroup(D, H, G):
+    # enough tiles for the two-head workgroups, the last portions ragged
+    segs = [(130, 130)] * 12 + [(1000, 65), (64, 64), (61, 61)]
+    b = _batch(segs, G, D, 16, H, 8)
+    T = b["q"].shape[0]
+    assert b["ts"].shape[0] * H // 2 >= 512
+    got = ops.paged_attention_prefill(
+        b["q"].view(T, H, D), b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+        tile_qstart=b["tq"])
+    _check(got.view(T, -1), b, D, D ** -0.5, H)
+
+
+OPTIONS = [
+    dict(window=1), dict(window=64), dict(window=65, softcap=5.0), dict(chunk=48), dict(chunk=64, temp_coef=0.3, temp_every=16.0),
+    dict(weights="sigmoid", bias=True, window=100), dict(weights="sigmoid", softcap=3.0), dict(sink=True, gate="entry"),
+    dict(sink=True, gate="head", softcap=30.0, window=40), dict(scale=-0.2), dict(scale=0.0, window=33),
+    dict(temp_coef=-0.9, temp_every=8.0),
+]
+
+
+@pytest.mark.parametrize("opt", OPTIONS, ids=range(len(OPTIONS)))
+@pytest.mark.parametrize("D,H,G,many", [(128, 4, 2, False), (64, 6, 2, False), (128, 32, 8, True)])
+def test_options(opt, D, H, G, many):
+    opt = dict(opt)
+    segs = [(63, 63), (200, 137), (130, 1)] + ([(129, 129)] * 12 if many else [])
+    b = _batch(segs, G, D, 16, H, 9)
+    scale = opt.pop("scale", D ** -0.5)
+    if opt.pop("bias", False):
+        opt["score_bias"] = b["rnd"](H).float()
+    if opt.pop("sink", False):
+        opt["sink"] = b["rnd"](H).float()
+    gate = opt.pop("gate", None)
+    if gate:
+        T = b["q"].shape[0]
+        wide = b["rnd"](T, H * D + H + 3)
+        opt["gate"] = wide[:, 3 : 3 + (H if gate == "head" else H * D)]
+        opt["gate_per_head"] = gate == "head"
+    got = ops.paged_attention_prefill_tiles(
+        b["q"], b["k"], b["v"], b["tab"], b["starts"], b["ctx"], b["ts"], b["tq"], scale, H, **opt)
+    _check(got, b, D, scale, H, **opt)
+
+
+def test_infinite_and_lowest_scores():
+    """A key whose score is -inf or the type's lowest weighs nothing, NaN stays in its own row and head."""
+    D, H, G = 128, 2, 1
+    b = _batch([(70, 70)], G, D, 16, H, 10)
+    low = torch.finfo(BF).min
+    q = b["q"].view(70, H, D)
+    q[:, :, 0] = 1.0
+    blk = b["tab"][0]
+    b["k"][blk[0], 0, 3, 0] = -float("inf")
+    b["k"][blk[1], 0, 5, 0] = low
+    got = ops.paged_attention_prefill(q, b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+                                      tile_qstart=b["tq"])
+    _check(got.view(70, -1), b, D, D ** -0.5, H)
+    q[9, 1, 7] = float("nan")
+    bad = ops.paged_attention_prefill(q, b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+                                      tile_qstart=b["tq"])
+    assert bad[9, 1].isnan().all()
+    keep = torch.ones(70, H, dtype=torch.bool, device="cuda")
+    keep[9, 1] = False
+    assert torch.equal(bad[keep], got[keep])
