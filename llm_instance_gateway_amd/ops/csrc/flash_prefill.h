@@ -84,10 +84,10 @@ LIG_DEVICE uint32_t pack_bf16(float a, float b) {
   return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
 }
 
-// CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
+// PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
 // sigmoid(score + bias) weights.  EXTRA: temperature, gate, sink, chunk and
 // window are looked at (the plain causal kernel leaves them out).
-template <int D, int GH, bool CAP, bool SIG, bool EXTRA>
+template <int D, int GH, bool PB, bool CAP, bool SIG, bool EXTRA>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   constexpr int RB = GH;       // blocks of 16 rows per wave
 
@@ -198,25 +198,26 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   const size_t block_rows = (size_t)a.num_kv_heads * a.block_size;
   u32x4 kreg[TPT], vreg[TPT];
 
-  // keys past the end repeat the last one.  Where the block size is a multiple
-  // of 4 the TPT keys of a thread lie in one block (tiles start at multiples
-  // of 64), whose number is read one tile ahead
-  const bool one_block = (a.block_size & 3) == 0;
-  auto block_index = [&](int t) { return a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size; };
-  auto block_of = [&](int kv0) { return bt[block_index(min(kv0 + st * TPT, ctx - 1))]; };
+  // keys past the end repeat the last one.  PB: the TPT keys of a thread lie in
+  // one block (tiles start at multiples of 64), whose number is read one tile
+  // ahead; no branch may stand between the loads, or each would be waited for
+  auto block_of = [&](int kv0) { return PB ? bt[min(kv0 + st * TPT, ctx - 1) >> a.block_shift] : 0; };
   auto fetch = [&](int kv0, int blk) {
-    int b0 = block_index(min(kv0 + st * TPT, ctx - 1)) * a.block_size;
+    size_t row[TPT];
 #pragma unroll
     for (int i = 0; i < TPT; ++i) {
       const int t = min(kv0 + st * TPT + i, ctx - 1);
-      if (!one_block) {
-        const int b = block_index(t);
-        blk = bt[b];
-        b0 = b * a.block_size;
+      if constexpr (PB) {
+        row[i] = (size_t)blk * block_rows + kv_head_rows + (t & (a.block_size - 1));
+      } else {
+        const int b = t / a.block_size;
+        row[i] = (size_t)bt[b] * block_rows + kv_head_rows + (t - b * a.block_size);
       }
-      const size_t row = (size_t)blk * block_rows + kv_head_rows + (t - b0);
-      kreg[i] = *reinterpret_cast<const u32x4*>(a.k_cache + row * D + ch * 8);
-      vreg[i] = *reinterpret_cast<const u32x4*>(a.v_cache + row * a.v_row + ch * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < TPT; ++i) {
+      kreg[i] = *reinterpret_cast<const u32x4*>(a.k_cache + row[i] * D + ch * 8);
+      vreg[i] = *reinterpret_cast<const u32x4*>(a.v_cache + row[i] * a.v_row + ch * 8);
     }
   };
   auto stage = [&](int buf) {
@@ -431,6 +432,15 @@ static inline bool serves(const Args& a, int D, int Dv) {
          al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
 }
 
+template <int D, int GH, bool CAP, bool SIG, bool EXTRA>
+static void launch_heads(const Args& a, int ntiles, hipStream_t stream) {
+  const dim3 grid(a.num_q_heads / GH, ntiles), block(256);
+  if (a.block_shift >= 2)
+    hipLaunchKernelGGL((flash_prefill_kernel<D, GH, true, CAP, SIG, EXTRA>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((flash_prefill_kernel<D, GH, false, CAP, SIG, EXTRA>), grid, block, 0, stream, a);
+}
+
 template <int D, bool CAP, bool SIG, bool EXTRA>
 static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
   // Two heads per workgroup halve the reads of K and V; the line is where
@@ -439,11 +449,9 @@ static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
   // 495 against 680, but 96 workgroups 34 us against 25, 64 12.6 against 10.1
   const int group = a.num_q_heads / a.num_kv_heads;
   if (group % 2 == 0 && (long)ntiles * (a.num_q_heads / 2) >= 512)
-    hipLaunchKernelGGL((flash_prefill_kernel<D, 2, CAP, SIG, EXTRA>), dim3(a.num_q_heads / 2, ntiles), dim3(256), 0,
-                       stream, a);
+    launch_heads<D, 2, CAP, SIG, EXTRA>(a, ntiles, stream);
   else
-    hipLaunchKernelGGL((flash_prefill_kernel<D, 1, CAP, SIG, EXTRA>), dim3(a.num_q_heads, ntiles), dim3(256), 0,
-                       stream, a);
+    launch_heads<D, 1, CAP, SIG, EXTRA>(a, ntiles, stream);
 }
 
 static inline int shift_of(int block_size) {
