@@ -107,14 +107,15 @@ def reshape_and_cache(
     torch_ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
-# Flash-decoding context split (ROADMAP r01 #1, measured in
-# profiles/r01_flash_decode_split.txt: 13.7x at N=4/ctx=16k, neutral at
-# chip-filling batch).  The single-pass kernel launches N*Hkv workgroups;
-# when that is far below the chip's 256 CUs and the context is long, split
-# the context across `ns` workgroups + a combine pass (bit-exact merge).
+# Context split of the paged decode kernel: with rows x kv heads workgroups
+# short of four per CU, every walk is cut into parts of at least 512 keys that
+# other workgroups take, and a second kernel merges them.  Measured, 8 kv heads
+# of 128: 33 requests of 3000-6000 tokens 147 us uncut, 126 in 2 parts, 114 in
+# 4 or 8, 122 in 16; 4 of 3000-8000 27 us in 8, 31 in 16; one of 2048 22 us
+# uncut, 12.9 in 4; one of 381 8.8 uncut, 11.1 in 2.
 _NUM_CUS = 256
-_SPLIT_MIN_CTX = 1024      # short contexts: single-pass latency already fine
-_SPLIT_MIN_PER_SPLIT = 256  # keep each split's K/V walk worth a workgroup
+_SPLIT_MIN_CTX = 1024
+_SPLIT_MIN_PER_SPLIT = 512
 _SPLIT_MAX = 32
 _SPLIT_SCRATCH: dict = {}   # device -> fp32 scratch tensor
 # Superseded scratches stay referenced: a captured hipGraph bakes the pointer
@@ -126,7 +127,7 @@ _SPLIT_SCRATCH_RETIRED: list = []
 def decode_nsplits(n_seqs: int, n_kv_heads: int, max_ctx: int) -> int:
     """Context-split factor for the paged decode kernel (1 = single-pass)."""
     wg = n_seqs * n_kv_heads
-    target = 2 * _NUM_CUS
+    target = 4 * _NUM_CUS
     if wg == 0 or wg >= target or max_ctx < _SPLIT_MIN_CTX:
         return 1
     ns = min(_SPLIT_MAX, (target + wg - 1) // wg)
@@ -526,6 +527,13 @@ def paged_attention_general(
         assert out.shape == (R, num_heads * Dv) and out.is_contiguous() and out.dtype == q.dtype
         ev = float(temp_every)
         ev_int = int(ev) if ev == int(ev) and ev >= 1 else 0
+        # few rows with a long walk: cut over workgroups (the matrix kernel only)
+        visible = block_tables.shape[1] * bs
+        for bound in (chunk, window):
+            visible = min(visible, bound) if bound > 0 else visible
+        nsplits, scratch = decode_nsplits(R, G, visible), None
+        if nsplits > 1 and q.dtype == torch.bfloat16 and D == Dv and D in (64, 128):
+            scratch = torch.empty(R * num_heads * nsplits * (D + 2), dtype=torch.float32, device=q.device)
         _hl().lig_paged_attention_general(
             _ptr(out), _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache),
             _ptr(block_tables), block_tables.shape[1], _ptr(tok_seq),
@@ -533,7 +541,7 @@ def paged_attention_general(
             _ptr(sink), float(scale), float(temp_coef), ev, ev_int, R, num_heads,
             G, D, Dv, v_row, bs, int(chunk), int(window), _ptr(score_bias),
             int(weights == "sigmoid"), int(bool(gate_per_head and gate is not None)),
-            float(softcap), _is_f32(q), _stream(),
+            float(softcap), nsplits, _ptr(scratch), _is_f32(q), _stream(),
         )
         return out
     res = torch_ref.paged_attention_general(

@@ -1,8 +1,10 @@
 // Paged causal attention for any head sizes, bf16 or fp32 storage, fp32
 // scores and softmax, gfx950.
 //
-// Serves the shapes the MFMA kernels do not: key size != value size, sizes
-// that are not 64/128, fp32 caches.  One wave per (token, query head part) walks
+// bf16 caches with equal key and value heads of 64 or 128 and up to 16 query
+// heads per key/value head run flash_decode.h's matrix kernel; the one here
+// serves what that does not: key size != value size, other sizes, fp32
+// caches.  One wave per (token, query head part) walks
 // the sequence's pages 64 keys at a time: lane j scores key j against the
 // query held in LDS, the wave keeps a running max / sum (online softmax),
 // then the lanes switch to value columns and accumulate sum_j p_j V[j, :].
@@ -39,6 +41,7 @@
 // own; a latent cache passes the key rows themselves, v_row == D).
 
 #include "elem_types.h"
+#include "flash_decode.h"
 
 #define ATT_MAX_DV_PER_LANE 8  // Dv <= 512
 
@@ -423,8 +426,58 @@ void lig_paged_attention_general(
     long gate_stride, const float* sink, float scale, float temp_coef,
     float temp_every, int temp_every_int, int R, int H, int G, int D, int Dv,
     int v_row, int BS, int chunk, int window, const float* score_bias,
-    int sigmoid_weights, int gate_per_head, float softcap, int is_f32, hipStream_t s) {
+    int sigmoid_weights, int gate_per_head, float softcap, int nsplits, float* scratch,
+    int is_f32, hipStream_t s) {
   if (R <= 0) return;
+  flash_decode::Args fa{};
+  fa.out = (uint16_t*)out;
+  fa.q = (const uint16_t*)q;
+  fa.q_stride = q_stride;
+  fa.k_cache = (const uint16_t*)k_cache;
+  fa.v_cache = (const uint16_t*)v_cache;
+  fa.gate = (const uint16_t*)gate;
+  fa.gate_stride = gate_stride;
+  fa.sink = sink;
+  fa.score_bias = score_bias;
+  fa.block_tables = block_tables;
+  fa.tok_seq = tok_seq;
+  fa.positions = positions;
+  fa.scratch = scratch;
+  fa.scale = scale;
+  fa.temp_coef = temp_coef;
+  fa.temp_every = temp_every;
+  fa.temp_every_int = temp_every_int;
+  fa.rows = R;
+  fa.num_q_heads = H;
+  fa.num_kv_heads = G;
+  fa.v_row = v_row;
+  fa.block_size = BS;
+  fa.block_shift = flash_decode::shift_of(BS);
+  fa.max_blocks = max_blocks;
+  fa.chunk = chunk;
+  fa.window = window;
+  fa.gate_per_head = gate_per_head;
+  fa.softcap = softcap;
+  fa.nsplits = scratch ? nsplits : 1;
+  if (!is_f32 && flash_decode::serves(fa, D, Dv)) {
+#define LIG_LAUNCH_FD(HD)                                          \
+  do {                                                             \
+    if (softcap > 0.f && sigmoid_weights)                          \
+      flash_decode::launch_mode<HD, true, true, true>(fa, s);      \
+    else if (softcap > 0.f)                                        \
+      flash_decode::launch_mode<HD, true, false, true>(fa, s);     \
+    else if (sigmoid_weights)                                      \
+      flash_decode::launch_mode<HD, false, true, true>(fa, s);     \
+    else                                                           \
+      flash_decode::launch_mode<HD, false, false, true>(fa, s);    \
+  } while (0)
+    if (D == 64)
+      LIG_LAUNCH_FD(64);
+    else
+      LIG_LAUNCH_FD(128);
+#undef LIG_LAUNCH_FD
+    return;
+  }
   // heads of one key/value head that a wave serves together: as many as
   // divide the group, but fewer while that would leave the chip short of
   // waves (a small batch of single tokens wants parallel walks first)

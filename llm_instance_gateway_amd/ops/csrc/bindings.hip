@@ -41,11 +41,7 @@ void lig_reshape_and_cache_launch(const uint16_t*, const uint16_t*, uint16_t*,
                                   int, hipStream_t);
 void lig_silu_and_mul_launch(uint16_t*, const uint16_t*, int, int,
                              hipStream_t);
-void lig_paged_attention_decode_launch(uint16_t*, const uint16_t*,
-                                       const uint16_t*, const uint16_t*,
-                                       const int*, const int*, float, int,
-                                       int, int, int, int, int, hipStream_t);
-void lig_paged_attention_decode_split_launch(
+void lig_paged_attention_decode_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*,
     const int*, const int*, float*, float, int, int, int, int, int, int,
     int, hipStream_t);
@@ -181,13 +177,12 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                   "decode context_lens");
   lig_paged_attention_decode_launch(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k_cache), bf16_cptr(v_cache),
-      block_tables.data_ptr<int>(), context_lens.data_ptr<int>(),
-      (float)scale, N, Hq, Hkv, D, BS, max_blocks, as_stream(stream));
+      block_tables.data_ptr<int>(), context_lens.data_ptr<int>(), nullptr,
+      (float)scale, N, Hq, Hkv, D, BS, max_blocks, 1, as_stream(stream));
 }
 
-// Flash-decoding variant: context split across nsplits workgroups with an
-// fp32 partial scratch [N, Hq, nsplits, D+2] and a combine pass (ROADMAP #1;
-// experimental — not yet on the default dispatch path).
+// Flash-decoding variant: every context cut over up to nsplits workgroups with
+// an fp32 partial scratch [N, Hq, nsplits, D+2] and a merging pass.
 void paged_attention_decode_split(torch::Tensor out, torch::Tensor q,
                                   torch::Tensor k_cache,
                                   torch::Tensor v_cache,
@@ -206,10 +201,11 @@ void paged_attention_decode_split(torch::Tensor out, torch::Tensor q,
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(D == 16 || D == 64 || D == 128, "head_dim must be 16/64/128");
   TORCH_CHECK(Hq % Hkv == 0 && Hq / Hkv <= 16, "bad GQA group size");
+  TORCH_CHECK(nsplits >= 1, "nsplits must be positive");
   TORCH_CHECK(scratch.numel() >= (int64_t)N * Hq * nsplits * (D + 2),
               "scratch too small");
   if (N == 0) return;
-  lig_paged_attention_decode_split_launch(
+  lig_paged_attention_decode_launch(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k_cache), bf16_cptr(v_cache),
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(),
       scratch.data_ptr<float>(), (float)scale, N, Hq, Hkv, D, BS,

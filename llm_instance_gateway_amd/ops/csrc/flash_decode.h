@@ -1,0 +1,480 @@
+// Paged attention of single query rows on MFMA tiles: bf16, key and value
+// heads of the same size 64 or 128, up to 16 query heads per key/value head,
+// gfx950.  Shared by the Llama decode path (torch extension) and the hybrid
+// families' row kernel (light library).
+//
+// What bounds it: every cached key and value is read once, so HBM.  The kernel
+// this replaces gave every query head a wave of its own: each cache line came
+// through the vector L1 once per head of the group, every product was a VALU
+// instruction, and 8 keys per step with a serial softmax left too little in
+// flight (1.5 TB/s on long ragged contexts, 2.7 at 384 requests).  Here one
+// wave serves all heads of the group and takes 32 keys per step:
+//   * S^T = K Q^T and O^T += V^T P^T are matrix instructions whose spare
+//     columns carry the group's heads; operands come straight from global
+//     memory in 16-byte loads of whole rows, no LDS;
+//   * keys are dealt to the rows of the two S^T tiles so that a lane's scores
+//     are its part of the second product's operand; V is transposed by byte
+//     permutes in registers; a lane keeps one head's statistics;
+//   * weights enter the second product as the sum of two bf16 numbers (17
+//     bits).  With up to 8 heads the low parts ride in columns 8..15, which
+//     would be idle, and are added at the end;
+//   * the next step's K is requested once S^T is formed, its V once O^T is, so
+//     a wave always has 8 to 16 KB on the way;
+//   * the waves of a workgroup take steps in turn and merge through LDS; long
+//     contexts are also cut over workgroups (nsplits) and merged by a second
+//     kernel.
+// Measured, 32 query and 8 key/value heads of 128, before -> after: 384
+// requests of 190-381 tokens 173 -> 84 us (5.3 TB/s; a large copy reaches 4.9);
+// 33 of 3000-6000 370 -> 114 us; 16 of 190-381 30 -> 8.3 us; 64 rows with a
+// window of 512 and sigmoid weights 64 -> 28 us.  Eight waves per workgroup
+// were slower from 64 requests on (101 us at 384), two on few (9.2 us at 16).
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace flash_decode {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int KT = 32;  // keys per step
+constexpr float LOG2E = 1.44269504088896340736f;
+
+struct Args {
+  uint16_t* out;            // [R, Hq * D]
+  const uint16_t* q;        // rows q_stride entries apart
+  long q_stride;
+  const uint16_t* k_cache;  // [blocks, Hkv, BS, D]
+  const uint16_t* v_cache;  // rows v_row entries apart
+  const uint16_t* gate;     // nullable
+  long gate_stride;
+  const float* sink;        // nullable, [Hq]
+  const float* score_bias;  // nullable, [Hq]
+  const int* block_tables;  // [S, max_blocks]
+  // row r belongs to table row tok_seq[r] (negative: none) and sees keys up to
+  // positions[r]; without them it is table row r, up to context_lens[r] - 1
+  const int* tok_seq;
+  const int64_t* positions;
+  const int* context_lens;
+  float* scratch;           // [R, Hq, nsplits, D + 2] with nsplits > 1
+  float scale;
+  float temp_coef, temp_every;
+  int temp_every_int;
+  int rows, num_q_heads, num_kv_heads;
+  int v_row;
+  int block_size, block_shift;  // block_shift < 0: not a power of two
+  int max_blocks;
+  int chunk, window;
+  int gate_per_head;
+  float softcap;
+  int nsplits;
+};
+
+LIG_DEVICE float swap_max(float x) {  // max over the four 16-lane groups
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t v = __builtin_bit_cast(uint32_t, y);
+  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+// The steps of a row: its position and lower bound, and into how many parts
+// its walk is cut: the caller's number, but no part under 16 steps (512 keys),
+// which one workgroup takes in the time of the merge.
+struct Walk {
+  int seq, pos, key_lo, first, steps, parts;
+};
+template <bool EXTRA>
+LIG_DEVICE Walk walk_of(const Args& a, int row) {
+  Walk w;
+  w.seq = a.tok_seq ? a.tok_seq[row] : row;
+  w.pos = w.seq < 0 ? -1 : a.positions ? (int)a.positions[row] : a.context_lens[row] - 1;
+  w.key_lo = 0;
+  if (EXTRA && w.pos >= 0) {
+    if (a.chunk > 0) w.key_lo = (w.pos / a.chunk) * a.chunk;
+    if (a.window > 0) w.key_lo = max(w.key_lo, w.pos - a.window + 1);
+  }
+  w.first = w.key_lo / KT;
+  w.steps = w.pos < 0 ? 0 : w.pos / KT + 1 - w.first;
+  w.parts = max(1, min(a.nsplits, w.steps / 16));
+  return w;
+}
+
+// final scaling of 4 entries of a (row, head), common to both kernels
+template <int D, bool EXTRA>
+LIG_DEVICE void store_entries(const Args& a, int row, int h, int d, const float (&o)[4], float f) {
+  const uint16_t* gp = nullptr;
+  if (EXTRA && a.gate) {
+    gp = a.gate + (size_t)row * a.gate_stride;
+    if (a.gate_per_head) {
+      f *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[h])));
+      gp = nullptr;
+    } else {
+      gp += (size_t)h * D + d;
+    }
+  }
+  u32x2 w;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float x = o[2 * i] * f, y = o[2 * i + 1] * f;
+    if (EXTRA && gp) {
+      x *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[2 * i])));
+      y *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[2 * i + 1])));
+    }
+    w[i] = (uint32_t)f32_to_bf16(x) | ((uint32_t)f32_to_bf16(y) << 16);
+  }
+  *reinterpret_cast<u32x2*>(a.out + ((size_t)row * a.num_q_heads + h) * D + d) = w;
+}
+
+// W waves per workgroup; LOWCOL: at most 8 heads per group, the weights' low
+// parts in columns 8..15; PB: block size a power of two, at least 8.  CAP, SIG, EXTRA as in the prompt kernel.
+template <int D, int W, bool LOWCOL, bool PB, bool CAP, bool SIG, bool EXTRA>
+__global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
+  constexpr int KS = D / 32;
+  constexpr int DV = D / 16;          // entries of a value row per lane
+  constexpr int GM = LOWCOL ? 8 : 16;  // heads a wave can hold
+  using vload = typename std::conditional<DV == 8, u32x4, u32x2>::type;
+
+  // [W][group][D] sums, [W][GM] maxima, [W][GM] weight sums
+  extern __shared__ float smem[];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int kvh = blockIdx.x % a.num_kv_heads;
+  const int row = blockIdx.x / a.num_kv_heads;
+  const int group = a.num_q_heads / a.num_kv_heads;
+  float* const m_s = smem + W * group * D;
+  float* const l_s = m_s + W * GM;
+
+  const Walk wk = walk_of<EXTRA>(a, row);
+  if ((int)blockIdx.y >= wk.parts) return;
+  if (wk.seq < 0) {  // a row of no sequence
+    for (int d = tid; d < group * D; d += 64 * W) a.out[((size_t)row * a.num_q_heads + kvh * group) * D + d] = 0;
+    return;
+  }
+  const int pos = wk.pos, key_lo = wk.key_lo;
+  const int* bt = a.block_tables + (size_t)wk.seq * a.max_blocks;
+  float sc = a.scale;
+  if (EXTRA && a.temp_coef != 0.f) {
+    const float t = a.temp_every_int > 0 ? (float)((pos + 1) / a.temp_every_int)
+                                         : floorf((float)(pos + 1) / a.temp_every);
+    sc *= 1.f + a.temp_coef * logf(t + 1.f);
+  }
+  const int span = (wk.steps + wk.parts - 1) / wk.parts;
+  const int c0 = wk.first + blockIdx.y * span;
+  const int c1 = min(wk.first + wk.steps, c0 + span);
+
+  // a negative scale goes into the sign of the query, so that the largest raw
+  // score is the largest scaled one
+  const uint32_t flip = sc < 0.f ? 0x80008000u : 0u;
+  sc = fabsf(sc);
+  const float c = CAP ? sc / a.softcap : sc * LOG2E;
+  const float cap2 = CAP ? a.softcap * LOG2E : 0.f;
+  const int hl = LOWCOL ? li & 7 : li;       // head of this lane in the group
+  const int h = kvh * group + min(hl, group - 1);
+  const float bias = SIG && a.score_bias ? a.score_bias[h] : 0.f;
+  bf16x8_t q_frag[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    u32x4 raw = *reinterpret_cast<const u32x4*>(a.q + (size_t)row * a.q_stride + (size_t)h * D + ks * 32 + lg * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) raw[e] ^= flip;
+    q_frag[ks] = __builtin_bit_cast(bf16x8_t, raw);
+  }
+
+  // rows of a step: S^T tile row li stands for key (li/4)*8 + li%4 (+4 in the
+  // second tile), this lane's values are keys lg*8 .. +8.  Keys past the end
+  // repeat the last one.  PB: a lane's 8 keys lie in one block, whose number
+  // is read one step ahead; no branch may stand between the loads, or each
+  // would be waited for by itself
+  const size_t block_rows = (size_t)a.num_kv_heads * a.block_size;
+  const size_t head_rows = (size_t)kvh * a.block_size;
+  const int kt0 = (li >> 2) * 8, vt0 = lg * 8;
+  const int shift = a.block_shift;
+  auto block_at = [&](int st, int t0) { return PB ? bt[min(st * KT + t0, pos) >> shift] : 0; };
+  u32x4 kreg[2][KS];
+  vload vreg[8];
+  // cache rows of N keys of the 8 from t0 on
+  auto rows_of = [&](int t0, int first_t, int by, int blk, auto& r) {
+    constexpr int N = sizeof(r) / sizeof(r[0]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int t = min(t0 + first_t + i * by, pos);
+      if constexpr (PB) {
+        r[i] = (size_t)blk * block_rows + head_rows + (t & (a.block_size - 1));
+      } else {
+        const int b = t / a.block_size;
+        r[i] = (size_t)bt[b] * block_rows + head_rows + (t - b * a.block_size);
+      }
+    }
+  };
+  auto fetch_k = [&](int st, int blk) {
+    size_t r[2];
+    rows_of(st * KT + kt0, li & 3, 4, blk, r);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        kreg[x][ks] = *reinterpret_cast<const u32x4*>(a.k_cache + r[x] * D + lg * 8 + ks * 32);
+  };
+  auto fetch_v = [&](int st, int blk) {
+    size_t r[8];
+    rows_of(st * KT + vt0, 0, 1, blk, r);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) vreg[t] = *reinterpret_cast<const vload*>(a.v_cache + r[t] * a.v_row + li * DV);
+  };
+
+  float m = -INFINITY, l = 0.f;
+  f32x4_t acc[DV];  // O^T: head column li, entries (lg*4 + i) * DV + j
+#pragma unroll
+  for (int j = 0; j < DV; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  int st = c0 + wave;
+  if (st < c1) {
+    int kb = block_at(st, kt0), vb = block_at(st, vt0);
+    fetch_k(st, kb);
+    fetch_v(st, vb);
+    kb = block_at(st + W, kt0);
+    vb = block_at(st + W, vt0);
+    for (; st < c1; st += W) {
+      const bool more = st + W < c1;
+      f32x4_t s4[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        s4[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          s4[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kreg[x][ks]), q_frag[ks], s4[x],
+                                                          0, 0, 0);
+      }
+      // the block numbers of the step after next are asked for first: loads
+      // return in order, so waiting for them must not mean waiting for V
+      const int kb2 = block_at(st + 2 * W, kt0), vb2 = block_at(st + 2 * W, vt0);
+      if (more) fetch_k(st + W, kb);
+
+      // weights of keys st*32 + lg*8 + e
+      const bool masked = st * KT + KT - 1 > pos || st * KT < key_lo;
+      float p[8];
+      uint32_t dead = 0;
+      if (masked) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = st * KT + lg * 8 + e;
+          if (key > pos || key < key_lo) {
+            dead |= 1u << e;
+            s4[e >> 2][e & 3] = -INFINITY;
+          }
+        }
+      }
+      float mm = 0.f;
+      if constexpr (!SIG) {
+        float mx = s4[0][0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s4[e >> 2][e & 3]);
+        mx = swap_max(mx);
+        if constexpr (CAP)
+          mx = mx == -INFINITY ? mx : cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
+                                                              1.f + __builtin_amdgcn_exp2f(mx * c * (2.f * LOG2E))));
+        else
+          mx = mx == -INFINITY ? mx : mx * c;
+        if (__any(mx > m)) {
+          const float m_new = fmaxf(m, mx);
+          const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+          m = m_new;
+          l *= alpha;
+#pragma unroll
+          for (int j = 0; j < DV; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[j][i] *= alpha;
+        }
+        mm = m == -INFINITY ? 0.f : m;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = s4[e >> 2][e & 3];
+        float w;
+        if constexpr (CAP) {
+          const float b = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
+                                                  1.f + __builtin_amdgcn_exp2f(v * c * (2.f * LOG2E))));
+          if constexpr (SIG)
+            w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(b + bias * LOG2E)));
+          else
+            w = __builtin_amdgcn_exp2f(b - mm);
+        } else if constexpr (SIG) {
+          w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * c + bias * LOG2E)));
+        } else {
+          w = __builtin_amdgcn_exp2f(__builtin_fmaf(v, c, -mm));
+        }
+        p[e] = w;
+      }
+      if (masked) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = (dead >> e) & 1 ? 0.f : p[e];
+      }
+      u32x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint16_t a0 = f32_to_bf16(p[2 * e]), a1 = f32_to_bf16(p[2 * e + 1]);
+        const uint16_t b0 = f32_to_bf16(p[2 * e] - bf16_to_f32(a0)), b1 = f32_to_bf16(p[2 * e + 1] - bf16_to_f32(a1));
+        hi[e] = (uint32_t)a0 | ((uint32_t)a1 << 16);
+        lo[e] = (uint32_t)b0 | ((uint32_t)b1 << 16);
+        if constexpr (!SIG) l += p[2 * e] + p[2 * e + 1];
+      }
+      bf16x8_t pf = __builtin_bit_cast(bf16x8_t, hi), pl = __builtin_bit_cast(bf16x8_t, lo);
+      if constexpr (LOWCOL) pf = li < 8 ? pf : pl;
+
+#pragma unroll
+      for (int j = 0; j < DV; ++j) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+        u32x4 vt;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) vt[w] = __builtin_amdgcn_perm(vreg[2 * w + 1][j / 2], vreg[2 * w][j / 2], sel);
+        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, vt);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, acc[j], 0, 0, 0);
+        if constexpr (!LOWCOL) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, acc[j], 0, 0, 0);
+      }
+      if (more) fetch_v(st + W, vb);
+      kb = kb2;
+      vb = vb2;
+    }
+  }
+
+  // ---- merge the waves: low columns onto their heads, then over the waves ------
+  if constexpr (LOWCOL) {
+#pragma unroll
+    for (int j = 0; j < DV; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][i] += __shfl_xor(acc[j][i], 8, 64);
+  }
+  if constexpr (!SIG) {
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+  }
+  if (li < group && li < GM) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < DV; j += 4)
+        *reinterpret_cast<f32x4_t*>(&smem[(wave * group + li) * D + (lg * 4 + i) * DV + j]) =
+            f32x4_t{acc[j][i], acc[j + 1][i], acc[j + 2][i], acc[j + 3][i]};
+    if (lg == 0) {
+      m_s[wave * GM + li] = m;
+      l_s[wave * GM + li] = l;
+    }
+  }
+  __syncthreads();
+  for (int it = tid; it < group * (D / 4); it += 64 * W) {
+    const int hh = it / (D / 4), d = (it % (D / 4)) * 4;
+    const int head = kvh * group + hh;
+    const bool sink = EXTRA && !SIG && a.sink && wk.parts == 1;
+    float gm = sink ? a.sink[head] * LOG2E : -INFINITY;
+    float gl = 0.f;
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!SIG) {
+      const float sm = gm;
+#pragma unroll
+      for (int w = 0; w < W; ++w) gm = fmaxf(gm, m_s[w * GM + hh]);
+      if (sink) gl = __builtin_amdgcn_exp2f(sm - gm);
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      float f = 1.f;
+      if constexpr (!SIG) {
+        f = m_s[w * GM + hh] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_s[w * GM + hh] - gm);
+        gl += l_s[w * GM + hh] * f;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] += smem[(w * group + hh) * D + d + i] * f;
+    }
+    if (wk.parts > 1) {
+      float* sp = a.scratch + (((size_t)row * a.num_q_heads + head) * a.nsplits + blockIdx.y) * (D + 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sp[d + i] = o[i];
+      if (d == 0) {
+        sp[D] = gm;
+        sp[D + 1] = gl;
+      }
+    } else {
+      const float f = SIG ? 1.f : (gl > 0.f ? 1.f / gl : (gl == 0.f ? 0.f : gl));
+      store_entries<D, EXTRA>(a, row, head, d, o, f);
+    }
+  }
+}
+
+// merges the parts of a (row, head), 4 entries per lane
+template <int D, bool SIG, bool EXTRA>
+__global__ __launch_bounds__(64) void flash_decode_merge_kernel(const Args a) {
+  constexpr int LP = D / 4;  // lanes per (row, head)
+  const int item = blockIdx.x * (64 / LP) + threadIdx.x / LP;
+  if (item >= a.rows * a.num_q_heads) return;
+  const int row = item / a.num_q_heads, head = item % a.num_q_heads;
+  const int parts = walk_of<EXTRA>(a, row).parts;
+  if (parts == 1) return;  // stored by the first kernel
+  const int d = (threadIdx.x % LP) * 4;
+  const float* base = a.scratch + (size_t)item * a.nsplits * (D + 2);
+  const bool sink = EXTRA && !SIG && a.sink;
+  float gm = sink ? a.sink[head] * LOG2E : -INFINITY, gl = 0.f;
+  if constexpr (!SIG) {
+    const float sm = gm;
+    for (int z = 0; z < parts; ++z) gm = fmaxf(gm, base[(size_t)z * (D + 2) + D]);
+    if (sink) gl = __builtin_amdgcn_exp2f(sm - gm);
+  }
+  float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int z = 0; z < parts; ++z) {
+    const float* sp = base + (size_t)z * (D + 2);
+    float f = 1.f;
+    if constexpr (!SIG) {
+      f = sp[D] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sp[D] - gm);
+      gl += sp[D + 1] * f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] += sp[d + i] * f;
+  }
+  const float f = SIG ? 1.f : (gl > 0.f ? 1.f / gl : (gl == 0.f ? 0.f : gl));
+  store_entries<D, EXTRA>(a, row, head, d, o, f);
+}
+
+// What the kernel takes.
+static inline bool serves(const Args& a, int D, int Dv) {
+  auto al = [](const void* p, unsigned to) { return (reinterpret_cast<uintptr_t>(p) & (to - 1)) == 0; };
+  return D == Dv && (D == 64 || D == 128) && a.num_q_heads % a.num_kv_heads == 0 &&
+         a.num_q_heads / a.num_kv_heads <= 16 && a.q_stride % 8 == 0 && a.v_row % 8 == 0 && a.v_row >= D &&
+         al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
+}
+
+static inline int shift_of(int block_size) {
+  return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
+}
+
+template <int D, bool CAP, bool SIG, bool EXTRA>
+static void launch_mode(const Args& a, hipStream_t stream) {
+  constexpr int W = 4;
+  const int group = a.num_q_heads / a.num_kv_heads;
+  const dim3 grid(a.rows * a.num_kv_heads, a.nsplits), block(64 * W);
+  const bool low = group <= 8, pb = a.block_shift >= 3;
+  const size_t lds = (size_t)W * (group * D + 2 * (low ? 8 : 16)) * sizeof(float);
+  if (low && pb)
+    hipLaunchKernelGGL((flash_decode_kernel<D, W, true, true, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
+  else if (low)
+    hipLaunchKernelGGL((flash_decode_kernel<D, W, true, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
+  else if (pb)
+    hipLaunchKernelGGL((flash_decode_kernel<D, W, false, true, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
+  else
+    hipLaunchKernelGGL((flash_decode_kernel<D, W, false, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
+  if (a.nsplits > 1) {
+    const long lanes = (long)a.rows * a.num_q_heads * (D / 4);
+    hipLaunchKernelGGL((flash_decode_merge_kernel<D, SIG, EXTRA>), dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0,
+                       stream, a);
+  }
+}
+
+}  // namespace flash_decode

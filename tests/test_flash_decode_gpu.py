@@ -1,0 +1,124 @@
+"""The shared matrix kernel for single query rows at the sizes where it can go
+wrong: contexts around its 32-key steps and 512-key parts, group sizes on both
+sides of the low-part columns, block sizes that keep or split a lane's keys,
+and the options' bounds.
+
+Tolerance: weights enter the second product as two bf16 numbers, 16 significant
+bits (off by at most 2^-16, once more for the split), results are rounded to
+bf16 once (8 significant bits: at most 2^-8 of the value), sums are fp32."""
+
+import pytest
+import torch
+
+from llm_instance_gateway_amd import ops
+from llm_instance_gateway_amd.ops import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+CTX = [1, 2, 8, 31, 32, 33, 63, 64, 65, 127, 129, 511, 513, 1000, 1056]
+
+
+def _batch(ctx, G, D, bs, H, seed, pad=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(BF)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    need = [(c + bs - 1) // bs for c in ctx]
+    pool = sum(need) + 3
+    perm = torch.randperm(pool, generator=torch.Generator().manual_seed(seed))[: sum(need)].tolist()
+    tab, at = [], 0
+    for k in need:
+        tab.append(perm[at : at + k] + [0] * (max(need) - k))
+        at += k
+    n = len(ctx)
+    return dict(
+        q=rnd(n + pad, H * D), k=rnd(pool, G, bs, D), v=rnd(pool, G, bs, D), tab=i32(tab), ctx=i32(ctx), rnd=rnd,
+        tok_seq=i32(list(range(n)) + [-1] * pad),
+        pos=torch.tensor([c - 1 for c in ctx] + [0] * pad, device="cuda"),
+    )
+
+
+def _check(got, b, scale, H, **kw):
+    args = (b["k"].double(), b["v"].double(), b["tab"], b["tok_seq"], b["pos"], scale, H)
+    f = lambda v: torch_ref.paged_attention_general(b["q"].float(), args[0].float(), v.float(), *args[2:], **kw)
+    ref, mag = f(args[1]), f(args[1].abs())
+    assert torch.isfinite(got.float()).all()
+    # 2e-5: the reference's own fp32 scores and sums
+    assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-5 * mag + 1e-6).all()
+
+
+@pytest.mark.parametrize("nsplits", [1, 2, 5])
+@pytest.mark.parametrize(
+    "D,H,G,bs", [(128, 8, 2, 16), (128, 3, 1, 6), (128, 16, 2, 8), (128, 18, 2, 16), (64, 16, 1, 32), (64, 4, 4, 2), (128, 11, 1, 5)]
+)
+def test_decode(D, H, G, bs, nsplits):
+    b = _batch(CTX, G, D, bs, H, 3)
+    got = ops.paged_attention_decode(
+        b["q"].view(-1, H, D), b["k"], b["v"], b["tab"], b["ctx"], D ** -0.5, nsplits=nsplits)
+    _check(got.view(len(CTX), -1), b, D ** -0.5, H)
+
+
+def test_decode_empty_context():
+    b = _batch([5, 40], 2, 128, 16, 8, 4)
+    b["ctx"][0] = 0
+    got = ops.paged_attention_decode(b["q"].view(-1, 8, 128), b["k"], b["v"], b["tab"], b["ctx"], 0.1)
+    assert (got[0] == 0).all() and (got[1] != 0).any()
+
+
+OPTIONS = [
+    {}, dict(window=1), dict(window=64), dict(window=600), dict(window=65, softcap=5.0), dict(chunk=48),
+    dict(chunk=640, temp_coef=0.3, temp_every=16.0), dict(weights="sigmoid", bias=True, window=100),
+    dict(weights="sigmoid", softcap=3.0), dict(sink=True, gate="entry"), dict(sink=True, gate="head", softcap=30.0, window=40),
+    dict(scale=-0.2), dict(scale=0.0, window=33), dict(temp_coef=-0.9, temp_every=8.0),
+]
+
+
+@pytest.mark.parametrize("opt", OPTIONS, ids=range(len(OPTIONS)))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 4, 2, 16), (64, 12, 1, 16), (128, 6, 2, 3)])
+def test_options(opt, D, H, G, bs):
+    opt = dict(opt)
+    b = _batch(CTX, G, D, bs, H, 5, pad=2)
+    R = b["q"].shape[0]
+    scale = opt.pop("scale", D ** -0.5)
+    if opt.pop("bias", False):
+        opt["score_bias"] = b["rnd"](H).float()
+    if opt.pop("sink", False):
+        opt["sink"] = b["rnd"](H).float()
+    gate = opt.pop("gate", None)
+    if gate:
+        wide = b["rnd"](R, H * D + H + 3)
+        opt["gate"] = wide[:, 3 : 3 + (H if gate == "head" else H * D)]
+        opt["gate_per_head"] = gate == "head"
+    wide = torch.cat([b["rnd"](R, 8), b["q"]], dim=1)  # a column block
+    got = ops.paged_attention_general(
+        wide[:, 8:], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], scale, H, **opt)
+    _check(got, b, scale, H, **opt)
+    assert (got[-2:] == 0).all()
+
+
+@pytest.mark.parametrize("D,H,G", [(128, 32, 8), (64, 8, 4)])
+def test_values_of_a_wider_row(D, H, G):
+    """Values read from the head of the key rows (a latent cache)."""
+    b = _batch(CTX, G, D, 16, H, 6)
+    wide = b["rnd"](b["k"].shape[0], G, 16, D + 64)
+    b["v"] = wide[..., :D]
+    got = ops.paged_attention_general(b["q"], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], D ** -0.5, H)
+    _check(got, b, D ** -0.5, H)
+
+
+def test_infinite_and_lowest_scores():
+    D, H, G = 128, 4, 2
+    b = _batch([70, 70], G, D, 16, H, 10)
+    q = b["q"].view(2, H, D)
+    q[:, :, 0] = 1.0
+    blk = b["tab"]
+    b["k"][blk[0, 0], 0, 3, 0] = -float("inf")
+    b["k"][blk[0, 1], 0, 5, 0] = torch.finfo(BF).min
+    got = ops.paged_attention_decode(q, b["k"], b["v"], b["tab"], b["ctx"], D ** -0.5)
+    _check(got.view(2, -1), b, D ** -0.5, H)
+    q[0, 1, 7] = float("nan")
+    bad = ops.paged_attention_decode(q, b["k"], b["v"], b["tab"], b["ctx"], D ** -0.5)
+    assert bad[0, 1].isnan().all()
+    keep = torch.ones(2, H, dtype=torch.bool, device="cuda")
+    keep[0, 1] = False
+    assert torch.equal(bad[keep], got[keep])
