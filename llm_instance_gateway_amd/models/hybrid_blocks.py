@@ -149,16 +149,16 @@ class GatedAttention(nn.Module):
         np_, nd = meta.num_prefill_tokens, meta.num_decode_tokens
         out = torch.zeros_like(qh) if np_ + nd < qh.shape[0] else torch.empty_like(qh)
         if np_ > 0:
-            out[:np_] = ops.paged_attention_prefill(
+            ops.paged_attention_prefill(
                 qh[:np_], k_cache, v_cache, meta.prefill_block_tables,
                 meta.prefill_query_start_locs, meta.prefill_context_lens, self.scale,
-                tile_seq=meta.prefill_tile_seq, tile_qstart=meta.prefill_tile_qstart,
+                tile_seq=meta.prefill_tile_seq, tile_qstart=meta.prefill_tile_qstart, out=out[:np_],
             )
         if nd > 0:
-            out[np_ : np_ + nd] = ops.paged_attention_decode(
+            ops.paged_attention_decode(
                 qh[np_ : np_ + nd], k_cache, v_cache, meta.decode_block_tables,
                 meta.decode_context_lens, self.scale, max_ctx=meta.max_decode_ctx,
-                nsplits=meta.decode_nsplits,
+                nsplits=meta.decode_nsplits, out=out[np_ : np_ + nd],
             )
         o = out.view(-1, self.heads * self.vdim)
         if gate is not None:

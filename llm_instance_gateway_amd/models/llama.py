@@ -70,19 +70,15 @@ class Attention(nn.Module):
         qkv = self.qkv_proj(hidden)
         if self._lora is not None:
             self._lora.apply(self._layer_idx, "qkv", hidden, qkv, meta)
-        q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
-        q = q.contiguous()
-        k = k.contiguous()
-        q, k = ops.rotary_embedding(positions, q, k, cos_sin_cache, self.head_dim)
-
         k_cache, v_cache = kv_cache
-        ops.reshape_and_cache(k, v.contiguous(), k_cache, v_cache, meta.slot_mapping)
-
+        q = ops.qkv_rope_cache(
+            qkv, positions, cos_sin_cache, k_cache, v_cache, meta.slot_mapping, self.num_heads
+        )
         qh = q.view(-1, self.num_heads, self.head_dim)
         np_, nd = meta.num_prefill_tokens, meta.num_decode_tokens
         out = torch.empty_like(qh)
         if np_ > 0:
-            out[:np_] = ops.paged_attention_prefill(
+            ops.paged_attention_prefill(
                 qh[:np_],
                 k_cache,
                 v_cache,
@@ -94,11 +90,12 @@ class Attention(nn.Module):
                 tok_context_lens=meta.prefill_tok_context_lens,
                 tile_seq=meta.prefill_tile_seq,
                 tile_qstart=meta.prefill_tile_qstart,
+                out=out[:np_],
             )
         if nd > 0:
             # slice end is explicit: the flat batch may carry GEMM-bucketing
             # pad rows after the decode partition
-            out[np_:np_ + nd] = ops.paged_attention_decode(
+            ops.paged_attention_decode(
                 qh[np_:np_ + nd],
                 k_cache,
                 v_cache,
@@ -107,6 +104,7 @@ class Attention(nn.Module):
                 self.scale,
                 max_ctx=meta.max_decode_ctx,
                 nsplits=meta.decode_nsplits,
+                out=out[np_:np_ + nd],
             )
         attn_flat = out.view(-1, self.num_heads * self.head_dim)
         o = self.o_proj(attn_flat)

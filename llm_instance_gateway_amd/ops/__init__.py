@@ -107,6 +107,31 @@ def reshape_and_cache(
     torch_ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
+def qkv_rope_cache(
+    qkv: torch.Tensor,
+    positions: torch.Tensor,
+    cos_sin_cache: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    num_heads: int,
+) -> torch.Tensor:
+    """Between a fused projection qkv [T, (heads + 2 kv heads) * D] and the
+    attention over it: rotates q and k, writes k and v to the paged caches and
+    returns q [T, heads * D] contiguous.  qkv may be changed.  bf16 rows with
+    heads of a multiple of 64 take one kernel."""
+    D = k_cache.shape[-1]
+    nq, nk = num_heads * D, k_cache.shape[1] * D
+    if qkv.dtype == torch.bfloat16 and D % 64 == 0 and qkv.is_contiguous() and _use_native(qkv):
+        q = torch.empty(qkv.shape[0], nq, dtype=qkv.dtype, device=qkv.device)
+        _EXT.qkv_rope_cache(q, qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, _stream())
+        return q
+    q, k, v = qkv.split([nq, nk, nk], dim=-1)
+    q, k = rotary_embedding(positions, q.contiguous(), k.contiguous(), cos_sin_cache, D)
+    reshape_and_cache(k, v.contiguous(), k_cache, v_cache, slot_mapping)
+    return q
+
+
 # Context split of the paged decode kernel: with rows x kv heads workgroups
 # short of four per CU, every walk is cut into parts of at least 512 keys that
 # other workgroups take, and a second kernel merges them.  Measured, 8 kv heads
@@ -157,12 +182,15 @@ def paged_attention_decode(
     scale: float,
     max_ctx: int = 0,
     nsplits: int = 0,
+    out: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """`max_ctx` is a host-side hint (no device sync) driving the split
     heuristic; `nsplits` > 0 pins the factor (the hipGraph path captures a
-    bucket-static value)."""
+    bucket-static value).  `out`: contiguous, like q."""
     if _use_native(q):
-        out = torch.empty_like(q)
+        if out is None:
+            out = torch.empty_like(q)
+        assert out.shape == q.shape and out.dtype == q.dtype
         N, Hq, D = q.shape
         Hkv = k_cache.shape[1]
         ns = nsplits if nsplits > 0 else decode_nsplits(N, Hkv, max_ctx)
@@ -178,9 +206,10 @@ def paged_attention_decode(
                 _stream()
             )
         return out
-    return torch_ref.paged_attention_decode(
+    res = torch_ref.paged_attention_decode(
         q, k_cache, v_cache, block_tables, context_lens, scale
     )
+    return res if out is None else out.copy_(res)
 
 
 def paged_attention_prefill(
@@ -195,7 +224,10 @@ def paged_attention_prefill(
     tok_context_lens: "Optional[torch.Tensor]" = None,
     tile_seq: "Optional[torch.Tensor]" = None,
     tile_qstart: "Optional[torch.Tensor]" = None,
+    out: "Optional[torch.Tensor]" = None,
 ) -> torch.Tensor:
+    """`out`: contiguous, like q."""
+    assert out is None or (out.shape == q.shape and out.dtype == q.dtype)
     if _use_native(q):
         head_dim = q.shape[-1]
         if head_dim in (64, 128):
@@ -210,7 +242,8 @@ def paged_attention_prefill(
                 dev = q.device
                 tile_seq = torch.tensor(ts, dtype=torch.int32, device=dev)
                 tile_qstart = torch.tensor(tq, dtype=torch.int32, device=dev)
-            out = torch.empty_like(q)
+            if out is None:
+                out = torch.empty_like(q)
             _EXT.paged_attention_prefill(
                 out, q, k_cache, v_cache, tile_seq, tile_qstart,
                 query_start_locs, context_lens, block_tables, scale, _stream()
@@ -219,7 +252,7 @@ def paged_attention_prefill(
         if tok_block_tables is not None and tok_context_lens is not None:
             # per-token expansion precomputed once per step by the model runner
             return paged_attention_decode(
-                q, k_cache, v_cache, tok_block_tables, tok_context_lens, scale
+                q, k_cache, v_cache, tok_block_tables, tok_context_lens, scale, out=out
             )
         # v1 native path: run each chunk query row as a "decode" against its
         # causal context prefix (context = L - n + j + 1).  The GROUP waves of
@@ -237,11 +270,12 @@ def paged_attention_prefill(
         ).int()
         bt_per_tok = torch.repeat_interleave(block_tables, n_per, dim=0).contiguous()
         return paged_attention_decode(
-            q, k_cache, v_cache, bt_per_tok, ctx_per_tok, scale
+            q, k_cache, v_cache, bt_per_tok, ctx_per_tok, scale, out=out
         )
-    return torch_ref.paged_attention_prefill(
+    res = torch_ref.paged_attention_prefill(
         q, k_cache, v_cache, block_tables, query_start_locs, context_lens, scale
     )
+    return res if out is None else out.copy_(res)
 
 
 def quant_fp8_rowwise(x: torch.Tensor):

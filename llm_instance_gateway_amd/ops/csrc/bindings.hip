@@ -39,6 +39,10 @@ void lig_rope_launch(const int64_t*, uint16_t*, uint16_t*, const float*, int,
 void lig_reshape_and_cache_launch(const uint16_t*, const uint16_t*, uint16_t*,
                                   uint16_t*, const int64_t*, int, int, int,
                                   int, hipStream_t);
+void lig_qkv_rope_cache_launch(uint16_t*, const uint16_t*, const int64_t*,
+                               const float*, uint16_t*, uint16_t*,
+                               const int64_t*, int, int, int, int, int,
+                               hipStream_t);
 void lig_silu_and_mul_launch(uint16_t*, const uint16_t*, int, int,
                              hipStream_t);
 void lig_paged_attention_decode_launch(
@@ -146,6 +150,32 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v,
                                bf16_ptr(v_cache),
                                slot_mapping.data_ptr<int64_t>(), T, Hkv, D, BS,
                                as_stream(stream));
+}
+
+void qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
+                    torch::Tensor positions, torch::Tensor cos_sin,
+                    torch::Tensor k_cache, torch::Tensor v_cache,
+                    torch::Tensor slot_mapping, int64_t stream) {
+  TORCH_CHECK(positions.scalar_type() == torch::kInt64);
+  TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 && cos_sin.is_contiguous());
+  const int T = qkv.size(0);
+  const int Hkv = k_cache.size(1);
+  const int BS = k_cache.size(2);
+  const int D = k_cache.size(3);
+  const int Hq = q_out.size(1) / D;
+  TORCH_CHECK(D % 64 == 0, "head_dim must be a multiple of 64");
+  TORCH_CHECK(cos_sin.size(1) == D && v_cache.sizes() == k_cache.sizes());
+  TORCH_CHECK(qkv.size(1) == (int64_t)(Hq + 2 * Hkv) * D && q_out.size(0) == T &&
+                  q_out.size(1) == (int64_t)Hq * D,
+              "qkv rows must hold the query, key and value heads");
+  TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
+  if (T == 0) return;
+  lig_qkv_rope_cache_launch(bf16_ptr(q_out), bf16_cptr(qkv),
+                            positions.data_ptr<int64_t>(),
+                            cos_sin.data_ptr<float>(), bf16_ptr(k_cache),
+                            bf16_ptr(v_cache), slot_mapping.data_ptr<int64_t>(),
+                            T, Hq, Hkv, D, BS, as_stream(stream));
 }
 
 void silu_and_mul(torch::Tensor out, torch::Tensor x, int64_t stream) {
@@ -401,6 +431,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rms_norm", &fused_add_rms_norm);
   m.def("rotary_embedding", &rotary_embedding);
   m.def("reshape_and_cache", &reshape_and_cache);
+  m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("paged_attention_decode", &paged_attention_decode);
   m.def("paged_attention_decode_split", &paged_attention_decode_split);
