@@ -12,14 +12,29 @@
 // (first row, token count, context length after the step), and a row's
 // causal bound is its token's position.
 //
-// Per 32-key tile: each 16-byte chunk of a cache row is loaded once and
-// stored twice in LDS, row-major for S^T = K Q^T and transposed for O += P V
-// (mfma_f32_16x16x32_bf16, zero padding to the template's DKP / DVP).
-// Consecutive lanes stage consecutive KEYS of one chunk column, so the
-// transposed 2-byte stores of a wave fall into consecutive LDS words; LDS
-// rows are padded by 16 bytes so that the 16-byte fragment reads of 16
-// different rows spread over all banks.  The loads of the next tile are
-// issued before the current tile's arithmetic (one tile in registers).
+// What bounds it: a decode step reads every cache row once (HBM), a prompt
+// portion does 2 * (D + Dv) flops per (row, key) on matrix cores.  Per tile:
+//   * cache rows go from memory straight into LDS (16 bytes per lane, no
+//     registers), once, XOR-swizzled by key through the choice of what a lane
+//     fetches; the next tile is on its way while this one is used;
+//   * S^T = K Q^T reads keys in the order in which a lane's scores are the
+//     operand of O^T += V^T P^T, so weights stay in registers and a row's
+//     statistics are one scalar per lane;
+//   * V^T comes from the SAME rows through transposing LDS reads
+//     (ds_read_b64_tr_b16).
+// The kernel this replaces staged every row through registers, stored it a
+// second time transposed in 2-byte pieces, sent the weights through LDS, and
+// with one 83 KB workgroup per CU had 36 KB on the way.
+// A wave owns 16 rows. Segments of more than 32 rows: 64 per workgroup, tiles of
+// 32 keys, two workgroups per CU. Others (one token of up to 32 heads): 32 per
+// workgroup, tiles of 64 keys of which waves 0-1 and 2-3 take a half each and
+// merge at the end, one workgroup with 144 KB on the way or in use per CU.
+// Measured with rows of 576 and values of 512, before -> after: 256 single tokens
+// on 700-1024 keys, 32 heads 156 -> 75 us (3.4 TB/s), 16 heads 150 -> 71; 32 such
+// tokens 37 -> 25; 4 prompts of 700-1000, 16 heads 306 -> 118 us (154 -> 399
+// TFLOP/s), 32 heads 540 -> 180. Two row blocks per wave, which halve the LDS
+// reads, lost more by leaving one wave per SIMD (keys of 320: 372 us before, 136
+// now, 208 so; of 128: 149, 73, 135).
 // Scores, running max and sum are fp32; an optional per-head sink starts a
 // row's running max at sink_h and its sum at one; an optional gate multiplies
 // the (token, head) output row by one sigmoid (it commutes with whatever
@@ -28,7 +43,7 @@
 // window > 0 restricts a row at position p to keys j with p - j < window; a
 // tile's walk starts at the oldest key its first token sees.
 //
-// Grid = (ceil(max segment rows / 64), segments, splits); workgroups past a
+// Grid = (ceil(max segment rows / 64 or 32), segments, splits); workgroups past a
 // segment's last row exit at once.  With splits > 1 (few rows, long
 // contexts) each z-slice walks an equal share of the tile's visible keys and
 // leaves its unnormalised sum with its running max and sum in an fp32
@@ -37,36 +52,30 @@
 
 #include "elem_types.h"
 
-typedef __bf16 lr_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float lr_f32x4 __attribute__((ext_vector_type(4)));
+namespace {
 
-#define LR_KVBLK 32
-#define LR_ROWS 64
-#define LR_PAD 8
-#define LR_PART_PAD 4  // a slice row is Dv values, running max, running sum, 2 unused
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-// NCH 16-byte chunks of one cache row (columns sd0, sd0 + 64, ...) into
-// registers; zeros for a key past the visible range (blk < 0) and for
-// columns at or past D.
-template <int NCH>
-LIG_DEVICE void lr_load_chunks(u16x8* stage, const uint16_t* __restrict__ cache, int blk,
-                               int t, int block_size, int D, int sd0) {
-  const uint16_t* rowp =
-      cache + ((size_t)(blk < 0 ? 0 : blk) * block_size + (t % block_size)) * D;
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int d0 = sd0 + j * 64;
-    if (blk >= 0 && d0 < D) {
-      stage[j] = *reinterpret_cast<const u16x8*>(rowp + d0);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) stage[j][e] = 0;
-    }
-  }
+constexpr int LR_PART_PAD = 4;  // a slice row is Dv values, running max (log2 units), running sum, 2 unused
+constexpr float LR_LOG2E = 1.44269504088896340736f;
+
+LIG_DEVICE float lr_group_max(float x) {  // max over the four 16-lane groups
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t v = __builtin_bit_cast(uint32_t, y);
+  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
 }
 
-template <int DKP, int DVP>
-__global__ __launch_bounds__(256) void latent_attention_rows_kernel(
+// KG key groups of 32 keys per tile, 4 / KG waves of 16 rows for each.
+// FULL: D == DKP, Dv == DVP and the block size is a power of two, at least 8
+template <int DKP, int DVP, int KG, bool FULL>
+__global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_kernel(
     uint16_t* __restrict__ out,          // [R, H * Dv]
     const uint16_t* __restrict__ q,      // [R, H * D] contiguous
     const uint16_t* __restrict__ cache,  // [blocks, 1, BS, D]
@@ -75,256 +84,327 @@ __global__ __launch_bounds__(256) void latent_attention_rows_kernel(
     const int* __restrict__ seg_start, const int* __restrict__ seg_len,
     const int* __restrict__ seg_ctx,     // tokens of the sequence after this step
     const int* __restrict__ block_tables, int max_blocks, float scale, int H,
-    int D, int Dv, int block_size, int window, int nsplit,
+    int D_, int Dv_, int block_size, int block_shift, int window, int nsplit,
     float* __restrict__ partial) {  // [R * H, nsplit, Dv + 4] when nsplit > 1
-  static_assert(DVP <= DKP, "values are a prefix of the key row");
+  const int D = FULL ? DKP : D_, Dv = FULL ? DVP : Dv_;
+  static_assert(DVP <= DKP && DKP % 64 == 0 && DVP % 16 == 0, "values are a prefix of the key row");
   constexpr int DB = DVP / 16;
   constexpr int KB = DKP / 32;
-
-  struct Shared {
-    uint16_t K[LR_KVBLK][DKP + LR_PAD];
-    uint16_t VT[DVP][LR_KVBLK + LR_PAD];
-    uint16_t P[4][16][LR_KVBLK + LR_PAD];
-  };
-  __shared__ Shared sm;
+  constexpr int CHP = DKP / 8;              // 16-byte chunks of an LDS row, a multiple of 8
+  constexpr int KT = 32 * KG;               // keys per tile
+  constexpr int NI = KT * CHP / 256;        // fetches per wave and tile
+  constexpr int ROWS = 64 / KG;
+  constexpr int TILE = KT * DKP;
+  constexpr int MERGE = KG > 1 ? 2 * 16 * (DVP + 4) * 2 : 0;  // fp32 rows of two waves, in 16-bit units
+  constexpr int LDS = 2 * TILE > MERGE ? 2 * TILE : MERGE;
+  __shared__ __align__(16) uint16_t sm[LDS];
 
   const int s = blockIdx.y;
   const int n = seg_len[s];
   const long nrows = (long)n * H;
-  const long rho0 = (long)blockIdx.x * LR_ROWS;
+  const long rho0 = (long)(gridDim.x - 1 - blockIdx.x) * ROWS;  // the longest walks first
   if (rho0 >= nrows) return;
   const long lo = seg_start[s];
   const int ctx = seg_ctx[s];
   const int* bt = block_tables + (size_t)s * max_blocks;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int li = lane & 15;
   const int lg = lane >> 4;
+  const int rblk = wave % (4 / KG);
+  const int kg = wave / (4 / KG);
 
-  const long rho = rho0 + wave * 16 + li;
-  const bool row_valid = rho < nrows;
-  // a wave whose 16 rows all lie past the segment only helps staging
-  const bool wave_active = rho0 + wave * 16 < nrows;
-  const int tok = (int)((row_valid ? rho : rho0) / H);
-  const int head = (int)((row_valid ? rho : rho0) - (long)tok * H);
+  // a wave whose rows all lie past the segment only helps fetching
+  const bool wave_active = rho0 + rblk * 16 < nrows;
+  const long rho = rho0 + rblk * 16 + li;
+  const long rr = rho < nrows ? rho : rho0;
+  const int tok = (int)(rr / H);
+  const int head = (int)(rr - (long)tok * H);
   const int qpos = ctx - n + tok;
 
-  lr_bf16x8 q_frag[KB];
+  const int z = blockIdx.z;
+  const long last_rho = (rho0 + ROWS < nrows ? rho0 + ROWS : nrows) - 1;
+  const int first_tok = (int)(rho0 / H);
+  const int kv_end = ctx - n + (int)(last_rho / H) + 1;  // keys any row of the tile sees
+  // oldest key any row of the tile sees, at the start of a piece of 8
+  const int kv_first = window > 0 ? max(0, ctx - n + first_tok - window + 1) & ~7 : 0;
+  int kv_lo = kv_first, kv_hi = kv_end;
+  if (nsplit > 1) {
+    const int nt = (kv_end - kv_first + KT - 1) / KT;
+    const int per = (nt + nsplit - 1) / nsplit;
+    kv_lo = kv_first + z * per * KT;  // past the end: an empty slice
+    kv_hi = min(kv_end, kv_lo + per * KT);
+  }
+  // bounds that hold for every row of the tile: no mask between them
+  const int all_end = ctx - n + first_tok + 1;
+  const int all_lo = window > 0 ? kv_end - window : 0;
+
+  // ---- fetching: chunk c of key t of a tile goes to LDS chunk t * CHP + (c ^ f(t)).
+  // Keys past the end repeat the last one.
+  // FULL: 8 keys, aligned, are one contiguous piece of a block; a wave takes
+  // KT / 32 such pieces of CHP / 8 fetches.  Lane j looks up the block of piece j
+  // of the tile after next.  Else every lane looks for its own key's block.
+  const int CH = D / 8;
+  constexpr int NP = CHP / 8;  // fetches per piece
+  auto block_of = [&](int kv0) {
+    const int t = min(kv0 + (FULL ? (lane & 7) * 8 : lane & (KT - 1)), kv_end - 1);
+    return bt[FULL ? t >> block_shift : t / block_size];
+  };
+  auto fetch = [&](int kv0, int blks, int buf) {
+    int here = lane;
+    if (KG == 1) asm volatile("" : "+v"(here));  // worked out anew for each tile: held for the loop, it would spill
+    if constexpr (FULL) {
+#pragma unroll
+      for (int w = 0; w < KG; ++w) {
+        const int piece = wave * KG + w;
+        const int t0 = min(kv0 + piece * 8, (kv_end - 1) & ~7);
+        const int blk = __builtin_amdgcn_readlane(blks, piece);
+        const uint16_t* g = cache + ((size_t)blk * block_size + (t0 & (block_size - 1))) * D;
+        const int last = kv_end - 1 - t0;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          const int p = i * 64 + here;
+          const int key = p / CHP;  // of the piece
+          const int c = (p % CHP) ^ ((key & 3) | ((piece & 1) << 2));
+          __builtin_amdgcn_global_load_lds(
+              (const __attribute__((address_space(1))) void*)(g + (min(key, last) * DKP + c * 8)),
+              (__attribute__((address_space(3))) void*)(sm + buf * TILE + (piece * NP + i) * 512), 16, 0, 0);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int base = (wave * NI + i) * 64;
+        const int p = base + here;
+        const int key = p / CHP;
+        const int c = (p % CHP) ^ ((key & 3) | ((key >> 1) & 4));
+        const int off = min(kv0 + key, kv_end - 1) % block_size;
+        const int blk = __shfl(blks, key, 64);
+        if (c < CH)
+          __builtin_amdgcn_global_load_lds(
+              (const __attribute__((address_space(1))) void*)(cache + ((size_t)blk * block_size + off) * D + c * 8),
+              (__attribute__((address_space(3))) void*)(sm + buf * TILE + base * 8), 16, 0, 0);
+      }
+    }
+  };
+
+  if (!FULL && CH < CHP) {  // the chunks past a row's end are never fetched
+    for (int i = tid; i < LDS / 8; i += 256) reinterpret_cast<u32x4*>(sm)[i] = u32x4{0, 0, 0, 0};
+    __syncthreads();
+  }
+  int blks = kv_lo < kv_hi ? block_of(kv_lo) : 0;
+  if (kv_lo < kv_hi) {
+    fetch(kv_lo, blks, 0);
+    blks = block_of(kv_lo + KT);
+  }
+
+  // a negative scale goes into the sign of the query
+  const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
+  const float c2 = fabsf(scale) * LR_LOG2E;
+  bf16x8_t q_frag[KB];
   {
-    const uint16_t* qp = q + ((size_t)lo * H + (row_valid ? rho : rho0)) * D;
+    const uint16_t* qp = q + ((size_t)lo * H + rr) * D;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const int d0 = kb * 32 + lg * 8;
-      u16x8 raw;
-      if (d0 < D) {
-        raw = *reinterpret_cast<const u16x8*>(qp + d0);
-      } else {
+      u32x4 raw = u32x4{0, 0, 0, 0};
+      if (FULL || d0 < D) raw = *reinterpret_cast<const u32x4*>(qp + d0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) raw[e] = 0;
-      }
-      q_frag[kb] = *reinterpret_cast<lr_bf16x8*>(&raw);
+      for (int e = 0; e < 4; ++e) raw[e] ^= flip;
+      q_frag[kb] = __builtin_bit_cast(bf16x8_t, raw);
     }
   }
 
-  const int z = blockIdx.z;
-  const bool with_sink = sink != nullptr && z == 0;
-  float m = with_sink ? sink[head] : -INFINITY;
-  float l = with_sink ? 1.0f : 0.0f;
-  lr_f32x4 acc_o[DB];
+  const bool with_sink = sink != nullptr && z == 0 && kg == 0;
+  float m = with_sink ? sink[head] * LR_LOG2E : -INFINITY;
+  float l = with_sink && lg == 0 ? 1.0f : 0.0f;  // this lane's part of the sum
+  f32x4_t acc[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) acc_o[db] = lr_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const long last_rho = (rho0 + LR_ROWS < nrows ? rho0 + LR_ROWS : nrows) - 1;
-  const int kv_end = ctx - n + (int)(last_rho / H) + 1;  // keys any row of the tile sees
-
-  // oldest key any row of the tile sees, and the one this lane's row sees
-  const int kv_first = window > 0 ? max(0, ctx - n + (int)(rho0 / H) - window + 1) : 0;
-  const int key_lo = window > 0 ? qpos - window + 1 : 0;
-  int kv_lo = kv_first, kv_hi = kv_end;
-  if (nsplit > 1) {
-    const int nt = (kv_end - kv_first + LR_KVBLK - 1) / LR_KVBLK;
-    const int per = (nt + nsplit - 1) / nsplit;
-    kv_lo = min(kv_end, kv_first + z * per * LR_KVBLK);
-    kv_hi = min(kv_end, kv_lo + per * LR_KVBLK);
-  }
-
-  // Staging is software-pipelined: a thread always stages the same key row of
-  // a tile (256 threads = 8 chunk columns x 32 keys, NCH column groups), so it
-  // needs ONE block-table entry per tile.  The chunks of tile i+1 are loaded
-  // into registers, and the table entry of tile i+2 is fetched, while tile i
-  // is being multiplied; they are written to LDS at the top of the next turn.
-  constexpr int NCH = DKP / 64;
-  const int srow = tid % LR_KVBLK;
-  const int sd0 = (tid / LR_KVBLK) * 8;
-  u16x8 stage[NCH];
-  int blk_next;
-  {
-    const int t = kv_lo + srow;
-    const int blk = (kv_lo < kv_hi && t < kv_end) ? bt[t / block_size] : -1;
-    lr_load_chunks<NCH>(stage, cache, blk, t, block_size, D, sd0);
-    const int t2 = t + LR_KVBLK;
-    blk_next = (kv_lo + LR_KVBLK < kv_hi && t2 < kv_end) ? bt[t2 / block_size] : -1;
-  }
-
-  for (int kv0 = kv_lo; kv0 < kv_hi; kv0 += LR_KVBLK) {
-    // ---- registers -> LDS: row-major for S^T = K Q^T, transposed for O += P V ----
-#pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const int d0 = sd0 + j * 64;
-      const u16x8 kval = stage[j];
-      *reinterpret_cast<u16x8*>(&sm.K[srow][d0]) = kval;
-      if (d0 < DVP) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sm.VT[d0 + e][srow] = (d0 + e < Dv) ? kval[e] : (uint16_t)0;
-      }
+  int buf = 0;
+  for (int kv0 = kv_lo; kv0 < kv_hi; kv0 += KT, buf ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tile is in LDS
+    __syncthreads();                     // everybody's is, and the other buffer is free
+    if (kv0 + KT < kv_hi) {
+      fetch(kv0 + KT, blks, buf ^ 1);
+      blks = block_of(kv0 + 2 * KT);
     }
-    __syncthreads();
-    {  // prefetch the next tile (loads stay in flight through the arithmetic below)
-      const int kvn = kv0 + LR_KVBLK;
-      if (kvn < kv_hi) {
-        const int t = kvn + srow;
-        lr_load_chunks<NCH>(stage, cache, blk_next, t, block_size, D, sd0);
-        const int t2 = t + LR_KVBLK;
-        blk_next = (kvn + LR_KVBLK < kv_hi && t2 < kv_end) ? bt[t2 / block_size] : -1;
+    const int k0 = kv0 + kg * 32;  // this wave's keys
+    if (!wave_active || k0 >= kv_hi) continue;
+    const uint16_t* tile = sm + buf * TILE + kg * 32 * DKP;
+
+    // Operands are read from LDS in batches of 4, the next batch ahead of the
+    // products of this one.
+    // S^T = K Q^T: tile row li stands for key (li/4)*8 + li%4 (+4 in the second).
+    // The swizzle only touches a chunk number's low 3 bits, so two addresses and
+    // constants reach all of a row
+    f32x4_t s4[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+    {
+      const int key = ((li >> 2) << 3) | (li & 3);
+      const int f = (key & 3) | ((key >> 1) & 4);  // the same for key + 4
+      const uint16_t* kp[2] = {tile + key * DKP + (lg ^ f) * 8, tile + key * DKP + ((4 + lg) ^ f) * 8};
+      bf16x8_t kf[2][4];
+      auto load = [&](int b) {  // steps 2b and 2b+1 of both tiles
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          kf[b & 1][j] = __builtin_bit_cast(
+              bf16x8_t, *reinterpret_cast<const u32x4*>(kp[j >> 1] + (j & 1) * 4 * DKP + b * 64));
+      };
+      load(0);
+#pragma unroll
+      for (int b = 0; b < KB / 2; ++b) {
+        if (b + 1 < KB / 2) load(b + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s4[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[b & 1][j], q_frag[b * 2 + (j >> 1)], s4[j & 1], 0, 0, 0);
       }
     }
 
-    if (wave_active) {
-    // ---- S^T = K Q^T ----------------------------------------------------------
-    lr_f32x4 acc_s[2];
+    // V^T: lane li of a 16-lane group reads 4 entries of key li/4 and receives
+    // entry li of keys 0..3
+    const int vkey = lg * 8 + (li >> 2);
+    const int vf_swz = (vkey & 3) | ((vkey >> 1) & 4);  // the same for key + 4
+    const uint16_t* vp[4];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      acc_s[kt] = lr_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 4; ++j) vp[j] = tile + vkey * DKP + ((j * 2 + ((li >> 1) & 1)) ^ vf_swz) * 8 + (li & 1) * 4;
+    bf16x8_t vf[2][4];
+    auto load_v = [&](int b) {  // entry blocks 4b .. 4b+3
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        u16x8 raw =
-            *reinterpret_cast<const u16x8*>(&sm.K[kt * 16 + li][kb * 32 + lg * 8]);
-        lr_bf16x8 a_frag = *reinterpret_cast<lr_bf16x8*>(&raw);
-        acc_s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            a_frag, q_frag[kb], acc_s[kt], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        const uint16_t* v0 = vp[j] + b * 64;
+        const u32x2 b0 = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)v0));
+        const u32x2 b1 = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + 4 * DKP)));
+        vf[b & 1][j] = __builtin_bit_cast(bf16x8_t, (u32x4{b0[0], b0[1], b1[0], b1[1]}));
       }
-    }
+    };
+    load_v(0);
 
-    // ---- mask + online softmax (this lane owns row rho) -------------------------
-    float sc[8];
-    float rowmax = -INFINITY;
+    // ---- weights of keys k0 + lg*8 + e -----------------------------------------
+    const bool masked = k0 + 32 > min(all_end, kv_hi) || k0 < all_lo;
+    uint32_t dead = 0;
+    if (masked) {
+      const int key_lo = window > 0 ? qpos - window + 1 : 0;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = kv0 + kt * 16 + lg * 4 + r;
-        float v = acc_s[kt][r] * scale;
-        if (!row_valid || key > qpos || key < key_lo) v = -INFINITY;
-        sc[kt * 4 + r] = v;
-        rowmax = fmaxf(rowmax, v);
+      for (int e = 0; e < 8; ++e) {
+        const int key = k0 + lg * 8 + e;
+        if (key > qpos || key < key_lo || key >= kv_hi) {
+          dead |= 1u << e;
+          s4[e >> 2][e & 3] = -INFINITY;
+        }
       }
     }
-    rowmax = stride_reduce_max<16, 4>(rowmax);
-    const float m_new = fmaxf(m, rowmax);
-    float alpha;
-    float psum = 0.0f;
-    float p[8];
-    if (m_new == -INFINITY) {
-      alpha = 1.0f;
+    float mx = s4[0][0];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = 0.0f;
-    } else {
-      alpha = (m == -INFINITY) ? 0.0f : __expf(m - m_new);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        p[i] = (sc[i] == -INFINITY) ? 0.0f : __expf(sc[i] - m_new);
-        psum += p[i];
-      }
+    for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s4[e >> 2][e & 3]);
+    mx = lr_group_max(mx);
+    mx = mx == -INFINITY ? mx : mx * c2;
+    if (__any(mx > m)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
       m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[db][i] *= alpha;
     }
-    psum = stride_reduce_sum<16, 4>(psum);
-    l = l * alpha + psum;
-    // acc_o rows follow the MFMA C layout (row = lg*4 + r); the softmax stats
-    // of row x live in lane x (replicated over the lg groups)
-    float alpha_r[4];
+    const float mm = m == -INFINITY ? 0.f : m;
+    float p[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) alpha_r[r] = __shfl(alpha, lg * 4 + r, 64);
+    for (int e = 0; e < 8; ++e)
+      p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[e >> 2][e & 3], c2, -mm));
+    if (masked) {
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc_o[db][r] *= alpha_r[r];
+      for (int e = 0; e < 8; ++e) p[e] = (dead >> e) & 1 ? 0.f : p[e];
     }
+    u32x4 pw;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      l += p[2 * e] + p[2 * e + 1];
+      pw[e] = (uint32_t)f32_to_bf16(p[2 * e]) | ((uint32_t)f32_to_bf16(p[2 * e + 1]) << 16);
+    }
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pw);
 
-    // ---- P: C layout -> A-fragment layout through the wave's LDS slab ---------
+    // ---- O^T += V^T P^T -----------------------------------------------------------
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int b = 0; b < DB / 4; ++b) {
+      if (b + 1 < DB / 4) load_v(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sm.P[wave][li][kt * 16 + lg * 4 + r] = f32_to_bf16(p[kt * 4 + r]);
+      for (int j = 0; j < 4; ++j)
+        acc[b * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[b & 1][j], pf, acc[b * 4 + j], 0, 0, 0);
+    }
+  }
+
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  // ---- the second key group hands its sums to the first ---------------------------
+  if constexpr (KG > 1) {
+    __syncthreads();
+    float* fs = reinterpret_cast<float*>(sm) + (rblk * 16 + li) * (DVP + 4);
+    if (kg == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4_t*>(fs + db * 16 + lg * 4) = acc[db];
+      if (lg == 0) {
+        fs[DVP] = m;
+        fs[DVP + 1] = l;
       }
     }
-    u16x8 praw = *reinterpret_cast<const u16x8*>(&sm.P[wave][li][lg * 8]);
-    lr_bf16x8 p_frag = *reinterpret_cast<lr_bf16x8*>(&praw);
-
-    // ---- O += P V -----------------------------------------------------------------
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = fs[DVP], l1 = fs[DVP + 1];
+    const float gm = fmaxf(m, m1);
+    const float w0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - gm);
+    const float w1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - gm);
+    m = gm;
+    l = l * w0 + l1 * w1;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      u16x8 vraw =
-          *reinterpret_cast<const u16x8*>(&sm.VT[db * 16 + li][lg * 8]);
-      lr_bf16x8 v_frag = *reinterpret_cast<lr_bf16x8*>(&vraw);
-      acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p_frag, v_frag,
-                                                          acc_o[db], 0, 0, 0);
+      const f32x4_t o1 = *reinterpret_cast<const f32x4_t*>(fs + db * 16 + lg * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[db][i] = acc[db][i] * w0 + o1[i] * w1;
     }
-    }  // wave_active
-    __syncthreads();
   }
+  if (rho >= nrows) return;
 
   if (nsplit > 1) {
     // ---- partial result: unnormalised sums, running max and sum -------------------
-    const size_t stride = (size_t)Dv + LR_PART_PAD;
-    if (row_valid && lg == 0) {
-      float* pp = partial + (((size_t)lo * H + rho) * nsplit + z) * stride;
+    float* pp = partial + (((size_t)lo * H + rho) * nsplit + z) * ((size_t)Dv + LR_PART_PAD);
+    if (lg == 0) {
       pp[Dv] = m;
       pp[Dv + 1] = l;
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const long orho = rho0 + wave * 16 + lg * 4 + r;
-      if (orho >= nrows) continue;
-      float* pp = partial + (((size_t)lo * H + orho) * nsplit + z) * stride;
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const int d = db * 16 + li;
-        if (d < Dv) pp[d] = acc_o[db][r];
-      }
+    for (int db = 0; db < DB; ++db) {
+      const int d = db * 16 + lg * 4;
+      if (FULL || d < Dv) *reinterpret_cast<f32x4_t*>(pp + d) = acc[db];
     }
     return;
   }
 
-  // ---- epilogue: normalise and store ------------------------------------------------
-  float inv_l[4];
+  // ---- normalise, gate, store --------------------------------------------------------
+  float f = l > 0.f ? 1.0f / l : (l == 0.f ? 0.f : l);
+  if (gate != nullptr) f *= sigmoid_fast(bf16_to_f32(gate[(lo + tok) * gate_stride + head]));
+  uint16_t* op = out + ((size_t)lo * H + rho) * Dv;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float lr = __shfl(l, lg * 4 + r, 64);  // all lanes active here
-    inv_l[r] = lr > 0.f ? 1.0f / lr : 0.0f;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const long orho = rho0 + wave * 16 + lg * 4 + r;
-    if (orho >= nrows) continue;
-    uint16_t* op = out + ((size_t)lo * H + orho) * Dv;
-    if (gate != nullptr) {
-      const long ot = orho / H;
-      inv_l[r] *= sigmoid_fast(bf16_to_f32(gate[(lo + ot) * gate_stride + (orho - ot * H)]));
-    }
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const int d = db * 16 + li;
-      if (d < Dv) op[d] = f32_to_bf16(acc_o[db][r] * inv_l[r]);
-    }
+  for (int db = 0; db < DB; ++db) {
+    const int d = db * 16 + lg * 4;
+    if (!FULL && d >= Dv) continue;
+    u32x2 w;
+    w[0] = (uint32_t)f32_to_bf16(acc[db][0] * f) | ((uint32_t)f32_to_bf16(acc[db][1] * f) << 16);
+    w[1] = (uint32_t)f32_to_bf16(acc[db][2] * f) | ((uint32_t)f32_to_bf16(acc[db][3] * f) << 16);
+    *reinterpret_cast<u32x2*>(op + d) = w;
   }
 }
 
-
-// Merge the z-slices of every row: m* = max m_z, out = sum_z e^(m_z - m*) acc_z
-// / sum_z e^(m_z - m*) l_z.  One wave per row.  Lane z holds slice z's weight
+// Merge the z-slices of every row: m* = max m_z, out = sum_z 2^(m_z - m*) acc_z
+// / sum_z 2^(m_z - m*) l_z.  One wave per row.  Lane z holds slice z's weight
 // (up to 64 slices); the lanes then own float4 columns of the value row and
 // add up the slices with independent 16-byte loads (slice rows are padded
 // to Dv + 4 floats so that they stay 16-byte aligned).
@@ -346,7 +426,7 @@ __global__ __launch_bounds__(256) void latent_attention_rows_combine_kernel(
     lz = pp[lane * stride + Dv + 1];
   }
   const float mstar = wave_reduce_max(mz);
-  const float wz = (mz == -INFINITY) ? 0.f : __expf(mz - mstar);
+  const float wz = (mz == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mz - mstar);
   const float lsum = wave_reduce_sum(wz * lz);
   float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
   if (gate != nullptr) {
@@ -388,6 +468,8 @@ __global__ __launch_bounds__(256) void latent_attention_rows_combine_kernel(
   }
 }
 
+}  // namespace
+
 // Returns 0 when launched, 1 when the shape is not served (the caller then
 // uses another kernel).
 extern "C" int lig_latent_attention_rows(
@@ -401,18 +483,33 @@ extern "C" int lig_latent_attention_rows(
       Dv > 512 || !aligned16(q) || !aligned16(cache) || H <= 0)
     return 1;
   if (num_segs <= 0 || max_seg_len <= 0) return 0;
-  const long tiles = ((long)max_seg_len * H + LR_ROWS - 1) / LR_ROWS;
+  // one token of up to 32 heads: all four waves on 32 rows
+  const bool few = (long)max_seg_len * H <= 32;
+  const int rows = few ? 32 : 64;
+  const long tiles = ((long)max_seg_len * H + rows - 1) / rows;
+  const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
   if (tiles > 2147483647L || num_segs > 65535) return 1;
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && partial == nullptr)) return 1;
   dim3 grid((unsigned)tiles, num_segs, nsplit);
   dim3 block(256);
-#define LAUNCH_LR(DKP, DVP)                                                    \
-  hipLaunchKernelGGL((latent_attention_rows_kernel<DKP, DVP>), grid, block, 0, \
-                     stream, (uint16_t*)out, (const uint16_t*)q,               \
-                     (const uint16_t*)cache, sink,                             \
-                     (const uint16_t*)gate, gate_stride, seg_start, seg_len,         \
-                     seg_ctx, block_tables, max_blocks, scale, H, D, Dv,       \
-                     block_size, window, nsplit, partial)
+#define LAUNCH_LR_KG(DKP, DVP, KG, FULL)                                                      \
+  hipLaunchKernelGGL((latent_attention_rows_kernel<DKP, DVP, KG, FULL>), grid, block, 0,      \
+                     stream, (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)cache, sink, \
+                     (const uint16_t*)gate, gate_stride, seg_start, seg_len, seg_ctx,         \
+                     block_tables, max_blocks, scale, H, D, Dv, block_size, shift, window,    \
+                     nsplit, partial)
+#define LAUNCH_LR(DKP, DVP)                                \
+  do {                                                     \
+    const bool full = D == DKP && Dv == DVP && shift >= 3; \
+    if (few && full)                                       \
+      LAUNCH_LR_KG(DKP, DVP, 2, true);                     \
+    else if (few)                                          \
+      LAUNCH_LR_KG(DKP, DVP, 2, false);                    \
+    else if (full)                                         \
+      LAUNCH_LR_KG(DKP, DVP, 1, true);                     \
+    else                                                   \
+      LAUNCH_LR_KG(DKP, DVP, 1, false);                    \
+  } while (0)
   if (D <= 64 && Dv <= 64) LAUNCH_LR(64, 64);
   else if (D <= 128 && Dv <= 64) LAUNCH_LR(128, 64);
   else if (D <= 128) LAUNCH_LR(128, 128);
@@ -420,6 +517,7 @@ extern "C" int lig_latent_attention_rows(
   else if (D <= 320 && Dv <= 256) LAUNCH_LR(320, 256);
   else LAUNCH_LR(576, 512);
 #undef LAUNCH_LR
+#undef LAUNCH_LR_KG
   if (nsplit > 1) {
     const long rows4 = ((long)max_seg_len * H + 3) / 4;
     hipLaunchKernelGGL(latent_attention_rows_combine_kernel,
