@@ -107,6 +107,7 @@ class DecodeGraphRunner:
         self.logits: Dict[int, torch.Tensor] = {}
         self._pool = None
         self.with_lora = False
+        self.lora_in_layer = False
 
     def _graph_nsplits(self, B: int) -> int:
         """Bucket-static flash-decode split factor: replay can't branch on
@@ -155,8 +156,26 @@ class DecodeGraphRunner:
             lora_unit_len=self.lora_ulen[:B] if self.with_lora else None,
             lora_unit_slot=self.lora_uslot[:B] if self.with_lora else None,
             lora_ws=self.lora_ws,
+            **self._lora_rows(B),
             decode_nsplits=self._graph_nsplits(B),
         )
+
+    def _lora_rows(self, B: int) -> dict:
+        """The bucket's row tiles where the model carries LoRA in its layers:
+        as many as B tokens can need, the unused ones empty."""
+        if not (self.with_lora and self.lora_in_layer):
+            return {}
+        n = self._max_rows(B)
+        return dict(
+            lora_rows_tok=self.lora_tok[: n * 16].view(n, 16),
+            lora_rows_len=self.lora_ulen[:n],
+            lora_rows_slot=self.lora_uslot[:n],
+        )
+
+    def _max_rows(self, B: int) -> int:
+        from ..lora.manager import max_lora_rows
+
+        return max_lora_rows(B, self.runner.adapter_manager.max_slots)
 
     def _forward(self, B: int) -> torch.Tensor:
         model = self.runner.model
@@ -166,8 +185,15 @@ class DecodeGraphRunner:
 
     def capture(self, with_lora: bool) -> None:
         self.with_lora = with_lora
+        mgr = self.runner.adapter_manager
+        self.lora_in_layer = with_lora and getattr(mgr, "in_layer", False)
+        if self.lora_in_layer:
+            n = self._max_rows(self.max_bs) * 16
+            self.lora_tok = torch.zeros(n, dtype=torch.int32, device=self.device)
+            self.h_tok = torch.zeros(n, dtype=torch.int32, pin_memory=True)
+            self.n_tok = self.h_tok.numpy()
+            self.lora_ulen.zero_()  # the tiles of a capture list nothing
         if with_lora and self.lora_ws is None:
-            mgr = self.runner.adapter_manager
             self.lora_ws = torch.zeros(
                 self.max_bs, mgr.rank, dtype=mgr.dtype, device=self.device
             )
@@ -283,20 +309,26 @@ class DecodeGraphRunner:
         self.block_tables[:B].copy_(self.h_bt[:B], non_blocking=True)
         self.context_lens[:B].copy_(self.h_ctx[:B], non_blocking=True)
         if self.with_lora:
-            from ..lora.manager import build_lora_units
+            from ..lora.manager import build_lora_rows, build_lora_units
 
-            order, ut0, ulen, uslot = build_lora_units(self.n_lora[:B])
-            u = len(ut0)
-            self.n_order[:B] = order
-            self.n_ut0[:u] = ut0
+            if self.lora_in_layer:
+                toks, ulen, uslot = build_lora_rows(self.n_lora[:B])
+                u, room = len(ulen), self._max_rows(B)
+                self.n_tok[: u * 16] = toks.reshape(-1)
+                self.lora_tok[: room * 16].copy_(self.h_tok[: room * 16], non_blocking=True)
+            else:
+                order, ut0, ulen, uslot = build_lora_units(self.n_lora[:B])
+                u, room = len(ut0), B
+                self.n_order[:B] = order
+                self.n_ut0[:u] = ut0
+                self.lora_slots[:B].copy_(self.h_lora[:B], non_blocking=True)
+                self.lora_order[:B].copy_(self.h_order[:B], non_blocking=True)
+                self.lora_ut0[:B].copy_(self.h_ut0[:B], non_blocking=True)
             self.n_ulen[:u] = ulen
-            self.n_ulen[u:B] = 0  # padding units: no-op in the kernels
+            self.n_ulen[u:room] = 0  # padding tiles or units: no-op in the kernels
             self.n_uslot[:u] = uslot
-            self.n_uslot[u:B] = -1
-            self.lora_slots[:B].copy_(self.h_lora[:B], non_blocking=True)
-            self.lora_order[:B].copy_(self.h_order[:B], non_blocking=True)
-            self.lora_ut0[:B].copy_(self.h_ut0[:B], non_blocking=True)
-            self.lora_ulen[:B].copy_(self.h_ulen[:B], non_blocking=True)
-            self.lora_uslot[:B].copy_(self.h_uslot[:B], non_blocking=True)
+            self.n_uslot[u:room] = -1
+            self.lora_ulen[:room].copy_(self.h_ulen[:room], non_blocking=True)
+            self.lora_uslot[:room].copy_(self.h_uslot[:room], non_blocking=True)
         self.graphs[B].replay()
         return self.logits[B][:n]

@@ -61,6 +61,11 @@ class BatchMeta:
     lora_unit_t0: Optional[torch.Tensor] = None    # [U] int32 (into order)
     lora_unit_len: Optional[torch.Tensor] = None   # [U] int32
     lora_unit_slot: Optional[torch.Tensor] = None  # [U] int32
+    # Row tiles of the kernels that carry LoRA inside a layer: up to 16 tokens
+    # of one adapter (-1: none), together every row of the batch.
+    lora_rows_tok: Optional[torch.Tensor] = None   # [N, 16] int32
+    lora_rows_len: Optional[torch.Tensor] = None   # [N] int32
+    lora_rows_slot: Optional[torch.Tensor] = None  # [N] int32
     # Private LoRA shrink workspace for this batch (the decode graph owns its
     # own so graph replay and a concurrent eager prefill never share u).
     lora_ws: Optional[torch.Tensor] = None

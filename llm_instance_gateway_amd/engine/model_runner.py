@@ -334,7 +334,15 @@ class ModelRunner:
             meta.lora_slot_per_token = torch.tensor(slots, dtype=torch.int32).to(
                 dev, non_blocking=True
             )
-            if self.device.type == "cuda":
+            if getattr(mgr, "in_layer", False):
+                # row tiles over the whole batch (lora/manager.py::build_lora_rows)
+                from ..lora.manager import build_lora_rows
+
+                arrays = build_lora_rows(slots)
+                meta.lora_rows_tok, meta.lora_rows_len, meta.lora_rows_slot = (
+                    torch.from_numpy(a).to(dev, non_blocking=True) for a in arrays
+                )
+            elif self.device.type == "cuda":
                 # slot-grouped SGMV units (lora/manager.py::build_lora_units)
                 from ..lora.manager import build_lora_units
 

@@ -76,6 +76,34 @@ def build_lora_units(slots_np, cap: int = 32):
     )
 
 
+def build_lora_rows(slots_np, cap: int = 16):
+    """Tiles of the kernels that carry LoRA inside a layer: like
+    `build_lora_units`, but listing EVERY token (slot -1 too), since those
+    kernels do the layer's own work on the rows as well.
+
+    Returns int32 numpy arrays (tokens[N, cap], the places past len
+    repeating a token of the tile; len[N]; slot[N])."""
+    import numpy as np
+
+    arr = np.asarray(slots_np, dtype=np.int32)
+    order = np.argsort(arr, kind="stable").astype(np.int32)
+    runs = arr[order]
+    first = np.flatnonzero(np.r_[True, runs[1:] != runs[:-1]]) if len(runs) else np.zeros(0, dtype=np.int64)
+    size = np.diff(np.r_[first, len(runs)])
+    tiles = (size + cap - 1) // cap
+    run = np.repeat(np.arange(len(first)), tiles)
+    within = (np.arange(len(run)) - np.repeat(np.cumsum(tiles) - tiles, tiles)) * cap
+    t0 = first[run] + within
+    length = np.minimum(cap, size[run] - within)
+    at = t0[:, None] + np.minimum(np.arange(cap)[None], length[:, None] - 1)
+    return order[at].reshape(len(t0), cap), length.astype(np.int32), runs[t0].astype(np.int32)
+
+
+def max_lora_rows(num_tokens: int, max_slots: int, cap: int = 16) -> int:
+    """Most tiles `build_lora_rows` can make of that many tokens."""
+    return min(num_tokens, num_tokens // cap + min(num_tokens, max_slots + 1))
+
+
 # module name -> (in_features, out_features) resolver
 def _module_dims(mc, tp_size: int) -> Dict[str, Tuple[int, int]]:
     h = mc.hidden_size
@@ -158,6 +186,19 @@ class AdapterManager:
             torch.cuda.Stream(device=self.device)
             if self.device.type == "cuda"
             else None
+        )
+        # whether the model runs LoRA inside its own kernels (the runner then
+        # lists row tiles instead of SGMV units); not where deltas must be
+        # summed over ranks before they are used
+        self.in_layer = bool(
+            self.device.type == "cuda"
+            and (runner.tp is None or runner.tp.world_size == 1)
+            and self.dtype == torch.bfloat16
+            and _UNITS_SGMV
+            and not _TILED_SGMV
+            and os.environ.get("LIG_FORCE_TORCH_OPS") != "1"
+            and hasattr(runner.model, "lora_in_layer")
+            and runner.model.lora_in_layer(rank, self.dims)
         )
         # attach to the model's layers
         self._attach(runner.model)

@@ -74,6 +74,17 @@ class Attention(nn.Module):
         q = ops.qkv_rope_cache(
             qkv, positions, cos_sin_cache, k_cache, v_cache, meta.slot_mapping, self.num_heads
         )
+        attn_flat = self.attend(q, kv_cache, meta)
+        o = self.o_proj(attn_flat)
+        if self._lora is not None:
+            self._lora.apply(self._layer_idx, "o", attn_flat, o, meta)
+        if self.tp is not None:
+            o = self.tp.all_reduce(o)
+        return o
+
+    def attend(self, q: torch.Tensor, kv_cache, meta: BatchMeta) -> torch.Tensor:
+        """Attention of the rotated queries [T, heads * D] over the paged cache."""
+        k_cache, v_cache = kv_cache
         qh = q.view(-1, self.num_heads, self.head_dim)
         np_, nd = meta.num_prefill_tokens, meta.num_decode_tokens
         out = torch.empty_like(qh)
@@ -106,13 +117,7 @@ class Attention(nn.Module):
                 nsplits=meta.decode_nsplits,
                 out=out[np_:np_ + nd],
             )
-        attn_flat = out.view(-1, self.num_heads * self.head_dim)
-        o = self.o_proj(attn_flat)
-        if self._lora is not None:
-            self._lora.apply(self._layer_idx, "o", attn_flat, o, meta)
-        if self.tp is not None:
-            o = self.tp.all_reduce(o)
-        return o
+        return out.view(-1, self.num_heads * self.head_dim)
 
 
 class MLP(nn.Module):
@@ -201,6 +206,8 @@ class LlamaForCausalLM(nn.Module):
         meta: BatchMeta,
     ) -> torch.Tensor:
         hidden = self.embed_tokens(input_ids)
+        if meta.lora_rows_tok is not None:
+            return self._forward_lora(hidden, positions, kv_caches, meta)
         residual = None
         for layer, kv in zip(self.layers, kv_caches):
             hidden, residual = layer(
@@ -208,6 +215,54 @@ class LlamaForCausalLM(nn.Module):
             )
         hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
+
+    def lora_in_layer(self, rank: int, dims: dict) -> bool:
+        """Whether `_forward_lora` serves adapters of that rank over those
+        modules: what the kernels of ops/csrc/lora_rows.hip take."""
+        c = self.cfg
+        return (
+            rank == 16
+            and set(dims) == {"qkv", "o", "gate_up", "down"}
+            and c.hidden_size in ops.LORA_ROWS_WIDTHS
+            and c.intermediate_size % 32 == 0
+            and c.head_dim % 64 == 0
+            and (c.num_heads * c.head_dim) % 32 == 0
+        )
+
+    def _forward_lora(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
+        """The layers with every adapter's products carried by the kernels
+        between the projections instead of kernels of their own: B u is added
+        where a projection's output is read, A x formed where its input is
+        written."""
+        lora = self.layers[0].self_attn._lora
+        rows = (meta.lora_rows_tok, meta.lora_rows_len, meta.lora_rows_slot)
+        c = self.cfg
+        ws, u_o, u_down = ops.lora_workspace(
+            rows, c.hidden_size, c.num_heads * c.head_dim, c.intermediate_size)
+        a, b = lora.a_stacks, lora.b_stacks
+        residual, y, last = None, hidden, None
+        for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
+            attn, mlp = layer.self_attn, layer.mlp
+            if last is None:
+                h, u = ops.lora_rms_norm(
+                    y, None, layer.input_layernorm, layer.eps, rows, a_stack=a[(i, "qkv")], u_out=ws)
+                residual = hidden
+            else:
+                h, u = ops.lora_rms_norm(
+                    y, residual, layer.input_layernorm, layer.eps, rows, u_down, b[(last, "down")], a[(i, "qkv")], ws)
+            q = ops.lora_qkv_rope_cache(
+                attn.qkv_proj(h), positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping,
+                attn.num_heads, rows, u, b[(i, "qkv")])
+            o = attn.attend(q, kv, meta)
+            ops.lora_shrink(o, rows, a[(i, "o")], u_o)
+            h, u = ops.lora_rms_norm(
+                attn.o_proj(o), residual, layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")],
+                a[(i, "gate_up")], ws)
+            act = ops.lora_silu_and_mul(
+                mlp.gate_up_proj(h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down)
+            y, last = mlp.down_proj(act), i
+        return ops.lora_rms_norm(
+            y, residual, self.norm, self.cfg.rms_norm_eps, rows, u_down, b[(last, "down")])[0]
 
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """Logits only at the sampled positions (last token of each finished

@@ -324,6 +324,66 @@ def sgmv_expand(u, b_stack, slots, y, scaling=1.0):
     torch_ref.sgmv_expand(u, b_stack, slots, y, scaling)
 
 
+# -- LoRA inside a layer's kernels (ops/csrc/lora_rows.hip); GPU, bf16, rank 16 ------------
+# `rows` = (tokens [tiles, 16], len, slot): tiles of up to 16 tokens of one
+# adapter that together list every row (BatchMeta.lora_rows_*).  u: fp32
+# [parts, tiles, 16, 16], the products with A on their way to B.
+
+LORA_ROWS_WIDTHS = (256, 512, 1024, 2048, 3072, 4096)  # lora_rms_norm's
+
+
+# Below this many tiles lora_rms_norm takes strips of columns in two launches
+# instead of a workgroup per tile in one.  Norms of 4096 columns with both
+# products, in one launch and in two: 9 tiles 21.4 us and 9.2, 45 tiles 23.3 and
+# 15.6, 99 tiles 24.3 and 25.9, 198 tiles 26.0 and 38.9 (two read it all twice).
+LORA_NORM_STRIPS_BELOW = 96
+
+
+def lora_workspace(rows, hidden: int, attn: int, width: int):
+    """(u, u_o, u_down): workspaces of a forward pass over `rows`, in as many
+    parts as lora_rms_norm makes of `hidden` columns, lora_shrink of `attn` and
+    lora_silu_and_mul of `width`.  What a kernel reads and what it writes must
+    not be the same one."""
+    n, dev, ext = rows[1].shape[0], rows[1].device, _load_ext()
+    strips = (ext.lora_norm_strip(), ext.lora_shrink_strip(), ext.lora_silu_strip())
+    parts = [(w + s - 1) // s for w, s in zip((hidden, attn, width), strips)]
+    return torch.empty(sum(parts), n, 16, 16, dtype=torch.float32, device=dev).split(parts)
+
+
+def lora_rms_norm(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_stack=None, u_out=None):
+    """residual += x + B u_in in place (without a residual: x itself is
+    normed), h = rms_norm(residual) * weight, u_out = A h.  Returns h and the
+    parts of u_out that were written."""
+    out = torch.empty_like(x)
+    n, H, strip = rows[1].shape[0], x.shape[1], _EXT.lora_norm_strip()
+    sums, parts = None, 1
+    if n < LORA_NORM_STRIPS_BELOW and H % strip == 0:
+        parts = H // strip
+        sums = torch.empty(n * parts * 16, dtype=torch.float32, device=x.device)
+    _EXT.lora_rms_norm(out, x, residual, weight, eps, *rows, u_in, b_stack, a_stack, u_out, sums, _stream())
+    return out, None if u_out is None else u_out[:parts]
+
+
+def lora_silu_and_mul(x, rows, u_in, b_stack, a_stack, u_out):
+    """silu(gate + B u_in) * (up + B u_in) of x = [gate | up]; u_out = A of it."""
+    out = torch.empty(x.shape[0], x.shape[1] // 2, dtype=x.dtype, device=x.device)
+    _EXT.lora_silu(out, x, *rows, u_in, b_stack, a_stack, u_out, _stream())
+    return out
+
+
+def lora_shrink(x, rows, a_stack, u_out) -> None:
+    """u_out = A x."""
+    _EXT.lora_shrink(x, *rows, a_stack, u_out, _stream())
+
+
+def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, num_heads, rows, u_in, b_stack):
+    """`qkv_rope_cache` of qkv + B u_in."""
+    q = torch.empty(qkv.shape[0], num_heads * k_cache.shape[-1], dtype=qkv.dtype, device=qkv.device)
+    _EXT.lora_qkv_rope_cache(
+        q, qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, *rows, u_in, b_stack, _stream())
+    return q
+
+
 # MEASURED DEAD END (benchmarks/bench_gemm.py on MI355X): the hand-written
 # skinny-M MFMA GEMM (ops/csrc/skinny_gemm.hip) reaches only ~0.5 TB/s of W
 # streaming vs hipBLASLt's 2.4 TB/s at M=128 — and the CDNA guide's own

@@ -5,6 +5,8 @@
 // serialize correctly with the library GEMMs on torch's stream without
 // depending on the HIP/CUDA stream-masquerading ATen headers.
 
+#include <optional>
+
 #include <torch/extension.h>
 
 #include "common.h"
@@ -77,6 +79,29 @@ void lig_sgmv_shrink_tiled_launch(uint16_t*, const uint16_t*, const uint16_t*,
 void lig_sgmv_expand_tiled_launch(uint16_t*, const uint16_t*, const uint16_t*,
                                   const int*, const int*, const int*, int,
                                   float, int, int, int, hipStream_t);
+int lig_lora_rms_norm_launch(uint16_t*, const uint16_t*, uint16_t*,
+                             const uint16_t*, float, int, const int*,
+                             const int*, const int*, int,
+                             const float*, int, int, const uint16_t*,
+                             const uint16_t*, float*, hipStream_t);
+int lig_lora_silu_strip();
+int lig_lora_norm_strip();
+void lig_lora_rms_norm_strips_launch(
+    uint16_t*, const uint16_t*, uint16_t*, const uint16_t*, float, int,
+    const int*, const int*, const int*, int, const float*, int, int,
+    const uint16_t*, const uint16_t*, float*, int, float*, hipStream_t);
+void lig_lora_silu_launch(uint16_t*, const uint16_t*, int, const int*,
+                          const int*, const int*, int, const float*, int, int,
+                          const uint16_t*, const uint16_t*, float*, int,
+                          hipStream_t);
+void lig_lora_shrink_launch(const uint16_t*, int, const int*, const int*,
+                            const int*, int, const uint16_t*, float*, int,
+                            hipStream_t);
+int lig_lora_shrink_strip();
+void lig_lora_qkv_rope_cache_launch(
+    uint16_t*, const uint16_t*, const int64_t*, const float*, uint16_t*,
+    uint16_t*, const int64_t*, int, int, int, int, const int*, const int*,
+    const int*, int, const float*, int, int, const uint16_t*, hipStream_t);
 void lig_paged_attention_prefill_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const int*,
     const int*, const int*, const int*, const int*, float, int, int, int,
@@ -423,6 +448,142 @@ void quant_fp8_rowwise(torch::Tensor xq, torch::Tensor xs, torch::Tensor x,
                                as_stream(stream));
 }
 
+// ---- LoRA inside the layer's kernels (lora_rows.hip) ------------------------
+// toks [tiles, 16], len, slot: tiles of up to 16 tokens of one adapter that
+// together list every row; u: fp32 [parts, tiles, 16, 16]; A [slots, 16, in], B [slots,
+// out, 16].
+
+inline const int* i32_cptr(const torch::Tensor& t) {
+  TORCH_CHECK(t.scalar_type() == torch::kInt32 && t.is_contiguous() && t.is_cuda());
+  return t.data_ptr<int>();
+}
+
+inline float* u_ptr(const torch::Tensor& u, int64_t parts, int64_t ntiles) {
+  TORCH_CHECK(u.scalar_type() == torch::kFloat32 && u.is_contiguous() && u.is_cuda());
+  TORCH_CHECK(u.dim() == 4 && u.size(0) >= parts && u.size(1) >= ntiles &&
+                  u.size(2) == 16 && u.size(3) == 16,
+              "u is [parts, tiles, 16, 16]");
+  return u.data_ptr<float>();
+}
+
+inline const uint16_t* a_ptr(const torch::Tensor& a, int64_t width) {
+  TORCH_CHECK(a.dim() == 3 && a.size(1) == 16 && a.size(2) == width, "A stack mismatch");
+  return bf16_cptr(a);
+}
+
+inline const uint16_t* b_ptr(const torch::Tensor& b, int64_t width) {
+  TORCH_CHECK(b.dim() == 3 && b.size(1) == width && b.size(2) == 16, "B stack mismatch");
+  return bf16_cptr(b);
+}
+
+inline int check_tiles(const torch::Tensor& toks, const torch::Tensor& len,
+                       const torch::Tensor& slot, int64_t T, int64_t slots) {
+  TORCH_CHECK(toks.numel() == 16 * len.numel() && slot.numel() == len.numel());
+  LIG_CHECK_RANGE(toks, 0, T, "lora rows toks");
+  LIG_CHECK_RANGE(len, 0, 17, "lora rows len");
+  LIG_CHECK_RANGE(slot, -1, slots, "lora rows slot");
+  return len.numel();
+}
+
+void lora_rms_norm(torch::Tensor out, torch::Tensor x,
+                   std::optional<torch::Tensor> residual, torch::Tensor weight,
+                   double eps, torch::Tensor toks,
+                   torch::Tensor len, torch::Tensor slot,
+                   std::optional<torch::Tensor> u_in,
+                   std::optional<torch::Tensor> b_stack,
+                   std::optional<torch::Tensor> a_stack,
+                   std::optional<torch::Tensor> u_out,
+                   std::optional<torch::Tensor> sums, int64_t stream) {
+  const int T = x.size(0), H = x.size(1);
+  TORCH_CHECK(out.sizes() == x.sizes() && weight.numel() == H);
+  TORCH_CHECK(!residual || residual->sizes() == x.sizes());
+  TORCH_CHECK(u_in.has_value() == b_stack.has_value() && u_out.has_value() == a_stack.has_value());
+  const int64_t slots = b_stack ? b_stack->size(0) : a_stack ? a_stack->size(0) : 1 << 30;
+  const int n = check_tiles(toks, len, slot, T, slots);
+  if (n == 0 || T == 0) return;
+  if (sums) {  // strips of columns in two launches; u_out has a part for each
+    const int strip = lig_lora_norm_strip();
+    TORCH_CHECK(H % strip == 0 && sums->scalar_type() == torch::kFloat32 &&
+                sums->is_cuda() && sums->numel() >= (int64_t)n * (H / strip) * 16);
+    lig_lora_rms_norm_strips_launch(
+        bf16_ptr(out), bf16_cptr(x), residual ? bf16_ptr(*residual) : nullptr,
+        bf16_cptr(weight), (float)eps, H, i32_cptr(toks), i32_cptr(len),
+        i32_cptr(slot), n, u_in ? u_ptr(*u_in, 1, n) : nullptr,
+        u_in ? (int)u_in->size(0) : 0, u_in ? (int)u_in->size(1) : 0,
+        b_stack ? b_ptr(*b_stack, H) : nullptr,
+        a_stack ? a_ptr(*a_stack, H) : nullptr,
+        u_out ? u_ptr(*u_out, H / strip, n) : nullptr,
+        u_out ? (int)u_out->size(1) : 0, sums->data_ptr<float>(), as_stream(stream));
+    return;
+  }
+  const int rc = lig_lora_rms_norm_launch(
+      bf16_ptr(out), bf16_cptr(x), residual ? bf16_ptr(*residual) : nullptr,
+      bf16_cptr(weight), (float)eps, H, i32_cptr(toks),
+      i32_cptr(len), i32_cptr(slot), n,
+      u_in ? u_ptr(*u_in, 1, n) : nullptr, u_in ? (int)u_in->size(0) : 0,
+      u_in ? (int)u_in->size(1) : 0, b_stack ? b_ptr(*b_stack, H) : nullptr,
+      a_stack ? a_ptr(*a_stack, H) : nullptr,
+      u_out ? u_ptr(*u_out, 1, n) : nullptr, as_stream(stream));
+  TORCH_CHECK(rc == 0, "lora_rms_norm: rows of ", H, " entries not served");
+}
+
+void lora_silu(torch::Tensor out, torch::Tensor x, torch::Tensor toks,
+               torch::Tensor len, torch::Tensor slot,
+               torch::Tensor u_in, torch::Tensor b_stack,
+               torch::Tensor a_stack, torch::Tensor u_out, int64_t stream) {
+  const int T = x.size(0), d = out.size(1);
+  TORCH_CHECK(out.size(0) == T && x.size(1) == 2 * (int64_t)d && d % 32 == 0);
+  const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
+  if (n == 0 || T == 0) return;
+  const int strip = lig_lora_silu_strip();
+  TORCH_CHECK(a_stack.size(0) == b_stack.size(0));
+  lig_lora_silu_launch(bf16_ptr(out), bf16_cptr(x), d, i32_cptr(toks),
+                       i32_cptr(len), i32_cptr(slot), n,
+                       u_ptr(u_in, 1, n), (int)u_in.size(0), (int)u_in.size(1),
+                       b_ptr(b_stack, 2 * (int64_t)d),
+                       a_ptr(a_stack, d), u_ptr(u_out, (d + strip - 1) / strip, n),
+                       (int)u_out.size(1), as_stream(stream));
+}
+
+void lora_shrink(torch::Tensor x, torch::Tensor toks,
+                 torch::Tensor len, torch::Tensor slot, torch::Tensor a_stack,
+                 torch::Tensor u_out, int64_t stream) {
+  const int T = x.size(0), W = x.size(1);
+  TORCH_CHECK(W % 32 == 0, "row width must be a multiple of 32");
+  const int n = check_tiles(toks, len, slot, T, a_stack.size(0));
+  if (n == 0 || T == 0) return;
+  lig_lora_shrink_launch(bf16_cptr(x), W, i32_cptr(toks),
+                         i32_cptr(len), i32_cptr(slot), n, a_ptr(a_stack, W),
+                         u_ptr(u_out, (W + lig_lora_shrink_strip() - 1) / lig_lora_shrink_strip(), n),
+                         (int)u_out.size(1), as_stream(stream));
+}
+
+void lora_qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slot_mapping, torch::Tensor toks,
+                         torch::Tensor len,
+                         torch::Tensor slot, torch::Tensor u_in,
+                         torch::Tensor b_stack, int64_t stream) {
+  TORCH_CHECK(positions.scalar_type() == torch::kInt64);
+  TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 && cos_sin.is_contiguous());
+  const int T = qkv.size(0), Hkv = k_cache.size(1), BS = k_cache.size(2), D = k_cache.size(3);
+  const int Hq = q_out.size(1) / D;
+  TORCH_CHECK(D % 64 == 0 && cos_sin.size(1) == D && v_cache.sizes() == k_cache.sizes());
+  TORCH_CHECK(qkv.size(1) == (int64_t)(Hq + 2 * Hkv) * D && q_out.size(0) == T &&
+              q_out.size(1) == (int64_t)Hq * D);
+  TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
+  const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
+  if (n == 0 || T == 0) return;
+  lig_lora_qkv_rope_cache_launch(
+      bf16_ptr(q_out), bf16_cptr(qkv), positions.data_ptr<int64_t>(),
+      cos_sin.data_ptr<float>(), bf16_ptr(k_cache), bf16_ptr(v_cache),
+      slot_mapping.data_ptr<int64_t>(), Hq, Hkv, D, BS, i32_cptr(toks),
+      i32_cptr(len), i32_cptr(slot), n, u_ptr(u_in, 1, n),
+      (int)u_in.size(0), (int)u_in.size(1), b_ptr(b_stack, qkv.size(1)), as_stream(stream));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -443,6 +604,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sgmv_apply_tiled", &sgmv_apply_tiled);
   m.def("sgmv_expand", &sgmv_expand);
   m.def("quant_fp8_rowwise", &quant_fp8_rowwise);
+  m.def("lora_rms_norm", &lora_rms_norm);
+  m.def("lora_silu", &lora_silu);
+  m.def("lora_silu_strip", &lig_lora_silu_strip);
+  m.def("lora_norm_strip", &lig_lora_norm_strip);
+  m.def("lora_shrink_strip", &lig_lora_shrink_strip);
+  m.def("lora_shrink", &lora_shrink);
+  m.def("lora_qkv_rope_cache", &lora_qkv_rope_cache);
   m.def("mfma_probe", [](torch::Tensor out, torch::Tensor a, torch::Tensor b,
                          int64_t stream) {
     TORCH_CHECK(out.scalar_type() == torch::kFloat32);

@@ -1,0 +1,631 @@
+// Multi-LoRA of a Llama layer inside the kernels that stand between its GEMMs;
+// bf16, rank 16, gfx950.
+//
+// y = W x + B (A x) with an adapter per token.  As kernels of their own, the
+// products with A read every GEMM input once more and those with B read and
+// wrote every GEMM output once more: 3.5 of 15.3 ms of a step with 4000 prompt
+// tokens over 8 layers, and two launches of 5-12 us per GEMM in decode steps.
+// (Now 12.9 ms for that step; norm with both products of 33 tokens of 8 adapters
+// 11.6 us for 15 before, of 384 of 32 16.8 for 26, of 4000 38 for 133.)
+// Here
+//   * B u is added where the GEMM's output is read anyway: the rotation and
+//     cache write (qkv), the residual add and norm (o, down), the gated silu
+//     (gate_up);
+//   * A x is formed where the GEMM's input is written anyway (norm -> qkv and
+//     gate_up, silu -> down); only the attention's output needs a pass (o);
+//   * u stays fp32 between the two, where a bf16 workspace held it before.
+// Both are matrix instructions.  The rows of a launch are tiles of up to 16
+// tokens of one adapter (or of none), listed by the host 16 places a tile, so
+// that a lane finds its row in one load.  In all kernels lane
+// (li, lg) holds 8 neighbouring columns lg*8 .. of token li in a group of 32:
+//   * u^T = A x^T: those 8 values are the second operand as they are;
+//   * y^T += B u^T: with B's rows dealt to two tiles (rows lg*4+i hold columns
+//     lg*8+i and lg*8+4+i) the result lands on them.  K is 32 and the rank 16:
+//     the upper half of K carries the low parts of u = hi + lo against the same
+//     B, so u enters with 16 significant bits at no further instruction.
+//
+// u: fp32 [parts][tiles][16 tokens][16], summed over the parts by the reader.
+
+#include "common.h"
+
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int R = 16;  // rank
+
+struct Tile {
+  int n, slot;  // tokens, adapter (negative: none)
+  int row;      // token of this lane (some token of the tile for lanes past n)
+  bool valid;
+};
+
+LIG_DEVICE Tile tile_of(const int* toks, const int* len, const int* slot, int tile, int li) {
+  Tile t;
+  t.row = toks[tile * 16 + li];
+  t.n = len[tile];
+  t.slot = slot[tile];
+  t.valid = li < t.n;
+  return t;
+}
+
+// this lane's operand of B u^T: ranks (lg & 1) * 8 .. of token li, high parts in
+// lanes lg < 2 and low parts in the others; u: [16 tokens][16]
+LIG_DEVICE bf16x8_t u_operand(const float* u, int li, int lg, bool valid) {
+  const f32x4_t a = *reinterpret_cast<const f32x4_t*>(u + li * R + (lg & 1) * 8);
+  const f32x4_t b = *reinterpret_cast<const f32x4_t*>(u + li * R + (lg & 1) * 8 + 4);
+  u16x8 o;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float v = valid ? (i < 4 ? a[i & 3] : b[i & 3]) : 0.f;
+    const uint16_t hi = f32_to_bf16(v);
+    o[i] = lg < 2 ? hi : f32_to_bf16(v - bf16_to_f32(hi));
+  }
+  return __builtin_bit_cast(bf16x8_t, o);
+}
+
+// the same from a u in several parts, added up through LDS (256 floats);
+// called by all threads of the workgroup
+LIG_DEVICE bf16x8_t u_of(const float* u, int parts, int tiles, float* smem, int li, int lg, bool valid) {
+  if (parts == 1) return u_operand(u, li, lg, valid);
+  for (int e = threadIdx.x; e < 16 * R; e += blockDim.x) {
+    float v = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < parts; ++k) v += u[(size_t)k * tiles * 16 * R + e];
+    smem[e] = v;
+  }
+  __syncthreads();
+  const bf16x8_t o = u_operand(smem, li, lg, valid);
+  __syncthreads();  // smem is used again
+  return o;
+}
+
+// In the kernels below the loads of several groups come first and no branch
+// stands between them: as `if (lora)` around each group's products, every load
+// was waited for by itself (36 us for the norm of 33 rows, 19 so).
+
+// the operands of columns c0 + lg*8 .. +8 of (B u); b: [columns][16] of the adapter
+struct BOperand {
+  u16x8 lo, hi;
+};
+LIG_DEVICE BOperand load_b(const uint16_t* b, int c0, int li, int lg) {
+  const uint16_t* p = b + (size_t)(c0 + ((li >> 2) << 3) + (li & 3)) * R + (lg & 1) * 8;
+  return {*reinterpret_cast<const u16x8*>(p), *reinterpret_cast<const u16x8*>(p + 4 * R)};
+}
+LIG_DEVICE f32x8 expand(const BOperand& b, bf16x8_t u) {
+  const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+  const f32x4_t x = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b.lo), u, z, 0, 0, 0);
+  const f32x4_t y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b.hi), u, z, 0, 0, 0);
+  f32x8 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    o[i] = x[i];
+    o[4 + i] = y[i];
+  }
+  return o;
+}
+
+// columns c0 + lg*8 .. of rank li; a: [16][width] of the adapter
+LIG_DEVICE u16x8 load_a(const uint16_t* a, size_t width, int c0, int li, int lg) {
+  return *reinterpret_cast<const u16x8*>(a + li * width + c0 + lg * 8);
+}
+LIG_DEVICE f32x4_t shrink(u16x8 a, u16x8 x, f32x4_t acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, x), acc,
+                                                 0, 0, 0);
+}
+LIG_DEVICE u16x8 load8(const uint16_t* p) { return *reinterpret_cast<const u16x8*>(p); }
+
+// the W waves' sums of u to u_out[tile] (tokens past the tile's end: whatever)
+template <int W>
+LIG_DEVICE void store_u(float* u_out, f32x4_t acc, float (*red)[16][R], int wave, int li, int lg) {
+  *reinterpret_cast<f32x4_t*>(&red[wave][li][lg * 4]) = acc;
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * R; i += 64 * W) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) s += red[w][i / R][i % R];
+    u_out[i] = s;
+  }
+}
+
+// residual += x + B u (ADD), h = rms_norm(residual) * weight, u_out = A h.  One
+// workgroup per tile holds its rows in registers in between: 8 waves, each every
+// eighth group of 32 columns, NG of them.
+template <bool ADD, int NG, bool DELTA, bool TO_U>
+LIG_DEVICE void norm_rows(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+                          uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, const float eps,
+                          const bf16x8_t u, const uint16_t* __restrict__ b, const uint16_t* __restrict__ a,
+                          float* u_out, float (*ss_s)[16], float (*red)[16][R], int wave, int li, int lg) {
+  constexpr int hidden = NG * 256;
+  constexpr int NB = NG % 8 == 0 ? 8 : NG % 4 == 0 ? 4 : NG;  // groups whose loads are issued together
+  constexpr int NB2 = NG % 4 == 0 ? 4 : NG;
+  const size_t base = (size_t)t.row * hidden + lg * 8;
+  f32x8 v[NG];
+  float ss = 0.f;
+#pragma unroll
+  for (int i0 = 0; i0 < NG; i0 += NB) {
+    u16x8 xr[NB], rr[NB];
+    BOperand br[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int c0 = ((i0 + i) * 8 + wave) * 32;
+      xr[i] = load8(x + base + c0);
+      if constexpr (ADD) rr[i] = load8(residual + base + c0);
+      if constexpr (DELTA) br[i] = load_b(b, c0, li, lg);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      f32x8& w = v[i0 + i];
+      w = bf16x8_to_f32x8(xr[i]);
+      if constexpr (ADD) w += bf16x8_to_f32x8(rr[i]);
+      if constexpr (DELTA) w += expand(br[i], u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += w[j] * w[j];
+    }
+  }
+  if (ADD && t.valid) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
+      *reinterpret_cast<u16x8*>(residual + base + (i * 8 + wave) * 32) = f32x8_to_bf16x8(v[i]);
+  }
+  u16x8 wr[NB2], ar[NB2];
+  auto load_second = [&](int i0) {
+#pragma unroll
+    for (int i = 0; i < NB2; ++i) {
+      const int c0 = ((i0 + i) * 8 + wave) * 32;
+      wr[i] = load8(weight + c0 + lg * 8);
+      if constexpr (TO_U) ar[i] = load_a(a, hidden, c0, li, lg);
+    }
+  };
+  load_second(0);  // on their way while the sums meet
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  if (lg == 0) ss_s[wave][li] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) ss += ss_s[w][li];
+  const float inv = rsqrtf(ss / hidden + eps);
+
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  u16x8 h[NG];
+#pragma unroll
+  for (int i0 = 0; i0 < NG; i0 += NB2) {
+    if (i0 > 0) load_second(i0);
+#pragma unroll
+    for (int i = 0; i < NB2; ++i) {
+      const f32x8 w = bf16x8_to_f32x8(wr[i]);
+      f32x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = v[i0 + i][j] * inv * w[j];
+      h[i0 + i] = f32x8_to_bf16x8(o);
+      if constexpr (TO_U) acc = shrink(ar[i], h[i0 + i], acc);
+    }
+  }
+  if (t.valid) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) *reinterpret_cast<u16x8*>(out + base + (i * 8 + wave) * 32) = h[i];
+  }
+  if constexpr (TO_U) store_u<8>(u_out, acc, red, wave, li, lg);
+}
+
+template <bool ADD, int NG>
+__global__ __launch_bounds__(512) void lora_rms_norm_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, uint16_t* __restrict__ residual,
+    const uint16_t* __restrict__ weight, const float eps, const int* __restrict__ toks,
+    const int* __restrict__ len, const int* __restrict__ slot,
+    const float* u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
+    const uint16_t* __restrict__ a_stack, float* u_out) {
+  constexpr int hidden = NG * 256;
+  __shared__ float ss_s[8][16];
+  __shared__ __align__(16) float red[8][16][R];
+  const int tile = blockIdx.x;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Tile t = tile_of(toks, len, slot, tile, li);
+  if (t.n == 0) return;
+  const bool delta = u_in != nullptr && t.slot >= 0, to_u = u_out != nullptr && t.slot >= 0;
+  const bf16x8_t u = delta ? u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid) : bf16x8_t{};
+  const uint16_t* b = delta ? b_stack + (size_t)t.slot * hidden * R : nullptr;
+  const uint16_t* a = to_u ? a_stack + (size_t)t.slot * R * hidden : nullptr;
+  float* uo = to_u ? u_out + (size_t)tile * 16 * R : nullptr;
+#define ROWS(DELTA, TO_U) \
+  norm_rows<ADD, NG, DELTA, TO_U>(t, out, x, residual, weight, eps, u, b, a, uo, ss_s, red, wave, li, lg)
+  if (ADD && delta && to_u) ROWS(ADD, true);
+  else if (ADD && delta) ROWS(ADD, false);
+  else if (to_u) ROWS(false, true);
+  else ROWS(false, false);
+#undef ROWS
+}
+
+// The same in two launches for steps of few tiles: one workgroup per tile pulls
+// the adapter's 2 x 128 KB and the rows at a single CU's rate (18 us for 9 tiles
+// of 4096 columns).  Workgroups here take 512 columns of a tile; the first kernel
+// leaves the sums of squares of its columns, the second forms the same values
+// again and has the whole row's sum at hand.  u_out gets a part per 512 columns.
+constexpr int NORM_STRIP = 512;
+
+template <bool ADD, bool DELTA, bool TO_U, bool SUM>
+LIG_DEVICE void norm_strip(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+                           uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, const float eps,
+                           const int hidden, const float* u_in, const int parts, const int tiles,
+                           const uint16_t* __restrict__ b, const uint16_t* __restrict__ a, float* u_out,
+                           const int tiles_out, float* sums,
+                           float* smem, int wave, int li, int lg) {
+  constexpr int NB = NORM_STRIP / 128;
+  const int c_first = blockIdx.y * NORM_STRIP + wave * 32;
+  const size_t base = (size_t)t.row * hidden + lg * 8;
+  u16x8 xr[NB], rr[NB], wr[NB], ar[NB];
+  BOperand br[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int c0 = c_first + i * 128;
+    xr[i] = load8(x + base + c0);
+    if constexpr (ADD) rr[i] = load8(residual + base + c0);
+    if constexpr (DELTA) br[i] = load_b(b, c0, li, lg);
+    if constexpr (!SUM) wr[i] = load8(weight + c0 + lg * 8);
+    if constexpr (!SUM && TO_U) ar[i] = load_a(a, hidden, c0, li, lg);
+  }
+  const int strips = hidden / NORM_STRIP;
+  float total = 0.f;
+  if constexpr (!SUM) {
+#pragma unroll 8
+    for (int k = 0; k < strips; ++k) total += sums[k * 16 + li];
+  }
+  bf16x8_t u = {};
+  if constexpr (DELTA) u = u_of(u_in, parts, tiles, smem, li, lg, t.valid);
+  f32x8 v[NB];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    v[i] = bf16x8_to_f32x8(xr[i]);
+    if constexpr (ADD) v[i] += bf16x8_to_f32x8(rr[i]);
+    if constexpr (DELTA) v[i] += expand(br[i], u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
+  }
+  if constexpr (SUM) {
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    if (lg == 0) smem[wave * 16 + li] = ss;
+    __syncthreads();
+    if (threadIdx.x < 16)
+      sums[blockIdx.y * 16 + threadIdx.x] =
+          smem[threadIdx.x] + smem[16 + threadIdx.x] + smem[32 + threadIdx.x] + smem[48 + threadIdx.x];
+  } else {
+    const float inv = rsqrtf(total / hidden + eps);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    u16x8 h[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const f32x8 w = bf16x8_to_f32x8(wr[i]);
+      f32x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = v[i][j] * inv * w[j];
+      h[i] = f32x8_to_bf16x8(o);
+      if constexpr (TO_U) acc = shrink(ar[i], h[i], acc);
+    }
+    if (t.valid) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int c0 = c_first + i * 128;
+        *reinterpret_cast<u16x8*>(out + base + c0) = h[i];
+        if constexpr (ADD) *reinterpret_cast<u16x8*>(residual + base + c0) = f32x8_to_bf16x8(v[i]);
+      }
+    }
+    if constexpr (TO_U) {
+      float(*red)[16][R] = reinterpret_cast<float(*)[16][R]>(smem);
+      store_u<4>(u_out + (size_t)blockIdx.y * tiles_out * 16 * R, acc, red, wave, li, lg);
+    }
+  }
+}
+
+template <bool ADD, bool SUM>
+__global__ __launch_bounds__(256) void lora_norm_strip_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, uint16_t* __restrict__ residual,
+    const uint16_t* __restrict__ weight, const float eps, const int hidden, const int* __restrict__ toks,
+    const int* __restrict__ len, const int* __restrict__ slot, const float* u_in, const int parts, const int tiles,
+    const uint16_t* __restrict__ b_stack, const uint16_t* __restrict__ a_stack, float* u_out, const int tiles_out,
+    float* sums) {
+  __shared__ __align__(16) float smem[4 * 16 * R];
+  const int tile = blockIdx.x;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Tile t = tile_of(toks, len, slot, tile, li);
+  if (t.n == 0) return;
+  const bool delta = u_in != nullptr && t.slot >= 0, to_u = u_out != nullptr && t.slot >= 0;
+  const float* ui = delta ? u_in + (size_t)tile * 16 * R : nullptr;
+  const uint16_t* b = delta ? b_stack + (size_t)t.slot * hidden * R : nullptr;
+  const uint16_t* a = to_u ? a_stack + (size_t)t.slot * R * hidden : nullptr;
+  float* uo = to_u ? u_out + (size_t)tile * 16 * R : nullptr;
+  float* sm = sums + (size_t)tile * (hidden / NORM_STRIP) * 16;
+#define STRIP(DELTA, TO_U)                                                                                          \
+  norm_strip<ADD, DELTA, TO_U, SUM>(t, out, x, residual, weight, eps, hidden, ui, parts, tiles, b, a, uo, tiles_out, sm, \
+                                    smem, wave, li, lg)
+  if (ADD && delta && to_u) STRIP(ADD, true);
+  else if (ADD && delta) STRIP(ADD, false);
+  else if (to_u) STRIP(false, true);
+  else STRIP(false, false);
+#undef STRIP
+}
+
+// out = silu(gate + B u) * (up + B u), u_out[strip] = A_down out.  Workgroups of
+// a tile take strips of 1024 of the d columns.
+constexpr int SILU_STRIP = 1024;
+
+template <bool LORA>
+LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d,
+                             const int c_first, const bf16x8_t u, const uint16_t* __restrict__ b,
+                             const uint16_t* __restrict__ a, int li, int lg) {
+  constexpr int NB = 4;  // groups whose loads are issued together
+  const uint16_t* g = x + (size_t)t.row * 2 * d + lg * 8;
+  uint16_t* o = out + (size_t)t.row * d + lg * 8;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < SILU_STRIP / 128; i0 += NB) {
+    u16x8 gr[NB], ur[NB], ar[NB];
+    BOperand bg[NB], bu[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int c0 = min(c_first + (i0 + i) * 128, d - 32);  // groups past the end: the last one again, unused
+      gr[i] = load8(g + c0);
+      ur[i] = load8(g + d + c0);
+      if constexpr (LORA) {
+        bg[i] = load_b(b, c0, li, lg);
+        bu[i] = load_b(b, d + c0, li, lg);
+        ar[i] = load_a(a, d, c0, li, lg);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int c0 = c_first + (i0 + i) * 128;
+      if (c0 >= d) break;
+      f32x8 gv = bf16x8_to_f32x8(gr[i]), uv = bf16x8_to_f32x8(ur[i]), r;
+      if constexpr (LORA) {
+        gv += expand(bg[i], u);
+        uv += expand(bu[i], u);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r[j] = gv[j] / (1.0f + __expf(-gv[j])) * uv[j];
+      const u16x8 rb = f32x8_to_bf16x8(r);
+      if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
+      if constexpr (LORA) acc = shrink(ar[i], rb, acc);
+    }
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(256) void lora_silu_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
+    const int* __restrict__ len, const int* __restrict__ slot,
+    const float* __restrict__ u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
+    const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out) {
+  __shared__ __align__(16) float red[4][16][R];
+  const int tile = blockIdx.x, strip = blockIdx.y;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Tile t = tile_of(toks, len, slot, tile, li);
+  if (t.n == 0) return;
+  const int c_first = strip * SILU_STRIP + wave * 32;
+  if (t.slot < 0) {
+    silu_rows<false>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, li, lg);
+    return;
+  }
+  const f32x4_t acc =
+      silu_rows<true>(t, out, x, d, c_first,
+                      u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid),
+                      b_stack + (size_t)t.slot * 2 * d * R, a_stack + (size_t)t.slot * R * d, li, lg);
+  store_u<4>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+}
+
+// u_out = A x, a part per strip of 512 columns
+constexpr int SHRINK_STRIP = 512;
+
+__global__ __launch_bounds__(256) void lora_shrink_kernel(
+    const uint16_t* __restrict__ x, const int width, const int* __restrict__ toks, const int* __restrict__ len,
+    const int* __restrict__ slot, const uint16_t* __restrict__ a_stack, float* __restrict__ u_out,
+    const int tiles_out) {
+  constexpr int NB = SHRINK_STRIP / 128;
+  __shared__ __align__(16) float red[4][16][R];
+  const int tile = blockIdx.x;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Tile t = tile_of(toks, len, slot, tile, li);
+  if (t.n == 0 || t.slot < 0) return;
+  const uint16_t* a = a_stack + (size_t)t.slot * R * width;
+  const uint16_t* row = x + (size_t)t.row * width + lg * 8;
+  const int c_first = blockIdx.y * SHRINK_STRIP + wave * 32;
+  u16x8 xr[NB], ar[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int c0 = min(c_first + i * 128, width - 32);  // groups past the end: the last one again, unused
+    xr[i] = load8(row + c0);
+    ar[i] = load_a(a, width, c0, li, lg);
+  }
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    if (c_first + i * 128 < width) acc = shrink(ar[i], xr[i], acc);
+  store_u<4>(u_out + ((size_t)blockIdx.y * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+}
+
+// qkv_rope.hip's pass with B u added to the projection on the way in
+constexpr int QR_HEADS = 4;
+
+__global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
+    uint16_t* __restrict__ q_out, const uint16_t* __restrict__ qkv, const int64_t* __restrict__ positions,
+    const float* __restrict__ cos_sin, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
+    const int64_t* __restrict__ slot_mapping, const int num_q_heads, const int num_kv_heads, const int head_dim,
+    const int block_size, const int* __restrict__ toks, const int* __restrict__ len,
+    const int* __restrict__ slot, const float* __restrict__ u_in, const int u_parts, const int tiles,
+    const uint16_t* __restrict__ b_stack) {
+  __shared__ __align__(16) float smem[16 * R];
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int parts = head_dim / 64;  // of 32 rotation pairs
+  const int wid = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int heads = num_q_heads + 2 * num_kv_heads;
+  const int h0 = (wid / parts) * QR_HEADS;
+  const Tile t = tile_of(toks, len, slot, blockIdx.x, li);
+  if (t.n == 0) return;
+  bf16x8_t u = {};
+  if (t.slot >= 0) u = u_of(u_in + (size_t)blockIdx.x * 16 * R, u_parts, tiles, smem, li, lg, t.valid);
+  if (h0 >= heads) return;  // whole waves: no lane may miss the matrix instructions
+  const int half = head_dim / 2;
+  const int p0 = (wid % parts) * 32, c = p0 + lg * 8;
+
+  const float* cs = cos_sin + positions[t.row] * head_dim + c;
+  float co[8], si[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(cs + i);
+    const f32x4 b = *reinterpret_cast<const f32x4*>(cs + half + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      co[i + j] = a[j];
+      si[i + j] = b[j];
+    }
+  }
+  const int64_t at = slot_mapping[t.row];
+  const size_t blk = at < 0 ? 0 : at / block_size;
+  const size_t off = at < 0 ? 0 : at % block_size;
+  const uint16_t* src = qkv + ((size_t)t.row * heads + h0) * head_dim + c;
+  u16x8 x[QR_HEADS][2];
+#pragma unroll
+  for (int i = 0; i < QR_HEADS; ++i) {
+    const int h = min(h0 + i, heads - 1) - h0;
+    x[i][0] = load8(src + h * head_dim);
+    x[i][1] = load8(src + h * head_dim + half);
+  }
+  f32x8 v[QR_HEADS][2];
+#pragma unroll
+  for (int i = 0; i < QR_HEADS; ++i) {
+    v[i][0] = bf16x8_to_f32x8(x[i][0]);
+    v[i][1] = bf16x8_to_f32x8(x[i][1]);
+  }
+  if (t.slot >= 0) {
+    const uint16_t* b = b_stack + (size_t)t.slot * heads * head_dim * R;
+    BOperand br[QR_HEADS][2];
+#pragma unroll
+    for (int i = 0; i < QR_HEADS; ++i) {
+      const int h = min(h0 + i, heads - 1);
+      br[i][0] = load_b(b, h * head_dim + p0, li, lg);
+      br[i][1] = load_b(b, h * head_dim + half + p0, li, lg);
+    }
+#pragma unroll
+    for (int i = 0; i < QR_HEADS; ++i) {
+      v[i][0] += expand(br[i][0], u);
+      v[i][1] += expand(br[i][1], u);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < QR_HEADS; ++i) {
+    const int h = h0 + i;
+    if (h >= heads) break;
+    const bool turned = h < num_q_heads + num_kv_heads;
+    if (turned) {
+      f32x8 o1, o2;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        o1[j] = v[i][0][j] * co[j] - v[i][1][j] * si[j];
+        o2[j] = v[i][1][j] * co[j] + v[i][0][j] * si[j];
+      }
+      v[i][0] = o1;
+      v[i][1] = o2;
+    }
+    uint16_t* dst;
+    if (h < num_q_heads) {
+      dst = q_out + ((size_t)t.row * num_q_heads + h) * head_dim;
+    } else {
+      const int g = h - num_q_heads - (turned ? 0 : num_kv_heads);
+      dst = (turned ? k_cache : v_cache) + ((blk * num_kv_heads + g) * block_size + off) * head_dim;
+    }
+    if (t.valid && (h < num_q_heads || at >= 0)) {
+      *reinterpret_cast<u16x8*>(dst + c) = f32x8_to_bf16x8(v[i][0]);
+      *reinterpret_cast<u16x8*>(dst + half + c) = f32x8_to_bf16x8(v[i][1]);
+    }
+  }
+}
+
+}  // namespace
+
+extern "C" {
+
+// Returns 1 for a row width that is not served.
+int lig_lora_rms_norm_launch(uint16_t* out, const uint16_t* x, uint16_t* residual, const uint16_t* weight, float eps,
+                             int hidden, const int* toks, const int* len, const int* slot, int ntiles,
+                             const float* u_in, int parts, int tiles, const uint16_t* b_stack,
+                             const uint16_t* a_stack, float* u_out, hipStream_t stream) {
+#define LAUNCH_N(NG)                                                                                                 \
+  case NG * 256:                                                                                                     \
+    if (residual)                                                                                                    \
+      hipLaunchKernelGGL((lora_rms_norm_kernel<true, NG>), dim3(ntiles), dim3(512), 0, stream, out, x, residual,     \
+                         weight, eps, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out);            \
+    else                                                                                                             \
+      hipLaunchKernelGGL((lora_rms_norm_kernel<false, NG>), dim3(ntiles), dim3(512), 0, stream, out, x, residual,    \
+                         weight, eps, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out);            \
+    return 0
+  switch (hidden) {
+    LAUNCH_N(1);
+    LAUNCH_N(2);
+    LAUNCH_N(4);
+    LAUNCH_N(8);
+    LAUNCH_N(12);
+    LAUNCH_N(16);
+  }
+#undef LAUNCH_N
+  return 1;
+}
+
+int lig_lora_silu_strip() { return SILU_STRIP; }
+int lig_lora_norm_strip() { return NORM_STRIP; }
+
+// sums: fp32 [tiles, hidden / strip, 16]; hidden a multiple of the strip
+void lig_lora_rms_norm_strips_launch(uint16_t* out, const uint16_t* x, uint16_t* residual, const uint16_t* weight,
+                                     float eps, int hidden, const int* toks, const int* len, const int* slot, int ntiles,
+                                     const float* u_in, int parts, int tiles, const uint16_t* b_stack,
+                                     const uint16_t* a_stack, float* u_out, int tiles_out, float* sums,
+                                     hipStream_t stream) {
+#define LAUNCH_S(ADD, SUM)                                                                                      \
+  hipLaunchKernelGGL((lora_norm_strip_kernel<ADD, SUM>), dim3(ntiles, hidden / NORM_STRIP), dim3(256), 0, stream, out, \
+                     x, residual, weight, eps, hidden, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out,  \
+                     tiles_out, sums)
+  if (residual) {
+    LAUNCH_S(true, true);
+    LAUNCH_S(true, false);
+  } else {
+    LAUNCH_S(false, true);
+    LAUNCH_S(false, false);
+  }
+#undef LAUNCH_S
+}
+
+void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* toks, const int* len,
+                          const int* slot, int ntiles, const float* u_in, int parts, int tiles,
+                          const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
+                          hipStream_t stream) {
+  hipLaunchKernelGGL(lora_silu_kernel, dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(256), 0, stream, out, x, d,
+                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out);
+}
+
+int lig_lora_shrink_strip() { return SHRINK_STRIP; }
+
+void lig_lora_shrink_launch(const uint16_t* x, int width, const int* toks, const int* len, const int* slot, int ntiles,
+                            const uint16_t* a_stack, float* u_out, int tiles_out, hipStream_t stream) {
+  hipLaunchKernelGGL(lora_shrink_kernel, dim3(ntiles, (width + SHRINK_STRIP - 1) / SHRINK_STRIP), dim3(256), 0, stream, x,
+                     width, toks, len, slot, a_stack, u_out, tiles_out);
+}
+
+void lig_lora_qkv_rope_cache_launch(uint16_t* q_out, const uint16_t* qkv, const int64_t* positions,
+                                    const float* cos_sin, uint16_t* k_cache, uint16_t* v_cache,
+                                    const int64_t* slot_mapping, int num_q_heads, int num_kv_heads, int head_dim,
+                                    int block_size, const int* toks, const int* len, const int* slot,
+                                    int ntiles, const float* u_in, int u_parts, int tiles, const uint16_t* b_stack,
+                                    hipStream_t stream) {
+  const int heads = num_q_heads + 2 * num_kv_heads;
+  const int waves = (head_dim / 64) * ((heads + QR_HEADS - 1) / QR_HEADS);
+  hipLaunchKernelGGL(lora_qkv_rope_cache_kernel, dim3(ntiles, (waves + 3) / 4), dim3(256), 0, stream, q_out, qkv,
+                     positions, cos_sin, k_cache, v_cache, slot_mapping, num_q_heads, num_kv_heads, head_dim,
+                     block_size, toks, len, slot, u_in, u_parts, tiles, b_stack);
+}
+
+}  // extern "C"

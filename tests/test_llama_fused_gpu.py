@@ -38,3 +38,178 @@ def test_qkv_rope_cache(T, Hq, Hkv, D, bs):
     for a, b in ((got, qr), (kc, kw), (vc, vw)):
         assert ((a.float() - b).abs() <= 2.0 ** -8 * b.abs() + 1e-5).all()
     assert torch.equal(vc.float(), vw)
+
+
+# -- LoRA inside the layer's kernels ------------------------------------------------------
+# u keeps 16 significant bits on its way through the second product, sums are
+# fp32: 2^-16 of the summed magnitudes, besides the one rounding of a result.
+
+SLOTS = [[0], [-1], [2] * 15, [1] * 16 + [-1], [3, 0, -1, 1] * 10 + [2] * 17]
+
+
+def _lora(slots, seed):
+    from llm_instance_gateway_amd.lora.manager import build_lora_rows
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    toks, ln, us = (torch.from_numpy(a).cuda() for a in build_lora_rows(slots))
+    # three empty tiles behind, as a decode graph pads them
+    z = torch.zeros(3, 16, dtype=torch.int32, device="cuda")
+    rows = (torch.cat([toks, z]), torch.cat([ln, z[:, 0]]), torch.cat([us, z[:, 0] - 1]))
+    return rnd, rows, torch.tensor(slots, device="cuda")
+
+
+def _delta(u, b, slots):
+    """B u and the magnitude of its terms; u fp32 [T, 16]."""
+    on = (slots >= 0).float()[:, None]
+    bs = b.float()[slots.clamp(min=0)]
+    return torch.einsum("tor,tr->to", bs, u) * on, torch.einsum("tor,tr->to", bs.abs(), u.abs()) * on
+
+
+def _pack(u, rows, parts=1):
+    """[T, 16] -> [parts, tiles, 16, 16], the parts adding up to it."""
+    toks, ln, _ = (r.tolist() for r in rows)
+    out = torch.full((parts, len(ln), 16, 16), float("nan"), device="cuda")
+    for i, n in enumerate(ln):
+        out[:, i, :n] = u[toks[i][:n]] / parts
+    return out
+
+
+def _unpack(u, rows, T):
+    toks, ln, _ = (r.tolist() for r in rows)
+    out = torch.zeros(T, 16, device="cuda")
+    for i, n in enumerate(ln):
+        out[toks[i][:n]] = u[:, i, :n].sum(0)
+    return out
+
+
+def _check_u(got, x, a, slots, rows):
+    """A x of the rows that have an adapter."""
+    on = slots >= 0
+    ref = torch.einsum("trk,tk->tr", a.float()[slots.clamp(min=0)], x.float())
+    mag = torch.einsum("trk,tk->tr", a.float()[slots.clamp(min=0)].abs(), x.float().abs())
+    d = (_unpack(got, rows, len(slots)) - ref).abs()
+    assert (d[on] <= 2.0 ** -20 * mag[on] * x.shape[1] ** 0.5 + 1e-6).all()
+
+
+@pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
+@pytest.mark.parametrize("H", [256, 1024, 3072, 4096])
+def test_lora_rms_norm(slots, H, monkeypatch):
+    rnd, rows, sl = _lora(slots, H)
+    T = len(slots)
+    x, res, w = rnd(T, H).to(BF), rnd(T, H).to(BF), (1 + 0.1 * rnd(H)).to(BF)
+    a, b, u = rnd(4, 16, H).to(BF), (0.1 * rnd(4, H, 16)).to(BF), rnd(T, 16)
+    ws, _, _ = ops.lora_workspace(rows, H, 32, 32)
+    d, mag = _delta(u, b, sl)
+    # a workgroup per tile, then strips of columns where the width has whole ones
+    for limit, parts in ((0, 1), (0, 15), (0, 0), (10**6, 1), (10**6, 15), (10**6, 0)):
+        monkeypatch.setattr(ops, "LORA_NORM_STRIPS_BELOW", limit)
+        residual = res.clone() if parts else None
+        if residual is None:
+            h, u_out = ops.lora_rms_norm(x, None, w, 1e-5, rows, a_stack=a, u_out=ws)
+            s, tol = x.float(), 0.0
+        else:
+            h, u_out = ops.lora_rms_norm(x, residual, w, 1e-5, rows, _pack(u, rows, parts), b, a, ws)
+            s, tol = x.float() + res.float() + d, 2.0 ** -16 * mag + 1e-6
+            assert ((residual.float() - s).abs() <= 2.0 ** -8 * s.abs() + tol).all()
+        ref = s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * w.float()
+        rms = s.pow(2).mean(-1, keepdim=True).sqrt()
+        assert ((h.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * tol / rms + 1e-5).all()
+        _check_u(u_out, h, a, sl, rows)
+
+
+@pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
+@pytest.mark.parametrize("d", [32, 160, 1024, 1056, 3584])
+def test_lora_silu_and_mul(slots, d):
+    rnd, rows, sl = _lora(slots, d)
+    T = len(slots)
+    x, u = rnd(T, 2 * d).to(BF), rnd(T, 16)
+    a, b = rnd(4, 16, d).to(BF), (0.1 * rnd(4, 2 * d, 16)).to(BF)
+    _, _, u_out = ops.lora_workspace(rows, 256, 32, d)
+    got = ops.lora_silu_and_mul(x, rows, _pack(u, rows, 1 if d % 64 else 3), b, a, u_out)
+    dl, mag = _delta(u, b, sl)
+    gate, up = (x.float() + dl).chunk(2, dim=-1)
+    ref = gate * torch.sigmoid(gate) * up
+    mg, mu = mag.chunk(2, dim=-1)
+    # silu' is at most 1.1
+    tol = 2.0 ** -16 * (1.1 * mg * up.abs() + mu * (gate * torch.sigmoid(gate)).abs()) + 1e-5 * (1 + ref.abs())
+    assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + tol).all()
+    _check_u(u_out, got, a, sl, rows)
+
+
+@pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
+@pytest.mark.parametrize("width", [32, 288, 4096])
+def test_lora_shrink(slots, width):
+    rnd, rows, sl = _lora(slots, width)
+    x, a = rnd(len(slots), width).to(BF), rnd(4, 16, width).to(BF)
+    _, u, _ = ops.lora_workspace(rows, 256, width, 32)
+    ops.lora_shrink(x, rows, a, u)
+    _check_u(u, x, a, sl, rows)
+
+
+@pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
+@pytest.mark.parametrize("Hq,Hkv,D,bs", [(32, 8, 128, 16), (4, 2, 64, 32), (3, 1, 128, 6)])
+def test_lora_qkv_rope_cache(slots, Hq, Hkv, D, bs):
+    rnd, rows, sl = _lora(slots, D)
+    T, W = len(slots), (Hq + 2 * Hkv) * D
+    qkv, u, b = rnd(T, W).to(BF), rnd(T, 16), (0.1 * rnd(4, W, 16)).to(BF)
+    blocks = (T + bs - 1) // bs + 2
+    kc, vc = rnd(blocks, Hkv, bs, D).to(BF), rnd(blocks, Hkv, bs, D).to(BF)
+    cs = ops.build_cos_sin_cache(D, 500, 1e4, "cuda").float()
+    pos = torch.randint(0, 500, (T,), device="cuda")
+    at = torch.randperm(blocks * bs, device="cuda")[:T]
+    if T > 3:
+        at[2] = -1
+    dl, mag = _delta(u, b, sl)
+    q, k, v = (qkv.float() + dl).split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+    qr, kr = torch_ref.rotary_embedding(pos, q, k, cs, D)
+    kw, vw = kc.float(), vc.float()
+    live = at >= 0
+    torch_ref.reshape_and_cache(kr[live], v[live], kw, vw, at[live])
+    got = ops.lora_qkv_rope_cache(qkv, pos, cs, kc, vc, at, Hq, rows, _pack(u, rows, 1 if D == 64 else 8), b)
+    tol = 2.0 ** -15 * mag.max() + 1e-5  # a rotation adds two entries' errors
+    for x, y in ((got, qr), (kc, kw), (vc, vw)):
+        assert ((x.float() - y).abs() <= 2.0 ** -8 * y.abs() + tol).all()
+
+
+def test_engine_matches_unit_kernels(monkeypatch):
+    """A whole step through the in-layer kernels beside one through the SGMV
+    kernels, prompts and decodes, eager and through the decode graph."""
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.lora import manager
+    from llm_instance_gateway_amd.models.config import ModelConfig
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=512, num_layers=3, num_heads=8, num_kv_heads=2,
+                     intermediate_size=768, head_dim=64, max_position_embeddings=512)
+    outs = []
+    for units in (False, True):
+        monkeypatch.setattr(manager, "_TILED_SGMV", False)
+        torch.manual_seed(0)
+        eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=200, max_num_seqs=8, max_model_len=256), device="cuda:0")
+        mgr = manager.AdapterManager(eng, max_slots=3, rank=16)
+        assert mgr.in_layer
+        mgr.in_layer = not units
+        for i in range(3):
+            mgr.register_random(f"l{i}", seed=i)
+        g = torch.Generator().manual_seed(5)
+        for i, n in enumerate((3, 17, 40, 64, 5)):
+            eng.add_request(torch.randint(1, 500, (n,), generator=g).tolist(), SamplingParams(max_new_tokens=1),
+                            lora_name=["l0", "", "l2", "l1", "l0"][i])
+        logits = []
+        execute = eng.runner.model.compute_logits
+        monkeypatch.setattr(eng.runner.model, "compute_logits", lambda h, idx: logits.append(execute(h, idx)) or logits[-1])
+        eng.step()
+        first = logits[-1][:5].clone()
+        seqs = [eng.add_request([7 + i] * (9 + i), SamplingParams(max_new_tokens=4), lora_name=["l2", "", "l0"][i % 3]) for i in range(5)]
+        eng.step()
+        for s in seqs:  # the same continuation on both sides
+            s.output_token_ids[-1] = 11
+        for _ in range(2):  # graph replays
+            eng.step()
+            for s in seqs:
+                s.output_token_ids[-1] = 12
+        gr = eng.runner.graph_runner
+        outs.append((first, gr.logits[gr.pick_size(5)][:5].float().clone()))
+    for a, b in zip(*outs):
+        # two correct orders of bf16 rounding, 3 layers deep
+        assert (a - b).norm() <= 0.03 * b.norm()

@@ -227,6 +227,27 @@ def test_preemption_with_adapter_eviction_interplay():
     assert out_c == out_r
 
 
+@pytest.mark.parametrize(
+    "slots", [[], [0], [-1], [2] * 16, [2] * 17, [-1] * 33, [0, 1, 0, -1, 3, 1], list(range(5)) * 20 + [-1] * 7]
+)
+def test_build_lora_rows(slots):
+    """Every token once, one adapter per tile, at most 16 tokens, and never more
+    tiles than the decode graphs leave room for."""
+    from llm_instance_gateway_amd.lora.manager import build_lora_rows, max_lora_rows
+
+    toks, ln, us = build_lora_rows(slots)
+    assert toks.shape == (len(ln), 16)
+    seen = []
+    for row, n, s in zip(toks.tolist(), ln, us):
+        assert 1 <= n <= 16
+        assert {slots[t] for t in row} == {s}  # the places past n included
+        seen += row[:n]
+    assert sorted(seen) == list(range(len(slots)))
+    assert len(ln) <= max_lora_rows(len(slots), 5)
+    for arr in (toks, ln, us):
+        assert arr.dtype == "int32"
+
+
 def test_build_lora_units():
     """Slot-grouped unit building: stable sort, -1 excluded, runs chunked."""
     import numpy as np
