@@ -12,7 +12,8 @@ Static-buffer contract: per padded batch size B the graph reads
   lora_slots[B]
 and writes logits[B, vocab] (bf16).  Padding rows decode a scratch KV block
 (one extra block appended to the cache pool) with context_len=1 so they
-compute garbage without touching live state.
+compute garbage without touching live state.  The inputs of a bucket lie in
+one device buffer, so a replay needs one copy from the host.
 
 Prefill / mixed steps stay eager (their shapes vary too much to bucket).
 """
@@ -21,10 +22,13 @@ from __future__ import annotations
 
 import gc
 import logging
+from types import SimpleNamespace
 from typing import Dict, List, Optional
 
+import numpy as np
 import torch
 
+from .batch_arrays import device_view, lay_out, pack_rows
 from .metadata import BatchMeta
 
 log = logging.getLogger(__name__)
@@ -46,44 +50,9 @@ class DecodeGraphRunner:
             self.sizes.append(self.max_bs)
         dev = self.device
         B = self.max_bs
-        self.ids = torch.zeros(B, dtype=torch.int64, device=dev)
-        self.pos = torch.zeros(B, dtype=torch.int64, device=dev)
-        self.slot_mapping = torch.zeros(B, dtype=torch.int64, device=dev)
-        self.block_tables = torch.zeros(
-            B, self.max_blocks, dtype=torch.int32, device=dev
-        )
-        self.context_lens = torch.ones(B, dtype=torch.int32, device=dev)
-        self.lora_slots = torch.full((B,), -1, dtype=torch.int32, device=dev)
-        # slot-grouped SGMV unit buffers (U == B, empty units padded len=0)
-        self.lora_order = torch.zeros(B, dtype=torch.int32, device=dev)
-        self.lora_ut0 = torch.zeros(B, dtype=torch.int32, device=dev)
-        self.lora_ulen = torch.zeros(B, dtype=torch.int32, device=dev)
-        self.lora_uslot = torch.full((B,), -1, dtype=torch.int32, device=dev)
         # graph-private LoRA shrink workspace (see metadata.lora_ws): replay
         # must not share u with a concurrently-running eager prefill
         self.lora_ws: Optional[torch.Tensor] = None
-        # pinned host staging (one copy per tensor per step)
-        self.h_ids = torch.zeros(B, dtype=torch.int64, pin_memory=True)
-        self.h_pos = torch.zeros(B, dtype=torch.int64, pin_memory=True)
-        self.h_slot = torch.zeros(B, dtype=torch.int64, pin_memory=True)
-        self.h_bt = torch.zeros(B, self.max_blocks, dtype=torch.int32, pin_memory=True)
-        self.h_ctx = torch.ones(B, dtype=torch.int32, pin_memory=True)
-        self.h_lora = torch.full((B,), -1, dtype=torch.int32, pin_memory=True)
-        self.h_order = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        self.h_ut0 = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        self.h_ulen = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        self.h_uslot = torch.full((B,), -1, dtype=torch.int32, pin_memory=True)
-        # numpy views of the pinned staging (fast per-row fills from lists)
-        self.n_ids = self.h_ids.numpy()
-        self.n_pos = self.h_pos.numpy()
-        self.n_slot = self.h_slot.numpy()
-        self.n_bt = self.h_bt.numpy()
-        self.n_ctx = self.h_ctx.numpy()
-        self.n_lora = self.h_lora.numpy()
-        self.n_order = self.h_order.numpy()
-        self.n_ut0 = self.h_ut0.numpy()
-        self.n_ulen = self.h_ulen.numpy()
-        self.n_uslot = self.h_uslot.numpy()
         # Models that address the batch per sequence (general-size attention,
         # recurrent layers): a decode step is B one-token segments, row i ==
         # sequence i; only the state slot and the starts-here flag vary.
@@ -95,17 +64,12 @@ class DecodeGraphRunner:
             self.seg_len = torch.ones(B, dtype=torch.int32, device=dev)
             # scratch state slot for padding rows = one past the pool
             self.scratch_slot = getattr(runner, "num_state_slots", 0)
-            self.seg_slot = torch.full((B,), self.scratch_slot, dtype=torch.int32, device=dev)
-            self.seg_fresh = torch.ones(B, dtype=torch.int32, device=dev)
-            self.h_sslot = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-            self.h_sfresh = torch.ones(B, dtype=torch.int32, pin_memory=True)
-            self.n_sslot = self.h_sslot.numpy()
-            self.n_sfresh = self.h_sfresh.numpy()
         # scratch KV block for padding rows = last block of the (extended) pool
         self.scratch_block = runner.config.num_kv_blocks  # extra block id
         self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self.logits: Dict[int, torch.Tensor] = {}
         self._pool = None
+        self._inputs: Dict[int, SimpleNamespace] = {}
         self.with_lora = False
         self.lora_in_layer = False
 
@@ -130,46 +94,68 @@ class DecodeGraphRunner:
         attn = model.layers[0].self_attn
         return attn.num_heads, attn.num_kv_heads, attn.head_dim
 
+    def _fields(self, B: int) -> dict:
+        """name -> (dtype, shape) of what a bucket's graph reads anew each replay."""
+        f = dict(ids=(torch.int64, (B,)), pos=(torch.int64, (B,)), slot_mapping=(torch.int64, (B,)),
+                 block_tables=(torch.int32, (B, self.max_blocks)), context_lens=(torch.int32, (B,)))
+        if self.seq_tables:
+            f.update(seg_slot=(torch.int32, (B,)), seg_fresh=(torch.int32, (B,)))
+        if self.with_lora and self.lora_in_layer:
+            # row tiles, as many as B tokens can need, the unused ones empty
+            n = self._max_rows(B)
+            f.update(lora_tok=(torch.int32, (n, 16)), lora_len=(torch.int32, (n,)), lora_slot=(torch.int32, (n,)))
+        elif self.with_lora:
+            # slot-grouped SGMV units, empty ones padded with length 0
+            f.update(lora_slots=(torch.int32, (B,)), lora_order=(torch.int32, (B,)), lora_t0=(torch.int32, (B,)),
+                     lora_len=(torch.int32, (B,)), lora_slot=(torch.int32, (B,)))
+        return f
+
+    def _views(self, B: int) -> SimpleNamespace:
+        """A bucket's inputs: `dev` tensors, the `host` arrays they are copied
+        from, and the two byte ranges that the copy moves."""
+        if B not in self._inputs:
+            fields = self._fields(B)
+            offsets, total = lay_out(fields.values())
+            dev, host = SimpleNamespace(), SimpleNamespace()
+            for (name, (dtype, shape)), o in zip(fields.items(), offsets):
+                setattr(dev, name, device_view(self._dev, o, dtype, shape))
+                setattr(host, name, device_view(self._host, o, dtype, shape).numpy())
+            self._inputs[B] = SimpleNamespace(dev=dev, host=host, to=self._dev[:total], src=self._host[:total])
+        return self._inputs[B]
+
     def _meta(self, B: int) -> BatchMeta:
+        x = self._views(B).dev
         extra = {}
         if self.seq_tables:
             extra = dict(
-                seq_block_tables=self.block_tables[:B],
+                seq_block_tables=x.block_tables,
                 tok_seq=self.tok_seq[:B],
                 seg_start=self.seg_start[:B],
                 seg_len=self.seg_len[:B],
-                seg_slot=self.seg_slot[:B],
-                seg_fresh=self.seg_fresh[:B],
-                seg_ctx=self.context_lens[:B],
+                seg_slot=x.seg_slot,
+                seg_fresh=x.seg_fresh,
+                seg_ctx=x.context_lens,
                 max_seg_len=1,
+            )
+        if self.with_lora and self.lora_in_layer:
+            extra.update(lora_rows_tok=x.lora_tok, lora_rows_len=x.lora_len, lora_rows_slot=x.lora_slot)
+        elif self.with_lora:
+            extra.update(
+                lora_slot_per_token=x.lora_slots,
+                lora_order=x.lora_order,
+                lora_unit_t0=x.lora_t0,
+                lora_unit_len=x.lora_len,
+                lora_unit_slot=x.lora_slot,
             )
         return BatchMeta(
             **extra,
             num_prefill_tokens=0,
             num_decode_tokens=B,
-            slot_mapping=self.slot_mapping[:B],
-            decode_block_tables=self.block_tables[:B],
-            decode_context_lens=self.context_lens[:B],
-            lora_slot_per_token=self.lora_slots[:B] if self.with_lora else None,
-            lora_order=self.lora_order[:B] if self.with_lora else None,
-            lora_unit_t0=self.lora_ut0[:B] if self.with_lora else None,
-            lora_unit_len=self.lora_ulen[:B] if self.with_lora else None,
-            lora_unit_slot=self.lora_uslot[:B] if self.with_lora else None,
+            slot_mapping=x.slot_mapping,
+            decode_block_tables=x.block_tables,
+            decode_context_lens=x.context_lens,
             lora_ws=self.lora_ws,
-            **self._lora_rows(B),
             decode_nsplits=self._graph_nsplits(B),
-        )
-
-    def _lora_rows(self, B: int) -> dict:
-        """The bucket's row tiles where the model carries LoRA in its layers:
-        as many as B tokens can need, the unused ones empty."""
-        if not (self.with_lora and self.lora_in_layer):
-            return {}
-        n = self._max_rows(B)
-        return dict(
-            lora_rows_tok=self.lora_tok[: n * 16].view(n, 16),
-            lora_rows_len=self.lora_ulen[:n],
-            lora_rows_slot=self.lora_uslot[:n],
         )
 
     def _max_rows(self, B: int) -> int:
@@ -179,7 +165,8 @@ class DecodeGraphRunner:
 
     def _forward(self, B: int) -> torch.Tensor:
         model = self.runner.model
-        hidden = model(self.ids[:B], self.pos[:B], self.runner.kv_caches, self._meta(B))
+        x = self._views(B).dev
+        hidden = model(x.ids, x.pos, self.runner.kv_caches, self._meta(B))
         idx = torch.arange(B, device=self.device)
         return model.compute_logits(hidden, idx).to(self.runner.dtype)
 
@@ -187,12 +174,11 @@ class DecodeGraphRunner:
         self.with_lora = with_lora
         mgr = self.runner.adapter_manager
         self.lora_in_layer = with_lora and getattr(mgr, "in_layer", False)
-        if self.lora_in_layer:
-            n = self._max_rows(self.max_bs) * 16
-            self.lora_tok = torch.zeros(n, dtype=torch.int32, device=self.device)
-            self.h_tok = torch.zeros(n, dtype=torch.int32, pin_memory=True)
-            self.n_tok = self.h_tok.numpy()
-            self.lora_ulen.zero_()  # the tiles of a capture list nothing
+        # one buffer for the inputs of any bucket (the largest needs the most)
+        total = lay_out(self._fields(self.max_bs).values())[1]
+        self._dev = torch.zeros(total, dtype=torch.uint8, device=self.device)
+        self._host = torch.zeros(total, dtype=torch.uint8, pin_memory=True)
+        self._inputs = {}
         if with_lora and self.lora_ws is None:
             self.lora_ws = torch.zeros(
                 self.max_bs, mgr.rank, dtype=mgr.dtype, device=self.device
@@ -211,12 +197,6 @@ class DecodeGraphRunner:
         )
         if max_scratch > 0 and self.device.type == "cuda":
             ops.split_scratch(self.device, max_scratch)
-        # seed static buffers with safe values (padding semantics)
-        self.block_tables.fill_(0)
-        self.block_tables[:, 0] = self.scratch_block
-        self.context_lens.fill_(1)
-        self.slot_mapping.fill_(self.scratch_block * self.block_size)
-        self.lora_slots.fill_(-1)
         torch.cuda.synchronize(self.device)
         # Warmup on a side stream (torch.cuda.graph requirement) — at EVERY
         # capture batch size: hipBLASLt picks its algorithm + allocates its
@@ -229,7 +209,9 @@ class DecodeGraphRunner:
         s.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(s):
             for B in self.sizes:
+                self._fill(B, [], None)  # padding rows only
                 self._forward(B)
+                s.synchronize()  # before the next bucket's rows overwrite the host's
         torch.cuda.current_stream(self.device).wait_stream(s)
         torch.cuda.synchronize(self.device)
         # Graphs of an engine that is no longer referenced sit in reference
@@ -268,67 +250,56 @@ class DecodeGraphRunner:
         decodes,  # List[ScheduledSeq]
         slot_of,  # callable(name) -> int, or None
     ) -> torch.Tensor:
-        """Fill static buffers, replay the right graph, return logits[:n]."""
+        """Fill the bucket's inputs, replay its graph, return logits[:n]."""
         n = len(decodes)
         B = self.pick_size(n)
         assert B is not None
-        bs = self.block_size
-        n_ids, n_pos, n_slot = self.n_ids, self.n_pos, self.n_slot
-        n_bt, n_ctx, n_lora = self.n_bt, self.n_ctx, self.n_lora
-        for i, ss in enumerate(decodes):
-            seq = ss.seq
-            p = seq.num_computed_tokens
-            n_ids[i] = seq.all_token_ids[p]
-            n_pos[i] = p
-            n_slot[i] = seq.block_table[p // bs] * bs + p % bs
-            nb = len(seq.block_table)
-            n_bt[i, :nb] = seq.block_table
-            n_ctx[i] = p + 1
-            if self.with_lora:
-                n_lora[i] = slot_of(seq.lora_name) if seq.lora_name else -1
-            if self.seq_tables:
-                self.n_sslot[i] = max(seq.state_slot, 0)
-                self.n_sfresh[i] = 1 if p == 0 else 0
+        self._fill(B, decodes, slot_of)
+        self.graphs[B].replay()
+        return self.logits[B][:n]
+
+    def _fill(self, B: int, decodes, slot_of) -> None:
+        """The inputs of `decodes`, padding rows behind them, to the device."""
+        n, bs = len(decodes), self.block_size
+        v = self._views(B)
+        x = v.host
+        seqs = [ss.seq for ss in decodes]
+        pos = [q.num_computed_tokens for q in seqs]
+        x.ids[n:] = 0
+        pack_rows([q.tokens(p, p + 1) for q, p in zip(seqs, pos)], x.ids[:n])
+        x.pos[:n] = pos
+        x.pos[n:] = 0
+        x.block_tables[:] = 0  # another bucket's arrays lay here
+        pack_rows([q.block_table for q in seqs], x.block_tables[:n])
+        if any(p // bs >= len(q.block_table) for q, p in zip(seqs, pos)):
+            raise IndexError("a sequence has fewer cache blocks than tokens")
+        x.block_tables[n:, 0] = self.scratch_block
+        at = x.pos // bs
+        x.slot_mapping[:] = x.block_tables[np.arange(B), at].astype(np.int64) * bs + x.pos - at * bs
+        x.context_lens[:] = x.pos + 1
         if self.seq_tables:
-            self.n_sslot[n:B] = self.scratch_slot
-            self.n_sfresh[n:B] = 1
-            self.seg_slot[:B].copy_(self.h_sslot[:B], non_blocking=True)
-            self.seg_fresh[:B].copy_(self.h_sfresh[:B], non_blocking=True)
-        # padding rows
-        if B > n:
-            n_ids[n:B] = 0
-            n_pos[n:B] = 0
-            n_slot[n:B] = self.scratch_block * bs
-            n_bt[n:B, :] = 0
-            n_bt[n:B, 0] = self.scratch_block
-            n_ctx[n:B] = 1
-            n_lora[n:B] = -1
-        self.ids[:B].copy_(self.h_ids[:B], non_blocking=True)
-        self.pos[:B].copy_(self.h_pos[:B], non_blocking=True)
-        self.slot_mapping[:B].copy_(self.h_slot[:B], non_blocking=True)
-        self.block_tables[:B].copy_(self.h_bt[:B], non_blocking=True)
-        self.context_lens[:B].copy_(self.h_ctx[:B], non_blocking=True)
+            x.seg_slot[:n] = [max(q.state_slot, 0) for q in seqs]
+            x.seg_slot[n:] = self.scratch_slot
+            x.seg_fresh[:] = x.pos == 0
         if self.with_lora:
             from ..lora.manager import build_lora_rows, build_lora_units
 
+            slots = np.full(B, -1, dtype=np.int32)
+            of = {name: slot_of(name) if name else -1 for name in {q.lora_name for q in seqs}}
+            slots[:n] = [of[q.lora_name] for q in seqs]
             if self.lora_in_layer:
-                toks, ulen, uslot = build_lora_rows(self.n_lora[:B])
-                u, room = len(ulen), self._max_rows(B)
-                self.n_tok[: u * 16] = toks.reshape(-1)
-                self.lora_tok[: room * 16].copy_(self.h_tok[: room * 16], non_blocking=True)
+                toks, ulen, uslot = build_lora_rows(slots)
+                u = len(ulen)
+                x.lora_tok[:u] = toks
+                x.lora_tok[u:] = 0
             else:
-                order, ut0, ulen, uslot = build_lora_units(self.n_lora[:B])
-                u, room = len(ut0), B
-                self.n_order[:B] = order
-                self.n_ut0[:u] = ut0
-                self.lora_slots[:B].copy_(self.h_lora[:B], non_blocking=True)
-                self.lora_order[:B].copy_(self.h_order[:B], non_blocking=True)
-                self.lora_ut0[:B].copy_(self.h_ut0[:B], non_blocking=True)
-            self.n_ulen[:u] = ulen
-            self.n_ulen[u:room] = 0  # padding tiles or units: no-op in the kernels
-            self.n_uslot[:u] = uslot
-            self.n_uslot[u:room] = -1
-            self.lora_ulen[:room].copy_(self.h_ulen[:room], non_blocking=True)
-            self.lora_uslot[:room].copy_(self.h_uslot[:room], non_blocking=True)
-        self.graphs[B].replay()
-        return self.logits[B][:n]
+                x.lora_slots[:] = slots
+                x.lora_order[:], ut0, ulen, uslot = build_lora_units(slots)
+                u = len(ut0)
+                x.lora_t0[:u] = ut0
+                x.lora_t0[u:] = 0
+            x.lora_len[:u] = ulen
+            x.lora_len[u:] = 0  # padding tiles or units: no-op in the kernels
+            x.lora_slot[:u] = uslot
+            x.lora_slot[u:] = -1
+        v.to.copy_(v.src, non_blocking=True)

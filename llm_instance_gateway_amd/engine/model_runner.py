@@ -3,8 +3,7 @@ execution (batch build → forward → sample).
 
 MI355X notes: the KV cache is sized against the 288 GB HBM3E pool at engine
 init (`determine_num_kv_blocks`); batches are flat/unpadded; all per-step
-index tensors are built on host and copied once (a single H2D per tensor per
-step).
+index tensors are built on host and copied in one piece.
 """
 
 from __future__ import annotations
@@ -12,10 +11,12 @@ from __future__ import annotations
 import logging
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from ..models.config import ModelConfig
 from ..utils.tunableop import eager_tuned
+from .batch_arrays import pack_rows, table_rows, upload
 from .config import EngineConfig
 from .metadata import BatchMeta
 from ..utils.tracing import gpu_range
@@ -178,43 +179,24 @@ class ModelRunner:
             (decodes if ss.num_tokens == 1 else prefills).append(ss)
 
         bs = self.config.block_size
-        input_ids: List[int] = []
-        positions: List[int] = []
-        slots: List[int] = []
+        ordered = prefills + decodes
+        seqs = [ss.seq for ss in ordered]
+        S, n_pre = len(ordered), len(prefills)
+        start = np.array([q.num_computed_tokens for q in seqs], dtype=np.int64)
+        length = np.array([ss.num_tokens for ss in ordered], dtype=np.int64)
+        ctx = start + length
+        first = np.concatenate(([0], np.cumsum(length)))  # a sequence's first flat row
+        rows, ends = first.tolist(), ctx.tolist()
+        T, num_prefill_tokens = rows[-1], rows[n_pre]
+
+        # the sequences whose last known token this step processes: every
+        # decode, and prompts with their final portion
         sample_seqs: List[Sequence] = []
         sample_idx: List[int] = []
-
-        qsl = [0]
-        p_ctx: List[int] = []
-        p_bts: List[List[int]] = []
-        for ss in prefills:
-            seq = ss.seq
-            c, n = seq.num_computed_tokens, ss.num_tokens
-            toks = seq.all_token_ids[c : c + n]
-            input_ids.extend(toks)
-            positions.extend(range(c, c + n))
-            for pos in range(c, c + n):
-                slots.append(seq.block_table[pos // bs] * bs + pos % bs)
-            qsl.append(qsl[-1] + n)
-            p_ctx.append(c + n)
-            p_bts.append(seq.block_table)
-            if c + n == seq.total_len:
-                sample_seqs.append(seq)
-                sample_idx.append(qsl[-1] - 1)
-
-        num_prefill_tokens = len(input_ids)
-        d_ctx: List[int] = []
-        d_bts: List[List[int]] = []
-        for ss in decodes:
-            seq = ss.seq
-            pos = seq.num_computed_tokens  # == total_len - 1
-            input_ids.append(seq.all_token_ids[pos])
-            positions.append(pos)
-            slots.append(seq.block_table[pos // bs] * bs + pos % bs)
-            d_ctx.append(pos + 1)
-            d_bts.append(seq.block_table)
-            sample_seqs.append(seq)
-            sample_idx.append(len(input_ids) - 1)
+        for i, q in enumerate(seqs):
+            if i >= n_pre or ends[i] == q.total_len:
+                sample_seqs.append(q)
+                sample_idx.append(rows[i + 1] - 1)
 
         # GEMM M-bucketing: pad the flat batch tail so every projection GEMM
         # sees M % pad_batch_multiple == 0 (few stable shapes -> hipBLASLt
@@ -227,48 +209,49 @@ class ModelRunner:
             padm > 0
             and self.device.type == "cuda"
             and not self.config.model.is_moe
-            and len(input_ids) % padm != 0
+            and T % padm != 0
         ):
-            num_pad_tokens = padm - len(input_ids) % padm
-            scratch_slot = self.config.num_kv_blocks * bs
-            input_ids.extend([0] * num_pad_tokens)
-            positions.extend([0] * num_pad_tokens)
-            slots.extend([scratch_slot] * num_pad_tokens)
+            num_pad_tokens = padm - T % padm
 
+        # token ids, positions and cache slots of the flat rows, pad rows behind
+        input_ids = np.zeros(T + num_pad_tokens, dtype=np.int64)
+        positions = np.zeros(T + num_pad_tokens, dtype=np.int64)
+        slots = np.full(T + num_pad_tokens, self.config.num_kv_blocks * bs, dtype=np.int64)
+        pack_rows([q.tokens(q.num_computed_tokens, e) for q, e in zip(seqs, ends)], input_ids[:T])
+        tok_seq = np.repeat(np.arange(S, dtype=np.int32), length)
+        positions[:T] = np.arange(T) - (first[:-1] - start)[tok_seq]
+        p_bts = [q.block_table for q in seqs[:n_pre]]
+        d_bts = [q.block_table for q in seqs[n_pre:]]
+        if any(len(q.block_table) * bs < c for q, c in zip(seqs, ends)):
+            raise IndexError("a sequence has fewer cache blocks than tokens")
+        p_tab = table_rows(p_bts) if p_bts else None
+        d_tab = table_rows(d_bts) if d_bts else None
+        for tab, lo, hi in ((p_tab, 0, n_pre), (d_tab, n_pre, S)):
+            if tab is not None:
+                r = slice(rows[lo], rows[hi])
+                pos = positions[r]
+                slots[r] = tab[tok_seq[r] - lo, pos // bs].astype(np.int64) * bs + pos % bs
+
+        # every table of the step goes to the device in one copy at the end
         dev = self.device
+        fields: List[Tuple[str, np.ndarray]] = []
 
-        def pad_tables(bts: List[List[int]]) -> Optional[torch.Tensor]:
-            if not bts:
-                return None
-            m = max(len(b) for b in bts)
-            t = torch.zeros(len(bts), m, dtype=torch.int32)
-            for i, b in enumerate(bts):
-                t[i, : len(b)] = torch.tensor(b, dtype=torch.int32)
-            return t.to(dev, non_blocking=True)
+        def put(name: str, values) -> None:
+            fields.append((name, np.asarray(values, dtype=np.int32)))
 
         meta = BatchMeta(
             num_prefill_tokens=num_prefill_tokens,
             num_decode_tokens=len(decodes),
-            slot_mapping=torch.tensor(slots, dtype=torch.int64).to(dev, non_blocking=True),
-            prefill_query_start_locs=(
-                torch.tensor(qsl, dtype=torch.int32).to(dev, non_blocking=True)
-                if prefills
-                else None
-            ),
-            prefill_context_lens=(
-                torch.tensor(p_ctx, dtype=torch.int32).to(dev, non_blocking=True)
-                if prefills
-                else None
-            ),
-            prefill_block_tables=pad_tables(p_bts),
-            decode_block_tables=pad_tables(d_bts),
-            decode_context_lens=(
-                torch.tensor(d_ctx, dtype=torch.int32).to(dev, non_blocking=True)
-                if decodes
-                else None
-            ),
-            max_decode_ctx=max(d_ctx) if d_ctx else 0,
+            slot_mapping=None,  # these come with the upload below
+            max_decode_ctx=int(ctx[n_pre:].max()) if decodes else 0,
         )
+        if prefills:
+            put("prefill_query_start_locs", first[: n_pre + 1])
+            put("prefill_context_lens", ctx[:n_pre])
+            put("prefill_block_tables", p_tab)
+        if decodes:
+            put("decode_block_tables", d_tab)
+            put("decode_context_lens", ctx[n_pre:])
         # Per-token prefill expansion, once per step (the attention layers of
         # every transformer block reuse it; see profiles/r01_bench_kernel_stats.md).
         if prefills:
@@ -281,127 +264,68 @@ class ModelRunner:
                 )
             if use_mfma:
                 # 64-row query tiles for the MFMA flash-prefill kernel.
-                ts: List[int] = []
-                tq: List[int] = []
-                for si, ss in enumerate(prefills):
-                    for qb in range(0, ss.num_tokens, 64):
-                        ts.append(si)
-                        tq.append(qb)
-                meta.prefill_tile_seq = torch.tensor(ts, dtype=torch.int32).to(
-                    dev, non_blocking=True
-                )
-                meta.prefill_tile_qstart = torch.tensor(tq, dtype=torch.int32).to(
-                    dev, non_blocking=True
-                )
+                tiles = (length[:n_pre] + 63) // 64
+                ts = np.repeat(np.arange(n_pre), tiles)
+                put("prefill_tile_seq", ts)
+                put("prefill_tile_qstart", (np.arange(len(ts)) - np.repeat(np.cumsum(tiles) - tiles, tiles)) * 64)
             elif not getattr(self.model, "needs_seq_tables", False):
-                ctx_tok: List[int] = []
-                n_per: List[int] = []
-                for ss in prefills:
-                    c, n = ss.seq.num_computed_tokens, ss.num_tokens
-                    ctx_tok.extend(range(c + 1, c + n + 1))
-                    n_per.append(n)
-                meta.prefill_tok_context_lens = torch.tensor(
-                    ctx_tok, dtype=torch.int32
-                ).to(dev, non_blocking=True)
-                meta.prefill_tok_block_tables = torch.repeat_interleave(
-                    meta.prefill_block_tables,
-                    torch.tensor(n_per, dtype=torch.int64, device=dev),
-                    dim=0,
-                ).contiguous()
+                put("prefill_tok_context_lens", positions[:num_prefill_tokens] + 1)
+                put("prefill_tok_block_tables", p_tab[tok_seq[:num_prefill_tokens]])
 
         # multi-LoRA: per-token adapter slot ids (-1 = base model only)
         mgr = getattr(self, "adapter_manager", None)
         if mgr is not None and any(ss.seq.lora_name for ss in prefills + decodes):
-            slots: List[int] = []
-            # prefill tokens are sequence-contiguous: emit 64-token segment
-            # tiles per same-slot run for the MFMA SGMV path
-            t0s: List[int] = []
-            tlens: List[int] = []
-            tslots: List[int] = []
-            for ss in prefills:
-                s_id = mgr.slot_of(ss.seq.lora_name)
-                base = len(slots)
-                slots.extend([s_id] * ss.num_tokens)
-                if s_id >= 0:
-                    for off in range(0, ss.num_tokens, 64):
-                        t0s.append(base + off)
-                        tlens.append(min(64, ss.num_tokens - off))
-                        tslots.append(s_id)
-            for ss in decodes:
-                slots.append(mgr.slot_of(ss.seq.lora_name))
-            if num_pad_tokens:
-                slots.extend([-1] * num_pad_tokens)  # pad rows: base model only
-            meta.lora_slot_per_token = torch.tensor(slots, dtype=torch.int32).to(
-                dev, non_blocking=True
-            )
+            slot = {name: mgr.slot_of(name) for name in {q.lora_name for q in seqs}}
+            seq_slot = np.array([slot[q.lora_name] for q in seqs], dtype=np.int32)
+            lora_slots = np.full(T + num_pad_tokens, -1, dtype=np.int32)  # pad rows: base model only
+            lora_slots[:T] = seq_slot[tok_seq]
+            put("lora_slot_per_token", lora_slots)
             if getattr(mgr, "in_layer", False):
                 # row tiles over the whole batch (lora/manager.py::build_lora_rows)
                 from ..lora.manager import build_lora_rows
 
-                arrays = build_lora_rows(slots)
-                meta.lora_rows_tok, meta.lora_rows_len, meta.lora_rows_slot = (
-                    torch.from_numpy(a).to(dev, non_blocking=True) for a in arrays
-                )
+                for name, a in zip(("tok", "len", "slot"), build_lora_rows(lora_slots)):
+                    put("lora_rows_" + name, a)
             elif self.device.type == "cuda":
                 # slot-grouped SGMV units (lora/manager.py::build_lora_units)
                 from ..lora.manager import build_lora_units
 
-                order, ut0, ulen, uslot = build_lora_units(slots)
-                if len(ut0):
-                    meta.lora_order = torch.from_numpy(order).to(dev, non_blocking=True)
-                    meta.lora_unit_t0 = torch.from_numpy(ut0).to(dev, non_blocking=True)
-                    meta.lora_unit_len = torch.from_numpy(ulen).to(dev, non_blocking=True)
-                    meta.lora_unit_slot = torch.from_numpy(uslot).to(dev, non_blocking=True)
-            if t0s:
-                meta.lora_tile_t0 = torch.tensor(t0s, dtype=torch.int32).to(
-                    dev, non_blocking=True
-                )
-                meta.lora_tile_len = torch.tensor(tlens, dtype=torch.int32).to(
-                    dev, non_blocking=True
-                )
-                meta.lora_tile_slot = torch.tensor(tslots, dtype=torch.int32).to(
-                    dev, non_blocking=True
-                )
+                order, *units = build_lora_units(lora_slots)
+                if len(units[0]):
+                    put("lora_order", order)
+                    for name, a in zip(("t0", "len", "slot"), units):
+                        put("lora_unit_" + name, a)
+            # prefill tokens are sequence-contiguous: 64-token segment tiles
+            # per same-slot run for the MFMA SGMV path
+            on = np.flatnonzero(seq_slot[:n_pre] >= 0)
+            if len(on):
+                tiles = (length[on] + 63) // 64
+                of = np.repeat(on, tiles)
+                off = (np.arange(len(of)) - np.repeat(np.cumsum(tiles) - tiles, tiles)) * 64
+                put("lora_tile_t0", first[of] + off)
+                put("lora_tile_len", np.minimum(64, length[of] - off))
+                put("lora_tile_slot", seq_slot[of])
 
-        ordered = prefills + decodes
         # first flat row of every scheduled sequence (replay reads logits at
         # offsets from it)
-        self._row_start = {}
-        r0 = 0
-        for ss in ordered:
-            self._row_start[ss.seq.seq_id] = r0
-            r0 += ss.num_tokens
+        self._row_start = {q.seq_id: r for q, r in zip(seqs, rows)}
         if getattr(self.model, "needs_seq_tables", False):
             # Per-token / per-sequence addressing for general-size attention
             # and recurrent layers: one block-table row and one segment per
             # scheduled sequence, prefill portions first, then decodes.
-            tok_seq: List[int] = []
-            s_start: List[int] = []
-            s_len: List[int] = []
-            s_slot: List[int] = []
-            s_fresh: List[int] = []
-            s_ctx: List[int] = []
-            for si, ss in enumerate(ordered):
-                s_ctx.append(ss.seq.num_computed_tokens + ss.num_tokens)
-                s_start.append(len(tok_seq))
-                s_len.append(ss.num_tokens)
-                s_slot.append(max(ss.seq.state_slot, 0))
-                s_fresh.append(1 if ss.seq.num_computed_tokens == 0 else 0)
-                tok_seq.extend([si] * ss.num_tokens)
-            tok_seq.extend([-1] * num_pad_tokens)
+            put("seq_block_tables", table_rows(p_bts + d_bts))
+            put("tok_seq", np.concatenate((tok_seq, np.full(num_pad_tokens, -1, dtype=np.int32))))
+            put("seg_start", first[:-1])
+            put("seg_len", length)
+            put("seg_slot", [max(q.state_slot, 0) for q in seqs])
+            put("seg_fresh", start == 0)
+            put("seg_ctx", ctx)
+            meta.max_seg_len = int(length.max()) if S else 0
 
-            def i32(v: List[int]) -> torch.Tensor:
-                return torch.tensor(v, dtype=torch.int32).to(dev, non_blocking=True)
-
-            meta.seq_block_tables = pad_tables(p_bts + d_bts)
-            meta.tok_seq = i32(tok_seq)
-            meta.seg_start, meta.seg_len = i32(s_start), i32(s_len)
-            meta.seg_slot, meta.seg_fresh = i32(s_slot), i32(s_fresh)
-            meta.seg_ctx = i32(s_ctx)
-            meta.max_seg_len = max(s_len) if s_len else 0
-
-        ids_t = torch.tensor(input_ids, dtype=torch.int64).to(dev, non_blocking=True)
-        pos_t = torch.tensor(positions, dtype=torch.int64).to(dev, non_blocking=True)
+        ids_t, pos_t, meta.slot_mapping, *tables = upload(
+            [input_ids, positions, slots] + [a for _, a in fields], dev)
+        for (name, _), t in zip(fields, tables):
+            setattr(meta, name, t)
         return ids_t, pos_t, meta, sample_seqs, sample_idx, ordered
 
     # -- one step --------------------------------------------------------------

@@ -123,6 +123,15 @@ class Sequence:
     def all_token_ids(self) -> List[int]:
         return self.prompt_token_ids + self.output_token_ids
 
+    def tokens(self, start: int, end: int) -> List[int]:
+        """all_token_ids[start:end] without joining the two lists."""
+        p = len(self.prompt_token_ids)
+        if end <= p:
+            return self.prompt_token_ids[start:end]
+        if start >= p:
+            return self.output_token_ids[start - p : end - p]
+        return self.prompt_token_ids[start:] + self.output_token_ids[: end - p]
+
     def next_chunk_tokens(self, budget: int) -> int:
         """How many tokens the next prefill chunk would process (the final
         chunk includes the last known token, whose logit is sampled)."""

@@ -8,6 +8,7 @@
 #include <optional>
 
 #include <torch/extension.h>
+#include <pybind11/numpy.h>
 
 #include "common.h"
 
@@ -586,6 +587,44 @@ void lora_qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
 
 }  // namespace
 
+// Row i of `rows` (whole numbers) to out[i, :len], or one after another into a
+// one-dimensional `out` (int32 or int64).
+namespace py = pybind11;
+
+template <typename I>
+static void pack_rows_as(const py::sequence& rows, py::array& out) {
+  const bool flat = out.ndim() == 1;
+  const ssize_t n = py::len(rows), width = flat ? out.shape(0) : out.shape(1);
+  TORCH_CHECK(flat || n <= out.shape(0), "more rows than room");
+  I* dst = (I*)out.mutable_data();
+  ssize_t at = 0;
+  for (ssize_t i = 0; i < n; ++i) {
+    const py::object row =
+        py::reinterpret_steal<py::object>(PySequence_Fast(py::object(rows[i]).ptr(), "a row is a list"));
+    if (!row) throw py::error_already_set();
+    const ssize_t len = PySequence_Fast_GET_SIZE(row.ptr());
+    I* to = flat ? dst + at : dst + i * width;
+    TORCH_CHECK(len <= width - (flat ? at : 0), "a row of ", len, " numbers is longer than its room");
+    for (ssize_t j = 0; j < len; ++j) {
+      PyObject* e = PySequence_Fast_GET_ITEM(row.ptr(), j);
+      const long long v = PyLong_Check(e) ? PyLong_AsLongLong(e)
+                                          : py::reinterpret_borrow<py::object>(e).cast<long long>();
+      if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
+      TORCH_CHECK(v == (long long)(I)v, v, " does not fit");
+      to[j] = (I)v;
+    }
+    at += len;
+  }
+  TORCH_CHECK(!flat || at == width, at, " numbers for ", width, " places");
+}
+
+static void pack_rows(py::sequence rows, py::array out) {
+  TORCH_CHECK((out.ndim() == 1 || out.ndim() == 2) && (out.flags() & py::array::c_style), "1-d or 2-d in row order");
+  if (py::isinstance<py::array_t<int32_t>>(out)) pack_rows_as<int32_t>(rows, out);
+  else if (py::isinstance<py::array_t<int64_t>>(out)) pack_rows_as<int64_t>(rows, out);
+  else TORCH_CHECK(false, "int32 or int64");
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "MI355X (gfx950) native kernels for llm_instance_gateway_amd";
   m.def("rms_norm", &rms_norm);
@@ -611,6 +650,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lora_shrink_strip", &lig_lora_shrink_strip);
   m.def("lora_shrink", &lora_shrink);
   m.def("lora_qkv_rope_cache", &lora_qkv_rope_cache);
+  m.def("pack_rows", &pack_rows);
   m.def("mfma_probe", [](torch::Tensor out, torch::Tensor a, torch::Tensor b,
                          int64_t stream) {
     TORCH_CHECK(out.scalar_type() == torch::kFloat32);

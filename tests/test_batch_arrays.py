@@ -1,0 +1,96 @@
+"""Host arrays of a step against the plain per-token construction."""
+
+import numpy as np
+import pytest
+import torch
+
+from llm_instance_gateway_amd import ops
+from llm_instance_gateway_amd.engine import batch_arrays as ba
+from llm_instance_gateway_amd.engine.sequence import Sequence
+
+CPU = torch.device("cpu")
+
+
+@pytest.fixture(params=["native", "numpy"])
+def path(request, monkeypatch):
+    if request.param == "numpy":
+        monkeypatch.setattr(ops, "_load_ext", lambda: None)
+    elif ops._load_ext() is None:
+        pytest.skip("extension not built")
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_pack_rows(path, dtype):
+    rows = [[3, 1, 2**31 - 1], [], [7], [np.int64(5), -1, 0, 9]]
+    out = np.full((5, 4), -7, dtype=dtype)
+    ba.pack_rows(rows, out)
+    assert out.tolist() == [[3, 1, 2**31 - 1, -7], [-7] * 4, [7, -7, -7, -7], [5, -1, 0, 9], [-7] * 4]
+    flat = np.zeros(8, dtype=dtype)
+    ba.pack_rows(rows, flat)
+    assert flat.tolist() == [3, 1, 2**31 - 1, 7, 5, -1, 0, 9]
+    assert ba.table_rows(rows).tolist() == [[3, 1, 2**31 - 1, 0], [0] * 4, [7, 0, 0, 0], [5, -1, 0, 9]]
+
+
+@pytest.mark.parametrize("rows,shape", [
+    ([[1, 2, 3]], (1, 2)), ([[1], [2]], (1, 2)), ([[1, 2]], (3,)), ([[1, 2], [3, 4]], (3,)),
+    ([[2**31]], (1, 1)), ([["a"]], (1, 1)), ([5], (1, 1)),
+])
+def test_pack_rows_refuses(path, rows, shape):
+    with pytest.raises(Exception):
+        ba.pack_rows(rows, np.zeros(shape, dtype=np.int32))
+
+
+def test_upload_keeps_values_and_alignment():
+    arrays = [np.arange(3, dtype=np.int64), np.zeros((0, 4), np.int32), np.arange(10, dtype=np.int32).reshape(5, 2),
+              np.arange(12, dtype=np.int32).reshape(3, 4).T, np.array([9], dtype=np.int64)]
+    got = ba.upload(arrays, CPU)
+    for a, t in zip(arrays, got):
+        assert t.numpy().dtype == a.dtype and t.tolist() == a.tolist() and t.is_contiguous()
+        assert (t.data_ptr() - got[0].data_ptr()) % ba.ALIGN == 0
+
+
+@pytest.mark.parametrize("out", [0, 4])
+def test_sequence_tokens(out):
+    s = Sequence([1, 2, 3])
+    s.output_token_ids = list(range(10, 10 + out))
+    for a in range(3 + out + 1):
+        for b in range(a, 3 + out + 1):
+            assert s.tokens(a, b) == s.all_token_ids[a:b]
+
+
+def test_build_batch_matches_per_token_construction():
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine
+    from llm_instance_gateway_amd.engine.scheduler import ScheduledSeq
+    from llm_instance_gateway_amd.models.config import get_model_config
+
+    eng = LLMEngine(EngineConfig(model=get_model_config("tiny"), num_kv_blocks=64, max_num_seqs=8,
+                                 max_num_batched_tokens=256, max_model_len=256), device="cpu")
+    r, bs = eng.runner, eng.config.block_size if hasattr(eng, "config") else eng.runner.config.block_size
+    blocks = iter(range(63, 0, -1))
+    sched, order = [], []
+    for cached, n, extra in ((0, 1, 0), (0, 5, 0), (bs, bs + 1, 3), (2 * bs - 1, 1, 0), (3, bs, 0), (bs, 1, 7)):
+        s = Sequence(list(range(100, 100 + cached + n + extra)))
+        s.num_computed_tokens = cached
+        s.block_table = [next(blocks) for _ in range(-(-(cached + n + extra) // bs))]
+        sched.append(ScheduledSeq(s, n))
+    ids, pos, meta, seqs, idx, ordered = r._build_batch(sched)
+    order = [x for x in sched if x.num_tokens > 1] + [x for x in sched if x.num_tokens == 1]
+    assert [x.seq for x in ordered] == [x.seq for x in order]
+    want = [(x.seq, p) for x in order for p in range(x.seq.num_computed_tokens, x.seq.num_computed_tokens + x.num_tokens)]
+    assert ids.tolist() == [s.all_token_ids[p] for s, p in want] and pos.tolist() == [p for _, p in want]
+    assert meta.slot_mapping.tolist() == [s.block_table[p // bs] * bs + p % bs for s, p in want]
+    assert meta.num_prefill_tokens == 5 + bs + 1 + bs and meta.num_decode_tokens == 3
+    assert meta.prefill_query_start_locs.tolist() == [0, 5, 6 + bs, 6 + 2 * bs]
+    assert meta.prefill_context_lens.tolist() == [5, 2 * bs + 1, 3 + bs]
+    assert meta.decode_context_lens.tolist() == [1, 2 * bs, bs + 1] and meta.max_decode_ctx == 2 * bs
+    for tab, part in ((meta.prefill_block_tables, order[:3]), (meta.decode_block_tables, order[3:])):
+        w = max(len(x.seq.block_table) for x in part)
+        assert tab.tolist() == [x.seq.block_table + [0] * (w - len(x.seq.block_table)) for x in part]
+    # a prompt's unfinished portion samples nothing, every one-token row does
+    done = [i for i, x in enumerate(order) if x.num_tokens == 1 or x.seq.num_computed_tokens + x.num_tokens == x.seq.total_len]
+    assert seqs == [order[i].seq for i in done]
+    assert [ids[i].item() for i in idx] == [
+        s.all_token_ids[x.seq.num_computed_tokens + x.num_tokens - 1] for s, x in ((order[i].seq, order[i]) for i in done)]
+    sched[0].seq.block_table = []
+    with pytest.raises(IndexError):
+        r._build_batch(sched)
