@@ -167,6 +167,8 @@ class DecodeGraphRunner:
         model = self.runner.model
         x = self._views(B).dev
         hidden = model(x.ids, x.pos, self.runner.kv_caches, self._meta(B))
+        if hasattr(model, "head_logits"):
+            return model.head_logits(hidden).to(self.runner.dtype)
         idx = torch.arange(B, device=self.device)
         return model.compute_logits(hidden, idx).to(self.runner.dtype)
 

@@ -449,7 +449,7 @@ class ModelRunner:
                 ):
                     sampled[seq.seq_id] = tok
             d_seqs = [ss.seq for ss in decodes]
-            for seq, tok in zip(d_seqs, sample_tokens(logits_d.float(), d_seqs)):
+            for seq, tok in zip(d_seqs, sample_tokens(logits_d, d_seqs)):
                 sampled[seq.seq_id] = tok
         for ss in out.scheduled:
             ss.seq.num_computed_tokens += ss.num_tokens
@@ -475,7 +475,7 @@ class ModelRunner:
         )
         logits = gr.run(decodes, slot_of)
         seqs = [ss.seq for ss in decodes]
-        tokens = sample_tokens(logits.float(), seqs)
+        tokens = sample_tokens(logits, seqs)
         for ss in decodes:
             ss.seq.num_computed_tokens += 1
         return {seq.seq_id: tok for seq, tok in zip(seqs, tokens)}

@@ -6,7 +6,7 @@ with vLLM-style presence/frequency/repetition penalties and OpenAI
 (The reference delegates sampling to vLLM; this owns it natively.)
 
 The common serving fast path (all-greedy, no penalties, no logprobs — the
-benchmark workload) stays one batched argmax; every extension below is
+benchmark workload) stays one batched argmax over the logits as the head wrote them; every extension below is
 skipped unless some sequence in the batch asks for it.
 """
 
@@ -16,6 +16,7 @@ from typing import List
 
 import torch
 
+from ..ops import argmax_rows
 from .sequence import Sequence
 
 
@@ -76,13 +77,14 @@ def _record_logprobs(row: torch.Tensor, chosen: int, seq: Sequence) -> None:
 
 @torch.no_grad()
 def sample_tokens(logits: torch.Tensor, seqs: List[Sequence]) -> List[int]:
-    """logits: [N, vocab] fp32 — one row per sampling sequence."""
+    """logits: [N, vocab], fp32 or the model's dtype — one row per sampling sequence."""
     assert logits.shape[0] == len(seqs)
     if all(
         s.sampling.temperature == 0.0 and not _wants_extras(s.sampling)
         for s in seqs
     ):
-        return logits.argmax(dim=-1).tolist()
+        return argmax_rows(logits).tolist()
+    logits = logits.float()
     out: List[int] = []
     for i, seq in enumerate(seqs):
         sp = seq.sampling

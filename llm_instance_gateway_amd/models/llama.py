@@ -264,12 +264,14 @@ class LlamaForCausalLM(nn.Module):
         return ops.lora_rms_norm(
             y, residual, self.norm, self.cfg.rms_norm_eps, rows, u_down, b[(last, "down")])[0]
 
-    def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
-        """Logits only at the sampled positions (last token of each finished
-        chunk / each decode)."""
-        h = hidden[indices]
+    def head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        """Logits of all rows, as the product leaves them."""
         w = self.embed_tokens.weight if self.lm_head is None else self.lm_head.weight
         # hidden is replicated across the TP group (each block ends in an
         # all-reduce), so every rank computes identical full-vocab logits.
-        logits = h @ w.t()
-        return logits.float()
+        return hidden @ w.t()
+
+    def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
+        """fp32 logits only at the sampled positions (last token of each
+        finished chunk / each decode)."""
+        return self.head_logits(hidden[indices]).float()

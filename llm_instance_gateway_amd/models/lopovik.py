@@ -225,5 +225,8 @@ class LopovikForCausalLM(nn.Module):
             x = ops.residual_add(x.clone() if x is x0 else x, *pending)
         return ops.offset_rms_norm(x, self.final_norm, eps)
 
+    def head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        return hidden @ self.embed.t()
+
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
-        return (hidden[indices] @ self.embed.t()).float()
+        return self.head_logits(hidden[indices]).float()

@@ -252,7 +252,8 @@ class MixtralForCausalLM(nn.Module):
         hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
+    def head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        return hidden @ self.lm_head.weight.t()
+
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
-        h = hidden[indices]
-        logits = h @ self.lm_head.weight.t()
-        return logits.float()
+        return self.head_logits(hidden[indices]).float()

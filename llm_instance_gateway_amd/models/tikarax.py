@@ -200,5 +200,8 @@ class TikaraxForCausalLM(nn.Module):
                 self.capture_residuals.append(x.clone())
         return h  # final-normed hidden states
 
+    def head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        return hidden @ self.head.t()
+
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
-        return (hidden[indices] @ self.head.t()).float()
+        return self.head_logits(hidden[indices]).float()

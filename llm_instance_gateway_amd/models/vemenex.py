@@ -280,5 +280,8 @@ class VemenexForCausalLM(nn.Module):
                 self.capture_residuals.append(xs.sum(dim=1))
         return step(self.final_port)
 
+    def head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        return hidden @ self.head.t()
+
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
-        return (hidden[indices] @ self.head.t()).float()
+        return self.head_logits(hidden[indices]).float()

@@ -304,6 +304,16 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_and_mul(x)
 
 
+def argmax_rows(x: torch.Tensor) -> torch.Tensor:
+    """x.argmax(-1) of [N, V]; the first of equals."""
+    if (x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float32) and 0 < x.shape[1] < 2**31 - 1024
+            and x.stride(1) == 1 and _use_native(x)):
+        out = torch.empty(x.shape[0], dtype=torch.int64, device=x.device)
+        _EXT.argmax_rows(out, x, _stream())
+        return out
+    return x.argmax(dim=-1)
+
+
 build_cos_sin_cache = torch_ref.build_cos_sin_cache
 
 

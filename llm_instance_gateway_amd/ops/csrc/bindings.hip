@@ -46,6 +46,7 @@ void lig_qkv_rope_cache_launch(uint16_t*, const uint16_t*, const int64_t*,
                                const float*, uint16_t*, uint16_t*,
                                const int64_t*, int, int, int, int, int,
                                hipStream_t);
+void lig_argmax_rows_launch(const void*, bool, long, int, int, int64_t*, hipStream_t);
 void lig_silu_and_mul_launch(uint16_t*, const uint16_t*, int, int,
                              hipStream_t);
 void lig_paged_attention_decode_launch(
@@ -202,6 +203,18 @@ void qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
                             cos_sin.data_ptr<float>(), bf16_ptr(k_cache),
                             bf16_ptr(v_cache), slot_mapping.data_ptr<int64_t>(),
                             T, Hq, Hkv, D, BS, as_stream(stream));
+}
+
+void argmax_rows(torch::Tensor out, torch::Tensor x, int64_t stream) {
+  const bool bf16 = x.scalar_type() == torch::kBFloat16;
+  TORCH_CHECK(x.is_cuda() && (bf16 || x.scalar_type() == torch::kFloat32), "bf16 or fp32 rows on the device");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.size(1) > 0 && x.size(1) < (1L << 31) - 1024 &&
+                  x.size(0) < (1L << 31),
+              "[N, V] rows");
+  TORCH_CHECK(out.is_cuda() && out.scalar_type() == torch::kInt64 && out.is_contiguous() && out.dim() == 1 &&
+              out.size(0) == x.size(0));
+  lig_argmax_rows_launch(x.data_ptr(), bf16, x.stride(0), (int)x.size(0), (int)x.size(1), out.data_ptr<int64_t>(),
+                         as_stream(stream));
 }
 
 void silu_and_mul(torch::Tensor out, torch::Tensor x, int64_t stream) {
@@ -633,6 +646,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("reshape_and_cache", &reshape_and_cache);
   m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
+  m.def("argmax_rows", &argmax_rows);
   m.def("paged_attention_decode", &paged_attention_decode);
   m.def("paged_attention_decode_split", &paged_attention_decode_split);
   m.def("paged_attention_prefill", &paged_attention_prefill);
