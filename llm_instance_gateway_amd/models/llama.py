@@ -208,12 +208,49 @@ class LlamaForCausalLM(nn.Module):
         hidden = self.embed_tokens(input_ids)
         if meta.lora_rows_tok is not None:
             return self._forward_lora(hidden, positions, kv_caches, meta)
+        if hidden.shape[0] == 1 and meta.lora_slot_per_token is None and self._row_products():
+            return self._forward_row(hidden, positions, kv_caches, meta)
         residual = None
         for layer, kv in zip(self.layers, kv_caches):
             hidden, residual = layer(
                 hidden, residual, positions, kv, meta, self.cos_sin_cache
             )
         hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
+        return hidden
+
+    def _row_products(self) -> bool:
+        """Whether every projection of a layer is one that `ops.row_product` serves."""
+        if self.tp is not None:
+            return False
+        return all(
+            type(m) is nn.Linear and m.bias is None and ops.row_product_serves(m.weight, norm)
+            for layer in self.layers
+            for m, norm in (
+                (layer.self_attn.qkv_proj, True),
+                (layer.self_attn.o_proj, False),
+                (layer.mlp.gate_up_proj, True),
+                (layer.mlp.down_proj, False),
+            )
+        )
+
+    def _forward_row(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
+        """The layers for a single token: norms and the activation live in the
+        projections' kernels."""
+        residual, x = None, hidden
+        for layer, kv in zip(self.layers, kv_caches):
+            attn, mlp = layer.self_attn, layer.mlp
+            if residual is None:
+                qkv = ops.row_product(x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps)
+                residual = x
+            else:
+                qkv, residual = ops.row_product(x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps, residual)
+            q = ops.qkv_rope_cache(
+                qkv, positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping, attn.num_heads)
+            o = ops.row_product(attn.attend(q, kv, meta), attn.o_proj.weight)
+            act, residual = ops.row_product(
+                o, mlp.gate_up_proj.weight, layer.post_attention_layernorm, layer.eps, residual, silu=True)
+            x = ops.row_product(act, mlp.down_proj.weight)
+        hidden, _ = ops.fused_add_rms_norm(x, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
     def lora_in_layer(self, rank: int, dims: dict) -> bool:

@@ -304,6 +304,28 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_and_mul(x)
 
 
+def row_product_serves(weight: torch.Tensor, norm: bool) -> bool:
+    """Whether `row_product` takes a projection's weight."""
+    return (
+        weight.dtype == torch.bfloat16
+        and weight.is_contiguous()
+        and weight.data_ptr() % 16 == 0
+        and weight.shape[1] % 512 == 0
+        and _use_native(weight)
+        and weight.shape[1] <= _load_ext().row_product_max(norm)
+    )
+
+
+def row_product(x, weight, norm=None, eps=0.0, residual=None, silu=False):
+    """weight @ h of one row x [1, K]: h = x, or rms_norm(x + residual) * norm;
+    with silu, silu(gate) * up of the product's halves.  Returns the product and,
+    where a residual was given, x + residual."""
+    y = torch.empty(1, weight.shape[0] // (2 if silu else 1), dtype=x.dtype, device=x.device)
+    out = None if residual is None else torch.empty_like(residual)
+    _EXT.row_product(y, weight, x, residual, out, norm, eps, silu, _stream())
+    return y if out is None else (y, out)
+
+
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:
     """x.argmax(-1) of [N, V]; the first of equals."""
     if (x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float32) and 0 < x.shape[1] < 2**31 - 1024

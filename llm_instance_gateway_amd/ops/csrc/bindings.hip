@@ -46,6 +46,9 @@ void lig_qkv_rope_cache_launch(uint16_t*, const uint16_t*, const int64_t*,
                                const float*, uint16_t*, uint16_t*,
                                const int64_t*, int, int, int, int, int,
                                hipStream_t);
+int lig_row_product_max(bool);
+void lig_row_product_launch(uint16_t*, const uint16_t*, int, int, const uint16_t*, const uint16_t*, uint16_t*,
+                            const uint16_t*, float, bool, hipStream_t);
 void lig_argmax_rows_launch(const void*, bool, long, int, int, int64_t*, hipStream_t);
 void lig_silu_and_mul_launch(uint16_t*, const uint16_t*, int, int,
                              hipStream_t);
@@ -203,6 +206,27 @@ void qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
                             cos_sin.data_ptr<float>(), bf16_ptr(k_cache),
                             bf16_ptr(v_cache), slot_mapping.data_ptr<int64_t>(),
                             T, Hq, Hkv, D, BS, as_stream(stream));
+}
+
+// y = W h of one row: h = x, or the norm of x (+ residual, whose sum goes to
+// residual_out) with `weight`; silu: W = [gate | up], y = silu(gate h) * (up h).
+void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optional<torch::Tensor> residual,
+                 c10::optional<torch::Tensor> residual_out, c10::optional<torch::Tensor> weight, double eps, bool silu,
+                 int64_t stream) {
+  TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && w.size(0) < (1 << 30));
+  const int N = (int)w.size(0), K = (int)w.size(1);
+  TORCH_CHECK(K > 0 && K % 512 == 0 && K <= lig_row_product_max(weight.has_value()), "width ", K);
+  TORCH_CHECK(N > 0 && (!silu || (N % 2 == 0 && weight.has_value())));
+  auto row = [&](torch::Tensor t, int n) {
+    TORCH_CHECK(t.is_contiguous() && t.numel() == n && ((uintptr_t)t.data_ptr() & 15) == 0, "a contiguous row of ", n);
+    return bf16_ptr(t);
+  };
+  TORCH_CHECK(residual.has_value() == residual_out.has_value() && (weight.has_value() || !residual.has_value()));
+  TORCH_CHECK(((uintptr_t)w.data_ptr() & 15) == 0);
+  TORCH_CHECK(y.is_contiguous() && y.numel() == (silu ? N / 2 : N));
+  lig_row_product_launch(bf16_ptr(y), bf16_cptr(w), N, K, row(x, K), residual ? row(*residual, K) : nullptr,
+                         residual_out ? row(*residual_out, K) : nullptr, weight ? row(*weight, K) : nullptr, (float)eps,
+                         silu, as_stream(stream));
 }
 
 void argmax_rows(torch::Tensor out, torch::Tensor x, int64_t stream) {
@@ -647,6 +671,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("argmax_rows", &argmax_rows);
+  m.def("row_product", &row_product);
+  m.def("row_product_max", &lig_row_product_max);
   m.def("paged_attention_decode", &paged_attention_decode);
   m.def("paged_attention_decode_split", &paged_attention_decode_split);
   m.def("paged_attention_prefill", &paged_attention_prefill);

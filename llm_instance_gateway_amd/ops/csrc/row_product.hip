@@ -1,0 +1,157 @@
+// Projections of a single token, gfx950, bf16: y = W h for one row h, with the
+// norm before it and the activation behind it in the same kernel.
+//
+// Bound by streaming W once.  A wave takes two rows of W and keeps eight to
+// sixteen 16-byte loads a lane on their way, the first of them issued before h
+// is ready; h is formed by every workgroup for itself in LDS (24 KB from the
+// L2 against 64 KB and more of W) and shared by its waves.
+//   norm: residual' = x + residual, h = rms_norm(residual') * weight, as
+//         fused_add_rms_norm (the norm over the unrounded sum); the first
+//         workgroup writes residual' to a place of its own, since the others
+//         may still read the old one.
+//   silu: the two rows are a gate and its up row, y = silu(gate) * up of both
+//         rounded to bf16, as silu_and_mul after the projection.
+// Widths of Llama-3-8B, weights not in any cache, against the library's product
+// with the norm and activation as kernels of their own: norm + qkv 14.3 us (18.5),
+// o 8.2 (13.0), norm + gate_up + silu 45.7 (69.2, now 5.1 TB/s), down 25.5 (26.5).
+#include "common.h"
+
+namespace {
+
+constexpr int NORM_MAX = 8192;  // columns of a row with a norm
+constexpr int PLAIN_MAX = 16384;
+constexpr int U = 4;  // loads of a row per batch, 512 columns each
+
+template <int NTHR, bool NORM, bool SILU>
+__global__ __launch_bounds__(NTHR) void row_product_kernel(
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ w, const int N, const int K, const uint16_t* __restrict__ x,
+    const uint16_t* __restrict__ residual, uint16_t* __restrict__ residual_out, const uint16_t* __restrict__ weight,
+    const float eps) {
+  constexpr int NW = NTHR / WAVE_SIZE, MAXC = NORM_MAX / 8 / NTHR;
+  extern __shared__ __align__(16) uint16_t h[];  // [K]
+  __shared__ float part[NW];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // outputs, of which a wave makes two (one from two rows with SILU)
+  const int outs = SILU ? N / 2 : N;
+  const int n0 = (blockIdx.x * NW + wave) * (SILU ? 1 : 2);
+  const int ra = min(n0, outs - 1), rb = SILU ? ra + outs : min(n0 + 1, outs - 1);
+  const uint16_t* wr[2] = {w + (size_t)ra * K + lane * 8, w + (size_t)rb * K + lane * 8};
+  const int batches = (K / 512 + U - 1) / U;
+
+  u16x8 buf[2][U][2];
+  auto load = [&](int b, int batch) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int c = min((batch * U + i) * 512, K - 512);  // past the end: the last columns again, unused
+#pragma unroll
+      for (int r = 0; r < 2; ++r) buf[b][i][r] = *reinterpret_cast<const u16x8*>(wr[r] + c);
+    }
+  };
+  load(0, 0);
+  load(1, 1);
+
+  // ---- h ------------------------------------------------------------------------
+  const int chunks = K / 8;
+  if (NORM) {
+    f32x8 v[MAXC];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < MAXC; ++j) {
+      const int c = tid + j * NTHR;
+      if (j * NTHR >= chunks) break;
+      if (c < chunks) {
+        v[j] = bf16x8_to_f32x8(*reinterpret_cast<const u16x8*>(x + c * 8));
+        if (residual) {
+          const f32x8 r = bf16x8_to_f32x8(*reinterpret_cast<const u16x8*>(residual + c * 8));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[j][i] += r[i];
+          if (blockIdx.x == 0) *reinterpret_cast<u16x8*>(residual_out + c * 8) = f32x8_to_bf16x8(v[j]);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += v[j][i] * v[j][i];
+      }
+    }
+    ss = wave_reduce_sum(ss);
+    if (lane == 0) part[wave] = ss;
+    __syncthreads();
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) total += part[i];
+    const float inv = rsqrtf(total / K + eps);
+#pragma unroll
+    for (int j = 0; j < MAXC; ++j) {
+      const int c = tid + j * NTHR;
+      if (j * NTHR >= chunks) break;
+      if (c < chunks) {
+        const f32x8 g = bf16x8_to_f32x8(*reinterpret_cast<const u16x8*>(weight + c * 8));
+        f32x8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = v[j][i] * inv * g[i];
+        *reinterpret_cast<u16x8*>(h + c * 8) = f32x8_to_bf16x8(o);
+      }
+    }
+  } else {
+    for (int c = tid; c < chunks; c += NTHR)
+      *reinterpret_cast<u16x8*>(h + c * 8) = *reinterpret_cast<const u16x8*>(x + c * 8);
+  }
+  __syncthreads();
+
+  // ---- products --------------------------------------------------------------------
+  float acc[2] = {0.f, 0.f};
+  auto compute = [&](int b, int batch) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int c = (batch * U + i) * 512;
+      if (c < K) {
+        const f32x8 hv = bf16x8_to_f32x8(*reinterpret_cast<const u16x8*>(h + c + lane * 8));
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const f32x8 wv = bf16x8_to_f32x8(buf[b][i][r]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[r] = fmaf(wv[e], hv[e], acc[r]);
+        }
+      }
+    }
+  };
+  for (int batch = 0;; batch += 2) {
+    compute(0, batch);
+    if (batch + 2 >= batches) {
+      compute(1, batch + 1);
+      break;
+    }
+    load(0, batch + 2);
+    compute(1, batch + 1);
+    load(1, batch + 3);
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) acc[r] = wave_reduce_sum(acc[r]);
+  if (lane == 0 && n0 < outs) {
+    if (SILU) {
+      const float g = bf16_to_f32(f32_to_bf16(acc[0])), u = bf16_to_f32(f32_to_bf16(acc[1]));
+      y[n0] = f32_to_bf16(g / (1.0f + __expf(-g)) * u);
+    } else {
+      y[n0] = f32_to_bf16(acc[0]);
+      if (n0 + 1 < outs) y[n0 + 1] = f32_to_bf16(acc[1]);
+    }
+  }
+}
+
+}  // namespace
+
+extern "C" int lig_row_product_max(bool norm) { return norm ? NORM_MAX : PLAIN_MAX; }
+
+extern "C" void lig_row_product_launch(uint16_t* y, const uint16_t* w, int N, int K, const uint16_t* x,
+                                       const uint16_t* residual, uint16_t* residual_out, const uint16_t* weight,
+                                       float eps, bool silu, hipStream_t stream) {
+  // large projections: more waves share the h they form
+#define LIG_RP(NTHR, NORM, SILU)                                                                                    \
+  hipLaunchKernelGGL((row_product_kernel<NTHR, NORM, SILU>),                                                        \
+                     dim3((N + NTHR / WAVE_SIZE * 2 - 1) / (NTHR / WAVE_SIZE * 2)), dim3(NTHR), (size_t)K * 2, stream, \
+                     y, w, N, K, x, residual, residual_out, weight, eps)
+  if (silu) LIG_RP(512, true, true);
+  else if (weight && N >= 16384) LIG_RP(512, true, false);
+  else if (weight) LIG_RP(256, true, false);
+  else LIG_RP(256, false, false);
+#undef LIG_RP
+}

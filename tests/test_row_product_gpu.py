@@ -1,0 +1,89 @@
+"""Projections of a single token against fp32 torch: with and without the norm,
+the residual and the activation, at widths of one and several batches of loads
+and at row counts that leave waves and workgroups partly idle."""
+
+import pytest
+import torch
+
+from llm_instance_gateway_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _rnd(g, *shape):
+    return torch.randn(*shape, generator=g, device="cuda")
+
+
+def _norm(s, w):
+    return s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * w.float()
+
+
+@pytest.mark.parametrize("K", [512, 1024, 2048, 2560, 4096, 8192])
+@pytest.mark.parametrize("N", [2, 10, 96, 1030, 16390])
+def test_row_product(N, K):
+    g = torch.Generator("cuda").manual_seed(N + K)
+    x, res = _rnd(g, 1, K).to(BF), _rnd(g, 1, K).to(BF)
+    w, nw = (_rnd(g, N, K) * K ** -0.5).to(BF), (1 + 0.1 * _rnd(g, K)).to(BF)
+    mag = w.float().abs() @ torch.ones(K, device="cuda")
+    for norm, residual in ((None, None), (nw, None), (nw, res)):
+        for silu in (False, True) if norm is not None else (False,):
+            assert ops.row_product_serves(w, norm is not None)
+            got = ops.row_product(x, w, norm, 1e-5, residual, silu)
+            s = x.float() if residual is None else x.float() + res.float()
+            if residual is not None:
+                got, r = got
+                assert torch.equal(r, s.to(BF))
+            h = s if norm is None else _norm(s, nw)
+            y = (w.float() @ h[0])
+            # h is rounded to 8 bits (2^-8 of each term, like a walk), y too
+            walk = 2.0 ** -8 * (w.float() ** 2 @ h[0] ** 2).sqrt() * 4 if norm is not None else 2.0 ** -18 * mag
+            tol = walk + 2.0 ** -8 * y.abs() + 1e-6
+            if silu:
+                a, b, ta, tb = *y.chunk(2), *tol.chunk(2)
+                y = torch.nn.functional.silu(a) * b
+                # |silu'| <= 1.1
+                tol = 1.1 * ta * (b.abs() + tb) + torch.nn.functional.silu(a).abs() * tb + 2.0 ** -7 * y.abs() + 1e-6
+            assert got.shape == (1, len(y)) and ((got[0].float() - y).abs() <= tol).all()
+
+
+def test_row_product_wide_and_refused():
+    g = torch.Generator("cuda").manual_seed(1)
+    for K in (14336, 16384):
+        x, w = _rnd(g, 1, K).to(BF), (_rnd(g, 40, K) * K ** -0.5).to(BF)
+        y = w.float() @ x[0].float()
+        assert ((ops.row_product(x, w)[0].float() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-3).all()
+        assert not ops.row_product_serves(w, True)
+    for w in (_rnd(g, 8, 520).to(BF), _rnd(g, 8, 512), _rnd(g, 8, 17 * 1024).to(BF), _rnd(g, 512, 8).to(BF).t()):
+        assert not ops.row_product_serves(w, False)
+
+
+def test_single_decode_matches_layer_kernels(monkeypatch):
+    """A lone request's steps, replayed from the graph, against the same engine
+    with the projections as products of their own."""
+    from dataclasses import replace
+
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.models.config import get_model_config
+    from llm_instance_gateway_amd.models.llama import LlamaForCausalLM
+
+    mc = replace(get_model_config("llama3-8b"), num_layers=3, vocab_size=1024)
+    outs = []
+    for row in (True, False):
+        if not row:
+            monkeypatch.setattr(LlamaForCausalLM, "_row_products", lambda self: False)
+        torch.manual_seed(3)
+        eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=32, max_num_seqs=2, max_num_batched_tokens=256,
+                                     max_model_len=256), device="cuda")
+        if row:
+            assert eng.runner.model._row_products()
+        s = eng.add_request(list(range(7, 40)), SamplingParams(max_new_tokens=8))
+        logits = []
+        for i in range(4):
+            eng.step()
+            s.output_token_ids[-1] = 11 + i  # the same continuation on both sides
+            if eng.runner.graph_runner is not None:
+                logits.append(eng.runner.graph_runner.logits[1][:1].float().clone())
+        outs.append(torch.cat(logits))
+    # two correct orders of bf16 rounding, 3 layers deep
+    assert (outs[0] - outs[1]).norm() <= 0.03 * outs[1].norm()
