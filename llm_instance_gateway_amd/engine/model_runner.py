@@ -161,8 +161,7 @@ class ModelRunner:
             and (tp is None or _os.environ.get("LIG_TP_GRAPHS", "0") == "1")
         )
         # Mixed-step prefill/decode stream overlap — MEASURED DEAD END as a
-        # default: 51.4 vs 56.5 req/s at the serving shape (gpurun
-        # bench_mixed vs bench_mixed_noov) — the graph replay and the eager
+        # default: 51.4 vs 56.5 req/s at the serving shape — the graph replay and the eager
         # prefill contend for the same CUs, so splitting the step into two
         # streams only added sync overhead; the single flat mixed batch
         # already keeps the chip full.  Kept opt-in (LIG_OVERLAP=1) for

@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256) void sgmv_expand_tiled_kernel(
 //
 // v1 units kernels (register-resident B, thread = (unit, 8 outs) with a
 // serial token loop) were a MEASURED DEAD END: 31.0 vs 52.6 req/s e2e
-// (gpurun bench_units vs bench_nounits) — they traded occupancy for
+// — they traded occupancy for
 // locality (decode: 384-512 waves on a 256-CU chip) and the adapter set is
 // L2-resident anyway, so the binding constraint was LATENCY, exactly what
 // the v2 kernels' design note says.  Kept below for the record.
