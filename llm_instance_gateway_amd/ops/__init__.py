@@ -625,7 +625,9 @@ def paged_attention_general(
     q/gate may be column-block views with a row stride; v_cache may be a view
     of the leading entries of k_cache's rows (a latent cache).  chunk > 0:
     only keys of the query's own chunk, floor(j/chunk) == floor(p/chunk).
-    window > 0: only keys j with p - j < window.  weights "sigmoid": every
+    window > 0: only keys j with p - j < window.  Keys before a row's first
+    visible one are not read, nor are the table entries of blocks that end
+    before it.  weights "sigmoid": every
     visible key weighs sigmoid(score + score_bias[head]) (fp32 [heads],
     optional) and nothing is normalised.  gate_per_head: gate is [R, heads],
     one logistic gate per head.  softcap > 0: score <- softcap *

@@ -192,14 +192,17 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
 
   // rows of a step: S^T tile row li stands for key (li/4)*8 + li%4 (+4 in the
   // second tile), this lane's values are keys lg*8 .. +8.  Keys past the end
-  // repeat the last one.  PB: a lane's 8 keys lie in one block, whose number
+  // repeat the last one, keys before the first visible one that one: their
+  // weight is zero, but what they hold would still meet it in a product, and
+  // their blocks may be gone.  PB: a lane's 8 keys lie in one block, whose number
   // is read one step ahead; no branch may stand between the loads, or each
   // would be waited for by itself
   const size_t block_rows = (size_t)a.num_kv_heads * a.block_size;
   const size_t head_rows = (size_t)kvh * a.block_size;
   const int kt0 = (li >> 2) * 8, vt0 = lg * 8;
   const int shift = a.block_shift;
-  auto block_at = [&](int st, int t0) { return PB ? bt[min(st * KT + t0, pos) >> shift] : 0; };
+  auto visible = [&](int t) { return min(EXTRA ? max(t, key_lo) : t, pos); };
+  auto block_at = [&](int st, int t0) { return PB ? bt[visible(st * KT + t0) >> shift] : 0; };
   u32x4 kreg[2][KS];
   vload vreg[8];
   // cache rows of N keys of the 8 from t0 on
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
     constexpr int N = sizeof(r) / sizeof(r[0]);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const int t = min(t0 + first_t + i * by, pos);
+      const int t = visible(t0 + first_t + i * by);
       if constexpr (PB) {
         r[i] = (size_t)blk * block_rows + head_rows + (t & (a.block_size - 1));
       } else {

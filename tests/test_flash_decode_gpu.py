@@ -122,3 +122,23 @@ def test_infinite_and_lowest_scores():
     keep = torch.ones(2, H, dtype=torch.bool, device="cuda")
     keep[0, 1] = False
     assert torch.equal(bad[keep], got[keep])
+
+
+@pytest.mark.parametrize(
+    "opt", [dict(window=1), dict(window=33), dict(window=64), dict(window=600), dict(chunk=48),
+            dict(weights="sigmoid", window=100)], ids=range(6))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 12, 1, 16), (128, 18, 2, 8), (128, 6, 2, 3)])
+def test_keys_before_the_first_visible_one(opt, D, H, G, bs):
+    """They may hold anything, and the blocks before may be gone."""
+    b = _batch(CTX, G, D, bs, H, 11)
+    k, v, tab = b["k"].clone(), b["v"].clone(), b["tab"].clone()
+    used = {t for row, c in zip(b["tab"].tolist(), CTX) for t in row[: (c + bs - 1) // bs]}
+    gone = next(i for i in range(k.shape[0]) if i not in used)
+    k[gone], v[gone] = float("nan"), float("inf")
+    for s, c in enumerate(CTX):
+        first = max(0, c - opt["window"]) if "window" in opt else (c - 1) // opt["chunk"] * opt["chunk"]
+        tab[s, : first // bs] = gone
+        if first % bs:
+            k[tab[s, first // bs], :, : first % bs], v[tab[s, first // bs], :, : first % bs] = float("nan"), float("inf")
+    got = ops.paged_attention_general(b["q"], k, v, tab, b["tok_seq"], b["pos"], D ** -0.5, H, **opt)
+    _check(got, b, D ** -0.5, H, **opt)
