@@ -748,8 +748,10 @@ def paged_attention_prefill_tiles(
     tile_qstart name the 64-row query tiles.  Temperature, sigmoid gate and
     softmax sink are fused; v_cache may view the head of k_cache's rows; chunk
     > 0 restricts every row to the keys of its own chunk, window > 0 to the
-    last `window` keys up to its own.  weights "sigmoid", score_bias,
-    gate_per_head and softcap as in `paged_attention_general`.  GPU only."""
+    last `window` keys up to its own; keys that no row of a 64-row tile sees are
+    not read, nor are the table entries of blocks without others.  weights
+    "sigmoid", score_bias, gate_per_head and softcap as in
+    `paged_attention_general`.  GPU only."""
     assert weights in ("softmax", "sigmoid") and (weights == "sigmoid" or score_bias is None)
     nb, G, bs, D = k_cache.shape
     Dv = v_cache.shape[-1]

@@ -182,12 +182,13 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   // ---- walk ------------------------------------------------------------------
   const int qpos0 = ctx - n + qt;
   const int kv_end = min(ctx, qpos0 + TQ);
-  int kv_begin = 0;
+  int first_key = 0;  // that some row sees
   if (EXTRA) {
-    if (a.chunk > 0) kv_begin = (qpos0 / a.chunk) * a.chunk;
-    if (a.window > 0) kv_begin = max(kv_begin, qpos0 - a.window + 1);
-    kv_begin = max(kv_begin, 0) & ~(KT - 1);
+    if (a.chunk > 0) first_key = (qpos0 / a.chunk) * a.chunk;
+    if (a.window > 0) first_key = max(first_key, qpos0 - a.window + 1);
+    first_key = max(first_key, 0);
   }
+  const int kv_begin = first_key & ~(KT - 1);
   const int wave_first = ctx - n + row0;                                   // position of the wave's first row
   const int wave_last_lo = __builtin_amdgcn_readlane(key_lo[RB - 1], 15);  // largest lower bound
 
@@ -198,15 +199,18 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   const size_t block_rows = (size_t)a.num_kv_heads * a.block_size;
   u32x4 kreg[TPT], vreg[TPT];
 
-  // keys past the end repeat the last one.  PB: the TPT keys of a thread lie in
-  // one block (tiles start at multiples of 64), whose number is read one tile
+  // Keys that no row of the tile sees are replaced by the nearest one that some
+  // row does: their weight is zero, but what they hold would still meet it in a
+  // product, and the blocks before may be gone.  PB: the TPT keys of a thread lie
+  // in one block (tiles start at multiples of 64), whose number is read one tile
   // ahead; no branch may stand between the loads, or each would be waited for
-  auto block_of = [&](int kv0) { return PB ? bt[min(kv0 + st * TPT, ctx - 1) >> a.block_shift] : 0; };
+  auto visible = [&](int t) { return min(EXTRA ? max(t, first_key) : t, kv_end - 1); };
+  auto block_of = [&](int kv0) { return PB ? bt[visible(kv0 + st * TPT) >> a.block_shift] : 0; };
   auto fetch = [&](int kv0, int blk) {
     size_t row[TPT];
 #pragma unroll
     for (int i = 0; i < TPT; ++i) {
-      const int t = min(kv0 + st * TPT + i, ctx - 1);
+      const int t = visible(kv0 + st * TPT + i);
       if constexpr (PB) {
         row[i] = (size_t)blk * block_rows + kv_head_rows + (t & (a.block_size - 1));
       } else {

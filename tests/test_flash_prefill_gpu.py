@@ -129,3 +129,36 @@ def test_infinite_and_lowest_scores():
     keep = torch.ones(70, H, dtype=torch.bool, device="cuda")
     keep[9, 1] = False
     assert torch.equal(bad[keep], got[keep])
+
+
+@pytest.mark.parametrize("opt", [dict(window=1), dict(window=33), dict(window=70, softcap=30.0), dict(chunk=48)], ids=range(4))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 4, 2, 16), (64, 6, 2, 8), (128, 3, 1, 6)])
+def test_keys_that_no_row_of_the_tile_sees(opt, D, H, G, bs):
+    """Keys before a tile's first visible one may hold anything, and the blocks
+    before may be gone; so may the keys behind its last row's."""
+    segs = [(200, 60), (700, 50), (129, 1)]
+    b = _batch(segs, G, D, bs, H, 11)
+    k, v, tab = b["k"].clone(), b["v"].clone(), b["tab"].clone()
+    used = {t for row, (c, _) in zip(b["tab"].tolist(), segs) for t in row[: (c + bs - 1) // bs]}
+    gone = next(i for i in range(k.shape[0]) if i not in used)
+    k[gone], v[gone] = float("nan"), float("inf")
+    for s, (c, n) in enumerate(segs):
+        first = max(0, c - n - opt["window"] + 1) if "window" in opt else (c - n) // opt["chunk"] * opt["chunk"]
+        tab[s, : first // bs] = gone
+        if first % bs:
+            k[tab[s, first // bs], :, : first % bs], v[tab[s, first // bs], :, : first % bs] = float("nan"), float("inf")
+    got = ops.paged_attention_prefill_tiles(
+        b["q"], k, v, tab, b["starts"], b["ctx"], b["ts"], b["tq"], D ** -0.5, H, **opt)
+    _check(got, b, D, D ** -0.5, H, **opt)
+
+
+@pytest.mark.parametrize("D,H,G,bs", [(128, 4, 2, 16), (64, 6, 2, 8), (128, 3, 1, 6)])
+def test_keys_behind_the_last_row_of_the_tile(D, H, G, bs):
+    # the first tile's rows stand at positions 30 to 93
+    b = _batch([(230, 200)], G, D, bs, H, 12)
+    v = b["v"].clone()
+    v[b["tab"][0, 100 // bs], :, 100 % bs] = float("nan")
+    args = (b["tab"], b["starts"], b["ctx"], b["ts"], b["tq"], D ** -0.5, H)
+    got = ops.paged_attention_prefill_tiles(b["q"], b["k"], v, *args)
+    want = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], *args)
+    assert torch.equal(got[:64], want[:64]) and got[70:].isnan().all()
