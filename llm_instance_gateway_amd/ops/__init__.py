@@ -832,7 +832,8 @@ def latent_attention_rows(
     tile's visible keys into that many slices run by separate workgroups and
     merged afterwards (0: chosen from the row count and the longest context
     the block tables can hold).  window > 0: a token at position p sees keys
-    j with p - j < window.  GPU, bf16."""
+    j with p - j < window; keys that no row of a tile sees are not read, nor
+    are the table entries of blocks without others.  GPU, bf16."""
     nb, G, bs, row = cache.shape
     R = q.shape[0]
     assert G == 1 and q.is_cuda and q.dtype == torch.bfloat16 and cache.dtype == q.dtype

@@ -128,8 +128,9 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   const long last_rho = (rho0 + ROWS < nrows ? rho0 + ROWS : nrows) - 1;
   const int first_tok = (int)(rho0 / H);
   const int kv_end = ctx - n + (int)(last_rho / H) + 1;  // keys any row of the tile sees
-  // oldest key any row of the tile sees, at the start of a piece of 8
-  const int kv_first = window > 0 ? max(0, ctx - n + first_tok - window + 1) & ~7 : 0;
+  // oldest key any row of the tile sees, and the start of its piece of 8
+  const int kv_seen = window > 0 ? max(0, ctx - n + first_tok - window + 1) : 0;
+  const int kv_first = kv_seen & ~7;
   int kv_lo = kv_first, kv_hi = kv_end;
   if (nsplit > 1) {
     const int nt = (kv_end - kv_first + KT - 1) / KT;
@@ -142,14 +143,16 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   const int all_lo = window > 0 ? kv_end - window : 0;
 
   // ---- fetching: chunk c of key t of a tile goes to LDS chunk t * CHP + (c ^ f(t)).
-  // Keys past the end repeat the last one.
+  // Keys past the end repeat the last one, keys before the first that some row
+  // sees that one: their weight is zero, but what they hold would still meet it in
+  // a product, and the blocks before may be gone.
   // FULL: 8 keys, aligned, are one contiguous piece of a block; a wave takes
   // KT / 32 such pieces of CHP / 8 fetches.  Lane j looks up the block of piece j
   // of the tile after next.  Else every lane looks for its own key's block.
   const int CH = D / 8;
   constexpr int NP = CHP / 8;  // fetches per piece
   auto block_of = [&](int kv0) {
-    const int t = min(kv0 + (FULL ? (lane & 7) * 8 : lane & (KT - 1)), kv_end - 1);
+    const int t = min(max(kv0 + (FULL ? (lane & 7) * 8 : lane & (KT - 1)), kv_seen), kv_end - 1);
     return bt[FULL ? t >> block_shift : t / block_size];
   };
   auto fetch = [&](int kv0, int blks, int buf) {
@@ -162,14 +165,14 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int t0 = min(kv0 + piece * 8, (kv_end - 1) & ~7);
         const int blk = __builtin_amdgcn_readlane(blks, piece);
         const uint16_t* g = cache + ((size_t)blk * block_size + (t0 & (block_size - 1))) * D;
-        const int last = kv_end - 1 - t0;
+        const int last = kv_end - 1 - t0, first = kv_seen - t0;
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
           const int p = i * 64 + here;
           const int key = p / CHP;  // of the piece
           const int c = (p % CHP) ^ ((key & 3) | ((piece & 1) << 2));
           __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void*)(g + (min(key, last) * DKP + c * 8)),
+              (const __attribute__((address_space(1))) void*)(g + (min(max(key, first), last) * DKP + c * 8)),
               (__attribute__((address_space(3))) void*)(sm + buf * TILE + (piece * NP + i) * 512), 16, 0, 0);
         }
       }
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int p = base + here;
         const int key = p / CHP;
         const int c = (p % CHP) ^ ((key & 3) | ((key >> 1) & 4));
-        const int off = min(kv0 + key, kv_end - 1) % block_size;
+        const int off = min(max(kv0 + key, kv_seen), kv_end - 1) % block_size;
         const int blk = __shfl(blks, key, 64);
         if (c < CH)
           __builtin_amdgcn_global_load_lds(

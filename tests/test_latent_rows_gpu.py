@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 
 
-def _run(segs, H, D, Dv, bs, window, nsplit, gate, seed=1, scale=None):
+def _run(segs, H, D, Dv, bs, window, nsplit, gate, seed=1, scale=None, forget=False):
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
@@ -38,11 +38,21 @@ def _run(segs, H, D, Dv, bs, window, nsplit, gate, seed=1, scale=None):
     sink = rnd(H)
     gt = rnd(T, H + 1).to(BF)[:, 1:] if gate else None
     scale = (D ** -0.5) if scale is None else scale
+    kept, kept_tab = cache, tab
+    if forget:  # keys before the first visible one hold anything, the blocks before are gone
+        cache, tab = cache.clone(), [list(t) for t in tab]
+        gone = next(i for i in range(pool) if i not in perm)
+        cache[gone] = float("nan")
+        for s, (c, n) in enumerate(segs):
+            first = max(0, c - n - window + 1)
+            tab[s][: first // bs] = [gone] * (first // bs)
+            if first % bs:
+                cache[tab[s][first // bs], 0, : first % bs] = float("nan")
     got = ops.latent_attention_rows(
         q, cache, Dv, i32(tab), i32(starts), i32([n for _, n in segs]), i32([c for c, _ in segs]),
         max(n for _, n in segs), scale, H, sink=sink, nsplit=nsplit, gate=gt, window=window)
     for s, (c, n) in enumerate(segs):
-        rows = cache[torch.tensor(tab[s][: need[s]], device="cuda")].reshape(-1, D)[:c].double()
+        rows = kept[torch.tensor(kept_tab[s][: need[s]], device="cuda")].reshape(-1, D)[:c].double()
         qq = q[starts[s] : starts[s] + n].view(n, H, D).transpose(0, 1).double()
         p, j = torch.arange(c - n, c, device="cuda")[:, None], torch.arange(c, device="cuda")[None]
         hide = (j > p) | ((p - j >= window) if window else (j > p))
@@ -71,3 +81,11 @@ def test_edges(segs, H, D, Dv, bs, window, nsplit):
 def test_scale_signs(scale):
     _run(ONE, 16, 192, 128, 16, 0, 1, gate=False, scale=scale)
     _run(MANY, 16, 192, 128, 16, 0, 2, gate=True, scale=scale)
+
+
+@pytest.mark.parametrize("nsplit", [1, 2])
+@pytest.mark.parametrize("window", [1, 13, 40, 70])
+@pytest.mark.parametrize("segs,H", [(ONE, 32), (MANY, 16), (MANY, 3)], ids=["one32", "many16", "many3"])
+@pytest.mark.parametrize("D,Dv,bs", [(576, 512, 16), (576, 512, 8), (320, 256, 6), (72, 64, 16)])
+def test_keys_before_the_first_visible_one(segs, H, D, Dv, bs, window, nsplit):
+    _run(segs, H, D, Dv, bs, window, nsplit, gate=False, forget=True)
