@@ -458,6 +458,14 @@ static inline int shift_of(int block_size) {
   return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
 }
 
+template <int D, bool SIG, bool EXTRA>
+static void launch_merge(const Args& a, hipStream_t stream) {
+  if (a.nsplits <= 1) return;
+  const long lanes = (long)a.rows * a.num_q_heads * (D / 4);
+  hipLaunchKernelGGL((flash_decode_merge_kernel<D, SIG, EXTRA>), dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0,
+                     stream, a);
+}
+
 template <int D, bool CAP, bool SIG, bool EXTRA>
 static void launch_mode(const Args& a, hipStream_t stream) {
   constexpr int W = 4;
@@ -473,11 +481,7 @@ static void launch_mode(const Args& a, hipStream_t stream) {
     hipLaunchKernelGGL((flash_decode_kernel<D, W, false, true, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
   else
     hipLaunchKernelGGL((flash_decode_kernel<D, W, false, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
-  if (a.nsplits > 1) {
-    const long lanes = (long)a.rows * a.num_q_heads * (D / 4);
-    hipLaunchKernelGGL((flash_decode_merge_kernel<D, SIG, EXTRA>), dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0,
-                       stream, a);
-  }
+  launch_merge<D, SIG, EXTRA>(a, stream);
 }
 
 }  // namespace flash_decode

@@ -142,3 +142,32 @@ def test_keys_before_the_first_visible_one(opt, D, H, G, bs):
             k[tab[s, first // bs], :, : first % bs], v[tab[s, first // bs], :, : first % bs] = float("nan"), float("inf")
     got = ops.paged_attention_general(b["q"], k, v, tab, b["tok_seq"], b["pos"], D ** -0.5, H, **opt)
     _check(got, b, D ** -0.5, H, **opt)
+
+
+# up to 32 parts; of 9248 keys' 18 parts the last is empty (17 take 17 steps each)
+LONG = [1, 500, 1030, 2600, 9248, 12512, 16384]
+
+
+@pytest.mark.parametrize("nsplits", [1, 5, 32])
+def test_heads_of_16(nsplits):
+    H, G, D = 4, 2, 16
+    for ctx in (CTX, LONG):
+        b = _batch(ctx, G, D, 16, H, 13)
+        b["ctx"][0] = 0
+        got = ops.paged_attention_decode(
+            b["q"].view(-1, H, D), b["k"], b["v"], b["tab"], b["ctx"], D ** -0.5, nsplits=nsplits)
+        assert (got[0] == 0).all()
+        b = dict(b, q=b["q"][1:], tab=b["tab"][1:], tok_seq=b["tok_seq"][:-1], pos=b["pos"][1:])
+        _check(got[1:].reshape(len(ctx) - 1, -1), b, D ** -0.5, H)
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+def test_long_walks_are_cut(D):
+    H, G, ns = 4, 2, 5
+    b = _batch([2600, 3], G, D, 16, H, 14)
+    out = torch.empty(2, H, D, dtype=BF, device="cuda")
+    parts = torch.full((2, H, ns, D + 2), 7e7, device="cuda")
+    ops._EXT.paged_attention_decode_split(
+        out, b["q"].view(2, H, D), b["k"], b["v"], b["tab"], b["ctx"], parts, D ** -0.5, ns, ops._stream())
+    assert (parts[0] != 7e7).all() and (parts[1] == 7e7).all()
+    _check(out.view(2, -1), b, D ** -0.5, H)
