@@ -167,7 +167,7 @@ def test_long_walks_are_cut(D):
     b = _batch([2600, 3], G, D, 16, H, 14)
     out = torch.empty(2, H, D, dtype=BF, device="cuda")
     parts = torch.full((2, H, ns, D + 2), 7e7, device="cuda")
-    ops._EXT.paged_attention_decode_split(
+    ops._load_ext().paged_attention_decode_split(
         out, b["q"].view(2, H, D), b["k"], b["v"], b["tab"], b["ctx"], parts, D ** -0.5, ns, ops._stream())
     assert (parts[0] != 7e7).all() and (parts[1] == 7e7).all()
     _check(out.view(2, -1), b, D ** -0.5, H)
