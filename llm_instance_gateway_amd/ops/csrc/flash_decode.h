@@ -283,11 +283,7 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
 #pragma unroll
         for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s4[e >> 2][e & 3]);
         mx = swap_max(mx);
-        if constexpr (CAP)
-          mx = mx == -INFINITY ? mx : cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
-                                                              1.f + __builtin_amdgcn_exp2f(mx * c * (2.f * LOG2E))));
-        else
-          mx = mx == -INFINITY ? mx : mx * c;
+        mx = mx == -INFINITY ? mx : CAP ? cap2 * tanhf(mx * c) : mx * c;
         if (__any(mx > m)) {
           const float m_new = fmaxf(m, mx);
           const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
@@ -305,8 +301,8 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
         const float v = s4[e >> 2][e & 3];
         float w;
         if constexpr (CAP) {
-          const float b = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
-                                                  1.f + __builtin_amdgcn_exp2f(v * c * (2.f * LOG2E))));
+          // tanhf: forms by the exponential alone are off by 1e-7 of the cap, however small the score
+          const float b = cap2 * tanhf(v * c);
           if constexpr (SIG)
             w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(b + bias * LOG2E)));
           else

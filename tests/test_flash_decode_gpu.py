@@ -171,3 +171,15 @@ def test_long_walks_are_cut(D):
         out, b["q"].view(2, H, D), b["k"], b["v"], b["tab"], b["ctx"], parts, D ** -0.5, ns, ops._stream())
     assert (parts[0] != 7e7).all() and (parts[1] == 7e7).all()
     _check(out.view(2, -1), b, D ** -0.5, H)
+
+
+@pytest.mark.parametrize("weights", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("cap", [30.0, 1e4, 1e6])
+def test_soft_caps_keep_small_scores(cap, weights):
+    """A cap far above the scores changes nothing: tanh near zero may not lose
+    digits (1 - 2 / (1 + e^2x) is off by 1e-7 of the cap)."""
+    D, H, G = 128, 8, 2
+    b = _batch(CTX, G, D, 16, H, 15)
+    got = ops.paged_attention_general(
+        b["q"], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], D ** -0.5, H, softcap=cap, weights=weights)
+    _check(got, b, D ** -0.5, H, softcap=cap, weights=weights)
