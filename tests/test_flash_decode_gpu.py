@@ -3,9 +3,9 @@ wrong: contexts around its 32-key steps and 512-key parts, group sizes on both
 sides of the low-part columns, block sizes that keep or split a lane's keys,
 and the options' bounds.
 
-Tolerance: weights enter the second product as two bf16 numbers, 16 significant
-bits (off by at most 2^-16, once more for the split), results are rounded to
-bf16 once (8 significant bits: at most 2^-8 of the value), sums are fp32."""
+Tolerance: weights enter the second product as three bf16 numbers, all of their
+24 bits, results are rounded to bf16 once (8 significant bits: at most 2^-8 of
+the value), sums are fp32."""
 
 import pytest
 import torch
@@ -183,3 +183,21 @@ def test_soft_caps_keep_small_scores(cap, weights):
     got = ops.paged_attention_general(
         b["q"], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], D ** -0.5, H, softcap=cap, weights=weights)
     _check(got, b, D ** -0.5, H, softcap=cap, weights=weights)
+
+
+@pytest.mark.parametrize("H,G,bias", [(32, 8, None), (32, 2, None), (32, 8, -1.0)])
+def test_weights_keep_32_bits(H, G, bias):
+    """Values of one sign, so that a result is off by little more than 2^-24 of
+    itself.  It then differs from the rounded exact one where that lies as close
+    to the middle between two bf16 numbers, which are 2^-8 to 2^-7 apart: some 2 *
+    2^-24 * 180 = 2e-5 of all.  Weights of 16 bits: 1e-4 and more."""
+    D, R, ctx, bs = 128, 512, 3, 16
+    b = _batch([ctx] * R, G, D, bs, H, 16)
+    b["v"] = 1 + b["v"].float().abs().clamp_max(1).to(BF)
+    kw = {} if bias is None else dict(weights="sigmoid", score_bias=torch.full((H,), bias, device="cuda"))
+    got = ops.paged_attention_general(b["q"], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], D ** -0.5, H, **kw)
+    k, v = (b[x][b["tab"][:, 0].long(), :, :ctx].double() for x in "kv")
+    s = b["q"].view(R, G, H // G, D).double() @ k.transpose(-1, -2).contiguous() * D ** -0.5
+    w = s.softmax(-1) if bias is None else torch.sigmoid(s + bias)
+    ref = (w @ v).view(R, -1).float().to(BF)
+    assert (got != ref).double().mean().item() < 4e-5
