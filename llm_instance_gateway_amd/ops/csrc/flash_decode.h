@@ -482,7 +482,7 @@ static void launch_merge(const Args& a, hipStream_t stream) {
 }
 
 template <int D, bool CAP, bool SIG, bool EXTRA>
-static void launch_mode(const Args& a, hipStream_t stream) {
+static void launch_rows(const Args& a, hipStream_t stream) {
   constexpr int W = 4;
   const int group = a.num_q_heads / a.num_kv_heads;
   const dim3 grid(a.rows * a.num_kv_heads, a.nsplits), block(64 * W);
@@ -497,6 +497,31 @@ static void launch_mode(const Args& a, hipStream_t stream) {
   else
     hipLaunchKernelGGL((flash_decode_kernel<D, W, false, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
   launch_merge<D, SIG, EXTRA>(a, stream);
+}
+
+template <int D, bool CAP, bool SIG, bool EXTRA>
+static void launch_mode(Args a, hipStream_t stream) {
+  // a grid holds less than 2^32 threads a dimension, and drops the rest without an
+  // error: 256 per (row, key/value head) here, D / 4 per (row, head) in the merge
+  const long per_row = (long)a.num_kv_heads * 256 > (long)a.num_q_heads * (D / 4) ? (long)a.num_kv_heads * 256
+                                                                                 : (long)a.num_q_heads * (D / 4);
+  const long most = ((1L << 32) - 256) / per_row;
+  for (long left = a.rows; left > 0; left -= most) {
+    a.rows = (int)(left < most ? left : most);
+    launch_rows<D, CAP, SIG, EXTRA>(a, stream);
+    const long r = a.rows, heads = r * a.num_q_heads;
+    a.out += heads * D;
+    a.q += r * a.q_stride;
+    if (a.gate) a.gate += r * a.gate_stride;
+    if (a.tok_seq) {
+      a.tok_seq += r;
+    } else {
+      a.block_tables += r * a.max_blocks;
+    }
+    if (a.positions) a.positions += r;
+    if (a.context_lens) a.context_lens += r;
+    if (a.scratch) a.scratch += heads * a.nsplits * (D + 2);
+  }
 }
 
 }  // namespace flash_decode

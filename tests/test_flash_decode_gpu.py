@@ -201,3 +201,20 @@ def test_weights_keep_32_bits(H, G, bias):
     w = s.softmax(-1) if bias is None else torch.sigmoid(s + bias)
     ref = (w @ v).view(R, -1).float().to(BF)
     assert (got != ref).double().mean().item() < 4e-5
+
+
+def test_more_rows_than_a_grid_dimension_holds():
+    """256 threads per (row, key/value head) reach 2^32 at 16 x 1048576."""
+    R, H, G, D = 1048576 + 5, 16, 16, 64
+    b = _batch([1, 1], G, D, 16, H, 18)  # one key: the result is its value
+    tok_seq = torch.arange(R, dtype=torch.int32, device="cuda") % 2
+    q = b["rnd"](1, H * D).expand(R, H * D).contiguous()
+    want = b["v"][b["tab"][:, 0].long(), :, 0].reshape(2, H * D)
+    pos = torch.zeros(R, dtype=torch.int64, device="cuda")
+    for got in (
+        ops.paged_attention_general(q, b["k"], b["v"], b["tab"], tok_seq, pos, D ** -0.5, H),
+        ops.paged_attention_decode(
+            q.view(R, H, D), b["k"], b["v"], b["tab"][tok_seq.long()].contiguous(), tok_seq * 0 + 1, D ** -0.5),
+    ):
+        got = got.view(R, H * D)
+        assert torch.equal(got[0::2], want[:1].expand(R // 2 + 1, -1)) and torch.equal(got[1::2], want[1:].expand(R // 2, -1))
