@@ -327,9 +327,10 @@ def row_product(x, weight, norm=None, eps=0.0, residual=None, silu=False):
 
 
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:
-    """x.argmax(-1) of [N, V]; the first of equals."""
+    """x.argmax(-1) of [N, V]; the first of equals.  The kernel takes fewer than
+    2^22 rows: 1024 threads each, and a grid holds less than 2^32."""
     if (x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float32) and 0 < x.shape[1] < 2**31 - 1024
-            and x.stride(1) == 1 and _use_native(x)):
+            and x.shape[0] < 2**22 and x.stride(1) == 1 and _use_native(x)):
         out = torch.empty(x.shape[0], dtype=torch.int64, device=x.device)
         _EXT.argmax_rows(out, x, _stream())
         return out

@@ -233,7 +233,7 @@ void argmax_rows(torch::Tensor out, torch::Tensor x, int64_t stream) {
   const bool bf16 = x.scalar_type() == torch::kBFloat16;
   TORCH_CHECK(x.is_cuda() && (bf16 || x.scalar_type() == torch::kFloat32), "bf16 or fp32 rows on the device");
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.size(1) > 0 && x.size(1) < (1L << 31) - 1024 &&
-                  x.size(0) < (1L << 31),
+                  x.size(0) < (1L << 22),
               "[N, V] rows");
   TORCH_CHECK(out.is_cuda() && out.scalar_type() == torch::kInt64 && out.is_contiguous() && out.dim() == 1 &&
               out.size(0) == x.size(0));

@@ -35,3 +35,10 @@ def test_argmax_rows(dtype, V, off):
     assert ops.argmax_rows(dev).tolist() == want
     assert ops.argmax_rows(dev[:0]).tolist() == []
     assert ops.argmax_rows(dev.t().contiguous().t()).tolist() == dev.argmax(-1).tolist()  # other strides: torch
+
+
+def test_more_rows_than_a_grid_holds():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(0, 9, (2**22 + 3, 5), generator=g, device="cuda").float()
+    got = ops.argmax_rows(x)
+    assert torch.equal(x.gather(1, got[:, None]).squeeze(1), x.amax(1)) and got.max() < 5 and got.min() >= 0
