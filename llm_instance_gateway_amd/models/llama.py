@@ -22,10 +22,18 @@ from typing import List
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..engine.metadata import BatchMeta
 from .config import ModelConfig
+
+
+def _plain(module: nn.Module) -> bool:
+    """Whether calling the module runs its class's forward and nothing else, so
+    that kernels may take its place."""
+    d = module.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
 
 
 def _linear(in_f: int, out_f: int, device, dtype) -> nn.Linear:
@@ -206,7 +214,8 @@ class LlamaForCausalLM(nn.Module):
         meta: BatchMeta,
     ) -> torch.Tensor:
         hidden = self.embed_tokens(input_ids)
-        if meta.lora_rows_tok is not None:
+        # (a graph being captured brings row tiles only, and would not run hooks again)
+        if meta.lora_rows_tok is not None and (meta.lora_slot_per_token is None or self._plain_layers()):
             return self._forward_lora(hidden, positions, kv_caches, meta)
         if hidden.shape[0] == 1 and meta.lora_slot_per_token is None and self._row_products():
             return self._forward_row(hidden, positions, kv_caches, meta)
@@ -218,12 +227,17 @@ class LlamaForCausalLM(nn.Module):
         hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
+    def _plain_layers(self) -> bool:
+        return not _has_any_global_hook() and all(
+            _plain(m) for layer in self.layers for m in (layer, layer.self_attn, layer.mlp)
+        )
+
     def _row_products(self) -> bool:
         """Whether every projection of a layer is one that `ops.row_product` serves."""
-        if self.tp is not None:
+        if self.tp is not None or not self._plain_layers():
             return False
         return all(
-            type(m) is nn.Linear and m.bias is None and ops.row_product_serves(m.weight, norm)
+            type(m) is nn.Linear and _plain(m) and m.bias is None and ops.row_product_serves(m.weight, norm)
             for layer in self.layers
             for m, norm in (
                 (layer.self_attn.qkv_proj, True),

@@ -213,3 +213,47 @@ def test_engine_matches_unit_kernels(monkeypatch):
     for a, b in zip(*outs):
         # two correct orders of bf16 rounding, 3 layers deep
         assert (a - b).norm() <= 0.03 * b.norm()
+
+
+@pytest.mark.parametrize("lora", [False, True])
+def test_module_hooks_run(lora):
+    """The fused forwards stand aside for hooks on the modules they replace."""
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.lora import manager
+    from llm_instance_gateway_amd.models.config import ModelConfig
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=512, num_layers=2, num_heads=8, num_kv_heads=2,
+                     intermediate_size=1024, head_dim=64, max_position_embeddings=512)
+    torch.manual_seed(0)
+    eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=50, max_num_seqs=2, max_model_len=256, enforce_eager=True,
+                                 pad_batch_multiple=0), device="cuda:0")
+    model = eng.runner.model
+    if lora:
+        mgr = manager.AdapterManager(eng, max_slots=1, rank=16)
+        assert mgr.in_layer
+        mgr.register_random("l0", seed=1)
+    seq = eng.add_request([5] * 9, SamplingParams(max_new_tokens=30), lora_name="l0" if lora else "")
+    eng.step()
+
+    def step():  # one token, the same each time, and what the head reads
+        seq.output_token_ids[-1] = 11
+        out, execute = [], model.compute_logits
+        model.compute_logits = lambda h, idx: out.append(h.float()) or execute(h, idx)
+        eng.step()
+        del model.compute_logits
+        seq.output_token_ids.pop()
+        seq.num_computed_tokens -= 1
+        return out[0]
+
+    plain = step()
+    assert lora or model._row_products()
+    for m in (model.layers[0], model.layers[1].self_attn, model.layers[1].mlp) + (
+            () if lora else (model.layers[0].mlp.down_proj,)):
+        for register in (m.register_forward_hook, m.register_forward_pre_hook):
+            calls = []
+            handle = register(lambda *a: calls.append(1))
+            got = step()
+            handle.remove()
+            assert len(calls) == 1
+            assert (got - plain).norm() <= 0.03 * plain.norm()  # two orders of bf16 rounding
+    assert torch.equal(step(), plain)
