@@ -236,16 +236,16 @@ class LlamaForCausalLM(nn.Module):
         """Whether every projection of a layer is one that `ops.row_product` serves."""
         if self.tp is not None or not self._plain_layers():
             return False
-        return all(
-            type(m) is nn.Linear and _plain(m) and m.bias is None and ops.row_product_serves(m.weight, norm)
-            for layer in self.layers
-            for m, norm in (
-                (layer.self_attn.qkv_proj, True),
-                (layer.self_attn.o_proj, False),
-                (layer.mlp.gate_up_proj, True),
-                (layer.mlp.down_proj, False),
-            )
-        )
+        most = ops.row_product_most(self.norm)
+        for layer in self.layers:
+            attn, mlp = layer.self_attn, layer.mlp
+            for m, norm in ((attn.qkv_proj, True), (attn.o_proj, False), (mlp.gate_up_proj, True), (mlp.down_proj, False)):
+                if type(m) is not nn.Linear or not _plain(m):
+                    return False
+                p = m._parameters
+                if p["bias"] is not None or not ops.row_product_serves(p["weight"], norm, most):
+                    return False
+        return True
 
     def _forward_row(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
         """The layers for a single token: norms and the activation live in the

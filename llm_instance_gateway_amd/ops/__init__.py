@@ -304,15 +304,23 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_and_mul(x)
 
 
-def row_product_serves(weight: torch.Tensor, norm: bool) -> bool:
-    """Whether `row_product` takes a projection's weight."""
+def row_product_most(like: torch.Tensor) -> tuple:
+    """Most columns that `row_product` takes without and with a norm."""
+    if not _use_native(like):
+        return 0, 0
+    ext = _load_ext()
+    return ext.row_product_max(False), ext.row_product_max(True)
+
+
+def row_product_serves(weight: torch.Tensor, norm: bool, most: Optional[tuple] = None) -> bool:
+    """Whether `row_product` takes a projection's weight.  `most`:
+    `row_product_most`, for a caller that asks about many."""
     return (
         weight.dtype == torch.bfloat16
         and weight.is_contiguous()
         and weight.data_ptr() % 16 == 0
         and weight.shape[1] % 512 == 0
-        and _use_native(weight)
-        and weight.shape[1] <= _load_ext().row_product_max(norm)
+        and weight.shape[1] <= (most or row_product_most(weight))[norm]
     )
 
 
