@@ -163,11 +163,20 @@ class DecodeGraphRunner:
 
         return max_lora_rows(B, self.runner.adapter_manager.max_slots)
 
+    def _plain_head(self) -> bool:
+        """Whether compute_logits is nothing but head_logits of the rows asked
+        for, in fp32: not where it was overridden without the other."""
+        model = self.runner.model
+        for owner in (model, *type(model).__mro__):
+            if "compute_logits" in vars(owner):
+                return "head_logits" in vars(owner)
+        return False
+
     def _forward(self, B: int) -> torch.Tensor:
         model = self.runner.model
         x = self._views(B).dev
         hidden = model(x.ids, x.pos, self.runner.kv_caches, self._meta(B))
-        if hasattr(model, "head_logits"):
+        if self._plain_head():
             return model.head_logits(hidden).to(self.runner.dtype)
         idx = torch.arange(B, device=self.device)
         return model.compute_logits(hidden, idx).to(self.runner.dtype)

@@ -257,3 +257,27 @@ def test_module_hooks_run(lora):
             assert len(calls) == 1
             assert (got - plain).norm() <= 0.03 * plain.norm()  # two orders of bf16 rounding
     assert torch.equal(step(), plain)
+
+
+def test_overridden_head_reaches_the_graph():
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.models.config import get_model_config
+    from llm_instance_gateway_amd.models.llama import LlamaForCausalLM
+
+    class Negated(LlamaForCausalLM):
+        def compute_logits(self, hidden, indices):
+            return -super().compute_logits(hidden, indices)
+
+    logits = []
+    for cls in (LlamaForCausalLM, Negated):
+        torch.manual_seed(0)
+        eng = LLMEngine(EngineConfig(model=get_model_config("tiny"), num_kv_blocks=50, max_num_seqs=2, max_model_len=256),
+                        device="cuda:0")
+        eng.runner.model.__class__ = cls
+        seq = eng.add_request([5] * 9, SamplingParams(max_new_tokens=4))
+        eng.step()
+        seq.output_token_ids[-1] = 11
+        eng.step()
+        logits.append(eng.runner.graph_runner.logits[1][:1].float().clone())
+        assert seq.output_token_ids[-1] == int(logits[-1].argmax())
+    assert torch.equal(logits[1], -logits[0])
