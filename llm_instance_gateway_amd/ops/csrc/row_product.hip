@@ -12,7 +12,7 @@
 //   silu: the two rows are a gate and its up row, y = silu(gate) * up of both
 //         rounded to bf16, as silu_and_mul after the projection.
 // Widths of Llama-3-8B, weights not in any cache, against the library's product
-// with the norm and activation as kernels of their own: norm + qkv 14.3 us (18.5),
+// with the norm and activation as kernels of their own: norm + qkv 12.7 us (18.5),
 // o 8.2 (13.0), norm + gate_up + silu 45.7 (69.2, now 5.1 TB/s), down 25.5 (26.5).
 #include "common.h"
 
@@ -144,14 +144,14 @@ extern "C" int lig_row_product_max(bool norm) { return norm ? NORM_MAX : PLAIN_M
 extern "C" void lig_row_product_launch(uint16_t* y, const uint16_t* w, int N, int K, const uint16_t* x,
                                        const uint16_t* residual, uint16_t* residual_out, const uint16_t* weight,
                                        float eps, bool silu, hipStream_t stream) {
-  // large projections: more waves share the h they form
+  // with a norm 8 waves share the h they form: 6144 x 4096 12.7 us (14.8 with 4
+  // waves), 12288 x 4096 20.5 (25.2), 24576 x 8192 72 (76), 3072 x 2048 8.1 (8.5)
 #define LIG_RP(NTHR, NORM, SILU)                                                                                    \
   hipLaunchKernelGGL((row_product_kernel<NTHR, NORM, SILU>),                                                        \
                      dim3((N + NTHR / WAVE_SIZE * 2 - 1) / (NTHR / WAVE_SIZE * 2)), dim3(NTHR), (size_t)K * 2, stream, \
                      y, w, N, K, x, residual, residual_out, weight, eps)
   if (silu) LIG_RP(512, true, true);
-  else if (weight && N >= 16384) LIG_RP(512, true, false);
-  else if (weight) LIG_RP(256, true, false);
+  else if (weight) LIG_RP(512, true, false);
   else LIG_RP(256, false, false);
 #undef LIG_RP
 }
