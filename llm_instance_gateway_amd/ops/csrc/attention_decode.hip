@@ -8,20 +8,21 @@
 
 #include "flash_decode.h"
 
-// One wave per (sequence, query head, part of the walk): 8 lanes of 2 entries
+// One wave per (sequence, query head, part of the walk), four heads to a workgroup: 8 lanes of 2 entries
 // per key, 32 keys a step of which a group of lanes takes 4, each group with its
 // own running maximum, merged at the end.  Parts are flash_decode.h's and merged
 // by its second kernel.  What bounds it is the chain of a step (table entry, key,
 // reduction, exponential) and not bandwidth, hence 4 keys at once and the cut.
-// 4 query and 2 key/value heads: one row of 16000 keys 25 us, 4 of 4000 18, 64
+// 4 query and 2 key/value heads: one row of 16000 keys 26 us, 4 of 4000 19, 64
 // of 3000 24; with 8 keys a step and uncut 775, 197 and 156.
-__global__ __launch_bounds__(WAVE_SIZE) void paged_attention_decode_16_kernel(const flash_decode::Args a) {
+__global__ __launch_bounds__(4 * WAVE_SIZE) void paged_attention_decode_16_kernel(const flash_decode::Args a) {
   constexpr int D = 16, U = flash_decode::KT / 8;
-  const int seq = blockIdx.x, qh = blockIdx.y;
+  const int seq = blockIdx.x, qh = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (qh >= a.num_q_heads) return;
   const flash_decode::Walk wk = flash_decode::walk_of<false>(a, seq);
   if ((int)blockIdx.z >= wk.parts) return;
   const int kvh = qh / (a.num_q_heads / a.num_kv_heads);
-  const int tok = threadIdx.x >> 3, d = (threadIdx.x & 7) * 2;
+  const int tok = (threadIdx.x & 63) >> 3, d = (threadIdx.x & 7) * 2;
   const int* bt = a.block_tables + (size_t)seq * a.max_blocks;
   const size_t item = (size_t)seq * a.num_q_heads + qh, at = item * D + d;
   const float c = a.scale * flash_decode::LOG2E;
@@ -114,8 +115,8 @@ extern "C" void lig_paged_attention_decode_launch(
   a.max_blocks = max_blocks;
   a.nsplits = nsplits;
   if (head_dim == 16) {
-    hipLaunchKernelGGL(paged_attention_decode_16_kernel, dim3(num_seqs, num_q_heads, nsplits), dim3(WAVE_SIZE), 0,
-                       stream, a);
+    hipLaunchKernelGGL(paged_attention_decode_16_kernel, dim3(num_seqs, (num_q_heads + 3) / 4, nsplits),
+                       dim3(4 * WAVE_SIZE), 0, stream, a);
     flash_decode::launch_merge<16, false, false>(a, stream);
   } else if (head_dim == 64)
     flash_decode::launch_mode<64, false, false, false>(a, stream);
