@@ -74,10 +74,10 @@ class DecodeGraphRunner:
         self.lora_in_layer = False
 
     def _graph_nsplits(self, B: int) -> int:
-        """Bucket-static flash-decode split factor: replay can't branch on
-        live context lengths, so pick from the bucket size + the engine's max
-        context (empty split ranges merge as no-ops — bit-exact either way,
-        profiles/r01_flash_decode_split.txt)."""
+        """How many parts a bucket's decode walks may be cut into: a replay's
+        launches are fixed, so this follows from the bucket's size and the
+        engine's longest context.  The kernel takes fewer where a row is short
+        (at least 512 keys a part); the other workgroups leave at once."""
         from .. import ops
 
         shape = self._attn_shape()

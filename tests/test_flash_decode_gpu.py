@@ -148,6 +148,31 @@ def test_keys_before_the_first_visible_one(opt, D, H, G, bs):
 LONG = [1, 500, 1030, 2600, 9248, 12512, 16384]
 
 
+@pytest.mark.parametrize("nsplits", [5, 32])
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 16, 1, 32), (128, 3, 1, 6)])
+def test_many_parts(D, H, G, bs, nsplits):
+    b = _batch(LONG, G, D, bs, H, 19)
+    got = ops.paged_attention_decode(
+        b["q"].view(-1, H, D), b["k"], b["v"], b["tab"], b["ctx"], D ** -0.5, nsplits=nsplits)
+    _check(got.view(len(LONG), -1), b, D ** -0.5, H)
+
+
+@pytest.mark.parametrize("opt", [dict(sink=True, gate=True), dict(weights="sigmoid", gate=True), dict(softcap=8.0, window=9000)],
+                         ids=range(3))
+@pytest.mark.parametrize("D,H,G", [(128, 4, 1), (64, 16, 1)])
+def test_many_parts_with_options(opt, D, H, G):
+    opt = dict(opt)
+    b = _batch(LONG, G, D, 16, H, 20, pad=1)
+    assert ops.decode_nsplits(len(LONG) + 1, G, opt.get("window", 16384)) >= 17
+    if opt.pop("sink", False):
+        opt["sink"] = b["rnd"](H).float()
+    if opt.pop("gate", False):
+        opt["gate"] = b["rnd"](len(LONG) + 1, H * D)
+    got = ops.paged_attention_general(b["q"], b["k"], b["v"], b["tab"], b["tok_seq"], b["pos"], D ** -0.5, H, **opt)
+    _check(got, b, D ** -0.5, H, **opt)
+    assert (got[-1] == 0).all()
+
+
 @pytest.mark.parametrize("nsplits", [1, 5, 32])
 def test_heads_of_16(nsplits):
     H, G, D = 4, 2, 16

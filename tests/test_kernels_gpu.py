@@ -269,9 +269,9 @@ def test_sgmv_tiled_matches_ref(R, O):
 
 @pytest.mark.parametrize("N,ctx", [(4, 2048), (2, 1536)])
 def test_decode_split_default_dispatch(N, ctx):
-    """ops.paged_attention_decode with the max_ctx hint routes small-batch
-    long-context decodes to the split kernel (heuristic: N*Hkv workgroups
-    << 2*CUs) and matches the single-pass result."""
+    """ops.paged_attention_decode with the max_ctx hint cuts the walks of
+    small batches with long contexts (N*Hkv workgroups short of four per CU)
+    and matches the single-pass result."""
     HKV, HQ, D, BS = 8, 32, 128, 16
     assert ops.decode_nsplits(N, HKV, ctx) > 1  # heuristic fires for this shape
     kc, vc, bt, cl = _rand_cache_and_tables(N, HKV, D, BS, ctx, seed=21)
@@ -287,11 +287,10 @@ def test_decode_split_default_dispatch(N, ctx):
     close(pinned, single)
 
 
-@pytest.mark.parametrize("N,ctx,ns", [(4, 300, 2), (16, 1024, 4), (3, 7, 3), (8, 2048, 16)])
+# a part holds at least 512 keys: 2, 4, 3 and 16 parts, and walks too short to be cut
+@pytest.mark.parametrize("N,ctx,ns", [(4, 1300, 2), (16, 2100, 4), (3, 1540, 3), (8, 8200, 16), (4, 300, 2), (3, 7, 3)])
 def test_paged_attention_decode_split_matches(N, ctx, ns):
-    """Flash-decoding context split + combine == single-pass kernel
-    (validated 13.7x faster at N=4/ctx=16k with ns=32 —
-    profiles/r01_flash_decode_split.txt)."""
+    """A walk cut over workgroups and merged == the single pass."""
     HKV, HQ, D, BS = 8, 32, 128, 16
     kc, vc, bt, cl = _rand_cache_and_tables(N, HKV, D, BS, ctx, seed=13)
     q = torch.randn(N, HQ, D, dtype=torch.bfloat16, device=DEV) * 0.3
