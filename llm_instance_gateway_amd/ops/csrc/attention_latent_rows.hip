@@ -50,6 +50,8 @@
 // scratch; a second kernel merges the slices.  The sink is counted by slice
 // zero only.
 
+#include <type_traits>
+
 #include "elem_types.h"
 
 namespace {
@@ -152,10 +154,12 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   const int CH = D / 8;
   constexpr int NP = CHP / 8;  // fetches per piece
   auto block_of = [&](int kv0) {
-    const int t = min(max(kv0 + (FULL ? (lane & 7) * 8 : lane & (KT - 1)), kv_seen), kv_end - 1);
+    const int t = min(FULL ? kv0 + (lane & 7) * 8 : max(kv0 + (lane & (KT - 1)), kv_seen), kv_end - 1);
     return bt[FULL ? t >> block_shift : t / block_size];
   };
-  auto fetch = [&](int kv0, int blks, int buf) {
+  // Only a walk's first tile can hold keys before the first visible one (FIRST).
+  auto fetch = [&](auto first_tile, int kv0, int blks, int buf) {
+    constexpr bool FIRST = decltype(first_tile)::value;
     int here = lane;
     if (KG == 1) asm volatile("" : "+v"(here));  // worked out anew for each tile: held for the loop, it would spill
     if constexpr (FULL) {
@@ -165,14 +169,15 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int t0 = min(kv0 + piece * 8, (kv_end - 1) & ~7);
         const int blk = __builtin_amdgcn_readlane(blks, piece);
         const uint16_t* g = cache + ((size_t)blk * block_size + (t0 & (block_size - 1))) * D;
-        const int last = kv_end - 1 - t0, first = kv_seen - t0;
+        const int last = kv_end - 1 - t0;
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
           const int p = i * 64 + here;
           const int key = p / CHP;  // of the piece
           const int c = (p % CHP) ^ ((key & 3) | ((piece & 1) << 2));
+          const int from = FIRST ? max(key, kv_seen - t0) : key;
           __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void*)(g + (min(max(key, first), last) * DKP + c * 8)),
+              (const __attribute__((address_space(1))) void*)(g + (min(from, last) * DKP + c * 8)),
               (__attribute__((address_space(3))) void*)(sm + buf * TILE + (piece * NP + i) * 512), 16, 0, 0);
         }
       }
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int p = base + here;
         const int key = p / CHP;
         const int c = (p % CHP) ^ ((key & 3) | ((key >> 1) & 4));
-        const int off = min(max(kv0 + key, kv_seen), kv_end - 1) % block_size;
+        const int off = min(FIRST ? max(kv0 + key, kv_seen) : kv0 + key, kv_end - 1) % block_size;
         const int blk = __shfl(blks, key, 64);
         if (c < CH)
           __builtin_amdgcn_global_load_lds(
@@ -199,7 +204,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   }
   int blks = kv_lo < kv_hi ? block_of(kv_lo) : 0;
   if (kv_lo < kv_hi) {
-    fetch(kv_lo, blks, 0);
+    fetch(std::true_type{}, kv_lo, blks, 0);
     blks = block_of(kv_lo + KT);
   }
 
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tile is in LDS
     __syncthreads();                     // everybody's is, and the other buffer is free
     if (kv0 + KT < kv_hi) {
-      fetch(kv0 + KT, blks, buf ^ 1);
+      fetch(std::false_type{}, kv0 + KT, blks, buf ^ 1);
       blks = block_of(kv0 + 2 * KT);
     }
     const int k0 = kv0 + kg * 32;  // this wave's keys
