@@ -373,10 +373,14 @@ def sgmv_expand(u, b_stack, slots, y, scaling=1.0):
 LORA_ROWS_WIDTHS = (256, 512, 1024, 2048, 3072, 4096)  # lora_rms_norm's
 
 
-# Below this many tiles lora_rms_norm takes strips of columns in two launches
-# instead of a workgroup per tile in one.  Norms of 4096 columns with both
-# products, in one launch and in two: 9 tiles 21.4 us and 9.2, 45 tiles 23.3 and
-# 15.6, 99 tiles 24.3 and 25.9, 198 tiles 26.0 and 38.9 (two read it all twice).
+# Below this many tiles of 4096 columns, and in proportion for narrower rows down
+# to 2048, lora_rms_norm takes strips of columns in two launches instead of a
+# workgroup per tile in one: few workgroups wait for one CU's loads, many read it
+# all twice.  Both products, replayed from a graph, strips and one launch in us:
+#   4096 columns  24 tiles 11.3, 22.8   72 22.6, 25.8   104 31.2, 26.3   200 54.8, 29.7
+#   3072          24       11.6, 18.6   72 18.0, 21.1   104 23.5, 21.8   200 44.7, 24.8
+#   2048          24       11.0, 12.6   48 11.6, 13.0    72 15.7, 13.5   104 17.5, 15.4
+#   1024          24       10.6,  7.7   72 11.1,  8.2;  512 24 10.5, 5.5
 LORA_NORM_STRIPS_BELOW = 96
 
 
@@ -398,7 +402,7 @@ def lora_rms_norm(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_sta
     out = torch.empty_like(x)
     n, H, strip = rows[1].shape[0], x.shape[1], _EXT.lora_norm_strip()
     sums, parts = None, 1
-    if n < LORA_NORM_STRIPS_BELOW and H % strip == 0:
+    if H >= 2048 and n * 4096 < LORA_NORM_STRIPS_BELOW * H and H % strip == 0:
         parts = H // strip
         sums = torch.empty(n * parts * 16, dtype=torch.float32, device=x.device)
     _EXT.lora_rms_norm(out, x, residual, weight, eps, *rows, u_in, b_stack, a_stack, u_out, sums, _stream())
