@@ -821,8 +821,11 @@ def latent_rows_supported(q_dtype, row: int, v_dim: int, is_cuda: bool) -> bool:
 
 def latent_rows_nsplit(rows: int, segs: int, heads: int, max_ctx: int) -> int:
     """Context slices for the latent row kernel: 1 when the step's rows fill
-    the chip by themselves, else enough slices for about two workgroups per
-    CU, each with at least 128 keys of the longest possible context."""
+    the chip by themselves, counted in 64-row workgroups and one more a segment,
+    else enough slices for twice as many of those as CUs, each with at least 128
+    keys of the longest possible context.  (Single tokens of up to 32 heads run in
+    32-row workgroups, one to a segment and one to a CU at a time, so 171 to 255 of
+    them with 32 heads count as filling the chip and leave some CUs idle.)"""
     blocks = (rows * heads + 63) // 64 + segs
     if blocks >= _NUM_CUS or max_ctx < 512:
         return 1

@@ -6,8 +6,8 @@
 // workgroup of 16 waves takes a row, 16 bytes a lane and load.  Per 16 bytes
 // only the largest value is formed and compared with the best so far (3 ops a
 // value); the place inside the winning 16 bytes is looked up at the end.
-// 384 rows 25.7 us (3.8 TB/s), one row 8.8; torch's reduction after a conversion
-// to fp32 took 104 and 39, without it 59 and 31.
+// 384 rows 23 us (4.3 TB/s; 25 in an engine step), one row 8.7 (11); torch's
+// reduction after a conversion to fp32 took 104 and 39, without it 59 and 31.
 #include "common.h"
 
 namespace {

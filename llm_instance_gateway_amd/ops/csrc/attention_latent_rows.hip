@@ -30,9 +30,10 @@
 // workgroup, tiles of 64 keys of which waves 0-1 and 2-3 take a half each and
 // merge at the end, one workgroup with 144 KB on the way or in use per CU.
 // Measured with rows of 576 and values of 512, before -> after: 256 single tokens
-// on 700-1024 keys, 32 heads 156 -> 75 us (3.4 TB/s), 16 heads 150 -> 71; 32 such
-// tokens 37 -> 25; 4 prompts of 700-1000, 16 heads 306 -> 118 us (154 -> 399
-// TFLOP/s), 32 heads 540 -> 180. Two row blocks per wave, which halve the LDS
+// on 700-1024 keys, 32 heads 148 -> 72 us (255 MB of rows, 3.6 TB/s; 62 us where
+// they are still in the last-level cache), 16 heads 146 -> 69; 32 such tokens 37 ->
+// 23; 4 prompts of 700-1000, 16 heads 322 -> 121 us (164 -> 437 TFLOP/s), 32 heads
+// 540 -> 185. Two row blocks per wave, which halve the LDS
 // reads, lost more by leaving one wave per SIMD (keys of 320: 372 us before, 136
 // now, 208 so; of 128: 149, 73, 135).
 // Scores, running max and sum are fp32; an optional per-head sink starts a

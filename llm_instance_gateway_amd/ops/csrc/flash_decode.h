@@ -29,8 +29,9 @@
 //     kernel.
 // Measured, 32 query and 8 key/value heads of 128, before -> after: 384
 // requests of 190-381 tokens 173 -> 84 us (5.3 TB/s; a large copy reaches 4.9);
-// 33 of 3000-6000 370 -> 114 us; 16 of 190-381 30 -> 8.3 us; 64 rows with a
-// window of 512 and sigmoid weights 64 -> 28 us.  Eight waves per workgroup
+// 33 of 3000-6000 370 -> 119 us (5.0 TB/s); 16 of 190-381 30 -> 8.2 us; 64 rows
+// with a window of 512 and sigmoid weights 54 -> 28 us, 44 -> 24 where their 134 MB
+// are still in the last-level cache.  Eight waves per workgroup
 // were slower from 64 requests on (101 us at 384), two on few (9.2 us at 16).
 #pragma once
 

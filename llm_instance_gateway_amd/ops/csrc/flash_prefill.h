@@ -23,9 +23,10 @@
 //   * the accumulators are only rescaled when a row's maximum grew, and masks
 //     are only evaluated on tiles that cross a row's visible range.
 // Measured, 32 query and 8 key/value heads of 128, before -> after: 4096 rows
-// on 4000 cached keys 3409 -> 495 us (119 -> 820 TFLOP/s); 20 prompts of 200
-// 130 -> 42 us; one of 202 20.6 -> 10.1 us; 8 of 1000 with a window of 512
-// 571 -> 114 us, with a soft cap 578 -> 137, with sigmoid weights 566 -> 110.
+// on 4000 cached keys 3409 -> 495 us (119 -> 820 TFLOP/s; 571 us, 711 TFLOP/s,
+// between the products of an engine step); 20 prompts of 200 130 -> 37 us; one of
+// 202 20.6 -> 8.9 us; 8 of 1000 with a window of 512 571 -> 110 us, with a soft cap
+// 578 -> 133, with sigmoid weights 566 -> 103.
 // Four heads per workgroup and 64 rows per wave (all 512 registers, one wave
 // per SIMD) was slower everywhere: 781 us in the first of these.
 #pragma once
@@ -429,7 +430,9 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   }
 }
 
-// What the kernel takes; callers without another kernel check it themselves.
+// What the kernel takes.  The Llama path has no other kernel and does not ask: its
+// binding admits contiguous bf16 tensors with heads of 64 or 128 only, and relies
+// on the allocator's alignment and on head counts that divide.
 static inline bool serves(const Args& a, int D, int Dv) {
   auto al = [](const void* p, unsigned to) { return (reinterpret_cast<uintptr_t>(p) & (to - 1)) == 0; };
   return D == Dv && (D == 64 || D == 128) && a.q_stride % 8 == 0 && a.v_row % 8 == 0 && a.v_row >= D &&
@@ -448,9 +451,11 @@ static void launch_heads(const Args& a, int ntiles, hipStream_t stream) {
 template <int D, bool CAP, bool SIG, bool EXTRA>
 static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
   // Two heads per workgroup halve the reads of K and V; the line is where
-  // that leaves two workgroups for every CU (heads of 128, 32 over 8):
-  // 1280 workgroups 41.6 us against 47.8 with one head, 4096 rows on 4000 keys
-  // 495 against 680, but 96 workgroups 34 us against 25, 64 12.6 against 10.1
+  // that leaves two workgroups for every CU (heads of 128, 32 over 8; two heads
+  // against one): 1280 workgroups 37.5 us against 44.0, 512 of 200 keys 17.0
+  // against 21.8, of 2048 71.4 against 72.6, 4096 rows on 4000 keys 498 against
+  // 683, but 256 workgroups of 4000 keys 126 us against 109, 96 of 1000 37.9
+  // against 28.3, 64 11.5 against 8.9
   const int group = a.num_q_heads / a.num_kv_heads;
   if (group % 2 == 0 && (long)ntiles * (a.num_q_heads / 2) >= 512)
     launch_heads<D, 2, CAP, SIG, EXTRA>(a, ntiles, stream);

@@ -12,8 +12,8 @@
 //   silu: the two rows are a gate and its up row, y = silu(gate) * up of both
 //         rounded to bf16, as silu_and_mul after the projection.
 // Widths of Llama-3-8B, weights not in any cache, against the library's product
-// with the norm and activation as kernels of their own: norm + qkv 12.7 us (18.5),
-// o 8.2 (13.0), norm + gate_up + silu 45.7 (69.2, now 5.1 TB/s), down 25.5 (26.5).
+// with the norm and activation as kernels of their own: norm + qkv 12.6 us (18.5),
+// o 8.5 (13.0), norm + gate_up + silu 43.0 (69.2, now 5.5 TB/s), down 24.2 (26.5).
 #include "common.h"
 
 namespace {
