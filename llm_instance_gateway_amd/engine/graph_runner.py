@@ -184,7 +184,8 @@ class DecodeGraphRunner:
     def capture(self, with_lora: bool) -> None:
         self.with_lora = with_lora
         mgr = self.runner.adapter_manager
-        self.lora_in_layer = with_lora and getattr(mgr, "in_layer", False)
+        # (not over modules whose hooks or replaced forwards belong into the graph)
+        self.lora_in_layer = with_lora and getattr(mgr, "in_layer", False) and self.runner.model.plain_layers()
         # one buffer for the inputs of any bucket (the largest needs the most)
         total = lay_out(self._fields(self.max_bs).values())[1]
         self._dev = torch.zeros(total, dtype=torch.uint8, device=self.device)

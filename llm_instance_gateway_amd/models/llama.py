@@ -214,8 +214,8 @@ class LlamaForCausalLM(nn.Module):
         meta: BatchMeta,
     ) -> torch.Tensor:
         hidden = self.embed_tokens(input_ids)
-        # (a graph being captured brings row tiles only, and would not run hooks again)
-        if meta.lora_rows_tok is not None and (meta.lora_slot_per_token is None or self._plain_layers()):
+        # (a graph being captured brings row tiles only where plain_layers() allowed them)
+        if meta.lora_rows_tok is not None and (meta.lora_slot_per_token is None or self.plain_layers()):
             return self._forward_lora(hidden, positions, kv_caches, meta)
         if hidden.shape[0] == 1 and meta.lora_slot_per_token is None and self._row_products():
             return self._forward_row(hidden, positions, kv_caches, meta)
@@ -227,14 +227,16 @@ class LlamaForCausalLM(nn.Module):
         hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
-    def _plain_layers(self) -> bool:
+    def plain_layers(self) -> bool:
+        """Whether no layer, attention or feed-forward module carries a forward
+        hook or a forward of its own that kernels in its place would pass by."""
         return not _has_any_global_hook() and all(
             _plain(m) for layer in self.layers for m in (layer, layer.self_attn, layer.mlp)
         )
 
     def _row_products(self) -> bool:
         """Whether every projection of a layer is one that `ops.row_product` serves."""
-        if self.tp is not None or not self._plain_layers():
+        if self.tp is not None or not self.plain_layers():
             return False
         most = ops.row_product_most(self.norm)
         for layer in self.layers:

@@ -281,3 +281,39 @@ def test_overridden_head_reaches_the_graph():
         logits.append(eng.runner.graph_runner.logits[1][:1].float().clone())
         assert seq.output_token_ids[-1] == int(logits[-1].argmax())
     assert torch.equal(logits[1], -logits[0])
+
+
+@pytest.mark.parametrize("lora", [False, True])
+def test_hooks_are_captured(lora):
+    """What a forward hook does to a module's output is part of the decode graph."""
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.lora import manager
+    from llm_instance_gateway_amd.models.config import ModelConfig
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=512, num_layers=2, num_heads=8, num_kv_heads=2,
+                     intermediate_size=1024, head_dim=64, max_position_embeddings=512)
+    logits = {}
+    for eager in (True, False):
+        torch.manual_seed(0)
+        eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=50, max_num_seqs=2, max_model_len=256,
+                                     enforce_eager=eager, pad_batch_multiple=0), device="cuda:0")
+        model = eng.runner.model
+        model.layers[0].mlp.register_forward_hook(lambda m, a, out: -out)
+        if lora:
+            mgr = manager.AdapterManager(eng, max_slots=1, rank=16)
+            mgr.register_random("l0", seed=1)
+        seqs = [eng.add_request([5 + i] * 9, SamplingParams(max_new_tokens=30),
+                                lora_name="l0" if lora and i else "") for i in range(2)]
+        eng.step()
+        out, head = [], model.compute_logits
+        for _ in range(3):
+            for i, q in enumerate(seqs):
+                q.output_token_ids[-1] = 11 + i
+            if eager:
+                model.compute_logits = lambda h, idx: out.append(head(h, idx)) or out[-1]
+            eng.step()
+            if not eager:
+                out.append(eng.runner.graph_runner.logits[2][:2].float().clone())
+        logits[eager] = out
+    for a, b in zip(logits[False], logits[True]):
+        assert (a - b).norm() <= 0.03 * b.norm()  # two orders of bf16 rounding
