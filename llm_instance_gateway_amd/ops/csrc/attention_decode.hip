@@ -25,7 +25,7 @@ __global__ __launch_bounds__(4 * WAVE_SIZE) void paged_attention_decode_16_kerne
   const int tok = (threadIdx.x & 63) >> 3, d = (threadIdx.x & 7) * 2;
   const int* bt = a.block_tables + (size_t)seq * a.max_blocks;
   const size_t item = (size_t)seq * a.num_q_heads + qh, at = item * D + d;
-  const float c = a.scale * flash_decode::LOG2E;
+  const float c = a.scale * LOG2E;
   const float q0 = bf16_to_f32(a.q[at]), q1 = bf16_to_f32(a.q[at + 1]);
   const int span = (wk.steps + wk.parts - 1) / wk.parts;
   const int s0 = blockIdx.z * span, s1 = min(wk.steps, s0 + span);
@@ -111,7 +111,7 @@ extern "C" void lig_paged_attention_decode_launch(
   a.num_kv_heads = num_kv_heads;
   a.v_row = head_dim;
   a.block_size = block_size;
-  a.block_shift = flash_decode::shift_of(block_size);
+  a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
   a.nsplits = nsplits;
   if (head_dim == 16) {

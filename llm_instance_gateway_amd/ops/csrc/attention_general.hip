@@ -452,7 +452,7 @@ void lig_paged_attention_general(
   fa.num_kv_heads = G;
   fa.v_row = v_row;
   fa.block_size = BS;
-  fa.block_shift = flash_decode::shift_of(BS);
+  fa.block_shift = shift_of(BS);
   fa.max_blocks = max_blocks;
   fa.chunk = chunk;
   fa.window = window;

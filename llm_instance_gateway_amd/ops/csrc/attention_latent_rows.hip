@@ -64,16 +64,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int LR_PART_PAD = 4;  // a slice row is Dv values, running max (log2 units), running sum, 2 unused
-constexpr float LR_LOG2E = 1.44269504088896340736f;
-
-LIG_DEVICE float lr_group_max(float x) {  // max over the four 16-lane groups
-  const uint32_t u = __builtin_bit_cast(uint32_t, x);
-  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
-  const uint32_t v = __builtin_bit_cast(uint32_t, y);
-  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
-}
 
 // KG key groups of 32 keys per tile, 4 / KG waves of 16 rows for each.
 // FULL: D == DKP, Dv == DVP and the block size is a power of two, at least 8
@@ -211,7 +201,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
 
   // a negative scale goes into the sign of the query
   const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
-  const float c2 = fabsf(scale) * LR_LOG2E;
+  const float c2 = fabsf(scale) * LOG2E;
   bf16x8_t q_frag[KB];
   {
     const uint16_t* qp = q + ((size_t)lo * H + rr) * D;
@@ -227,7 +217,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   }
 
   const bool with_sink = sink != nullptr && z == 0 && kg == 0;
-  float m = with_sink ? sink[head] * LR_LOG2E : -INFINITY;
+  float m = with_sink ? sink[head] * LOG2E : -INFINITY;
   float l = with_sink && lg == 0 ? 1.0f : 0.0f;  // this lane's part of the sum
   f32x4_t acc[DB];
 #pragma unroll
@@ -311,7 +301,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     float mx = s4[0][0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s4[e >> 2][e & 3]);
-    mx = lr_group_max(mx);
+    mx = max_over_groups(mx);
     mx = mx == -INFINITY ? mx : mx * c2;
     if (__any(mx > m)) {
       const float m_new = fmaxf(m, mx);

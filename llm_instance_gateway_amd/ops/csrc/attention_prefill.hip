@@ -29,7 +29,7 @@ extern "C" void lig_paged_attention_prefill_launch(
   a.num_kv_heads = num_kv_heads;
   a.v_row = head_dim;
   a.block_size = block_size;
-  a.block_shift = flash_prefill::shift_of(block_size);
+  a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
   if (head_dim == 64)
     flash_prefill::launch_mode<64, false, false, false>(a, ntiles, stream);

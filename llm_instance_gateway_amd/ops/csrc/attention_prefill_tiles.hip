@@ -332,7 +332,7 @@ extern "C" int lig_paged_attention_prefill_tiles(
   a.num_kv_heads = num_kv_heads;
   a.v_row = v_row;
   a.block_size = block_size;
-  a.block_shift = flash_prefill::shift_of(block_size);
+  a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
   a.chunk = chunk;
   a.window = window;

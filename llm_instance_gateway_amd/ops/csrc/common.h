@@ -29,8 +29,8 @@ LIG_DEVICE uint16_t f32_to_bf16(float f) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
-// 8 bf16 = 16 B: the unit of a fully-coalesced per-lane load (guide §2:
-// 16 B/lane x 64 lanes = 1 KiB per instruction).
+// 8 bf16 = 16 B: the unit of a fully-coalesced per-lane load (16 B/lane x
+// 64 lanes = 1 KiB per instruction).
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -86,6 +86,23 @@ LIG_DEVICE float stride_reduce_max(float v) {
   for (int off = STRIDE; off < STRIDE * N; off <<= 1)
     v = fmaxf(v, __shfl_xor(v, off, WAVE_SIZE));
   return v;
+}
+
+// Max over the four 16-lane groups, result in all of them; no LDS traffic.
+LIG_DEVICE float max_over_groups(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t v = __builtin_bit_cast(uint32_t, y);
+  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+constexpr float LOG2E = 1.44269504088896340736f;
+
+// log2 of a cache's block size, -1 if that is no power of two
+static inline int shift_of(int block_size) {
+  return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
 }
 
 LIG_DEVICE int cdiv(int a, int b) { return (a + b - 1) / b; }

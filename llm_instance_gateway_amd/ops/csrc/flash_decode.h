@@ -47,7 +47,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int KT = 32;  // keys per step
-constexpr float LOG2E = 1.44269504088896340736f;
 
 struct Args {
   uint16_t* out;            // [R, Hq * D]
@@ -78,15 +77,6 @@ struct Args {
   float softcap;
   int nsplits;
 };
-
-LIG_DEVICE float swap_max(float x) {  // max over the four 16-lane groups
-  const uint32_t u = __builtin_bit_cast(uint32_t, x);
-  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
-  const uint32_t v = __builtin_bit_cast(uint32_t, y);
-  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
-}
 
 // The steps of a row: its position and lower bound, and into how many parts
 // its walk is cut: the caller's number, but no part under 16 steps (512 keys),
@@ -293,7 +283,7 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
         float mx = s4[0][0];
 #pragma unroll
         for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s4[e >> 2][e & 3]);
-        mx = swap_max(mx);
+        mx = max_over_groups(mx);
         mx = mx == -INFINITY ? mx : CAP ? cap2 * tanhf(mx * c) : mx * c;
         if (__any(mx > m)) {
           const float m_new = fmaxf(m, mx);
@@ -491,10 +481,6 @@ static inline bool serves(const Args& a, int D, int Dv) {
   return D == Dv && (D == 64 || D == 128) && a.num_q_heads % a.num_kv_heads == 0 &&
          a.num_q_heads / a.num_kv_heads <= 16 && a.q_stride % 8 == 0 && a.v_row % 8 == 0 && a.v_row >= D &&
          al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
-}
-
-static inline int shift_of(int block_size) {
-  return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
 }
 
 template <int D, bool SIG, bool EXTRA>

@@ -42,7 +42,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int KT = 64;      // keys per tile
 constexpr int TQ = 64;      // query rows of a tile of the caller's tile list
-constexpr float LOG2E = 1.44269504088896340736f;
 
 struct Args {
   uint16_t* out;            // [R, Hq * D]
@@ -70,16 +69,6 @@ struct Args {
   int gate_per_head;
   float softcap;
 };
-
-// max over the four 16-lane groups, result in all of them
-LIG_DEVICE float max_over_groups(float x) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, x);
-  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
-  const uint32_t v = __builtin_bit_cast(uint32_t, y);
-  auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
-}
 
 LIG_DEVICE uint32_t pack_bf16(float a, float b) {
   return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
@@ -461,10 +450,6 @@ static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
     launch_heads<D, 2, CAP, SIG, EXTRA>(a, ntiles, stream);
   else
     launch_heads<D, 1, CAP, SIG, EXTRA>(a, ntiles, stream);
-}
-
-static inline int shift_of(int block_size) {
-  return block_size > 0 && (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
 }
 
 }  // namespace flash_prefill
