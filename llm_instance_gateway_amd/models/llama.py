@@ -29,10 +29,9 @@ from ..engine.metadata import BatchMeta
 from .config import ModelConfig
 
 
-def _plain(module: nn.Module) -> bool:
-    """Whether calling the module runs its class's forward and nothing else, so
-    that kernels may take its place."""
-    d = module.__dict__
+def _plain(d: dict) -> bool:
+    """Whether calling the module with these attributes runs its class's forward
+    and nothing else, so that kernels may take its place."""
     return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
 
 
@@ -228,11 +227,22 @@ class LlamaForCausalLM(nn.Module):
         return hidden
 
     def plain_layers(self) -> bool:
-        """Whether no layer, attention or feed-forward module carries a forward
-        hook or a forward of its own that kernels in its place would pass by."""
-        return not _has_any_global_hook() and all(
-            _plain(m) for layer in self.layers for m in (layer, layer.self_attn, layer.mlp)
-        )
+        """Whether the layers, their attention and feed-forward modules run this
+        file's forwards and nothing else: no forward hook, no other class, no
+        forward of an instance's own that kernels in their place would pass by.
+        Asked on every eager step, so it goes by the modules' dictionaries."""
+        if _has_any_global_hook():
+            return False
+        for layer in self.layers:
+            if type(layer) is not DecoderLayer or not _plain(layer.__dict__):
+                return False
+            parts = layer.__dict__["_modules"]
+            attn, mlp = parts["self_attn"], parts["mlp"]
+            if type(attn) is not Attention or type(mlp) is not MLP:
+                return False
+            if not (_plain(attn.__dict__) and _plain(mlp.__dict__)):
+                return False
+        return True
 
     def _row_products(self) -> bool:
         """Whether every projection of a layer is one that `ops.row_product` serves."""
@@ -242,7 +252,7 @@ class LlamaForCausalLM(nn.Module):
         for layer in self.layers:
             attn, mlp = layer.self_attn, layer.mlp
             for m, norm in ((attn.qkv_proj, True), (attn.o_proj, False), (mlp.gate_up_proj, True), (mlp.down_proj, False)):
-                if type(m) is not nn.Linear or not _plain(m):
+                if type(m) is not nn.Linear or not _plain(m.__dict__):
                     return False
                 p = m._parameters
                 if p["bias"] is not None or not ops.row_product_serves(p["weight"], norm, most):

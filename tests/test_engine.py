@@ -309,3 +309,33 @@ def test_max_new_tokens_clamped_to_context_window():
     assert seq.sampling.max_new_tokens == 14  # 64 - 50
     eng.generate_all()
     assert seq.total_len <= 64
+
+
+def test_plain_layers():
+    """Kernels may take the place of Llama's modules only where these are the
+    model's own and run nothing beside their forward."""
+    import torch.nn as nn
+
+    from llm_instance_gateway_amd.models.config import get_model_config
+    from llm_instance_gateway_amd.models.llama import MLP, LlamaForCausalLM
+
+    class Other(MLP):
+        pass
+
+    model = LlamaForCausalLM(get_model_config("tiny"), dtype=torch.float32)
+    assert model.plain_layers()
+    last = model.layers[len(model.layers) - 1]
+    for m in (last, last.self_attn, last.mlp):
+        for register in (m.register_forward_hook, m.register_forward_pre_hook):
+            handle = register(lambda *a: None)
+            assert not model.plain_layers()
+            handle.remove()
+        m.forward = m.forward
+        assert not model.plain_layers()
+        del m.forward
+        assert model.plain_layers()
+    handle = nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not model.plain_layers()
+    handle.remove()
+    last.mlp.__class__ = Other
+    assert not model.plain_layers()
