@@ -155,12 +155,17 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
     for (int d = tid; d < group * D; d += 64 * W) a.out[((size_t)row * a.num_q_heads + kvh * group) * D + d] = 0;
     return;
   }
-  // A walk of one step: the other waves would hold their registers against the
-  // workgroups that wait, and there is nothing to merge.  384 rows of 20 keys 9.8
-  // us (19.6 with all four waves at the barrier, 14.7 in the kernel before), 335
-  // of 7 with 64 heads 8.7 (28, 17); the branch costs walks of 3 or 4 steps 3 %
+  // Waves without a step would hold their registers against the workgroups that
+  // wait, and a walk of one step has nothing to merge.  384 rows of 10-20 keys 10.7
+  // us (20.4 with all four waves at the barrier, 15.9 in the kernel before), of
+  // 30-60 19.1 (23.2, 28.4), with 64 heads 25.6 (32.6, 52); walks of 3 to 5 steps
+  // up to 5 % slower.  Where every head has keys of its own, short rows remain
+  // slower than before, with a matrix for one head: 32 heads, 384 rows of 10-20
+  // keys 29 (51, 20), of 30-60 56 (65, 48), of 50-100 87 (92, 96).  One wave per
+  // key/value head and four of these to a workgroup was slower: 22 for the first.
   const bool one_step = wk.steps <= 1;
-  if (one_step && wave != 0) return;
+  const int nw = min(W, max(1, wk.steps));
+  if (wave >= nw) return;  // a barrier waits only for waves that have not ended
   const int pos = wk.pos, key_lo = wk.key_lo;
   const int* bt = a.block_tables + (size_t)wk.seq * a.max_blocks;
   float sc = a.scale;
@@ -403,7 +408,7 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
     }
   }
   __syncthreads();
-  for (int it = tid; it < group * (D / 4); it += 64 * W) {
+  for (int it = tid; it < group * (D / 4); it += 64 * nw) {
     const int hh = it / (D / 4), d = (it % (D / 4)) * 4;
     const int head = kvh * group + hh;
     const bool sink = EXTRA && !SIG && a.sink && wk.parts == 1;
@@ -413,11 +418,13 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
     if constexpr (!SIG) {
       const float sm = gm;
 #pragma unroll
-      for (int w = 0; w < W; ++w) gm = fmaxf(gm, m_s[w * GM + hh]);
+      for (int w = 0; w < W; ++w)
+        if (w < nw) gm = fmaxf(gm, m_s[w * GM + hh]);
       if (sink) gl = __builtin_amdgcn_exp2f(sm - gm);
     }
 #pragma unroll
     for (int w = 0; w < W; ++w) {
+      if (w >= nw) break;
       float f = 1.f;
       if constexpr (!SIG) {
         f = m_s[w * GM + hh] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_s[w * GM + hh] - gm);
