@@ -74,7 +74,7 @@ def main() -> None:
     ap.add_argument("--steps", type=int, default=128)
     ap.add_argument("--warmup", type=int, default=32)
     ap.add_argument("--model", default="llama3-8b")
-    # conc sweep on MI355X (gpurun_out/sw_c*.log): 256→54.2, 384→67.0,
+    # conc sweep on MI355X: 256→54.2, 384→67.0,
     # 512→67.0 req/s with worsening TPOT; 384 saturates the chip
     # (~25.4k tok/s) with TTFT p95 ~44 ms and is the default operating point.
     ap.add_argument("--concurrency", type=int, default=384)
@@ -330,7 +330,7 @@ def main() -> None:
     # -- warmup (untimed) ----------------------------------------------------
     # Contract floor: W untimed steps.  Then warm BY STATE: the closed loop
     # starts with `concurrency` simultaneous arrivals whose prefill flood
-    # dominates any short timed window (r01's 5.95 vs 32.9 req/s defect).
+    # dominates any short timed window (5.95 against 32.9 req/s once).
     # Keep stepping until EVERY member of that initial flood has finished —
     # any survivor would carry its cold-start admission wait (measured: the
     # last flood prompts admit ~2 s after t=0 at conc=256) into the timed

@@ -54,7 +54,7 @@ class BatchMeta:
     lora_tile_t0: Optional[torch.Tensor] = None    # [ntiles] int32
     lora_tile_len: Optional[torch.Tensor] = None   # [ntiles] int32
     lora_tile_slot: Optional[torch.Tensor] = None  # [ntiles] int32
-    # Slot-grouped SGMV units (r02 default path): tokens sorted by adapter
+    # Slot-grouped SGMV units (the default path): tokens sorted by adapter
     # slot (`lora_order`), chunked into <=32-token same-slot units so the
     # kernels read each adapter's weights once per unit.
     lora_order: Optional[torch.Tensor] = None      # [T] int32

@@ -39,7 +39,7 @@ log = logging.getLogger(__name__)
 # further work; the wide per-token kernels are the default.
 _TILED_SGMV = os.environ.get("LIG_TILED_SGMV", "0") == "1"
 
-# Slot-grouped unit kernels (r02): default ON; LIG_SGMV_UNITS=0 falls back to
+# Slot-grouped unit kernels: default ON; LIG_SGMV_UNITS=0 falls back to
 # the per-token/wide kernels for A/B.
 _UNITS_SGMV = os.environ.get("LIG_SGMV_UNITS", "1") == "1"
 
@@ -427,7 +427,7 @@ class AdapterManager:
             if ws is None:
                 ws = self._u_ws
             assert ws.shape[0] >= T, "LoRA workspace smaller than flat batch"
-            # slot-grouped units (r02 default): shrink on the occupancy-first
+            # slot-grouped units (the default): shrink on the occupancy-first
             # v2 kernels, expand via the LDS-staged unit kernel (B read once
             # per <=32-token unit; profiles/r02_kernel_stats.md)
             order = getattr(meta, "lora_order", None)

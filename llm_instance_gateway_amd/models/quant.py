@@ -23,14 +23,12 @@ reported separately and marked as such.  Reference analogue: vLLM's
 --quantization fp8 serving mode on the fleet the reference routes to
 (SURVEY.md §2.3); implementation is original and MI355X-native.
 
-MEASURED STATUS (r02, 1x MI355X, tests/test_quant_gpu.py 7/7 green):
+MEASURED STATUS (1x MI355X, tests/test_quant_gpu.py 7/7 green):
   * with torch elementwise activation quant (~4 launches + 3 passes over
-    x per projection): a NON-win — 69.4 vs 74.6 req/s at conc=384
-    (gpurun_out/bench_fp8.log);
+    x per projection): a NON-win — 69.4 vs 74.6 req/s at conc=384;
   * with the fused ONE-launch quant kernel (ops.quant_fp8_rowwise,
     ops/csrc/quant.hip): **84.97 vs 74.6 req/s at conc=384 (+14%)** and
-    35.7 vs 31.6 at conc=64 (+13%) — bench_fp8_fused.log,
-    bench_c64_fp8_fused.log.  The quant overhead was the entire penalty.
+    35.7 vs 31.6 at conc=64 (+13%).  The quant overhead was the entire penalty.
 The headline benchmark still reports bf16 (BASELINE's dtype); fp8 runs
 carry dtype="fp8" in the bench JSON.
 

@@ -370,7 +370,7 @@ void sgmv_apply(torch::Tensor y, torch::Tensor x, torch::Tensor a_stack,
                          use_wide, st);
 }
 
-// Slot-grouped units (r02): shrink via the proven v2 kernels (occupancy-
+// Slot-grouped units: shrink via the proven v2 kernels (occupancy-
 // first), expand via the LDS-staged unit kernel — full per-token thread
 // parallelism with B read once per <=32-token unit instead of per token
 // (profiles/r02_kernel_stats.md: the per-token kernels were 27% of all

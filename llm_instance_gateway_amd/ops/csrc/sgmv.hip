@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) void sgmv_expand_tiled_kernel(
   }
 }
 
-// ---- slot-grouped "unit" kernels (r02) -------------------------------------
+// ---- slot-grouped "unit" kernels -------------------------------------
 //
 // r02 steady-state profile (profiles/r02_kernel_stats.md): the four SGMV
 // kernels above are 27% of all kernel time, dominated by re-reading adapter

@@ -38,7 +38,7 @@ def maybe_enable_tunableop() -> bool:
 
     Serving mode loads the tuned results but leaves TunableOp DISABLED
     globally; the model runner flips it on only around eager forwards
-    (``eager_tuned()``).  MEASURED on MI355X (r01, gpurun_out/bench4.log):
+    (``eager_tuned()``).  MEASURED on MI355X:
     TunableOp active during hipGraph capture made the bench 3x slower
     (35.8 vs 12.4 ms/step) — the tunable GEMM wrapper defeats capture, so
     graphs keep the default algorithms and only eager (mixed prefill)

@@ -19,7 +19,7 @@ if str(REPO_ROOT) not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line(
-        "markers", "gpu: tests that require an MI355X GPU (run via gpurun)"
+        "markers", "gpu: tests that require an MI355X GPU"
     )
     # hang protection for the driver's round checks (pytest-timeout)
     if config.getoption("--timeout", None) in (None, 0):
