@@ -29,11 +29,12 @@
 // 32 keys, two workgroups per CU. Others (one token of up to 32 heads): 32 per
 // workgroup, tiles of 64 keys of which waves 0-1 and 2-3 take a half each and
 // merge at the end, one workgroup with 144 KB on the way or in use per CU.
-// Measured with rows of 576 and values of 512, before -> after: 256 single tokens
-// on 700-1024 keys, 32 heads 148 -> 72 us (255 MB of rows, 3.6 TB/s; 62 us where
-// they are still in the last-level cache), 16 heads 146 -> 69; 32 such tokens 37 ->
-// 23; 4 prompts of 700-1000, 16 heads 322 -> 121 us (164 -> 437 TFLOP/s), 32 heads
-// 540 -> 185. Two row blocks per wave, which halve the LDS
+// The fetches are load_to_lds: as the compiler's builtin, the first LDS read of a
+// tile waited for the next tile's fetches too, and nothing was on its way meanwhile.
+// Measured with rows of 576 and values of 512 (us; a kernel that staged through
+// registers -> with the builtin -> now): 256 single tokens on 700-1024 keys, 32
+// heads 148 -> 72 -> 63 (255 MB of rows, 4.1 TB/s); 4 prompts of 700-1000, 16 heads
+// 322 -> 121 -> 97 (546 TFLOP/s). Two row blocks per wave, which halve the LDS
 // reads, lost more by leaving one wave per SIMD (keys of 320: 372 us before, 136
 // now, 208 so; of 128: 149, 73, 135).
 // Scores, running max and sum are fp32; an optional per-head sink starts a
@@ -142,6 +143,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   // FULL: 8 keys, aligned, are one contiguous piece of a block; a wave takes
   // KT / 32 such pieces of CHP / 8 fetches.  Lane j looks up the block of piece j
   // of the tile after next.  Else every lane looks for its own key's block.
+  const uint32_t lds = lds_address(sm);
   const int CH = D / 8;
   constexpr int NP = CHP / 8;  // fetches per piece
   auto block_of = [&](int kv0) {
@@ -167,9 +169,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
           const int key = p / CHP;  // of the piece
           const int c = (p % CHP) ^ ((key & 3) | ((piece & 1) << 2));
           const int from = FIRST ? max(key, kv_seen - t0) : key;
-          __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void*)(g + (min(from, last) * DKP + c * 8)),
-              (__attribute__((address_space(3))) void*)(sm + buf * TILE + (piece * NP + i) * 512), 16, 0, 0);
+          load_to_lds(g, (min(from, last) * DKP + c * 8) * 2, lds + (buf * TILE + (piece * NP + i) * 512) * 2);
         }
       }
     } else {
@@ -182,9 +182,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int off = min(FIRST ? max(kv0 + key, kv_seen) : kv0 + key, kv_end - 1) % block_size;
         const int blk = __shfl(blks, key, 64);
         if (c < CH)
-          __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void*)(cache + ((size_t)blk * block_size + off) * D + c * 8),
-              (__attribute__((address_space(3))) void*)(sm + buf * TILE + base * 8), 16, 0, 0);
+          load_to_lds(cache + ((size_t)blk * block_size + off) * D + c * 8, lds + (buf * TILE + base * 8) * 2);
       }
     }
   };
@@ -225,8 +223,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
 
   int buf = 0;
   for (int kv0 = kv_lo; kv0 < kv_hi; kv0 += KT, buf ^= 1) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tile is in LDS
-    __syncthreads();                     // everybody's is, and the other buffer is free
+    loads_landed<0>();  // the tile is in LDS, and the other buffer is free
     if (kv0 + KT < kv_hi) {
       fetch(std::false_type{}, kv0 + KT, blks, buf ^ 1);
       blks = block_of(kv0 + 2 * KT);
@@ -234,6 +231,11 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     const int k0 = kv0 + kg * 32;  // this wave's keys
     if (!wave_active || k0 >= kv_hi) continue;
     const uint16_t* tile = sm + buf * TILE + kg * 32 * DKP;
+    // LDS addresses anew for each tile as well: a spilled one is loaded back
+    // behind the next tile's fetches, and waits for them
+    int here = lane;
+    if (KG == 1) asm volatile("" : "+v"(here));
+    const int li = here & 15, lg = here >> 4;
 
     // Operands are read from LDS in batches of 4, the next batch ahead of the
     // products of this one.

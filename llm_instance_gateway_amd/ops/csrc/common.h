@@ -98,6 +98,30 @@ LIG_DEVICE float max_over_groups(float x) {
   return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
 }
 
+// ---- memory -> LDS ------------------------------------------------------------
+// 16 bytes per lane to `lds` (uniform) + lane * 16, no registers in between.  As
+// the builtin, every LDS read behind it would wait for it, whatever it reads: a
+// tile could not be on its way while another is used.  So these are invisible to
+// the compiler's counting, and the code that reads the bytes waits by itself:
+// loads_landed<n> before the barrier behind which they are read.  (The compiler's
+// own waits for loads count in order and can only be longer for it.)
+// One wait state between a write to m0 and its use.
+LIG_DEVICE uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p);
+}
+LIG_DEVICE void load_to_lds(const void* base, uint32_t offset, uint32_t lds) {  // base: uniform
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(offset), "{m0}"(lds) : "memory");
+}
+LIG_DEVICE void load_to_lds(const void* p, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "{m0}"(lds) : "memory");
+}
+// All but this wave's last N loads have landed and its LDS reads are done, and so
+// are those of the other waves.
+template <int N>
+LIG_DEVICE void loads_landed() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 constexpr float LOG2E = 1.44269504088896340736f;
 
 // log2 of a cache's block size, -1 if that is no power of two
