@@ -199,18 +199,17 @@ class ModelRunner:
 
         # GEMM M-bucketing: pad the flat batch tail so every projection GEMM
         # sees M % pad_batch_multiple == 0 (few stable shapes -> hipBLASLt
-        # algo reuse + tile-friendly M).  Pad rows: token 0 at position 0,
-        # K/V scattered to the scratch block (same slot — racy garbage is
-        # fine there), outside both attention partitions and the sample set.
+        # algo reuse + tile-friendly M), where the model does not ask for less.
+        # Pad rows: token 0 at position 0, K/V scattered to the scratch block
+        # (same slot — racy garbage is fine there), outside both attention
+        # partitions and the sample set.
         num_pad_tokens = 0
         padm = self.config.pad_batch_multiple
-        if (
-            padm > 0
-            and self.device.type == "cuda"
-            and not self.config.model.is_moe
-            and T % padm != 0
-        ):
-            num_pad_tokens = padm - T % padm
+        if padm > 0 and self.device.type == "cuda" and not self.config.model.is_moe:
+            if hasattr(self.model, "batch_rows"):
+                num_pad_tokens = self.model.batch_rows(T, padm) - T
+            else:
+                num_pad_tokens = -T % padm
 
         # token ids, positions and cache slots of the flat rows, pad rows behind
         input_ids = np.zeros(T + num_pad_tokens, dtype=np.int64)

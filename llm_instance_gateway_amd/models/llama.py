@@ -7,8 +7,8 @@ BASELINE.json: Llama-3-8B / 70B).  Built MI355X-first:
   * flat unpadded token batches (prefill chunks + decodes in one forward);
   * custom CDNA4 kernels via the ops layer for RMSNorm (fused residual add),
     RoPE, KV-cache scatter, paged prefill/decode attention and SwiGLU;
-  * plain library GEMMs (rocBLAS/hipBLASLt via torch.matmul) for the
-    projections; LoRA deltas ride the SGMV path (`..lora`);
+  * the projections by `ops.linear`: a kernel of this package for few rows or
+    few tiles, library GEMMs elsewhere; LoRA deltas ride the SGMV path (`..lora`);
   * optional tensor parallelism: column-sharded QKV/gate-up, row-sharded
     O/down with one RCCL all-reduce per block over xGMI (`..parallel`).
 
@@ -44,6 +44,13 @@ def _linear(in_f: int, out_f: int, device, dtype) -> nn.Linear:
     return lin
 
 
+def _project(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """m(x); a plain linear layer's product by `ops.linear`."""
+    if type(m) is nn.Linear and _plain(m.__dict__) and m._parameters["bias"] is None and not _has_any_global_hook():
+        return ops.linear(x, m._parameters["weight"])
+    return m(x)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: ModelConfig, device, dtype, tp=None) -> None:
         super().__init__()
@@ -74,7 +81,7 @@ class Attention(nn.Module):
         meta: BatchMeta,
         cos_sin_cache: torch.Tensor,
     ) -> torch.Tensor:
-        qkv = self.qkv_proj(hidden)
+        qkv = _project(self.qkv_proj, hidden)
         if self._lora is not None:
             self._lora.apply(self._layer_idx, "qkv", hidden, qkv, meta)
         k_cache, v_cache = kv_cache
@@ -82,7 +89,7 @@ class Attention(nn.Module):
             qkv, positions, cos_sin_cache, k_cache, v_cache, meta.slot_mapping, self.num_heads
         )
         attn_flat = self.attend(q, kv_cache, meta)
-        o = self.o_proj(attn_flat)
+        o = _project(self.o_proj, attn_flat)
         if self._lora is not None:
             self._lora.apply(self._layer_idx, "o", attn_flat, o, meta)
         if self.tp is not None:
@@ -142,11 +149,11 @@ class MLP(nn.Module):
         self._layer_idx = -1
 
     def forward(self, x: torch.Tensor, meta=None) -> torch.Tensor:
-        gu = self.gate_up_proj(x)
+        gu = _project(self.gate_up_proj, x)
         if self._lora is not None:
             self._lora.apply(self._layer_idx, "gate_up", x, gu, meta)
         act = ops.silu_and_mul(gu)
-        y = self.down_proj(act)
+        y = _project(self.down_proj, act)
         if self._lora is not None:
             self._lora.apply(self._layer_idx, "down", act, y, meta)
         if self.tp is not None:
@@ -244,6 +251,19 @@ class LlamaForCausalLM(nn.Module):
                 return False
         return True
 
+    def batch_rows(self, tokens: int, multiple: int) -> int:
+        """Rows to pad a flat batch of tokens to.  The library's products want few,
+        tile-friendly counts, those of `ops.linear` take any: none is added where
+        all of a layer's projections run there, few where some do (782 tokens: 832
+        rows, not 1024)."""
+        attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
+        served = [type(m) is nn.Linear and ops.linear_served(tokens, m.weight)
+                  for m in (attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ()))]
+        if all(served):
+            return tokens
+        step = min(64, multiple) if any(served) else multiple
+        return -(-tokens // step) * step
+
     def _row_products(self) -> bool:
         """Whether every projection of a layer is one that `ops.row_product` serves."""
         if self.tp is not None or not self.plain_layers():
@@ -314,16 +334,16 @@ class LlamaForCausalLM(nn.Module):
                 h, u = ops.lora_rms_norm(
                     y, residual, layer.input_layernorm, layer.eps, rows, u_down, b[(last, "down")], a[(i, "qkv")], ws)
             q = ops.lora_qkv_rope_cache(
-                attn.qkv_proj(h), positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping,
+                _project(attn.qkv_proj, h), positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping,
                 attn.num_heads, rows, u, b[(i, "qkv")])
             o = attn.attend(q, kv, meta)
             ops.lora_shrink(o, rows, a[(i, "o")], u_o)
             h, u = ops.lora_rms_norm(
-                attn.o_proj(o), residual, layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")],
+                _project(attn.o_proj, o), residual, layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")],
                 a[(i, "gate_up")], ws)
             act = ops.lora_silu_and_mul(
-                mlp.gate_up_proj(h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down)
-            y, last = mlp.down_proj(act), i
+                _project(mlp.gate_up_proj, h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down)
+            y, last = _project(mlp.down_proj, act), i
         return ops.lora_rms_norm(
             y, residual, self.norm, self.cfg.rms_norm_eps, rows, u_down, b[(last, "down")])[0]
 
@@ -332,7 +352,7 @@ class LlamaForCausalLM(nn.Module):
         w = self.embed_tokens.weight if self.lm_head is None else self.lm_head.weight
         # hidden is replicated across the TP group (each block ends in an
         # all-reduce), so every rank computes identical full-vocab logits.
-        return hidden @ w.t()
+        return ops.linear(hidden, w)
 
     def compute_logits(self, hidden: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """fp32 logits only at the sampled positions (last token of each

@@ -429,32 +429,41 @@ def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_ma
     return q
 
 
-# MEASURED DEAD END (benchmarks/bench_gemm.py on MI355X): the hand-written
-# skinny-M MFMA GEMM (ops/csrc/skinny_gemm.hip) reaches only ~0.5 TB/s of W
-# streaming vs hipBLASLt's 2.4 TB/s at M=128 — and the CDNA guide's own
-# best-effort decode-projection recipe tops out at 1.3-1.6 TB/s ("per-CU
-# load-path/latency-bound ... nowhere near the HBM roofline").  hipBLASLt
-# wins this regime; dispatch is disabled (LIG_SKINNY_GEMM_MAX_M to
-# re-enable for experiments), kernel + microbench kept as evidence.
-SKINNY_GEMM_MAX_M = int(os.environ.get("LIG_SKINNY_GEMM_MAX_M", "0"))
+def linear_served(rows: int, weight: torch.Tensor) -> bool:
+    """Whether `linear` runs that many rows on the kernels of projection.hip."""
+    return (
+        weight.is_cuda
+        and weight.dtype == torch.bfloat16
+        and weight.dim() == 2
+        and weight.is_contiguous()
+        and weight.data_ptr() % 16 == 0
+        and _use_native(weight)
+        and _EXT.projection_serves(rows, *weight.shape)
+    )
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """y = x @ weight.T (nn.Linear, no bias).  Dispatch: custom MFMA kernel
-    for decode-sized M on GPU; library GEMM otherwise."""
+    """y = x @ weight.T (nn.Linear, no bias): the framework's kernel where it is
+    the faster one, the library's elsewhere and where a derivative or a transform
+    has to see the product."""
     if (
-        x.is_cuda
+        type(x) is torch.Tensor
+        and type(weight) in (torch.Tensor, torch.nn.Parameter)
+        and x.is_cuda
+        and x.device == weight.device
         and x.dtype == torch.bfloat16
-        and 0 < x.shape[0] <= SKINNY_GEMM_MAX_M
-        and weight.shape[1] % 32 == 0
-        and weight.shape[0] % 64 == 0
-        and _use_native(x)
+        and x.dim() == 2
+        and x.shape[1] == weight.shape[-1]
+        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
+        and linear_served(x.shape[0], weight)
+        and x.is_contiguous()
+        and x.data_ptr() % 16 == 0
     ):
-        out = torch.empty(
-            x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device
-        )
-        _EXT.skinny_gemm(out, x.contiguous(), weight, _stream())
-        return out
+        y = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
+        _EXT.projection(y, x, weight, _stream())
+        return y
     return torch.nn.functional.linear(x, weight)
 
 

@@ -46,6 +46,11 @@ void lig_qkv_rope_cache_launch(uint16_t*, const uint16_t*, const int64_t*,
                                const float*, uint16_t*, uint16_t*,
                                const int64_t*, int, int, int, int, int,
                                hipStream_t);
+bool lig_projection_serves(long, long, long);
+int lig_projection_plan(int, int, int);
+int lig_projection_splits(int);
+int lig_projection_tile(int);
+void lig_projection_launch(int, uint16_t*, float*, const uint16_t*, const uint16_t*, int, int, int, hipStream_t);
 int lig_row_product_max(bool);
 void lig_row_product_launch(uint16_t*, const uint16_t*, int, int, const uint16_t*, const uint16_t*, uint16_t*,
                             const uint16_t*, float, bool, hipStream_t);
@@ -63,8 +68,6 @@ void lig_sgmv_shrink_launch(uint16_t*, const uint16_t*, const uint16_t*,
 void lig_sgmv_expand_launch(uint16_t*, const uint16_t*, const uint16_t*,
                             const int*, float, int, int, int, int,
                             hipStream_t);
-void lig_skinny_gemm_launch(uint16_t*, const uint16_t*, const uint16_t*,
-                            int, int, int, hipStream_t);
 void lig_quant_fp8_rowwise_launch(uint8_t*, float*, const uint16_t*, int,
                                   int, hipStream_t);
 void lig_sgmv_shrink_units_launch(uint16_t*, const uint16_t*, const uint16_t*,
@@ -227,6 +230,27 @@ void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optiona
   lig_row_product_launch(bf16_ptr(y), bf16_cptr(w), N, K, row(x, K), residual ? row(*residual, K) : nullptr,
                          residual_out ? row(*residual_out, K) : nullptr, weight ? row(*weight, K) : nullptr, (float)eps,
                          silu, as_stream(stream));
+}
+
+// y = x W^T of up to 1024 rows (projection.hip); sizes that it does not serve are refused
+void projection(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t stream) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2);
+  const long M = x.size(0), N = w.size(0), K = w.size(1);
+  TORCH_CHECK(x.size(1) == K && y.size(0) == M && y.size(1) == N && lig_projection_serves(M, N, K), "shape");
+  for (const torch::Tensor* t : {&x, &w, &y})
+    TORCH_CHECK(t->is_cuda() && t->is_contiguous() && ((uintptr_t)t->data_ptr() & 15) == 0, "contiguous, aligned");
+  const int plan = lig_projection_plan((int)M, (int)N, (int)K), splits = lig_projection_splits(plan);
+  torch::Tensor part;
+  if (splits > 1) part = torch::empty({splits, M, N}, x.options().dtype(torch::kFloat32));
+  lig_projection_launch(plan, bf16_ptr(y), splits > 1 ? part.data_ptr<float>() : nullptr, bf16_cptr(x), bf16_cptr(w),
+                        (int)M, (int)N, (int)K, as_stream(stream));
+}
+
+// (rows of y, columns of y) of the tile that a served size runs on, and the parts of K
+std::tuple<int, int, int> projection_plan(int M, int N, int K) {
+  TORCH_CHECK(lig_projection_serves(M, N, K), "shape");
+  const int plan = lig_projection_plan(M, N, K), tile = lig_projection_tile(plan);
+  return {tile / 1000, tile % 1000, lig_projection_splits(plan)};
 }
 
 void argmax_rows(torch::Tensor out, torch::Tensor x, int64_t stream) {
@@ -439,20 +463,6 @@ void sgmv_apply_tiled(torch::Tensor y, torch::Tensor x, torch::Tensor a_stack,
                                tile_len.data_ptr<int>(),
                                tile_slot.data_ptr<int>(), ntiles,
                                (float)scaling, T, R, O, st);
-}
-
-void skinny_gemm(torch::Tensor c, torch::Tensor a, torch::Tensor w,
-                 int64_t stream) {
-  const int M = a.size(0);
-  const int K = a.size(1);
-  const int N = w.size(0);
-  TORCH_CHECK(w.size(1) == K && c.size(0) == M && c.size(1) == N,
-              "skinny_gemm shape mismatch");
-  TORCH_CHECK(K % 32 == 0 && N % 64 == 0, "skinny_gemm needs K%32==0, N%64==0");
-  TORCH_CHECK(a.is_contiguous() && w.is_contiguous() && c.is_contiguous());
-  if (M == 0) return;
-  lig_skinny_gemm_launch(bf16_ptr(c), bf16_cptr(a), bf16_cptr(w), M, N, K,
-                         as_stream(stream));
 }
 
 void sgmv_expand(torch::Tensor y, torch::Tensor u, torch::Tensor b_stack,
@@ -671,6 +681,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("argmax_rows", &argmax_rows);
+  m.def("projection", &projection);
+  m.def("projection_plan", &projection_plan);
+  m.def("projection_serves", &lig_projection_serves);
   m.def("row_product", &row_product);
   m.def("row_product_max", &lig_row_product_max);
   m.def("paged_attention_decode", &paged_attention_decode);
@@ -679,7 +692,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sgmv_shrink", &sgmv_shrink);
   m.def("sgmv_apply", &sgmv_apply);
   m.def("sgmv_apply_units", &sgmv_apply_units);
-  m.def("skinny_gemm", &skinny_gemm);
   m.def("sgmv_apply_tiled", &sgmv_apply_tiled);
   m.def("sgmv_expand", &sgmv_expand);
   m.def("quant_fp8_rowwise", &quant_fp8_rowwise);

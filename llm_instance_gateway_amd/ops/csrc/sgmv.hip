@@ -231,7 +231,7 @@ __global__ void sgmv_expand_wide_kernel(
 //   shrink: per tile, u[64,R] = x[64,H] @ A_s[R,H]^T — K-loop over H.
 //   expand: per (tile, 64-out chunk), y[64,64] += u[64,R] @ B_s[64,R]^T —
 //           K = R zero-padded to the mfma's K=32.
-// Fragment layout as verified by csrc/mfma_probe.hip (see skinny_gemm.hip):
+// Fragment layout as verified by csrc/mfma_probe.hip:
 // mfma_f32_16x16x32_bf16(a,b,c): C[i][j] += sum_k A[i,k]B[j,k]; a: lane li=i;
 // b: lane li=j; both k = lg*8..+7; C: row i = lg*4+r, col j = li.
 

@@ -1,0 +1,58 @@
+"""The projection kernels against 64-bit torch, at sizes that reach every tile,
+its remainders and cuts of K, and the calls that stay with the library."""
+
+import pytest
+import torch
+
+from llm_instance_gateway_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+SIZES = [
+    # (rows, outputs, columns): edges of the tiles' rows and columns
+    (1, 8, 64), (5, 24, 128), (16, 4096, 4096), (16, 4104, 14336), (17, 520, 192), (33, 4096, 4096), (32, 1288, 8192),
+    (48, 6144, 4096), (63, 28672, 256), (65, 8200, 3584), (97, 4096, 4096), (96, 12288, 1024), (129, 6152, 4096),
+    (160, 4096, 1088), (193, 4096, 14336), (202, 28680, 128), (225, 12288, 4096), (256, 22016, 512), (255, 6144, 4096),
+    (257, 1288, 8192), (384, 6144, 4096), (786, 4096, 14336), (1000, 4040, 4096), (1024, 16, 64), (130, 4096, 4096), (343, 6144, 8192),
+]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_projection(M, N, K):
+    g = torch.Generator("cuda").manual_seed(M * 7 + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(BF)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF)
+    assert ops.linear_served(M, w)
+    with torch.no_grad():
+        got = ops.linear(x, w)
+    ref = x.double() @ w.double().t()
+    # one rounding to 8 bits; 24-bit sums over K terms, whose errors walk
+    size = (x.double().pow(2) @ w.double().pow(2).t()).sqrt()
+    tol = 2.0 ** -8 * ref.abs() + 2.0 ** -23 * K ** 0.5 * 4 * size
+    assert got.shape == (M, N) and got.dtype == BF
+    assert ((got.double() - ref).abs() <= tol).all()
+
+
+def test_every_tile_is_reached():
+    plan = ops._load_ext().projection_plan
+    seen = {plan(*s) for s in SIZES}
+    wide = {plan(m, n, k)[:2] for m in range(1, 1025, 5) for n in (1280, 4096, 6144, 12288, 28672, 128256)
+            for k in (1024, 4096, 14336) if ops._EXT.projection_serves(m, n, k)}
+    assert {s[:2] for s in seen} >= wide
+    assert {s[2] for s in seen} >= {1, 2, 8}
+
+
+def test_other_calls_stay_with_the_library():
+    g = torch.Generator("cuda").manual_seed(2)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    w = r(64, 128).to(BF)
+    for x, v in ((r(8, 128), w.float()), (r(8, 72).to(BF), r(64, 72).to(BF)), (r(8, 128).to(BF), r(12, 128).to(BF)),
+                 (r(128, 8).to(BF).t(), w), (r(2, 8, 128).to(BF), w), (r(8, 128).to(BF), r(128, 64).to(BF).t()),
+                 (r(0, 128).to(BF), w), (r(8 * 128 + 1).to(BF)[1:].view(8, 128), w)):
+        assert torch.equal(ops.linear(x, v), torch.nn.functional.linear(x, v))
+    assert not ops.linear_served(1025, w) and not ops.linear_served(512, r(28672, 64).to(BF))
+    p = torch.nn.Parameter(w)
+    ops.linear(r(8, 128).to(BF), p).sum().backward()
+    assert p.grad is not None
+    with pytest.raises(RuntimeError):
+        ops.linear(r(8, 64).to(BF), w)
