@@ -44,11 +44,20 @@ def _linear(in_f: int, out_f: int, device, dtype) -> nn.Linear:
     return lin
 
 
-def _project(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """m(x); a plain linear layer's product by `ops.linear`."""
-    if type(m) is nn.Linear and _plain(m.__dict__) and m._parameters["bias"] is None and not _has_any_global_hook():
-        return ops.linear(x, m._parameters["weight"])
-    return m(x)
+def _product_alone(m: nn.Module) -> bool:
+    """Whether m(x) is x @ m.weight.T and nothing else."""
+    return (type(m) is nn.Linear and _plain(m.__dict__) and m._parameters["bias"] is None
+            and not _has_any_global_hook())
+
+
+def _project(m: nn.Module, x: torch.Tensor, product=ops.linear) -> torch.Tensor:
+    """m(x); a plain linear layer's product by `ops.linear` (or `ops.linear_parts`)."""
+    return product(x, m._parameters["weight"]) if _product_alone(m) else m(x)
+
+
+def _served(m: nn.Module, rows: int) -> bool:
+    """Whether `_project` of that many rows runs on our kernels."""
+    return _product_alone(m) and ops.linear_served(rows, m._parameters["weight"])
 
 
 class Attention(nn.Module):
@@ -255,10 +264,11 @@ class LlamaForCausalLM(nn.Module):
         """Rows to pad a flat batch of tokens to.  The library's products want few,
         tile-friendly counts, those of `ops.linear` take any: none is added where
         all of a layer's projections run there, few where some do (782 tokens: 832
-        rows, not 1024)."""
+        rows, not 1024).  Under 2^20 weights a projection takes its launch's time at
+        either count, and the multiple stays."""
         attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
-        served = [type(m) is nn.Linear and ops.linear_served(tokens, m.weight)
-                  for m in (attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ()))]
+        modules = [attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ())]
+        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 for m in modules]
         if all(served):
             return tokens
         step = min(64, multiple) if any(served) else multiple
@@ -324,26 +334,32 @@ class LlamaForCausalLM(nn.Module):
             rows, c.hidden_size, c.num_heads * c.head_dim, c.intermediate_size)
         a, b = lora.a_stacks, lora.b_stacks
         residual, y, last = None, hidden, None
+        # Norms whose readers can take the rows' factor themselves are one launch, and
+        # add up the product before them.  The rotation takes it with fp32 parts
+        # only: a rounded product would be rounded once more on its way to V.
+        opens = ops.lora_norm_opens(rows, c.hidden_size)
+        open_in = [opens and _served(layer.self_attn.qkv_proj, len(hidden)) for layer in self.layers] + [False]
         for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
             attn, mlp = layer.self_attn, layer.mlp
+            norm = ops.lora_norm_open if open_in[i] else ops.lora_rms_norm
             if last is None:
-                h, u = ops.lora_rms_norm(
-                    y, None, layer.input_layernorm, layer.eps, rows, a_stack=a[(i, "qkv")], u_out=ws)
+                h, u, *scale = norm(y, None, layer.input_layernorm, layer.eps, rows, a_stack=a[(i, "qkv")], u_out=ws)
                 residual = hidden
             else:
-                h, u = ops.lora_rms_norm(
+                h, u, *scale = norm(
                     y, residual, layer.input_layernorm, layer.eps, rows, u_down, b[(last, "down")], a[(i, "qkv")], ws)
             q = ops.lora_qkv_rope_cache(
-                _project(attn.qkv_proj, h), positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping,
-                attn.num_heads, rows, u, b[(i, "qkv")])
+                _project(attn.qkv_proj, h, ops.linear_parts if open_in[i] else ops.linear), positions, self.cos_sin_cache,
+                kv[0], kv[1], meta.slot_mapping, attn.num_heads, rows, u, b[(i, "qkv")], *scale)
             o = attn.attend(q, kv, meta)
             ops.lora_shrink(o, rows, a[(i, "o")], u_o)
-            h, u = ops.lora_rms_norm(
-                _project(attn.o_proj, o), residual, layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")],
-                a[(i, "gate_up")], ws)
+            norm = ops.lora_norm_open if opens else ops.lora_rms_norm
+            h, u, *scale = norm(
+                _project(attn.o_proj, o, ops.linear_parts if opens else ops.linear), residual,
+                layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")], a[(i, "gate_up")], ws)
             act = ops.lora_silu_and_mul(
-                _project(mlp.gate_up_proj, h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down)
-            y, last = _project(mlp.down_proj, act), i
+                _project(mlp.gate_up_proj, h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down, *scale)
+            y, last = _project(mlp.down_proj, act, ops.linear_parts if open_in[i + 1] else ops.linear), i
         return ops.lora_rms_norm(
             y, residual, self.norm, self.cfg.rms_norm_eps, rows, u_down, b[(last, "down")])[0]
 

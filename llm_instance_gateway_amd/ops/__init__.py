@@ -409,10 +409,29 @@ def lora_rms_norm(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_sta
     return out, None if u_out is None else u_out[:parts]
 
 
-def lora_silu_and_mul(x, rows, u_in, b_stack, a_stack, u_out):
-    """silu(gate + B u_in) * (up + B u_in) of x = [gate | up]; u_out = A of it."""
+def lora_norm_opens(rows, width: int) -> bool:
+    """Whether `lora_norm_open` is for these tiles: where the norm takes strips."""
+    return (width >= 2048 and rows[1].shape[0] * 4096 < LORA_NORM_STRIPS_BELOW * width
+            and width % _load_ext().lora_norm_strip() == 0)
+
+
+def lora_norm_open(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_stack=None, u_out=None):
+    """`lora_rms_norm` with the factor 1 / rms of each row left out of h (and so of
+    u_out, and of any product of h); x may be `linear_parts` of a product.  Returns
+    h, the parts of u_out and what the reader of the product finds the factor by."""
+    T, H = x.shape[-2:]
+    n, parts = rows[1].shape[0], H // _EXT.lora_norm_strip()
+    out = torch.empty(T, H, dtype=weight.dtype, device=x.device)
+    sums = torch.empty(n * parts * 16, dtype=torch.float32, device=x.device)
+    _EXT.lora_norm_open(out, x, residual, weight, *rows, u_in, b_stack, a_stack, u_out, sums, _stream())
+    return out, u_out[:parts], (sums, H, eps)
+
+
+def lora_silu_and_mul(x, rows, u_in, b_stack, a_stack, u_out, norm=(None, 0, 0.0)):
+    """silu(gate + B u_in) * (up + B u_in) of x = [gate | up]; u_out = A of it.
+    `norm`: from `lora_norm_open`, where x and u_in lack its factor."""
     out = torch.empty(x.shape[0], x.shape[1] // 2, dtype=x.dtype, device=x.device)
-    _EXT.lora_silu(out, x, *rows, u_in, b_stack, a_stack, u_out, _stream())
+    _EXT.lora_silu(out, x, *rows, u_in, b_stack, a_stack, u_out, *norm, _stream())
     return out
 
 
@@ -421,11 +440,13 @@ def lora_shrink(x, rows, a_stack, u_out) -> None:
     _EXT.lora_shrink(x, *rows, a_stack, u_out, _stream())
 
 
-def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, num_heads, rows, u_in, b_stack):
-    """`qkv_rope_cache` of qkv + B u_in."""
-    q = torch.empty(qkv.shape[0], num_heads * k_cache.shape[-1], dtype=qkv.dtype, device=qkv.device)
+def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, num_heads, rows, u_in, b_stack,
+                        norm=(None, 0, 0.0)):
+    """`qkv_rope_cache` of qkv + B u_in; qkv may be `linear_parts` of the product,
+    which, like u_in, may then lack the factor of `norm` from `lora_norm_open`."""
+    q = torch.empty(qkv.shape[-2], num_heads * k_cache.shape[-1], dtype=k_cache.dtype, device=qkv.device)
     _EXT.lora_qkv_rope_cache(
-        q, qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, *rows, u_in, b_stack, _stream())
+        q, qkv, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, *rows, u_in, b_stack, *norm, _stream())
     return q
 
 
@@ -442,11 +463,10 @@ def linear_served(rows: int, weight: torch.Tensor) -> bool:
     )
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """y = x @ weight.T (nn.Linear, no bias): the framework's kernel where it is
-    the faster one, the library's elsewhere and where a derivative or a transform
-    has to see the product."""
-    if (
+def _linear_here(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether x @ weight.T is for our kernels: not where a derivative or a
+    transform has to see the product."""
+    return (
         type(x) is torch.Tensor
         and type(weight) in (torch.Tensor, torch.nn.Parameter)
         and x.is_cuda
@@ -460,10 +480,24 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         and linear_served(x.shape[0], weight)
         and x.is_contiguous()
         and x.data_ptr() % 16 == 0
-    ):
+    )
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """y = x @ weight.T (nn.Linear, no bias): the framework's kernel where it is
+    the faster one, the library's elsewhere."""
+    if _linear_here(x, weight):
         y = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
         _EXT.projection(y, x, weight, _stream())
         return y
+    return torch.nn.functional.linear(x, weight)
+
+
+def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """`linear` for a reader that adds up itself: fp32 [parts, rows, outputs], or
+    the rounded product where that is the library's."""
+    if _linear_here(x, weight):
+        return _EXT.projection_parts(x, weight, _stream())
     return torch.nn.functional.linear(x, weight)
 
 

@@ -98,16 +98,19 @@ void lig_lora_rms_norm_strips_launch(
     uint16_t*, const uint16_t*, uint16_t*, const uint16_t*, float, int,
     const int*, const int*, const int*, int, const float*, int, int,
     const uint16_t*, const uint16_t*, float*, int, float*, hipStream_t);
+void lig_lora_norm_open_launch(uint16_t*, const uint16_t*, const float*, int, long, uint16_t*, const uint16_t*, int,
+                               const int*, const int*, const int*, int, const float*, int, int, const uint16_t*,
+                               const uint16_t*, float*, int, float*, hipStream_t);
 void lig_lora_silu_launch(uint16_t*, const uint16_t*, int, const int*,
                           const int*, const int*, int, const float*, int, int,
                           const uint16_t*, const uint16_t*, float*, int,
-                          hipStream_t);
+                          const float*, int, float, hipStream_t);
 void lig_lora_shrink_launch(const uint16_t*, int, const int*, const int*,
                             const int*, int, const uint16_t*, float*, int,
                             hipStream_t);
 int lig_lora_shrink_strip();
 void lig_lora_qkv_rope_cache_launch(
-    uint16_t*, const uint16_t*, const int64_t*, const float*, uint16_t*,
+    uint16_t*, const uint16_t*, const float*, int, long, const float*, int, float, const int64_t*, const float*, uint16_t*,
     uint16_t*, const int64_t*, int, int, int, int, const int*, const int*,
     const int*, int, const float*, int, int, const uint16_t*, hipStream_t);
 void lig_paged_attention_prefill_launch(
@@ -244,6 +247,20 @@ void projection(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t strea
   if (splits > 1) part = torch::empty({splits, M, N}, x.options().dtype(torch::kFloat32));
   lig_projection_launch(plan, bf16_ptr(y), splits > 1 ? part.data_ptr<float>() : nullptr, bf16_cptr(x), bf16_cptr(w),
                         (int)M, (int)N, (int)K, as_stream(stream));
+}
+
+// The same as fp32 [parts, M, N] that add up to it
+torch::Tensor projection_parts(torch::Tensor x, torch::Tensor w, int64_t stream) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2);
+  const long M = x.size(0), N = w.size(0), K = w.size(1);
+  TORCH_CHECK(x.size(1) == K && lig_projection_serves(M, N, K), "shape");
+  for (const torch::Tensor* t : {&x, &w})
+    TORCH_CHECK(t->is_cuda() && t->is_contiguous() && ((uintptr_t)t->data_ptr() & 15) == 0, "contiguous, aligned");
+  const int plan = lig_projection_plan((int)M, (int)N, (int)K);
+  torch::Tensor part = torch::empty({lig_projection_splits(plan), M, N}, x.options().dtype(torch::kFloat32));
+  lig_projection_launch(plan, nullptr, part.data_ptr<float>(), bf16_cptr(x), bf16_cptr(w), (int)M, (int)N, (int)K,
+                        as_stream(stream));
+  return part;
 }
 
 // (rows of y, columns of y) of the tile that a served size runs on, and the parts of K
@@ -575,10 +592,42 @@ void lora_rms_norm(torch::Tensor out, torch::Tensor x,
   TORCH_CHECK(rc == 0, "lora_rms_norm: rows of ", H, " entries not served");
 }
 
+// sums of squares per tile and strip of rows of `width` columns
+inline float* sums_ptr(const std::optional<torch::Tensor>& sums, int64_t width, int64_t n) {
+  if (!sums) return nullptr;
+  const int strip = lig_lora_norm_strip();
+  TORCH_CHECK(width > 0 && width % strip == 0 && sums->scalar_type() == torch::kFloat32 && sums->is_cuda() &&
+              sums->is_contiguous() && sums->numel() >= n * (width / strip) * 16);
+  return sums->data_ptr<float>();
+}
+
+// out = (residual + x + B u_in) * weight, which residual becomes without the weight, u_out = A out and
+// `sums` for the norm's factor; x bf16 [T, H] or the fp32 parts [S, T, H] of a product
+void lora_norm_open(torch::Tensor out, torch::Tensor x, std::optional<torch::Tensor> residual, torch::Tensor weight,
+                    torch::Tensor toks, torch::Tensor len, torch::Tensor slot, std::optional<torch::Tensor> u_in,
+                    std::optional<torch::Tensor> b_stack, torch::Tensor a_stack, torch::Tensor u_out,
+                    torch::Tensor sums, int64_t stream) {
+  const bool parts = x.dim() == 3;
+  const int T = out.size(0), H = out.size(1);
+  TORCH_CHECK(x.size(-1) == H && x.size(-2) == T && x.is_contiguous() && x.is_cuda() && weight.numel() == H);
+  TORCH_CHECK(!parts || (x.scalar_type() == torch::kFloat32 && x.size(0) > 0 && residual));
+  TORCH_CHECK(!residual || residual->sizes() == out.sizes());
+  TORCH_CHECK(u_in.has_value() == b_stack.has_value() && (!u_in || residual));
+  const int n = check_tiles(toks, len, slot, T, a_stack.size(0));
+  if (n == 0 || T == 0) return;
+  lig_lora_norm_open_launch(
+      bf16_ptr(out), parts ? nullptr : bf16_cptr(x), parts ? x.data_ptr<float>() : nullptr, parts ? (int)x.size(0) : 0,
+      (long)T * H, residual ? bf16_ptr(*residual) : nullptr, bf16_cptr(weight), H, i32_cptr(toks), i32_cptr(len),
+      i32_cptr(slot), n, u_in ? u_ptr(*u_in, 1, n) : nullptr, u_in ? (int)u_in->size(0) : 0,
+      u_in ? (int)u_in->size(1) : 0, b_stack ? b_ptr(*b_stack, H) : nullptr, a_ptr(a_stack, H),
+      u_ptr(u_out, H / lig_lora_norm_strip(), n), (int)u_out.size(1), sums_ptr(sums, H, n), as_stream(stream));
+}
+
 void lora_silu(torch::Tensor out, torch::Tensor x, torch::Tensor toks,
                torch::Tensor len, torch::Tensor slot,
                torch::Tensor u_in, torch::Tensor b_stack,
-               torch::Tensor a_stack, torch::Tensor u_out, int64_t stream) {
+               torch::Tensor a_stack, torch::Tensor u_out, std::optional<torch::Tensor> sums, int64_t width, double eps,
+               int64_t stream) {
   const int T = x.size(0), d = out.size(1);
   TORCH_CHECK(out.size(0) == T && x.size(1) == 2 * (int64_t)d && d % 32 == 0);
   const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
@@ -590,7 +639,7 @@ void lora_silu(torch::Tensor out, torch::Tensor x, torch::Tensor toks,
                        u_ptr(u_in, 1, n), (int)u_in.size(0), (int)u_in.size(1),
                        b_ptr(b_stack, 2 * (int64_t)d),
                        a_ptr(a_stack, d), u_ptr(u_out, (d + strip - 1) / strip, n),
-                       (int)u_out.size(1), as_stream(stream));
+                       (int)u_out.size(1), sums_ptr(sums, width, n), (int)width, (float)eps, as_stream(stream));
 }
 
 void lora_shrink(torch::Tensor x, torch::Tensor toks,
@@ -612,24 +661,29 @@ void lora_qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
                          torch::Tensor slot_mapping, torch::Tensor toks,
                          torch::Tensor len,
                          torch::Tensor slot, torch::Tensor u_in,
-                         torch::Tensor b_stack, int64_t stream) {
+                         torch::Tensor b_stack, std::optional<torch::Tensor> sums, int64_t width, double eps,
+                         int64_t stream) {
   TORCH_CHECK(positions.scalar_type() == torch::kInt64);
   TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
   TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 && cos_sin.is_contiguous());
-  const int T = qkv.size(0), Hkv = k_cache.size(1), BS = k_cache.size(2), D = k_cache.size(3);
+  const bool parts = qkv.dim() == 3;  // fp32 parts of the product
+  TORCH_CHECK(!parts || (qkv.scalar_type() == torch::kFloat32 && qkv.is_contiguous() && qkv.is_cuda() && qkv.size(0) > 0));
+  const int T = qkv.size(-2), Hkv = k_cache.size(1), BS = k_cache.size(2), D = k_cache.size(3);
   const int Hq = q_out.size(1) / D;
   TORCH_CHECK(D % 64 == 0 && cos_sin.size(1) == D && v_cache.sizes() == k_cache.sizes());
-  TORCH_CHECK(qkv.size(1) == (int64_t)(Hq + 2 * Hkv) * D && q_out.size(0) == T &&
+  TORCH_CHECK(qkv.size(-1) == (int64_t)(Hq + 2 * Hkv) * D && q_out.size(0) == T &&
               q_out.size(1) == (int64_t)Hq * D);
   TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
   const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
   if (n == 0 || T == 0) return;
   lig_lora_qkv_rope_cache_launch(
-      bf16_ptr(q_out), bf16_cptr(qkv), positions.data_ptr<int64_t>(),
+      bf16_ptr(q_out), parts ? nullptr : bf16_cptr(qkv), parts ? qkv.data_ptr<float>() : nullptr,
+      parts ? (int)qkv.size(0) : 0, (long)T * qkv.size(-1), sums_ptr(sums, width, n), (int)width, (float)eps,
+      positions.data_ptr<int64_t>(),
       cos_sin.data_ptr<float>(), bf16_ptr(k_cache), bf16_ptr(v_cache),
       slot_mapping.data_ptr<int64_t>(), Hq, Hkv, D, BS, i32_cptr(toks),
       i32_cptr(len), i32_cptr(slot), n, u_ptr(u_in, 1, n),
-      (int)u_in.size(0), (int)u_in.size(1), b_ptr(b_stack, qkv.size(1)), as_stream(stream));
+      (int)u_in.size(0), (int)u_in.size(1), b_ptr(b_stack, qkv.size(-1)), as_stream(stream));
 }
 
 }  // namespace
@@ -682,6 +736,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_and_mul", &silu_and_mul);
   m.def("argmax_rows", &argmax_rows);
   m.def("projection", &projection);
+  m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);
   m.def("projection_serves", &lig_projection_serves);
   m.def("row_product", &row_product);
@@ -696,6 +751,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sgmv_expand", &sgmv_expand);
   m.def("quant_fp8_rowwise", &quant_fp8_rowwise);
   m.def("lora_rms_norm", &lora_rms_norm);
+  m.def("lora_norm_open", &lora_norm_open);
   m.def("lora_silu", &lora_silu);
   m.def("lora_silu_strip", &lig_lora_silu_strip);
   m.def("lora_norm_strip", &lig_lora_norm_strip);

@@ -241,10 +241,10 @@ __global__ __launch_bounds__(512) void lora_rms_norm_kernel(
 
 // The same in two launches for steps of few tiles: one workgroup per tile pulls
 // the adapter's 2 x 128 KB and the rows at a single CU's rate (18 us for 9 tiles
-// of 4096 columns).  Workgroups here take 512 columns of a tile; the first kernel
+// of 4096 columns).  Workgroups here take 256 columns of a tile; the first kernel
 // leaves the sums of squares of its columns, the second forms the same values
-// again and has the whole row's sum at hand.  u_out gets a part per 512 columns.
-constexpr int NORM_STRIP = 512;
+// again and has the whole row's sum at hand.  u_out gets a part per 256 columns.
+constexpr int NORM_STRIP = 256;
 
 template <bool ADD, bool DELTA, bool TO_U, bool SUM>
 LIG_DEVICE void norm_strip(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
@@ -350,6 +350,147 @@ __global__ __launch_bounds__(256) void lora_norm_strip_kernel(
 #undef STRIP
 }
 
+// G groups of 8 columns of a product in fp32 parts.  Four parts are asked
+// for at a time, past the last one that one again.
+template <int G>
+LIG_DEVICE void add_parts(f32x8 (&v)[G], const float* __restrict__ p, const int parts, const size_t stride, const int (&at)[G]) {
+#pragma unroll
+  for (int i = 0; i < G; ++i) v[i] = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < parts; k += 4) {
+    f32x8 r[4][G];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < G; ++i) r[j][i] = *reinterpret_cast<const f32x8*>(p + min(k + j, parts - 1) * stride + at[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < G; ++i)
+        if (k + j < parts) v[i] += r[j][i];
+  }
+}
+
+// The same strips in one launch, for readers that can wait for the norm's factor:
+// out = residual' * weight, u_out = A out, and the sums of squares of each strip.
+// A product's rows carry the factor through, so it is left to the kernel that reads
+// the product (factor_of).  x may come as the parts that projection.hip cuts K into.
+// As sum of the parts, sums of squares and norm these were three launches.  With both
+// adapter products, 4096 columns, in a step: 48 rows, 4 parts 16.6 -> 7.1 us; 202 rows,
+// 4 and 8 parts 17.4 -> 9.3; 384 rows 22.7 -> 13.4.  With strips of 512 columns 8.9, 13.5
+// and 14.2.
+template <bool ADD, bool DELTA, bool TO_U, bool PARTS>
+LIG_DEVICE void open_strip(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+                           const float* __restrict__ xp, const int xparts, const size_t xstride,
+                           uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, const int hidden,
+                           const float* u_in, const int parts, const int tiles, const uint16_t* __restrict__ b,
+                           const uint16_t* __restrict__ a, float* u_out, const int tiles_out, float* sums, float* smem,
+                           int wave, int li, int lg) {
+  constexpr int NB = NORM_STRIP / 128;
+  const int c_first = blockIdx.y * NORM_STRIP + wave * 32;
+  const size_t base = (size_t)t.row * hidden + lg * 8;
+  u16x8 xr[NB], rr[NB], wr[NB], ar[NB];
+  BOperand br[NB];
+  f32x8 v[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int c0 = c_first + i * 128;
+    if constexpr (!PARTS) xr[i] = load8(x + base + c0);
+    if constexpr (ADD) rr[i] = load8(residual + base + c0);
+    if constexpr (DELTA) br[i] = load_b(b, c0, li, lg);
+    wr[i] = load8(weight + c0 + lg * 8);
+    if constexpr (TO_U) ar[i] = load_a(a, hidden, c0, li, lg);
+  }
+  if constexpr (PARTS) {
+    int at[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) at[i] = c_first + i * 128;
+    add_parts(v, xp + base, xparts, xstride, at);
+  }
+  bf16x8_t u = {};
+  if constexpr (DELTA) u = u_of(u_in, parts, tiles, smem, li, lg, t.valid);
+  float ss = 0.f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  u16x8 h[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if constexpr (!PARTS) v[i] = bf16x8_to_f32x8(xr[i]);
+    if constexpr (ADD) v[i] += bf16x8_to_f32x8(rr[i]);
+    if constexpr (DELTA) v[i] += expand(br[i], u);
+    const f32x8 w = bf16x8_to_f32x8(wr[i]);
+    f32x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      ss += v[i][j] * v[i][j];
+      o[j] = v[i][j] * w[j];
+    }
+    h[i] = f32x8_to_bf16x8(o);
+    if constexpr (TO_U) acc = shrink(ar[i], h[i], acc);
+  }
+  if (t.valid) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int c0 = c_first + i * 128;
+      *reinterpret_cast<u16x8*>(out + base + c0) = h[i];
+      if constexpr (ADD) *reinterpret_cast<u16x8*>(residual + base + c0) = f32x8_to_bf16x8(v[i]);
+    }
+  }
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  if (lg == 0) smem[wave * 16 + li] = ss;
+  __syncthreads();
+  if (threadIdx.x < 16)
+    sums[blockIdx.y * 16 + threadIdx.x] =
+        smem[threadIdx.x] + smem[16 + threadIdx.x] + smem[32 + threadIdx.x] + smem[48 + threadIdx.x];
+  if constexpr (TO_U) {
+    __syncthreads();
+    store_u<4>(u_out + (size_t)blockIdx.y * tiles_out * 16 * R, acc, reinterpret_cast<float(*)[16][R]>(smem), wave, li, lg);
+  }
+}
+
+template <bool ADD, bool PARTS>
+__global__ __launch_bounds__(256) void lora_norm_open_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const float* __restrict__ xp, const int xparts,
+    const size_t xstride, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, const int hidden,
+    const int* __restrict__ toks, const int* __restrict__ len, const int* __restrict__ slot, const float* u_in,
+    const int parts, const int tiles, const uint16_t* __restrict__ b_stack, const uint16_t* __restrict__ a_stack,
+    float* u_out, const int tiles_out, float* sums) {
+  __shared__ __align__(16) float smem[4 * 16 * R];
+  const int tile = blockIdx.x;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Tile t = tile_of(toks, len, slot, tile, li);
+  if (t.n == 0) return;
+  const bool delta = u_in != nullptr && t.slot >= 0, to_u = t.slot >= 0;
+  const float* ui = delta ? u_in + (size_t)tile * 16 * R : nullptr;
+  const uint16_t* b = delta ? b_stack + (size_t)t.slot * hidden * R : nullptr;
+  const uint16_t* a = to_u ? a_stack + (size_t)t.slot * R * hidden : nullptr;
+  float* uo = to_u ? u_out + (size_t)tile * 16 * R : nullptr;
+  float* sm = sums + (size_t)tile * (hidden / NORM_STRIP) * 16;
+#define STRIP(DELTA, TO_U)                                                                                          \
+  open_strip<ADD, DELTA, TO_U, PARTS>(t, out, x, xp, xparts, xstride, residual, weight, hidden, ui, parts, tiles, b, a, \
+                                      uo, tiles_out, sm, smem, wave, li, lg)
+  if (ADD && delta) STRIP(ADD, true);
+  else if (to_u) STRIP(false, true);
+  else STRIP(false, false);
+#undef STRIP
+}
+
+// The factor that lora_norm_open left out, of token li of a tile; without sums none was.
+struct Factor {
+  const float* sums;  // [tiles][width / strip][16]
+  int width;
+  float eps;
+};
+LIG_DEVICE float factor_of(const Factor& f, int tile, int li) {
+  if (f.sums == nullptr) return 1.f;
+  const int strips = f.width / NORM_STRIP;
+  const float* s = f.sums + (size_t)tile * strips * 16 + li;
+  float total = 0.f;
+#pragma unroll 8
+  for (int k = 0; k < strips; ++k) total += s[k * 16];
+  return rsqrtf(total / f.width + f.eps);
+}
+
 // out = silu(gate + B u) * (up + B u), u_out[strip] = A_down out.  Workgroups of
 // a tile take strips of 1024 of the d columns.
 constexpr int SILU_STRIP = 1024;
@@ -357,7 +498,7 @@ constexpr int SILU_STRIP = 1024;
 template <bool LORA>
 LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d,
                              const int c_first, const bf16x8_t u, const uint16_t* __restrict__ b,
-                             const uint16_t* __restrict__ a, int li, int lg) {
+                             const uint16_t* __restrict__ a, const float factor, int li, int lg) {
   constexpr int NB = 4;  // groups whose loads are issued together
   const uint16_t* g = x + (size_t)t.row * 2 * d + lg * 8;
   uint16_t* o = out + (size_t)t.row * d + lg * 8;
@@ -385,6 +526,8 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
         gv += expand(bg[i], u);
         uv += expand(bu[i], u);
       }
+      gv *= factor;
+      uv *= factor;
 #pragma unroll
       for (int j = 0; j < 8; ++j) r[j] = gv[j] / (1.0f + __expf(-gv[j])) * uv[j];
       const u16x8 rb = f32x8_to_bf16x8(r);
@@ -399,7 +542,7 @@ __global__ __launch_bounds__(256) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
     const int* __restrict__ len, const int* __restrict__ slot,
     const float* __restrict__ u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
-    const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out) {
+    const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm) {
   __shared__ __align__(16) float red[4][16][R];
   const int tile = blockIdx.x, strip = blockIdx.y;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
@@ -407,14 +550,15 @@ __global__ __launch_bounds__(256) void lora_silu_kernel(
   const Tile t = tile_of(toks, len, slot, tile, li);
   if (t.n == 0) return;
   const int c_first = strip * SILU_STRIP + wave * 32;
+  const float factor = factor_of(norm, tile, li);
   if (t.slot < 0) {
-    silu_rows<false>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, li, lg);
+    silu_rows<false>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, factor, li, lg);
     return;
   }
   const f32x4_t acc =
       silu_rows<true>(t, out, x, d, c_first,
                       u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid),
-                      b_stack + (size_t)t.slot * 2 * d * R, a_stack + (size_t)t.slot * R * d, li, lg);
+                      b_stack + (size_t)t.slot * 2 * d * R, a_stack + (size_t)t.slot * R * d, factor, li, lg);
   store_u<4>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
 }
 
@@ -449,16 +593,20 @@ __global__ __launch_bounds__(256) void lora_shrink_kernel(
   store_u<4>(u_out + ((size_t)blockIdx.y * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
 }
 
-// qkv_rope.hip's pass with B u added to the projection on the way in
-constexpr int QR_HEADS = 4;
-
+// qkv_rope.hip's pass with B u added to the projection on the way in.  PARTS: the
+// projection as fp32 parts of K.
+// Waves take 4 heads, of parts one: 2 to 8 times the bytes (48 rows in 4 parts 8.3 us,
+// 12.7 with 4 heads; sum and rotation as two launches 11.1).
+template <bool PARTS>
 __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
-    uint16_t* __restrict__ q_out, const uint16_t* __restrict__ qkv, const int64_t* __restrict__ positions,
+    uint16_t* __restrict__ q_out, const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_parts, const int nparts,
+    const size_t part_stride, const Factor norm, const int64_t* __restrict__ positions,
     const float* __restrict__ cos_sin, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
     const int64_t* __restrict__ slot_mapping, const int num_q_heads, const int num_kv_heads, const int head_dim,
     const int block_size, const int* __restrict__ toks, const int* __restrict__ len,
     const int* __restrict__ slot, const float* __restrict__ u_in, const int u_parts, const int tiles,
     const uint16_t* __restrict__ b_stack) {
+  constexpr int QR_HEADS = PARTS ? 1 : 4;
   __shared__ __align__(16) float smem[16 * R];
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int parts = head_dim / 64;  // of 32 rotation pairs
@@ -488,19 +636,27 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
   const int64_t at = slot_mapping[t.row];
   const size_t blk = at < 0 ? 0 : at / block_size;
   const size_t off = at < 0 ? 0 : at % block_size;
-  const uint16_t* src = qkv + ((size_t)t.row * heads + h0) * head_dim + c;
-  u16x8 x[QR_HEADS][2];
-#pragma unroll
-  for (int i = 0; i < QR_HEADS; ++i) {
-    const int h = min(h0 + i, heads - 1) - h0;
-    x[i][0] = load8(src + h * head_dim);
-    x[i][1] = load8(src + h * head_dim + half);
-  }
+  const size_t src = ((size_t)t.row * heads + h0) * head_dim + c;
   f32x8 v[QR_HEADS][2];
+  if constexpr (PARTS) {
+    f32x8 y[2];
+    const int at[2] = {0, half};
+    add_parts(y, qkv_parts + src, nparts, part_stride, at);
+    v[0][0] = y[0];
+    v[0][1] = y[1];
+  } else {
+    u16x8 x[QR_HEADS][2];
 #pragma unroll
-  for (int i = 0; i < QR_HEADS; ++i) {
-    v[i][0] = bf16x8_to_f32x8(x[i][0]);
-    v[i][1] = bf16x8_to_f32x8(x[i][1]);
+    for (int i = 0; i < QR_HEADS; ++i) {
+      const int h = min(h0 + i, heads - 1) - h0;
+      x[i][0] = load8(qkv + src + h * head_dim);
+      x[i][1] = load8(qkv + src + h * head_dim + half);
+    }
+#pragma unroll
+    for (int i = 0; i < QR_HEADS; ++i) {
+      v[i][0] = bf16x8_to_f32x8(x[i][0]);
+      v[i][1] = bf16x8_to_f32x8(x[i][1]);
+    }
   }
   if (t.slot >= 0) {
     const uint16_t* b = b_stack + (size_t)t.slot * heads * head_dim * R;
@@ -516,6 +672,12 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
       v[i][0] += expand(br[i][0], u);
       v[i][1] += expand(br[i][1], u);
     }
+  }
+  const float factor = factor_of(norm, blockIdx.x, li);
+#pragma unroll
+  for (int i = 0; i < QR_HEADS; ++i) {
+    v[i][0] *= factor;
+    v[i][1] *= factor;
   }
 #pragma unroll
   for (int i = 0; i < QR_HEADS; ++i) {
@@ -599,12 +761,29 @@ void lig_lora_rms_norm_strips_launch(uint16_t* out, const uint16_t* x, uint16_t*
 #undef LAUNCH_S
 }
 
+// sums as above; x bf16, or xparts fp32 parts of rows * hidden each in xp.  Without
+// a residual x itself, in bf16, is what is normed
+void lig_lora_norm_open_launch(uint16_t* out, const uint16_t* x, const float* xp, int xparts, long xstride,
+                               uint16_t* residual, const uint16_t* weight, int hidden, const int* toks, const int* len,
+                               const int* slot, int ntiles, const float* u_in, int parts, int tiles,
+                               const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
+                               float* sums, hipStream_t stream) {
+#define LAUNCH_O(ADD, PARTS)                                                                                        \
+  hipLaunchKernelGGL((lora_norm_open_kernel<ADD, PARTS>), dim3(ntiles, hidden / NORM_STRIP), dim3(256), 0, stream, out, \
+                     x, xp, xparts, (size_t)xstride, residual, weight, hidden, toks, len, slot, u_in, parts, tiles,  \
+                     b_stack, a_stack, u_out, tiles_out, sums)
+  if (!residual) LAUNCH_O(false, false);
+  else if (xp) LAUNCH_O(true, true);
+  else LAUNCH_O(true, false);
+#undef LAUNCH_O
+}
+
 void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* toks, const int* len,
                           const int* slot, int ntiles, const float* u_in, int parts, int tiles,
                           const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
-                          hipStream_t stream) {
+                          const float* sums, int width, float eps, hipStream_t stream) {
   hipLaunchKernelGGL(lora_silu_kernel, dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(256), 0, stream, out, x, d,
-                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out);
+                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out, Factor{sums, width, eps});
 }
 
 int lig_lora_shrink_strip() { return SHRINK_STRIP; }
@@ -615,17 +794,23 @@ void lig_lora_shrink_launch(const uint16_t* x, int width, const int* toks, const
                      width, toks, len, slot, a_stack, u_out, tiles_out);
 }
 
-void lig_lora_qkv_rope_cache_launch(uint16_t* q_out, const uint16_t* qkv, const int64_t* positions,
+void lig_lora_qkv_rope_cache_launch(uint16_t* q_out, const uint16_t* qkv, const float* qkv_parts, int nparts,
+                                    long part_stride, const float* sums, int width, float eps, const int64_t* positions,
                                     const float* cos_sin, uint16_t* k_cache, uint16_t* v_cache,
                                     const int64_t* slot_mapping, int num_q_heads, int num_kv_heads, int head_dim,
                                     int block_size, const int* toks, const int* len, const int* slot,
                                     int ntiles, const float* u_in, int u_parts, int tiles, const uint16_t* b_stack,
                                     hipStream_t stream) {
   const int heads = num_q_heads + 2 * num_kv_heads;
-  const int waves = (head_dim / 64) * ((heads + QR_HEADS - 1) / QR_HEADS);
-  hipLaunchKernelGGL(lora_qkv_rope_cache_kernel, dim3(ntiles, (waves + 3) / 4), dim3(256), 0, stream, q_out, qkv,
-                     positions, cos_sin, k_cache, v_cache, slot_mapping, num_q_heads, num_kv_heads, head_dim,
-                     block_size, toks, len, slot, u_in, u_parts, tiles, b_stack);
+  const int waves = (head_dim / 64) * (qkv_parts ? heads : (heads + 3) / 4);
+#define LAUNCH_R(PARTS)                                                                                             \
+  hipLaunchKernelGGL((lora_qkv_rope_cache_kernel<PARTS>), dim3(ntiles, (waves + 3) / 4), dim3(256), 0, stream, q_out, qkv, \
+                     qkv_parts, nparts, (size_t)part_stride, Factor{sums, width, eps}, positions, cos_sin, k_cache,   \
+                     v_cache, slot_mapping, num_q_heads, num_kv_heads, head_dim, block_size, toks, len, slot, u_in,   \
+                     u_parts, tiles, b_stack)
+  if (qkv_parts) LAUNCH_R(true);
+  else LAUNCH_R(false);
+#undef LAUNCH_R
 }
 
 }  // extern "C"

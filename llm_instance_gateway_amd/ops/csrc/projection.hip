@@ -283,7 +283,9 @@ bool lig_projection_serves(long M, long N, long K) {
   return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64;
 }
 
-// Tile and parts of K, as one number; the parts need fp32 sums of [M, N] each.
+// Tile and parts of K, as one number.  To launch it: y alone where K is in one part,
+// y and room for the fp32 sums [parts, M, N], or that room alone, which then holds the
+// parts for the caller to add up.
 int lig_projection_plan(int M, int N, int K) {
   const Plan p = plan(M, N, K);
   return p.tile * (MAX_SPLITS + 1) + p.splits;
@@ -298,7 +300,7 @@ void lig_projection_launch(int p, uint16_t* y, float* part, const uint16_t* x, c
 #define X(BM, BN, WM, WN, WK, PK, ST)                                                                             \
   if (tile == i++) {                                                                                              \
     const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;                                             \
-    if (splits > 1)                                                                                               \
+    if (part)                                                                                                     \
       hipLaunchKernelGGL((projection_kernel<BM, BN, WM, WN, WK, PK, ST, true>), dim3(mtiles * ntiles * splits),   \
                          dim3(64 * WM * WN * WK), 0, stream, y, part, x, w, M, N, K, mtiles, ntiles);             \
     else                                                                                                          \
@@ -307,7 +309,7 @@ void lig_projection_launch(int p, uint16_t* y, float* part, const uint16_t* x, c
   }
   LIG_TILES(X)
 #undef X
-  if (splits > 1) {
+  if (part && y) {
     const long n = (long)M * N;
     hipLaunchKernelGGL(projection_sum_kernel, dim3((n / 8 + 255) / 256), dim3(256), 0, stream, y, part, n, splits);
   }

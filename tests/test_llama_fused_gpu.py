@@ -172,6 +172,57 @@ def test_lora_qkv_rope_cache(slots, Hq, Hkv, D, bs):
         assert ((x.float() - y).abs() <= 2.0 ** -8 * y.abs() + tol).all()
 
 
+@pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
+@pytest.mark.parametrize("H,cut", [(2048, 1), (3072, 3), (4096, 8), (4096, 0)])
+def test_lora_norm_open(slots, H, cut):
+    """The norm that leaves its factor to the readers of the product: its own
+    outputs, then the rotation and the gated silu with the factor."""
+    rnd, rows, sl = _lora(slots, H + cut)
+    T = len(slots)
+    assert ops.lora_norm_opens(rows, H)
+    res, w, u = rnd(T, H).to(BF), (1 + 0.1 * rnd(H)).to(BF), rnd(T, 16)
+    a, b = rnd(4, 16, H).to(BF), (0.1 * rnd(4, H, 16)).to(BF)
+    x = rnd(cut, T, H) if cut else rnd(T, H).to(BF)
+    ws, _, wd = ops.lora_workspace(rows, H, 32, 1024)
+    d, mag = _delta(u, b, sl)
+    for with_res in (True, False):
+        residual = res.clone() if with_res else None
+        if with_res:
+            h, u_out, norm = ops.lora_norm_open(x, residual, w, 1e-5, rows, _pack(u, rows, 3), b, a, ws)
+            s, tol = (x.sum(0) if cut else x.float()) + res.float() + d, 2.0 ** -16 * mag + 1e-5
+            assert ((residual.float() - s).abs() <= 2.0 ** -8 * s.abs() + tol).all()
+        else:
+            h, u_out, norm = ops.lora_norm_open(res, None, w, 1e-5, rows, a_stack=a, u_out=ws)
+            s, tol = res.float(), 0.0
+        assert ((h.float() - s * w.float()).abs() <= 2.0 ** -8 * (s * w.float()).abs() + 2 * tol).all()
+        _check_u(u_out, h, a, sl, rows)
+        f = torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5)
+        # readers: `y` and B u lack f; 2^-16 of the sums of B u, 2^-18 for f itself
+        y, bd = rnd(T, 2048).to(BF), (0.1 * rnd(4, 2048, 16)).to(BF)
+        up = _unpack(u_out, rows, T)
+        dl, m2 = _delta(up, bd, sl)
+        v, vm = (y.float() + dl) * f, (2.0 ** -15 * m2 + 2.0 ** -18 * y.float().abs()) * f
+        got = ops.lora_silu_and_mul(y, rows, u_out, bd, rnd(4, 16, 1024).to(BF), wd, norm)
+        gate, uu = v.chunk(2, dim=-1)
+        tg, tu = vm.chunk(2, dim=-1)
+        ref = gate * torch.sigmoid(gate) * uu
+        tol = 1.1 * tg * uu.abs() + tu * (gate * torch.sigmoid(gate)).abs() + 1e-5 * (1 + ref.abs())
+        assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + tol).all()
+        # 8 query, 4 key and 4 value heads of 128, the product in parts
+        kc, vc = rnd(9, 4, 16, 128).to(BF), rnd(9, 4, 16, 128).to(BF)
+        cs = ops.build_cos_sin_cache(128, 500, 1e4, "cuda").float()
+        pos, at = torch.arange(T, device="cuda"), torch.randperm(144, device="cuda")[:T]
+        yp = rnd(2, T, 2048)
+        q, k, vv = ((yp.sum(0) + dl) * f).split([1024, 512, 512], dim=-1)
+        qr, kr = torch_ref.rotary_embedding(pos, q, k, cs, 128)
+        kw, vw = kc.float(), vc.float()
+        torch_ref.reshape_and_cache(kr, vv, kw, vw, at)
+        got = ops.lora_qkv_rope_cache(yp, pos, cs, kc, vc, at, 8, rows, u_out, bd, norm)
+        tol = 2.0 ** -14 * (m2 * f).max() + 2.0 ** -17 * q.abs().max() + 1e-5
+        for p, r in ((got, qr), (kc, kw), (vc, vw)):
+            assert ((p.float() - r).abs() <= 2.0 ** -8 * r.abs() + tol).all()
+
+
 def test_engine_matches_unit_kernels(monkeypatch):
     """A whole step through the in-layer kernels beside one through the SGMV
     kernels, prompts and decodes, eager and through the decode graph."""
