@@ -234,6 +234,8 @@ class LlamaForCausalLM(nn.Module):
             return self._forward_lora(hidden, positions, kv_caches, meta)
         if hidden.shape[0] == 1 and meta.lora_slot_per_token is None and self._row_products():
             return self._forward_row(hidden, positions, kv_caches, meta)
+        if meta.lora_slot_per_token is None and self._open_norms(len(hidden)):
+            return self._forward_open(hidden, positions, kv_caches, meta)
         residual = None
         for layer, kv in zip(self.layers, kv_caches):
             hidden, residual = layer(
@@ -309,6 +311,40 @@ class LlamaForCausalLM(nn.Module):
         hidden, _ = ops.fused_add_rms_norm(x, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
+    def _open_norms(self, rows: int) -> bool:
+        """Whether `_forward_open` is for a step of that many rows without adapters:
+        where `ops.linear` runs its products (asked of one layer: a product that
+        runs elsewhere comes rounded, which the kernels behind it take as well)."""
+        c = self.cfg
+        if (self.tp is not None or not self.norm.is_cuda or self.norm.dtype != torch.bfloat16
+                or c.intermediate_size % 32 or c.head_dim % 64 or not ops.lora_norm_opens(ops.BASE_ROWS, rows, c.hidden_size)):
+            return False
+        layer = self.layers[0]
+        attn, mlp = layer.self_attn, getattr(layer, "mlp", None)
+        return type(mlp) is MLP and self.plain_layers() and all(
+            _served(m, rows) for m in (attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj))
+
+    def _forward_open(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
+        """The layers with each norm as one kernel that adds up the product before
+        it and leaves its factor to the rotation and the activation."""
+        rows = ops.BASE_ROWS
+        residual, y = None, hidden
+        for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
+            attn, mlp = layer.self_attn, layer.mlp
+            h, _, norm = ops.lora_norm_open(y, residual, layer.input_layernorm, layer.eps, rows)
+            if residual is None:
+                residual = hidden
+            q = ops.lora_qkv_rope_cache(
+                _project(attn.qkv_proj, h, ops.linear_parts), positions, self.cos_sin_cache, kv[0], kv[1],
+                meta.slot_mapping, attn.num_heads, rows, None, None, norm)
+            o = attn.attend(q, kv, meta)
+            h, _, norm = ops.lora_norm_open(
+                _project(attn.o_proj, o, ops.linear_parts), residual, layer.post_attention_layernorm, layer.eps, rows)
+            act = ops.lora_silu_and_mul(_project(mlp.gate_up_proj, h), rows, None, None, None, None, norm)
+            last = i + 1 == len(self.layers)
+            y = _project(mlp.down_proj, act, ops.linear if last else ops.linear_parts)
+        return ops.fused_add_rms_norm(y, residual, self.norm, self.cfg.rms_norm_eps)[0]
+
     def lora_in_layer(self, rank: int, dims: dict) -> bool:
         """Whether `_forward_lora` serves adapters of that rank over those
         modules: what the kernels of ops/csrc/lora_rows.hip take."""
@@ -337,11 +373,15 @@ class LlamaForCausalLM(nn.Module):
         # Norms whose readers can take the rows' factor themselves are one launch, and
         # add up the product before them.  The rotation takes it with fp32 parts
         # only: a rounded product would be rounded once more on its way to V.
-        opens = ops.lora_norm_opens(rows, c.hidden_size)
-        open_in = [opens and _served(layer.self_attn.qkv_proj, len(hidden)) for layer in self.layers] + [False]
+        opens = ops.lora_norm_opens(rows, len(hidden), c.hidden_size)
+
+        def open_in(i):  # the norm at layer i's entry
+            return opens and i < len(self.layers) and _served(self.layers[i].self_attn.qkv_proj, len(hidden))
+
+        parts = open_in(0)
         for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
             attn, mlp = layer.self_attn, layer.mlp
-            norm = ops.lora_norm_open if open_in[i] else ops.lora_rms_norm
+            norm = ops.lora_norm_open if parts else ops.lora_rms_norm
             if last is None:
                 h, u, *scale = norm(y, None, layer.input_layernorm, layer.eps, rows, a_stack=a[(i, "qkv")], u_out=ws)
                 residual = hidden
@@ -349,7 +389,7 @@ class LlamaForCausalLM(nn.Module):
                 h, u, *scale = norm(
                     y, residual, layer.input_layernorm, layer.eps, rows, u_down, b[(last, "down")], a[(i, "qkv")], ws)
             q = ops.lora_qkv_rope_cache(
-                _project(attn.qkv_proj, h, ops.linear_parts if open_in[i] else ops.linear), positions, self.cos_sin_cache,
+                _project(attn.qkv_proj, h, ops.linear_parts if parts else ops.linear), positions, self.cos_sin_cache,
                 kv[0], kv[1], meta.slot_mapping, attn.num_heads, rows, u, b[(i, "qkv")], *scale)
             o = attn.attend(q, kv, meta)
             ops.lora_shrink(o, rows, a[(i, "o")], u_o)
@@ -359,7 +399,8 @@ class LlamaForCausalLM(nn.Module):
                 layer.post_attention_layernorm, layer.eps, rows, u_o, b[(i, "o")], a[(i, "gate_up")], ws)
             act = ops.lora_silu_and_mul(
                 _project(mlp.gate_up_proj, h), rows, u, b[(i, "gate_up")], a[(i, "down")], u_down, *scale)
-            y, last = _project(mlp.down_proj, act, ops.linear_parts if open_in[i + 1] else ops.linear), i
+            parts = open_in(i + 1)
+            y, last = _project(mlp.down_proj, act, ops.linear_parts if parts else ops.linear), i
         return ops.lora_rms_norm(
             y, residual, self.norm, self.cfg.rms_norm_eps, rows, u_down, b[(last, "down")])[0]
 

@@ -409,9 +409,17 @@ def lora_rms_norm(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_sta
     return out, None if u_out is None else u_out[:parts]
 
 
-def lora_norm_opens(rows, width: int) -> bool:
+# `rows` of a step without adapters, for the kernels that take it: all rows in order
+BASE_ROWS = (None, None, None)
+
+
+def _tiles(rows, T: int) -> int:
+    return -(-T // 16) if rows[1] is None else rows[1].shape[0]
+
+
+def lora_norm_opens(rows, T: int, width: int) -> bool:
     """Whether `lora_norm_open` is for these tiles: where the norm takes strips."""
-    return (width >= 2048 and rows[1].shape[0] * 4096 < LORA_NORM_STRIPS_BELOW * width
+    return (width >= 2048 and _tiles(rows, T) * 4096 < LORA_NORM_STRIPS_BELOW * width
             and width % _load_ext().lora_norm_strip() == 0)
 
 
@@ -420,11 +428,11 @@ def lora_norm_open(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_st
     u_out, and of any product of h); x may be `linear_parts` of a product.  Returns
     h, the parts of u_out and what the reader of the product finds the factor by."""
     T, H = x.shape[-2:]
-    n, parts = rows[1].shape[0], H // _EXT.lora_norm_strip()
+    n, parts = _tiles(rows, T), H // _EXT.lora_norm_strip()
     out = torch.empty(T, H, dtype=weight.dtype, device=x.device)
     sums = torch.empty(n * parts * 16, dtype=torch.float32, device=x.device)
     _EXT.lora_norm_open(out, x, residual, weight, *rows, u_in, b_stack, a_stack, u_out, sums, _stream())
-    return out, u_out[:parts], (sums, H, eps)
+    return out, None if u_out is None else u_out[:parts], (sums, H, eps)
 
 
 def lora_silu_and_mul(x, rows, u_in, b_stack, a_stack, u_out, norm=(None, 0, 0.0)):

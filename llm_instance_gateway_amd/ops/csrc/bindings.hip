@@ -100,11 +100,11 @@ void lig_lora_rms_norm_strips_launch(
     const uint16_t*, const uint16_t*, float*, int, float*, hipStream_t);
 void lig_lora_norm_open_launch(uint16_t*, const uint16_t*, const float*, int, long, uint16_t*, const uint16_t*, int,
                                const int*, const int*, const int*, int, const float*, int, int, const uint16_t*,
-                               const uint16_t*, float*, int, float*, hipStream_t);
+                               const uint16_t*, float*, int, float*, int, hipStream_t);
 void lig_lora_silu_launch(uint16_t*, const uint16_t*, int, const int*,
                           const int*, const int*, int, const float*, int, int,
                           const uint16_t*, const uint16_t*, float*, int,
-                          const float*, int, float, hipStream_t);
+                          const float*, int, float, int, hipStream_t);
 void lig_lora_shrink_launch(const uint16_t*, int, const int*, const int*,
                             const int*, int, const uint16_t*, float*, int,
                             hipStream_t);
@@ -112,7 +112,7 @@ int lig_lora_shrink_strip();
 void lig_lora_qkv_rope_cache_launch(
     uint16_t*, const uint16_t*, const float*, int, long, const float*, int, float, const int64_t*, const float*, uint16_t*,
     uint16_t*, const int64_t*, int, int, int, int, const int*, const int*,
-    const int*, int, const float*, int, int, const uint16_t*, hipStream_t);
+    const int*, int, const float*, int, int, const uint16_t*, int, hipStream_t);
 void lig_paged_attention_prefill_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const int*,
     const int*, const int*, const int*, const int*, float, int, int, int,
@@ -592,6 +592,8 @@ void lora_rms_norm(torch::Tensor out, torch::Tensor x,
   TORCH_CHECK(rc == 0, "lora_rms_norm: rows of ", H, " entries not served");
 }
 
+using OptTensor = std::optional<torch::Tensor>;
+
 // sums of squares per tile and strip of rows of `width` columns
 inline float* sums_ptr(const std::optional<torch::Tensor>& sums, int64_t width, int64_t n) {
   if (!sums) return nullptr;
@@ -601,45 +603,64 @@ inline float* sums_ptr(const std::optional<torch::Tensor>& sums, int64_t width, 
   return sums->data_ptr<float>();
 }
 
+// tiles of a step: listed, or the rows in their order without adapters
+struct RowTiles {
+  const int *toks = nullptr, *len = nullptr, *slot = nullptr;
+  int n;
+};
+inline RowTiles tiles_of(const OptTensor& toks, const OptTensor& len, const OptTensor& slot, int64_t T, int64_t slots) {
+  RowTiles t;
+  TORCH_CHECK(toks.has_value() == len.has_value() && toks.has_value() == slot.has_value());
+  if (!toks) {
+    t.n = (int)((T + 15) / 16);
+    return t;
+  }
+  t.n = check_tiles(*toks, *len, *slot, T, slots);
+  t.toks = i32_cptr(*toks);
+  t.len = i32_cptr(*len);
+  t.slot = i32_cptr(*slot);
+  return t;
+}
+
 // out = (residual + x + B u_in) * weight, which residual becomes without the weight, u_out = A out and
 // `sums` for the norm's factor; x bf16 [T, H] or the fp32 parts [S, T, H] of a product
-void lora_norm_open(torch::Tensor out, torch::Tensor x, std::optional<torch::Tensor> residual, torch::Tensor weight,
-                    torch::Tensor toks, torch::Tensor len, torch::Tensor slot, std::optional<torch::Tensor> u_in,
-                    std::optional<torch::Tensor> b_stack, torch::Tensor a_stack, torch::Tensor u_out,
-                    torch::Tensor sums, int64_t stream) {
+void lora_norm_open(torch::Tensor out, torch::Tensor x, OptTensor residual, torch::Tensor weight, OptTensor toks,
+                    OptTensor len, OptTensor slot, OptTensor u_in, OptTensor b_stack, OptTensor a_stack,
+                    OptTensor u_out, torch::Tensor sums, int64_t stream) {
   const bool parts = x.dim() == 3;
   const int T = out.size(0), H = out.size(1);
   TORCH_CHECK(x.size(-1) == H && x.size(-2) == T && x.is_contiguous() && x.is_cuda() && weight.numel() == H);
   TORCH_CHECK(!parts || (x.scalar_type() == torch::kFloat32 && x.size(0) > 0 && residual));
   TORCH_CHECK(!residual || residual->sizes() == out.sizes());
   TORCH_CHECK(u_in.has_value() == b_stack.has_value() && (!u_in || residual));
-  const int n = check_tiles(toks, len, slot, T, a_stack.size(0));
-  if (n == 0 || T == 0) return;
+  TORCH_CHECK(u_out.has_value() == a_stack.has_value() && u_out.has_value() == toks.has_value());
+  const RowTiles t = tiles_of(toks, len, slot, T, a_stack ? a_stack->size(0) : 0);
+  if (t.n == 0 || T == 0) return;
   lig_lora_norm_open_launch(
       bf16_ptr(out), parts ? nullptr : bf16_cptr(x), parts ? x.data_ptr<float>() : nullptr, parts ? (int)x.size(0) : 0,
-      (long)T * H, residual ? bf16_ptr(*residual) : nullptr, bf16_cptr(weight), H, i32_cptr(toks), i32_cptr(len),
-      i32_cptr(slot), n, u_in ? u_ptr(*u_in, 1, n) : nullptr, u_in ? (int)u_in->size(0) : 0,
-      u_in ? (int)u_in->size(1) : 0, b_stack ? b_ptr(*b_stack, H) : nullptr, a_ptr(a_stack, H),
-      u_ptr(u_out, H / lig_lora_norm_strip(), n), (int)u_out.size(1), sums_ptr(sums, H, n), as_stream(stream));
+      (long)T * H, residual ? bf16_ptr(*residual) : nullptr, bf16_cptr(weight), H, t.toks, t.len, t.slot, t.n,
+      u_in ? u_ptr(*u_in, 1, t.n) : nullptr, u_in ? (int)u_in->size(0) : 0, u_in ? (int)u_in->size(1) : 0,
+      b_stack ? b_ptr(*b_stack, H) : nullptr, a_stack ? a_ptr(*a_stack, H) : nullptr,
+      u_out ? u_ptr(*u_out, H / lig_lora_norm_strip(), t.n) : nullptr, u_out ? (int)u_out->size(1) : 0,
+      sums_ptr(sums, H, t.n), T, as_stream(stream));
 }
 
-void lora_silu(torch::Tensor out, torch::Tensor x, torch::Tensor toks,
-               torch::Tensor len, torch::Tensor slot,
-               torch::Tensor u_in, torch::Tensor b_stack,
-               torch::Tensor a_stack, torch::Tensor u_out, std::optional<torch::Tensor> sums, int64_t width, double eps,
+void lora_silu(torch::Tensor out, torch::Tensor x, OptTensor toks, OptTensor len, OptTensor slot, OptTensor u_in,
+               OptTensor b_stack, OptTensor a_stack, OptTensor u_out, OptTensor sums, int64_t width, double eps,
                int64_t stream) {
   const int T = x.size(0), d = out.size(1);
   TORCH_CHECK(out.size(0) == T && x.size(1) == 2 * (int64_t)d && d % 32 == 0);
-  const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
-  if (n == 0 || T == 0) return;
+  for (const OptTensor* o : {&u_in, &b_stack, &a_stack, &u_out}) TORCH_CHECK(o->has_value() == toks.has_value());
+  const RowTiles t = tiles_of(toks, len, slot, T, b_stack ? b_stack->size(0) : 0);
+  if (t.n == 0 || T == 0) return;
   const int strip = lig_lora_silu_strip();
-  TORCH_CHECK(a_stack.size(0) == b_stack.size(0));
-  lig_lora_silu_launch(bf16_ptr(out), bf16_cptr(x), d, i32_cptr(toks),
-                       i32_cptr(len), i32_cptr(slot), n,
-                       u_ptr(u_in, 1, n), (int)u_in.size(0), (int)u_in.size(1),
-                       b_ptr(b_stack, 2 * (int64_t)d),
-                       a_ptr(a_stack, d), u_ptr(u_out, (d + strip - 1) / strip, n),
-                       (int)u_out.size(1), sums_ptr(sums, width, n), (int)width, (float)eps, as_stream(stream));
+  TORCH_CHECK(!toks || a_stack->size(0) == b_stack->size(0));
+  lig_lora_silu_launch(bf16_ptr(out), bf16_cptr(x), d, t.toks, t.len, t.slot, t.n,
+                       toks ? u_ptr(*u_in, 1, t.n) : nullptr, toks ? (int)u_in->size(0) : 0,
+                       toks ? (int)u_in->size(1) : 0, toks ? b_ptr(*b_stack, 2 * (int64_t)d) : nullptr,
+                       toks ? a_ptr(*a_stack, d) : nullptr, toks ? u_ptr(*u_out, (d + strip - 1) / strip, t.n) : nullptr,
+                       toks ? (int)u_out->size(1) : 0, sums_ptr(sums, width, t.n), (int)width, (float)eps, T,
+                       as_stream(stream));
 }
 
 void lora_shrink(torch::Tensor x, torch::Tensor toks,
@@ -658,10 +679,8 @@ void lora_shrink(torch::Tensor x, torch::Tensor toks,
 void lora_qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
                          torch::Tensor positions, torch::Tensor cos_sin,
                          torch::Tensor k_cache, torch::Tensor v_cache,
-                         torch::Tensor slot_mapping, torch::Tensor toks,
-                         torch::Tensor len,
-                         torch::Tensor slot, torch::Tensor u_in,
-                         torch::Tensor b_stack, std::optional<torch::Tensor> sums, int64_t width, double eps,
+                         torch::Tensor slot_mapping, OptTensor toks, OptTensor len, OptTensor slot,
+                         OptTensor u_in, OptTensor b_stack, OptTensor sums, int64_t width, double eps,
                          int64_t stream) {
   TORCH_CHECK(positions.scalar_type() == torch::kInt64);
   TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
@@ -674,16 +693,16 @@ void lora_qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
   TORCH_CHECK(qkv.size(-1) == (int64_t)(Hq + 2 * Hkv) * D && q_out.size(0) == T &&
               q_out.size(1) == (int64_t)Hq * D);
   TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
-  const int n = check_tiles(toks, len, slot, T, b_stack.size(0));
-  if (n == 0 || T == 0) return;
+  TORCH_CHECK(u_in.has_value() == toks.has_value() && b_stack.has_value() == toks.has_value());
+  const RowTiles t = tiles_of(toks, len, slot, T, b_stack ? b_stack->size(0) : 0);
+  if (t.n == 0 || T == 0) return;
   lig_lora_qkv_rope_cache_launch(
       bf16_ptr(q_out), parts ? nullptr : bf16_cptr(qkv), parts ? qkv.data_ptr<float>() : nullptr,
-      parts ? (int)qkv.size(0) : 0, (long)T * qkv.size(-1), sums_ptr(sums, width, n), (int)width, (float)eps,
-      positions.data_ptr<int64_t>(),
-      cos_sin.data_ptr<float>(), bf16_ptr(k_cache), bf16_ptr(v_cache),
-      slot_mapping.data_ptr<int64_t>(), Hq, Hkv, D, BS, i32_cptr(toks),
-      i32_cptr(len), i32_cptr(slot), n, u_ptr(u_in, 1, n),
-      (int)u_in.size(0), (int)u_in.size(1), b_ptr(b_stack, qkv.size(-1)), as_stream(stream));
+      parts ? (int)qkv.size(0) : 0, (long)T * qkv.size(-1), sums_ptr(sums, width, t.n), (int)width, (float)eps,
+      positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), bf16_ptr(k_cache), bf16_ptr(v_cache),
+      slot_mapping.data_ptr<int64_t>(), Hq, Hkv, D, BS, t.toks, t.len, t.slot, t.n,
+      toks ? u_ptr(*u_in, 1, t.n) : nullptr, toks ? (int)u_in->size(0) : 0, toks ? (int)u_in->size(1) : 0,
+      toks ? b_ptr(*b_stack, qkv.size(-1)) : nullptr, T, as_stream(stream));
 }
 
 }  // namespace

@@ -16,7 +16,7 @@
 //   * u stays fp32 between the two, where a bf16 workspace held it before.
 // Both are matrix instructions.  The rows of a launch are tiles of up to 16
 // tokens of one adapter (or of none), listed by the host 16 places a tile, so
-// that a lane finds its row in one load.  In all kernels lane
+// that a lane finds its row in one load; steps without adapters give no list.  In all kernels lane
 // (li, lg) holds 8 neighbouring columns lg*8 .. of token li in a group of 32:
 //   * u^T = A x^T: those 8 values are the second operand as they are;
 //   * y^T += B u^T: with B's rows dealt to two tiles (rows lg*4+i hold columns
@@ -41,8 +41,16 @@ struct Tile {
   bool valid;
 };
 
-LIG_DEVICE Tile tile_of(const int* toks, const int* len, const int* slot, int tile, int li) {
+// without a list: rows in their order, none with an adapter
+LIG_DEVICE Tile tile_of(const int* toks, const int* len, const int* slot, int tile, int li, int rows = 0) {
   Tile t;
+  if (toks == nullptr) {
+    t.n = min(16, rows - tile * 16);
+    t.slot = -1;
+    t.row = tile * 16 + min(li, t.n - 1);
+    t.valid = li < t.n;
+    return t;
+  }
   t.row = toks[tile * 16 + li];
   t.n = len[tile];
   t.slot = slot[tile];
@@ -453,12 +461,12 @@ __global__ __launch_bounds__(256) void lora_norm_open_kernel(
     const size_t xstride, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, const int hidden,
     const int* __restrict__ toks, const int* __restrict__ len, const int* __restrict__ slot, const float* u_in,
     const int parts, const int tiles, const uint16_t* __restrict__ b_stack, const uint16_t* __restrict__ a_stack,
-    float* u_out, const int tiles_out, float* sums) {
+    float* u_out, const int tiles_out, float* sums, const int rows) {
   __shared__ __align__(16) float smem[4 * 16 * R];
   const int tile = blockIdx.x;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const Tile t = tile_of(toks, len, slot, tile, li);
+  const Tile t = tile_of(toks, len, slot, tile, li, rows);
   if (t.n == 0) return;
   const bool delta = u_in != nullptr && t.slot >= 0, to_u = t.slot >= 0;
   const float* ui = delta ? u_in + (size_t)tile * 16 * R : nullptr;
@@ -542,12 +550,13 @@ __global__ __launch_bounds__(256) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
     const int* __restrict__ len, const int* __restrict__ slot,
     const float* __restrict__ u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
-    const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm) {
+    const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm,
+    const int rows) {
   __shared__ __align__(16) float red[4][16][R];
   const int tile = blockIdx.x, strip = blockIdx.y;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const Tile t = tile_of(toks, len, slot, tile, li);
+  const Tile t = tile_of(toks, len, slot, tile, li, rows);
   if (t.n == 0) return;
   const int c_first = strip * SILU_STRIP + wave * 32;
   const float factor = factor_of(norm, tile, li);
@@ -605,7 +614,7 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
     const int64_t* __restrict__ slot_mapping, const int num_q_heads, const int num_kv_heads, const int head_dim,
     const int block_size, const int* __restrict__ toks, const int* __restrict__ len,
     const int* __restrict__ slot, const float* __restrict__ u_in, const int u_parts, const int tiles,
-    const uint16_t* __restrict__ b_stack) {
+    const uint16_t* __restrict__ b_stack, const int rows) {
   constexpr int QR_HEADS = PARTS ? 1 : 4;
   __shared__ __align__(16) float smem[16 * R];
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
@@ -613,7 +622,7 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
   const int wid = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int heads = num_q_heads + 2 * num_kv_heads;
   const int h0 = (wid / parts) * QR_HEADS;
-  const Tile t = tile_of(toks, len, slot, blockIdx.x, li);
+  const Tile t = tile_of(toks, len, slot, blockIdx.x, li, rows);
   if (t.n == 0) return;
   bf16x8_t u = {};
   if (t.slot >= 0) u = u_of(u_in + (size_t)blockIdx.x * 16 * R, u_parts, tiles, smem, li, lg, t.valid);
@@ -767,11 +776,11 @@ void lig_lora_norm_open_launch(uint16_t* out, const uint16_t* x, const float* xp
                                uint16_t* residual, const uint16_t* weight, int hidden, const int* toks, const int* len,
                                const int* slot, int ntiles, const float* u_in, int parts, int tiles,
                                const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
-                               float* sums, hipStream_t stream) {
+                               float* sums, int rows, hipStream_t stream) {
 #define LAUNCH_O(ADD, PARTS)                                                                                        \
   hipLaunchKernelGGL((lora_norm_open_kernel<ADD, PARTS>), dim3(ntiles, hidden / NORM_STRIP), dim3(256), 0, stream, out, \
                      x, xp, xparts, (size_t)xstride, residual, weight, hidden, toks, len, slot, u_in, parts, tiles,  \
-                     b_stack, a_stack, u_out, tiles_out, sums)
+                     b_stack, a_stack, u_out, tiles_out, sums, rows)
   if (!residual) LAUNCH_O(false, false);
   else if (xp) LAUNCH_O(true, true);
   else LAUNCH_O(true, false);
@@ -781,9 +790,9 @@ void lig_lora_norm_open_launch(uint16_t* out, const uint16_t* x, const float* xp
 void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* toks, const int* len,
                           const int* slot, int ntiles, const float* u_in, int parts, int tiles,
                           const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
-                          const float* sums, int width, float eps, hipStream_t stream) {
+                          const float* sums, int width, float eps, int rows, hipStream_t stream) {
   hipLaunchKernelGGL(lora_silu_kernel, dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(256), 0, stream, out, x, d,
-                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out, Factor{sums, width, eps});
+                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out, Factor{sums, width, eps}, rows);
 }
 
 int lig_lora_shrink_strip() { return SHRINK_STRIP; }
@@ -800,14 +809,14 @@ void lig_lora_qkv_rope_cache_launch(uint16_t* q_out, const uint16_t* qkv, const 
                                     const int64_t* slot_mapping, int num_q_heads, int num_kv_heads, int head_dim,
                                     int block_size, const int* toks, const int* len, const int* slot,
                                     int ntiles, const float* u_in, int u_parts, int tiles, const uint16_t* b_stack,
-                                    hipStream_t stream) {
+                                    int rows, hipStream_t stream) {
   const int heads = num_q_heads + 2 * num_kv_heads;
   const int waves = (head_dim / 64) * (qkv_parts ? heads : (heads + 3) / 4);
 #define LAUNCH_R(PARTS)                                                                                             \
   hipLaunchKernelGGL((lora_qkv_rope_cache_kernel<PARTS>), dim3(ntiles, (waves + 3) / 4), dim3(256), 0, stream, q_out, qkv, \
                      qkv_parts, nparts, (size_t)part_stride, Factor{sums, width, eps}, positions, cos_sin, k_cache,   \
                      v_cache, slot_mapping, num_q_heads, num_kv_heads, head_dim, block_size, toks, len, slot, u_in,   \
-                     u_parts, tiles, b_stack)
+                     u_parts, tiles, b_stack, rows)
   if (qkv_parts) LAUNCH_R(true);
   else LAUNCH_R(false);
 #undef LAUNCH_R

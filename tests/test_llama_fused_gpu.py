@@ -179,7 +179,7 @@ def test_lora_norm_open(slots, H, cut):
     outputs, then the rotation and the gated silu with the factor."""
     rnd, rows, sl = _lora(slots, H + cut)
     T = len(slots)
-    assert ops.lora_norm_opens(rows, H)
+    assert ops.lora_norm_opens(rows, T, H)
     res, w, u = rnd(T, H).to(BF), (1 + 0.1 * rnd(H)).to(BF), rnd(T, 16)
     a, b = rnd(4, 16, H).to(BF), (0.1 * rnd(4, H, 16)).to(BF)
     x = rnd(cut, T, H) if cut else rnd(T, H).to(BF)
@@ -221,6 +221,35 @@ def test_lora_norm_open(slots, H, cut):
         tol = 2.0 ** -14 * (m2 * f).max() + 2.0 ** -17 * q.abs().max() + 1e-5
         for p, r in ((got, qr), (kc, kw), (vc, vw)):
             assert ((p.float() - r).abs() <= 2.0 ** -8 * r.abs() + tol).all()
+
+
+@pytest.mark.parametrize("T", [1, 16, 33])
+def test_base_rows(T):
+    """The same kernels without a list of tiles: every row, no adapters."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    H, rows = 2048, ops.BASE_ROWS
+    x, res, w = rnd(3, T, H), rnd(T, H).to(BF), (1 + 0.1 * rnd(H)).to(BF)
+    s, residual = x.sum(0) + res.float(), res.clone()
+    h, u, norm = ops.lora_norm_open(x, residual, w, 1e-5, rows)
+    assert u is None and ((residual.float() - s).abs() <= 2.0 ** -8 * s.abs() + 1e-5).all()
+    assert ((h.float() - s * w.float()).abs() <= 2.0 ** -8 * (s * w.float()).abs() + 1e-5).all()
+    f = torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5)
+    y = rnd(T, H).to(BF)
+    gate, up = (y.float() * f).chunk(2, dim=-1)
+    ref = gate * torch.sigmoid(gate) * up
+    got = ops.lora_silu_and_mul(y, rows, None, None, None, None, norm)
+    assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * (1 + ref.abs())).all()
+    kc, vc = rnd(9, 4, 16, 128).to(BF), rnd(9, 4, 16, 128).to(BF)
+    cs = ops.build_cos_sin_cache(128, 500, 1e4, "cuda").float()
+    pos, at = torch.arange(T, device="cuda"), torch.randperm(144, device="cuda")[:T]
+    q, k, v = (x.sum(0) * f).split([1024, 512, 512], dim=-1)
+    qr, kr = torch_ref.rotary_embedding(pos, q, k, cs, 128)
+    kw, vw = kc.float(), vc.float()
+    torch_ref.reshape_and_cache(kr, v, kw, vw, at)
+    got = ops.lora_qkv_rope_cache(x, pos, cs, kc, vc, at, 8, rows, None, None, norm)
+    for p, r in ((got, qr), (kc, kw), (vc, vw)):
+        assert ((p.float() - r).abs() <= 2.0 ** -8 * r.abs() + 2.0 ** -17 * q.abs().max() + 1e-5).all()
 
 
 def test_engine_matches_unit_kernels(monkeypatch):
