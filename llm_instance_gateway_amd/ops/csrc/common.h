@@ -42,11 +42,17 @@ LIG_DEVICE f32x8 bf16x8_to_f32x8(u16x8 h) {
   return out;
 }
 
+// As vectors: one conversion makes two numbers, element by element each takes a
+// conversion and the packing another.
 LIG_DEVICE u16x8 f32x8_to_bf16x8(f32x8 f) {
-  u16x8 out;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) out[i] = f32_to_bf16(f[i]);
-  return out;
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(u16x8, __builtin_convertvector(f, bf16x8));
+}
+
+LIG_DEVICE uint32_t pack_bf16(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
 // ---- wave reductions --------------------------------------------------------

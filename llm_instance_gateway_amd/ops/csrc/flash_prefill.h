@@ -70,10 +70,6 @@ struct Args {
   float softcap;
 };
 
-LIG_DEVICE uint32_t pack_bf16(float a, float b) {
-  return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
-}
-
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
 // sigmoid(score + bias) weights.  EXTRA: temperature, gate, sink, chunk and
 // window are looked at (the plain causal kernel leaves them out).
@@ -118,7 +114,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 
   // ---- rows of this wave: row rb*16 + li belongs to this lane ---------------
   bf16x8_t q_frag[RB][KS];
-  float c[RB];         // log2 units per unit of the raw score
+  float c[RB];         // log2 units per unit of the raw score; CAP: twice those of the score over the cap
   int key_lo[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -140,7 +136,8 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
     // raw score is the largest scaled one
     const uint32_t flip = sc < 0.f ? 0x80008000u : 0u;
     sc = fabsf(sc);
-    c[rb] = CAP ? sc / a.softcap : sc * LOG2E;
+    // not zero: a masked score is minus infinity, and stays so times c
+    c[rb] = CAP ? sc / a.softcap * (2.f * LOG2E) : fmaxf(sc * LOG2E, 1e-30f);
     const uint16_t* qp = a.q + (size_t)(lo + rr) * a.q_stride + (size_t)h * D;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -150,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
       q_frag[rb][ks] = __builtin_bit_cast(bf16x8_t, raw);
     }
   }
-  const float bias = SIG && a.score_bias ? a.score_bias[h] : 0.f;
+  const float bias = SIG && a.score_bias ? a.score_bias[h] * LOG2E : 0.f;
   const float cap2 = CAP ? a.softcap * LOG2E : 0.f;
 
   float m[RB], l[RB];
@@ -197,21 +194,30 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   auto visible = [&](int t) { return min(EXTRA ? max(t, first_key) : t, kv_end - 1); };
   auto block_of = [&](int kv0) { return PB ? bt[visible(kv0 + st * TPT) >> a.block_shift] : 0; };
   auto fetch = [&](int kv0, int blk) {
-    size_t row[TPT];
+    if constexpr (PB) {
+      const size_t rows = (size_t)blk * block_rows + kv_head_rows;
+      const uint16_t* kb = a.k_cache + rows * D + ch * 8;
+      const uint16_t* vb = a.v_cache + rows * a.v_row + ch * 8;
+      int row[TPT];
 #pragma unroll
-    for (int i = 0; i < TPT; ++i) {
-      const int t = visible(kv0 + st * TPT + i);
-      if constexpr (PB) {
-        row[i] = (size_t)blk * block_rows + kv_head_rows + (t & (a.block_size - 1));
-      } else {
-        const int b = t / a.block_size;
+      for (int i = 0; i < TPT; ++i) row[i] = visible(kv0 + st * TPT + i) & (a.block_size - 1);
+#pragma unroll
+      for (int i = 0; i < TPT; ++i) {
+        kreg[i] = *reinterpret_cast<const u32x4*>(kb + row[i] * D);
+        vreg[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)(uint32_t)row[i] * (uint32_t)a.v_row);
+      }
+    } else {
+      size_t row[TPT];
+#pragma unroll
+      for (int i = 0; i < TPT; ++i) {
+        const int t = visible(kv0 + st * TPT + i), b = t / a.block_size;
         row[i] = (size_t)bt[b] * block_rows + kv_head_rows + (t - b * a.block_size);
       }
-    }
 #pragma unroll
-    for (int i = 0; i < TPT; ++i) {
-      kreg[i] = *reinterpret_cast<const u32x4*>(a.k_cache + row[i] * D + ch * 8);
-      vreg[i] = *reinterpret_cast<const u32x4*>(a.v_cache + row[i] * a.v_row + ch * 8);
+      for (int i = 0; i < TPT; ++i) {
+        kreg[i] = *reinterpret_cast<const u32x4*>(a.k_cache + row[i] * D + ch * 8);
+        vreg[i] = *reinterpret_cast<const u32x4*>(a.v_cache + row[i] * a.v_row + ch * 8);
+      }
     }
   };
   auto stage = [&](int buf) {
@@ -305,28 +311,29 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
     bf16x8_t p_frag[RB][2];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      uint32_t dead = 0;  // bit per score of this lane
+      float(&v)[16] = reinterpret_cast<float(&)[16]>(s4[rb]);  // key kv0 + (e / 8) * 32 + lg * 8 + e % 8
+      // softcap * tanh(score * scale / softcap) in log2 units
+      if constexpr (CAP) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          v[e] = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v[e] * c[rb]));
+      }
+      // a masked score's weight is 2^-inf or 1 / (1 + 2^inf): no further select
       if (masked) {
-        const int qpos = ctx - n + row0 + rb * 16 + li;
+        const int first = kv0 + lg * 8;
+        const int last = min(ctx - n + row0 + rb * 16 + li, ctx - 1) - first, low = key_lo[rb] - first;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const int key = kv0 + (e >> 3) * 32 + lg * 8 + (e & 7);
-          if (key > qpos || key >= ctx || key < key_lo[rb]) {
-            dead |= 1u << e;
-            s4[rb][e >> 3][(e >> 2) & 1][e & 3] = -INFINITY;
-          }
+          const int k = (e >> 3) * 32 + (e & 7);
+          if (k > last || (EXTRA && k < low)) v[e] = -INFINITY;
         }
       }
-      float mx = -INFINITY;
       if constexpr (!SIG) {
+        float mx = v[0];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s4[rb][e >> 3][(e >> 2) & 1][e & 3]);
+        for (int e = 1; e < 16; ++e) mx = fmaxf(mx, v[e]);
         mx = max_over_groups(mx);
-        if constexpr (CAP)
-          mx = mx == -INFINITY ? mx : cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
-                                                              1.f + __builtin_amdgcn_exp2f(mx * c[rb] * (2.f * LOG2E))));
-        else
-          mx = mx == -INFINITY ? mx : mx * c[rb];
+        if constexpr (!CAP) mx *= c[rb];
         if (__any(mx > m[rb])) {
           const float m_new = fmaxf(m[rb], mx);
           const float alpha = m[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[rb] - m_new);
@@ -343,26 +350,11 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
       float sum = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const float v = s4[rb][e >> 3][(e >> 2) & 1][e & 3];
-        float w;
-        if constexpr (CAP) {
-          // softcap * tanh(v * scale / softcap) in log2 units
-          const float b = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(
-                                                  1.f + __builtin_amdgcn_exp2f(v * c[rb] * (2.f * LOG2E))));
-          if constexpr (SIG)
-            w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(b + bias * LOG2E)));
-          else
-            w = __builtin_amdgcn_exp2f(b - mm);
-        } else if constexpr (SIG) {
-          w = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * c[rb] + bias * LOG2E)));
-        } else {
-          w = __builtin_amdgcn_exp2f(__builtin_fmaf(v, c[rb], -mm));
-        }
-        p[e] = w;
-      }
-      if (masked) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) p[e] = (dead >> e) & 1 ? 0.f : p[e];
+        if constexpr (SIG)
+          p[e] = __builtin_amdgcn_rcpf(
+              1.f + __builtin_amdgcn_exp2f(CAP ? -v[e] - bias : __builtin_fmaf(v[e], -c[rb], -bias)));
+        else
+          p[e] = __builtin_amdgcn_exp2f(CAP ? v[e] - mm : __builtin_fmaf(v[e], c[rb], -mm));
       }
       if constexpr (!SIG) {
 #pragma unroll
