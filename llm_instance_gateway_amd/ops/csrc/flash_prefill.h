@@ -70,6 +70,20 @@ struct Args {
   float softcap;
 };
 
+// Where the 16-byte chunks of key t's row, and of entry d's row of keys, lie: chunk c
+// at c ^ swizzle.  The reads of 16 lanes (0-3, 12-15 and of the next 16 4-11, or the
+// others) then meet all 64 banks, and so do the writes of a key's row; those of V's
+// entries, rows 8 apart, meet half of them.  Heads of 64 have half the chunks in a
+// row of keys, and too few entries for the writes and reads of V to agree.
+template <int D>
+LIG_DEVICE int key_swizzle(int t) {
+  return D == 128 ? (t & 3) | ((t >> 1) & 12) : (t & 3) | ((t >> 1) & 4);
+}
+template <int D>
+LIG_DEVICE int entry_swizzle(int d) {
+  return (d ^ (D == 128 ? d >> 4 : d >> 3)) & 7;
+}
+
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
 // sigmoid(score + bias) weights.  EXTRA: temperature, gate, sink, chunk and
 // window are looked at (the plain causal kernel leaves them out).
@@ -224,14 +238,14 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 #pragma unroll
     for (int i = 0; i < TPT; ++i) {
       const int t = st * TPT + i;
-      const int f = (t & 3) | ((t >> 1) & 4);
+      const int f = key_swizzle<D>(t);
       *reinterpret_cast<u32x4*>(&sm.K[buf][t * D + ((ch ^ f) * 8)]) = kreg[i];
     }
     // entry e of key i -> row ch*8+e, key i; eight 16-byte units of 8 keys per row
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int d = ch * 8 + e;
-      const int unit = ((st * TPT) >> 3) ^ ((d ^ (d >> 3)) & 7);
+      const int unit = ((st * TPT) >> 3) ^ entry_swizzle<D>(d);
       uint16_t* p = &sm.VT[buf][d * KT + unit * 8 + ((st * TPT) & 7)];
       const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
       if constexpr (TPT == 4) {
@@ -288,7 +302,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
           const int t = t2 * 32 + key_row + x * 4;
-          const int f = (t & 3) | ((t >> 1) & 4);
+          const int f = key_swizzle<D>(t);
           bf16x8_t kf[KS];
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks)
@@ -376,7 +390,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int d = db * 16 + li;
-        const int unit = (t2 * 4 + lg) ^ ((d ^ (d >> 3)) & 7);
+        const int unit = (t2 * 4 + lg) ^ entry_swizzle<D>(d);
         const bf16x8_t vf =
             __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(&sm.VT[buf][d * KT + unit * 8]));
 #pragma unroll
