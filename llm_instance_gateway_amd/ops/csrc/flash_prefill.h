@@ -15,11 +15,11 @@
 //     which a lane's scores ARE the operand of O^T += V^T P^T (rows g*4+i of
 //     two tiles hold keys g*8+i and g*8+4+i), so the weights never leave the
 //     registers, and row statistics are one scalar per lane for both products;
-//   * V is transposed while it is staged (byte permutes in registers), both
-//     tiles are XOR-swizzled so that the 16-byte operand reads of 8
-//     consecutive lanes cover all LDS banks;
-//   * the next 64 keys are loaded into registers while the current ones are
-//     used, LDS is double-buffered: one barrier per 64 keys;
+//   * heads of 128: rows go from memory straight into LDS (load_to_lds), the next 64
+//     keys while the current ones are used, V transposed by the reads; chunks are
+//     XOR-swizzled by key through the choice of what a lane fetches, so that no read
+//     meets a bank twice.  Heads of 64 and odd block sizes: through registers, V
+//     transposed by byte permutes.  LDS is double-buffered: one barrier per 64 keys;
 //   * the accumulators are only rescaled when a row's maximum grew, and masks
 //     are only evaluated on tiles that cross a row's visible range.
 // Measured, 32 query and 8 key/value heads of 128, before -> after: 4096 rows
@@ -27,6 +27,10 @@
 // between the products of an engine step); 20 prompts of 200 130 -> 37 us; one of
 // 202 20.6 -> 8.9 us; 8 of 1000 with a window of 512 571 -> 110 us, with a soft cap
 // 578 -> 133, with sigmoid weights 566 -> 103.
+// What then bound it were vector instructions (64 % of the cycles, and LDS 53 %, half
+// of that conflicts).  Without selects for masked keys, with pairs rounded at once,
+// rows by DMA and their block's row number worked out once per group of keys: 4000
+// rows on 4000 keys 560 -> 441 us, 8 of 1000 with the window and a cap 120 -> 96.
 // Four heads per workgroup and 64 rows per wave (all 512 registers, one wave
 // per SIMD) was slower everywhere: 781 us in the first of these.
 #pragma once
@@ -70,18 +74,19 @@ struct Args {
   float softcap;
 };
 
-// Where the 16-byte chunks of key t's row, and of entry d's row of keys, lie: chunk c
-// at c ^ swizzle.  The reads of 16 lanes (0-3, 12-15 and of the next 16 4-11, or the
-// others) then meet all 64 banks, and so do the writes of a key's row; those of V's
-// entries, rows 8 apart, meet half of them.  Heads of 64 have half the chunks in a
-// row of keys, and too few entries for the writes and reads of V to agree.
+// Where the 16-byte chunks of key t's row, and (not DMA) of entry d's row of keys,
+// lie: chunk c at c ^ swizzle.  The reads of 16 lanes (0-3, 12-15 and of the next 16
+// 4-11, or the others) then meet all 64 banks, as do V's transposing reads of 8 keys,
+// whose pairs of chunks are spread by 2 ((t & 3) | (t / 8 % 2) * 4).
 template <int D>
 LIG_DEVICE int key_swizzle(int t) {
   return D == 128 ? (t & 3) | ((t >> 1) & 12) : (t & 3) | ((t >> 1) & 4);
 }
-template <int D>
-LIG_DEVICE int entry_swizzle(int d) {
-  return (d ^ (D == 128 ? d >> 4 : d >> 3)) & 7;
+LIG_DEVICE int entry_swizzle(int d) { return (d ^ (d >> 3)) & 7; }
+
+LIG_DEVICE u32x2 transposed(const uint16_t* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
 }
 
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
@@ -95,11 +100,12 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   constexpr int DB = D / 16;   // blocks of 16 output entries
   constexpr int CH = D / 8;    // 16-byte chunks of a row
   constexpr int TPT = KT * CH / 256;  // keys a thread stages: 4 (D = 128) or 2
+  constexpr bool DMA = PB && D == 128;  // rows go straight into LDS, 4 to an instruction
   static_assert(16 * RB * (4 / GH) == TQ, "a workgroup serves one query tile of each of its heads");
 
   struct Shared {
     uint16_t K[2][KT * D];
-    uint16_t VT[2][D * KT];
+    uint16_t VT[2][D * KT];  // DMA: V as it lies in memory, [KT][D]
   };
   __shared__ Shared sm;
 
@@ -245,7 +251,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int d = ch * 8 + e;
-      const int unit = ((st * TPT) >> 3) ^ entry_swizzle<D>(d);
+      const int unit = ((st * TPT) >> 3) ^ entry_swizzle(d);
       uint16_t* p = &sm.VT[buf][d * KT + unit * 8 + ((st * TPT) & 7)];
       const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
       if constexpr (TPT == 4) {
@@ -259,11 +265,53 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
     }
   };
 
-  int blk_next = block_of(kv_begin);
-  fetch(kv_begin, blk_next);
-  blk_next = block_of(kv_begin + KT);
-  stage(0);
-  __syncthreads();
+  // ---- DMA: a wave brings keys wave * 16 .. +16, four to an instruction (a block holds
+  // at least 4), whose 16 lanes a row choose the chunk that belongs to their place.
+  // Lane j knows the block of the tile's keys 4 j .. +4, read one tile ahead.  Tiles
+  // with all 64 keys visible take one offset per pair of fetches, the others clamp.
+  const uint32_t lds_k = lds_address(sm.K), lds_v = lds_address(sm.VT);
+  const int place = lane & 15, quarter = lane >> 4;  // chunk's place; row of the four
+  uint32_t k_off[2], v_off[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    k_off[j] = ((place ^ (quarter | ((wave * 2 + j) & 3) << 2)) << 4) + quarter * (D * 2);
+    v_off[j] = ((place ^ ((quarter | j << 2) << 1)) << 4) + quarter * (uint32_t)a.v_row * 2;
+  }
+  auto blocks_of = [&](int kv0) { return bt[visible(kv0 + (lane & 15) * 4) >> a.block_shift]; };
+  auto fetch_dma = [&](int kv0, int blks, int buf) {
+    // offsets have no sign: where keys are clamped they count from the block's first row
+    const bool whole = kv0 + KT <= kv_end && (!EXTRA || kv0 >= first_key);
+    // cache rows of 256 bytes and more: their number has 32 bits
+    const uint32_t first = (uint32_t)blks * (uint32_t)block_rows + (uint32_t)kv_head_rows +
+                           (whole ? (kv0 + (lane & 15) * 4) & (a.block_size - 1) : 0);
+    auto bring = [&](int j, uint32_t ko, uint32_t vo) __attribute__((always_inline)) {
+      const uint32_t row = __builtin_amdgcn_readlane(first, wave * 4 + j);
+      const uint32_t to = (buf * KT + wave * 16 + j * 4) * D * 2;
+      load_to_lds(a.k_cache + (size_t)row * D, ko, lds_k + to);
+      load_to_lds(a.v_cache + (size_t)row * (uint32_t)a.v_row, vo, lds_v + to);
+    };
+    if (whole) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bring(j, k_off[j >> 1], v_off[j >> 1]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int row = visible(kv0 + wave * 16 + j * 4 + quarter) & (a.block_size - 1), d = row - quarter;
+        bring(j, k_off[j >> 1] + d * (D * 2), v_off[j >> 1] + d * a.v_row * 2);
+      }
+    }
+  };
+
+  int blk_next = DMA ? blocks_of(kv_begin) : block_of(kv_begin);
+  if constexpr (DMA) {
+    fetch_dma(kv_begin, blk_next, 0);
+    blk_next = blocks_of(kv_begin + KT);
+  } else {
+    fetch(kv_begin, blk_next);
+    blk_next = block_of(kv_begin + KT);
+    stage(0);
+    __syncthreads();
+  }
 
   // A wave behind the portion's last row only stages, tile for tile with the
   // others, in a loop of its own: a branch in the one below costs full tiles 2 to
@@ -273,12 +321,18 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   // 70.8 and 24.6, 14.4, 56.7: with heads of 64 it fits more workgroups on a CU.
   if (row0 >= n) {
     for (int kv0 = kv_begin, buf = 1; kv0 < kv_end; kv0 += KT, buf ^= 1) {
+      if constexpr (DMA) loads_landed<0>();
       if (kv0 + KT < kv_end) {
-        fetch(kv0 + KT, blk_next);
-        blk_next = block_of(kv0 + 2 * KT);
-        stage(buf);
+        if constexpr (DMA) {
+          fetch_dma(kv0 + KT, blk_next, buf);
+          blk_next = blocks_of(kv0 + 2 * KT);
+        } else {
+          fetch(kv0 + KT, blk_next);
+          blk_next = block_of(kv0 + 2 * KT);
+          stage(buf);
+        }
       }
-      __syncthreads();
+      if constexpr (!DMA) __syncthreads();
     }
     return;
   }
@@ -286,9 +340,15 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   int buf = 0;
   for (int kv0 = kv_begin; kv0 < kv_end; kv0 += KT, buf ^= 1) {
     const bool more = kv0 + KT < kv_end;
+    if constexpr (DMA) loads_landed<0>();  // this tile is in LDS, and the other buffer is free
     if (more) {
-      fetch(kv0 + KT, blk_next);
-      blk_next = block_of(kv0 + 2 * KT);
+      if constexpr (DMA) {
+        fetch_dma(kv0 + KT, blk_next, buf ^ 1);
+        blk_next = blocks_of(kv0 + 2 * KT);
+      } else {
+        fetch(kv0 + KT, blk_next);
+        blk_next = block_of(kv0 + 2 * KT);
+      }
     }
 
     // ---- S^T = K Q^T --------------------------------------------------------------
@@ -389,18 +449,28 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
     for (int t2 = 0; t2 < 2; ++t2) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const int d = db * 16 + li;
-        const int unit = (t2 * 4 + lg) ^ entry_swizzle<D>(d);
-        const bf16x8_t vf =
-            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(&sm.VT[buf][d * KT + unit * 8]));
+        bf16x8_t vf;
+        if constexpr (DMA) {
+          // lane li of 16 reads 4 entries of key li / 4 and receives entry li of keys 0..3
+          const int key = t2 * 32 + lg * 8 + (li >> 2), w = (li >> 2) | (lg & 1) << 2;
+          const uint16_t* v0 = &sm.VT[buf][key * D + (db ^ w) * 16 + (li & 3) * 4];
+          const u32x2 b0 = transposed(v0), b1 = transposed(v0 + 4 * D);
+          vf = __builtin_bit_cast(bf16x8_t, (u32x4{b0[0], b0[1], b1[0], b1[1]}));
+        } else {
+          const int d = db * 16 + li;
+          const int unit = (t2 * 4 + lg) ^ entry_swizzle(d);
+          vf = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(&sm.VT[buf][d * KT + unit * 8]));
+        }
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
           acc[rb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_frag[rb][t2], acc[rb][db], 0, 0, 0);
       }
     }
 
-    if (more) stage(buf ^ 1);
-    __syncthreads();
+    if constexpr (!DMA) {
+      if (more) stage(buf ^ 1);
+      __syncthreads();
+    }
   }
 
   // ---- normalise, gate, store: this lane holds entries db*16 + lg*4 + i of its row ----
