@@ -41,6 +41,18 @@ struct Tile {
   bool valid;
 };
 
+// Workgroups are dealt to the 8 XCDs in turn.  (tile, strip) of this one such that an
+// XCD has neighbouring tiles of one strip: tiles of an adapter lie together, and its
+// weights come into one L2 instead of all.
+struct Place {
+  int tile, strip;
+};
+LIG_DEVICE Place place_of() {
+  const unsigned at = blockIdx.x + gridDim.x * blockIdx.y, total = gridDim.x * gridDim.y, xcd = at & 7;
+  const unsigned p = xcd * (total >> 3) + min(xcd, total & 7) + (at >> 3);
+  return {(int)(p % gridDim.x), (int)(p / gridDim.x)};
+}
+
 // without a list: rows in their order, none with an adapter
 LIG_DEVICE Tile tile_of(const int* toks, const int* len, const int* slot, int tile, int li, int rows = 0) {
   Tile t;
@@ -228,7 +240,7 @@ __global__ __launch_bounds__(512) void lora_rms_norm_kernel(
   constexpr int hidden = NG * 256;
   __shared__ float ss_s[8][16];
   __shared__ __align__(16) float red[8][16][R];
-  const int tile = blockIdx.x;
+  const int tile = place_of().tile;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Tile t = tile_of(toks, len, slot, tile, li);
@@ -262,7 +274,7 @@ LIG_DEVICE void norm_strip(const Tile& t, uint16_t* __restrict__ out, const uint
                            const int tiles_out, float* sums,
                            float* smem, int wave, int li, int lg) {
   constexpr int NB = NORM_STRIP / 128;
-  const int c_first = blockIdx.y * NORM_STRIP + wave * 32;
+  const int c_first = place_of().strip * NORM_STRIP + wave * 32;
   const size_t base = (size_t)t.row * hidden + lg * 8;
   u16x8 xr[NB], rr[NB], wr[NB], ar[NB];
   BOperand br[NB];
@@ -299,7 +311,7 @@ LIG_DEVICE void norm_strip(const Tile& t, uint16_t* __restrict__ out, const uint
     if (lg == 0) smem[wave * 16 + li] = ss;
     __syncthreads();
     if (threadIdx.x < 16)
-      sums[blockIdx.y * 16 + threadIdx.x] =
+      sums[place_of().strip * 16 + threadIdx.x] =
           smem[threadIdx.x] + smem[16 + threadIdx.x] + smem[32 + threadIdx.x] + smem[48 + threadIdx.x];
   } else {
     const float inv = rsqrtf(total / hidden + eps);
@@ -324,7 +336,7 @@ LIG_DEVICE void norm_strip(const Tile& t, uint16_t* __restrict__ out, const uint
     }
     if constexpr (TO_U) {
       float(*red)[16][R] = reinterpret_cast<float(*)[16][R]>(smem);
-      store_u<4>(u_out + (size_t)blockIdx.y * tiles_out * 16 * R, acc, red, wave, li, lg);
+      store_u<4>(u_out + (size_t)place_of().strip * tiles_out * 16 * R, acc, red, wave, li, lg);
     }
   }
 }
@@ -337,7 +349,7 @@ __global__ __launch_bounds__(256) void lora_norm_strip_kernel(
     const uint16_t* __restrict__ b_stack, const uint16_t* __restrict__ a_stack, float* u_out, const int tiles_out,
     float* sums) {
   __shared__ __align__(16) float smem[4 * 16 * R];
-  const int tile = blockIdx.x;
+  const int tile = place_of().tile;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Tile t = tile_of(toks, len, slot, tile, li);
@@ -394,7 +406,7 @@ LIG_DEVICE void open_strip(const Tile& t, uint16_t* __restrict__ out, const uint
                            const uint16_t* __restrict__ a, float* u_out, const int tiles_out, float* sums, float* smem,
                            int wave, int li, int lg) {
   constexpr int NB = NORM_STRIP / 128;
-  const int c_first = blockIdx.y * NORM_STRIP + wave * 32;
+  const int c_first = place_of().strip * NORM_STRIP + wave * 32;
   const size_t base = (size_t)t.row * hidden + lg * 8;
   u16x8 xr[NB], rr[NB], wr[NB], ar[NB];
   BOperand br[NB];
@@ -447,11 +459,11 @@ LIG_DEVICE void open_strip(const Tile& t, uint16_t* __restrict__ out, const uint
   if (lg == 0) smem[wave * 16 + li] = ss;
   __syncthreads();
   if (threadIdx.x < 16)
-    sums[blockIdx.y * 16 + threadIdx.x] =
+    sums[place_of().strip * 16 + threadIdx.x] =
         smem[threadIdx.x] + smem[16 + threadIdx.x] + smem[32 + threadIdx.x] + smem[48 + threadIdx.x];
   if constexpr (TO_U) {
     __syncthreads();
-    store_u<4>(u_out + (size_t)blockIdx.y * tiles_out * 16 * R, acc, reinterpret_cast<float(*)[16][R]>(smem), wave, li, lg);
+    store_u<4>(u_out + (size_t)place_of().strip * tiles_out * 16 * R, acc, reinterpret_cast<float(*)[16][R]>(smem), wave, li, lg);
   }
 }
 
@@ -463,7 +475,7 @@ __global__ __launch_bounds__(256) void lora_norm_open_kernel(
     const int parts, const int tiles, const uint16_t* __restrict__ b_stack, const uint16_t* __restrict__ a_stack,
     float* u_out, const int tiles_out, float* sums, const int rows) {
   __shared__ __align__(16) float smem[4 * 16 * R];
-  const int tile = blockIdx.x;
+  const int tile = place_of().tile;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Tile t = tile_of(toks, len, slot, tile, li, rows);
@@ -537,7 +549,7 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
       gv *= factor;
       uv *= factor;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = gv[j] / (1.0f + __expf(-gv[j])) * uv[j];
+      for (int j = 0; j < 8; ++j) r[j] = gv[j] * __builtin_amdgcn_rcpf(1.0f + __expf(-gv[j])) * uv[j];
       const u16x8 rb = f32x8_to_bf16x8(r);
       if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
       if constexpr (LORA) acc = shrink(ar[i], rb, acc);
@@ -553,7 +565,7 @@ __global__ __launch_bounds__(256) void lora_silu_kernel(
     const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm,
     const int rows) {
   __shared__ __align__(16) float red[4][16][R];
-  const int tile = blockIdx.x, strip = blockIdx.y;
+  const int tile = place_of().tile, strip = place_of().strip;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Tile t = tile_of(toks, len, slot, tile, li, rows);
@@ -580,14 +592,14 @@ __global__ __launch_bounds__(256) void lora_shrink_kernel(
     const int tiles_out) {
   constexpr int NB = SHRINK_STRIP / 128;
   __shared__ __align__(16) float red[4][16][R];
-  const int tile = blockIdx.x;
+  const int tile = place_of().tile;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Tile t = tile_of(toks, len, slot, tile, li);
   if (t.n == 0 || t.slot < 0) return;
   const uint16_t* a = a_stack + (size_t)t.slot * R * width;
   const uint16_t* row = x + (size_t)t.row * width + lg * 8;
-  const int c_first = blockIdx.y * SHRINK_STRIP + wave * 32;
+  const int c_first = place_of().strip * SHRINK_STRIP + wave * 32;
   u16x8 xr[NB], ar[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
@@ -599,7 +611,7 @@ __global__ __launch_bounds__(256) void lora_shrink_kernel(
 #pragma unroll
   for (int i = 0; i < NB; ++i)
     if (c_first + i * 128 < width) acc = shrink(ar[i], xr[i], acc);
-  store_u<4>(u_out + ((size_t)blockIdx.y * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+  store_u<4>(u_out + ((size_t)place_of().strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
 }
 
 // qkv_rope.hip's pass with B u added to the projection on the way in.  PARTS: the
@@ -619,13 +631,14 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
   __shared__ __align__(16) float smem[16 * R];
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int parts = head_dim / 64;  // of 32 rotation pairs
-  const int wid = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = place_of().tile;
+  const int wid = place_of().strip * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int heads = num_q_heads + 2 * num_kv_heads;
   const int h0 = (wid / parts) * QR_HEADS;
-  const Tile t = tile_of(toks, len, slot, blockIdx.x, li, rows);
+  const Tile t = tile_of(toks, len, slot, tile, li, rows);
   if (t.n == 0) return;
   bf16x8_t u = {};
-  if (t.slot >= 0) u = u_of(u_in + (size_t)blockIdx.x * 16 * R, u_parts, tiles, smem, li, lg, t.valid);
+  if (t.slot >= 0) u = u_of(u_in + (size_t)tile * 16 * R, u_parts, tiles, smem, li, lg, t.valid);
   if (h0 >= heads) return;  // whole waves: no lane may miss the matrix instructions
   const int half = head_dim / 2;
   const int p0 = (wid % parts) * 32, c = p0 + lg * 8;
@@ -682,7 +695,7 @@ __global__ __launch_bounds__(256) void lora_qkv_rope_cache_kernel(
       v[i][1] += expand(br[i][1], u);
     }
   }
-  const float factor = factor_of(norm, blockIdx.x, li);
+  const float factor = factor_of(norm, tile, li);
 #pragma unroll
   for (int i = 0; i < QR_HEADS; ++i) {
     v[i][0] *= factor;
