@@ -31,6 +31,20 @@ def pack_rows(rows: Seq[List[int]], out: np.ndarray) -> None:
         out[i, : len(r)] = r
 
 
+def pack_decodes(seqs: list, block_size: int, ids: np.ndarray, positions: np.ndarray, tables: np.ndarray) -> None:
+    """The token that each sequence processes at num_computed_tokens, that
+    position, and its cache blocks in a row of `tables` (zeros behind them)."""
+    ext = ops._load_ext()
+    if ext is not None:
+        ext.pack_decodes(seqs, block_size, ids, positions, tables)
+        return
+    positions[:] = [q.num_computed_tokens for q in seqs]
+    if any(p // block_size >= len(q.block_table) for q, p in zip(seqs, positions.tolist())):
+        raise IndexError("a sequence has fewer cache blocks than tokens")
+    ids[:] = [q.tokens(p, p + 1)[0] for q, p in zip(seqs, positions.tolist())]
+    pack_rows([q.block_table for q in seqs], tables)
+
+
 def table_rows(rows: Seq[List[int]]) -> np.ndarray:
     """int32 [len(rows), longest], zero past a row's end."""
     out = np.zeros((len(rows), max(len(r) for r in rows)), dtype=np.int32)

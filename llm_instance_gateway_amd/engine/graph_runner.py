@@ -28,7 +28,7 @@ from typing import Dict, List, Optional
 import numpy as np
 import torch
 
-from .batch_arrays import device_view, lay_out, pack_rows
+from .batch_arrays import device_view, lay_out, pack_decodes
 from .metadata import BatchMeta
 
 log = logging.getLogger(__name__)
@@ -276,15 +276,10 @@ class DecodeGraphRunner:
         v = self._views(B)
         x = v.host
         seqs = [ss.seq for ss in decodes]
-        pos = [q.num_computed_tokens for q in seqs]
         x.ids[n:] = 0
-        pack_rows([q.tokens(p, p + 1) for q, p in zip(seqs, pos)], x.ids[:n])
-        x.pos[:n] = pos
         x.pos[n:] = 0
         x.block_tables[:] = 0  # another bucket's arrays lay here
-        pack_rows([q.block_table for q in seqs], x.block_tables[:n])
-        if any(p // bs >= len(q.block_table) for q, p in zip(seqs, pos)):
-            raise IndexError("a sequence has fewer cache blocks than tokens")
+        pack_decodes(seqs, bs, x.ids[:n], x.pos[:n], x.block_tables[:n])
         x.block_tables[n:, 0] = self.scratch_block
         at = x.pos // bs
         x.slot_mapping[:] = x.block_tables[np.arange(B), at].astype(np.int64) * bs + x.pos - at * bs

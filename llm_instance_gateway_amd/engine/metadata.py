@@ -83,6 +83,9 @@ class BatchMeta:
     seg_ctx: Optional[torch.Tensor] = None    # [S] int32 tokens of the sequence after this step
     max_seg_len: int = 0                      # host-side max of seg_len
 
+    # rows of the batch whose logits the step hands out (padding repeats the first)
+    logit_rows: Optional[torch.Tensor] = None  # int64
+
     @property
     def num_tokens(self) -> int:
         return self.num_prefill_tokens + self.num_decode_tokens

@@ -16,7 +16,7 @@ import torch
 
 from ..models.config import ModelConfig
 from ..utils.tunableop import eager_tuned
-from .batch_arrays import pack_rows, table_rows, upload
+from .batch_arrays import pack_decodes, pack_rows, table_rows, upload
 from .config import EngineConfig
 from .metadata import BatchMeta
 from ..utils.tracing import gpu_range
@@ -170,7 +170,9 @@ class ModelRunner:
         self._decode_stream = None
 
     # -- batch construction ---------------------------------------------------
-    def _build_batch(self, out):
+    def _build_batch(self, out, replay: bool = False):
+        """`replay`: meta.logit_rows are those the sequences ask for, instead of
+        those to sample from."""
         scheduled = out.scheduled if isinstance(out, SchedulerOutput) else out
         prefills: List[ScheduledSeq] = []
         decodes: List[ScheduledSeq] = []
@@ -190,12 +192,24 @@ class ModelRunner:
 
         # the sequences whose last known token this step processes: every
         # decode, and prompts with their final portion
-        sample_seqs: List[Sequence] = []
-        sample_idx: List[int] = []
-        for i, q in enumerate(seqs):
-            if i >= n_pre or ends[i] == q.total_len:
-                sample_seqs.append(q)
-                sample_idx.append(rows[i + 1] - 1)
+        sampled = [i for i in range(n_pre) if ends[i] == seqs[i].total_len]
+        sample_seqs: List[Sequence] = [seqs[i] for i in sampled] + seqs[n_pre:]
+        sample_idx: List[int] = [rows[i + 1] - 1 for i in sampled] + list(range(num_prefill_tokens, T))
+        if replay:
+            logit_rows = []
+            for ss, base in zip(ordered, rows):
+                for off in ss.logit_offsets or ():
+                    if not 0 <= off < ss.num_tokens:
+                        raise ValueError("wanted logit offset outside the step's tokens")
+                    logit_rows.append(base + off)
+        else:
+            # Bucket the logits GEMM's M (ROADMAP r02 #4): sample counts
+            # vary 1..max_num_seqs per mixed step — pad the gather index
+            # to a multiple of 64 (repeat row 0) so the 128k-vocab GEMM
+            # sees a handful of stable shapes; pad rows sliced off.
+            logit_rows = list(sample_idx)
+            if sample_idx and self.device.type == "cuda" and self.config.pad_batch_multiple:
+                logit_rows += [sample_idx[0]] * (-len(sample_idx) % 64)
 
         # GEMM M-bucketing: pad the flat batch tail so every projection GEMM
         # sees M % pad_batch_multiple == 0 (few stable shapes -> hipBLASLt
@@ -215,15 +229,20 @@ class ModelRunner:
         input_ids = np.zeros(T + num_pad_tokens, dtype=np.int64)
         positions = np.zeros(T + num_pad_tokens, dtype=np.int64)
         slots = np.full(T + num_pad_tokens, self.config.num_kv_blocks * bs, dtype=np.int64)
-        pack_rows([q.tokens(q.num_computed_tokens, e) for q, e in zip(seqs, ends)], input_ids[:T])
         tok_seq = np.repeat(np.arange(S, dtype=np.int32), length)
-        positions[:T] = np.arange(T) - (first[:-1] - start)[tok_seq]
         p_bts = [q.block_table for q in seqs[:n_pre]]
         d_bts = [q.block_table for q in seqs[n_pre:]]
-        if any(len(q.block_table) * bs < c for q, c in zip(seqs, ends)):
-            raise IndexError("a sequence has fewer cache blocks than tokens")
-        p_tab = table_rows(p_bts) if p_bts else None
-        d_tab = table_rows(d_bts) if d_bts else None
+        p_tab = d_tab = None
+        if p_bts:
+            if any(len(t) * bs < c for t, c in zip(p_bts, ends)):
+                raise IndexError("a sequence has fewer cache blocks than tokens")
+            r = slice(0, num_prefill_tokens)
+            pack_rows([q.tokens(q.num_computed_tokens, e) for q, e in zip(seqs[:n_pre], ends)], input_ids[r])
+            positions[r] = np.arange(num_prefill_tokens) - (first[:-1] - start)[tok_seq[r]]
+            p_tab = table_rows(p_bts)
+        if d_bts:
+            d_tab = np.zeros((len(d_bts), max(len(t) for t in d_bts)), dtype=np.int32)
+            pack_decodes(seqs[n_pre:], bs, input_ids[num_prefill_tokens:T], positions[num_prefill_tokens:T], d_tab)
         for tab, lo, hi in ((p_tab, 0, n_pre), (d_tab, n_pre, S)):
             if tab is not None:
                 r = slice(rows[lo], rows[hi])
@@ -304,9 +323,6 @@ class ModelRunner:
                 put("lora_tile_len", np.minimum(64, length[of] - off))
                 put("lora_tile_slot", seq_slot[of])
 
-        # first flat row of every scheduled sequence (replay reads logits at
-        # offsets from it)
-        self._row_start = {q.seq_id: r for q, r in zip(seqs, rows)}
         if getattr(self.model, "needs_seq_tables", False):
             # Per-token / per-sequence addressing for general-size attention
             # and recurrent layers: one block-table row and one segment per
@@ -320,8 +336,10 @@ class ModelRunner:
             put("seg_ctx", ctx)
             meta.max_seg_len = int(length.max()) if S else 0
 
-        ids_t, pos_t, meta.slot_mapping, *tables = upload(
-            [input_ids, positions, slots] + [a for _, a in fields], dev)
+        # (the rows of the logits come along: an index made from a list later on
+        # would wait for everything before it)
+        ids_t, pos_t, meta.slot_mapping, meta.logit_rows, *tables = upload(
+            [input_ids, positions, slots, np.array(logit_rows, dtype=np.int64)] + [a for _, a in fields], dev)
         for (name, _), t in zip(fields, tables):
             setattr(meta, name, t)
         return ids_t, pos_t, meta, sample_seqs, sample_idx, ordered
@@ -349,22 +367,7 @@ class ModelRunner:
         sampled: Dict[int, int] = {}
         if sample_seqs:
             with gpu_range("sample"):
-                # Bucket the logits GEMM's M (ROADMAP r02 #4): sample counts
-                # vary 1..max_num_seqs per mixed step — pad the gather index
-                # to a multiple of 64 (repeat row 0) so the 128k-vocab GEMM
-                # sees a handful of stable shapes; pad rows sliced off.
-                M = len(sample_idx)
-                pad_m = 0
-                if self.device.type == "cuda" and self.config.pad_batch_multiple:
-                    pad_m = (-M) % 64
-                idx = torch.tensor(
-                    sample_idx + [sample_idx[0]] * pad_m,
-                    dtype=torch.int64,
-                    device=self.device,
-                )
-                logits = self.model.compute_logits(hidden, idx)
-                if pad_m:
-                    logits = logits[:M]
+                logits = self.model.compute_logits(hidden, meta.logit_rows)[: len(sample_seqs)]
                 tokens = sample_tokens(logits, sample_seqs)
             for seq, tok in zip(sample_seqs, tokens):
                 sampled[seq.seq_id] = tok
@@ -381,25 +384,14 @@ class ModelRunner:
         if out.is_empty:
             return {}
         with gpu_range("build_batch"):
-            ids, pos, meta, _, _, ordered = self._build_batch(out)
+            ids, pos, meta, _, _, ordered = self._build_batch(out, replay=True)
         with gpu_range("forward"), eager_tuned():
             hidden = self.model(ids, pos, self.kv_caches, meta)
-        rows: List[int] = []
-        for ss in ordered:
-            base = self._row_start[ss.seq.seq_id]
-            for off in ss.logit_offsets or []:
-                if not 0 <= off < ss.num_tokens:
-                    raise ValueError("wanted logit offset outside the step's tokens")
-                rows.append(base + off)
         res: Dict[int, torch.Tensor] = {}
-        if rows:
-            idx = torch.tensor(rows, dtype=torch.int64, device=self.device)
-            logits = self.model.compute_logits(hidden, idx)
-            at = 0
-            for ss in ordered:
-                n = len(ss.logit_offsets or [])
-                res[ss.seq.seq_id] = logits[at : at + n]
-                at += n
+        if len(meta.logit_rows):
+            logits = self.model.compute_logits(hidden, meta.logit_rows)
+            counts = [len(ss.logit_offsets or ()) for ss in ordered]
+            res = {ss.seq.seq_id: part for ss, part in zip(ordered, logits.split(counts))}
         for ss in ordered:
             ss.seq.num_computed_tokens += ss.num_tokens
         return res

@@ -745,6 +745,59 @@ static void pack_rows(py::sequence rows, py::array out) {
   else TORCH_CHECK(false, "int32 or int64");
 }
 
+// What sequences that each process their token at num_computed_tokens bring: that
+// token, its position, and their cache blocks in a row of `tables` (int32, zeros).
+static void pack_decodes(py::list seqs, int64_t block_size, py::array_t<int64_t> ids, py::array_t<int64_t> positions,
+                         py::array_t<int32_t> tables) {
+  const ssize_t n = py::len(seqs);
+  TORCH_CHECK(block_size > 0 && ids.ndim() == 1 && positions.ndim() == 1 && tables.ndim() == 2 && ids.shape(0) == n &&
+              positions.shape(0) == n && tables.shape(0) == n);
+  for (const py::array* a : {(py::array*)&ids, (py::array*)&positions, (py::array*)&tables})
+    TORCH_CHECK(a->flags() & py::array::c_style, "in row order");
+  static PyObject* names[4] = {PyUnicode_InternFromString("num_computed_tokens"), PyUnicode_InternFromString("block_table"),
+                               PyUnicode_InternFromString("prompt_token_ids"),
+                               PyUnicode_InternFromString("output_token_ids")};
+  auto get = [](PyObject* o, PyObject* name) {
+    PyObject* v = PyObject_GetAttr(o, name);
+    if (!v) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(v);
+  };
+  auto number = [](PyObject* e) {
+    const long long v = PyLong_Check(e) ? PyLong_AsLongLong(e) : py::reinterpret_borrow<py::object>(e).cast<long long>();
+    if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
+    return v;
+  };
+  auto fast = [](const py::object& o) {
+    PyObject* f = PySequence_Fast(o.ptr(), "a list of numbers");
+    if (!f) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(f);
+  };
+  int64_t *id = ids.mutable_data(), *at = positions.mutable_data();
+  int32_t* row = tables.mutable_data();
+  const ssize_t width = tables.shape(1);
+  for (ssize_t i = 0; i < n; ++i, row += width) {
+    PyObject* q = PyList_GET_ITEM(seqs.ptr(), i);
+    const long long p = number(get(q, names[0]).ptr());
+    const py::object blocks = fast(get(q, names[1])), prompt = fast(get(q, names[2]));
+    const ssize_t len = PySequence_Fast_GET_SIZE(blocks.ptr()), known = PySequence_Fast_GET_SIZE(prompt.ptr());
+    if (p < 0 || p / block_size >= len) throw py::index_error("a sequence has fewer cache blocks than tokens");
+    TORCH_CHECK(len <= width, "a row of ", len, " numbers is longer than its room");
+    for (ssize_t j = 0; j < len; ++j) {
+      const long long v = number(PySequence_Fast_GET_ITEM(blocks.ptr(), j));
+      TORCH_CHECK(v == (long long)(int32_t)v, v, " does not fit");
+      row[j] = (int32_t)v;
+    }
+    at[i] = p;
+    if (p < known) {
+      id[i] = number(PySequence_Fast_GET_ITEM(prompt.ptr(), p));
+    } else {
+      const py::object more = fast(get(q, names[3]));
+      if (p - known >= PySequence_Fast_GET_SIZE(more.ptr())) throw py::index_error("a sequence has no such token");
+      id[i] = number(PySequence_Fast_GET_ITEM(more.ptr(), p - known));
+    }
+  }
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "MI355X (gfx950) native kernels for llm_instance_gateway_amd";
   m.def("rms_norm", &rms_norm);
@@ -754,6 +807,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("argmax_rows", &argmax_rows);
+  m.def("pack_decodes", &pack_decodes);
   m.def("projection", &projection);
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);
