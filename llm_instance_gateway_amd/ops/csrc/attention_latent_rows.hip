@@ -136,13 +136,17 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   const int all_end = ctx - n + first_tok + 1;
   const int all_lo = window > 0 ? kv_end - window : 0;
 
-  // ---- fetching: chunk c of key t of a tile goes to LDS chunk t * CHP + (c ^ f(t)).
+  // ---- fetching: chunk c of key t of a tile goes to place (c % 8) ^ f(t) of the 8 that
+  // columns c / 8 * 64 on have there.
   // Keys past the end repeat the last one, keys before the first that some row
   // sees that one: their weight is zero, but what they hold would still meet it in
   // a product, and the blocks before may be gone.
+  // A fetch brings 64 columns (8 chunks) of 8 keys, 128 bytes a key side by side in
+  // LDS, so that a lane's offset is the same for all fetches of 8 keys (as whole rows
+  // the offsets took 27 slow multiplications a tile, as long as the products).
   // FULL: 8 keys, aligned, are one contiguous piece of a block; a wave takes
-  // KT / 32 such pieces of CHP / 8 fetches.  Lane j looks up the block of piece j
-  // of the tile after next.  Else every lane looks for its own key's block.
+  // KT / 32 such pieces.  Lane j looks up the block of piece j of the tile after
+  // next.  Else every lane looks for its own key's block.
   const uint32_t lds = lds_address(sm);
   const int CH = D / 8;
   constexpr int NP = CHP / 8;  // fetches per piece
@@ -155,6 +159,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     constexpr bool FIRST = decltype(first_tile)::value;
     int here = lane;
     if (KG == 1) asm volatile("" : "+v"(here));  // worked out anew for each tile: held for the loop, it would spill
+    const int row = here >> 3, place = here & 7;
     if constexpr (FULL) {
 #pragma unroll
       for (int w = 0; w < KG; ++w) {
@@ -163,26 +168,20 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
         const int blk = __builtin_amdgcn_readlane(blks, piece);
         const uint16_t* g = cache + ((size_t)blk * block_size + (t0 & (block_size - 1))) * D;
         const int last = kv_end - 1 - t0;
+        const int from = min(FIRST ? max(row, kv_seen - t0) : row, last);
+        const uint32_t off = __umul24(from, DKP * 2) + ((place ^ ((row & 3) | ((piece & 1) << 2))) << 4);
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-          const int p = i * 64 + here;
-          const int key = p / CHP;  // of the piece
-          const int c = (p % CHP) ^ ((key & 3) | ((piece & 1) << 2));
-          const int from = FIRST ? max(key, kv_seen - t0) : key;
-          load_to_lds(g, (min(from, last) * DKP + c * 8) * 2, lds + (buf * TILE + (piece * NP + i) * 512) * 2);
-        }
+        for (int i = 0; i < NP; ++i) load_to_lds(g + i * 64, off, lds + (buf * TILE + (piece * NP + i) * 512) * 2);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int base = (wave * NI + i) * 64;
-        const int p = base + here;
-        const int key = p / CHP;
-        const int c = (p % CHP) ^ ((key & 3) | ((key >> 1) & 4));
+        const int f = wave * NI + i, key = f / NP * 8 + row;
+        const int c = f % NP * 8 + (place ^ ((key & 3) | ((key >> 1) & 4)));
         const int off = min(FIRST ? max(kv0 + key, kv_seen) : kv0 + key, kv_end - 1) % block_size;
         const int blk = __shfl(blks, key, 64);
         if (c < CH)
-          load_to_lds(cache + ((size_t)blk * block_size + off) * D + c * 8, lds + (buf * TILE + base * 8) * 2);
+          load_to_lds(cache + ((size_t)blk * block_size + off) * D + c * 8, lds + (buf * TILE + f * 512) * 2);
       }
     }
   };
@@ -240,19 +239,19 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     // Operands are read from LDS in batches of 4, the next batch ahead of the
     // products of this one.
     // S^T = K Q^T: tile row li stands for key (li/4)*8 + li%4 (+4 in the second).
-    // The swizzle only touches a chunk number's low 3 bits, so two addresses and
-    // constants reach all of a row
+    // Two addresses and constants reach all of a row
     f32x4_t s4[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
     {
       const int key = ((li >> 2) << 3) | (li & 3);
       const int f = (key & 3) | ((key >> 1) & 4);  // the same for key + 4
-      const uint16_t* kp[2] = {tile + key * DKP + (lg ^ f) * 8, tile + key * DKP + ((4 + lg) ^ f) * 8};
+      const uint16_t* row = tile + (key >> 3) * 8 * DKP + (key & 7) * 64;
+      const uint16_t* kp[2] = {row + (lg ^ f) * 8, row + ((4 + lg) ^ f) * 8};
       bf16x8_t kf[2][4];
       auto load = [&](int b) {  // steps 2b and 2b+1 of both tiles
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           kf[b & 1][j] = __builtin_bit_cast(
-              bf16x8_t, *reinterpret_cast<const u32x4*>(kp[j >> 1] + (j & 1) * 4 * DKP + b * 64));
+              bf16x8_t, *reinterpret_cast<const u32x4*>(kp[j >> 1] + (j & 1) * 4 * 64 + b * 512));
       };
       load(0);
 #pragma unroll
@@ -271,16 +270,17 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     const int vf_swz = (vkey & 3) | ((vkey >> 1) & 4);  // the same for key + 4
     const uint16_t* vp[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) vp[j] = tile + vkey * DKP + ((j * 2 + ((li >> 1) & 1)) ^ vf_swz) * 8 + (li & 1) * 4;
+    for (int j = 0; j < 4; ++j)
+      vp[j] = tile + (vkey >> 3) * 8 * DKP + (vkey & 7) * 64 + ((j * 2 + ((li >> 1) & 1)) ^ vf_swz) * 8 + (li & 1) * 4;
     bf16x8_t vf[2][4];
     auto load_v = [&](int b) {  // entry blocks 4b .. 4b+3
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint16_t* v0 = vp[j] + b * 64;
+        const uint16_t* v0 = vp[j] + b * 512;
         const u32x2 b0 = __builtin_bit_cast(
             u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)v0));
         const u32x2 b1 = __builtin_bit_cast(
-            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + 4 * DKP)));
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + 4 * 64)));
         vf[b & 1][j] = __builtin_bit_cast(bf16x8_t, (u32x4{b0[0], b0[1], b1[0], b1[1]}));
       }
     };
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       l += p[2 * e] + p[2 * e + 1];
-      pw[e] = (uint32_t)f32_to_bf16(p[2 * e]) | ((uint32_t)f32_to_bf16(p[2 * e + 1]) << 16);
+      pw[e] = pack_bf16(p[2 * e], p[2 * e + 1]);
     }
     const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pw);
 
@@ -398,8 +398,8 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     const int d = db * 16 + lg * 4;
     if (!FULL && d >= Dv) continue;
     u32x2 w;
-    w[0] = (uint32_t)f32_to_bf16(acc[db][0] * f) | ((uint32_t)f32_to_bf16(acc[db][1] * f) << 16);
-    w[1] = (uint32_t)f32_to_bf16(acc[db][2] * f) | ((uint32_t)f32_to_bf16(acc[db][3] * f) << 16);
+    w[0] = pack_bf16(acc[db][0] * f, acc[db][1] * f);
+    w[1] = pack_bf16(acc[db][2] * f, acc[db][3] * f);
     *reinterpret_cast<u32x2*>(op + d) = w;
   }
 }
