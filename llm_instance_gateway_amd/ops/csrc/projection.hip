@@ -227,7 +227,8 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   X(192, 128, 4, 2, 1, 1, 3)  \
   X(224, 128, 2, 4, 1, 1, 3)  \
   X(128, 256, 2, 4, 1, 1, 3)  \
-  X(256, 96, 4, 2, 1, 1, 3)
+  X(256, 96, 4, 2, 1, 1, 3)   \
+  X(208, 256, 1, 8, 1, 1, 2)
 
 struct TileShape {
   int bm, bn, k_step;
