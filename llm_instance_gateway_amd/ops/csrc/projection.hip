@@ -228,7 +228,9 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   X(224, 128, 2, 4, 1, 1, 3)  \
   X(128, 256, 2, 4, 1, 1, 3)  \
   X(256, 96, 4, 2, 1, 1, 3)   \
-  X(208, 256, 1, 8, 1, 1, 2)
+  X(208, 256, 1, 8, 1, 1, 2)  \
+  X(192, 256, 2, 4, 1, 1, 2)  \
+  X(256, 256, 2, 4, 1, 1, 2)
 
 struct TileShape {
   int bm, bn, k_step;
@@ -278,10 +280,11 @@ extern "C" {
 // Whether these kernels are the ones to take: the library's large tiles are ahead
 // where they are enough for the chip (384 x 28672 x 4096: 101 us here, 80 there;
 // 786 x 6144 x 4096: 51 and 47), and behind where N needs a cut of K (786 x 4096 x
-// 14336: 100 and 118; 384: 57 and 77) or rows are few.
+// 14336: 100 and 118; 384: 57 and 77) or rows are few; and it is slower than its
+// large tiles could be on a vocabulary (384 x 128256 x 4096: 388 us here, 431 there).
 bool lig_projection_serves(long M, long N, long K) {
   if (M < 1 || M > 1024 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
-  return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64;
+  return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || (M <= 384 && N >= 65536);
 }
 
 // Tile and parts of K, as one number.  To launch it: y alone where K is in one part,

@@ -13,7 +13,8 @@ SIZES = [
     (1, 8, 64), (5, 24, 128), (16, 4096, 4096), (16, 4104, 14336), (17, 520, 192), (33, 4096, 4096), (32, 1288, 8192),
     (48, 6144, 4096), (63, 28672, 256), (65, 8200, 3584), (97, 4096, 4096), (96, 12288, 1024), (129, 6152, 4096),
     (160, 4096, 1088), (193, 4096, 14336), (202, 28680, 128), (225, 12288, 4096), (256, 22016, 512), (255, 6144, 4096),
-    (257, 1288, 8192), (384, 6144, 4096), (786, 4096, 14336), (1000, 4040, 4096), (1024, 16, 64), (130, 4096, 4096), (343, 6144, 8192), (241, 12296, 14336),
+    (257, 1288, 8192), (384, 6144, 4096), (786, 4096, 14336), (1000, 4040, 4096), (1024, 16, 64),
+    (130, 4096, 4096), (343, 6144, 8192), (241, 12296, 14336), (236, 28680, 1024), (384, 65544, 256),
 ]
 
 
