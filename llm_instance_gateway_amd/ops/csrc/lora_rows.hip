@@ -515,7 +515,7 @@ LIG_DEVICE float factor_of(const Factor& f, int tile, int li) {
 // a tile take strips of 1024 of the d columns.
 constexpr int SILU_STRIP = 1024;
 
-template <bool LORA>
+template <bool LORA, int W>
 LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d,
                              const int c_first, const bf16x8_t u, const uint16_t* __restrict__ b,
                              const uint16_t* __restrict__ a, const float factor, int li, int lg) {
@@ -523,12 +523,12 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
   const uint16_t* g = x + (size_t)t.row * 2 * d + lg * 8;
   uint16_t* o = out + (size_t)t.row * d + lg * 8;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int i0 = 0; i0 < SILU_STRIP / 128; i0 += NB) {
+  for (int i0 = 0; i0 < SILU_STRIP / (W * 32); i0 += NB) {
     u16x8 gr[NB], ur[NB], ar[NB];
     BOperand bg[NB], bu[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int c0 = min(c_first + (i0 + i) * 128, d - 32);  // groups past the end: the last one again, unused
+      const int c0 = min(c_first + (i0 + i) * (W * 32), d - 32);  // groups past the end: the last one again, unused
       gr[i] = load8(g + c0);
       ur[i] = load8(g + d + c0);
       if constexpr (LORA) {
@@ -539,7 +539,7 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int c0 = c_first + (i0 + i) * 128;
+      const int c0 = c_first + (i0 + i) * (W * 32);
       if (c0 >= d) break;
       f32x8 gv = bf16x8_to_f32x8(gr[i]), uv = bf16x8_to_f32x8(ur[i]), r;
       if constexpr (LORA) {
@@ -558,13 +558,16 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
   return acc;
 }
 
-__global__ __launch_bounds__(256) void lora_silu_kernel(
+// 8 waves take a strip in one pass each, 4 in two: 9 tiles 9.7 us (11.0 with 4), 13
+// 10.6 (12.0), 240 120 (108), where the chip is full either way.
+template <int W>
+__global__ __launch_bounds__(64 * W) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
     const int* __restrict__ len, const int* __restrict__ slot,
     const float* __restrict__ u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
     const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm,
     const int rows) {
-  __shared__ __align__(16) float red[4][16][R];
+  __shared__ __align__(16) float red[W][16][R];
   const int tile = place_of().tile, strip = place_of().strip;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -573,14 +576,14 @@ __global__ __launch_bounds__(256) void lora_silu_kernel(
   const int c_first = strip * SILU_STRIP + wave * 32;
   const float factor = factor_of(norm, tile, li);
   if (t.slot < 0) {
-    silu_rows<false>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, factor, li, lg);
+    silu_rows<false, W>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, factor, li, lg);
     return;
   }
   const f32x4_t acc =
-      silu_rows<true>(t, out, x, d, c_first,
+      silu_rows<true, W>(t, out, x, d, c_first,
                       u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid),
                       b_stack + (size_t)t.slot * 2 * d * R, a_stack + (size_t)t.slot * R * d, factor, li, lg);
-  store_u<4>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+  store_u<W>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
 }
 
 // u_out = A x, a part per strip of 512 columns
@@ -804,8 +807,13 @@ void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* to
                           const int* slot, int ntiles, const float* u_in, int parts, int tiles,
                           const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
                           const float* sums, int width, float eps, int rows, hipStream_t stream) {
-  hipLaunchKernelGGL(lora_silu_kernel, dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(256), 0, stream, out, x, d,
-                     toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out, Factor{sums, width, eps}, rows);
+#define LAUNCH_A(W)                                                                                                  \
+  hipLaunchKernelGGL((lora_silu_kernel<W>), dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(64 * W), 0, stream, \
+                     out, x, d, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out,             \
+                     Factor{sums, width, eps}, rows)
+  if (ntiles <= 64) LAUNCH_A(8);
+  else LAUNCH_A(4);
+#undef LAUNCH_A
 }
 
 int lig_lora_shrink_strip() { return SHRINK_STRIP; }

@@ -137,6 +137,10 @@ def test_lora_silu_and_mul(slots, d):
     _check_u(u_out, got, a, sl, rows)
 
 
+def test_lora_silu_of_many_tiles():
+    test_lora_silu_and_mul([2] * 600 + [-1] * 300 + [0] * 200, 1056)  # 70 tiles: 4 waves a workgroup
+
+
 @pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
 @pytest.mark.parametrize("width", [32, 288, 4096])
 def test_lora_shrink(slots, width):
