@@ -118,9 +118,19 @@ LIG_DEVICE uint32_t lds_address(const void* p) {
 LIG_DEVICE void load_to_lds(const void* base, uint32_t offset, uint32_t lds) {  // base: uniform
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(offset), "{m0}"(lds) : "memory");
 }
+// of bytes that nobody reads again: they do not displace others in the caches
+LIG_DEVICE void stream_to_lds(const void* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %0 nt" ::"s"(base), "v"(offset), "{m0}"(lds) : "memory");
+}
 LIG_DEVICE void load_to_lds(const void* p, uint32_t lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "{m0}"(lds) : "memory");
 }
+// Whether a weight [N, K] that one workgroup reads once is loaded as a stream, past
+// the caches: from 32 MiB on, where a model's weights together no longer stay in the
+// 256 MB of the last-level cache from one step to the next.  Streams of 32 MiB and
+// more gain 4 to 13 % (row_product.hip), smaller ones nothing, and a model small
+// enough to stay in that cache would lose up to 10 %.
+__host__ __device__ constexpr bool streams(int N, int K) { return (long)N * K >= 1L << 24; }
 // All but this wave's last N loads have landed and its LDS reads are done, and so
 // are those of the other waves.
 template <int N>

@@ -26,7 +26,9 @@
 //    202         59 ( 72)       42 ( 62)    19 ( 25)    25 ( 27)  (library at 256)
 //    384             (77)       56 ( 77)    26 ( 24)    33 ( 36)
 //   1024                       115 (127)    41 ( 41)
-// gate_up at 48 rows reads W at 5.7 TB/s.
+// gate_up at 48 rows reads W at 5.7 TB/s.  Where one tile holds all rows, loads of a
+// large W are non-temporal (`streams`): a step of 33 decodes with all its products
+// 2326 -> 2267 us, of a prompt of 202 rows 1793 -> 1753.
 #include "common.h"
 
 namespace {
@@ -87,6 +89,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void projectio
   constexpr bool PAIRS = TN % 2 == 0;
   auto f_w = [](int r) { return PAIRS ? (r & 3) | ((r >> 1) & 4) : r & 7; };
   const uint32_t lds = lds_address(sm);
+  const bool stream_w = mtiles == 1 && streams(N, K);  // no second workgroup reads these rows
   uint32_t off[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
@@ -104,8 +107,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void projectio
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int idx = min(wave * NI + i, NF - 1);
-      const uint16_t* base = (idx % (ROWS / 8) * 8 < BN ? wp : xp) + (size_t)at * 64 * PK;
-      load_to_lds(base, off[i], lds + (step % ST * STAGE + idx * 512) * 2);
+      const bool of_w = idx % (ROWS / 8) * 8 < BN;
+      const uint16_t* base = (of_w ? wp : xp) + (size_t)at * 64 * PK;
+      const uint32_t to = lds + (step % ST * STAGE + idx * 512) * 2;
+      if (of_w && stream_w) stream_to_lds(base, off[i], to);
+      else load_to_lds(base, off[i], to);
     }
   };
 

@@ -12,8 +12,11 @@
 //   silu: the two rows are a gate and its up row, y = silu(gate) * up of both
 //         rounded to bf16, as silu_and_mul after the projection.
 // Widths of Llama-3-8B, weights not in any cache, against the library's product
-// with the norm and activation as kernels of their own: norm + qkv 12.6 us (18.5),
-// o 8.5 (13.0), norm + gate_up + silu 43.0 (69.2, now 5.5 TB/s), down 24.2 (26.5).
+// with the norm and activation as kernels of their own: norm + qkv 12.7 us (18.5),
+// o 8.4 (13.0), norm + gate_up + silu 40.9 (69.2, now 5.7 TB/s), down 21.7 (26.5).
+// Loads of a large W are non-temporal (`streams`): without that gate_up 43.9, down
+// 24.7, qkv 13.5, o 8.8, a gate_up of 24576 x 8192 63.9 instead of 69.6.  Starting the
+// waves at different columns changed nothing.
 #include "common.h"
 
 namespace {
@@ -22,7 +25,7 @@ constexpr int NORM_MAX = 8192;  // columns of a row with a norm
 constexpr int PLAIN_MAX = 16384;
 constexpr int U = 4;  // loads of a row per batch, 512 columns each
 
-template <int NTHR, bool NORM, bool SILU>
+template <int NTHR, bool NORM, bool SILU, bool STREAM>
 __global__ __launch_bounds__(NTHR) void row_product_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ w, const int N, const int K, const uint16_t* __restrict__ x,
     const uint16_t* __restrict__ residual, uint16_t* __restrict__ residual_out, const uint16_t* __restrict__ weight,
@@ -45,7 +48,10 @@ __global__ __launch_bounds__(NTHR) void row_product_kernel(
     for (int i = 0; i < U; ++i) {
       const int c = min((batch * U + i) * 512, K - 512);  // past the end: the last columns again, unused
 #pragma unroll
-      for (int r = 0; r < 2; ++r) buf[b][i][r] = *reinterpret_cast<const u16x8*>(wr[r] + c);
+      for (int r = 0; r < 2; ++r) {
+        const u16x8* src = reinterpret_cast<const u16x8*>(wr[r] + c);
+        buf[b][i][r] = STREAM ? __builtin_nontemporal_load(src) : *src;
+      }
     }
   };
   load(0, 0);
@@ -146,12 +152,19 @@ extern "C" void lig_row_product_launch(uint16_t* y, const uint16_t* w, int N, in
                                        float eps, bool silu, hipStream_t stream) {
   // with a norm 8 waves share the h they form: 6144 x 4096 12.7 us (14.8 with 4
   // waves), 12288 x 4096 20.5 (25.2), 24576 x 8192 72 (76), 3072 x 2048 8.1 (8.5)
-#define LIG_RP(NTHR, NORM, SILU)                                                                                    \
-  hipLaunchKernelGGL((row_product_kernel<NTHR, NORM, SILU>),                                                        \
+  const bool stream_w = streams(N, K);
+#define LIG_RP1(NTHR, NORM, SILU, STREAM)                                                                           \
+  hipLaunchKernelGGL((row_product_kernel<NTHR, NORM, SILU, STREAM>),                                                \
                      dim3((N + NTHR / WAVE_SIZE * 2 - 1) / (NTHR / WAVE_SIZE * 2)), dim3(NTHR), (size_t)K * 2, stream, \
                      y, w, N, K, x, residual, residual_out, weight, eps)
+#define LIG_RP(NTHR, NORM, SILU)                   \
+  do {                                             \
+    if (stream_w) LIG_RP1(NTHR, NORM, SILU, true); \
+    else LIG_RP1(NTHR, NORM, SILU, false);         \
+  } while (0)
   if (silu) LIG_RP(512, true, true);
   else if (weight) LIG_RP(512, true, false);
   else LIG_RP(256, false, false);
 #undef LIG_RP
+#undef LIG_RP1
 }
