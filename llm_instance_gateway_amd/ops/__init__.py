@@ -728,7 +728,7 @@ def paged_attention_general(
             scratch = torch.empty(R * num_heads * nsplits * (D + 2), dtype=torch.float32, device=q.device)
         _hl().lig_paged_attention_general(
             _ptr(out), _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache),
-            _ptr(block_tables), block_tables.shape[1], _ptr(tok_seq),
+            _ptr(block_tables), block_tables.shape[0], block_tables.shape[1], _ptr(tok_seq),
             _ptr(positions), _ptr(gate), 0 if gate is None else gate.stride(0),
             _ptr(sink), float(scale), float(temp_coef), ev, ev_int, R, num_heads,
             G, D, Dv, v_row, bs, int(chunk), int(window), _ptr(score_bias),

@@ -103,6 +103,7 @@ extern "C" void lig_paged_attention_decode_launch(
   a.k_cache = k_cache;
   a.v_cache = v_cache;
   a.block_tables = block_tables;
+  a.tables = num_seqs;
   a.context_lens = context_lens;
   a.scratch = scratch;
   a.scale = scale;

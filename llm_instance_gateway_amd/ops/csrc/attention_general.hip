@@ -421,7 +421,7 @@ void lig_temperature_scale_rows(void* out, const void* q, long q_stride,
 
 void lig_paged_attention_general(
     void* out, const void* q, long q_stride, const void* k_cache,
-    const void* v_cache, const int* block_tables, int max_blocks,
+    const void* v_cache, const int* block_tables, int tables, int max_blocks,
     const int* tok_seq, const int64_t* positions, const void* gate,
     long gate_stride, const float* sink, float scale, float temp_coef,
     float temp_every, int temp_every_int, int R, int H, int G, int D, int Dv,
@@ -440,6 +440,7 @@ void lig_paged_attention_general(
   fa.sink = sink;
   fa.score_bias = score_bias;
   fa.block_tables = block_tables;
+  fa.tables = tables;
   fa.tok_seq = tok_seq;
   fa.positions = positions;
   fa.scratch = scratch;

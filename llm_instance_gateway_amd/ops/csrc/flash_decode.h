@@ -30,8 +30,8 @@
 // Measured, 32 query and 8 key/value heads of 128, before -> after: 384
 // requests of 190-381 tokens 173 -> 84 us (5.3 TB/s; a large copy reaches 4.9);
 // 33 of 3000-6000 370 -> 119 us (5.0 TB/s); 16 of 190-381 30 -> 8.2 us; 64 rows
-// with a window of 512 and sigmoid weights 54 -> 28 us, 44 -> 24 where their 134 MB
-// are still in the last-level cache.  Eight waves per workgroup
+// with a window of 512 and sigmoid weights 54 -> 24.5 us (28.3 before values were
+// loaded as streams).  Eight waves per workgroup
 // were slower from 64 requests on (101 us at 384), two on few (9.2 us at 16).
 #pragma once
 
@@ -58,7 +58,8 @@ struct Args {
   long gate_stride;
   const float* sink;        // nullable, [Hq]
   const float* score_bias;  // nullable, [Hq]
-  const int* block_tables;  // [S, max_blocks]
+  const int* block_tables;  // [tables, max_blocks]
+  int tables;
   // row r belongs to table row tok_seq[r] (negative: none) and sees keys up to
   // positions[r]; without them it is table row r, up to context_lens[r] - 1
   const int* tok_seq;
@@ -128,7 +129,7 @@ LIG_DEVICE void store_entries(const Args& a, int row, int h, int d, const float 
 
 // W waves per workgroup; LOWCOL: at most 8 heads per group, the weights' middle
 // parts in columns 8..15; PB: block size a power of two, at least 8.  CAP, SIG, EXTRA as in the prompt kernel.
-template <int D, int W, bool LOWCOL, bool PB, bool CAP, bool SIG, bool EXTRA>
+template <int D, int W, bool LOWCOL, bool PB, bool STREAM, bool CAP, bool SIG, bool EXTRA>
 __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
   constexpr int KS = D / 32;
   constexpr int DV = D / 16;          // entries of a value row per lane
@@ -238,7 +239,10 @@ __global__ __launch_bounds__(64 * W, 2) void flash_decode_kernel(const Args a) {
     size_t r[8];
     rows_of(st * KT + vt0, 0, 1, blk, r);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) vreg[t] = *reinterpret_cast<const vload*>(a.v_cache + r[t] * a.v_row + li * DV);
+    for (int t = 0; t < 8; ++t) {
+      const vload* src = reinterpret_cast<const vload*>(a.v_cache + r[t] * a.v_row + li * DV);
+      vreg[t] = STREAM ? __builtin_nontemporal_load(src) : *src;
+    }
   };
 
   float m = -INFINITY, l = 0.f;
@@ -505,14 +509,23 @@ static void launch_rows(const Args& a, hipStream_t stream) {
   const dim3 grid(a.rows * a.num_kv_heads, a.nsplits), block(64 * W);
   const bool low = group <= 8, pb = a.block_shift >= 3;
   const size_t lds = (size_t)W * (group * D + 2 * (low ? 8 : 16)) * sizeof(float);
-  if (low && pb)
-    hipLaunchKernelGGL((flash_decode_kernel<D, W, true, true, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
-  else if (low)
-    hipLaunchKernelGGL((flash_decode_kernel<D, W, true, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
-  else if (pb)
-    hipLaunchKernelGGL((flash_decode_kernel<D, W, false, true, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
-  else
-    hipLaunchKernelGGL((flash_decode_kernel<D, W, false, false, CAP, SIG, EXTRA>), grid, block, lds, stream, a);
+  // Values as a stream past the caches (non-temporal) where no other row reads them,
+  // as far as the host can tell, and where rows are many: their caches don't stay in
+  // the last-level cache from one step to the next.  One row of a few hundred keys has
+  // them there, and a step of it is 1 % slower with streams; 8 rows on each of 32 tables
+  // of 1000 keys 83 -> 91 us.  Streamed: 64 rows of 1000 keys 47.7 -> 43.5 us, 40 of 300
+  // 15.1 -> 14.3, 64 with a window of 512 28.3 -> 24.5; all of 64 x 100 to 64 x 500 still
+  // cached: the same.  Keys too, whose lines take two loads, gives half of that back.
+  const bool many = (long)a.rows * a.num_kv_heads >= 256 && a.rows <= a.tables;
+#define LIG_FD(LOWCOL, PB, STREAM)                                                                             \
+  hipLaunchKernelGGL((flash_decode_kernel<D, W, LOWCOL, PB, STREAM, CAP, SIG, EXTRA>), grid, block, lds, stream, a)
+  if (low && pb && many) LIG_FD(true, true, true);
+  else if (low && pb) LIG_FD(true, true, false);
+  else if (low) LIG_FD(true, false, false);
+  else if (pb && many) LIG_FD(false, true, true);
+  else if (pb) LIG_FD(false, true, false);
+  else LIG_FD(false, false, false);
+#undef LIG_FD
   launch_merge<D, SIG, EXTRA>(a, stream);
 }
 

@@ -93,7 +93,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "lig_sigmoid_gate_mul": [p, p, l, i, i, i, p],
         "lig_mingru_scan": [p, p, p, p, l, p, p, p, p, p, p, i, i, i, i, p],
         "lig_paged_attention_general": [
-            p, p, l, p, p, p, i, p, p, p, l, p, f, f, f, i, i, i, i, i, i, i, i, i,
+            p, p, l, p, p, p, i, i, p, p, p, l, p, f, f, f, i, i, i, i, i, i, i, i, i,
             i, p, i, i, f, i, p, i, p,
         ],
         "lig_offset_norm_shift": [p, p, p, p, p, p, p, p, p, p, p, p, p, p, p, f, i, i, i, p],

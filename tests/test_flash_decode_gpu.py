@@ -243,3 +243,23 @@ def test_more_rows_than_a_grid_dimension_holds():
     ):
         got = got.view(R, H * D)
         assert torch.equal(got[0::2], want[:1].expand(R // 2 + 1, -1)) and torch.equal(got[1::2], want[1:].expand(R // 2, -1))
+
+
+@pytest.mark.parametrize("opt", [None, {}, dict(weights="sigmoid", window=100)], ids=range(3))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 8, 16), (128, 18, 2, 8), (64, 16, 4, 32)])
+def test_many_rows_are_the_few(D, H, G, bs, opt):
+    """A row's result does not depend on how many come with it (from 256 rows of
+    key/value heads on, values are loaded past the caches)."""
+    n = 256 // G
+    b = _batch([CTX[i % len(CTX)] for i in range(n)], G, D, bs, H, 23)
+
+    def run(to):
+        if opt is None:
+            return ops.paged_attention_decode(b["q"][:to].view(-1, H, D), b["k"], b["v"], b["tab"][:to].contiguous(),
+                                              b["ctx"][:to].contiguous(), D ** -0.5, nsplits=2).view(to, -1)
+        return ops.paged_attention_general(b["q"][:to], b["k"], b["v"], b["tab"], b["tok_seq"][:to].contiguous(),
+                                           b["pos"][:to].contiguous(), D ** -0.5, H, **opt)
+
+    many = run(n)
+    _check(many, b, D ** -0.5, H, **(opt or {}))
+    assert torch.equal(many[: n - 1], run(n - 1))
