@@ -33,7 +33,7 @@ def pack_rows(rows: Seq[List[int]], out: np.ndarray) -> None:
 
 def pack_decodes(seqs: list, block_size: int, ids: np.ndarray, positions: np.ndarray, tables: np.ndarray) -> None:
     """The token that each sequence processes at num_computed_tokens, that
-    position, and its cache blocks in a row of `tables` (zeros behind them)."""
+    position, and its cache blocks at the start of a row of `tables`."""
     ext = ops._load_ext()
     if ext is not None:
         ext.pack_decodes(seqs, block_size, ids, positions, tables)

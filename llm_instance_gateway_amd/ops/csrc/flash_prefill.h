@@ -22,15 +22,16 @@
 //     transposed by byte permutes.  LDS is double-buffered: one barrier per 64 keys;
 //   * the accumulators are only rescaled when a row's maximum grew, and masks
 //     are only evaluated on tiles that cross a row's visible range.
-// Measured, 32 query and 8 key/value heads of 128, before -> after: 4096 rows
-// on 4000 cached keys 3409 -> 495 us (119 -> 820 TFLOP/s; 571 us, 711 TFLOP/s,
-// between the products of an engine step); 20 prompts of 200 130 -> 37 us; one of
-// 202 20.6 -> 8.9 us; 8 of 1000 with a window of 512 571 -> 110 us, with a soft cap
-// 578 -> 133, with sigmoid weights 566 -> 103.
+// Measured so far, 32 query and 8 key/value heads of 128, with rows still through
+// registers, against the kernel this replaces: 4096 rows on 4000 cached keys 3409 ->
+// 495 us (820 TFLOP/s; 571 between the products of an engine step); 20 prompts of
+// 200 130 -> 37 us; one of 202 20.6 -> 8.9 us; 8 of 1000 with a window of 512 571 ->
+// 110 us, with a soft cap 578 -> 133, with sigmoid weights 566 -> 103.
 // What then bound it were vector instructions (64 % of the cycles, and LDS 53 %, half
 // of that conflicts).  Without selects for masked keys, with pairs rounded at once,
 // rows by DMA and their block's row number worked out once per group of keys: 4000
-// rows on 4000 keys 560 -> 441 us, 8 of 1000 with the window and a cap 120 -> 96.
+// rows on 4000 keys 560 -> 441 us (between products), 20 prompts of 200 37 -> 33, one
+// of 202 8.9 -> 7.9, 8 of 1000 with the window and a cap 120 -> 96.
 // Four heads per workgroup and 64 rows per wave (all 512 registers, one wave
 // per SIMD) was slower everywhere: 781 us in the first of these.
 #pragma once

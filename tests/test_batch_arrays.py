@@ -40,6 +40,29 @@ def test_pack_rows_refuses(path, rows, shape):
         ba.pack_rows(rows, np.zeros(shape, dtype=np.int32))
 
 
+def _decode(computed, blocks):
+    s = Sequence([5, 6, 7])
+    s.output_token_ids = [8, 9]
+    s.num_computed_tokens, s.block_table = computed, blocks
+    return s
+
+
+def test_pack_decodes(path):
+    seqs = [_decode(2, [4]), _decode(3, [1, 2**31 - 1]), _decode(4, [9, 3, 6])]  # prompt's end, outputs, spare block
+    ids, pos, tab = np.zeros(3, np.int64), np.zeros(3, np.int64), np.full((3, 4), -7, np.int32)
+    ba.pack_decodes(seqs, 4, ids, pos, tab)
+    assert ids.tolist() == [7, 8, 9] and pos.tolist() == [2, 3, 4]
+    assert tab.tolist() == [[4, -7, -7, -7], [1, 2**31 - 1, -7, -7], [9, 3, 6, -7]]
+
+
+@pytest.mark.parametrize("computed,blocks,room", [(4, [1], 4), (2, [], 4), (5, [1, 2], 4), (2, [1, 2, 3], 2)])
+def test_pack_decodes_refuses(path, computed, blocks, room):
+    """too few blocks, none, no such token, more blocks than room"""
+    with pytest.raises(Exception):
+        ba.pack_decodes([_decode(computed, blocks)], 4, np.zeros(1, np.int64), np.zeros(1, np.int64),
+                        np.zeros((1, room), np.int32))
+
+
 def test_upload_keeps_values_and_alignment():
     arrays = [np.arange(3, dtype=np.int64), np.zeros((0, 4), np.int32), np.arange(10, dtype=np.int32).reshape(5, 2),
               np.arange(12, dtype=np.int32).reshape(3, 4).T, np.array([9], dtype=np.int64)]
