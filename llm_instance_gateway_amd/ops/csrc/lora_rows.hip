@@ -5,7 +5,7 @@
 // products with A read every GEMM input once more and those with B read and
 // wrote every GEMM output once more: 3.5 of 15.3 ms of a step with 4000 prompt
 // tokens over 8 layers, and two launches of 5-12 us per GEMM in decode steps.
-// (That step takes 11.9 ms now; norm with both products of 33 tokens of 8 adapters
+// (That step takes 11.5 ms now; norm with both products of 33 tokens of 8 adapters
 // 11.6 us for 15 before, of 384 of 32 16.8 for 26, of 4000 38 for 133.)
 // Here
 //   * B u is added where the GEMM's output is read anyway: the rotation and

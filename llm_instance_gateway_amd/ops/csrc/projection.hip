@@ -25,7 +25,9 @@
 //     48         41 ( 60)       26 ( 37)    11 ( 15)    15 ( 17)
 //    202         59 ( 72)       42 ( 62)    19 ( 25)    25 ( 27)  (library at 256)
 //    384             (77)       56 ( 77)    26 ( 24)    33 ( 36)
+//    832                       103 (115 with tiles of 256 rows)
 //   1024                       115 (127)    41 ( 41)
+// A head of 128256 x 4096: 256 rows 253 (297), 384 rows 388 (431).
 // gate_up at 48 rows reads W at 5.7 TB/s.  Where one tile holds all rows, loads of a
 // large W are non-temporal (`streams`): a step of 33 decodes with all its products
 // 2326 -> 2267 us, of a prompt of 202 rows 1793 -> 1753.
