@@ -312,24 +312,34 @@ class LlamaForCausalLM(nn.Module):
         return hidden
 
     def _open_norms(self, rows: int) -> bool:
-        """Whether `_forward_open` is for a step of that many rows without adapters:
-        where `ops.linear` runs its products (asked of one layer: a product that
-        runs elsewhere comes rounded, which the kernels behind it take as well)."""
+        """Whether `_forward_open` is for a step of that many rows without adapters."""
         c = self.cfg
-        if (self.tp is not None or not self.norm.is_cuda or self.norm.dtype != torch.bfloat16
-                or c.intermediate_size % 32 or c.head_dim % 64 or not ops.lora_norm_opens(ops.BASE_ROWS, rows, c.hidden_size)):
+        return (self.tp is None and self.norm.is_cuda and self.norm.dtype == torch.bfloat16 and c.head_dim % 64 == 0
+                and ops.lora_norm_opens(ops.BASE_ROWS, rows, c.hidden_size) and self.plain_layers()
+                and self._opens(0, rows))
+
+    def _opens(self, i: int, rows: int) -> bool:
+        """Whether layer i's norms may leave their factor to what reads the products
+        behind them, and come after products in parts: where all its projections
+        are products and nothing else, by our kernels."""
+        if i >= len(self.layers):
             return False
-        layer = self.layers[0]
-        attn, mlp = layer.self_attn, getattr(layer, "mlp", None)
-        return type(mlp) is MLP and self.plain_layers() and all(
-            _served(m, rows) for m in (attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj))
+        attn, mlp = self.layers[i].self_attn, self.layers[i].mlp
+        return (all(_served(m, rows) for m in (attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj))
+                and mlp.gate_up_proj.out_features % 64 == 0)
 
     def _forward_open(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
         """The layers with each norm as one kernel that adds up the product before
-        it and leaves its factor to the rotation and the activation."""
+        it and leaves its factor to the rotation and the activation; layers that
+        do more than multiply run their own forward."""
         rows = ops.BASE_ROWS
-        residual, y = None, hidden
+        residual, y, opens = None, hidden, self._opens(0, len(hidden))
         for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
+            after = self._opens(i + 1, len(hidden))
+            if not opens:
+                y, residual = layer(y, residual, positions, kv, meta, self.cos_sin_cache)
+                opens = after
+                continue
             attn, mlp = layer.self_attn, layer.mlp
             h, _, norm = ops.lora_norm_open(y, residual, layer.input_layernorm, layer.eps, rows)
             if residual is None:
@@ -341,8 +351,7 @@ class LlamaForCausalLM(nn.Module):
             h, _, norm = ops.lora_norm_open(
                 _project(attn.o_proj, o, ops.linear_parts), residual, layer.post_attention_layernorm, layer.eps, rows)
             act = ops.lora_silu_and_mul(_project(mlp.gate_up_proj, h), rows, None, None, None, None, norm)
-            last = i + 1 == len(self.layers)
-            y = _project(mlp.down_proj, act, ops.linear if last else ops.linear_parts)
+            y, opens = _project(mlp.down_proj, act, ops.linear_parts if after else ops.linear), after
         return ops.fused_add_rms_norm(y, residual, self.norm, self.cfg.rms_norm_eps)[0]
 
     def lora_in_layer(self, rank: int, dims: dict) -> bool:
@@ -371,16 +380,18 @@ class LlamaForCausalLM(nn.Module):
         a, b = lora.a_stacks, lora.b_stacks
         residual, y, last = None, hidden, None
         # Norms whose readers can take the rows' factor themselves are one launch, and
-        # add up the product before them.  The rotation takes it with fp32 parts
-        # only: a rounded product would be rounded once more on its way to V.
-        opens = ops.lora_norm_opens(rows, len(hidden), c.hidden_size)
+        # add up the product before them.  Only products carry the factor through: a
+        # module with a bias or a hook gets normed rows.  The rotation takes it with
+        # fp32 parts only: a rounded product would be rounded once more on its way to V.
+        can_open = ops.lora_norm_opens(rows, len(hidden), c.hidden_size)
 
         def open_in(i):  # the norm at layer i's entry
-            return opens and i < len(self.layers) and _served(self.layers[i].self_attn.qkv_proj, len(hidden))
+            return can_open and i < len(self.layers) and _served(self.layers[i].self_attn.qkv_proj, len(hidden))
 
         parts = open_in(0)
         for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
             attn, mlp = layer.self_attn, layer.mlp
+            opens = can_open and _product_alone(mlp.gate_up_proj)  # the norm behind the attention
             norm = ops.lora_norm_open if parts else ops.lora_rms_norm
             if last is None:
                 h, u, *scale = norm(y, None, layer.input_layernorm, layer.eps, rows, a_stack=a[(i, "qkv")], u_out=ws)

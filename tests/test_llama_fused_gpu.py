@@ -299,6 +299,69 @@ def test_engine_matches_unit_kernels(monkeypatch):
         assert (a - b).norm() <= 0.03 * b.norm()
 
 
+def _wide_steps(lora, change, prompts):
+    """Logits of a prompt step and of a replayed decode step of a model wide enough
+    for norms that leave their factor to the readers, and how many norms did."""
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.lora import manager
+    from llm_instance_gateway_amd.models.config import ModelConfig
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=2048, num_layers=3, num_heads=16, num_kv_heads=4,
+                     intermediate_size=8192, head_dim=128, max_position_embeddings=512)
+    torch.manual_seed(0)
+    eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=200, max_num_seqs=8, max_num_batched_tokens=512,
+                                 max_model_len=256), device="cuda:0")
+    model = eng.runner.model
+    if lora:
+        mgr = manager.AdapterManager(eng, max_slots=3, rank=16)
+        assert mgr.in_layer
+        for i in range(3):
+            mgr.register_random(f"l{i}", seed=i)
+    if change is not None:
+        name, how = change
+        m = getattr(model.layers[1].mlp if name == "gate_up_proj" else model.layers[1].self_attn, name)
+        if how == "bias":
+            g = torch.Generator(device="cuda").manual_seed(3)
+            m.bias = torch.nn.Parameter(0.5 * torch.randn(m.out_features, device="cuda", generator=g).to(BF))
+        else:
+            m.register_forward_pre_hook(lambda mod, args: (args[0].clamp(-0.5, 0.5),))
+    g = torch.Generator().manual_seed(5)
+    seqs = [eng.add_request(torch.randint(1, 500, (n,), generator=g).tolist(), SamplingParams(max_new_tokens=4),
+                            lora_name=["l0", "", "l2", "l1", "l0"][i] if lora else "") for i, n in enumerate(prompts)]
+    logits, head, opened, norm = [], model.compute_logits, [], ops.lora_norm_open
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(model, "compute_logits", lambda h, idx: logits.append(head(h, idx)) or logits[-1])
+        mp.setattr(ops, "lora_norm_open", lambda *a, **k: opened.append(1) or norm(*a, **k))
+        eng.step()
+        first, n = logits[0][: len(seqs)].clone(), len(opened)
+        for s in seqs:  # the same continuation on both sides
+            s.output_token_ids[-1] = 11
+        eng.step()
+    gr = eng.runner.graph_runner
+    return first, gr.logits[gr.pick_size(len(seqs))][: len(seqs)].float().clone(), n
+
+
+CHANGES = [None] + [(m, how) for m in ("gate_up_proj", "qkv_proj") for how in ("bias", "hook")]
+
+
+@pytest.mark.parametrize("change", CHANGES, ids=str)
+@pytest.mark.parametrize("lora", [False, True])
+def test_open_norms_match_closed(monkeypatch, lora, change):
+    """Norms that leave their factor to the readers beside norms that do not, also
+    where a layer's projection does more than multiply: such a module gets normed rows."""
+    # 310 rows: qkv, o and down by our kernels, gate_up by the library's
+    for prompts in ((5,), (33,), (100, 120, 90), (3, 17, 40, 64, 5)) if change is None else ((3, 17, 40, 64, 5),):
+        a, b, n = _wide_steps(lora, change, prompts)
+        with monkeypatch.context() as mp:
+            mp.setattr(ops, "lora_norm_opens", lambda *a: False)
+            x, y, none = _wide_steps(lora, change, prompts)
+        # two correct orders of bf16 rounding, 3 layers deep
+        assert (a - x).norm() <= 0.03 * x.norm() and (b - y).norm() <= 0.03 * y.norm()
+        # of 6 norms; without adapters a layer of products that are not all ours is closed, and so are all in 310 rows
+        want = (6 if lora or sum(prompts) <= 256 else 0) if change is None else (5 if lora else 4)
+        assert (n, none) == (want, 0)
+
+
 @pytest.mark.parametrize("lora", [False, True])
 def test_module_hooks_run(lora):
     """The fused forwards stand aside for hooks on the modules they replace."""
