@@ -549,7 +549,7 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
       gv *= factor;
       uv *= factor;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = gv[j] * __builtin_amdgcn_rcpf(1.0f + __expf(-gv[j])) * uv[j];
+      for (int j = 0; j < 8; ++j) r[j] = gv[j] / (1.0f + __expf(-gv[j])) * uv[j];
       const u16x8 rb = f32x8_to_bf16x8(r);
       if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
       if constexpr (LORA) acc = shrink(ar[i], rb, acc);

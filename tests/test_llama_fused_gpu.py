@@ -141,6 +141,18 @@ def test_lora_silu_of_many_tiles():
     test_lora_silu_and_mul([2] * 600 + [-1] * 300 + [0] * 200, 1056)  # 70 tiles: 4 waves a workgroup
 
 
+@pytest.mark.parametrize("T", [400, 1100])  # 8 and 4 waves a workgroup
+def test_lora_silu_divides(T):
+    """Rows without an adapter come out as those of `silu_and_mul`, bit for bit."""
+    rnd, rows, _ = _lora([-1] * T, T)
+    x = (3 * rnd(T, 2 * 14336)).to(BF)
+    want = ops.silu_and_mul(x)
+    assert torch.equal(ops.lora_silu_and_mul(x, ops.BASE_ROWS, None, None, None, None), want)
+    u, a, b = rnd(1, len(rows[1]), 16, 16), rnd(1, 16, 14336).to(BF), rnd(1, 2 * 14336, 16).to(BF)
+    ws = torch.empty(14, len(rows[1]), 16, 16, device="cuda")
+    assert torch.equal(ops.lora_silu_and_mul(x, rows, u, b, a, ws), want)
+
+
 @pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
 @pytest.mark.parametrize("width", [32, 288, 4096])
 def test_lora_shrink(slots, width):
