@@ -420,7 +420,7 @@ def _tiles(rows, T: int) -> int:
 def lora_norm_opens(rows, T: int, width: int) -> bool:
     """Whether `lora_norm_open` is for these tiles: where the norm takes strips."""
     return (width >= 2048 and _tiles(rows, T) * 4096 < LORA_NORM_STRIPS_BELOW * width
-            and width % _load_ext().lora_norm_strip() == 0)
+            and _load_ext() is not None and width % _EXT.lora_norm_strip() == 0)
 
 
 def lora_norm_open(x, residual, weight, eps, rows, u_in=None, b_stack=None, a_stack=None, u_out=None):

@@ -272,3 +272,11 @@ def test_build_lora_units():
     # all -1 -> no units
     _, t0e, _, _ = build_lora_units([-1, -1])
     assert len(t0e) == 0
+
+
+def test_norms_stay_closed_without_the_extension(monkeypatch):
+    """With LIG_FORCE_TORCH_OPS a step runs where nothing is built."""
+    from llm_instance_gateway_amd import ops
+
+    monkeypatch.setattr(ops, "_load_ext", lambda: None)
+    assert not ops.lora_norm_opens(ops.BASE_ROWS, 16, 4096)
