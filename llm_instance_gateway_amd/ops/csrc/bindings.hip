@@ -747,6 +747,8 @@ static void pack_rows(py::sequence rows, py::array out) {
 
 // What sequences that each process their token at num_computed_tokens bring: that
 // token, its position, and their cache blocks in a row of `tables` (int32, zeros).
+// Arrays of other types are refused (noconvert): a converted one would be filled and
+// dropped.
 static void pack_decodes(py::list seqs, int64_t block_size, py::array_t<int64_t> ids, py::array_t<int64_t> positions,
                          py::array_t<int32_t> tables) {
   const ssize_t n = py::len(seqs);
@@ -807,7 +809,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_cache", &qkv_rope_cache);
   m.def("silu_and_mul", &silu_and_mul);
   m.def("argmax_rows", &argmax_rows);
-  m.def("pack_decodes", &pack_decodes);
+  m.def("pack_decodes", &pack_decodes, py::arg("seqs"), py::arg("block_size"), py::arg("ids").noconvert(),
+        py::arg("positions").noconvert(), py::arg("tables").noconvert());
   m.def("projection", &projection);
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);

@@ -63,6 +63,19 @@ def test_pack_decodes_refuses(path, computed, blocks, room):
                         np.zeros((1, room), np.int32))
 
 
+@pytest.mark.parametrize("which", range(3))
+def test_pack_decodes_fills_or_refuses(path, which):
+    """Arrays of another type are not filled as a copy and dropped."""
+    types = [np.int64, np.int64, np.int32]
+    types[which] = np.int16
+    ids, pos, tab = (np.zeros(shape, t) for shape, t in zip((1, 1, (1, 2)), types))
+    try:
+        ba.pack_decodes([_decode(3, [6])], 4, ids, pos, tab)
+    except TypeError:
+        return
+    assert (ids.tolist(), pos.tolist(), tab.tolist()) == ([8], [3], [[6, 0]])
+
+
 def test_upload_keeps_values_and_alignment():
     arrays = [np.arange(3, dtype=np.int64), np.zeros((0, 4), np.int32), np.arange(10, dtype=np.int32).reshape(5, 2),
               np.arange(12, dtype=np.int32).reshape(3, 4).T, np.array([9], dtype=np.int64)]
