@@ -459,35 +459,36 @@ def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_ma
 
 
 def linear_served(rows: int, weight: torch.Tensor) -> bool:
-    """Whether `linear` runs that many rows on the kernels of projection.hip."""
+    """Whether `linear` runs that many rows on the kernels of projection.hip: not
+    where a derivative or a transform has to see the product."""
     return (
-        weight.is_cuda
+        type(weight) in (torch.Tensor, torch.nn.Parameter)
+        and weight.is_cuda
         and weight.dtype == torch.bfloat16
         and weight.dim() == 2
         and weight.is_contiguous()
         and weight.data_ptr() % 16 == 0
+        and not (weight.requires_grad and torch.is_grad_enabled())
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
         and _use_native(weight)
         and _EXT.projection_serves(rows, *weight.shape)
     )
 
 
 def _linear_here(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether x @ weight.T is for our kernels: not where a derivative or a
-    transform has to see the product."""
+    """Whether x @ weight.T is for our kernels."""
     return (
         type(x) is torch.Tensor
-        and type(weight) in (torch.Tensor, torch.nn.Parameter)
         and x.is_cuda
         and x.device == weight.device
         and x.dtype == torch.bfloat16
         and x.dim() == 2
         and x.shape[1] == weight.shape[-1]
-        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
-        and torch._C._functorch.peek_interpreter_stack() is None
-        and torch.autograd.forward_ad._current_level < 0
-        and linear_served(x.shape[0], weight)
         and x.is_contiguous()
         and x.data_ptr() % 16 == 0
+        and not (x.requires_grad and torch.is_grad_enabled())
+        and linear_served(x.shape[0], weight)
     )
 
 

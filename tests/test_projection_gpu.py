@@ -57,3 +57,23 @@ def test_other_calls_stay_with_the_library():
     assert p.grad is not None
     with pytest.raises(RuntimeError):
         ops.linear(r(8, 64).to(BF), w)
+
+
+def test_served_is_what_linear_does():
+    """A layer that leaves a norm open must know that the product comes in parts: with
+    a gradient to record, under a transform or forward-mode, it comes rounded."""
+    w = torch.nn.Parameter(torch.ones(64, 128, device="cuda", dtype=BF))
+    x = torch.ones(8, 128, device="cuda", dtype=BF)
+    seen = []
+
+    def ask(v):
+        seen.append((ops.linear_served(8, w), ops.linear_parts(x, w).dim() == 3))
+        return v
+
+    ask(None)
+    with torch.no_grad():
+        ask(None)
+        torch.vmap(ask)(torch.zeros(2))
+        with torch.autograd.forward_ad.dual_level():
+            ask(None)
+    assert seen == [(False, False), (True, True), (False, False), (False, False)]
