@@ -460,10 +460,12 @@ def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_ma
 
 def linear_served(rows: int, weight: torch.Tensor) -> bool:
     """Whether `linear` runs that many rows on the kernels of projection.hip: not
-    where a derivative or a transform has to see the product."""
+    where a derivative or a transform has to see the product, nor on another device
+    than the current one, whose stream a launch would go to."""
     return (
         type(weight) in (torch.Tensor, torch.nn.Parameter)
         and weight.is_cuda
+        and weight.device.index == torch.cuda.current_device()
         and weight.dtype == torch.bfloat16
         and weight.dim() == 2
         and weight.is_contiguous()

@@ -77,3 +77,10 @@ def test_served_is_what_linear_does():
         with torch.autograd.forward_ad.dual_level():
             ask(None)
     assert seen == [(False, False), (True, True), (False, False), (False, False)]
+
+
+def test_another_device_stays_with_the_library(monkeypatch):
+    w, x = torch.ones(64, 128, device="cuda", dtype=BF), torch.ones(8, 128, device="cuda", dtype=BF)
+    assert ops.linear_served(8, w)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not ops.linear_served(8, w) and ops.linear_parts(x, w).dim() == 2
