@@ -45,8 +45,9 @@ def _linear(in_f: int, out_f: int, device, dtype) -> nn.Linear:
 
 
 def _product_alone(m: nn.Module) -> bool:
-    """Whether m(x) is x @ m.weight.T and nothing else."""
-    return (type(m) is nn.Linear and _plain(m.__dict__) and m._parameters["bias"] is None
+    """Whether m(x) is x @ m.weight.T and nothing else, its weight a parameter."""
+    p = m._parameters
+    return (type(m) is nn.Linear and _plain(m.__dict__) and p.get("weight") is not None and p.get("bias", p) is None
             and not _has_any_global_hook())
 
 

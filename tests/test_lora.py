@@ -280,3 +280,15 @@ def test_norms_stay_closed_without_the_extension(monkeypatch):
 
     monkeypatch.setattr(ops, "_load_ext", lambda: None)
     assert not ops.lora_norm_opens(ops.BASE_ROWS, 16, 4096)
+
+
+def test_projection_whose_weight_is_no_parameter():
+    """Wrappers that put a plain tensor in a layer's weight keep working."""
+    from llm_instance_gateway_amd.models.llama import _product_alone, _project
+
+    m = torch.nn.Linear(8, 4, bias=False)
+    w = m.weight.detach().clone()
+    del m.weight
+    m.weight = w
+    x = torch.randn(3, 8)
+    assert torch.equal(_project(m, x), x @ w.t()) and not _product_alone(m)
