@@ -317,42 +317,49 @@ class LlamaForCausalLM(nn.Module):
         c = self.cfg
         return (self.tp is None and self.norm.is_cuda and self.norm.dtype == torch.bfloat16 and c.head_dim % 64 == 0
                 and ops.lora_norm_opens(ops.BASE_ROWS, rows, c.hidden_size) and self.plain_layers()
-                and self._opens(0, rows))
+                and self._open_weights(self.layers[0], rows) is not None)
 
-    def _opens(self, i: int, rows: int) -> bool:
-        """Whether layer i's norms may leave their factor to what reads the products
-        behind them, and come after products in parts: where all its projections
-        are products and nothing else, by our kernels."""
-        if i >= len(self.layers):
-            return False
-        attn, mlp = self.layers[i].self_attn, self.layers[i].mlp
-        return (all(_served(m, rows) for m in (attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj))
-                and mlp.gate_up_proj.out_features % 64 == 0)
+    @staticmethod
+    def _open_weights(layer: DecoderLayer, rows: int):
+        """The weights of qkv, o, gate_up and down of a layer whose norms may leave
+        their factor to what reads the products behind them, and come after products
+        in parts: where all four are products and nothing else, by our kernels."""
+        m = layer.__dict__["_modules"]
+        attn, mlp = m["self_attn"].__dict__["_modules"], m["mlp"].__dict__["_modules"]
+        out = []
+        for lin in (attn["qkv_proj"], attn["o_proj"], mlp["gate_up_proj"], mlp["down_proj"]):
+            if not _served(lin, rows):
+                return None
+            out.append(lin._parameters["weight"])
+        return out if out[2].shape[0] % 64 == 0 else None
 
     def _forward_open(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
         """The layers with each norm as one kernel that adds up the product before
         it and leaves its factor to the rotation and the activation; layers that
         do more than multiply run their own forward."""
         rows = ops.BASE_ROWS
-        residual, y, opens = None, hidden, self._opens(0, len(hidden))
-        for i, (layer, kv) in enumerate(zip(self.layers, kv_caches)):
-            after = self._opens(i + 1, len(hidden))
-            if not opens:
+        layers = list(zip(self.layers, kv_caches))
+        residual, y, weights = None, hidden, self._open_weights(layers[0][0], len(hidden))
+        for i, (layer, kv) in enumerate(layers):
+            after = self._open_weights(layers[i + 1][0], len(hidden)) if i + 1 < len(layers) else None
+            if weights is None:
                 y, residual = layer(y, residual, positions, kv, meta, self.cos_sin_cache)
-                opens = after
+                weights = after
                 continue
-            attn, mlp = layer.self_attn, layer.mlp
+            qkv, o, gate_up, down = weights
             h, _, norm = ops.lora_norm_open(y, residual, layer.input_layernorm, layer.eps, rows)
             if residual is None:
                 residual = hidden
+            attn = layer.self_attn
             q = ops.lora_qkv_rope_cache(
-                _project(attn.qkv_proj, h, ops.linear_parts), positions, self.cos_sin_cache, kv[0], kv[1],
-                meta.slot_mapping, attn.num_heads, rows, None, None, norm)
-            o = attn.attend(q, kv, meta)
+                ops.projection_parts(h, qkv), positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping,
+                attn.num_heads, rows, None, None, norm)
             h, _, norm = ops.lora_norm_open(
-                _project(attn.o_proj, o, ops.linear_parts), residual, layer.post_attention_layernorm, layer.eps, rows)
-            act = ops.lora_silu_and_mul(_project(mlp.gate_up_proj, h), rows, None, None, None, None, norm)
-            y, opens = _project(mlp.down_proj, act, ops.linear_parts if after else ops.linear), after
+                ops.projection_parts(attn.attend(q, kv, meta), o), residual, layer.post_attention_layernorm, layer.eps,
+                rows)
+            act = ops.lora_silu_and_mul(ops.linear(h, gate_up), rows, None, None, None, None, norm)
+            y = (ops.linear if after is None else ops.projection_parts)(act, down)
+            weights = after
         return ops.fused_add_rms_norm(y, residual, self.norm, self.cfg.rms_norm_eps)[0]
 
     def lora_in_layer(self, rank: int, dims: dict) -> bool:

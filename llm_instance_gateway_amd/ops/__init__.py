@@ -458,40 +458,26 @@ def lora_qkv_rope_cache(qkv, positions, cos_sin_cache, k_cache, v_cache, slot_ma
     return q
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _product_native(t: torch.Tensor) -> bool:
+    """Whether no transform has to see the products of t, and t is where launches go."""
+    return (_use_native(t) and t.get_device() == torch.cuda.current_device()
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+
+
 def linear_served(rows: int, weight: torch.Tensor) -> bool:
-    """Whether `linear` runs that many rows on the kernels of projection.hip: not
+    """Whether `linear_parts` runs that many rows on the kernels of projection.hip: not
     where a derivative or a transform has to see the product, nor on another device
     than the current one, whose stream a launch would go to."""
-    return (
-        type(weight) in (torch.Tensor, torch.nn.Parameter)
-        and weight.is_cuda
-        and weight.device.index == torch.cuda.current_device()
-        and weight.dtype == torch.bfloat16
-        and weight.dim() == 2
-        and weight.is_contiguous()
-        and weight.data_ptr() % 16 == 0
-        and not (weight.requires_grad and torch.is_grad_enabled())
-        and torch._C._functorch.peek_interpreter_stack() is None
-        and torch.autograd.forward_ad._current_level < 0
-        and _use_native(weight)
-        and _EXT.projection_serves(rows, *weight.shape)
-    )
+    return type(weight) in _PLAIN and _product_native(weight) and _EXT.projection_takes(weight, rows)
 
 
 def _linear_here(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether x @ weight.T is for our kernels."""
-    return (
-        type(x) is torch.Tensor
-        and x.is_cuda
-        and x.device == weight.device
-        and x.dtype == torch.bfloat16
-        and x.dim() == 2
-        and x.shape[1] == weight.shape[-1]
-        and x.is_contiguous()
-        and x.data_ptr() % 16 == 0
-        and not (x.requires_grad and torch.is_grad_enabled())
-        and linear_served(x.shape[0], weight)
-    )
+    return (type(x) is torch.Tensor and type(weight) in _PLAIN and _product_native(x)
+            and _EXT.projection_takes_rows(x, weight))
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -504,11 +490,17 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, weight)
 
 
+def projection_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight.T as fp32 [parts, rows, outputs], of a weight and as many rows as
+    `linear_served` says."""
+    return _EXT.projection_parts(x, weight, _stream())
+
+
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """`linear` for a reader that adds up itself: fp32 [parts, rows, outputs], or
-    the rounded product where that is the library's."""
+    """`linear` for a reader that adds up itself: `projection_parts`, or the rounded
+    product where that is the library's."""
     if _linear_here(x, weight):
-        return _EXT.projection_parts(x, weight, _stream())
+        return projection_parts(x, weight)
     return torch.nn.functional.linear(x, weight)
 
 

@@ -235,6 +235,22 @@ void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optiona
                          silu, as_stream(stream));
 }
 
+// Whether the kernels of projection.hip take that many rows against w, in parts: what
+// Python would ask in a dozen attributes, ten times a layer (3 us each time)
+bool projection_takes(const torch::Tensor& w, int64_t rows) {
+  return w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() &&
+         ((uintptr_t)w.data_ptr() & 15) == 0 && !(w.requires_grad() && at::GradMode::is_enabled()) &&
+         lig_projection_serves(rows, w.size(0), w.size(1));
+}
+
+// and of the rows x
+bool projection_takes_rows(const torch::Tensor& x, const torch::Tensor& w) {
+  return x.is_cuda() && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && w.dim() == 2 &&
+         x.size(1) == w.size(1) && x.device() == w.device() && x.is_contiguous() &&
+         ((uintptr_t)x.data_ptr() & 15) == 0 && !(x.requires_grad() && at::GradMode::is_enabled()) &&
+         projection_takes(w, x.size(0));
+}
+
 // y = x W^T of up to 1024 rows (projection.hip); sizes that it does not serve are refused
 void projection(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t stream) {
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2);
@@ -815,6 +831,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);
   m.def("projection_serves", &lig_projection_serves);
+  m.def("projection_takes", &projection_takes);
+  m.def("projection_takes_rows", &projection_takes_rows);
   m.def("row_product", &row_product);
   m.def("row_product_max", &lig_row_product_max);
   m.def("paged_attention_decode", &paged_attention_decode);
