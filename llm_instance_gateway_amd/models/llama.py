@@ -56,9 +56,10 @@ def _project(m: nn.Module, x: torch.Tensor, product=ops.linear) -> torch.Tensor:
     return product(x, m._parameters["weight"]) if _product_alone(m) else m(x)
 
 
-def _served(m: nn.Module, rows: int) -> bool:
-    """Whether `_project` of that many rows runs on our kernels."""
-    return _product_alone(m) and ops.linear_served(rows, m._parameters["weight"])
+def _served(m: nn.Module, rows: int, parts: bool = True) -> bool:
+    """Whether `_project` of that many rows runs on our kernels, in parts or rounded."""
+    w = m._parameters.get("weight")
+    return _product_alone(m) and ops.linear_served(rows, w) and (parts or ops.linear_pays(rows, w))
 
 
 class Attention(nn.Module):
@@ -270,8 +271,12 @@ class LlamaForCausalLM(nn.Module):
         rows, not 1024).  Under 2^20 weights a projection takes its launch's time at
         either count, and the multiple stays."""
         attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
-        modules = [attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ())]
-        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 for m in modules]
+        # only gate_up's reader needs it rounded; under tensor parallelism all do
+        parts = self.tp is None
+        modules = [(attn.qkv_proj, parts), (attn.o_proj, parts)]
+        if type(mlp) is MLP:
+            modules += [(mlp.gate_up_proj, False), (mlp.down_proj, parts)]
+        served = [_served(m, tokens, p) and m.weight.numel() >= 1 << 20 for m, p in modules]
         if all(served):
             return tokens
         step = min(64, multiple) if any(served) else multiple

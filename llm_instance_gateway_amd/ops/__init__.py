@@ -480,10 +480,15 @@ def _linear_here(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and _EXT.projection_takes_rows(x, weight))
 
 
+def linear_pays(rows: int, weight: torch.Tensor) -> bool:
+    """Whether `linear` of served rows, which has to round, runs on them too."""
+    return _EXT.projection_pays(rows, *weight.shape)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """y = x @ weight.T (nn.Linear, no bias): the framework's kernel where it is
     the faster one, the library's elsewhere."""
-    if _linear_here(x, weight):
+    if _linear_here(x, weight) and linear_pays(x.shape[0], weight):
         y = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
         _EXT.projection(y, x, weight, _stream())
         return y

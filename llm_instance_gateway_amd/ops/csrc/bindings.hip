@@ -47,6 +47,7 @@ void lig_qkv_rope_cache_launch(uint16_t*, const uint16_t*, const int64_t*,
                                const int64_t*, int, int, int, int, int,
                                hipStream_t);
 bool lig_projection_serves(long, long, long);
+bool lig_projection_pays(long, long, long);
 int lig_projection_plan(int, int, int);
 int lig_projection_splits(int);
 int lig_projection_tile(int);
@@ -831,6 +832,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);
   m.def("projection_serves", &lig_projection_serves);
+  m.def("projection_pays", &lig_projection_pays);
   m.def("projection_takes", &projection_takes);
   m.def("projection_takes_rows", &projection_takes_rows);
   m.def("row_product", &row_product);

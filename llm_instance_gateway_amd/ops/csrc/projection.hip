@@ -285,14 +285,38 @@ Plan plan(int M, int N, int K) {
 
 extern "C" {
 
-// Whether these kernels are the ones to take: the library's large tiles are ahead
-// where they are enough for the chip (384 x 28672 x 4096: 101 us here, 80 there;
-// 786 x 6144 x 4096: 51 and 47), and behind where N needs a cut of K (786 x 4096 x
-// 14336: 100 and 118; 384: 57 and 77) or rows are few; and it is slower than its
-// large tiles could be on a vocabulary (384 x 128256 x 4096: 388 us here, 431 there).
+// Sizes that these kernels are for where their reader adds up the parts of K: the
+// library's large tiles are ahead where they are enough for the chip (384 x 28672 x
+// 4096: 101 us here, 80 there; 786 x 6144 x 4096: 51 and 47), and behind where N needs
+// a cut of K (786 x 4096 x 14336: 100 and 118; 384: 57 and 77) or rows are few; and it
+// is slower than its large tiles could be on a vocabulary (384 x 128256 x 4096: 388 us
+// here, 431 there).
 bool lig_projection_serves(long M, long N, long K) {
   if (M < 1 || M > 1024 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
   return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || (M <= 384 && N >= 65536);
+}
+
+// Whether a served product that has to come rounded, its parts added up by a launch
+// of its own, is the faster one here.  Drawn from 1912 products, N of 1024 to 128256,
+// K of 1024 to 28672, 22 row counts, weights from memory (us here, the library's):
+//   * to 128 rows it is, 1.3 times in the mean (100 x 28672 x 4096: 46, 56);
+//   * a vocabulary's worth of short rows of W is not (24 x 57344 x 1024: 35, 24);
+//   * to 256 rows it is where K is cut (160 x 4096 x 7168: 28, 46), by 1.3 in the mean.
+//     In one part it is where N makes about one full round of the chip (202 x 28672 x
+//     4096: 64, 67; 256: 75, 69, but the same in a step), not for fewer or longer tiles
+//     (256 x 4096 x 4096: 25.9, 22.8; 256 x 57344 x 8192: 263, 220);
+//   * above, only a cut into many parts gains more than its sum costs (384 x 4096 x
+//     14336: 64, 78; in two 448 x 6144 x 4096: 40, 33; in one 300 x 6144 x 4096: 37, 29).
+// Of smaller weights that is a few us, less than what the library's call takes longer
+// on the host, which steps of narrow models wait for: 300 rows, 16 layers of 2048
+// columns 2106 us, 2488 with the library's.
+bool lig_projection_pays(long M, long N, long K) {
+  if (M > 16 && N > 32768 && K < 2048) return false;
+  if (M <= 128 || N >= 65536 || N * K < 1L << 24) return true;
+  const int splits = plan((int)M, (int)N, (int)K).splits;
+  if (M > 256) return splits >= 4;
+  if (splits > 1) return splits > 2 || (N >= 4096 && N <= 16384);
+  return K <= 4096 && N >= 8192 && N <= 32768;
 }
 
 // Tile and parts of K, as one number.  To launch it: y alone where K is in one part,

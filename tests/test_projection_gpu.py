@@ -84,3 +84,14 @@ def test_another_device_stays_with_the_library(monkeypatch):
     assert ops.linear_served(8, w)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
     assert not ops.linear_served(8, w) and ops.linear_parts(x, w).dim() == 2
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 57344, 1024), (256, 4096, 4096), (256, 57344, 4096), (300, 6144, 4096),
+                                   (448, 6144, 4096), (1000, 4096, 4096)])
+def test_slower_rounded_products_stay_with_the_library(M, N, K):
+    """Sizes at which the parts pay for themselves only with a reader that adds them up."""
+    x = torch.randn(M, K, device="cuda").to(BF)
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).to(BF)
+    with torch.no_grad():
+        assert torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
+        assert ops.linear_served(M, w) and ops.linear_parts(x, w).dim() == 3
