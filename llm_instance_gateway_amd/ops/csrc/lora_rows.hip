@@ -511,6 +511,16 @@ LIG_DEVICE float factor_of(const Factor& f, int tile, int li) {
   return rsqrtf(total / f.width + f.eps);
 }
 
+// g / (1 + e^-g), the quotient as a division rounds it: corrected once by its
+// remainder (Markstein 1990), which v_rcp_f32's 1 ulp allows, both sides over 4 so
+// that no reciprocal is subnormal; v_div_fixup_f32 sees to infinities and NaN.  The
+// compiler's division takes twice the instructions.
+LIG_DEVICE float silu_of(float g) {
+  const float n = 0.25f * g, d = __builtin_fmaf(__expf(-g), 0.25f, 0.25f);
+  const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, n), r, q), d, n);
+}
+
 // out = silu(gate + B u) * (up + B u), u_out[strip] = A_down out.  Workgroups of
 // a tile take strips of 1024 of the d columns.
 constexpr int SILU_STRIP = 1024;
@@ -549,7 +559,7 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
       gv *= factor;
       uv *= factor;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = gv[j] / (1.0f + __expf(-gv[j])) * uv[j];
+      for (int j = 0; j < 8; ++j) r[j] = silu_of(gv[j]) * uv[j];
       const u16x8 rb = f32x8_to_bf16x8(r);
       if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
       if constexpr (LORA) acc = shrink(ar[i], rb, acc);

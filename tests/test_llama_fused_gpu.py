@@ -146,11 +146,25 @@ def test_lora_silu_divides(T):
     """Rows without an adapter come out as those of `silu_and_mul`, bit for bit."""
     rnd, rows, _ = _lora([-1] * T, T)
     x = (3 * rnd(T, 2 * 14336)).to(BF)
+    # where e^-g overflows, or nearly; the largest and smallest numbers, and none
+    edge = [-86.0, -87.0, -87.5, -88.0, -88.5, -89.0, -100.0, 100.0, 3e38, -3e38, 1e-38, -1e-38, 1e-40, 0.0, -0.0,
+            float("inf"), -float("inf"), float("nan")]
+    x[0, : len(edge)] = torch.tensor(edge, device="cuda").to(BF)
+    x[1, :14336] = torch.linspace(-95, 95, 14336, device="cuda").to(BF)
+    x[0, 14336 : 14336 + len(edge)] = 1
+
+    def bits(t):  # every NaN the same
+        return torch.where(t.isnan(), torch.tensor(1.5, device="cuda", dtype=BF), t).view(torch.int16)
+
+    def equal(a, b):
+        return torch.equal(a.isnan(), b.isnan()) and torch.equal(bits(a), bits(b))
+
     want = ops.silu_and_mul(x)
-    assert torch.equal(ops.lora_silu_and_mul(x, ops.BASE_ROWS, None, None, None, None), want)
+    assert want[0, :18].isnan().tolist() == [False] * 16 + [True] * 2
+    assert equal(ops.lora_silu_and_mul(x, ops.BASE_ROWS, None, None, None, None), want)
     u, a, b = rnd(1, len(rows[1]), 16, 16), rnd(1, 16, 14336).to(BF), rnd(1, 2 * 14336, 16).to(BF)
     ws = torch.empty(14, len(rows[1]), 16, 16, device="cuda")
-    assert torch.equal(ops.lora_silu_and_mul(x, rows, u, b, a, ws), want)
+    assert equal(ops.lora_silu_and_mul(x, rows, u, b, a, ws), want)
 
 
 @pytest.mark.parametrize("slots", SLOTS, ids=range(len(SLOTS)))
