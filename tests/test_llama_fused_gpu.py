@@ -282,15 +282,17 @@ def test_base_rows(T):
         assert ((p.float() - r).abs() <= 2.0 ** -8 * r.abs() + 2.0 ** -17 * q.abs().max() + 1e-5).all()
 
 
-def test_engine_matches_unit_kernels(monkeypatch):
+@pytest.mark.parametrize("hidden", [512, 2048])  # norms a workgroup per tile, and open
+def test_engine_matches_unit_kernels(monkeypatch, hidden):
     """A whole step through the in-layer kernels beside one through the SGMV
     kernels, prompts and decodes, eager and through the decode graph."""
     from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
     from llm_instance_gateway_amd.lora import manager
     from llm_instance_gateway_amd.models.config import ModelConfig
 
-    mc = ModelConfig(name="t", vocab_size=512, hidden_size=512, num_layers=3, num_heads=8, num_kv_heads=2,
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=hidden, num_layers=3, num_heads=8, num_kv_heads=2,
                      intermediate_size=768, head_dim=64, max_position_embeddings=512)
+    assert ops.lora_norm_opens(ops.BASE_ROWS, 129, hidden) == (hidden == 2048)
     outs = []
     for units in (False, True):
         monkeypatch.setattr(manager, "_TILED_SGMV", False)

@@ -15,6 +15,8 @@ SIZES = [
     (160, 4096, 1088), (193, 4096, 14336), (202, 28680, 128), (225, 12288, 4096), (256, 22016, 512), (255, 6144, 4096),
     (257, 1288, 8192), (384, 6144, 4096), (786, 4096, 14336), (1000, 4040, 4096), (1024, 16, 64),
     (130, 4096, 4096), (343, 6144, 8192), (241, 12296, 14336), (236, 28680, 1024), (384, 65544, 256),
+    (295, 8, 3072), (758, 136, 384), (833, 168, 512), (840, 8, 1344), (930, 152, 4288), (606, 4184, 4416),
+    (1023, 2456, 320), (168, 17656, 320), (197, 33128, 320), (212, 32968, 320),
 ]
 
 
@@ -24,22 +26,32 @@ def test_projection(M, N, K):
     x = torch.randn(M, K, generator=g, device="cuda").to(BF)
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(BF)
     assert ops.linear_served(M, w)
+    y = torch.empty(M, N, device="cuda", dtype=BF)  # by our kernel also where `linear` goes to the library
+    ops._EXT.projection(y, x, w, torch.cuda.current_stream().cuda_stream)
     with torch.no_grad():
-        got = ops.linear(x, w)
+        got, parts = ops.linear(x, w), ops.linear_parts(x, w)
     ref = x.double() @ w.double().t()
     # one rounding to 8 bits; 24-bit sums over K terms, whose errors walk
     size = (x.double().pow(2) @ w.double().pow(2).t()).sqrt()
-    tol = 2.0 ** -8 * ref.abs() + 2.0 ** -23 * K ** 0.5 * 4 * size
-    assert got.shape == (M, N) and got.dtype == BF
-    assert ((got.double() - ref).abs() <= tol).all()
+    sums = 2.0 ** -23 * K ** 0.5 * 4 * size
+    for v in (y, got):
+        assert v.shape == (M, N) and v.dtype == BF
+        assert ((v.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + sums).all()
+    # fp32, as many as K is cut into, each by the kernel that leaves sums
+    assert parts.shape == (ops._EXT.projection_plan(M, N, K)[2], M, N) and parts.dtype == torch.float32
+    assert ((parts.double().sum(0) - ref).abs() <= sums).all()
 
 
 def test_every_tile_is_reached():
+    """Each with its whole product rounded, which a size in one part runs, and with a
+    part's sums (`linear_parts` runs that kernel in one part as well)."""
     plan = ops._load_ext().projection_plan
     seen = {plan(*s) for s in SIZES}
-    wide = {plan(m, n, k)[:2] for m in range(1, 1025, 5) for n in (1280, 4096, 6144, 12288, 28672, 128256)
-            for k in (1024, 4096, 14336) if ops._EXT.projection_serves(m, n, k)}
-    assert {s[:2] for s in seen} >= wide
+    wide = {plan(m, n, k) for m in range(1, 1025, 5)
+            for n in (8, 136, 1024, 1280, 4096, 6144, 12288, 16872, 28672, 33128, 57344, 128256)
+            for k in (64, 128, 320, 512, 1024, 1344, 3072, 4096, 14336) if ops._EXT.projection_serves(m, n, k)}
+    kernels = lambda plans: {(m, n, cut > 1) for m, n, cut in plans}
+    assert len(kernels(wide)) == 34 and kernels(seen) >= kernels(wide)
     assert {s[2] for s in seen} >= {1, 2, 8}
 
 

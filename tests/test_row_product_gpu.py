@@ -72,6 +72,7 @@ def test_single_decode_matches_layer_kernels(monkeypatch):
     for row in (True, False):
         if not row:
             monkeypatch.setattr(LlamaForCausalLM, "_row_products", lambda self: False)
+            monkeypatch.setattr(LlamaForCausalLM, "_open_norms", lambda self, rows: False)
         torch.manual_seed(3)
         eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=32, max_num_seqs=2, max_num_batched_tokens=256,
                                      max_model_len=256), device="cuda")
