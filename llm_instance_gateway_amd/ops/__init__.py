@@ -17,6 +17,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import torch_ref
 
@@ -462,15 +463,22 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _product_native(t: torch.Tensor) -> bool:
-    """Whether no transform has to see the products of t, and t is where launches go."""
+    """Whether nothing has to see the products of t by their torch calls, and t is
+    where launches go.  (Dispatch modes, traces and transforms: projection_takes.)"""
     return (_use_native(t) and t.get_device() == torch.cuda.current_device()
-            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+            and torch.autograd.forward_ad._current_level < 0 and _default_device_alone())
+
+
+def _default_device_alone() -> bool:
+    """Whether no function mode is on but those of torch.device."""
+    n = torch._C._len_torch_function_stack()
+    return n == 0 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext) for i in range(n))
 
 
 def linear_served(rows: int, weight: torch.Tensor) -> bool:
     """Whether `linear_parts` runs that many rows on the kernels of projection.hip: not
-    where a derivative or a transform has to see the product, nor on another device
-    than the current one, whose stream a launch would go to."""
+    where a derivative, a transform, a trace or a mode has to see the product, nor on
+    another device than the current one, whose stream a launch would go to."""
     return type(weight) in _PLAIN and _product_native(weight) and _EXT.projection_takes(weight, rows)
 
 

@@ -8,6 +8,9 @@
 #include <optional>
 
 #include <torch/extension.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <pybind11/numpy.h>
 
 #include "common.h"
@@ -236,12 +239,18 @@ void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optiona
                          silu, as_stream(stream));
 }
 
+// Whether a dispatch mode, a trace or a transform follows what is called
+bool watched() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
 // Whether the kernels of projection.hip take that many rows against w, in parts: what
 // Python would ask in a dozen attributes, ten times a layer (3 us each time)
 bool projection_takes(const torch::Tensor& w, int64_t rows) {
   return w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() &&
          ((uintptr_t)w.data_ptr() & 15) == 0 && !(w.requires_grad() && at::GradMode::is_enabled()) &&
-         lig_projection_serves(rows, w.size(0), w.size(1));
+         !watched() && lig_projection_serves(rows, w.size(0), w.size(1));
 }
 
 // and of the rows x

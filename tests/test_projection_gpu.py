@@ -107,3 +107,27 @@ def test_slower_rounded_products_stay_with_the_library(M, N, K):
     with torch.no_grad():
         assert torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
         assert ops.linear_served(M, w) and ops.linear_parts(x, w).dim() == 3
+
+
+def test_watched_products_stay_with_the_library():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Calls(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            names.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    g = torch.Generator("cuda").manual_seed(4)
+    w, x, z = (torch.randn(n, 128, generator=g, device="cuda").to(BF) for n in (64, 8, 8))
+    want, names = torch.nn.functional.linear(z, w), []
+    with torch.no_grad():
+        with FlopCounterMode(display=False) as flops:
+            ops.linear(x, w)
+        assert flops.get_total_flops() == 2 * 8 * 64 * 128
+        assert torch.equal(torch.jit.trace(lambda v: ops.linear(v, w), x)(z), want)
+        with Calls():
+            ops.linear(x, w)
+        assert "linear" in names
+        with torch.device("cuda"):
+            assert ops.linear_served(8, w) and ops.linear_parts(x, w).dim() == 3
