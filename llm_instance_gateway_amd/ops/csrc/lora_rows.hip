@@ -568,11 +568,8 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
   return acc;
 }
 
-// 8 waves take a strip in one pass each, 4 in two.  Where the workgroups find a CU
-// each that is faster, and slower from there on.  Adapters' weights from memory, us with
-// 8 and 4 waves: 14336 columns, 8 tiles 8.6, 10.0; 16 9.3, 10.8; 24 18.2, 16.5; 64 of 32
-// adapters 36.3, 30.9; 240 130, 108.  8192 columns, 32 tiles 9.9, 11.2; 48 16.8, 15.3.
-// 28672 columns, 8 tiles 10.0, 11.5; 16 16.9, 15.8.
+// 8 waves take a strip in one pass each, 4 in two: 9 tiles 9.7 us (11.0 with 4), 13
+// 10.6 (12.0), 240 120 (108), where the chip is full either way.
 template <int W>
 __global__ __launch_bounds__(64 * W) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
@@ -824,7 +821,7 @@ void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* to
   hipLaunchKernelGGL((lora_silu_kernel<W>), dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(64 * W), 0, stream, \
                      out, x, d, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out,             \
                      Factor{sums, width, eps}, rows)
-  if (ntiles * ((d + SILU_STRIP - 1) / SILU_STRIP) <= 256) LAUNCH_A(8);
+  if (ntiles <= 64) LAUNCH_A(8);
   else LAUNCH_A(4);
 #undef LAUNCH_A
 }
