@@ -511,12 +511,12 @@ LIG_DEVICE float factor_of(const Factor& f, int tile, int li) {
   return rsqrtf(total / f.width + f.eps);
 }
 
-// g / (1 + e^-g), the quotient as a division rounds it: corrected once by its
-// remainder (Markstein 1990), which v_rcp_f32's 1 ulp allows, both sides over 4 so
+// g / (1 + e^-g) of n = g / 4, the quotient as a division rounds it: corrected once by
+// its remainder (Markstein 1990), which v_rcp_f32's 1 ulp allows, both sides over 4 so
 // that no reciprocal is subnormal; v_div_fixup_f32 sees to infinities and NaN.  The
 // compiler's division takes twice the instructions.
-LIG_DEVICE float silu_of(float g) {
-  const float n = 0.25f * g, d = __builtin_fmaf(__expf(-g), 0.25f, 0.25f);
+LIG_DEVICE float silu_of_quarter(float n) {
+  const float d = __builtin_fmaf(__builtin_amdgcn_exp2f(n * (-4.f * LOG2E)), 0.25f, 0.25f);
   const float r = __builtin_amdgcn_rcpf(d), q = n * r;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, n), r, q), d, n);
 }
@@ -556,10 +556,10 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
         gv += expand(bg[i], u);
         uv += expand(bu[i], u);
       }
-      gv *= factor;
+      gv *= 0.25f * factor;
       uv *= factor;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = silu_of(gv[j]) * uv[j];
+      for (int j = 0; j < 8; ++j) r[j] = silu_of_quarter(gv[j]) * uv[j];
       const u16x8 rb = f32x8_to_bf16x8(r);
       if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
       if constexpr (LORA) acc = shrink(ar[i], rb, acc);
