@@ -568,8 +568,11 @@ LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const ui
   return acc;
 }
 
-// 8 waves take a strip in one pass each, 4 in two: 9 tiles 9.7 us (11.0 with 4), 13
-// 10.6 (12.0), 240 120 (108), where the chip is full either way.
+// 8 waves take a strip in one pass each, 4 in two: faster where the workgroups find a
+// CU each, slower from there on, for a second of 8 waves fits a CU no more.  In steps of
+// 14 strips, 8 adapters (us with 8 and 4 waves): 96 decodes 10.6, 12.1; 256 (16 tiles)
+// 12.2, 18.4; 384 (24) 20.8, 19.2; prompts of 740 rows 30.9, 24.7; of 1108 50.6, 45.5; of
+// 1851 66.0, 61.4; 382 decodes and 2 prompts, 32 adapters 38.9, 31.8.
 template <int W>
 __global__ __launch_bounds__(64 * W) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
@@ -821,7 +824,10 @@ void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* to
   hipLaunchKernelGGL((lora_silu_kernel<W>), dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(64 * W), 0, stream, \
                      out, x, d, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out,             \
                      Factor{sums, width, eps}, rows)
-  if (ntiles <= 64) LAUNCH_A(8);
+  // A decode graph's list has room for one tile per adapter more than full ones, and of
+  // those few are in use where adapters have about as many requests each
+  const int likely = (ntiles + 3 * ((rows + 15) / 16)) / 4;
+  if (likely * ((d + SILU_STRIP - 1) / SILU_STRIP) <= 256) LAUNCH_A(8);
   else LAUNCH_A(4);
 #undef LAUNCH_A
 }

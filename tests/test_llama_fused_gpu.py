@@ -138,10 +138,10 @@ def test_lora_silu_and_mul(slots, d):
 
 
 def test_lora_silu_of_many_tiles():
-    test_lora_silu_and_mul([2] * 600 + [-1] * 300 + [0] * 200, 1056)  # 70 tiles: 4 waves a workgroup
+    test_lora_silu_and_mul([2] * 600 + [-1] * 300 + [0] * 200, 4128)  # 70 tiles of 5 strips: 4 waves a workgroup
 
 
-@pytest.mark.parametrize("T", [400, 1100])  # 8 and 4 waves a workgroup
+@pytest.mark.parametrize("T", [200, 1100])  # 8 and 4 waves a workgroup
 def test_lora_silu_divides(T):
     """Rows without an adapter come out as those of `silu_and_mul`, bit for bit."""
     rnd, rows, _ = _lora([-1] * T, T)
