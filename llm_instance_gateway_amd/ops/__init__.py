@@ -375,13 +375,16 @@ LORA_ROWS_WIDTHS = (256, 512, 1024, 2048, 3072, 4096)  # lora_rms_norm's
 
 
 # Below this many tiles of 4096 columns, and in proportion for narrower rows down
-# to 2048, lora_rms_norm takes strips of columns in two launches instead of a
-# workgroup per tile in one: few workgroups wait for one CU's loads, many read it
-# all twice.  Both products, replayed from a graph, strips and one launch in us:
-#   4096 columns  24 tiles 11.3, 22.8   72 22.6, 25.8   104 31.2, 26.3   200 54.8, 29.7
-#   3072          24       11.6, 18.6   72 18.0, 21.1   104 23.5, 21.8   200 44.7, 24.8
-#   2048          24       11.0, 12.6   48 11.6, 13.0    72 15.7, 13.5   104 17.5, 15.4
-#   1024          24       10.6,  7.7   72 11.1,  8.2;  512 24 10.5, 5.5
+# to 2048, norms take strips of 256 columns instead of a workgroup per tile in one
+# launch: few workgroups wait for one CU's loads.  lora_norm_open is one launch of
+# strips, lora_rms_norm two, which read all twice and set the line.  Both products,
+# replayed from a graph; open, two launches of strips, a workgroup per tile in us:
+#   4096 columns  24 tiles 6.9, 11.2, 22.9   84 13.6, 21.8, 24.7   104 15.4, 24.8, 24.9
+#                 128 17.6, 28.6, 25.2   200 30.3, 44.4, 30.9
+#   3072          24 6.8, 11.6, 18.8   72 11.3, 18.4, 20.3   96 13.2, 23.3, 20.7
+#   2048          24 4.9, 8.4, 12.7    48 7.0, 11.5, 13.2    72 8.6, 14.0, 13.7
+# (Above the line the open form would still be the faster one; there qkv and gate_up
+# are mostly the library's, and its reader in the rotation needs parts.)
 LORA_NORM_STRIPS_BELOW = 96
 
 

@@ -30,8 +30,8 @@
 // Measured, 32 query and 8 key/value heads of 128, before -> after: 384
 // requests of 190-381 tokens 173 -> 84 us (5.3 TB/s; a large copy reaches 4.9);
 // 33 of 3000-6000 370 -> 119 us (5.0 TB/s); 16 of 190-381 30 -> 8.2 us; 64 rows
-// with a window of 512 and sigmoid weights 54 -> 24.5 us (28.3 before values were
-// loaded as streams).  Eight waves per workgroup
+// with a window of 512 and sigmoid weights 54 -> 25.2 us (27.1 before values were
+// loaded as streams; on rows just read 23.5 either way).  Eight waves per workgroup
 // were slower from 64 requests on (101 us at 384), two on few (9.2 us at 16).
 #pragma once
 
@@ -513,9 +513,11 @@ static void launch_rows(const Args& a, hipStream_t stream) {
   // as far as the host can tell, and where rows are many: their caches don't stay in
   // the last-level cache from one step to the next.  One row of a few hundred keys has
   // them there, and a step of it is 1 % slower with streams; 8 rows on each of 32 tables
-  // of 1000 keys 83 -> 91 us.  Streamed: 64 rows of 1000 keys 47.7 -> 43.5 us, 40 of 300
-  // 15.1 -> 14.3, 64 with a window of 512 28.3 -> 24.5; all of 64 x 100 to 64 x 500 still
-  // cached: the same.  Keys too, whose lines take two loads, gives half of that back.
+  // of 1000 keys 83 -> 91 us.  Streamed, over 1 GB of caches in turn: 64 rows of 1000
+  // keys 47.9 -> 43.7 us, 384 of 286 84.0 -> 75.8, 32 of 4000 98.4 -> 89.8, 40 of 300
+  // 15.1 -> 14.6, 64 x 100 9.6 -> 9.3; with a window of 512 64 rows 27.1 -> 25.2, 32 rows
+  // 16.0 -> 15.0.  The same rows again (64 with the window, 134 MB): 23.1 -> 23.5.
+  // Keys too, whose lines take two loads, gives half of that back.
   const bool many = (long)a.rows * a.num_kv_heads >= 256 && a.rows <= a.tables;
 #define LIG_FD(LOWCOL, PB, STREAM)                                                                             \
   hipLaunchKernelGGL((flash_decode_kernel<D, W, LOWCOL, PB, STREAM, CAP, SIG, EXTRA>), grid, block, lds, stream, a)

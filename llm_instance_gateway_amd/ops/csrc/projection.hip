@@ -27,7 +27,7 @@
 //    384             (77)       56 ( 77)    26 ( 24)    33 ( 36)
 //    832                       103 (115 with tiles of 256 rows)
 //   1024                       115 (127)    41 ( 41)
-// A head of 128256 x 4096: 256 rows 253 (297), 384 rows 388 (431).
+// A head of 128256 x 4096: 256 rows 261 (295), 384 rows 409 (433).
 // gate_up at 48 rows reads W at 5.7 TB/s.  Where one tile holds all rows, loads of a
 // large W are non-temporal (`streams`): a step of 33 decodes with all its products
 // 2326 -> 2267 us, of a prompt of 202 rows 1793 -> 1753.
@@ -288,9 +288,9 @@ extern "C" {
 // Sizes that these kernels are for where their reader adds up the parts of K: the
 // library's large tiles are ahead where they are enough for the chip (384 x 28672 x
 // 4096: 101 us here, 80 there; 786 x 6144 x 4096: 51 and 47), and behind where N needs
-// a cut of K (786 x 4096 x 14336: 100 and 118; 384: 57 and 77) or rows are few; and it
-// is slower than its large tiles could be on a vocabulary (384 x 128256 x 4096: 388 us
-// here, 431 there).
+// a cut of K (786 x 4096 x 14336: 100 and 118; 384: 57 and 77) or rows are few.  On a
+// vocabulary of 128256 x 4096 it falls behind up to 384 rows: 256 rows 261 us here, 295
+// there; 320 399, 401; 384 409, 433; 448 491, 490; 640 709, 620.
 bool lig_projection_serves(long M, long N, long K) {
   if (M < 1 || M > 1024 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
   return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || (M <= 384 && N >= 65536);

@@ -150,8 +150,9 @@ extern "C" int lig_row_product_max(bool norm) { return norm ? NORM_MAX : PLAIN_M
 extern "C" void lig_row_product_launch(uint16_t* y, const uint16_t* w, int N, int K, const uint16_t* x,
                                        const uint16_t* residual, uint16_t* residual_out, const uint16_t* weight,
                                        float eps, bool silu, hipStream_t stream) {
-  // with a norm 8 waves share the h they form: 6144 x 4096 12.7 us (14.8 with 4
-  // waves), 12288 x 4096 20.5 (25.2), 24576 x 8192 72 (76), 3072 x 2048 8.1 (8.5)
+  // with a norm 8 waves share the h they form.  Measured with cached loads of W: 6144 x
+  // 4096 12.7 us (14.8 with 4 waves), 12288 x 4096 20.5 (25.2), 24576 x 8192 72 (76),
+  // 3072 x 2048 8.1 (8.5)
   const bool stream_w = streams(N, K);
 #define LIG_RP1(NTHR, NORM, SILU, STREAM)                                                                           \
   hipLaunchKernelGGL((row_product_kernel<NTHR, NORM, SILU, STREAM>),                                                \
