@@ -56,10 +56,9 @@ def _project(m: nn.Module, x: torch.Tensor, product=ops.linear) -> torch.Tensor:
     return product(x, m._parameters["weight"]) if _product_alone(m) else m(x)
 
 
-def _served(m: nn.Module, rows: int, parts: bool = True) -> bool:
-    """Whether `_project` of that many rows runs on our kernels, in parts or rounded."""
-    w = m._parameters.get("weight")
-    return _product_alone(m) and ops.linear_served(rows, w) and (parts or ops.linear_pays(rows, w))
+def _served(m: nn.Module, rows: int) -> bool:
+    """Whether `_project` of that many rows runs on our kernels, in parts."""
+    return _product_alone(m) and ops.linear_served(rows, m._parameters["weight"])
 
 
 class Attention(nn.Module):
@@ -273,12 +272,8 @@ class LlamaForCausalLM(nn.Module):
         800 prompt tokens 4.20 ms at 1024 rows, 3.85 at 832).  Under 2^20 weights a projection takes its launch's time at
         either count, and the multiple stays."""
         attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
-        # only gate_up's reader needs it rounded; under tensor parallelism all do
-        parts = self.tp is None
-        modules = [(attn.qkv_proj, parts), (attn.o_proj, parts)]
-        if type(mlp) is MLP:
-            modules += [(mlp.gate_up_proj, False), (mlp.down_proj, parts)]
-        served = [_served(m, tokens, p) and m.weight.numel() >= 1 << 20 for m, p in modules]
+        modules = [attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ())]
+        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 for m in modules]
         if all(served):
             return tokens
         step = min(64, multiple) if any(served) else multiple
