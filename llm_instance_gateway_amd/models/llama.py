@@ -266,14 +266,17 @@ class LlamaForCausalLM(nn.Module):
     def batch_rows(self, tokens: int, multiple: int) -> int:
         """Rows to pad a flat batch of tokens to.  The library's products want few,
         tile-friendly counts, those of `ops.linear` take any: none is added where
-        all of a layer's projections run there, few where some do (782 tokens: 832
-        rows, not 1024).  At such a count those left to the library miss its tuned
-        table, which knows multiples of 256: the rows saved are worth more (a step of
-        800 prompt tokens 4.20 ms at 1024 rows, 3.85 at 832).  Under 2^20 weights a projection takes its launch's time at
-        either count, and the multiple stays."""
+        all of a layer's projections run there (786 tokens: a step of 8B widths
+        takes 4.6 ms, 5.1 padded to 832 with qkv and gate_up at the library), few
+        where some do.  At such a count those left to the library miss its tuned
+        table, which knows multiples of 256: the rows saved are worth more.  Under
+        2^20 weights a projection takes its launch's time at either count, and the
+        multiple stays.  Sharded layers round every product, which has a rule of
+        its own."""
         attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
         modules = [attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ())]
-        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 for m in modules]
+        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 and (self.tp is None or ops.linear_pays(tokens, m.weight))
+                  for m in modules]
         if all(served):
             return tokens
         step = min(64, multiple) if any(served) else multiple

@@ -1,36 +1,21 @@
 // Projections of up to 1024 rows, gfx950, bf16: y = x W^T with x [M, K], W [N, K].
 //
-// Bound by how fast a CU gets its tiles: W once from HBM, x again for every tile
-// of W's rows from the L2.  A CU keeps about 32 KB of memory loads on their way,
-// whatever room it has for them, and they return in order, so the time of a step
-// of 64 columns is BN rows of W at the HBM's latency plus BM rows of x at the L2's
-// (2.9 and 2.0 ns a row), or the matrix products where those take longer (the tile
-// at 1.5 PFLOP/s over 256 CUs).  The launch picks tile and cut of K by that sum
-// (`plan`).  Therefore
-//   * rows go from memory straight into LDS, a ring of ST stages of PK * 64
-//     columns, XOR-swizzled through the choice of what a lane fetches (no bank
-//     conflicts, by the counter);
-//   * few rows get small tiles with the columns of a stage dealt to the waves
-//     (WK), whose sums meet in LDS;
-//   * XCDs start at different quarters of K: in step, all 256 CUs would ask for
-//     the same columns of rows 8 KB apart, that is for few memory channels
-//     (28672 x 4096, 48 rows: 41 us, 52 without).  Inside an XCD the CUs stay in
-//     step and find x in its L2; the tiles of an XCD lie side by side.
-//   * where N has too few tiles for the chip, K is cut into parts whose fp32 sums
-//     a second kernel adds up in order.
-// A deeper ring, one of 32-column stages, and operands read a product ahead into
-// registers brought nothing.
-// Llama-3-8B widths, weights not in any cache, against the library's products (us):
-//   rows            gate_up          down           o          qkv
-//     48         41 ( 60)       26 ( 37)    11 ( 15)    15 ( 17)
-//    202         59 ( 72)       42 ( 62)    19 ( 25)    25 ( 27)  (library at 256)
-//    384             (77)       56 ( 77)    26 ( 24)    33 ( 36)
-//    832                       103 (115 with tiles of 256 rows)
-//   1024                       115 (127)    41 ( 41)
-// A head of 128256 x 4096: 256 rows 261 (295), 384 rows 409 (433).
-// gate_up at 48 rows reads W at 5.7 TB/s.  Where one tile holds all rows, loads of a
-// large W are non-temporal (`streams`): a step of 33 decodes with all its products
-// 2326 -> 2267 us, of a prompt of 202 rows 1793 -> 1753.
+// Bound by how fast a CU gets its tiles, W once from HBM, x again for every tile of W's
+// rows from the L2, and with some hundred rows by the matrix products.  The launch picks
+// tile and cut of K by a sum of what these take (`plan`).
+//   * Rows go from memory straight into LDS, stages of 64 or 128 columns in a ring,
+//     XOR-swizzled through the choice of what a lane fetches (no bank conflicts, by the
+//     counter);
+//   * up to 32 rows of weights that are soon read: small tiles with the columns of a
+//     stage dealt to the waves, whose sums meet in LDS; else projection_wide_kernel;
+//   * XCDs start at different quarters of K: in step, all 256 CUs would ask for the same
+//     columns of rows 8 KB apart, that is for few memory channels.  Inside an XCD the CUs
+//     stay in step and find x in its L2; the tiles of an XCD lie side by side;
+//   * where N has too few tiles for the chip, K is cut into parts whose fp32 sums their
+//     reader, or a second kernel, adds up in order;
+//   * where one tile holds all rows, loads of a large W are non-temporal (`streams`).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -53,25 +38,61 @@ LIG_DEVICE void stages_landed(int behind) {
 
 constexpr int XCD_PHASES = 4;  // starting points in K
 
-// Tiles of BM x BN, WM x WN waves on them, times WK over the columns.
+// acc[i][j]: 16 columns i of W's tile by 16 rows j of x's, as the products leave them.
+// A lane holds row li of a tile's 16, 4 columns of it, 8 of a pair.
+template <int TM, int TN, bool PARTIAL>
+LIG_DEVICE void store_tile(const f32x4_t (&acc)[TN][TM], uint16_t* __restrict__ y, float* __restrict__ part, const int m_at,
+                           const int n_at, const int z, const int M, const int N) {
+  constexpr bool PAIRS = TN % 2 == 0;
+  const int li = threadIdx.x & 15, lg = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int m = m_at + j * 16 + li;
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < TN; i += PAIRS ? 2 : 1) {
+      const int n = n_at + i * 16 + lg * (PAIRS ? 8 : 4);
+      if (n >= N) continue;
+      if constexpr (PARTIAL) {
+        float* o = part + ((size_t)z * M + m) * N + n;
+        *reinterpret_cast<f32x4_t*>(o) = acc[i][j];
+        if constexpr (PAIRS) *reinterpret_cast<f32x4_t*>(o + 4) = acc[i + 1][j];
+      } else if constexpr (PAIRS) {
+        f32x8 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc[i][j][e];
+          v[4 + e] = acc[i + 1][j][e];
+        }
+        *reinterpret_cast<u16x8*>(y + (size_t)m * N + n) = f32x8_to_bf16x8(v);
+      } else {
+        u32x2 v;
+        v[0] = (uint32_t)f32_to_bf16(acc[i][j][0]) | ((uint32_t)f32_to_bf16(acc[i][j][1]) << 16);
+        v[1] = (uint32_t)f32_to_bf16(acc[i][j][2]) | ((uint32_t)f32_to_bf16(acc[i][j][3]) << 16);
+        *reinterpret_cast<u32x2*>(y + (size_t)m * N + n) = v;
+      }
+    }
+  }
+}
+
+// Few rows: tiles of BM x BN, each wave a quarter of a stage's 128 columns.
 // PARTIAL: fp32 sums of a part of K to part[z][M][N].
-template <int BM, int BN, int WM, int WN, int WK, int PK, int ST, bool PARTIAL>
-__global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void projection_kernel(
+template <int BM, int BN, int ST, bool PARTIAL>
+__global__ __launch_bounds__(256, 1) void projection_kernel(
     uint16_t* __restrict__ y, float* __restrict__ part, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const int M, const int N, const int K, const int mtiles, const int ntiles) {
-  constexpr int NW = WM * WN * WK;
+  constexpr int NW = 4, PK = 2;
   constexpr int ROWS = BN + BM;              // of a panel of 64 columns: W's, then x's
-  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+  constexpr int TM = BM / 16, TN = BN / 16;
   constexpr int NF = PK * ROWS / 8;          // fetches of 8 rows per stage
   constexpr int NI = (NF + NW - 1) / NW;     // of a wave; some of the last wave's may be done twice
   constexpr int STAGE = PK * ROWS * 64;
-  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && PK * 2 % WK == 0 && (ST - 2) * NI < 64, "");
-  constexpr int RING = ST * STAGE, SUMS = (WK - 1) * BM * BN * 2;  // in 16-bit units
+  static_assert(BM % 16 == 0 && BN % 16 == 0 && (ST - 2) * NI < 64, "");
+  constexpr int RING = ST * STAGE, SUMS = (NW - 1) * BM * BN * 2;  // in 16-bit units
   static_assert(RING <= 80 * 1024 && SUMS <= 80 * 1024, "LDS of a CU");
   __shared__ __align__(16) uint16_t sm[RING > SUMS ? RING : SUMS];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
 
   // blocks are dealt to the XCDs in turn; the tiles of one lie together
   const int total = gridDim.x, xcd = blockIdx.x & 7;
@@ -127,87 +148,239 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void projectio
   for (int s = 0; s < ST - 1; ++s)
     if (s < steps) fetch(s);
 
-  const int w_row = wn * TN * 16 + (PAIRS ? (li >> 2) * 8 + (li & 3) : li);
+  const int w_row = PAIRS ? (li >> 2) * 8 + (li & 3) : li;
   const int w_f = f_w(w_row);
-  const int x_row = BN + wm * TM * 16 + li;
+  const int x_row = BN + li;
+  const int c = (wave & 1) * 4 + lg;
   for (int s = 0; s < steps; ++s) {
     stages_landed<NI, ST - 2>(steps - 1 - s);  // and the stage before this one is free
     if (s + ST - 1 < steps) fetch(s + ST - 1);
-    const uint16_t* stage = sm + s % ST * STAGE;
+    const uint16_t* panel = sm + s % ST * STAGE + (wave >> 1) * ROWS * 64;
+    bf16x8_t a[TN], b[TM];
 #pragma unroll
-    for (int kk = 0; kk < PK * 2 / WK; ++kk) {
-      const int k32 = wk + kk * WK;
-      const uint16_t* panel = stage + (k32 >> 1) * ROWS * 64;
-      const int c = (k32 & 1) * 4 + lg;
-      bf16x8_t a[TN], b[TM];
+    for (int i = 0; i < TN; ++i) {
+      const int r = w_row + (PAIRS ? (i >> 1) * 32 + (i & 1) * 4 : i * 16);
+      a[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(panel + r * 64 + ((c ^ w_f) << 3)));
+    }
 #pragma unroll
-      for (int i = 0; i < TN; ++i) {
-        const int r = w_row + (PAIRS ? (i >> 1) * 32 + (i & 1) * 4 : i * 16);
-        a[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(panel + r * 64 + ((c ^ w_f) << 3)));
-      }
+    for (int j = 0; j < TM; ++j)
+      b[j] = __builtin_bit_cast(
+          bf16x8_t, *reinterpret_cast<const u32x4*>(panel + (x_row + j * 16) * 64 + ((c ^ (li & 7)) << 3)));
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j)
-        b[j] = __builtin_bit_cast(
-            bf16x8_t, *reinterpret_cast<const u32x4*>(panel + (x_row + j * 16) * 64 + ((c ^ (li & 7)) << 3)));
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+
+  float* sums = reinterpret_cast<float*>(sm) + lane * 4;
+  constexpr int WAVE = TM * TN * 256;
+  __syncthreads();
+  if (wave > 0) {
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < TM; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TM; ++j)
+        *reinterpret_cast<f32x4_t*>(sums + (wave - 1) * WAVE + (i * TM + j) * 256) = acc[i][j];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int k = 0; k < NW - 1; ++k)
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] += *reinterpret_cast<const f32x4_t*>(sums + k * WAVE + (i * TM + j) * 256);
+  store_tile<TM, TN, PARTIAL>(acc, y, part, m0, n0, z, M, N);
+}
+
+// c += a b with c in accumulation registers.  The compiler's own choice between them
+// and the others changed from one half of a step to the next, with copies of all of c.
+LIG_DEVICE void mfma_acc(f32x4_t& c, bf16x8_t a, bf16x8_t b) {
+  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+// It does not count the cycles to keep between other uses of c and these either.
+template <int TN, int TM>
+LIG_DEVICE void mfma_apart(f32x4_t (&c)[TN][TM]) {
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) asm volatile("" : "+a"(c[i][j]));
+  asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) asm volatile("" : "+a"(c[i][j]));
+}
+
+// Waits until no more of this wave's loads are on their way than those of the last
+// `left` stages, of which CX of x and CW of W can have been issued.
+template <int NX, int NWL, int CX, int CW>
+LIG_DEVICE void later_stages(int left) {
+  static_assert(CX * NX + CW * NWL < 64, "vmcnt has 6 bits");
+  if constexpr (CW == 0) {
+    loads_landed<0>();
+  } else {
+    if (left >= CW) loads_landed<CX * NX + CW * NWL>();
+    else later_stages<NX, NWL, (CX < CW - 1 ? CX : CW - 1), CW - 1>(left);
+  }
+}
+
+// Tiles of 64 rows and more: 2 x 2 waves, one per SIMD, each with a quarter of the
+// tile.  The one above needs two barriers' worth of waiting per step and reads every
+// row of x 2 to 4 times from LDS, W's as often; as four waves of larger quarters the reads
+// shrink to two thirds, and what other waves covered is laid out here by hand:
+//   * a step's products come in halves of 32 columns, and between them stand the reads
+//     of the next half's operands and the loads of later stages, evenly: neither the
+//     matrix cores nor the loads pause.  One barrier per step, at half time;
+//   * x has SX slots of 64 columns, W one more: its rows come from memory, x's from the
+//     L2.  With the whole LDS so used, two to three stages of W and one to five of x are
+//     on their way (a ring of two for both waited 0.5 us per step for its loads);
+//   * columns come 64 at a time, a full line of 128 bytes a row: 32 at a time, in a ring
+//     of finer grain, they arrived at little more than half the rate.
+// Llama-3-8B widths, weights not in any cache (us; kernel above -> this, the library):
+//   rows      gate_up               down                o                 qkv
+//    202   71 -> 55 ( 66)     36 -> 35 ( 57)     17 -> 15 (21)     22 -> 20 (25)
+//    384  110 -> 77 ( 79)     54 -> 49 ( 75)     23 -> 20 (24)     33 -> 29 (35)
+//    832  223 -> 172 (170)   103 -> 81 (128)     40 -> 33 (39)     56 -> 44 (47)
+// A head of 128256 x 4096: 202 rows 252 -> 197 (297), 384 rows 409 -> 333 (436).
+template <int BM, int BN, int SX, bool PARTIAL, bool STREAM>
+__global__ __launch_bounds__(256, 1) void projection_wide_kernel(
+    uint16_t* __restrict__ y, float* __restrict__ part, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+    const int M, const int N, const int K, const int mtiles, const int ntiles) {
+  constexpr int SW = SX + 1;
+  constexpr int TM = BM / 32, TN = BN / 32;  // 16 x 16 tiles of a wave, and its loads of 8 rows per stage
+  static_assert(BM % 32 == 0 && BN % 32 == 0 && TM * TN >= 4 && SX >= 2, "");
+  constexpr int XS = BM * 64, WS = BN * 64, X0 = SW * WS;
+  static_assert(X0 + SX * XS <= 80 * 1024, "LDS of a CU");
+  __shared__ __align__(16) uint16_t sm[X0 + SX * XS];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+
+  // as above: the tiles of an XCD lie together, XCDs start at different quarters of K
+  const int total = gridDim.x, xcd = blockIdx.x & 7;
+  const int t = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
+  const int mt = t % mtiles, nt = t / mtiles % ntiles, z = t / (mtiles * ntiles);
+  const int splits = total / (mtiles * ntiles);
+  const int m0 = mt * BM, n0 = nt * BN;
+  const int all = K / 64;
+  const int first = (int)((long)all * z / splits);
+  const int steps = (int)((long)all * (z + 1) / splits) - first;
+  const int shift = (xcd % XCD_PHASES) * steps / XCD_PHASES;
+
+  constexpr bool PAIRS = TN % 2 == 0;
+  auto f_w = [](int r) { return PAIRS ? (r & 3) | ((r >> 1) & 4) : r & 7; };
+  const uint32_t lds = lds_address(sm);
+  uint32_t xoff[TM], woff[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int r = (wave + i * 4) * 8 + (lane >> 3);
+    xoff[i] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)K * 2 + (((lane & 7) ^ (r & 7)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int r = (wave + i * 4) * 8 + (lane >> 3);
+    woff[i] = (uint32_t)min(r, N - 1 - n0) * (uint32_t)K * 2 + (((lane & 7) ^ f_w(r)) << 4);
+  }
+  const uint16_t* wp = w + (size_t)n0 * K + (size_t)first * 64;
+  const uint16_t* xp = x + (size_t)m0 * K + (size_t)first * 64;
+  auto at = [&](int step) {
+    const int a = step + shift;
+    return (size_t)(a >= steps ? a - steps : a) * 64;
+  };
+  auto fetch_x = [&](int step, int i) __attribute__((always_inline)) {
+    load_to_lds(xp + at(step), xoff[i], lds + (X0 + step % SX * XS + wave * 512) * 2 + i * 4096);
+  };
+  auto fetch_w = [&](int step, int i) __attribute__((always_inline)) {
+    const uint32_t to = lds + (step % SW * WS + wave * 512) * 2 + i * 4096;
+    if (STREAM) stream_to_lds(wp + at(step), woff[i], to);
+    else load_to_lds(wp + at(step), woff[i], to);
+  };
+
+  f32x4_t acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  mfma_apart(acc);
+
+  // loads go out in one order throughout: W(0), x(0), W(1), x(1), ...
+#pragma unroll
+  for (int s = 0; s < SX; ++s) {
+    if (s < steps) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) fetch_w(s, i);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fetch_x(s, i);
     }
   }
 
-  if constexpr (WK > 1) {
-    float* sums = reinterpret_cast<float*>(sm) + lane * 4;
-    constexpr int WAVE = TM * TN * 256;
-    __syncthreads();
-    if (wk > 0) {
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-          *reinterpret_cast<f32x4_t*>(sums + (wave - WM * WN) * WAVE + (i * TM + j) * 256) = acc[i][j];
+  const int w_row = wn * TN * 16 + (PAIRS ? (li >> 2) * 8 + (li & 3) : li);
+  const int w_f = f_w(w_row);
+  const int x_row = wm * TM * 16 + li;
+  const uint16_t* wl[2] = {sm + w_row * 64 + ((lg ^ w_f) << 3), sm + w_row * 64 + (((4 + lg) ^ w_f) << 3)};
+  const uint16_t* xl[2] = {sm + X0 + x_row * 64 + ((lg ^ (li & 7)) << 3), sm + X0 + x_row * 64 + (((4 + lg) ^ (li & 7)) << 3)};
+  bf16x8_t a[2][TN], b[2][TM];
+  // operand r of half kk of a stage: x's rows, then W's
+  auto read = [&](int kk, int ws, int xs, int r) __attribute__((always_inline)) {
+    if (r < TM) {
+      b[kk][r] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(xl[kk] + xs * XS + r * 16 * 64));
+    } else {
+      const int i = r - TM;
+      a[kk][i] = __builtin_bit_cast(
+          bf16x8_t, *reinterpret_cast<const u32x4*>(wl[kk] + ws * WS + (PAIRS ? (i >> 1) * 32 + (i & 1) * 4 : i * 16) * 64));
     }
-    __syncthreads();
-    if (wk > 0) return;
+  };
+  // The products of half kk of stage s.  READ: between them the operands of the half
+  // behind it, from slots ws and xs, over three quarters of the time; FETCH: the loads
+  // of stage s + SX, W's in the first half, into the slot of the stage before, x's in
+  // the second, into this one's, read by all at the barrier between.
+  constexpr int OPS = TM + TN, MM = TM * TN, BUSY = MM * 3 / 4;
+  auto half = [&](auto kk_, auto fetch_, auto read_, int s, int ws, int xs) __attribute__((always_inline)) {
+    constexpr int kk = decltype(kk_)::value;
+    constexpr bool FETCH = decltype(fetch_)::value, READ = decltype(read_)::value;
+    constexpr int LOADS = kk == 0 ? TN : TM;
 #pragma unroll
-    for (int k = 0; k < WK - 1; ++k)
+    for (int m = 0; m < MM; ++m) {
+      const int i = m / TM, j = m % TM;
+      mfma_acc(acc[i][j], a[kk][i], b[kk][j]);
+      if (READ) {
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-          acc[i][j] += *reinterpret_cast<const f32x4_t*>(sums + (k * WM * WN + wave) * WAVE + (i * TM + j) * 256);
-  }
-
-  // ---- lane: row li of a tile's 16, 4 columns of it, 8 of a pair -----------------------
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m = m0 + (wm * TM + j) * 16 + li;
-    if (m >= M) continue;
-#pragma unroll
-    for (int i = 0; i < TN; i += PAIRS ? 2 : 1) {
-      const int n = n0 + (wn * TN + i) * 16 + lg * (PAIRS ? 8 : 4);
-      if (n >= N) continue;
-      if constexpr (PARTIAL) {
-        float* o = part + ((size_t)z * M + m) * N + n;
-        *reinterpret_cast<f32x4_t*>(o) = acc[i][j];
-        if constexpr (PAIRS) *reinterpret_cast<f32x4_t*>(o + 4) = acc[i + 1][j];
-      } else if constexpr (PAIRS) {
-        f32x8 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = acc[i][j][e];
-          v[4 + e] = acc[i + 1][j][e];
-        }
-        *reinterpret_cast<u16x8*>(y + (size_t)m * N + n) = f32x8_to_bf16x8(v);
-      } else {
-        u32x2 v;
-        v[0] = (uint32_t)f32_to_bf16(acc[i][j][0]) | ((uint32_t)f32_to_bf16(acc[i][j][1]) << 16);
-        v[1] = (uint32_t)f32_to_bf16(acc[i][j][2]) | ((uint32_t)f32_to_bf16(acc[i][j][3]) << 16);
-        *reinterpret_cast<u32x2*>(y + (size_t)m * N + n) = v;
+        for (int r = (m * OPS + BUSY - 1) / BUSY; r < ((m + 1) * OPS + BUSY - 1) / BUSY && r < OPS; ++r) read(kk ^ 1, ws, xs, r);
       }
+      if (FETCH) {
+#pragma unroll
+        for (int r = (m * LOADS + MM - 1) / MM; r < ((m + 1) * LOADS + MM - 1) / MM && r < LOADS; ++r) {
+          if (kk == 0) fetch_w(s + SX, r);
+          else fetch_x(s + SX, r);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  constexpr std::integral_constant<int, 0> k0{};
+  constexpr std::integral_constant<int, 1> k1{};
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  later_stages<TM, TN, SX - 1, SX - 1>(steps - 1);
+#pragma unroll
+  for (int r = 0; r < OPS; ++r) read(0, 0, 0, r);
+  int s = 0;
+  for (; s + SX < steps; ++s) {
+    half(k0, yes, yes, s, s % SW, s % SX);
+    later_stages<TM, TN, SX - 2, SX - 1>(SX);  // the next stage is there; this one's operands have been read
+    half(k1, yes, yes, s, (s + 1) % SW, (s + 1) % SX);
   }
+  for (; s + 1 < steps; ++s) {
+    half(k0, no, yes, s, s % SW, s % SX);
+    later_stages<TM, TN, SX - 2, SX - 2>(steps - 2 - s);
+    half(k1, no, yes, s, (s + 1) % SW, (s + 1) % SX);
+  }
+  half(k0, no, yes, s, s % SW, s % SX);
+  half(k1, no, no, 0, 0, 0);
+  mfma_apart(acc);
+  store_tile<TM, TN, PARTIAL>(acc, y, part, m0 + wm * TM * 16, n0 + wn * TN * 16, z, M, N);
 }
 
 __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restrict__ y, const float* __restrict__ part,
@@ -219,35 +392,42 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   *reinterpret_cast<u16x8*>(y + e) = f32x8_to_bf16x8(s);
 }
 
-// BM, BN, WM, WN, WK, PK, ST: what is left of 40 shapes when those go that no size
-// of 12 projections and 21 row counts misses by more than a few per cent
-#define LIG_TILES(X)          \
-  X(16, 16, 1, 1, 4, 2, 8)    \
-  X(16, 32, 1, 1, 4, 2, 6)    \
-  X(32, 32, 1, 1, 4, 2, 8)    \
-  X(32, 64, 1, 4, 1, 1, 8)    \
-  X(64, 64, 2, 2, 1, 1, 6)    \
-  X(64, 128, 2, 4, 1, 1, 5)   \
-  X(96, 64, 2, 2, 1, 1, 5)    \
-  X(96, 96, 2, 2, 1, 1, 5)    \
-  X(128, 128, 2, 4, 1, 1, 4)  \
-  X(192, 64, 4, 2, 1, 1, 4)   \
-  X(192, 128, 4, 2, 1, 1, 3)  \
-  X(224, 128, 2, 4, 1, 1, 3)  \
-  X(128, 256, 2, 4, 1, 1, 3)  \
-  X(256, 96, 4, 2, 1, 1, 3)   \
-  X(208, 256, 1, 8, 1, 1, 2)  \
-  X(192, 256, 2, 4, 1, 1, 2)  \
-  X(256, 256, 2, 4, 1, 1, 2)
+// Few rows: BM, BN, ST of projection_kernel (4 waves over the columns, steps of 128).
+#define LIG_TILES(X) \
+  X(16, 16, 8)       \
+  X(16, 32, 6)       \
+  X(32, 32, 8)
+// Else BM, BN, SX of projection_wide_kernel.  What is left of 34 shapes when those go
+// that no size of 18 projections and 31 row counts misses by more than a few per cent:
+// the one picked is 1.8 % slower than the best of all in the mean.
+#define LIG_WIDE_TILES(X) \
+  X(64, 64, 5)            \
+  X(64, 96, 5)            \
+  X(64, 128, 4)           \
+  X(96, 128, 4)           \
+  X(128, 128, 3)          \
+  X(128, 192, 2)          \
+  X(128, 256, 2)          \
+  X(160, 128, 3)          \
+  X(160, 256, 2)          \
+  X(192, 256, 2)          \
+  X(224, 96, 3)           \
+  X(224, 128, 3)          \
+  X(224, 256, 2)          \
+  X(256, 256, 2)
 
 struct TileShape {
   int bm, bn, k_step;
 };
 constexpr TileShape TILES[] = {
-#define X(BM, BN, WM, WN, WK, PK, ST) {BM, BN, PK * 64},
+#define X(BM, BN, ST) {BM, BN, 128},
     LIG_TILES(X)
 #undef X
+#define X(BM, BN, SX) {BM, BN, 64},
+    LIG_WIDE_TILES(X)
+#undef X
 };
+constexpr int FEW = 3;  // tiles of the first kind
 constexpr int MAX_SPLITS = 8;
 constexpr int CUS = 256;
 
@@ -255,23 +435,36 @@ struct Plan {
   int tile, splits;
 };
 
-// Least estimated time, in us: launch; per round of workgroups, its steps of 64
-// columns, each the longer of fetching and multiplying; not below W from HBM; the
-// sums of a cut K.  The constants are a fit to 5500 measured times, within 8 % of
-// them; the tile picked was 1 % slower than the best one in the mean, 17 % at most.
+// What a kernel's time is made of, in us: per step of 64 columns of a tile its products,
+// its rows of W, its rows of x; launch, tile; W from memory at `hbm` TB/s; a cut of K
+// and, in millionths, every sum of it.  A fit to 17000 measured times, 6 % off them.
+struct Cost {
+  double area, w_row, x_row, step, launch, tile, hbm, cut, sum;
+};
+constexpr Cost FEW_COST = {0.0005405, -0.005728, -0.0135, 0.2466, 3.263, 0.1869, 8.987, -0.6106, 3.765};
+constexpr Cost WIDE_COST = {9.45e-06, 0.001368, 0.001277, 0.004109, 0.9942, 2.333, 7.596, -0.2958, 1.212};
+
+// Tiles of few rows are for small weights: 16 rows of 28672 x 4096 take 41 us on them, 36
+// on tiles of 64 x 128; of 4096 x 4096 both 7.7; of 2048 x 2048 4.1 and 4.7.  Tall tiles that
+// would be mostly padding were not measured.
 Plan plan(int M, int N, int K) {
+  // one wave of workgroups after the other, each over in a few us: 1 row of 128256 x 4096
+  // 149 us, 153 to 156 on the next best tiles; 8 rows of 57344 x 8192 140, 149; 16 rows level
+  if (M <= 8 && N > 32768 && K % TILES[0].k_step == 0) return {0, 1};
   Plan best = {-1, 0};
   double least = 0;
   for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
     const TileShape& s = TILES[i];
-    if (K % s.k_step) continue;
+    if (K % s.k_step || (i < FEW ? (long)N * K >= 1L << 24 : s.bm > 64 && 5 * M < 3 * s.bm)) continue;
+    const Cost& c = i < FEW ? FEW_COST : WIDE_COST;
     const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-    const double step = fmax(s.bm * s.bn * 2.08e-5, s.bn * 2.9e-3 + s.bm * 2.04e-3);
+    const double step = s.bm * s.bn * c.area + s.bn * c.w_row + s.bm * c.x_row + c.step;
+    const double stream = N * (double)K * 2e-6 / c.hbm;
     for (int splits = 1; splits <= MAX_SPLITS; ++splits) {
       if (splits > 1 && (tiles * splits > 2 * CUS + 88 || K / s.k_step / splits < 6)) break;
-      const long rounds = (tiles * splits + CUS - 1) / CUS;
-      double t = 3.3 + fmax(rounds * (K / 64.0 / splits * step + 0.2), N * (double)K * 2 / 5.9e6);
-      if (splits > 1) t += 2.4 + 2.1e-6 * splits * M * N;
+      const double work = (tiles * splits + CUS - 1) / CUS * (K / 64.0 / splits * step + c.tile);
+      double t = c.launch + sqrt(work * work + stream * stream);
+      if (splits > 1) t += c.cut + c.sum * 1e-6 * splits * M * N;
       if (best.tile < 0 || t < least) {
         least = t;
         best = {i, splits};
@@ -281,42 +474,75 @@ Plan plan(int M, int N, int K) {
   return best;
 }
 
+struct Product {
+  uint16_t* y;
+  float* part;
+  const uint16_t *x, *w;
+  int M, N, K;
+  hipStream_t stream;
+};
+
+template <int BM, int BN, int ST>
+void launch_few(const Product& p, int splits) {
+  const int mtiles = (p.M + BM - 1) / BM, ntiles = (p.N + BN - 1) / BN;
+  const dim3 grid(mtiles * ntiles * (p.part ? splits : 1)), block(256);
+#define LAUNCH(PARTIAL)                                                                                                \
+  hipLaunchKernelGGL((projection_kernel<BM, BN, ST, PARTIAL>), grid, block, 0, p.stream, p.y, p.part, p.x, p.w, p.M, p.N, \
+                     p.K, mtiles, ntiles)
+  if (p.part) LAUNCH(true);
+  else LAUNCH(false);
+#undef LAUNCH
+}
+
+template <int BM, int BN, int SX>
+void launch_wide(const Product& p, int splits) {
+  const int mtiles = (p.M + BM - 1) / BM, ntiles = (p.N + BN - 1) / BN;
+  const dim3 grid(mtiles * ntiles * (p.part ? splits : 1)), block(256);
+#define LAUNCH(PARTIAL, STREAM)                                                                                          \
+  hipLaunchKernelGGL((projection_wide_kernel<BM, BN, SX, PARTIAL, STREAM>), grid, block, 0, p.stream, p.y, p.part, p.x, p.w, \
+                     p.M, p.N, p.K, mtiles, ntiles)
+  const bool stream = mtiles == 1 && streams(p.N, p.K);  // no second workgroup reads these rows
+  if (p.part && stream) LAUNCH(true, true);
+  else if (p.part) LAUNCH(true, false);
+  else if (stream) LAUNCH(false, true);
+  else LAUNCH(false, false);
+#undef LAUNCH
+}
+
 }  // namespace
 
 extern "C" {
 
-// Sizes that these kernels are for where their reader adds up the parts of K: the
-// library's large tiles are ahead where they are enough for the chip (384 x 28672 x
-// 4096: 101 us here, 80 there; 786 x 6144 x 4096: 51 and 47), and behind where N needs
-// a cut of K (786 x 4096 x 14336: 100 and 118; 384: 57 and 77) or rows are few.  On a
-// vocabulary of 128256 x 4096 it falls behind up to 384 rows: 256 rows 261 us here, 295
-// there; 320 399, 401; 384 409, 433; 448 491, 490; 640 709, 620.
+// Sizes that these kernels are for where their reader adds up the parts of K.  Above 256
+// rows, from 3072 columns on, they take 0.6 to 1 of the library's time, of the largest
+// matrices 0.85 to 1.05 (384 rows: 6144 x 4096 29 us here, 35 there; 4096 x 14336 49, 75;
+// 28672 x 4096 77, 79; 960: 181, 175).  With many tiles of fewer columns neither is ahead
+// (16384 x 2048: 288 rows 24, 27; 384 29, 27).
 bool lig_projection_serves(long M, long N, long K) {
   if (M < 1 || M > 1024 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
-  return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || (M <= 384 && N >= 65536);
+  return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || K >= 3072 || (M <= 384 && N >= 65536);
 }
 
 // Whether a served product that has to come rounded, its parts added up by a launch
-// of its own, is the faster one here.  Drawn from 1912 products, N of 1024 to 128256,
-// K of 1024 to 28672, 22 row counts, weights from memory (us here, the library's):
-//   * to 128 rows it is, 1.3 times in the mean (100 x 28672 x 4096: 46, 56);
-//   * a vocabulary's worth of short rows of W is not (24 x 57344 x 1024: 35, 24);
-//   * to 256 rows it is where K is cut (160 x 4096 x 7168: 28, 46), by 1.3 in the mean.
-//     In one part it is where N makes about one full round of the chip (202 x 28672 x
-//     4096: 64, 67; 256: 75, 69, but the same in a step), not for fewer or longer tiles
-//     (256 x 4096 x 4096: 25.9, 22.8; 256 x 57344 x 8192: 263, 220);
-//   * above, only a cut into many parts gains more than its sum costs (384 x 4096 x
-//     14336: 64, 78; in two 448 x 6144 x 4096: 40, 33; in one 300 x 6144 x 4096: 37, 29).
-// Of smaller weights that is a few us, less than what the library's call takes longer
-// on the host, which steps of narrow models wait for: 300 rows, 16 layers of 2048
-// columns 2106 us, 2488 with the library's.
+// of its own, runs here too (us here, the library's):
+//   * to 128 rows it does (100 x 28672 x 4096: 42, 52), not a vocabulary's worth of short
+//     rows of W, 24 x 57344 x 1024;
+//   * to 256 rows where K is cut (202 x 4096 x 14336: 41, 57; 202 x 4096 x 4096: 19, 21, but
+//     256 of these 20, 22 with a launch more) or the weight large (202 x 28672 x 4096: 55, 66;
+//     202 x 57344 x 8192: 179, 215);
+//   * above, large weights do at any row count (384 x 4096 x 14336: 54, 75; 384 x 28672 x
+//     4096: 77, 79) and others where K is cut into many parts.  What is left gains a few us
+//     at most (1000 x 4096 x 4096: 36, 39; 448 x 6144 x 4096: 31, 33).
+// Of smaller weights the library's call takes longer on the host than is gained, which steps
+// of narrow models wait for: 300 rows, 16 layers of 2048 columns 2106 us, 2488 with its
+// products.
 bool lig_projection_pays(long M, long N, long K) {
   if (M > 16 && N > 32768 && K < 2048) return false;
   if (M <= 128 || N >= 65536 || N * K < 1L << 24) return true;
   const int splits = plan((int)M, (int)N, (int)K).splits;
-  if (M > 256) return splits >= 4;
-  if (splits > 1) return splits > 2 || (N >= 4096 && N <= 16384);
-  return K <= 4096 && N >= 8192 && N <= 32768;
+  if (M > 256) return splits >= 4 || N * K >= 1L << 25;
+  if (splits > 1) return (K > N || M <= 224 || N >= 6144) && (splits > 2 || (N >= 4096 && N <= 16384));
+  return (K <= 4096 && N >= 8192 && N <= 32768) || N * K >= 1L << 28;
 }
 
 // Tile and parts of K, as one number.  To launch it: y alone where K is in one part,
@@ -333,17 +559,14 @@ void lig_projection_launch(int p, uint16_t* y, float* part, const uint16_t* x, c
                            hipStream_t stream) {
   const int tile = p / (MAX_SPLITS + 1), splits = p % (MAX_SPLITS + 1);
   int i = 0;
-#define X(BM, BN, WM, WN, WK, PK, ST)                                                                             \
-  if (tile == i++) {                                                                                              \
-    const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;                                             \
-    if (part)                                                                                                     \
-      hipLaunchKernelGGL((projection_kernel<BM, BN, WM, WN, WK, PK, ST, true>), dim3(mtiles * ntiles * splits),   \
-                         dim3(64 * WM * WN * WK), 0, stream, y, part, x, w, M, N, K, mtiles, ntiles);             \
-    else                                                                                                          \
-      hipLaunchKernelGGL((projection_kernel<BM, BN, WM, WN, WK, PK, ST, false>), dim3(mtiles * ntiles),           \
-                         dim3(64 * WM * WN * WK), 0, stream, y, part, x, w, M, N, K, mtiles, ntiles);             \
-  }
+  const Product a = {y, part, x, w, M, N, K, stream};
+#define X(BM, BN, ST) \
+  if (tile == i++) launch_few<BM, BN, ST>(a, splits);
   LIG_TILES(X)
+#undef X
+#define X(BM, BN, SX) \
+  if (tile == i++) launch_wide<BM, BN, SX>(a, splits);
+  LIG_WIDE_TILES(X)
 #undef X
   if (part && y) {
     const long n = (long)M * N;

@@ -17,6 +17,8 @@ SIZES = [
     (130, 4096, 4096), (343, 6144, 8192), (241, 12296, 14336), (236, 28680, 1024), (384, 65544, 256),
     (295, 8, 3072), (758, 136, 384), (833, 168, 512), (840, 8, 1344), (930, 152, 4288), (606, 4184, 4416),
     (1023, 2456, 320), (168, 17656, 320), (197, 33128, 320), (212, 32968, 320),
+    (1, 928, 6400), (19, 712, 6400), (97, 4184, 4096), (129, 16648, 2112), (130, 16632, 64), (257, 23200, 3072),
+    (451, 21792, 3072),
 ]
 
 
@@ -53,6 +55,13 @@ def test_every_tile_is_reached():
     kernels = lambda plans: {(m, n, cut > 1) for m, n, cut in plans}
     assert len(kernels(wide)) == 34 and kernels(seen) >= kernels(wide)
     assert {s[2] for s in seen} >= {1, 2, 8}
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
+@pytest.mark.parametrize("M,N", [(60, 8200), (64, 1032), (130, 16632), (136, 11136), (200, 4104), (250, 70000)])
+def test_fewer_stages_than_the_ring(M, N, K):
+    """Column counts around the depths of the rings: what is loaded ahead and what a step waits for differ."""
+    test_projection(M, N, K)
 
 
 def test_other_calls_stay_with_the_library():
