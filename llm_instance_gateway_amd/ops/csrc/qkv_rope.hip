@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(
     uint16_t* __restrict__ v_cache,
     const int64_t* __restrict__ slot_mapping,  // [T], negative: not cached
     const int num_tokens, const int num_q_heads, const int num_kv_heads, const int head_dim,
-    const int block_size) {
+    const int block_size, const int block_shift) {
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int parts = head_dim / 64;  // of 32 pairs
   const int wid = blockIdx.y * 4 + (threadIdx.x >> 6);
@@ -50,8 +50,9 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(
     }
   }
   const int64_t slot = slot_mapping[row];
-  const size_t blk = slot < 0 ? 0 : slot / block_size;
-  const size_t off = slot < 0 ? 0 : slot % block_size;
+  // a division of 64 bits is some hundred instructions
+  const size_t blk = slot < 0 ? 0 : block_shift >= 0 ? slot >> block_shift : slot / block_size;
+  const size_t off = slot < 0 ? 0 : slot - (int64_t)blk * block_size;
 
   const uint16_t* src = qkv + ((size_t)row * heads + h0) * head_dim + c;
   u16x8 x[QR_HEADS][2];
@@ -98,5 +99,5 @@ extern "C" void lig_qkv_rope_cache_launch(uint16_t* q_out, const uint16_t* qkv, 
   const int waves = (head_dim / 64) * ((heads + QR_HEADS - 1) / QR_HEADS);
   hipLaunchKernelGGL(qkv_rope_cache_kernel, dim3((num_tokens + 15) / 16, (waves + 3) / 4), dim3(256), 0, stream, q_out,
                      qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_tokens, num_q_heads, num_kv_heads,
-                     head_dim, block_size);
+                     head_dim, block_size, shift_of(block_size));
 }

@@ -492,3 +492,31 @@ def test_hooks_are_captured(lora):
         logits[eager] = out
     for a, b in zip(logits[False], logits[True]):
         assert (a - b).norm() <= 0.03 * b.norm()  # two orders of bf16 rounding
+
+
+@pytest.mark.parametrize("parts", range(1, 10))
+def test_every_number_of_parts(parts):
+    """Norm and rotation add up a product in any number of parts, in order: the same
+    24-bit sums as torch's, rounded once; cache blocks of 16 and of 6 tokens."""
+    g = torch.Generator(device="cuda").manual_seed(parts)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    T, H = 19, 2048
+    x, res, w = rnd(parts, T, H), rnd(T, H).to(BF), (1 + 0.1 * rnd(H)).to(BF)
+    s = x[0].clone()
+    for p in x[1:]:
+        s += p
+    residual = res.clone()
+    h, _, norm = ops.lora_norm_open(x, residual, w, 1e-5, ops.BASE_ROWS)
+    assert torch.equal(residual, (s + res.float()).to(BF))
+    one = ops.lora_norm_open(s[None].contiguous(), res.clone(), w, 1e-5, ops.BASE_ROWS)[0]
+    assert torch.equal(h, one)
+    cs = ops.build_cos_sin_cache(128, 500, 1e4, "cuda").float()
+    pos, at = torch.arange(T, device="cuda") * 20, torch.randperm(144, device="cuda")[:T]
+    for bs in (16, 6):
+        out = []
+        for y in (x, s[None].contiguous()):
+            kc, vc = torch.zeros(144 // bs, 4, bs, 128, dtype=BF, device="cuda"), torch.zeros(144 // bs, 4, bs, 128, dtype=BF, device="cuda")
+            q = ops.lora_qkv_rope_cache(y, pos, cs, kc, vc, at, 8, ops.BASE_ROWS, None, None, norm)
+            out.append((q, kc, vc))
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
