@@ -45,6 +45,36 @@ def pack_decodes(seqs: list, block_size: int, ids: np.ndarray, positions: np.nda
     pack_rows([q.block_table for q in seqs], tables)
 
 
+def decode_slots(positions, tables, block_size: int, slots, context) -> None:
+    """slots[i], the cache slot of row i's position by its row of `tables`;
+    context[i], that position + 1."""
+    ext = ops._load_ext()
+    if ext is not None:
+        ext.decode_slots(positions, tables, block_size, slots, context)
+        return
+    at = positions // block_size
+    slots[:] = tables[np.arange(len(positions)), at].astype(np.int64) * block_size + positions - at * block_size
+    context[:] = positions + 1
+
+
+def decode_lora_rows(seqs: list, slot_of, rows: int, toks, length, slot) -> None:
+    """`lora.manager.build_lora_rows` of a decode bucket: row i is sequence i,
+    rows past them have no adapter; places past the last tile are empty tiles."""
+    ext = ops._load_ext()
+    if ext is not None:
+        ext.decode_lora_rows(seqs, slot_of, rows, toks, length, slot)
+        return
+    from ..lora.manager import build_lora_rows
+
+    of = {name: slot_of(name) if name and slot_of is not None else -1 for name in {q.lora_name for q in seqs}}
+    slots = np.full(rows, -1, dtype=np.int32)
+    slots[: len(seqs)] = [of[q.lora_name] for q in seqs]
+    tok, n, s = build_lora_rows(slots)
+    u = len(n)
+    toks[:u], length[:u], slot[:u] = tok, n, s
+    toks[u:], length[u:], slot[u:] = 0, 0, -1
+
+
 def table_rows(rows: Seq[List[int]]) -> np.ndarray:
     """int32 [len(rows), longest], zero past a row's end."""
     out = np.zeros((len(rows), max(len(r) for r in rows)), dtype=np.int32)

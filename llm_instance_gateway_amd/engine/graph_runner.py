@@ -28,7 +28,7 @@ from typing import Dict, List, Optional
 import numpy as np
 import torch
 
-from .batch_arrays import device_view, lay_out, pack_decodes
+from .batch_arrays import decode_lora_rows, decode_slots, device_view, lay_out, pack_decodes
 from .metadata import BatchMeta
 
 log = logging.getLogger(__name__)
@@ -281,32 +281,26 @@ class DecodeGraphRunner:
         x.block_tables[:] = 0  # another bucket's arrays lay here
         pack_decodes(seqs, bs, x.ids[:n], x.pos[:n], x.block_tables[:n])
         x.block_tables[n:, 0] = self.scratch_block
-        at = x.pos // bs
-        x.slot_mapping[:] = x.block_tables[np.arange(B), at].astype(np.int64) * bs + x.pos - at * bs
-        x.context_lens[:] = x.pos + 1
+        decode_slots(x.pos, x.block_tables, bs, x.slot_mapping, x.context_lens)
         if self.seq_tables:
             x.seg_slot[:n] = [max(q.state_slot, 0) for q in seqs]
             x.seg_slot[n:] = self.scratch_slot
             x.seg_fresh[:] = x.pos == 0
-        if self.with_lora:
-            from ..lora.manager import build_lora_rows, build_lora_units
+        if self.with_lora and self.lora_in_layer:
+            decode_lora_rows(seqs, slot_of, B, x.lora_tok, x.lora_len, x.lora_slot)
+        elif self.with_lora:
+            from ..lora.manager import build_lora_units
 
             slots = np.full(B, -1, dtype=np.int32)
             of = {name: slot_of(name) if name else -1 for name in {q.lora_name for q in seqs}}
             slots[:n] = [of[q.lora_name] for q in seqs]
-            if self.lora_in_layer:
-                toks, ulen, uslot = build_lora_rows(slots)
-                u = len(ulen)
-                x.lora_tok[:u] = toks
-                x.lora_tok[u:] = 0
-            else:
-                x.lora_slots[:] = slots
-                x.lora_order[:], ut0, ulen, uslot = build_lora_units(slots)
-                u = len(ut0)
-                x.lora_t0[:u] = ut0
-                x.lora_t0[u:] = 0
+            x.lora_slots[:] = slots
+            x.lora_order[:], ut0, ulen, uslot = build_lora_units(slots)
+            u = len(ut0)
+            x.lora_t0[:u] = ut0
+            x.lora_t0[u:] = 0
             x.lora_len[:u] = ulen
-            x.lora_len[u:] = 0  # padding tiles or units: no-op in the kernels
+            x.lora_len[u:] = 0  # padding units: no-op in the kernels
             x.lora_slot[:u] = uslot
             x.lora_slot[u:] = -1
         v.to.copy_(v.src, non_blocking=True)

@@ -464,8 +464,15 @@ class ModelRunner:
             self.adapter_manager.slot_of if self.adapter_manager is not None else None
         )
         logits = gr.run(decodes, slot_of)
+        # what the host has to do anyway, while the GPU is at it
         seqs = [ss.seq for ss in decodes]
-        tokens = sample_tokens(logits, seqs)
-        for ss in decodes:
-            ss.seq.num_computed_tokens += 1
-        return {seq.seq_id: tok for seq, tok in zip(seqs, tokens)}
+        ids = [seq.seq_id for seq in seqs]
+        for seq in seqs:
+            seq.num_computed_tokens += 1
+        try:
+            tokens = sample_tokens(logits, seqs)
+        except BaseException:
+            for seq in seqs:
+                seq.num_computed_tokens -= 1
+            raise
+        return dict(zip(ids, tokens))

@@ -5,13 +5,19 @@
 // serialize correctly with the library GEMMs on torch's stream without
 // depending on the HIP/CUDA stream-masquerading ATen headers.
 
+#include <algorithm>
+#include <map>
 #include <optional>
+#include <vector>
 
 #include <torch/extension.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <pybind11/numpy.h>
+#if PY_VERSION_HEX < 0x030B0000
+#include <longintrepr.h>
+#endif
 
 #include "common.h"
 
@@ -791,6 +797,10 @@ static void pack_decodes(py::list seqs, int64_t block_size, py::array_t<int64_t>
     return py::reinterpret_steal<py::object>(v);
   };
   auto number = [](PyObject* e) {
+#if PY_VERSION_HEX < 0x030B0000
+    // one digit, as cache blocks and tokens are: read in place, a fifth of the call's time
+    if (PyLong_CheckExact(e) && (size_t)Py_SIZE(e) <= 1) return (long long)(Py_SIZE(e) ? ((PyLongObject*)e)->ob_digit[0] : 0);
+#endif
     const long long v = PyLong_Check(e) ? PyLong_AsLongLong(e) : py::reinterpret_borrow<py::object>(e).cast<long long>();
     if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
     return v;
@@ -826,6 +836,78 @@ static void pack_decodes(py::list seqs, int64_t block_size, py::array_t<int64_t>
   }
 }
 
+// Cache slot and context length of a decode bucket's rows, from their positions and tables.
+static void decode_slots(py::array_t<int64_t> positions, py::array_t<int32_t> tables, int64_t block_size,
+                         py::array_t<int64_t> slots, py::array_t<int32_t> context) {
+  const ssize_t n = positions.size();
+  TORCH_CHECK(block_size > 0 && positions.ndim() == 1 && tables.ndim() == 2 && tables.shape(0) == n && slots.ndim() == 1 &&
+              slots.shape(0) == n && context.ndim() == 1 && context.shape(0) == n);
+  for (const py::array* a : {(py::array*)&positions, (py::array*)&tables, (py::array*)&slots, (py::array*)&context})
+    TORCH_CHECK(a->flags() & py::array::c_style, "in row order");
+  const int64_t* at = positions.data();
+  const int32_t* row = tables.data();
+  int64_t* slot = slots.mutable_data();
+  int32_t* ctx = context.mutable_data();
+  const ssize_t width = tables.shape(1);
+  for (ssize_t i = 0; i < n; ++i, row += width) {
+    const int64_t b = at[i] / block_size;
+    if (at[i] < 0 || b >= width) throw py::index_error("a position past its row of blocks");
+    slot[i] = row[b] * block_size + (at[i] - b * block_size);
+    ctx[i] = (int32_t)(at[i] + 1);
+  }
+}
+
+// lora/manager.py's tiles of a decode bucket: its rows by adapter slot (slot_of(name), -1
+// for rows past the sequences), up to 16 a tile; the tiles past the last one empty.
+// Returns their number.
+static int64_t decode_lora_rows(py::list seqs, py::object slot_of, int64_t rows, py::array_t<int32_t> toks,
+                                py::array_t<int32_t> len, py::array_t<int32_t> slot) {
+  const ssize_t n = py::len(seqs), room = len.size();
+  TORCH_CHECK(rows >= n && toks.ndim() == 2 && toks.shape(0) == room && toks.shape(1) == 16 && len.ndim() == 1 &&
+              slot.ndim() == 1 && slot.shape(0) == room);
+  for (const py::array* a : {(py::array*)&toks, (py::array*)&len, (py::array*)&slot})
+    TORCH_CHECK(a->flags() & py::array::c_style, "in row order");
+  static PyObject* name_attr = PyUnicode_InternFromString("lora_name");
+  std::map<int, std::vector<int32_t>> by_slot;
+  py::dict known;  // name -> slot, asked once per name
+  for (ssize_t i = 0; i < n; ++i) {
+    PyObject* v = PyObject_GetAttr(PyList_GET_ITEM(seqs.ptr(), i), name_attr);
+    if (!v) throw py::error_already_set();
+    const py::object name = py::reinterpret_steal<py::object>(v);
+    PyObject* found = PyDict_GetItemWithError(known.ptr(), v);
+    if (!found && PyErr_Occurred()) throw py::error_already_set();
+    int at;
+    if (found) {
+      at = (int)PyLong_AsLong(found);
+    } else {
+      const int truth = PyObject_IsTrue(v);
+      if (truth < 0) throw py::error_already_set();
+      at = truth && !slot_of.is_none() ? slot_of(name).cast<int>() : -1;
+      known[name] = at;
+    }
+    by_slot[at].push_back((int32_t)i);
+  }
+  for (ssize_t i = n; i < rows; ++i) by_slot[-1].push_back((int32_t)i);
+  int32_t *tok = toks.mutable_data(), *l = len.mutable_data(), *s = slot.mutable_data();
+  ssize_t t = 0;
+  for (const auto& [at, of] : by_slot) {
+    for (size_t first = 0; first < of.size(); first += 16, ++t) {
+      TORCH_CHECK(t < room, "more tiles than room");
+      const int m = (int)std::min<size_t>(16, of.size() - first);
+      for (int j = 0; j < 16; ++j) tok[t * 16 + j] = of[first + std::min(j, m - 1)];
+      l[t] = m;
+      s[t] = at;
+    }
+  }
+  const ssize_t used = t;
+  for (; t < room; ++t) {
+    std::fill(tok + t * 16, tok + t * 16 + 16, 0);
+    l[t] = 0;
+    s[t] = -1;
+  }
+  return used;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "MI355X (gfx950) native kernels for llm_instance_gateway_amd";
   m.def("rms_norm", &rms_norm);
@@ -837,6 +919,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("argmax_rows", &argmax_rows);
   m.def("pack_decodes", &pack_decodes, py::arg("seqs"), py::arg("block_size"), py::arg("ids").noconvert(),
         py::arg("positions").noconvert(), py::arg("tables").noconvert());
+  m.def("decode_slots", &decode_slots, py::arg("positions").noconvert(), py::arg("tables").noconvert(), py::arg("block_size"),
+        py::arg("slots").noconvert(), py::arg("context").noconvert());
+  m.def("decode_lora_rows", &decode_lora_rows, py::arg("seqs"), py::arg("slot_of"), py::arg("rows"), py::arg("toks").noconvert(),
+        py::arg("len").noconvert(), py::arg("slot").noconvert());
   m.def("projection", &projection);
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);

@@ -55,6 +55,16 @@ def test_pack_decodes(path):
     assert tab.tolist() == [[4, -7, -7, -7], [1, 2**31 - 1, -7, -7], [9, 3, 6, -7]]
 
 
+def test_pack_decodes_reads_numbers_of_any_kind(path):
+    """of one digit inside, of more, negative, zero, numpy's and truth values"""
+    seqs = [_decode(2, [b, 0]) for b in (2**30 - 1, 2**30, -1, 0, np.int64(6), True)]
+    for s, t in zip(seqs, (2**40, -5, 0, 2**30, np.int32(3), False)):
+        s.prompt_token_ids[2] = t
+    ids, pos, tab = np.zeros(6, np.int64), np.zeros(6, np.int64), np.full((6, 2), -7, np.int32)
+    ba.pack_decodes(seqs, 4, ids, pos, tab)
+    assert tab[:, 0].tolist() == [2**30 - 1, 2**30, -1, 0, 6, 1] and ids.tolist() == [2**40, -5, 0, 2**30, 3, 0]
+
+
 @pytest.mark.parametrize("computed,blocks,room", [(4, [1], 4), (2, [], 4), (5, [1, 2], 4), (2, [1, 2, 3], 2)])
 def test_pack_decodes_refuses(path, computed, blocks, room):
     """too few blocks, none, no such token, more blocks than room"""
@@ -74,6 +84,34 @@ def test_pack_decodes_fills_or_refuses(path, which):
     except TypeError:
         return
     assert (ids.tolist(), pos.tolist(), tab.tolist()) == ([8], [3], [[6, 0]])
+
+
+def test_decode_slots(path):
+    pos, tab = np.array([0, 7, 4, 11]), np.array([[3, 0, 0], [1, 2**31 - 1, 0], [5, 6, 0], [0, 0, 9]], np.int32)
+    slots, ctx = np.zeros(4, np.int64), np.zeros(4, np.int32)
+    ba.decode_slots(pos, tab, 4, slots, ctx)
+    assert slots.tolist() == [12, (2**31 - 1) * 4 + 3, 24, 39] and ctx.tolist() == [1, 8, 5, 12]
+    with pytest.raises(IndexError):
+        ba.decode_slots(pos + 8, tab, 4, slots, ctx)
+
+
+@pytest.mark.parametrize("names,rows", [([], 3), (["a"], 1), (["b", "", "a", "b", "x"], 8), (["a"] * 33 + [""] * 5 + ["b"] * 16, 64),
+                                        (["ab"[i % 2] for i in range(40)], 40)])
+def test_decode_lora_rows(path, names, rows):
+    from llm_instance_gateway_amd.lora.manager import build_lora_rows, max_lora_rows
+
+    asked = []
+    slot_of = lambda name: asked.append(name) or {"a": 4, "b": 0}.get(name, -1)
+    seqs = [Sequence([1], lora_name=n) for n in names]
+    room = max_lora_rows(rows, 6)
+    tok, n, slot = (np.full(s, -7, np.int32) for s in ((room, 16), room, room))
+    ba.decode_lora_rows(seqs, slot_of, rows, tok, n, slot)
+    want = build_lora_rows(np.array([{"a": 4, "b": 0}.get(x, -1) for x in names] + [-1] * (rows - len(names)), dtype=np.int32))
+    u = len(want[1])
+    for got, w in zip((tok, n, slot), want):
+        assert got[:u].tolist() == w.tolist()
+    assert not tok[u:].any() and not n[u:].any() and (slot[u:] == -1).all()
+    assert sorted(asked) == sorted({x for x in names if x})  # each name once, "" never
 
 
 def test_upload_keeps_values_and_alignment():
