@@ -57,6 +57,13 @@ def test_every_tile_is_reached():
     assert {s[2] for s in seen} >= {1, 2, 8}
 
 
+@pytest.mark.parametrize("M,N,K", [(1025, 4096, 8192), (1216, 4096, 14336), (1409, 8, 8192), (1537, 2056, 8256),
+                                   (2047, 4096, 8192), (2048, 1032, 8192), (1900, 8192, 16384)])
+def test_more_rows_of_long_weights(M, N, K):
+    test_projection(M, N, K)
+    assert not any(ops._EXT.projection_serves(*s) for s in ((2049, N, K), (M, N, 8128), (M, K // 2 + 8, K)))
+
+
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
 @pytest.mark.parametrize("M,N", [(60, 8200), (64, 1032), (130, 16632), (136, 11136), (200, 4104), (250, 70000)])
 def test_fewer_stages_than_the_ring(M, N, K):
