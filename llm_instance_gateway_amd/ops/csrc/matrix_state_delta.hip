@@ -42,7 +42,11 @@
 // 2-byte loads of values, 125 without the last two, 95 now: some 11 000 cycles
 // a chunk, of which the operand reads of q and k by all waves take 2600 (LDS
 // bandwidth) and the two barriers 1200.  Four waves per workgroup and two
-// workgroups per CU: slower by 15 us.
+// workgroups per CU: slower by 30 us, as q, k and the first kernel's blocks
+// come and go twice; but where that still leaves every workgroup a CU of its
+// own, a chunk takes 8700 cycles instead of 11000.  Two waves each, on up to
+// four times the CUs, are no faster than four.  A second set of staged rows,
+// one barrier a chunk: slower by 4 to 10 %.
 //
 // Precision: products of bf16 numbers are exact in fp32, sums are fp32, fp32
 // operands are split into two bf16 halves (lo * lo left out).  The unit norms
@@ -540,8 +544,12 @@ void ms_delta_chunks_launch(const MsArgs& a, int S, int max_seg_len, void* scrat
                             hipStream_t st) {
   DeltaChunk* sc = (DeltaChunk*)scratch;
   const dim3 gi((max_seg_len + MC_T - 1) / MC_T, S, a.H);
-  // two value blocks per workgroup share the staged operands where the
-  // registers of eight waves hold the state
+  // Two value blocks per workgroup share the staged operands where the
+  // registers of eight waves hold the state, and a workgroup each would not
+  // find a CU each.  Both calls, 32 heads of 128 x 128, one block here and two:
+  // 1 prompt of 4000 tokens 244 us, 298; of 1000 78, 95; 2 of these 85, 100;
+  // 4 (256 workgroups) 100, 114; 5 153, 123; 8 183, 151.
+  const bool pair = a.NB > 1 && (long)S * a.H * a.NB > 256;
   const bool vec = a.v_stride % 8 == 0 && aligned16(a.v);
 #define LIG_DS(DP, NW, VEC)                                                                   \
   hipLaunchKernelGGL((delta_chunk_scan_kernel<DP, NW, VEC>),                                  \
@@ -550,8 +558,8 @@ void ms_delta_chunks_launch(const MsArgs& a, int S, int max_seg_len, void* scrat
   do {                                                                                        \
     hipLaunchKernelGGL(delta_chunk_prepare_kernel<DP>, gi, dim3(DI_THREADS), 0, st, a, sc);   \
     constexpr int NW = DP <= 128 ? 8 : 4;                                                     \
-    if (a.NB > 1 && vec) LIG_DS(DP, NW, true);                                                \
-    else if (a.NB > 1) LIG_DS(DP, NW, false);                                                 \
+    if (pair && vec) LIG_DS(DP, NW, true);                                                    \
+    else if (pair) LIG_DS(DP, NW, false);                                                     \
     else if (vec) LIG_DS(DP, 4, true);                                                        \
     else LIG_DS(DP, 4, false);                                                                \
   } while (0)

@@ -67,3 +67,24 @@ def test_delta_chunks(lens, heads, kv, dim, vdim):
     # products of two halves without lo * lo lose 2^-16 of themselves; a correction goes through up to four of
     # them and 64 rows, whose errors add like a walk: 4 * 8 * 2^-16 of the largest output
     assert (got[0] - want).abs().max() <= 2.0 ** -11 * want.abs().max()
+
+
+@pytest.mark.parametrize("dim", [32, 64, 128])
+@pytest.mark.parametrize("vdim", [128, 192])
+def test_value_blocks_in_pairs(dim, vdim):
+    """Prompts that fill the chip share workgroups between value blocks, alone they do not: the same bits."""
+    lens, heads, kv = [17, 200, 64, 65, 130], 32, 16
+    test_delta_chunks(lens, heads, kv, dim, vdim)
+    g = torch.Generator("cuda").manual_seed(dim + vdim)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, z, nq = r(sum(lens), 2 * kv * dim + heads * vdim).to(BF), r(sum(lens), 2 * heads), kv * dim
+    rate, bias = r(heads) * 0.5, r(heads) - 3.0
+    def run(x, z, n):
+        state = torch.zeros(len(n), ops.matrix_state_width(heads, dim, vdim), device="cuda")
+        seg = _seg([sum(n[:i]) for i in range(len(n))], n, list(range(len(n))), [1] * len(n))
+        return ops.gated_delta_scan(x[:, :nq], x[:, nq : 2 * nq], x[:, 2 * nq :], (z[:, :heads], z[:, heads:]), rate, bias,
+                                    state, *[s.cuda() for s in seg], heads, kv, dim, vdim, q_scale=dim ** -0.5,
+                                    max_seg_len=max(n)), state
+    got, state = run(x, z, lens)
+    alone = [run(x[sum(lens[:i]) :][:n].contiguous(), z[sum(lens[:i]) :][:n].contiguous(), [n]) for i, n in enumerate(lens)]
+    assert torch.equal(got, torch.cat([o for o, _ in alone])) and torch.equal(state, torch.cat([s for _, s in alone]))
