@@ -89,3 +89,14 @@ def test_scale_signs(scale):
 @pytest.mark.parametrize("D,Dv,bs", [(576, 512, 16), (576, 512, 8), (320, 256, 6), (72, 64, 16)])
 def test_keys_before_the_first_visible_one(segs, H, D, Dv, bs, window, nsplit):
     _run(segs, H, D, Dv, bs, window, nsplit, gate=False, forget=True)
+
+
+@pytest.mark.parametrize("segs,H,cut", [
+    ([(1000, 1000)], 16, 1), ([(700, 100)], 16, 5), ([(600, 300), (520, 40)], 16, 2), ([(1500, 1)] * 16, 32, 11),
+    ([(520, 1)] * 160, 32, 1), ([(2000, 3), (16, 16)], 5, 15)])
+def test_chosen_slices(segs, H, cut):
+    """As many slices as the estimate takes, of at least 128 keys: the chip idle, filled once, filled more often."""
+    most = -(-max(c for c, _ in segs) // 16) * 16
+    args = sum(n for _, n in segs), len(segs), H, most, max(n for _, n in segs)
+    assert ops.latent_rows_nsplit(*args) == cut
+    _run(segs, H, 576, 512, 16, 0, 0, False)
