@@ -123,10 +123,11 @@ void lig_lora_qkv_rope_cache_launch(
     uint16_t*, const uint16_t*, const float*, int, long, const float*, int, float, const int64_t*, const float*, uint16_t*,
     uint16_t*, const int64_t*, int, int, int, int, const int*, const int*,
     const int*, int, const float*, int, int, const uint16_t*, int, hipStream_t);
+int lig_paged_attention_prefill_parts(long, long, int, int, long);
 void lig_paged_attention_prefill_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const int*,
     const int*, const int*, const int*, const int*, float, int, int, int,
-    int, int, int, hipStream_t);
+    int, int, int, int, float*, hipStream_t);
 }
 
 namespace {
@@ -398,12 +399,15 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(D == 64 || D == 128, "prefill MFMA kernel needs head_dim 64/128");
   if (ntiles == 0) return;
+  const int parts = lig_paged_attention_prefill_parts(ntiles, q.size(0), Hq, D, (long)max_blocks * BS);
+  torch::Tensor partial;
+  if (parts > 1) partial = torch::empty({q.size(0), Hq, parts, D + 4}, q.options().dtype(torch::kFloat32));
   lig_paged_attention_prefill_launch(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k_cache), bf16_cptr(v_cache),
       tile_seq.data_ptr<int>(), tile_qstart.data_ptr<int>(),
       query_start_locs.data_ptr<int>(), context_lens.data_ptr<int>(),
       block_tables.data_ptr<int>(), (float)scale, ntiles, Hq, Hkv, D, BS,
-      max_blocks, as_stream(stream));
+      max_blocks, parts, parts > 1 ? partial.data_ptr<float>() : nullptr, as_stream(stream));
 }
 
 void sgmv_shrink(torch::Tensor u, torch::Tensor x, torch::Tensor a_stack,
@@ -935,6 +939,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attention_decode", &paged_attention_decode);
   m.def("paged_attention_decode_split", &paged_attention_decode_split);
   m.def("paged_attention_prefill", &paged_attention_prefill);
+  m.def("paged_attention_prefill_parts", &lig_paged_attention_prefill_parts);
   m.def("sgmv_shrink", &sgmv_shrink);
   m.def("sgmv_apply", &sgmv_apply);
   m.def("sgmv_apply_units", &sgmv_apply_units);

@@ -73,7 +73,12 @@ struct Args {
   int chunk, window;
   int gate_per_head;
   float softcap;
+  int nsplit;               // SPLIT: parts of a tile's keys, and
+  float* partial;           // [R, Hq, nsplit, D + 4]: sums of weighted values, then largest score (log2) and sum of weights
 };
+
+// Tiles of keys to a part where nt are cut into nsplit: the last parts may be empty.
+LIG_DEVICE int tiles_of_part(int nt, int nsplit) { return (nt + nsplit - 1) / nsplit; }
 
 // Where the 16-byte chunks of key t's row, and (not DMA) of entry d's row of keys,
 // lie: chunk c at c ^ swizzle.  The reads of 16 lanes (0-3, 12-15 and of the next 16
@@ -92,8 +97,9 @@ LIG_DEVICE u32x2 transposed(const uint16_t* p) {
 
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
 // sigmoid(score + bias) weights.  EXTRA: temperature, gate, sink, chunk and
-// window are looked at (the plain causal kernel leaves them out).
-template <int D, int GH, bool PB, bool CAP, bool SIG, bool EXTRA>
+// window are looked at (the plain causal kernel leaves them out).  SPLIT: blockIdx.z
+// walks its part of the keys only and leaves sums that flash_prefill_merge_kernel adds up.
+template <int D, int GH, bool PB, bool CAP, bool SIG, bool EXTRA, bool SPLIT = false>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   constexpr int RB = GH;       // blocks of 16 rows per wave
 
@@ -102,6 +108,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   constexpr int CH = D / 8;    // 16-byte chunks of a row
   constexpr int TPT = KT * CH / 256;  // keys a thread stages: 4 (D = 128) or 2
   constexpr bool DMA = PB && D == 128;  // rows go straight into LDS, 4 to an instruction
+  static_assert(!SPLIT || !(CAP || SIG || EXTRA), "parts of the plain causal kernel");
   static_assert(16 * RB * (4 / GH) == TQ, "a workgroup serves one query tile of each of its heads");
 
   struct Shared {
@@ -196,7 +203,13 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
     if (a.window > 0) first_key = max(first_key, qpos0 - a.window + 1);
     first_key = max(first_key, 0);
   }
-  const int kv_begin = first_key & ~(KT - 1);
+  int kv_begin = first_key & ~(KT - 1), kv_stop = kv_end;
+  if constexpr (SPLIT) {
+    const int part = tiles_of_part((kv_end + KT - 1) / KT, a.nsplit) * KT;
+    kv_begin = blockIdx.z * part;
+    if (kv_begin >= kv_end) return;
+    kv_stop = min(kv_end, kv_begin + part);
+  }
   const int wave_first = ctx - n + row0;                                   // position of the wave's first row
   const int wave_last_lo = __builtin_amdgcn_readlane(key_lo[RB - 1], 15);  // largest lower bound
 
@@ -321,9 +334,9 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   // 29.5 -> 26.8, 16.5 -> 15.9, 43.8 -> 42.4.  The kernel before took 27.9, 15.9,
   // 70.8 and 24.6, 14.4, 56.7: with heads of 64 it fits more workgroups on a CU.
   if (row0 >= n) {
-    for (int kv0 = kv_begin, buf = 1; kv0 < kv_end; kv0 += KT, buf ^= 1) {
+    for (int kv0 = kv_begin, buf = 1; kv0 < kv_stop; kv0 += KT, buf ^= 1) {
       if constexpr (DMA) loads_landed<0>();
-      if (kv0 + KT < kv_end) {
+      if (kv0 + KT < kv_stop) {
         if constexpr (DMA) {
           fetch_dma(kv0 + KT, blk_next, buf);
           blk_next = blocks_of(kv0 + 2 * KT);
@@ -339,8 +352,8 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   }
 
   int buf = 0;
-  for (int kv0 = kv_begin; kv0 < kv_end; kv0 += KT, buf ^= 1) {
-    const bool more = kv0 + KT < kv_end;
+  for (int kv0 = kv_begin; kv0 < kv_stop; kv0 += KT, buf ^= 1) {
+    const bool more = kv0 + KT < kv_stop;
     if constexpr (DMA) loads_landed<0>();  // this tile is in LDS, and the other buffer is free
     if (more) {
       if constexpr (DMA) {
@@ -484,6 +497,17 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
       t += __shfl_xor(t, 16, 64);
       t += __shfl_xor(t, 32, 64);
       f = t > 0.f ? 1.f / t : (t == 0.f ? 0.f : t);
+      if constexpr (SPLIT) {
+        if (r >= n) continue;
+        float* sp = a.partial + (((size_t)(lo + r) * a.num_q_heads + h) * a.nsplit + blockIdx.z) * (D + 4);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4_t*>(sp + db * 16 + lg * 4) = acc[rb][db];
+        if (lg == 0) {
+          sp[D] = m[rb];
+          sp[D + 1] = t;
+        }
+        continue;
+      }
     }
     if (r >= n) continue;
     const uint16_t* gp = nullptr;
@@ -512,6 +536,39 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
       *reinterpret_cast<u32x2*>(op + d) = w;
     }
   }
+}
+
+// Adds up the parts of every (row, head) of a tile, 4 entries per lane.
+template <int D>
+__global__ __launch_bounds__(256) void flash_prefill_merge_kernel(const Args a) {
+  constexpr int LP = D / 4;
+  const int s = a.tile_seq[blockIdx.y], qt = a.tile_qstart[blockIdx.y];
+  const int lo = a.query_start_locs[s], n = a.query_start_locs[s + 1] - lo;
+  const int item = blockIdx.x * (256 / LP) + threadIdx.x / LP;
+  const int r = qt + item / a.num_q_heads, h = item % a.num_q_heads;
+  if (item >= TQ * a.num_q_heads || r >= n) return;
+  const int ctx = a.context_lens[s];
+  const int nt = (min(ctx, ctx - n + qt + TQ) + KT - 1) / KT, per = tiles_of_part(nt, a.nsplit);
+  const int parts = (nt + per - 1) / per;
+  const int d = (threadIdx.x % LP) * 4;
+  const float* base = a.partial + ((size_t)(lo + r) * a.num_q_heads + h) * a.nsplit * (D + 4);
+  float m = -INFINITY, l = 0.f;
+  for (int z = 0; z < parts; ++z) m = fmaxf(m, base[(size_t)z * (D + 4) + D]);
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int z = 0; z < parts; ++z) {
+    const float* sp = base + (size_t)z * (D + 4);
+    const float f = sp[D] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sp[D] - m);
+    l += sp[D + 1] * f;
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(sp + d);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] += v[i] * f;
+  }
+  const float f = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : l);
+  u32x2 w;
+  w[0] = pack_bf16(o[0] * f, o[1] * f);
+  w[1] = pack_bf16(o[2] * f, o[3] * f);
+  *reinterpret_cast<u32x2*>(a.out + ((size_t)(lo + r) * a.num_q_heads + h) * D + d) = w;
 }
 
 // What the kernel takes.  The Llama path has no other kernel and does not ask: its
@@ -545,6 +602,35 @@ static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
     launch_heads<D, 2, CAP, SIG, EXTRA>(a, ntiles, stream);
   else
     launch_heads<D, 1, CAP, SIG, EXTRA>(a, ntiles, stream);
+}
+
+// Parts to cut the keys of ntiles tiles into, by the least estimated time in us: a
+// workgroup takes 0.0145 a key alone on its CU and 0.02 beside a second one, the merge
+// and what begins and ends a part 8, their sums, written and read, at 6 TB/s.  A tile of
+// few rows on many keys is a chain of 64-key steps on an idle chip: steps of 8 layers of
+// 32 and 8 heads of 128, uncut and in parts, 20 rows on 4000 cached keys 1505 us, 1200;
+// 100 on 4000 1832, 1510; on 1200 1470, 1417; 300 on 3000 2268, 2147; 2 of 60 on 2000
+// 1604, 1488.  With 4 for the 8, 4 portions of 20 on 1000 lose 1 %.
+static inline int parts(long ntiles, long rows, int num_q_heads, int D, long keys) {
+  const long wgs = ntiles * num_q_heads;
+  int best = 1;
+  double least = keys * 0.0145;
+  for (int n = 2; n <= 16 && wgs * n <= 512 && keys / n >= 256; ++n) {
+    const double us = keys / (double)n * (wgs * n <= 256 ? 0.0145 : 0.02) + 8 + rows * num_q_heads * n * (D + 4) * 8e-6 / 6;
+    if (us < least) least = us, best = n;
+  }
+  return best;
+}
+
+template <int D>
+static void launch_parts(const Args& a, int ntiles, hipStream_t stream) {
+  const dim3 grid(a.num_q_heads, ntiles, a.nsplit), block(256);
+  if (a.block_shift >= 2)
+    hipLaunchKernelGGL((flash_prefill_kernel<D, 1, true, false, false, false, true>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((flash_prefill_kernel<D, 1, false, false, false, false, true>), grid, block, 0, stream, a);
+  hipLaunchKernelGGL(flash_prefill_merge_kernel<D>, dim3((TQ * a.num_q_heads * (D / 4) + 255) / 256, ntiles), block, 0, stream,
+                     a);
 }
 
 }  // namespace flash_prefill

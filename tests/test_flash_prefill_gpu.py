@@ -66,6 +66,20 @@ def test_causal(segs, D, H, G, bs):
     _check(got.view(T, -1), b, D, D ** -0.5, H)
 
 
+@pytest.mark.parametrize("segs", [[(1024, 1)], [(4100, 100)], [(2100, 17), (1, 1), (640, 63), (2090, 65)], [(2049, 64), (2048, 2)],
+                                  [(3000, 1), (130, 130)]], ids=range(5))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (128, 3, 1, 6), (64, 4, 4, 32), (64, 6, 1, 2), (128, 32, 8, 16)])
+def test_keys_in_parts(segs, D, H, G, bs):
+    """Few rows on many keys: parts that end between a tile's rows, and none for the shorter portions."""
+    b = _batch(segs, G, D, bs, H, 9)
+    T = b["q"].shape[0]
+    assert ops._load_ext().paged_attention_prefill_parts(len(b["ts"]), T, H, D, b["tab"].shape[1] * bs) > 1
+    got = ops.paged_attention_prefill(
+        b["q"].view(T, H, D), b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+        tile_qstart=b["tq"])
+    _check(got.view(T, -1), b, D, D ** -0.5, H)
+
+
 @pytest.mark.parametrize("D,H,G", [(128, 32, 8), (64, 32, 16)])
 def test_two_heads_per_workgroup(D, H, G):
     # enough tiles for the two-head workgroups, the last portions ragged
