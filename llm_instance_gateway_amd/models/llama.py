@@ -7,8 +7,8 @@ BASELINE.json: Llama-3-8B / 70B).  Built MI355X-first:
   * flat unpadded token batches (prefill chunks + decodes in one forward);
   * custom CDNA4 kernels via the ops layer for RMSNorm (fused residual add),
     RoPE, KV-cache scatter, paged prefill/decode attention and SwiGLU;
-  * the projections by `ops.linear`: a kernel of this package for few rows or
-    few tiles, library GEMMs elsewhere; LoRA deltas ride the SGMV path (`..lora`);
+  * the projections by `ops.linear`: a kernel of this package up to 1024 rows, of
+    long weights 2048, where it is the faster one, library GEMMs elsewhere; LoRA deltas ride the SGMV path (`..lora`);
   * optional tensor parallelism: column-sharded QKV/gate-up, row-sharded
     O/down with one RCCL all-reduce per block over xGMI (`..parallel`).
 

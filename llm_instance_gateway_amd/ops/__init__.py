@@ -384,8 +384,8 @@ LORA_ROWS_WIDTHS = (256, 512, 1024, 2048, 3072, 4096)  # lora_rms_norm's
 #                 128 17.6, 28.6, 25.2   200 30.3, 44.4, 30.9
 #   3072          24 6.8, 11.6, 18.8   72 11.3, 18.4, 20.3   96 13.2, 23.3, 20.7
 #   2048          24 4.9, 8.4, 12.7    48 7.0, 11.5, 13.2    72 8.6, 14.0, 13.7
-# (Above the line the open form would still be the faster one; there qkv and gate_up
-# are mostly the library's, and its reader in the rotation needs parts.)
+# (Above the line the open form would still be the faster one.  It needs the products
+# behind it in parts, for which many of those widths go to the library.)
 LORA_NORM_STRIPS_BELOW = 96
 
 

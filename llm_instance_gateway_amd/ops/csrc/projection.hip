@@ -227,9 +227,9 @@ LIG_DEVICE void later_stages(int left) {
 }
 
 // Tiles of 64 rows and more: 2 x 2 waves, one per SIMD, each with a quarter of the
-// tile.  The one above needs two barriers' worth of waiting per step and reads every
-// row of x 2 to 4 times from LDS, W's as often; as four waves of larger quarters the reads
-// shrink to two thirds, and what other waves covered is laid out here by hand:
+// tile.  Eight waves of an eighth each, which this replaces, read every row of x and W 2 to 4
+// times from LDS and waited for each other twice a step; four read two thirds of that, and
+// what other waves covered is laid out here by hand:
 //   * a step's products come in halves of 32 columns, and between them stand the reads
 //     of the next half's operands and the loads of later stages, evenly: neither the
 //     matrix cores nor the loads pause.  One barrier per step, at half time;
@@ -238,7 +238,7 @@ LIG_DEVICE void later_stages(int left) {
 //     on their way (a ring of two for both waited 0.5 us per step for its loads);
 //   * columns come 64 at a time, a full line of 128 bytes a row: 32 at a time, in a ring
 //     of finer grain, they arrived at little more than half the rate.
-// Llama-3-8B widths, weights not in any cache (us; kernel above -> this, the library):
+// Llama-3-8B widths, weights not in any cache (us; eight waves -> this, the library):
 //   rows      gate_up               down                o                 qkv
 //    202   71 -> 55 ( 66)     36 -> 35 ( 57)     17 -> 15 (21)     22 -> 20 (25)
 //    384  110 -> 77 ( 79)     54 -> 49 ( 75)     23 -> 20 (24)     33 -> 29 (35)
@@ -398,8 +398,8 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   X(16, 32, 6)       \
   X(32, 32, 8)
 // Else BM, BN, SX of projection_wide_kernel.  What is left of 34 shapes when those go
-// that no size of 18 projections and 31 row counts misses by more than a few per cent:
-// the one picked is 1.8 % slower than the best of all in the mean.
+// that no size of 17 projections and 23 row counts misses by more than a few per cent:
+// the one picked is 2 % slower than the best of all in the mean, 17 % at the worst.
 #define LIG_WIDE_TILES(X) \
   X(64, 64, 5)            \
   X(64, 96, 5)            \
