@@ -949,7 +949,7 @@ def latent_attention_rows(
         visible = block_tables.shape[1] * bs
         if window > 0:  # a 64-row tile sees the window and its own tokens
             visible = min(visible, window + 64)
-        nsplit = latent_rows_nsplit(R, S, num_heads, visible, max_seg_len)
+        nsplit = latent_rows_nsplit(int(R), int(S), int(num_heads), int(visible), int(max_seg_len))
     scratch = None
     if nsplit > 1:
         scratch = split_scratch(q.device, R * num_heads * nsplit * (v_dim + 4))

@@ -613,6 +613,7 @@ static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
 // 1604, 1488.  With 4 for the 8, 4 portions of 20 on 1000 lose 1 %.
 static inline int parts(long ntiles, long rows, int num_q_heads, int D, long keys) {
   const long wgs = ntiles * num_q_heads;
+  if (rows > ntiles * TQ) return 1;  // room for rows of no tile would have no bound
   int best = 1;
   double least = keys * 0.0145;
   for (int n = 2; n <= 16 && wgs * n <= 512 && keys / n >= 256; ++n) {

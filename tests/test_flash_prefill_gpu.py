@@ -73,7 +73,9 @@ def test_keys_in_parts(segs, D, H, G, bs):
     """Few rows on many keys: parts that end between a tile's rows, and none for the shorter portions."""
     b = _batch(segs, G, D, bs, H, 9)
     T = b["q"].shape[0]
-    assert ops._load_ext().paged_attention_prefill_parts(len(b["ts"]), T, H, D, b["tab"].shape[1] * bs) > 1
+    parts = ops._load_ext().paged_attention_prefill_parts
+    keys = b["tab"].shape[1] * bs
+    assert parts(len(b["ts"]), T, H, D, keys) > 1 and parts(len(b["ts"]), 64 * len(b["ts"]) + 1, H, D, keys) == 1
     got = ops.paged_attention_prefill(
         b["q"].view(T, H, D), b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
         tile_qstart=b["tq"])
