@@ -520,3 +520,23 @@ def test_every_number_of_parts(parts):
             out.append((q, kc, vc))
         for a, b in zip(*out):
             assert torch.equal(a, b)
+
+
+def _one_layer(hidden, inter, heads):
+    from llm_instance_gateway_amd.models.config import ModelConfig
+    from llm_instance_gateway_amd.models.llama import LlamaForCausalLM
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=hidden, num_layers=1, num_heads=heads, num_kv_heads=8,
+                     intermediate_size=inter, head_dim=128, max_position_embeddings=512)
+    return LlamaForCausalLM(mc, "cuda:0")
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("hidden,inter,heads,step", [(4096, 14336, 32, 128), (3072, 8192, 24, 128), (2048, 8192, 16, 256)])
+def test_rows_of_steps_by_the_library(hidden, inter, heads, step):
+    """Above 1024 rows, to counts at which its products are not slower than at the tuned ones."""
+    m = _one_layer(hidden, inter, heads)
+    for tokens in (1025, 1152, 1153, 1550, 1600, 1921, 2048):
+        assert m.batch_rows(tokens, 256) == -(-tokens // step) * step
+        assert m.batch_rows(tokens, 64) == -(-tokens // 64) * 64
+    assert m.batch_rows(2049, 256) == 2304
