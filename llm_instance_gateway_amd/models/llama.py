@@ -8,7 +8,7 @@ BASELINE.json: Llama-3-8B / 70B).  Built MI355X-first:
   * custom CDNA4 kernels via the ops layer for RMSNorm (fused residual add),
     RoPE, KV-cache scatter, paged prefill/decode attention and SwiGLU;
   * the projections by `ops.linear`: a kernel of this package up to 1024 rows, of
-    long weights 2048, where it is the faster one, library GEMMs elsewhere; LoRA deltas ride the SGMV path (`..lora`);
+    long weights 1792, where it is the faster one, library GEMMs elsewhere; LoRA deltas ride the SGMV path (`..lora`);
   * optional tensor parallelism: column-sharded QKV/gate-up, row-sharded
     O/down with one RCCL all-reduce per block over xGMI (`..parallel`).
 
@@ -274,7 +274,7 @@ class LlamaForCausalLM(nn.Module):
         multiple stays.  Sharded layers round every product, which has a rule of
         its own.
 
-        From 1025 to 2048 rows the library's products make a step, and of its untuned
+        From 1025 to 2048 rows a step is mostly the library's products, and of its untuned
         counts not every multiple of 64 is a good one: 1600 rows of 8B widths 6956 us, 1792
         6167.  Those of 128 are, all four of them measured at six widths from 2560 to 8192
         (8B: 1152 rows 4591 us, 1280 4789; 1408 5137, 1536 5259; 1664 6064, 1792 6167; 1920

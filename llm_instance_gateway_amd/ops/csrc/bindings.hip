@@ -268,7 +268,7 @@ bool projection_takes_rows(const torch::Tensor& x, const torch::Tensor& w) {
          projection_takes(w, x.size(0));
 }
 
-// y = x W^T of up to 2048 rows (projection.hip); sizes that it does not serve are refused
+// y = x W^T of up to 1792 rows (projection.hip); sizes that it does not serve are refused
 void projection(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t stream) {
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2);
   const long M = x.size(0), N = w.size(0), K = w.size(1);

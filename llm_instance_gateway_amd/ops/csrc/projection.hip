@@ -1,4 +1,4 @@
-// Projections of up to 2048 rows, gfx950, bf16: y = x W^T with x [M, K], W [N, K].
+// Projections of up to 1024 rows, long weights' of up to 1792, gfx950, bf16: y = x W^T with x [M, K], W [N, K].
 //
 // Bound by how fast a CU gets its tiles, W once from HBM, x again for every tile of W's
 // rows from the L2, and with some hundred rows by the matrix products.  The launch picks
@@ -517,13 +517,16 @@ extern "C" {
 // rows, from 3072 columns on, they take 0.6 to 1 of the library's time, of the largest
 // matrices 0.85 to 1.05 (384 rows: 6144 x 4096 29 us here, 35 there; 4096 x 14336 49, 75;
 // 28672 x 4096 77, 79; 960: 181, 175).  With many tiles of fewer columns neither is ahead
-// (16384 x 2048: 288 rows 24, 27; 384 29, 27).  Above 1024 rows long rows of W still win, as
-// K is cut where tiles of 256 x 256 leave CUs idle (us here, the library's; 4096 x 14336: 1216
-// rows 115, 149; 1536 132, 164; 2048 171, 205; 8192 x 28672: 1280 439, 453; 2048 635, 638);
-// of shorter ones, and from 2300 rows on, neither is steadily ahead.
+// (16384 x 2048: 288 rows 24, 27; 384 29, 27).
+// Above 1024 rows it is large weights with long rows, to 1792, where all of K in one part
+// fills the chip (here, the library's; 8192 x 28672: 1152 rows 518, 548; 1408 518, 520; 1792
+// 589, 802; 8192 x 16384: 1280 258, 276; 12288 x 28672: 1536 869, 1423; 5120 x 13824: 1792 213,
+// 221).  From 1793 on they lose as often as they win (1920: 644, 647; 373, 363; 16384 x 53248
+// 2438, 2299).  In parts 4096 x 14336 would win too (1216 rows 115, 149), but where a step's
+// other products are the library's nothing adds them up, and the sum takes what the cut gains.
 bool lig_projection_serves(long M, long N, long K) {
-  if (M < 1 || M > 2048 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
-  if (M > 1024) return K >= 8192 && K >= 2 * N;
+  if (M < 1 || M > 1792 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
+  if (M > 1024) return K >= 8192 && K >= 2 * N && N * K >= 1L << 26 && plan((int)M, (int)N, (int)K).splits == 1;
   return M <= 256 || ((M + 255) / 256) * ((N + 255) / 256) <= 64 || K >= 3072 || (M <= 384 && N >= 65536);
 }
 
@@ -539,13 +542,12 @@ bool lig_projection_serves(long M, long N, long K) {
 //     at most (1000 x 4096 x 4096: 36, 39; 448 x 6144 x 4096: 31, 33).
 // Of smaller weights the library's call takes longer on the host than is gained, which steps
 // of narrow models wait for: 300 rows, 16 layers of 2048 columns 2106 us, 2488 with its
-// products.  Above 1024 rows adding up takes what a cut of K gains (2048 x 4096 x 8192: 101
-// and 20, 108).
+// products.
 bool lig_projection_pays(long M, long N, long K) {
   if (M > 16 && N > 32768 && K < 2048) return false;
   if (M <= 128 || N >= 65536 || N * K < 1L << 24) return true;
+  if (M > 1024) return true;
   const int splits = plan((int)M, (int)N, (int)K).splits;
-  if (M > 1024) return splits == 1;
   if (M > 256) return splits >= 4 || N * K >= 1L << 25;
   if (splits > 1) return (K > N || M <= 224 || N >= 6144) && (splits > 2 || (N >= 4096 && N <= 16384));
   return (K <= 4096 && N >= 8192 && N <= 32768) || N * K >= 1L << 28;

@@ -60,8 +60,22 @@ def test_every_tile_is_reached():
 @pytest.mark.parametrize("M,N,K", [(1025, 4096, 8192), (1216, 4096, 14336), (1409, 8, 8192), (1537, 2056, 8256),
                                    (2047, 4096, 8192), (2048, 1032, 8192), (1900, 8192, 16384)])
 def test_more_rows_of_long_weights(M, N, K):
+    """Above 1024 rows the library's, as products of shorter weights are, where nothing
+    would add up the parts that they come in, or from 1793 rows on."""
+    x, w = torch.randn(M, K, device="cuda").to(BF), torch.randn(N, K, device="cuda").to(BF)
+    with torch.no_grad():
+        assert not ops.linear_served(M, w) and ops.linear_served(1024, w)
+        want = torch.nn.functional.linear(x, w)
+        assert torch.equal(ops.linear(x, w), want) and torch.equal(ops.linear_parts(x, w), want)
+    with pytest.raises(RuntimeError, match="shape"):
+        ops._EXT.projection(want, x, w, torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("M,N,K", [(1152, 8192, 16384), (1300, 8200, 16448), (1665, 7168, 18432), (1792, 5120, 13824)])
+def test_more_rows_in_one_part(M, N, K):
     test_projection(M, N, K)
-    assert not any(ops._EXT.projection_serves(*s) for s in ((2049, N, K), (M, N, 8128), (M, K // 2 + 8, K)))
+    w = torch.empty(N, K, device="cuda", dtype=BF)
+    assert ops.linear_pays(M, w) and not ops.linear_served(1793, w)
 
 
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
