@@ -219,9 +219,16 @@ class ModelRunner:
         # partitions and the sample set.
         num_pad_tokens = 0
         padm = self.config.pad_batch_multiple
+        mgr = getattr(self, "adapter_manager", None)
+        lora_tiles = None
+        if mgr is not None and any(q.lora_name for q in seqs):
+            slot = {name: mgr.slot_of(name) for name in {q.lora_name for q in seqs}}
+            seq_slot = np.array([slot[q.lora_name] for q in seqs], dtype=np.int32)
+            # of 16 rows of an adapter, or of none
+            lora_tiles = int((-(-np.bincount(seq_slot + 1, length) // 16)).sum()) if getattr(mgr, "in_layer", False) else 0
         if padm > 0 and self.device.type == "cuda" and not self.config.model.is_moe:
             if hasattr(self.model, "batch_rows"):
-                num_pad_tokens = self.model.batch_rows(T, padm) - T
+                num_pad_tokens = self.model.batch_rows(T, padm, lora_tiles) - T
             else:
                 num_pad_tokens = -T % padm
 
@@ -290,10 +297,7 @@ class ModelRunner:
                 put("prefill_tok_block_tables", p_tab[tok_seq[:num_prefill_tokens]])
 
         # multi-LoRA: per-token adapter slot ids (-1 = base model only)
-        mgr = getattr(self, "adapter_manager", None)
-        if mgr is not None and any(ss.seq.lora_name for ss in prefills + decodes):
-            slot = {name: mgr.slot_of(name) for name in {q.lora_name for q in seqs}}
-            seq_slot = np.array([slot[q.lora_name] for q in seqs], dtype=np.int32)
+        if lora_tiles is not None:
             lora_slots = np.full(T + num_pad_tokens, -1, dtype=np.int32)  # pad rows: base model only
             lora_slots[:T] = seq_slot[tok_seq]
             put("lora_slot_per_token", lora_slots)

@@ -263,16 +263,24 @@ class LlamaForCausalLM(nn.Module):
                 return False
         return True
 
-    def batch_rows(self, tokens: int, multiple: int) -> int:
-        """Rows to pad a flat batch of tokens to.  The library's products want few,
-        tile-friendly counts, those of `ops.linear` take any: none is added where
-        all of a layer's projections run there (786 tokens: a step of 8B widths
-        takes 4.6 ms, 5.1 padded to 832 with qkv and gate_up at the library), few
-        where some do.  At such a count those left to the library miss its tuned
-        table, which knows multiples of 256: the rows saved are worth more.  Under
-        2^20 weights a projection takes its launch's time at either count, and the
-        multiple stays.  Sharded layers round every product, which has a rule of
-        its own.
+    def batch_rows(self, tokens: int, multiple: int, lora_tiles: int | None = None) -> int:
+        """Rows to pad a flat batch of tokens to; `lora_tiles`: of a step with adapters,
+        its tiles of rows, 0 where adapters have kernels of their own.
+
+        The library's products want few, tile-friendly counts, those of `ops.linear`
+        take any: none is added where all of a layer's projections run there (786
+        tokens: a step of 8B widths takes 4.6 ms, 5.1 padded to 832 with qkv and gate_up
+        at the library), few where some do.  At such a count those left to the library
+        miss its tuned table, which knows multiples of 256: the rows saved are worth
+        more.  Under 2^20 weights a projection takes its launch's time at either count,
+        and the multiple stays.
+
+        Where norms and rotation do not add up parts (sharded layers, hooks, adapters of
+        their own kernels or of many tiles) every product has to come rounded, for which
+        fewer run here: at 786 rows of 8B widths qkv and o are the library's.  By itself a
+        step takes the same time at any such count (786 rows of adapters of rank 32 4881
+        us, 832 4933; 1000 5418, 1024 5389), but each count that the library meets for the
+        first time costs it 70 us a product: 12 multiples of 64 against 768 counts.
 
         From 1025 to 2048 rows a step is mostly the library's products, and of its untuned
         counts not every multiple of 64 is a good one: 1600 rows of 8B widths 6956 us, 1792
@@ -286,12 +294,21 @@ class LlamaForCausalLM(nn.Module):
             return -(-tokens // step) * step
         attn, mlp = self.layers[0].self_attn, getattr(self.layers[0], "mlp", None)
         modules = [attn.qkv_proj, attn.o_proj, *((mlp.gate_up_proj, mlp.down_proj) if type(mlp) is MLP else ())]
-        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 and (self.tp is None or ops.linear_pays(tokens, m.weight))
-                  for m in modules]
-        if all(served):
+        served = [_served(m, tokens) and m.weight.numel() >= 1 << 20 for m in modules]
+        here = [s and ops.linear_pays(tokens, m.weight) for s, m in zip(served, modules)]
+        if here != served and self._in_parts(tokens, lora_tiles):
+            here = served
+        if all(here):
             return tokens
-        step = min(64, multiple) if any(served) else multiple
+        step = min(64, multiple) if any(here) else multiple
         return -(-tokens // step) * step
+
+    def _in_parts(self, tokens: int, lora_tiles: int | None) -> bool:
+        """Whether what reads the products of such a step (`batch_rows`) adds up parts."""
+        if lora_tiles is None:
+            return self._open_norms(tokens)
+        return (self.tp is None and lora_tiles > 0 and ops.lora_norm_opens(ops.BASE_ROWS, 16 * lora_tiles, self.cfg.hidden_size)
+                and self.plain_layers())
 
     def _row_products(self) -> bool:
         """Whether every projection of a layer is one that `ops.row_product` serves."""

@@ -540,3 +540,40 @@ def test_rows_of_steps_by_the_library(hidden, inter, heads, step):
         assert m.batch_rows(tokens, 256) == -(-tokens // step) * step
         assert m.batch_rows(tokens, 64) == -(-tokens // 64) * 64
     assert m.batch_rows(2049, 256) == 2304
+
+
+@torch.no_grad()
+def test_rows_of_steps_whose_products_come_rounded():
+    """Where norms and rotation cannot add up parts, qkv and o of such counts are the
+    library's, and rows are added for them."""
+    m = _one_layer(4096, 14336, 32)
+    for tokens in (9, 130, 300, 786, 1000):
+        few, opens = -(-tokens // 64) * 64 if tokens > 256 else tokens, tokens
+        assert m.batch_rows(tokens, 256) == opens
+        assert m.batch_rows(tokens, 256, 60) == opens  # adapters inside the layers
+        assert m.batch_rows(tokens, 256, 96) == few  # of too many tiles for norms that open
+        assert m.batch_rows(tokens, 256, 0) == few  # by kernels of their own
+        hook = m.layers[0].register_forward_hook(lambda *a: None)
+        assert m.batch_rows(tokens, 256) == m.batch_rows(tokens, 256, 60) == few
+        hook.remove()
+
+
+@pytest.mark.parametrize("rank,names,tiles", [(16, ["", ""], None), (16, ["a", "", "b", "a"], 2 + 1 + 2), (32, ["a", ""], 0)])
+def test_rows_are_asked_for_with_the_adapters(monkeypatch, rank, names, tiles):
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.lora import manager
+    from llm_instance_gateway_amd.models.config import ModelConfig
+
+    mc = ModelConfig(name="t", vocab_size=512, hidden_size=512, num_layers=1, num_heads=8, num_kv_heads=2,
+                     intermediate_size=1024, head_dim=64, max_position_embeddings=512)
+    eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=50, max_num_seqs=8, max_model_len=256), device="cuda:0")
+    mgr = manager.AdapterManager(eng, max_slots=2, rank=rank)
+    for n in "ab":
+        mgr.register_random(n, seed=1)
+    lens = {"": 3, "a": 10, "b": 17}
+    for n in names:
+        eng.add_request([1] * lens[n], SamplingParams(max_new_tokens=2), lora_name=n)
+    model, asked = eng.runner.model, []
+    monkeypatch.setattr(model, "batch_rows", lambda t, m, tiles=None: asked.append((t, m, tiles)) or 256)
+    eng.step()
+    assert asked == [(sum(lens[n] for n in names), 256, tiles)]
