@@ -77,8 +77,9 @@ struct Args {
   float* partial;           // [R, Hq, nsplit, D + 4]: sums of weighted values, then largest score (log2) and sum of weights
 };
 
-// Tiles of keys to a part where nt are cut into nsplit: the last parts may be empty.
-LIG_DEVICE int tiles_of_part(int nt, int nsplit) { return (nt + nsplit - 1) / nsplit; }
+// Tiles of keys to a part where nt are cut into nsplit: the last parts may be empty, as
+// are all where a context is shorter than its own rows and a tile sees no key (nt <= 0).
+LIG_DEVICE int tiles_of_part(int nt, int nsplit) { return max(1, (nt + nsplit - 1) / nsplit); }
 
 // Where the 16-byte chunks of key t's row, and (not DMA) of entry d's row of keys,
 // lie: chunk c at c ^ swizzle.  The reads of 16 lanes (0-3, 12-15 and of the next 16

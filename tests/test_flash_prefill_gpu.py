@@ -82,6 +82,27 @@ def test_keys_in_parts(segs, D, H, G, bs):
     _check(got.view(T, -1), b, D, D ** -0.5, H)
 
 
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 6, 1, 2)])
+def test_tiles_without_keys_in_parts(D, H, G, bs):
+    """Contexts shorter than their rows, one of them empty: rows that see no key come out as zeros."""
+    b = _batch([(2100, 20), (130, 130), (64, 5), (300, 300)], G, D, bs, H, 10)
+    short = {1: 40, 2: 0, 3: 50}
+    for i, c in short.items():
+        b["ctx"][i] = c
+    T = b["q"].shape[0]
+    assert ops._load_ext().paged_attention_prefill_parts(len(b["ts"]), T, H, D, b["tab"].shape[1] * bs) > 1
+    got = ops.paged_attention_prefill(
+        b["q"].view(T, H, D), b["k"], b["v"], b["tab"], b["starts"], b["ctx"], D ** -0.5, tile_seq=b["ts"],
+        tile_qstart=b["tq"]).view(T, -1)
+    lens = (b["starts"][1:] - b["starts"][:-1]).long()
+    b["pos"] = torch.cat([torch.arange(int(n), device="cuda") + int(c) - int(n) for c, n in zip(b["ctx"], lens)])
+    sees = b["pos"] >= 0
+    assert not got[~sees].any() and int((~sees).sum()) == 90 + 5 + 250
+    for k in ("q", "tok_seq", "pos"):
+        b[k] = b[k][sees]
+    _check(got[sees], b, D, D ** -0.5, H)
+
+
 @pytest.mark.parametrize("D,H,G", [(128, 32, 8), (64, 32, 16)])
 def test_two_heads_per_workgroup(D, H, G):
     # enough tiles for the two-head workgroups, the last portions ragged
