@@ -13,7 +13,6 @@ Policy:
 
 from __future__ import annotations
 
-import functools
 import os
 from typing import Optional, Tuple
 
@@ -882,34 +881,24 @@ def latent_rows_supported(q_dtype, row: int, v_dim: int, is_cuda: bool) -> bool:
     )
 
 
-@functools.lru_cache(maxsize=512)
-def latent_rows_nsplit(rows: int, segs: int, heads: int, max_ctx: int, longest: int = 2**31) -> int:
-    """Context slices for the latent row kernel, each of at least 128 keys of the
-    longest possible context: the number with the least estimated time, in us with
-    rows of 576 and values of 512.  A workgroup takes 5 and per key 0.034 with single
-    tokens of up to 32 heads (`longest` segment; a workgroup to each, one at a time on
-    a CU), else 0.0455 alone on its CU and 0.066 beside a second one; the slices'
-    sums, written and read by a launch more, go at 6.2 TB/s, and are what twice as
-    many workgroups as CUs lose by.  Measured, that rule's time and this one's: a
-    prompt of 1000, 16 heads 65.8 (3 slices), 56.6 (1); behind a window of 512
-    61.3, 36.1; 100 tokens on 4000 46.2 (20), 44.3 (8); single tokens, 32 heads, 64
-    on 2000 keys 51.5 (6), 37.8 (4); 16 on 4000 41.0 (22), 29.5 (16); 160 on 1000
-    55.5 (3), 49.1 (1)."""
-    single = longest * heads <= 32
-    blocks = segs if single else min((rows * heads + 63) // 64 + segs, segs * ((longest * heads + 63) // 64))
+def latent_rows_nsplit(rows: int, segs: int, heads: int, max_ctx: int) -> int:
+    """Context slices for the latent row kernel: 1 when the step's rows fill
+    the chip by themselves, counted in 64-row workgroups and one more a segment,
+    else enough slices for twice as many of those as CUs, each with at least 128
+    keys of the longest possible context.  (Single tokens of up to 32 heads run in
+    32-row workgroups, one to a segment and one to a CU at a time, so 171 to 255 of
+    them with 32 heads count as filling the chip and leave some CUs idle.)
+
+    Fewer slices, by the least estimated time, would be faster by a fifth in the mean (8
+    portions of 75 of 614 keys, windows of 512, 55.1 us with 4, 37.3 with 1; 64 single tokens on 2000 51.5
+    with 6, 37.8 with 4), but not as exact: each slice rounds its weights to bf16 against its
+    own largest, which is 1 without rounding.  Against 64 bits, over 40 drawn calls: 1.7 %
+    more error in the mean, 0.001808 -> 0.001886 in the first of these.  A caller that wants
+    them has `nsplit`."""
+    blocks = (rows * heads + 63) // 64 + segs
     if blocks >= _NUM_CUS or max_ctx < 512:
         return 1
-
-    def us(n):
-        if single:
-            walks = -(-blocks * n // _NUM_CUS) * (5 + max_ctx / n * 0.034)
-        elif blocks * n <= _NUM_CUS:
-            walks = 5 + max_ctx / n * 0.0455
-        else:
-            walks = -(-blocks * n // (2 * _NUM_CUS)) * (5 + max_ctx / n * 0.066)
-        return walks + (3 + rows * heads * n * 0.00067 if n > 1 else 0)
-
-    return min(range(1, min(32, max_ctx // 128) + 1), key=us)
+    return max(1, min(32, (2 * _NUM_CUS + blocks - 1) // blocks, max_ctx // 128))
 
 
 def latent_attention_rows(
@@ -949,7 +938,7 @@ def latent_attention_rows(
         visible = block_tables.shape[1] * bs
         if window > 0:  # a 64-row tile sees the window and its own tokens
             visible = min(visible, window + 64)
-        nsplit = latent_rows_nsplit(int(R), int(S), int(num_heads), int(visible), int(max_seg_len))
+        nsplit = latent_rows_nsplit(R, S, num_heads, visible)
     scratch = None
     if nsplit > 1:
         scratch = split_scratch(q.device, R * num_heads * nsplit * (v_dim + 4))

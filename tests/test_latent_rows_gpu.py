@@ -91,12 +91,16 @@ def test_keys_before_the_first_visible_one(segs, H, D, Dv, bs, window, nsplit):
     _run(segs, H, D, Dv, bs, window, nsplit, gate=False, forget=True)
 
 
-@pytest.mark.parametrize("segs,H,cut", [
-    ([(1000, 1000)], 16, 1), ([(700, 100)], 16, 5), ([(600, 300), (520, 40)], 16, 2), ([(1500, 1)] * 16, 32, 11),
-    ([(520, 1)] * 160, 32, 1), ([(2000, 3), (16, 16)], 5, 15)])
-def test_chosen_slices(segs, H, cut):
-    """As many slices as the estimate takes, of at least 128 keys: the chip idle, filled once, filled more often."""
+@pytest.mark.parametrize("segs,H", [
+    ([(1000, 1000)], 16), ([(700, 100)], 16), ([(600, 300), (520, 40)], 16), ([(1500, 1)] * 16, 32), ([(520, 1)] * 160, 32),
+    ([(2000, 3), (16, 16)], 5)])
+def test_chosen_slices(segs, H):
+    """Two workgroups a CU or more, unless a slice had less than 128 keys or there were over 32:
+    fewer round more of the weights, and the error against 64 bits grows."""
     most = -(-max(c for c, _ in segs) // 16) * 16
-    args = sum(n for _, n in segs), len(segs), H, most, max(n for _, n in segs)
-    assert ops.latent_rows_nsplit(*args) == cut
+    rows = sum(n for _, n in segs)
+    cut = ops.latent_rows_nsplit(rows, len(segs), H, most)
+    blocks = (rows * H + 63) // 64 + len(segs)
+    assert 1 <= cut <= 32 and most // cut >= 128
+    assert cut * blocks >= 512 or cut == 32 or most // (cut + 1) < 128
     _run(segs, H, 576, 512, 16, 0, 0, False)
