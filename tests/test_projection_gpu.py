@@ -57,6 +57,40 @@ def test_every_tile_is_reached():
     assert {s[2] for s in seen} >= {1, 2, 8}
 
 
+# one tile of rows on weights from 2^24 entries on, which are loaded past the caches
+STREAMED = [
+    (3, 33136, 512), (10, 33128, 512), (22, 16384, 1024), (1, 57352, 320), (67, 16872, 1024), (97, 16872, 1024),
+    (79, 33128, 512), (97, 16872, 2048), (79, 57352, 320), (79, 16872, 3072), (130, 16872, 1024), (130, 33128, 512),
+    (163, 33128, 512), (163, 16872, 3072), (163, 16872, 1024), (193, 3080, 8192), (163, 28680, 1024), (193, 33128, 512),
+    (193, 16872, 4096), (226, 33128, 512), (33, 28672, 4096), (202, 28672, 4096),
+]
+
+
+@pytest.mark.parametrize("M,N,K", STREAMED)
+def test_streamed_weights(M, N, K):
+    test_projection(M, N, K)
+
+
+def test_every_kernel_is_reached():
+    """Tiles by whether they leave sums or the rounded product and by how they load W.  A
+    size in one part runs both, `linear` and `linear_parts`."""
+    plan = ops._load_ext().projection_plan
+
+    def kernels(sizes):
+        out = set()
+        for s in sizes:
+            bm, bn, cut = plan(*s)
+            streams = s[0] <= bm and s[1] * s[2] >= 1 << 24
+            out |= {(bm, bn, sums, streams) for sums in ((True,) if cut > 1 else (True, False))}
+        return out
+
+    wide = [(m, n, k) for m in (*range(1, 1025, 5), 1152, 1408, 1664, 1792)
+            for n in (8, 136, 1024, 1280, 3072, 4096, 6144, 8192, 12288, 16384, 16872, 28672, 33128, 57344, 128256)
+            for k in (64, 128, 320, 512, 1024, 1344, 2048, 3072, 4096, 8192, 14336, 28672) if ops._EXT.projection_serves(m, n, k)]
+    # 17 tiles, four ways each but 16 x 32 and 32 x 32, which are for small weights
+    assert len(kernels(wide)) == 64 and kernels(SIZES + STREAMED) >= kernels(wide)
+
+
 @pytest.mark.parametrize("M,N,K", [(1025, 4096, 8192), (1216, 4096, 14336), (1409, 8, 8192), (1537, 2056, 8256),
                                    (2047, 4096, 8192), (2048, 1032, 8192), (1900, 8192, 16384)])
 def test_more_rows_of_long_weights(M, N, K):
