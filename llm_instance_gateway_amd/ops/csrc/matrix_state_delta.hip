@@ -548,7 +548,9 @@ void ms_delta_chunks_launch(const MsArgs& a, int S, int max_seg_len, void* scrat
   // registers of eight waves hold the state, and a workgroup each would not
   // find a CU each.  Both calls, 32 heads of 128 x 128, one block here and two:
   // 1 prompt of 4000 tokens 244 us, 298; of 1000 78, 95; 2 of these 85, 100;
-  // 4 (256 workgroups) 100, 114; 5 153, 123; 8 183, 151.
+  // 4 (256 workgroups) 100, 114; 5 153, 123; 8 183, 151.  That is prompts alone: S counts
+  // every segment of a call, also those too short for these kernels, whose workgroups are
+  // over at once, so that a prompt beside a few single tokens gets pairs.
   const bool pair = a.NB > 1 && (long)S * a.H * a.NB > 256;
   const bool vec = a.v_stride % 8 == 0 && aligned16(a.v);
 #define LIG_DS(DP, NW, VEC)                                                                   \

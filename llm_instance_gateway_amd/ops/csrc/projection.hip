@@ -6,8 +6,10 @@
 //   * Rows go from memory straight into LDS, stages of 64 or 128 columns in a ring,
 //     XOR-swizzled through the choice of what a lane fetches (no bank conflicts, by the
 //     counter);
-//   * up to 32 rows of weights that are soon read: small tiles with the columns of a
-//     stage dealt to the waves, whose sums meet in LDS; else projection_wide_kernel;
+//   * weights under 2^24 entries, where the estimate says so (few rows, or many on so few
+//     outputs that larger tiles would be fewer than CUs), and up to 8 rows of a vocabulary:
+//     small tiles with the columns of a stage dealt to the waves, whose sums meet in LDS;
+//     else projection_wide_kernel;
 //   * XCDs start at different quarters of K: in step, all 256 CUs would ask for the same
 //     columns of rows 8 KB apart, that is for few memory channels.  Inside an XCD the CUs
 //     stay in step and find x in its L2; the tiles of an XCD lie side by side;
@@ -75,7 +77,7 @@ LIG_DEVICE void store_tile(const f32x4_t (&acc)[TN][TM], uint16_t* __restrict__ 
   }
 }
 
-// Few rows: tiles of BM x BN, each wave a quarter of a stage's 128 columns.
+// Small weights: tiles of BM x BN, each wave a quarter of a stage's 128 columns.
 // PARTIAL: fp32 sums of a part of K to part[z][M][N].
 template <int BM, int BN, int ST, bool PARTIAL>
 __global__ __launch_bounds__(256, 1) void projection_kernel(
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   *reinterpret_cast<u16x8*>(y + e) = f32x8_to_bf16x8(s);
 }
 
-// Few rows: BM, BN, ST of projection_kernel (4 waves over the columns, steps of 128).
+// Small weights: BM, BN, ST of projection_kernel (4 waves over the columns, steps of 128).
 #define LIG_TILES(X) \
   X(16, 16, 8)       \
   X(16, 32, 6)       \
@@ -435,16 +437,19 @@ struct Plan {
   int tile, splits;
 };
 
-// What a kernel's time is made of, in us: per step of 64 columns of a tile its products,
+// A kernel's time in us, as a regression on: per step of 64 columns of a tile its products,
 // its rows of W, its rows of x; launch, tile; W from memory at `hbm` TB/s; a cut of K
-// and, in millionths, every sum of it.  A fit to 17000 measured times, 6 % off them.
+// and, in millionths, every sum of it.  Fitted to 17000 measured times, 6 % off them: 1 to
+// 2048 rows (FEW_COST 1 to 128), 1536 to 128256 outputs, 2048 to 28672 columns.  Outside of
+// these it picks a tile that is right but was not measured, and its terms are no prices: with
+// few rows those of W and x come out negative.
 struct Cost {
   double area, w_row, x_row, step, launch, tile, hbm, cut, sum;
 };
 constexpr Cost FEW_COST = {0.0005405, -0.005728, -0.0135, 0.2466, 3.263, 0.1869, 8.987, -0.6106, 3.765};
 constexpr Cost WIDE_COST = {9.45e-06, 0.001368, 0.001277, 0.004109, 0.9942, 2.333, 7.596, -0.2958, 1.212};
 
-// Tiles of few rows are for small weights: 16 rows of 28672 x 4096 take 41 us on them, 36
+// The first tiles are for small weights: 16 rows of 28672 x 4096 take 41 us on them, 36
 // on tiles of 64 x 128; of 4096 x 4096 both 7.7; of 2048 x 2048 4.1 and 4.7.  Tall tiles that
 // would be mostly padding were not measured.
 Plan plan(int M, int N, int K) {
