@@ -284,7 +284,7 @@ class LlamaForCausalLM(nn.Module):
 
         From 1025 to 2048 rows a step is mostly the library's products, and of its untuned
         counts not every multiple of 64 is a good one: 1600 rows of 8B widths 6956 us, 1792
-        6167.  Those of 128 are, all four of them measured at six widths from 2560 to 8192
+        6167.  Those of 128 are, all four of them measured at seven shapes of 2560 to 8192 columns
         (8B: 1152 rows 4591 us, 1280 4789; 1408 5137, 1536 5259; 1664 6064, 1792 6167; 1920
         6560, 2048 6620; 5 adapters: 1152 5015, 1280 5129).  At 2048 columns 1152 rows
         take up to 1.5 % longer than 1280, and the multiple stays, as for sharded layers,
