@@ -529,82 +529,159 @@ LIG_DEVICE float silu_of_quarter(float n) {
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, n), r, q), d, n);
 }
 
+// load_b's two operands by one load: lanes lg < 2 bring the first, the others the second.
+LIG_DEVICE u16x8 load_b_once(const uint16_t* b, int c0, int li, int lg) {
+  return *reinterpret_cast<const u16x8*>(b + (size_t)(c0 + ((li >> 2) << 3) + (li & 3) + (lg >> 1) * 4) * R + (lg & 1) * 8);
+}
+LIG_DEVICE BOperand both_halves(u16x8 x) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 v = __builtin_bit_cast(u32x4, x);
+  u32x4 lo, hi;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v[i], v[i], false, false);
+    lo[i] = s[0];
+    hi[i] = s[1];
+  }
+  return {__builtin_bit_cast(u16x8, lo), __builtin_bit_cast(u16x8, hi)};
+}
+
 // out = silu(gate + B u) * (up + B u), u_out[strip] = A_down out.  Workgroups of
 // a tile take strips of 1024 of the d columns.
+// In the products' layout 16 lanes side by side hold 16 rows, and a load costs an access
+// of the L1 per lane instead of one per four: 331 accesses for 32 columns of a tile, which
+// took 62 % of the time at 4000 rows.  So rows come as they lie, 256 bytes of 4 rows to a
+// load, straight into LDS, and leave through it; 16-byte piece c of row r at c ^ r, for
+// reads and writes without conflicts.  A wave uses its own part of LDS only.
 constexpr int SILU_STRIP = 1024;
+constexpr int SILU_BATCH = 128;  // columns of a wave at a time
+constexpr int SILU_ROOM = 3 * 16 * SILU_BATCH;  // gate, up and A's rows of a batch, 16-bit units
 
-template <bool LORA, int W>
-LIG_DEVICE f32x4_t silu_rows(const Tile& t, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d,
-                             const int c_first, const bf16x8_t u, const uint16_t* __restrict__ b,
-                             const uint16_t* __restrict__ a, const float factor, int li, int lg) {
-  constexpr int NB = 4;  // groups whose loads are issued together
-  const uint16_t* g = x + (size_t)t.row * 2 * d + lg * 8;
-  uint16_t* o = out + (size_t)t.row * d + lg * 8;
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int i0 = 0; i0 < SILU_STRIP / (W * 32); i0 += NB) {
-    u16x8 gr[NB], ur[NB], ar[NB];
-    BOperand bg[NB], bu[NB];
+// A batch of columns on its way: rows and A's into LDS, B's operands.
+struct SiluBatch {
+  static constexpr int NB = SILU_BATCH / 32;
+  u16x8 gate[NB], up[NB];
+  int row[4];  // of tokens 4 j + lg, whose pieces this lane moves
+
+  LIG_DEVICE void issue(const uint16_t* x, const int d, const int c0, const uint16_t* b, const uint16_t* a, const uint16_t* room,
+                        int li, int lg) {
+    const uint32_t lds = lds_address(room);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int c0 = min(c_first + (i0 + i) * (W * 32), d - 32);  // groups past the end: the last one again, unused
-      gr[i] = load8(g + c0);
-      ur[i] = load8(g + d + c0);
-      if constexpr (LORA) {
-        bg[i] = load_b(b, c0, li, lg);
-        bu[i] = load_b(b, d + c0, li, lg);
-        ar[i] = load_a(a, d, c0, li, lg);
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int c = min(c0 + (li ^ (4 * j + lg)) * 8, d - 8);  // pieces past the end: the last one again, unused
+      load_to_lds(x + (size_t)row[j] * 2 * d + c, lds + j * 1024);
+      load_to_lds(x + (size_t)row[j] * 2 * d + d + c, lds + (4 + j) * 1024);
+      load_to_lds(a + (size_t)(4 * j + lg) * d + c, lds + (8 + j) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int c0 = c_first + (i0 + i) * (W * 32);
-      if (c0 >= d) break;
-      f32x8 gv = bf16x8_to_f32x8(gr[i]), uv = bf16x8_to_f32x8(ur[i]), r;
-      if constexpr (LORA) {
-        gv += expand(bg[i], u);
-        uv += expand(bu[i], u);
-      }
+      const int c = min(c0 + i * 32, d - 32);
+      gate[i] = load_b_once(b, c, li, lg);
+      up[i] = load_b_once(b, d + c, li, lg);
+    }
+  }
+
+  // acc + A out of the batch
+  LIG_DEVICE f32x4_t finish(const Tile& t, uint16_t* out, const int d, const int c0, const bf16x8_t u, const float factor,
+                            uint16_t* room, f32x4_t acc, int li, int lg) const {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (c0 + i * 32 >= d) break;
+      uint16_t* at = room + li * SILU_BATCH + ((i * 4 + lg) ^ li) * 8;
+      f32x8 gv = bf16x8_to_f32x8(load8(at)) + expand(both_halves(gate[i]), u), r;
+      f32x8 uv = bf16x8_to_f32x8(load8(at + 16 * SILU_BATCH)) + expand(both_halves(up[i]), u);
       gv *= 0.25f * factor;
       uv *= factor;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = silu_of_quarter(gv[j]) * uv[j];
+      for (int e = 0; e < 8; ++e) r[e] = silu_of_quarter(gv[e]) * uv[e];
       const u16x8 rb = f32x8_to_bf16x8(r);
-      if (t.valid) *reinterpret_cast<u16x8*>(o + c0) = rb;
-      if constexpr (LORA) acc = shrink(ar[i], rb, acc);
+      acc = shrink(load8(at + 32 * SILU_BATCH), rb, acc);
+      *reinterpret_cast<u16x8*>(at) = rb;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = c0 + (li ^ (4 * j + lg)) * 8;
+      const u16x8 rb = load8(room + (j * 64 + lg * 16 + li) * 8);
+      if (4 * j + lg < t.n && c < d) *reinterpret_cast<u16x8*>(out + (size_t)row[j] * d + c) = rb;
+    }
+    return acc;
+  }
+};
+
+// The columns c_first .. c_end of rows without an adapter, as they lie.
+LIG_DEVICE void silu_plain(const Tile& t, uint16_t* out, const uint16_t* x, const int d, const int c_first, const int c_end,
+                           const float factor, const int (&row)[4], int li, int lg) {
+  float own[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) own[j] = __shfl(factor, 4 * j + lg, 64);
+  for (int c0 = c_first; c0 < min(c_end, d); c0 += SILU_BATCH) {
+    const int c = min(c0 + li * 8, d - 8);  // pieces past the end: the last one again, unused
+    u16x8 gr[4], ur[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      gr[j] = load8(x + (size_t)row[j] * 2 * d + c);
+      ur[j] = load8(x + (size_t)row[j] * 2 * d + d + c);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x8 gv = bf16x8_to_f32x8(gr[j]), uv = bf16x8_to_f32x8(ur[j]), r;
+      gv *= 0.25f * own[j];
+      uv *= own[j];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = silu_of_quarter(gv[e]) * uv[e];
+      if (4 * j + lg < t.n && c0 + li * 8 < d) *reinterpret_cast<u16x8*>(out + (size_t)row[j] * d + c) = f32x8_to_bf16x8(r);
     }
   }
-  return acc;
 }
 
 // 8 waves take a strip in one pass each, 4 in two: faster where the workgroups find a
-// CU each, slower from there on, for a second of 8 waves fits a CU no more.  In steps of
-// 14 strips, 8 adapters (us with 8 and 4 waves): 96 decodes 10.6, 12.1; 256 (16 tiles)
-// 12.2, 18.4; 384 (24) 20.8, 19.2; prompts of 740 rows 30.9, 24.7; of 1108 50.6, 45.5; of
-// 1851 66.0, 61.4; 382 decodes and 2 prompts, 32 adapters 38.9, 31.8.
-template <int W>
+// CU each, slower from there on.  14 strips, weights of 8 or 32 adapters in no cache (us with
+// 8 and 4 waves): 96 rows 8.5, 10.2; 256 (16 tiles) 10.3, 12.2; 288 (24) 15.2, 13.6; 384
+// of 32 adapters 20.8, 18.7; 740 26.3, 21.4; 1851 56.1, 43.3.  As rows came in the products'
+// layout (and their fewer waves per CU notwithstanding): 384 rows of 32 adapters 20.4 -> 18.7,
+// 786 34.4 -> 28.8, 1500 of 5 48.0 -> 37.3, 4040 of 32 115.8 -> 91.5 (4.3 TB/s with the
+// adapters' weights once); without adapters 384 11.6 -> 10.5, 1000 24.3 -> 20.6.
+// Without LISTED no row has an adapter.
+template <int W, bool LISTED>
 __global__ __launch_bounds__(64 * W) void lora_silu_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const int d, const int* __restrict__ toks,
     const int* __restrict__ len, const int* __restrict__ slot,
     const float* __restrict__ u_in, const int parts, const int tiles, const uint16_t* __restrict__ b_stack,
     const uint16_t* __restrict__ a_stack, float* __restrict__ u_out, const int tiles_out, const Factor norm,
     const int rows) {
-  __shared__ __align__(16) float red[W][16][R];
   const int tile = place_of().tile, strip = place_of().strip;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const Tile t = tile_of(toks, len, slot, tile, li, rows);
+  const Tile t = tile_of(LISTED ? toks : nullptr, len, slot, tile, li, rows);
   if (t.n == 0) return;
-  const int c_first = strip * SILU_STRIP + wave * 32;
-  const float factor = factor_of(norm, tile, li);
-  if (t.slot < 0) {
-    silu_rows<false, W>(t, out, x, d, c_first, bf16x8_t{}, nullptr, nullptr, factor, li, lg);
+  const int c_first = strip * SILU_STRIP + wave * (SILU_STRIP / W), c_end = c_first + SILU_STRIP / W;
+  SiluBatch batch;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) batch.row[j] = LISTED ? __shfl(t.row, 4 * j + lg, 64) : tile * 16 + min(4 * j + lg, t.n - 1);
+  if (!LISTED || t.slot < 0) {
+    silu_plain(t, out, x, d, c_first, c_end, factor_of(norm, tile, li), batch.row, li, lg);
     return;
   }
-  const f32x4_t acc =
-      silu_rows<true, W>(t, out, x, d, c_first,
-                      u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid),
-                      b_stack + (size_t)t.slot * 2 * d * R, a_stack + (size_t)t.slot * R * d, factor, li, lg);
-  store_u<W>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+  if constexpr (LISTED) {
+    __shared__ __align__(16) float red[W][16][R];
+    __shared__ __align__(16) uint16_t rooms[W * SILU_ROOM];
+    uint16_t* room = rooms + wave * SILU_ROOM;
+    const uint16_t* b = b_stack + (size_t)t.slot * 2 * d * R;
+    const uint16_t* a = a_stack + (size_t)t.slot * R * d;
+    if (c_first < d) batch.issue(x, d, c_first, b, a, room, li, lg);
+    const float factor = factor_of(norm, tile, li);
+    const bf16x8_t u = u_of(u_in + (size_t)tile * 16 * R, parts, tiles, &red[0][0][0], li, lg, t.valid);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int c0 = c_first; c0 < min(c_end, d); c0 += SILU_BATCH) {
+      if (c0 > c_first) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the batch before has been read
+        batch.issue(x, d, c0, b, a, room, li, lg);
+      }
+      acc = batch.finish(t, out, d, c0, u, factor, room, acc, li, lg);
+    }
+    store_u<W>(u_out + ((size_t)strip * tiles_out + tile) * 16 * R, acc, red, wave, li, lg);
+  }
 }
 
 // u_out = A x, a part per strip of 512 columns
@@ -829,16 +906,22 @@ void lig_lora_silu_launch(uint16_t* out, const uint16_t* x, int d, const int* to
                           const int* slot, int ntiles, const float* u_in, int parts, int tiles,
                           const uint16_t* b_stack, const uint16_t* a_stack, float* u_out, int tiles_out,
                           const float* sums, int width, float eps, int rows, hipStream_t stream) {
-#define LAUNCH_A(W)                                                                                                  \
-  hipLaunchKernelGGL((lora_silu_kernel<W>), dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(64 * W), 0, stream, \
+#define LAUNCH_A1(W, LISTED)                                                                                         \
+  hipLaunchKernelGGL((lora_silu_kernel<W, LISTED>), dim3(ntiles, (d + SILU_STRIP - 1) / SILU_STRIP), dim3(64 * W), 0, stream, \
                      out, x, d, toks, len, slot, u_in, parts, tiles, b_stack, a_stack, u_out, tiles_out,             \
                      Factor{sums, width, eps}, rows)
+#define LAUNCH_A(W)               \
+  do {                            \
+    if (toks) LAUNCH_A1(W, true); \
+    else LAUNCH_A1(W, false);     \
+  } while (0)
   // A decode graph's list has room for one tile per adapter more than full ones, and of
   // those few are in use where adapters have about as many requests each
   const int likely = (ntiles + 3 * ((rows + 15) / 16)) / 4;
   if (likely * ((d + SILU_STRIP - 1) / SILU_STRIP) <= 256) LAUNCH_A(8);
   else LAUNCH_A(4);
 #undef LAUNCH_A
+#undef LAUNCH_A1
 }
 
 int lig_lora_shrink_strip() { return SHRINK_STRIP; }
