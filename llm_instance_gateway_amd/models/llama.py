@@ -326,19 +326,29 @@ class LlamaForCausalLM(nn.Module):
         return True
 
     def _forward_row(self, hidden, positions, kv_caches, meta: BatchMeta) -> torch.Tensor:
-        """The layers for a single token: norms and the activation live in the
-        projections' kernels."""
+        """The layers for a single token: norms, the activation, the rotation and what
+        merges the parts of the attention's walk live in the projections' kernels."""
         residual, x = None, hidden
+        rotates = self.cfg.head_dim % 64 == 0
         for layer, kv in zip(self.layers, kv_caches):
             attn, mlp = layer.self_attn, layer.mlp
-            if residual is None:
-                qkv = ops.row_product(x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps)
-                residual = x
+            if rotates:
+                q = ops.row_product_heads(
+                    x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps, residual, positions, self.cos_sin_cache, kv[0],
+                    kv[1], meta.slot_mapping, attn.num_heads)
+                q, residual = (q, x) if residual is None else q
             else:
-                qkv, residual = ops.row_product(x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps, residual)
-            q = ops.qkv_rope_cache(
-                qkv, positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping, attn.num_heads)
-            o = ops.row_product(attn.attend(q, kv, meta), attn.o_proj.weight)
+                qkv = ops.row_product(x, attn.qkv_proj.weight, layer.input_layernorm, layer.eps, residual)
+                qkv, residual = (qkv, x) if residual is None else qkv
+                q = ops.qkv_rope_cache(
+                    qkv, positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping, attn.num_heads)
+            if meta.num_decode_tokens == 1:
+                a, parts = ops.paged_attention_decode_open(
+                    q.view(1, attn.num_heads, -1), kv[0], kv[1], meta.decode_block_tables, meta.decode_context_lens, attn.scale,
+                    meta.max_decode_ctx, meta.decode_nsplits)
+            else:
+                a, parts = attn.attend(q, kv, meta), None
+            o = ops.row_product(a, attn.o_proj.weight, parts=parts)
             act, residual = ops.row_product(
                 o, mlp.gate_up_proj.weight, layer.post_attention_layernorm, layer.eps, residual, silu=True)
             x = ops.row_product(act, mlp.down_proj.weight)

@@ -213,6 +213,30 @@ def paged_attention_decode(
     return res if out is None else out.copy_(res)
 
 
+# Up to that many parts of a walk are merged by every workgroup of the product behind: attention
+# and a product of 4096 x 4096, 32 heads of 128, merged by a launch and by the product, 381
+# keys of at most 4 parts 17.8 us, 16.2 (in one part: the launch has nothing to do); 1100
+# 21.2, 20.1; 2000 22.9, 22.8; 4000 26.3, 27.2; but 4000 and 8000 of at most 16 24.6, 27.2
+# and 27.7, 37.4.
+_OPEN_PARTS = 4
+
+
+def paged_attention_decode_open(
+    q: torch.Tensor, k_cache, v_cache, block_tables, context_lens, scale: float, max_ctx: int = 0, nsplits: int = 0
+):
+    """The same of one row for `row_product`, which merges the parts of a walk by itself: the
+    row [1, heads * D], whole or not, and what it takes to merge it.  GPU."""
+    N, Hq, D = q.shape
+    ns = nsplits if nsplits > 0 else decode_nsplits(N, k_cache.shape[1], max_ctx)
+    if ns <= 1 or ns > _OPEN_PARTS:
+        return paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, nsplits=ns).view(1, -1), None
+    out = torch.empty_like(q)
+    scratch = split_scratch(q.device, N * Hq * ns * (D + 2))
+    _EXT.paged_attention_decode_open(
+        out, q, k_cache, v_cache, block_tables, context_lens, scratch, scale, ns, _stream())
+    return out.view(1, -1), (scratch, context_lens, ns, D)
+
+
 def paged_attention_prefill(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -325,14 +349,27 @@ def row_product_serves(weight: torch.Tensor, norm: bool, most: Optional[tuple] =
     )
 
 
-def row_product(x, weight, norm=None, eps=0.0, residual=None, silu=False):
+def row_product(x, weight, norm=None, eps=0.0, residual=None, silu=False, parts=None):
     """weight @ h of one row x [1, K]: h = x, or rms_norm(x + residual) * norm;
     with silu, silu(gate) * up of the product's halves.  Returns the product and,
-    where a residual was given, x + residual."""
+    where a residual was given, x + residual.  parts: of an x that may be in parts
+    (`paged_attention_decode_open`)."""
     y = torch.empty(1, weight.shape[0] // (2 if silu else 1), dtype=x.dtype, device=x.device)
     out = None if residual is None else torch.empty_like(residual)
-    _EXT.row_product(y, weight, x, residual, out, norm, eps, silu, _stream())
+    _EXT.row_product(y, weight, x, residual, out, norm, eps, silu, *(parts or (None, None, 0, 0)), _stream())
     return y if out is None else (y, out)
+
+
+def row_product_heads(
+    x, weight, norm, eps, residual, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, num_heads: int
+):
+    """`row_product` of a norm with a fused q, k and v projection, and `qkv_rope_cache` of the
+    product.  Returns q and, where a residual was given, x + residual."""
+    q = torch.empty(1, num_heads * k_cache.shape[-1], dtype=x.dtype, device=x.device)
+    out = None if residual is None else torch.empty_like(residual)
+    _EXT.row_product_heads(
+        q, weight, x, residual, out, norm, eps, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, _stream())
+    return q if out is None else (q, out)
 
 
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:

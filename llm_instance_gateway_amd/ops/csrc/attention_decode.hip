@@ -89,13 +89,14 @@ __global__ __launch_bounds__(4 * WAVE_SIZE) void paged_attention_decode_16_kerne
   }
 }
 
-// scratch: fp32 [N, Hq, nsplits, D + 2] where nsplits > 1, else unused
+// scratch: fp32 [N, Hq, nsplits, D + 2] where nsplits > 1, else unused.  Unmerged, rows
+// that were cut are left there for their reader.
 extern "C" void lig_paged_attention_decode_launch(
     uint16_t* out, const uint16_t* q, const uint16_t* k_cache,
     const uint16_t* v_cache, const int* block_tables,
     const int* context_lens, float* scratch, float scale, int num_seqs,
     int num_q_heads, int num_kv_heads, int head_dim, int block_size,
-    int max_blocks, int nsplits, hipStream_t stream) {
+    int max_blocks, int nsplits, int unmerged, hipStream_t stream) {
   flash_decode::Args a{};
   a.out = out;
   a.q = q;
@@ -115,6 +116,7 @@ extern "C" void lig_paged_attention_decode_launch(
   a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
   a.nsplits = nsplits;
+  a.unmerged = unmerged;
   if (head_dim == 16) {
     hipLaunchKernelGGL(paged_attention_decode_16_kernel, dim3(num_seqs, (num_q_heads + 3) / 4, nsplits),
                        dim3(4 * WAVE_SIZE), 0, stream, a);

@@ -63,14 +63,17 @@ int lig_projection_tile(int);
 void lig_projection_launch(int, uint16_t*, float*, const uint16_t*, const uint16_t*, int, int, int, hipStream_t);
 int lig_row_product_max(bool);
 void lig_row_product_launch(uint16_t*, const uint16_t*, int, int, const uint16_t*, const uint16_t*, uint16_t*,
-                            const uint16_t*, float, bool, hipStream_t);
+                            const uint16_t*, float, bool, const float*, const int*, int, int, hipStream_t);
+void lig_row_product_heads_launch(uint16_t*, const uint16_t*, int, int, const uint16_t*, const uint16_t*, uint16_t*,
+                                  const uint16_t*, float, const int64_t*, const float*, uint16_t*, uint16_t*,
+                                  const int64_t*, int, int, int, int, hipStream_t);
 void lig_argmax_rows_launch(const void*, bool, long, int, int, int64_t*, hipStream_t);
 void lig_silu_and_mul_launch(uint16_t*, const uint16_t*, int, int,
                              hipStream_t);
 void lig_paged_attention_decode_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*,
     const int*, const int*, float*, float, int, int, int, int, int, int,
-    int, hipStream_t);
+    int, int, hipStream_t);
 void lig_mfma_probe_launch(float*, const uint16_t*, const uint16_t*,
                            hipStream_t);
 void lig_sgmv_shrink_launch(uint16_t*, const uint16_t*, const uint16_t*,
@@ -229,7 +232,8 @@ void qkv_rope_cache(torch::Tensor q_out, torch::Tensor qkv,
 // residual_out) with `weight`; silu: W = [gate | up], y = silu(gate h) * (up h).
 void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optional<torch::Tensor> residual,
                  c10::optional<torch::Tensor> residual_out, c10::optional<torch::Tensor> weight, double eps, bool silu,
-                 int64_t stream) {
+                 c10::optional<torch::Tensor> scratch, c10::optional<torch::Tensor> context_lens, int64_t nsplits,
+                 int64_t head_dim, int64_t stream) {
   TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && w.size(0) < (1 << 30));
   const int N = (int)w.size(0), K = (int)w.size(1);
   TORCH_CHECK(K > 0 && K % 512 == 0 && K <= lig_row_product_max(weight.has_value()), "width ", K);
@@ -241,9 +245,44 @@ void row_product(torch::Tensor y, torch::Tensor w, torch::Tensor x, c10::optiona
   TORCH_CHECK(residual.has_value() == residual_out.has_value() && (weight.has_value() || !residual.has_value()));
   TORCH_CHECK(((uintptr_t)w.data_ptr() & 15) == 0);
   TORCH_CHECK(y.is_contiguous() && y.numel() == (silu ? N / 2 : N));
+  if (scratch) {
+    TORCH_CHECK(!weight && context_lens && context_lens->scalar_type() == torch::kInt32 && context_lens->numel() >= 1);
+    TORCH_CHECK(head_dim > 0 && head_dim % 8 == 0 && K % head_dim == 0 && nsplits >= 1 &&
+                scratch->scalar_type() == torch::kFloat32 && scratch->numel() >= K / head_dim * nsplits * (head_dim + 2));
+  }
   lig_row_product_launch(bf16_ptr(y), bf16_cptr(w), N, K, row(x, K), residual ? row(*residual, K) : nullptr,
                          residual_out ? row(*residual_out, K) : nullptr, weight ? row(*weight, K) : nullptr, (float)eps,
-                         silu, as_stream(stream));
+                         silu, scratch ? scratch->data_ptr<float>() : nullptr,
+                         scratch ? context_lens->data_ptr<int>() : nullptr, (int)nsplits, (int)head_dim, as_stream(stream));
+}
+
+// The same product of a norm with a fused q, k and v projection, whose heads go where
+// qkv_rope_cache puts them.
+void row_product_heads(torch::Tensor q_out, torch::Tensor w, torch::Tensor x, c10::optional<torch::Tensor> residual,
+                       c10::optional<torch::Tensor> residual_out, torch::Tensor weight, double eps, torch::Tensor positions,
+                       torch::Tensor cos_sin, torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor slot_mapping,
+                       int64_t stream) {
+  TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && w.size(0) < (1 << 30) && ((uintptr_t)w.data_ptr() & 15) == 0);
+  const int N = (int)w.size(0), K = (int)w.size(1);
+  TORCH_CHECK(K > 0 && K % 512 == 0 && K <= lig_row_product_max(true), "width ", K);
+  auto row = [&](torch::Tensor t, int n) {
+    TORCH_CHECK(t.is_contiguous() && t.numel() == n && ((uintptr_t)t.data_ptr() & 15) == 0, "a contiguous row of ", n);
+    return bf16_ptr(t);
+  };
+  TORCH_CHECK(residual.has_value() == residual_out.has_value());
+  TORCH_CHECK(positions.scalar_type() == torch::kInt64 && slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(positions.numel() >= 1 && slot_mapping.numel() >= 1);
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 && cos_sin.is_contiguous());
+  TORCH_CHECK(k_cache.dim() == 4 && v_cache.sizes() == k_cache.sizes() && k_cache.is_contiguous() && v_cache.is_contiguous());
+  const int Hkv = (int)k_cache.size(1), D = (int)k_cache.size(3);
+  TORCH_CHECK(D % 64 == 0 && cos_sin.size(1) == D && q_out.is_contiguous() && q_out.numel() % D == 0);
+  const int Hq = (int)(q_out.numel() / D);
+  TORCH_CHECK(N == (Hq + 2 * Hkv) * D, "w must hold the query, key and value heads");
+  lig_row_product_heads_launch(bf16_ptr(q_out), bf16_cptr(w), N, K, row(x, K), residual ? row(*residual, K) : nullptr,
+                               residual_out ? row(*residual_out, K) : nullptr, row(weight, K), (float)eps,
+                               positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), bf16_ptr(k_cache),
+                               bf16_ptr(v_cache), slot_mapping.data_ptr<int64_t>(), Hq, Hkv, D, (int)k_cache.size(2),
+                               as_stream(stream));
 }
 
 // Whether a dispatch mode, a trace or a transform follows what is called
@@ -345,11 +384,13 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   lig_paged_attention_decode_launch(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k_cache), bf16_cptr(v_cache),
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(), nullptr,
-      (float)scale, N, Hq, Hkv, D, BS, max_blocks, 1, as_stream(stream));
+      (float)scale, N, Hq, Hkv, D, BS, max_blocks, 1, 0, as_stream(stream));
 }
 
 // Flash-decoding variant: every context cut over up to nsplits workgroups with
-// an fp32 partial scratch [N, Hq, nsplits, D+2] and a merging pass.
+// an fp32 partial scratch [N, Hq, nsplits, D+2] and a merging pass, or without
+// that for a reader that merges by itself.
+template <bool MERGE>
 void paged_attention_decode_split(torch::Tensor out, torch::Tensor q,
                                   torch::Tensor k_cache,
                                   torch::Tensor v_cache,
@@ -376,7 +417,7 @@ void paged_attention_decode_split(torch::Tensor out, torch::Tensor q,
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k_cache), bf16_cptr(v_cache),
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(),
       scratch.data_ptr<float>(), (float)scale, N, Hq, Hkv, D, BS,
-      max_blocks, (int)nsplits, as_stream(stream));
+      max_blocks, (int)nsplits, !MERGE, as_stream(stream));
 }
 
 void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
@@ -935,9 +976,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("projection_takes", &projection_takes);
   m.def("projection_takes_rows", &projection_takes_rows);
   m.def("row_product", &row_product);
+  m.def("row_product_heads", &row_product_heads);
   m.def("row_product_max", &lig_row_product_max);
   m.def("paged_attention_decode", &paged_attention_decode);
-  m.def("paged_attention_decode_split", &paged_attention_decode_split);
+  m.def("paged_attention_decode_split", &paged_attention_decode_split<true>);
+  m.def("paged_attention_decode_open", &paged_attention_decode_split<false>);
   m.def("paged_attention_prefill", &paged_attention_prefill);
   m.def("paged_attention_prefill_parts", &lig_paged_attention_prefill_parts);
   m.def("sgmv_shrink", &sgmv_shrink);

@@ -77,6 +77,7 @@ struct Args {
   int gate_per_head;
   float softcap;
   int nsplits;
+  int unmerged;             // whoever reads the result merges the parts
 };
 
 // The steps of a row: its position and lower bound, and into how many parts
@@ -85,6 +86,7 @@ struct Args {
 struct Walk {
   int seq, pos, key_lo, first, steps, parts;
 };
+LIG_DEVICE int parts_of(int steps, int nsplits) { return max(1, min(nsplits, steps / 16)); }
 template <bool EXTRA>
 LIG_DEVICE Walk walk_of(const Args& a, int row) {
   Walk w;
@@ -97,7 +99,7 @@ LIG_DEVICE Walk walk_of(const Args& a, int row) {
   }
   w.first = w.key_lo / KT;
   w.steps = w.pos < 0 ? 0 : w.pos / KT + 1 - w.first;
-  w.parts = max(1, min(a.nsplits, w.steps / 16));
+  w.parts = parts_of(w.steps, a.nsplits);
   return w;
 }
 
@@ -496,7 +498,7 @@ static inline bool serves(const Args& a, int D, int Dv) {
 
 template <int D, bool SIG, bool EXTRA>
 static void launch_merge(const Args& a, hipStream_t stream) {
-  if (a.nsplits <= 1) return;
+  if (a.nsplits <= 1 || a.unmerged) return;
   const long lanes = (long)a.rows * a.num_q_heads * (D / 4);
   hipLaunchKernelGGL((flash_decode_merge_kernel<D, SIG, EXTRA>), dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0,
                      stream, a);

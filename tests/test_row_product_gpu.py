@@ -88,3 +88,49 @@ def test_single_decode_matches_layer_kernels(monkeypatch):
         outs.append(torch.cat(logits))
     # two correct orders of bf16 rounding, 3 layers deep
     assert (outs[0] - outs[1]).norm() <= 0.03 * outs[1].norm()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,BS", [(64, 3, 1, 16), (128, 8, 2, 16), (128, 4, 4, 24), (192, 2, 1, 8)])
+@pytest.mark.parametrize("slot", [0, 37, -1])  # of 40 and more
+def test_heads_of_a_row(D, Hq, Hkv, BS, slot):
+    """The product whose heads go where the rotation puts them, against the two by themselves."""
+    g = torch.Generator("cuda").manual_seed(D + Hq + BS + slot)
+    K, N = 1024, (Hq + 2 * Hkv) * D
+    x, res = _rnd(g, 1, K).to(BF), _rnd(g, 1, K).to(BF)
+    w, nw = (_rnd(g, N, K) * K ** -0.5).to(BF), (1 + 0.1 * _rnd(g, K)).to(BF)
+    cs = ops.build_cos_sin_cache(D, 64, 10000.0, "cuda").float()
+    pos, at = torch.tensor([29], device="cuda"), torch.tensor([slot], device="cuda")
+    for residual in (None, res):
+        caches = [[torch.full((5, Hkv, BS, D), 3.0, dtype=BF, device="cuda") for _ in "kv"] for _ in "ab"]
+        got = ops.row_product_heads(x, w, nw, 1e-5, residual, pos, cs, *caches[0], at, Hq)
+        y = ops.row_product(x, w, nw, 1e-5, residual)
+        if residual is not None:
+            got, r = got
+            y, want_r = y
+            assert torch.equal(r, want_r)
+        want = ops.qkv_rope_cache(y, pos, cs, *caches[1], at, Hq)
+        # one product of the two is rounded to 24 bits before it is added, either one: 2^-24
+        # of it, which may cross one rounding to 8 bits
+        for a, b in ((got, want), (caches[0][0], caches[1][0])):
+            a, b = a.float(), b.float()
+            assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-6).all() and (a != b).float().mean() < 1e-2
+        assert torch.equal(caches[0][1], caches[1][1])
+        if slot < 0:
+            assert (caches[0][0] == 3).all() and (caches[0][1] == 3).all()
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("ctx", [1, 700, 1023, 1024, 2077])
+@pytest.mark.parametrize("nsplits", [1, 2, 4, 16])
+def test_parts_of_a_walk(D, ctx, nsplits):
+    """A product that merges an attention's parts, against the one of the merged row: the same bits."""
+    g = torch.Generator("cuda").manual_seed(D + ctx + nsplits)
+    Hq, Hkv, BS = 1024 // D, 1024 // D // 4, 16
+    nb = (ctx + BS - 1) // BS
+    q, w = _rnd(g, 1, Hq, D).to(BF), (_rnd(g, 264, Hq * D) / 32).to(BF)
+    k, v = (_rnd(g, nb, Hkv, BS, D).to(BF) for _ in "kv")
+    table = torch.randperm(nb, generator=g, device="cuda").int().view(1, -1)
+    args = (q, k, v, table, torch.tensor([ctx], dtype=torch.int32, device="cuda"), D ** -0.5)
+    want = ops.row_product(ops.paged_attention_decode(*args, nsplits=nsplits).view(1, -1), w)
+    x, parts = ops.paged_attention_decode_open(*args, nsplits=nsplits)
+    assert torch.equal(ops.row_product(x, w, parts=parts), want)
