@@ -60,6 +60,7 @@ bool lig_projection_pays(long, long, long);
 int lig_projection_plan(int, int, int);
 int lig_projection_splits(int);
 int lig_projection_tile(int);
+int lig_projection_runs(int, int, int, int);
 void lig_projection_launch(int, uint16_t*, float*, const uint16_t*, const uint16_t*, int, int, int, hipStream_t);
 int lig_row_product_max(bool);
 void lig_row_product_launch(uint16_t*, const uint16_t*, int, int, const uint16_t*, const uint16_t*, uint16_t*,
@@ -335,11 +336,18 @@ torch::Tensor projection_parts(torch::Tensor x, torch::Tensor w, int64_t stream)
   return part;
 }
 
-// (rows of y, columns of y) of the tile that a served size runs on, and the parts of K
+// (rows of y, columns of y) of the tile that a served size is planned for, and the parts of K
 std::tuple<int, int, int> projection_plan(int M, int N, int K) {
   TORCH_CHECK(lig_projection_serves(M, N, K), "shape");
   const int plan = lig_projection_plan(M, N, K), tile = lig_projection_tile(plan);
   return {tile / 1000, tile % 1000, lig_projection_splits(plan)};
+}
+
+// and of the tile that runs in its place, or its own
+std::tuple<int, int> projection_runs(int M, int N, int K) {
+  TORCH_CHECK(lig_projection_serves(M, N, K), "shape");
+  const int tile = lig_projection_runs(lig_projection_plan(M, N, K), M, N, K);
+  return {tile / 1000, tile % 1000};
 }
 
 void argmax_rows(torch::Tensor out, torch::Tensor x, int64_t stream) {
@@ -971,6 +979,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("projection", &projection);
   m.def("projection_parts", &projection_parts);
   m.def("projection_plan", &projection_plan);
+  m.def("projection_runs", &projection_runs);
   m.def("projection_serves", &lig_projection_serves);
   m.def("projection_pays", &lig_projection_pays);
   m.def("projection_takes", &projection_takes);

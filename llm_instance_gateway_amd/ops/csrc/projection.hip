@@ -418,6 +418,26 @@ __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restric
   X(224, 256, 2)          \
   X(256, 256, 2)
 
+// And tiles that run in the place of one of these, with the same parts of K, where the
+// estimate is 3 % lower: of 224 and 288 columns where 28672 outputs are 112 tiles of 256
+// each row of tiles and leave the chip's last turn half empty, and other products likewise.
+// Llama-3-8B's gate_up (us, before -> after; launch behind launch, and between copies): 384
+// rows 79.6 -> 74.6, 83.7 -> 82.3; 512 97 -> 95, 93.5 -> 92.5; 786 166 -> 151, 163 -> 152; 1000 184 -> 180,
+// 180 -> 172.  They run 91 of 527 sizes of 19 projections at 48 to 1024 rows, 7 % faster in the
+// mean launch behind launch, one of them 1 % slower.  Stages of x and W by loaders of their own,
+// W's up to eight ahead, changed nothing (gate_up at 202 rows 54.5 us and 57): under that
+// load the chip runs at 1.7 to 1.9 GHz, and at 2.0 without any loads.
+#define LIG_OTHER_TILES(X) \
+  X(160, 224, 2)           \
+  X(160, 288, 2)           \
+  X(192, 128, 3)           \
+  X(192, 224, 2)           \
+  X(224, 192, 2)           \
+  X(224, 224, 2)           \
+  X(256, 192, 2)           \
+  X(256, 224, 2)           \
+  X(288, 224, 2)
+
 struct TileShape {
   int bm, bn, k_step;
 };
@@ -429,7 +449,13 @@ constexpr TileShape TILES[] = {
     LIG_WIDE_TILES(X)
 #undef X
 };
+constexpr TileShape OTHER_TILES[] = {
+#define X(BM, BN, SX) {BM, BN, 64},
+    LIG_OTHER_TILES(X)
+#undef X
+};
 constexpr int FEW = 3;  // tiles of the first kind
+constexpr int TILE_COUNT = sizeof(TILES) / sizeof(TILES[0]), OTHER_COUNT = sizeof(OTHER_TILES) / sizeof(OTHER_TILES[0]);
 constexpr int MAX_SPLITS = 8;
 constexpr int CUS = 256;
 
@@ -449,27 +475,33 @@ struct Cost {
 constexpr Cost FEW_COST = {0.0005405, -0.005728, -0.0135, 0.2466, 3.263, 0.1869, 8.987, -0.6106, 3.765};
 constexpr Cost WIDE_COST = {9.45e-06, 0.001368, 0.001277, 0.004109, 0.9942, 2.333, 7.596, -0.2958, 1.212};
 
+double estimate(const TileShape& s, const Cost& c, int splits, int M, int N, int K) {
+  const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+  const double step = s.bm * s.bn * c.area + s.bn * c.w_row + s.bm * c.x_row + c.step;
+  const double stream = N * (double)K * 2e-6 / c.hbm;
+  const double work = (tiles * splits + CUS - 1) / CUS * (K / 64.0 / splits * step + c.tile);
+  const double t = c.launch + sqrt(work * work + stream * stream);
+  return splits > 1 ? t + c.cut + c.sum * 1e-6 * splits * M * N : t;
+}
+
+// Tall tiles that would be mostly padding were not measured.
+bool padding(const TileShape& s, int M) { return s.bm > 64 && 5 * M < 3 * s.bm; }
+
 // The first tiles are for small weights: 16 rows of 28672 x 4096 take 41 us on them, 36
-// on tiles of 64 x 128; of 4096 x 4096 both 7.7; of 2048 x 2048 4.1 and 4.7.  Tall tiles that
-// would be mostly padding were not measured.
+// on tiles of 64 x 128; of 4096 x 4096 both 7.7; of 2048 x 2048 4.1 and 4.7.
 Plan plan(int M, int N, int K) {
   // one wave of workgroups after the other, each over in a few us: 1 row of 128256 x 4096
   // 149 us, 153 to 156 on the next best tiles; 8 rows of 57344 x 8192 140, 149; 16 rows level
   if (M <= 8 && N > 32768 && K % TILES[0].k_step == 0) return {0, 1};
   Plan best = {-1, 0};
   double least = 0;
-  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+  for (int i = 0; i < TILE_COUNT; ++i) {
     const TileShape& s = TILES[i];
-    if (K % s.k_step || (i < FEW ? (long)N * K >= 1L << 24 : s.bm > 64 && 5 * M < 3 * s.bm)) continue;
-    const Cost& c = i < FEW ? FEW_COST : WIDE_COST;
+    if (K % s.k_step || (i < FEW ? (long)N * K >= 1L << 24 : padding(s, M))) continue;
     const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-    const double step = s.bm * s.bn * c.area + s.bn * c.w_row + s.bm * c.x_row + c.step;
-    const double stream = N * (double)K * 2e-6 / c.hbm;
     for (int splits = 1; splits <= MAX_SPLITS; ++splits) {
       if (splits > 1 && (tiles * splits > 2 * CUS + 88 || K / s.k_step / splits < 6)) break;
-      const double work = (tiles * splits + CUS - 1) / CUS * (K / 64.0 / splits * step + c.tile);
-      double t = c.launch + sqrt(work * work + stream * stream);
-      if (splits > 1) t += c.cut + c.sum * 1e-6 * splits * M * N;
+      const double t = estimate(s, i < FEW ? FEW_COST : WIDE_COST, splits, M, N, K);
       if (best.tile < 0 || t < least) {
         least = t;
         best = {i, splits};
@@ -477,6 +509,22 @@ Plan plan(int M, int N, int K) {
     }
   }
   return best;
+}
+
+// The tile that runs a plan: its own, or TILE_COUNT and more for one of the others.
+int tile_of(const Plan& p, int M, int N, int K) {
+  if (p.tile < FEW || M > 1024) return p.tile;  // not measured
+  int tile = p.tile;
+  double least = 0.97 * estimate(TILES[tile], WIDE_COST, p.splits, M, N, K);
+  for (int i = 0; i < OTHER_COUNT; ++i) {
+    if (padding(OTHER_TILES[i], M)) continue;
+    const double t = estimate(OTHER_TILES[i], WIDE_COST, p.splits, M, N, K);
+    if (t < least) {
+      least = t;
+      tile = TILE_COUNT + i;
+    }
+  }
+  return tile;
 }
 
 struct Product {
@@ -558,7 +606,7 @@ bool lig_projection_pays(long M, long N, long K) {
   return (K <= 4096 && N >= 8192 && N <= 32768) || N * K >= 1L << 28;
 }
 
-// Tile and parts of K, as one number.  To launch it: y alone where K is in one part,
+// Tile and parts of K, as one number.  To launch it, on that tile or one in its place: y alone where K is in one part,
 // y and room for the fp32 sums [parts, M, N], or that room alone, which then holds the
 // parts for the caller to add up.
 int lig_projection_plan(int M, int N, int K) {
@@ -567,10 +615,15 @@ int lig_projection_plan(int M, int N, int K) {
 }
 int lig_projection_splits(int p) { return p % (MAX_SPLITS + 1); }
 int lig_projection_tile(int p) { return TILES[p / (MAX_SPLITS + 1)].bm * 1000 + TILES[p / (MAX_SPLITS + 1)].bn; }
+int lig_projection_runs(int p, int M, int N, int K) {
+  const int tile = tile_of({p / (MAX_SPLITS + 1), p % (MAX_SPLITS + 1)}, M, N, K);
+  const TileShape& s = tile < TILE_COUNT ? TILES[tile] : OTHER_TILES[tile - TILE_COUNT];
+  return s.bm * 1000 + s.bn;
+}
 
 void lig_projection_launch(int p, uint16_t* y, float* part, const uint16_t* x, const uint16_t* w, int M, int N, int K,
                            hipStream_t stream) {
-  const int tile = p / (MAX_SPLITS + 1), splits = p % (MAX_SPLITS + 1);
+  const int splits = p % (MAX_SPLITS + 1), tile = tile_of({p / (MAX_SPLITS + 1), splits}, M, N, K);
   int i = 0;
   const Product a = {y, part, x, w, M, N, K, stream};
 #define X(BM, BN, ST) \
@@ -580,6 +633,7 @@ void lig_projection_launch(int p, uint16_t* y, float* part, const uint16_t* x, c
 #define X(BM, BN, SX) \
   if (tile == i++) launch_wide<BM, BN, SX>(a, splits);
   LIG_WIDE_TILES(X)
+  LIG_OTHER_TILES(X)
 #undef X
   if (part && y) {
     const long n = (long)M * N;

@@ -195,3 +195,24 @@ def test_watched_products_stay_with_the_library():
         assert "linear" in names
         with torch.device("cuda"):
             assert ops.linear_served(8, w) and ops.linear_parts(x, w).dim() == 3
+
+
+# tiles that run in another's place: in one part and in several, weights past the caches and not
+OTHERS = [
+    (129, 33128, 128), (129, 33128, 576), (289, 8200, 3072), (129, 16392, 3072), (225, 33128, 64), (769, 7176, 8192),
+    (161, 24584, 128), (161, 24584, 1024), (897, 2056, 8192), (161, 8200, 4096), (897, 11272, 3072), (513, 3080, 14336),
+    (161, 16392, 3072), (193, 33128, 64), (161, 33128, 576), (641, 7176, 8192), (161, 22536, 8192), (641, 16392, 3072),
+    (385, 8200, 4096), (193, 16392, 4096), (225, 40968, 64), (225, 40968, 576), (705, 16392, 3072), (705, 3080, 14336),
+    (225, 16392, 4096), (769, 16392, 3072), (257, 40968, 3072), (786, 28672, 4096),
+]
+
+
+@pytest.mark.parametrize("M,N,K", OTHERS)
+def test_tiles_in_the_place_of_others(M, N, K):
+    ext = ops._load_ext()
+    assert ext.projection_runs(M, N, K) != ext.projection_plan(M, N, K)[:2]
+    test_projection(M, N, K)
+
+
+def test_other_tiles_are_reached():
+    assert len({ops._load_ext().projection_runs(*s) for s in OTHERS}) == 9
