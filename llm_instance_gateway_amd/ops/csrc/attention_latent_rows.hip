@@ -34,9 +34,11 @@
 // Measured with rows of 576 and values of 512 (us; a kernel that staged through
 // registers -> with the builtin -> now): 256 single tokens on 700-1024 keys, 32
 // heads 148 -> 72 -> 63 (255 MB of rows, 4.1 TB/s); 4 prompts of 700-1000, 16 heads
-// 322 -> 121 -> 97 (546 TFLOP/s). Two row blocks per wave, which halve the LDS
+// 322 -> 121 -> 97 (546 TFLOP/s; with the tiles dealt by length 83). Two row blocks per wave, which halve the LDS
 // reads, lost more by leaving one wave per SIMD (keys of 320: 372 us before, 136
 // now, 208 so; of 128: 149, 73, 135).
+// Weights handed to all waves, so that each adds up a quarter of the columns of all rows and
+// reads a quarter of the values from LDS, cost a second barrier and changed nothing (101 and 99 us).
 // Scores, running max and sum are fp32; an optional per-head sink starts a
 // row's running max at sink_h and its sum at one; an optional gate multiplies
 // the (token, head) output row by one sigmoid (it commutes with whatever
@@ -45,8 +47,8 @@
 // window > 0 restricts a row at position p to keys j with p - j < window; a
 // tile's walk starts at the oldest key its first token sees.
 //
-// Grid = (ceil(max segment rows / 64 or 32), segments, splits); workgroups past a
-// segment's last row exit at once.  With splits > 1 (few rows, long
+// Grid = (ceil(max segment rows / 64 or 32), segments, splits), dealt anew by `deal`; workgroups
+// without a tile exit at once.  With splits > 1 (few rows, long
 // contexts) each z-slice walks an equal share of the tile's visible keys and
 // leaves its unnormalised sum with its running max and sum in an fp32
 // scratch; a second kernel merges the slices.  The sink is counted by slice
@@ -63,8 +65,62 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_of8 __attribute__((ext_vector_type(4), aligned(8)));  // outputs are not asked for more
 
 constexpr int LR_PART_PAD = 4;  // a slice row is Dv values, running max (log2 units), running sum, 2 unused
+
+// Workgroups begin in the order of x, then y, one to each XCD in turn, and one whose
+// XCD is full holds up the others.  Segment for segment, a late one's longest walks
+// began when the others were at their last, and empty workgroups between left XCDs
+// unevenly full.  So the tiles that have rows are dealt by their number in the segment, the
+// highest of all segments first.  Of 4 prompts of 700-1000 with 16 heads 512 workgroups ran for
+// 60 us and less and less of them for 38 more: 94 -> 83 us, with results in 16-byte pieces and
+// one round of loads ahead of the block table less; 8 of them 197 -> 174, 16 of 70-100 23.1 -> 19.9.
+// More than 16 segments, whose keys would no longer stay in the L2 (64 prompts of 210-300: 190 us
+// in their order, 249 dealt), and single tiles stay as they are.  False: no tile is left.
+struct Walk {
+  int seg, tile, n, start, ctx;
+};
+LIG_DEVICE bool deal(const int* seg_start, const int* seg_len, const int* seg_ctx, int H, int rows, Walk& w) {
+  const unsigned segs = gridDim.y, most = gridDim.x;
+  if (most == 1 || segs == 1 || segs > 16 || most > 65535) {
+    w.seg = blockIdx.y;
+    w.tile = most - 1 - blockIdx.x;
+    w.n = seg_len[w.seg];
+    w.start = seg_start[w.seg];
+    w.ctx = seg_ctx[w.seg];
+    return (long)w.tile * rows < (long)w.n * H;
+  }
+  const int lane = threadIdx.x & 63, at = min(lane, (int)segs - 1);
+  const int n = seg_len[at], start = seg_start[at], ctx = seg_ctx[at];
+  // of this lane's segment
+  const int tiles = lane < (int)segs && n > 0 ? (int)min((long)most, ((long)n * H + rows - 1) / rows) : 0;
+  auto from = [&](int t) {  // tiles numbered t and higher: under 2^21
+    int c = 0;
+    for (unsigned g = 0; g < segs; ++g) c += max(__builtin_amdgcn_readlane(tiles, g) - t, 0);
+    return c;
+  };
+  const int i = blockIdx.y * most + blockIdx.x;
+  if (i >= __builtin_amdgcn_readfirstlane(from(0))) return false;
+  // the last number from which on there are more than i tiles: of 64 at a time
+  int lo = 0;
+  for (int width = most; width > 1;) {
+    const int step = (width + 63) / 64, t = lo + lane * step;
+    lo += (__popcll(__ballot(lane * step < width && from(t) > i)) - 1) * step;
+    width = step;
+  }
+  // the segments that have tile lo, in their order
+  const int k = i - __builtin_amdgcn_readfirstlane(from(lo + 1));
+  const uint64_t have = __ballot(tiles > lo);
+  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0));
+  const uint64_t mine = __ballot(tiles > lo && before == k);
+  w.seg = __builtin_ctzll(mine);
+  w.tile = lo;
+  w.n = __builtin_amdgcn_readlane(n, w.seg);
+  w.start = __builtin_amdgcn_readlane(start, w.seg);
+  w.ctx = __builtin_amdgcn_readlane(ctx, w.seg);
+  return true;
+}
 
 // KG key groups of 32 keys per tile, 4 / KG waves of 16 rows for each.
 // FULL: D == DKP, Dv == DVP and the block size is a power of two, at least 8
@@ -93,13 +149,12 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   constexpr int LDS = 2 * TILE > MERGE ? 2 * TILE : MERGE;
   __shared__ __align__(16) uint16_t sm[LDS];
 
-  const int s = blockIdx.y;
-  const int n = seg_len[s];
+  Walk walk;  // the longest first
+  if (!deal(seg_start, seg_len, seg_ctx, H, ROWS, walk)) return;
+  const int s = walk.seg, n = walk.n, ctx = walk.ctx;
+  const long lo = walk.start;
   const long nrows = (long)n * H;
-  const long rho0 = (long)(gridDim.x - 1 - blockIdx.x) * ROWS;  // the longest walks first
-  if (rho0 >= nrows) return;
-  const long lo = seg_start[s];
-  const int ctx = seg_ctx[s];
+  const long rho0 = (long)walk.tile * ROWS;
   const int* bt = block_tables + (size_t)s * max_blocks;
 
   const int tid = threadIdx.x;
@@ -372,9 +427,9 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
       for (int i = 0; i < 4; ++i) acc[db][i] = acc[db][i] * w0 + o1[i] * w1;
     }
   }
-  if (rho >= nrows) return;
 
   if (nsplit > 1) {
+    if (rho >= nrows) return;
     // ---- partial result: unnormalised sums, running max and sum -------------------
     float* pp = partial + (((size_t)lo * H + rho) * nsplit + z) * ((size_t)Dv + LR_PART_PAD);
     if (lg == 0) {
@@ -392,15 +447,20 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   // ---- normalise, gate, store --------------------------------------------------------
   float f = l > 0.f ? 1.0f / l : (l == 0.f ? 0.f : l);
   if (gate != nullptr) f *= sigmoid_fast(bf16_to_f32(gate[(lo + tok) * gate_stride + head]));
-  uint16_t* op = out + ((size_t)lo * H + rho) * Dv;
+  // a lane has 4 entries of each of two blocks: neighbouring groups swap, for 8 of one
+  const int col = (lg & 1) * 16 + (lg >> 1) * 8;
+  uint16_t* op = out + ((size_t)lo * H + rho) * Dv + col;
 #pragma unroll
-  for (int db = 0; db < DB; ++db) {
-    const int d = db * 16 + lg * 4;
-    if (!FULL && d >= Dv) continue;
-    u32x2 w;
-    w[0] = pack_bf16(acc[db][0] * f, acc[db][1] * f);
-    w[1] = pack_bf16(acc[db][2] * f, acc[db][3] * f);
-    *reinterpret_cast<u32x2*>(op + d) = w;
+  for (int db = 0; db < DB; db += 2) {
+    u32x4 w;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const auto both = __builtin_amdgcn_permlane16_swap(pack_bf16(acc[db][2 * e] * f, acc[db][2 * e + 1] * f),
+                                                         pack_bf16(acc[db + 1][2 * e] * f, acc[db + 1][2 * e + 1] * f), false, false);
+      w[e] = both[0];
+      w[2 + e] = both[1];
+    }
+    if ((FULL || db * 16 + col < Dv) && rho < nrows) *reinterpret_cast<u32x4_of8*>(op + db * 16) = w;
   }
 }
 

@@ -104,3 +104,21 @@ def test_chosen_slices(segs, H):
     assert 1 <= cut <= 32 and most // cut >= 128
     assert cut * blocks >= 512 or cut == 32 or most // (cut + 1) < 128
     _run(segs, H, 576, 512, 16, 0, 0, False)
+
+
+@pytest.mark.parametrize("count", [2, 3, 8, 15, 16, 17])
+@pytest.mark.parametrize("D,Dv,H", [(576, 512, 16), (72, 56, 3), (192, 128, 80)])
+def test_tiles_are_dealt_over_the_segments(D, Dv, H, count):
+    """Segments of no, few and many tiles; more than 16 of them are not dealt."""
+    new = [(29 * i) % 90 * (i % 4 > 0) for i in range(count)]
+    _run([(n + 1 + 37 * i % 200, n) for i, n in enumerate(new)], H, D, Dv, 16, 0, 1 + count % 2, gate=count == 3)
+
+
+def test_results_that_lie_8_bytes_off():
+    q = torch.randn(100, 16 * 72, device="cuda").to(BF)
+    cache = torch.randn(8, 1, 16, 72, device="cuda").to(BF)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    args = (q, cache, 56, i32([[3, 1, 0, 2], [4, 7, 5, 6]]), i32([0, 60]), i32([60, 40]), i32([60, 64]), 60, 0.1, 16)
+    out = torch.empty(100 * 16 * 56 + 4, device="cuda", dtype=BF)[4:].view(100, -1)
+    assert out.data_ptr() % 16 == 8
+    assert torch.equal(ops.latent_attention_rows(*args, out=out), ops.latent_attention_rows(*args))
