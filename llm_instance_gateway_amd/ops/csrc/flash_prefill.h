@@ -37,6 +37,9 @@
 // with and without a cap; 8 of 1000 with the window and a cap, replayed without pauses, 101 ->
 // 94 us, and results closer to the 64-bit ones (relative error 0.002041 -> 0.002026; without
 // a cap 0.001941 -> 0.001918), since what rounding adds to a weight it adds to the sum.
+// Results in 16-byte pieces, a lane's four entries of a block swapped with its neighbour's for
+// eight, instead of 8-byte ones: 20 prompts of 200 28.3 -> 24.4, 24 of 640 118 -> 107, 40 of 400 99.8 ->
+// 87.5; 8 of 1000 with the window and a cap, their tiles in turn by length as well, 94 -> 85.
 // Matrix and vector instructions hardly overlap (24 and 64 % of the cycles).  Products of the next
 // tile between the weights of this one spilled registers (121 us); three workgroups per CU,
 // values in one buffer, at 168 registers did too (107).
@@ -52,6 +55,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_of8 __attribute__((ext_vector_type(4), aligned(8)));  // outputs are not asked for more
 
 constexpr int KT = 64;      // keys per tile
 constexpr int TQ = 64;      // query rows of a tile of the caller's tile list
@@ -81,6 +85,7 @@ struct Args {
   int chunk, window;
   int gate_per_head;
   float softcap;
+  int turns;                // tiles take their turns by length: the most 64-key steps one walks, 0: they don't
   int nsplit;               // SPLIT: parts of a tile's keys, and
   float* partial;           // [R, Hq, nsplit, D + 4]: sums of weighted values, then largest score (log2) and sum of weights
 };
@@ -102,6 +107,51 @@ LIG_DEVICE int entry_swizzle(int d) { return (d ^ (d >> 3)) & 7; }
 LIG_DEVICE u32x2 transposed(const uint16_t* p) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
+}
+
+// Which tile of the caller's list is this workgroup's: the longest walks first, so that the
+// last workgroups to begin are the shortest.  A walk's length is taken from its tile's place
+// in the portion, and a window's; of equal ones the last in the list first.
+constexpr int TURN_TILES = 256;
+LIG_DEVICE void tile_in_turn(const Args& a, int& seq, int& qt) {
+  constexpr int MOST = TURN_TILES / 64;
+  const int lane = threadIdx.x & 63, nt = gridDim.y, longest = a.turns;
+  int s[MOST], q[MOST], key[MOST];
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    key[j] = -1;
+    if (j * 64 >= nt) continue;
+    const int at = nt - 1 - (j * 64 + lane);
+    s[j] = a.tile_seq[max(at, 0)];
+    q[j] = a.tile_qstart[max(at, 0)];
+    if (at >= 0) key[j] = min(max(q[j], 0) / TQ, longest);
+  }
+  auto from = [&](int k) {  // tiles with that key or a higher one
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < MOST; ++j)
+      if (j * 64 < nt) c += __popcll(__ballot(key[j] >= k));
+    return c;
+  };
+  const int turn = blockIdx.y;
+  int k = 0;  // the highest key from which on there are more than `turn` tiles
+  for (int bit = 1 << (31 - __builtin_clz(longest)); bit > 0; bit >>= 1)
+    if (from(k + bit) > turn) k += bit;
+  int before = turn - from(k + 1);
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    if (j * 64 >= nt) continue;
+    const uint64_t have = __ballot(key[j] == k);
+    const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0));
+    const uint64_t mine = __ballot(key[j] == k && at == before);
+    if (mine) {
+      const int l = __builtin_ctzll(mine);
+      seq = __builtin_amdgcn_readlane(s[j], l);
+      qt = __builtin_amdgcn_readlane(q[j], l);
+      return;
+    }
+    before -= __popcll(have);
+  }
 }
 
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
@@ -133,11 +183,14 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   const int lg = lane >> 4;
 
   // grid.x runs over the head groups, so that with a multiple of 8 of them
-  // every XCD keeps to some heads' keys in its own L2; the tile list runs
-  // backwards, so that of one prompt the rows with the most keys start first
-  const int tile = gridDim.y - 1 - blockIdx.y;
-  const int s = a.tile_seq[tile];
-  const int qt = a.tile_qstart[tile];
+  // every XCD keeps to some heads' keys in its own L2
+  int s, qt;
+  if (!SPLIT && a.turns > 0) {
+    tile_in_turn(a, s, qt);
+  } else {  // backwards, so that of one prompt the rows with the most keys start first
+    s = a.tile_seq[gridDim.y - 1 - blockIdx.y];
+    qt = a.tile_qstart[gridDim.y - 1 - blockIdx.y];
+  }
   const int lo = a.query_start_locs[s];
   const int n = a.query_start_locs[s + 1] - lo;
   if (qt >= n || n <= 0) return;
@@ -514,10 +567,11 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
         continue;
       }
     }
-    if (r >= n) continue;
+    const bool stored = r < n;
+    const int rr = stored ? r : n - 1;
     const uint16_t* gp = nullptr;
     if (EXTRA && a.gate) {
-      gp = a.gate + (size_t)(lo + r) * a.gate_stride;
+      gp = a.gate + (size_t)(lo + rr) * a.gate_stride;
       if (a.gate_per_head) {
         f *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[h])));
         gp = nullptr;
@@ -525,20 +579,30 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
         gp += (size_t)h * D;
       }
     }
-    uint16_t* op = a.out + ((size_t)(lo + r) * a.num_q_heads + h) * D;
+    // a lane has 4 entries of each of two blocks: neighbouring groups swap, for 8 of one
+    uint16_t* op = a.out + ((size_t)(lo + rr) * a.num_q_heads + h) * D + (lg & 1) * 16 + (lg >> 1) * 8;
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const int d = db * 16 + lg * 4;
-      float o[4];
+    for (int db = 0; db < DB; db += 2) {
+      uint32_t pair[2][2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o[i] = acc[rb][db][i] * f;
-        if (EXTRA && gp) o[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[d + i])));
+      for (int x = 0; x < 2; ++x) {
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[i] = acc[rb][db + x][i] * f;
+          if (EXTRA && gp) o[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-bf16_to_f32(gp[(db + x) * 16 + lg * 4 + i])));
+        }
+        pair[x][0] = pack_bf16(o[0], o[1]);
+        pair[x][1] = pack_bf16(o[2], o[3]);
       }
-      u32x2 w;
-      w[0] = pack_bf16(o[0], o[1]);
-      w[1] = pack_bf16(o[2], o[3]);
-      *reinterpret_cast<u32x2*>(op + d) = w;
+      u32x4 w;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const auto both = __builtin_amdgcn_permlane16_swap(pair[0][e], pair[1][e], false, false);
+        w[e] = both[0];
+        w[2 + e] = both[1];
+      }
+      if (stored) *reinterpret_cast<u32x4_of8*>(op + db * 16) = w;
     }
   }
 }
@@ -585,9 +649,21 @@ static inline bool serves(const Args& a, int D, int Dv) {
          al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
 }
 
+// Whether a launch's tiles take their turns by length.  It pays where a walk is long
+// against the look at the list and the chip is full few times over, so that the last walks
+// count (in the list's order, in turn, us; 32 query and 8 key/value heads of 128): windows of 512,
+// 8 prompts of 700-1000 102.7, 91.4; 3 of 1500 65.0, 56.6; without, 8 of 1000 91.8, 85.3.  20 of 202
+// (24.3; in turn 30.0) and 40 of 400 (87.5, 103.4) stay as listed.
+static inline int turns(const Args& a, long ntiles, long wgs) {
+  const long keys = (long)a.max_blocks * a.block_size, seen = a.window > 0 && a.window + TQ < keys ? a.window + TQ : keys;
+  return ntiles > 1 && ntiles <= TURN_TILES && wgs > 256 && wgs <= 2048 && seen >= 512 ? (int)(seen < 65472 ? seen / TQ + 1 : 1023) : 0;
+}
+
 template <int D, int GH, bool CAP, bool SIG, bool EXTRA>
-static void launch_heads(const Args& a, int ntiles, hipStream_t stream) {
-  const dim3 grid(a.num_q_heads / GH, ntiles), block(256);
+static void launch_heads(const Args& args, int ntiles, hipStream_t stream) {
+  const dim3 grid(args.num_q_heads / GH, ntiles), block(256);
+  Args a = args;
+  a.turns = turns(a, ntiles, (long)ntiles * (a.num_q_heads / GH));
   if (a.block_shift >= 2)
     hipLaunchKernelGGL((flash_prefill_kernel<D, GH, true, CAP, SIG, EXTRA>), grid, block, 0, stream, a);
   else

@@ -199,3 +199,20 @@ def test_keys_behind_the_last_row_of_the_tile(D, H, G, bs):
     got = ops.paged_attention_prefill_tiles(b["q"], b["k"], v, *args)
     want = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], *args)
     assert torch.equal(got[:64], want[:64]) and got[70:].isnan().all()
+
+
+@pytest.mark.parametrize("window", [0, 1, 64, 130, 5000])
+@pytest.mark.parametrize("count", [2, 63, 64, 65, 128, 255, 256, 257])
+def test_tiles_take_their_turns(count, window):
+    """Every tile once, whatever the list's order; more than 256 run as listed."""
+    lens, left = [], count
+    while left:
+        n = min((300, 20, 129, 64, 640)[len(lens) % 5], 64 * left)
+        lens.append(n)
+        left -= -(-n // 64)
+    b = _batch([(n + i % 3 * 50, n) for i, n in enumerate(lens)], 2, 128, 16, 4, 13)
+    assert len(b["ts"]) == count
+    order = torch.randperm(count, generator=torch.Generator().manual_seed(count)).cuda()
+    got = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], b["tab"], b["starts"], b["ctx"], b["ts"][order].contiguous(),
+                                            b["tq"][order].contiguous(), 128 ** -0.5, 4, window=window)
+    _check(got, b, 128, 128 ** -0.5, 4, **({"window": window} if window else {}))
