@@ -23,7 +23,9 @@
 // precision.  Bound by its chain of short steps (loads, norms, exponentials,
 // substitution, three levels), so a wave loads its own 16 rows only, all at
 // once, and takes the others' from LDS: 47 us for 8 prompts of 1000 tokens and
-// 32 heads, 65 with a load per tile in turn.
+// 32 heads, 65 with a load per tile in turn.  With the chunks of a portion side by side in
+// the grid the last of the longer ones fell to the same XCDs: heads side by side, both calls
+// 141.6 -> 138.8 us; 16 of 500, 64 heads 314 -> 291.
 //
 // delta_chunk_scan_kernel, one workgroup per (segment, head, one or two
 // blocks of 64 value columns), walks the chunks; wave w owns 16 columns of
@@ -107,9 +109,10 @@ extern "C" long lig_gated_delta_scratch(int R, int S, int H) {
 
 #define DI_THREADS 256
 #define DI_ROW 68  // padded fp32 LDS row
+#define DI_WAVES 5  // to a SIMD, at 96 registers; at 80, for six, it spills and gains nothing
 
 template <int DP, typename Chunk>
-__global__ __launch_bounds__(DI_THREADS) void delta_chunk_prepare_kernel(
+__global__ __launch_bounds__(DI_THREADS, DI_WAVES) void delta_chunk_prepare_kernel(
     const MsArgs A, Chunk* __restrict__ scratch) {
   constexpr bool WALK = __is_same(Chunk, DeltaWalkChunk);
   constexpr int KB = DP / 32;
@@ -128,18 +131,21 @@ __global__ __launch_bounds__(DI_THREADS) void delta_chunk_prepare_kernel(
   __shared__ __align__(16) float b_s[MC_T], ik_s[MC_T];
   __shared__ float iq_s[MC_T];
 
-  const int seg = blockIdx.y, h = blockIdx.z;
+  // XCDs take workgroups in turn: each gets an eighth of the heads, whose neighbours share
+  // keys, and as many chunks as the others
+  const int seg = blockIdx.y, chunk = blockIdx.x / A.H, x = blockIdx.x - chunk * A.H;
+  const int h = A.H % 8 == 0 ? (x & 7) * (A.H >> 3) + (x >> 3) : x;
   const int n = A.seg_len[seg];
-  const int c0 = blockIdx.x * MC_T;
+  const long r0 = A.seg_start[seg];
+  const int c0 = chunk * MC_T;
   if (c0 >= n || n < A.len_min) return;
   const int cnt = min(MC_T, n - c0);
-  const long r0 = A.seg_start[seg];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
   const uint16_t* k = (const uint16_t*)A.k + (h / A.rep) * A.D + (r0 + c0) * A.k_stride;
   const uint16_t* q = (const uint16_t*)A.q + (h / A.rep) * A.D + (r0 + c0) * A.q_stride;
-  Chunk* out = scratch + delta_chunk_slot(r0, blockIdx.x, seg) * A.H + h;
+  Chunk* out = scratch + delta_chunk_slot(r0, chunk, seg) * A.H + h;
   uint16_t(*scores)[DC_BLOCKS][16][16];  // high and low halves
   if constexpr (WALK) scores = out->scores;
   else scores = out->w[1];
@@ -921,7 +927,7 @@ bool ms_delta_chunks_served(const MsArgs& a) {
 void ms_delta_chunks_launch(const MsArgs& a, int S, int max_seg_len, void* scratch,
                             hipStream_t st) {
   DeltaChunk* sc = (DeltaChunk*)scratch;
-  const dim3 gi((max_seg_len + MC_T - 1) / MC_T, S, a.H);
+  const dim3 gi((max_seg_len + MC_T - 1) / MC_T * a.H, S);
   // Two value blocks per workgroup share the staged operands where the
   // registers of eight waves hold the state, and a workgroup each would not
   // find a CU each.  Both calls, 32 heads of 128 x 128, one block here and two:

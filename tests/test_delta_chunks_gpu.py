@@ -88,3 +88,8 @@ def test_value_blocks_in_pairs(dim, vdim):
     got, state = run(x, z, lens)
     alone = [run(x[sum(lens[:i]) :][:n].contiguous(), z[sum(lens[:i]) :][:n].contiguous(), [n]) for i, n in enumerate(lens)]
     assert torch.equal(got, torch.cat([o for o, _ in alone])) and torch.equal(state, torch.cat([s for _, s in alone]))
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(8, 4, 128), (16, 16, 64), (24, 12, 128), (9, 3, 128)])
+def test_heads_dealt_to_the_xcds(heads, kv, dim):
+    test_delta_chunks([17, 200, 64], heads, kv, dim, 64)
