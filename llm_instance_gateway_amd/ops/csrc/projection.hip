@@ -41,58 +41,52 @@ LIG_DEVICE void stages_landed(int behind) {
 constexpr int XCD_PHASES = 4;  // starting points in K
 
 // acc[i][j]: 16 columns i of W's tile by 16 rows j of x's, as the products leave them.
-// A lane holds row li of a tile's 16, 4 columns of it, 8 of a pair.  Rounded, they leave as 16
-// bytes also from an odd number of tiles, whose W rows are not dealt so: 850 rows of 28672 x
-// 4096 163 -> 158 us, 1000 179 -> 175.
+// A lane holds row li of a tile's 16, 4 columns of it, 8 of a pair: stored so, neighbouring
+// lanes are in 16 rows and every one of them is an access of its own, 64 to a kilobyte.  So
+// 16 rows at a time go through LDS (`room`, this wave's own) and leave in the order in which
+// they lie in memory: parts of 4096 x 14336 at 202 rows 35.0 -> 33.0 us, 384 46 -> 44.4; of 4096 x
+// 4096 at 786 32.8 -> 31.1; 28672 x 4096 rounded, 786 rows 151 -> 148; to 64 rows level.
+template <int TN, bool PARTIAL>
+constexpr int ROOM_ROW = TN * 16 * (PARTIAL ? 4 : 2) + 16;  // bytes of a row, for rows to start 4 banks apart
 template <int TM, int TN, bool PARTIAL>
 LIG_DEVICE void store_tile(const f32x4_t (&acc)[TN][TM], uint16_t* __restrict__ y, float* __restrict__ part, const int m_at,
-                           const int n_at, const int z, const int M, const int N) {
+                           const int n_at, const int z, const int M, const int N, char* room) {
   constexpr bool PAIRS = TN % 2 == 0;
-  const int li = threadIdx.x & 15, lg = (threadIdx.x & 63) >> 4;
+  constexpr int ROW = ROOM_ROW<TN, PARTIAL>, ES = PARTIAL ? 4 : 2, PIECES = TN * ES;  // 16-byte pieces of a row
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
-    const int m = m_at + j * 16 + li;
-    if (m >= M) continue;
-    auto packed = [&](int i) {
-      u32x2 v;
-      v[0] = (uint32_t)f32_to_bf16(acc[i][j][0]) | ((uint32_t)f32_to_bf16(acc[i][j][1]) << 16);
-      v[1] = (uint32_t)f32_to_bf16(acc[i][j][2]) | ((uint32_t)f32_to_bf16(acc[i][j][3]) << 16);
-      return v;
-    };
-    constexpr int STEP = PAIRS || !PARTIAL ? 2 : 1;
+    char* own = room + li * ROW + lg * (PAIRS ? 8 : 4) * ES;
 #pragma unroll
-    for (int i = 0; i < TN; i += STEP) {
-      if constexpr (PARTIAL || PAIRS) {
-        const int n = n_at + i * 16 + lg * (PAIRS ? 8 : 4);
-        if (n >= N) continue;
-        if constexpr (PARTIAL) {
-          float* o = part + ((size_t)z * M + m) * N + n;
-          *reinterpret_cast<f32x4_t*>(o) = acc[i][j];
-          if constexpr (PAIRS) *reinterpret_cast<f32x4_t*>(o + 4) = acc[i + 1][j];
-        } else {
-          f32x8 v;
+    for (int i = 0; i < TN; i += PAIRS ? 2 : 1) {
+      char* to = own + i * 16 * ES;
+      if constexpr (PARTIAL) {
+        *reinterpret_cast<f32x4_t*>(to) = acc[i][j];
+        if constexpr (PAIRS) *reinterpret_cast<f32x4_t*>(to + 16) = acc[i + 1][j];
+      } else if constexpr (PAIRS) {
+        f32x8 v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[e] = acc[i][j][e];
-            v[4 + e] = acc[i + 1][j][e];
-          }
-          *reinterpret_cast<u16x8*>(y + (size_t)m * N + n) = f32x8_to_bf16x8(v);
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc[i][j][e];
+          v[4 + e] = acc[i + 1][j][e];
         }
-      } else if (i + 1 < TN) {  // neighbouring groups of lanes swap, for 8 columns of one block
-        const u32x2 a = packed(i), b = packed(i + 1);
-        u32x4 v;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const auto both = __builtin_amdgcn_permlane16_swap(a[e], b[e], false, false);
-          v[e] = both[0];
-          v[2 + e] = both[1];
-        }
-        const int n = n_at + (i + (lg & 1)) * 16 + (lg >> 1) * 8;
-        if (n < N) *reinterpret_cast<u32x4*>(y + (size_t)m * N + n) = v;
+        *reinterpret_cast<u16x8*>(to) = f32x8_to_bf16x8(v);
       } else {
-        const int n = n_at + i * 16 + lg * 4;
-        if (n < N) *reinterpret_cast<u32x2*>(y + (size_t)m * N + n) = packed(i);
+        u32x2 v;
+        v[0] = (uint32_t)f32_to_bf16(acc[i][j][0]) | ((uint32_t)f32_to_bf16(acc[i][j][1]) << 16);
+        v[1] = (uint32_t)f32_to_bf16(acc[i][j][2]) | ((uint32_t)f32_to_bf16(acc[i][j][3]) << 16);
+        *reinterpret_cast<u32x2*>(to) = v;
       }
+    }
+#pragma unroll
+    for (int k = 0; k < (16 * PIECES + 63) / 64; ++k) {
+      const int piece = k * 64 + lane, r = piece / PIECES, c = piece % PIECES;
+      const int m = m_at + j * 16 + r, n = n_at + c * (16 / ES);
+      if (16 * PIECES % 64 && piece >= 16 * PIECES) continue;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(room + r * ROW + c * 16);
+      if (m >= M || n >= N) continue;
+      if constexpr (PARTIAL) *reinterpret_cast<u32x4*>(part + ((size_t)z * M + m) * N + n) = v;
+      else *reinterpret_cast<u32x4*>(y + (size_t)m * N + n) = v;
     }
   }
 }
@@ -213,7 +207,8 @@ __global__ __launch_bounds__(256, 1) void projection_kernel(
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] += *reinterpret_cast<const f32x4_t*>(sums + k * WAVE + (i * TM + j) * 256);
-  store_tile<TM, TN, PARTIAL>(acc, y, part, m0, n0, z, M, N);
+  static_assert(16 * ROOM_ROW<TN, PARTIAL> <= sizeof(sm), "");
+  store_tile<TM, TN, PARTIAL>(acc, y, part, m0, n0, z, M, N, reinterpret_cast<char*>(sm));
 }
 
 // c += a b with c in accumulation registers.  The compiler's own choice between them
@@ -402,7 +397,11 @@ __global__ __launch_bounds__(256, 1) void projection_wide_kernel(
   half(k0, no, yes, s, s % SW, s % SX);
   half(k1, no, no, 0, 0, 0);
   mfma_apart(acc);
-  store_tile<TM, TN, PARTIAL>(acc, y, part, m0 + wm * TM * 16, n0 + wn * TN * 16, z, M, N);
+  // the last stage has been read by all
+  __syncthreads();
+  constexpr int ROOM = 16 * ROOM_ROW<TN, PARTIAL>;
+  static_assert(4 * ROOM <= sizeof(sm), "");
+  store_tile<TM, TN, PARTIAL>(acc, y, part, m0 + wm * TM * 16, n0 + wn * TN * 16, z, M, N, reinterpret_cast<char*>(sm) + wave * ROOM);
 }
 
 __global__ __launch_bounds__(256) void projection_sum_kernel(uint16_t* __restrict__ y, const float* __restrict__ part,
