@@ -34,7 +34,7 @@
 // Measured with rows of 576 and values of 512 (us; a kernel that staged through
 // registers -> with the builtin -> now): 256 single tokens on 700-1024 keys, 32
 // heads 148 -> 72 -> 63 (255 MB of rows, 4.1 TB/s); 4 prompts of 700-1000, 16 heads
-// 322 -> 121 -> 97 (546 TFLOP/s; with the tiles dealt by length 83). Two row blocks per wave, which halve the LDS
+// 322 -> 121 -> 97 (546 TFLOP/s; with the tiles dealt by length 83, weights ahead of others' products 79). Two row blocks per wave, which halve the LDS
 // reads, lost more by leaving one wave per SIMD (keys of 320: 372 us before, 136
 // now, 208 so; of 128: 149, 73, 135).
 // Weights handed to all waves, so that each adds up a quarter of the columns of all rows and
@@ -341,6 +341,9 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     };
     load_v(0);
 
+    // the other workgroup's products give way to these few instructions, behind which
+    // this wave's own wait: 4 prompts of 700-1000 78.9 -> 75.0 us, one of 4000 298 -> 292
+    if constexpr (KG == 1) __builtin_amdgcn_s_setprio(1);
     // ---- weights of keys k0 + lg*8 + e -----------------------------------------
     const bool masked = k0 + 32 > min(all_end, kv_hi) || k0 < all_lo;
     uint32_t dead = 0;
@@ -387,6 +390,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     }
     const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pw);
 
+    if constexpr (KG == 1) __builtin_amdgcn_s_setprio(0);
     // ---- O^T += V^T P^T -----------------------------------------------------------
 #pragma unroll
     for (int b = 0; b < DB / 4; ++b) {
