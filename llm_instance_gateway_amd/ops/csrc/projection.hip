@@ -255,7 +255,8 @@ LIG_DEVICE void later_stages(int left) {
 //     on their way (a ring of two for both waited 0.5 us per step for its loads);
 //   * columns come 64 at a time, a full line of 128 bytes a row: 32 at a time, in a ring
 //     of finer grain, they arrived at little more than half the rate.
-// Llama-3-8B widths, weights not in any cache (us; eight waves -> this, the library):
+// Llama-3-8B widths, weights not in any cache (us; eight waves -> this, the library; without the
+// other tiles below and with results stored as lanes hold them):
 //   rows      gate_up               down                o                 qkv
 //    202   71 -> 55 ( 66)     36 -> 35 ( 57)     17 -> 15 (21)     22 -> 20 (25)
 //    384  110 -> 77 ( 79)     54 -> 49 ( 75)     23 -> 20 (24)     33 -> 29 (35)
