@@ -55,12 +55,6 @@ LIG_DEVICE uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
-// The two bf16 numbers of a pair added to s, in one instruction.
-LIG_DEVICE float add_pair(uint32_t pair, float s) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3f803f80u), s, false);
-}
-
 // ---- wave reductions --------------------------------------------------------
 // Butterfly over the full 64-lane wave; result replicated in every lane.
 

@@ -32,11 +32,10 @@
 // rows by DMA and their block's row number worked out once per group of keys: 4000
 // rows on 4000 keys 560 -> 441 us (between products), 20 prompts of 200 37 -> 33, one
 // of 202 8.9 -> 7.9, 8 of 1000 with the window and a cap 120 -> 96.
-// Weights are summed as the matrix cores see them, rounded, two to an instruction, and a
-// cap's tanh goes into the weight's exponent as it comes: 13 and 11 % fewer vector instructions
-// with and without a cap; 8 of 1000 with the window and a cap, replayed without pauses, 101 ->
-// 94 us, and results closer to the 64-bit ones (relative error 0.002041 -> 0.002026; without
-// a cap 0.001941 -> 0.001918), since what rounding adds to a weight it adds to the sum.
+// A cap's tanh goes into the weight's exponent as it comes.  Weights are summed in fp32, ahead of
+// their rounding; summed as the matrix cores see them, two to an instruction, they took as long
+// (8 of 1000 with the window and a cap 93.3 us, unrounded 92.5; 4000 rows of one prompt 150.7, 152.4; 24
+// of 640 107.5, 107.4; steps level).
 // Results in 16-byte pieces, a lane's four entries of a block swapped with its neighbour's for
 // eight, instead of 8-byte ones: 20 prompts of 200 28.3 -> 24.4, 24 of 640 118 -> 107, 40 of 400 99.8 ->
 // 87.5; 8 of 1000 with the window and a cap, their tiles in turn by length as well, 94 -> 85.
@@ -504,14 +503,17 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
         if constexpr (SIG) p[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], -slope, level)));
         else p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[e], slope, level));
       }
+      if constexpr (!SIG) {
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum += p[e];
+        l[rb] += sum;
+      }
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
         u32x4 w;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          w[e] = pack_bf16(p[t2 * 8 + 2 * e], p[t2 * 8 + 2 * e + 1]);
-          if constexpr (!SIG) l[rb] = add_pair(w[e], l[rb]);
-        }
+        for (int e = 0; e < 4; ++e) w[e] = pack_bf16(p[t2 * 8 + 2 * e], p[t2 * 8 + 2 * e + 1]);
         p_frag[rb][t2] = __builtin_bit_cast(bf16x8_t, w);
       }
     }

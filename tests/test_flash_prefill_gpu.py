@@ -216,3 +216,45 @@ def test_tiles_take_their_turns(count, window):
     got = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], b["tab"], b["starts"], b["ctx"], b["ts"][order].contiguous(),
                                             b["tq"][order].contiguous(), 128 ** -0.5, 4, window=window)
     _check(got, b, 128, 128 ** -0.5, 4, **({"window": window} if window else {}))
+
+
+def _uneven_weight():
+    """A score difference whose weight, just over a half, lies nearly half a step of bf16 from the nearest such number."""
+    d = torch.arange(141, 175, dtype=torch.float64) / 256  # bf16 numbers
+    w = torch.exp(-d)
+    return max(zip((w.to(BF).double() - w).abs().tolist(), d.tolist()))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("ctx,bs,cap", [(64, 16, 0.0), (64, 16, 30.0), (70, 6, 0.0), (2100, 16, None)])
+def test_weights_are_summed_unrounded(D, ctx, bs, cap):
+    """One key of 64 with a value, all others of equal weights w without: their share is 1 / (1 + n w),
+    with n w a sum in fp32 (None: the plain kernel's parts, each with such keys).
+
+    The result is rounded once, by up to 2^-8, as often up as down: over 8 D values six times the mean's
+    deviation is at most 6 * 2^-8 / sqrt(3 * 8 * D) = 6e-4 (D = 64).  With weights rounded by half a
+    step of 2^-8 the share is off by 2.8e-3 and more, all one way."""
+    H = 8
+    off, d = _uneven_weight()
+    assert off > 0.4 * 2.0 ** -8
+    b = _batch([(ctx, 1)], H, D, bs, H, 5)
+    at = torch.arange(37, ctx, 64, device="cuda")
+    blk, row = b["tab"][0, at // bs].long(), at % bs
+    for t in ("k", "v"):
+        b[t].zero_()
+    b["q"].zero_()
+    b["q"].view(1, H, D)[..., 0] = 1.0
+    b["k"][blk, :, row, 0] = d
+    v = 1 + torch.rand(H, D, device="cuda", generator=torch.Generator("cuda").manual_seed(D)).to(BF)
+    b["v"][blk, :, row] = v
+    args = b["tab"], b["starts"], b["ctx"]
+    if cap is None:
+        assert ops._load_ext().paged_attention_prefill_parts(1, 1, H, D, b["tab"].shape[1] * bs) > 1
+        got = ops.paged_attention_prefill(b["q"].view(1, H, D), b["k"], b["v"], *args, 1.0, tile_seq=b["ts"], tile_qstart=b["tq"])
+    else:
+        got = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], *args, b["ts"], b["tq"], 1.0, H, softcap=cap)
+    score = torch.tensor(d, dtype=torch.float64)
+    if cap:
+        score = cap * torch.tanh(score / cap)
+    want = v.double() / (1 + (ctx / len(at) - 1) * torch.exp(-score).item())
+    assert ((got.view(H, D).double() / want).mean() - 1).abs() <= 6 * 2.0 ** -8 / (3 * 8 * D) ** 0.5
