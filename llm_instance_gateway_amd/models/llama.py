@@ -342,7 +342,7 @@ class LlamaForCausalLM(nn.Module):
                 qkv, residual = (qkv, x) if residual is None else qkv
                 q = ops.qkv_rope_cache(
                     qkv, positions, self.cos_sin_cache, kv[0], kv[1], meta.slot_mapping, attn.num_heads)
-            if meta.num_decode_tokens == 1:
+            if meta.num_decode_tokens == 1 and "attend" not in attn.__dict__:
                 a, parts = ops.paged_attention_decode_open(
                     q.view(1, attn.num_heads, -1), kv[0], kv[1], meta.decode_block_tables, meta.decode_context_lens, attn.scale,
                     meta.max_decode_ctx, meta.decode_nsplits)

@@ -134,3 +134,29 @@ def test_parts_of_a_walk(D, ctx, nsplits):
     want = ops.row_product(ops.paged_attention_decode(*args, nsplits=nsplits).view(1, -1), w)
     x, parts = ops.paged_attention_decode_open(*args, nsplits=nsplits)
     assert torch.equal(ops.row_product(x, w, parts=parts), want)
+
+
+def test_an_attend_of_its_own_is_called():
+    """An instance's own `attend`, which its layer calls at any number of rows, for a single token too."""
+    from dataclasses import replace
+
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.models.config import get_model_config
+
+    mc = replace(get_model_config("llama3-8b"), num_layers=2, vocab_size=1024)
+    eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=32, max_num_seqs=2, max_num_batched_tokens=256, max_model_len=256,
+                                 enforce_eager=True), device="cuda")
+    model = eng.runner.model
+    assert model._row_products()
+    attn, rows = model.layers[1].self_attn, []
+    theirs = attn.attend
+
+    def attend(q, kv, meta):
+        rows.append(len(q))
+        return theirs(q, kv, meta)
+
+    attn.attend = attend
+    eng.add_request(list(range(7, 40)), SamplingParams(max_new_tokens=4))
+    for _ in range(3):
+        eng.step()
+    assert rows == [33, 1, 1]
