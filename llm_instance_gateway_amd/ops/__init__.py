@@ -892,6 +892,7 @@ def paged_attention_prefill_tiles(
         _ptr(tile_qstart), _ptr(query_start_locs), _ptr(context_lens),
         _ptr(block_tables), float(scale), float(temp_coef), ev, ev_int,
         tile_seq.shape[0], num_heads, G, D, Dv, v_row, bs, block_tables.shape[1],
+        min(query_start_locs.shape[0] - 1, context_lens.shape[0]),
         int(chunk), int(window), _ptr(score_bias), int(weights == "sigmoid"),
         int(bool(gate_per_head and gate is not None)), float(softcap), _stream(),
     )

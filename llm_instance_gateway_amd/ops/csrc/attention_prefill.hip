@@ -17,7 +17,7 @@ extern "C" void lig_paged_attention_prefill_launch(
     const uint16_t* v_cache, const int* tile_seq, const int* tile_qstart,
     const int* query_start_locs, const int* context_lens,
     const int* block_tables, float scale, int ntiles, int num_q_heads,
-    int num_kv_heads, int head_dim, int block_size, int max_blocks,
+    int num_kv_heads, int head_dim, int block_size, int max_blocks, int num_seqs,
     int nsplit, float* partial, hipStream_t stream) {
   flash_prefill::Args a{};
   a.out = out;
@@ -37,6 +37,7 @@ extern "C" void lig_paged_attention_prefill_launch(
   a.block_size = block_size;
   a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
+  a.num_seqs = num_seqs;
   a.nsplit = nsplit;
   a.partial = partial;
   if (nsplit > 1) {

@@ -292,6 +292,21 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_tiles_kernel(
   }
 }
 
+// Of a launch of heads of 64 or 128 (and of the Llama path's in one part): whether its tiles take
+// their turns by length, then above 0.  keys: what a row of the block table has room for.
+extern "C" int lig_paged_attention_prefill_turns(int ntiles, int num_seqs, int num_q_heads, int num_kv_heads, long keys,
+                                                 int chunk, int window) {
+  flash_prefill::Args a{};
+  a.num_q_heads = num_q_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.max_blocks = (int)keys;
+  a.block_size = 1;
+  a.num_seqs = num_seqs;
+  a.chunk = chunk;
+  a.window = window;
+  return flash_prefill::turns(a, ntiles);
+}
+
 // Returns 0 when launched, 1 when the shape is not served (the caller then
 // uses the any-shape kernel).
 extern "C" int lig_paged_attention_prefill_tiles(
@@ -301,7 +316,7 @@ extern "C" int lig_paged_attention_prefill_tiles(
     const int* context_lens, const int* block_tables, float scale,
     float temp_coef, float temp_every, int temp_every_int, int ntiles,
     int num_q_heads, int num_kv_heads, int D, int Dv, int v_row, int block_size,
-    int max_blocks, int chunk, int window, const float* score_bias,
+    int max_blocks, int num_seqs, int chunk, int window, const float* score_bias,
     int sigmoid_weights, int gate_per_head, float softcap, hipStream_t stream) {
   if (D % 8 != 0 || Dv % 8 != 0 || D > 128 || Dv > 128 || D <= 0 || Dv <= 0 ||
       v_row % 8 != 0 || v_row < Dv ||
@@ -334,6 +349,7 @@ extern "C" int lig_paged_attention_prefill_tiles(
   a.block_size = block_size;
   a.block_shift = shift_of(block_size);
   a.max_blocks = max_blocks;
+  a.num_seqs = num_seqs;
   a.chunk = chunk;
   a.window = window;
   a.gate_per_head = gate_per_head;

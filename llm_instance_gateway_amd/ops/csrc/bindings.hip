@@ -131,7 +131,7 @@ int lig_paged_attention_prefill_parts(long, long, int, int, long);
 void lig_paged_attention_prefill_launch(
     uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const int*,
     const int*, const int*, const int*, const int*, float, int, int, int,
-    int, int, int, int, float*, hipStream_t);
+    int, int, int, int, int, float*, hipStream_t);
 }
 
 namespace {
@@ -456,7 +456,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
       tile_seq.data_ptr<int>(), tile_qstart.data_ptr<int>(),
       query_start_locs.data_ptr<int>(), context_lens.data_ptr<int>(),
       block_tables.data_ptr<int>(), (float)scale, ntiles, Hq, Hkv, D, BS,
-      max_blocks, parts, parts > 1 ? partial.data_ptr<float>() : nullptr, as_stream(stream));
+      max_blocks, (int)std::min(query_start_locs.size(0) - 1, context_lens.size(0)), parts, parts > 1 ? partial.data_ptr<float>() : nullptr, as_stream(stream));
 }
 
 void sgmv_shrink(torch::Tensor u, torch::Tensor x, torch::Tensor a_stack,

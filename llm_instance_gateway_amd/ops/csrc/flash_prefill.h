@@ -46,6 +46,8 @@
 // per SIMD) was slower everywhere: 781 us in the first of these.
 #pragma once
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace flash_prefill {
@@ -81,6 +83,7 @@ struct Args {
   int v_row;
   int block_size, block_shift;  // block_shift < 0: not a power of two
   int max_blocks;
+  int num_seqs;             // portions that query_start_locs and context_lens hold
   int chunk, window;
   int gate_per_head;
   float softcap;
@@ -108,22 +111,52 @@ LIG_DEVICE u32x2 transposed(const uint16_t* p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
 }
 
-// Which tile of the caller's list is this workgroup's: the longest walks first, so that the
-// last workgroups to begin are the shortest.  A walk's length is taken from its tile's place
-// in the portion, and a window's; of equal ones the last in the list first.
-constexpr int TURN_TILES = 256;
-LIG_DEVICE void tile_in_turn(const Args& a, int& seq, int& qt) {
+// The oldest key that some row of a tile whose first row is at qpos0 sees.
+template <bool EXTRA>
+LIG_DEVICE int oldest_key(const Args& a, int qpos0) {
+  int first = 0;
+  if (EXTRA) {
+    if (a.chunk > 0) first = (qpos0 / a.chunk) * a.chunk;
+    if (a.window > 0) first = max(first, qpos0 - a.window + 1);
+    first = max(first, 0);
+  }
+  return first;
+}
+
+// A tile of the caller's list and its portion.
+struct Place {
+  int s, qt, lo, n, ctx;
+};
+
+// Which tile of the list is this workgroup's: the longest walks first, so that the last
+// workgroups to begin are the shortest; of equal ones the last in the list first.  Lane i
+// brings portion i's numbers in the round of loads that brings the list.
+constexpr int TURN_TILES = 256, TURN_PORTION = 8;  // at most, and at least for each portion
+template <bool EXTRA>
+LIG_DEVICE Place tile_in_turn(const Args& a) {
   constexpr int MOST = TURN_TILES / 64;
+  static_assert(TURN_TILES / TURN_PORTION < 64, "a lane for each portion and the end of the last");
   const int lane = threadIdx.x & 63, nt = gridDim.y, longest = a.turns;
-  int s[MOST], q[MOST], key[MOST];
+  const int first = a.query_start_locs[min(lane, a.num_seqs)], held = a.context_lens[min(lane, a.num_seqs - 1)];
+  Place p[MOST];
+  int key[MOST];
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    if (j * 64 >= nt) continue;
+    const int at = max(nt - 1 - (j * 64 + lane), 0);
+    p[j].s = a.tile_seq[at];
+    p[j].qt = a.tile_qstart[at];
+  }
 #pragma unroll
   for (int j = 0; j < MOST; ++j) {
     key[j] = -1;
     if (j * 64 >= nt) continue;
-    const int at = nt - 1 - (j * 64 + lane);
-    s[j] = a.tile_seq[max(at, 0)];
-    q[j] = a.tile_qstart[max(at, 0)];
-    if (at >= 0) key[j] = min(max(q[j], 0) / TQ, longest);
+    p[j].lo = __shfl(first, p[j].s, 64);
+    p[j].n = __shfl(first, p[j].s + 1, 64) - p[j].lo;
+    p[j].ctx = __shfl(held, p[j].s, 64);
+    const int qpos0 = p[j].ctx - p[j].n + p[j].qt;
+    const int steps = (min(p[j].ctx, qpos0 + TQ) + KT - 1) / KT - oldest_key<EXTRA>(a, qpos0) / KT;
+    if (j * 64 + lane < nt) key[j] = p[j].qt < p[j].n ? min(max(steps, 0), longest) : 0;
   }
   auto from = [&](int k) {  // tiles with that key or a higher one
     int c = 0;
@@ -145,12 +178,12 @@ LIG_DEVICE void tile_in_turn(const Args& a, int& seq, int& qt) {
     const uint64_t mine = __ballot(key[j] == k && at == before);
     if (mine) {
       const int l = __builtin_ctzll(mine);
-      seq = __builtin_amdgcn_readlane(s[j], l);
-      qt = __builtin_amdgcn_readlane(q[j], l);
-      return;
+      return {__builtin_amdgcn_readlane(p[j].s, l), __builtin_amdgcn_readlane(p[j].qt, l), __builtin_amdgcn_readlane(p[j].lo, l),
+              __builtin_amdgcn_readlane(p[j].n, l), __builtin_amdgcn_readlane(p[j].ctx, l)};
     }
     before -= __popcll(have);
   }
+  return {0, 0, 0, 0, 0};  // not reached: there are as many turns as tiles
 }
 
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
@@ -183,17 +216,18 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 
   // grid.x runs over the head groups, so that with a multiple of 8 of them
   // every XCD keeps to some heads' keys in its own L2
-  int s, qt;
+  Place own;
   if (!SPLIT && a.turns > 0) {
-    tile_in_turn(a, s, qt);
+    own = tile_in_turn<EXTRA>(a);
   } else {  // backwards, so that of one prompt the rows with the most keys start first
-    s = a.tile_seq[gridDim.y - 1 - blockIdx.y];
-    qt = a.tile_qstart[gridDim.y - 1 - blockIdx.y];
+    own.s = a.tile_seq[gridDim.y - 1 - blockIdx.y];
+    own.qt = a.tile_qstart[gridDim.y - 1 - blockIdx.y];
+    own.lo = a.query_start_locs[own.s];
+    own.n = a.query_start_locs[own.s + 1] - own.lo;
+    own.ctx = a.context_lens[own.s];
   }
-  const int lo = a.query_start_locs[s];
-  const int n = a.query_start_locs[s + 1] - lo;
+  const int s = own.s, qt = own.qt, lo = own.lo, n = own.n, ctx = own.ctx;
   if (qt >= n || n <= 0) return;
-  const int ctx = a.context_lens[s];
   const int* bt = a.block_tables + (size_t)s * a.max_blocks;
   const int group = a.num_q_heads / a.num_kv_heads;
   const int per_kv = group / GH;
@@ -258,12 +292,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   // ---- walk ------------------------------------------------------------------
   const int qpos0 = ctx - n + qt;
   const int kv_end = min(ctx, qpos0 + TQ);
-  int first_key = 0;  // that some row sees
-  if (EXTRA) {
-    if (a.chunk > 0) first_key = (qpos0 / a.chunk) * a.chunk;
-    if (a.window > 0) first_key = max(first_key, qpos0 - a.window + 1);
-    first_key = max(first_key, 0);
-  }
+  const int first_key = oldest_key<EXTRA>(a, qpos0);
   int kv_begin = first_key & ~(KT - 1), kv_stop = kv_end;
   if constexpr (SPLIT) {
     const int part = tiles_of_part((kv_end + KT - 1) / KT, a.nsplit) * KT;
@@ -651,21 +680,40 @@ static inline bool serves(const Args& a, int D, int Dv) {
          al(a.q, 16) && al(a.k_cache, 16) && al(a.v_cache, 16) && al(a.out, 8);
 }
 
-// Whether a launch's tiles take their turns by length.  It pays where a walk is long
-// against the look at the list and the chip is full few times over, so that the last walks
-// count (in the list's order, in turn, us; 32 query and 8 key/value heads of 128): windows of 512,
-// 8 prompts of 700-1000 102.7, 91.4; 3 of 1500 65.0, 56.6; without, 8 of 1000 91.8, 85.3.  20 of 202
-// (24.3; in turn 30.0) and 40 of 400 (87.5, 103.4) stay as listed.
-static inline int turns(const Args& a, long ntiles, long wgs) {
-  const long keys = (long)a.max_blocks * a.block_size, seen = a.window > 0 && a.window + TQ < keys ? a.window + TQ : keys;
-  return ntiles > 1 && ntiles <= TURN_TILES && wgs > 256 && wgs <= 2048 && seen >= 512 ? (int)(seen < 65472 ? seen / TQ + 1 : 1023) : 0;
+// Two heads per workgroup halve the reads of K and V; the line is where
+// that leaves two workgroups for every CU (heads of 128, 32 over 8; two heads
+// against one): 1280 workgroups 37.5 us against 44.0, 512 of 200 keys 17.0
+// against 21.8, of 2048 71.4 against 72.6, 4096 rows on 4000 keys 498 against
+// 683, but 256 workgroups of 4000 keys 126 us against 109, 96 of 1000 37.9
+// against 28.3, 64 11.5 against 8.9
+static inline int heads_of_workgroup(const Args& a, long ntiles) {
+  return a.num_q_heads / a.num_kv_heads % 2 == 0 && ntiles * (a.num_q_heads / 2) >= 512 ? 2 : 1;
+}
+
+// Whether a launch's tiles take their turns by length: Args::turns.  It pays where walks
+// are long against the look at the list, unlike each other, and the chip is full few times over, so
+// that the last ones count.  The host knows no lengths but the mean portion's rows and the most
+// that a row can see.  In the list's order, in turn (us; 32 query and 8 key/value heads of 128): 8
+// prompts of 1000 113.6, 100.2; with a window of 512 and a cap 99.1, 93.2; 14 of 512 61.2, 58.5; 4 of
+// 500 24.6, 21.6; 6 of 512 to 1000 rows on contexts of 600 to 4000 132.9, 109.1; 2 of 128 on 4000
+// listed ahead of 2 of 1500 130.8, 99.0.  As listed stay 20 of 202 (29.4, 30.7; with one of 600 33.4, 34.1),
+// 16 of 448 (54.4, 57.5), 24 of 640 (134.0, 141.7: 3840 workgroups) and one alone, which is in order (4000 rows
+// 145.5, 146.6).
+static inline int turns(const Args& a, long ntiles) {
+  const long wgs = ntiles * (a.num_q_heads / heads_of_workgroup(a, ntiles));
+  long seen = (long)a.max_blocks * a.block_size;  // by a tile
+  if (a.window > 0) seen = std::min(seen, (long)a.window + TQ);
+  if (a.chunk > 0) seen = std::min(seen, (long)a.chunk + TQ);
+  const bool pays = a.num_seqs > 1 && ntiles >= (long)TURN_PORTION * a.num_seqs && ntiles <= TURN_TILES && wgs > 256 &&
+                    wgs <= 2048 && seen >= 512;
+  return pays ? (int)(seen < 65472 ? seen / KT + 1 : 1023) : 0;
 }
 
 template <int D, int GH, bool CAP, bool SIG, bool EXTRA>
 static void launch_heads(const Args& args, int ntiles, hipStream_t stream) {
   const dim3 grid(args.num_q_heads / GH, ntiles), block(256);
   Args a = args;
-  a.turns = turns(a, ntiles, (long)ntiles * (a.num_q_heads / GH));
+  a.turns = turns(a, ntiles);
   if (a.block_shift >= 2)
     hipLaunchKernelGGL((flash_prefill_kernel<D, GH, true, CAP, SIG, EXTRA>), grid, block, 0, stream, a);
   else
@@ -674,14 +722,7 @@ static void launch_heads(const Args& args, int ntiles, hipStream_t stream) {
 
 template <int D, bool CAP, bool SIG, bool EXTRA>
 static void launch_mode(const Args& a, int ntiles, hipStream_t stream) {
-  // Two heads per workgroup halve the reads of K and V; the line is where
-  // that leaves two workgroups for every CU (heads of 128, 32 over 8; two heads
-  // against one): 1280 workgroups 37.5 us against 44.0, 512 of 200 keys 17.0
-  // against 21.8, of 2048 71.4 against 72.6, 4096 rows on 4000 keys 498 against
-  // 683, but 256 workgroups of 4000 keys 126 us against 109, 96 of 1000 37.9
-  // against 28.3, 64 11.5 against 8.9
-  const int group = a.num_q_heads / a.num_kv_heads;
-  if (group % 2 == 0 && (long)ntiles * (a.num_q_heads / 2) >= 512)
+  if (heads_of_workgroup(a, ntiles) == 2)
     launch_heads<D, 2, CAP, SIG, EXTRA>(a, ntiles, stream);
   else
     launch_heads<D, 1, CAP, SIG, EXTRA>(a, ntiles, stream);

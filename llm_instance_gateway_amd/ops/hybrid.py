@@ -129,9 +129,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     pt = lib.lig_paged_attention_prefill_tiles
     pt.argtypes = [
         p, p, l, p, p, p, l, p, p, p, p, p, p, f, f, f, i, i, i, i, i, i, i, i, i, i,
-        i, p, i, i, f, p,
+        i, i, p, i, i, f, p,
     ]
     pt.restype = ctypes.c_int
+    tu = lib.lig_paged_attention_prefill_turns
+    tu.argtypes = [i, i, i, i, l, i, i]
+    tu.restype = ctypes.c_int
     hs = lib.lig_hyper_step
     hs.argtypes = [p, p, p, p, f, p, p, f, p, i, i, i, i, p]
     hs.restype = ctypes.c_int

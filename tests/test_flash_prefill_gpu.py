@@ -201,21 +201,59 @@ def test_keys_behind_the_last_row_of_the_tile(D, H, G, bs):
     assert torch.equal(got[:64], want[:64]) and got[70:].isnan().all()
 
 
-@pytest.mark.parametrize("window", [0, 1, 64, 130, 5000])
-@pytest.mark.parametrize("count", [2, 63, 64, 65, 128, 255, 256, 257])
-def test_tiles_take_their_turns(count, window):
+def _turns(b, H, G, bs, chunk=0, window=0, **_):
+    """Whether tiles are dealt by the lengths of their walks."""
+    keys = b["tab"].shape[1] * bs
+    return ops._hl().lig_paged_attention_prefill_turns(len(b["ts"]), len(b["ctx"]), H, G, keys, chunk, window) > 0
+
+
+def _in_any_order(b, H, D, seed, **kw):
+    """The list shuffled, two entries behind a portion's end, rows of no tile left as they were."""
+    ts, tq = torch.cat([b["ts"], b["ts"][:2]]), torch.cat([b["tq"], torch.full_like(b["tq"][:2], 6400)])
+    order = torch.randperm(len(ts), generator=torch.Generator().manual_seed(seed)).cuda()
+    b["ts"], b["tq"] = ts[order].contiguous(), tq[order].contiguous()
+    out = torch.full((b["q"].shape[0], H * D), float("nan"), device="cuda", dtype=BF)
+    return lambda: ops.paged_attention_prefill_tiles(
+        b["q"], b["k"], b["v"], b["tab"], b["starts"], b["ctx"], b["ts"], b["tq"], D ** -0.5, H, out=out, **kw)
+
+
+@pytest.mark.parametrize("window", [0, 448, 512, 5000])
+@pytest.mark.parametrize("count,H", [(18, 16), (63, 8), (64, 8), (65, 8), (128, 16), (255, 16), (256, 16), (257, 16)])
+def test_tiles_take_their_turns(count, H, window):
     """Every tile once, whatever the list's order; more than 256 run as listed."""
-    lens, left = [], count
+    lens, left = [], count - 2
     while left:
-        n = min((300, 20, 129, 64, 640)[len(lens) % 5], 64 * left)
+        n = min((576, 1100, 20, 960, 640, 1000)[len(lens) % 6], 64 * left)
         lens.append(n)
         left -= -(-n // 64)
-    b = _batch([(n + i % 3 * 50, n) for i, n in enumerate(lens)], 2, 128, 16, 4, 13)
-    assert len(b["ts"]) == count
-    order = torch.randperm(count, generator=torch.Generator().manual_seed(count)).cuda()
-    got = ops.paged_attention_prefill_tiles(b["q"], b["k"], b["v"], b["tab"], b["starts"], b["ctx"], b["ts"][order].contiguous(),
-                                            b["tq"][order].contiguous(), 128 ** -0.5, 4, window=window)
-    _check(got, b, 128, 128 ** -0.5, 4, **({"window": window} if window else {}))
+    b = _batch([(n + i % 3 * 450, n) for i, n in enumerate(lens)], 2, 128, 16, H, 13)
+    run = _in_any_order(b, H, 128, count, window=window)
+    assert len(b["ts"]) == count and _turns(b, H, 2, 16, window=window) == (count <= 256)
+    _check(run(), b, 128, 128 ** -0.5, H, **({"window": window} if window else {}))
+
+
+@pytest.mark.parametrize("D,H,G,bs", [(128, 16, 2, 16), (64, 16, 16, 32), (64, 24, 8, 2), (128, 16, 4, 6)])
+@pytest.mark.parametrize("kw", [{"softcap": 5.0, "window": 512}, {"weights": "sigmoid", "window": 448}, {"chunk": 512},
+                                {"chunk": 700, "window": 600, "softcap": 5.0, "weights": "sigmoid"}, {}], ids=range(5))
+def test_turns_with_options(D, H, G, bs, kw):
+    """Walks of many lengths, long ones of few rows among them, and a portion without rows."""
+    b = _batch([(4000, 70), (1200, 1200), (900, 900), (700, 0), (2500, 640), (1100, 500), (640, 640)], G, D, bs, H, 19)
+    run = _in_any_order(b, H, D, 3, **kw)
+    assert _turns(b, H, G, bs, **kw)
+    _check(run(), b, D, D ** -0.5, H, **kw)
+
+
+@pytest.mark.parametrize("segs,kw,dealt", [
+    ([(1000, 1000)] * 8, {}, True), ([(202, 202)] * 20, {}, False), ([(202, 202)] * 20 + [(600, 600)], {}, False),
+    ([(4000, 4000)], {}, False), ([(400, 400)] * 36, {}, False), ([(1000, 1000)] * 8, {"window": 512}, True),
+    ([(1000, 1000)] * 8, {"window": 128}, False), ([(1000, 1000)] * 8, {"chunk": 64}, False),
+    ([(2000, 2000)] * 2, {"window": 512}, True), ([(2000, 2000)] * 2, {"window": 2 ** 31 - 1}, True),
+])
+def test_which_launches_are_dealt(segs, kw, dealt):
+    """Not prompts of a few tiles, also beside a long one, nor one alone, nor walks that chunks or windows cut short."""
+    tiles, keys = sum(-(-n // 64) for _, n in segs), max(c for c, _ in segs)
+    args = kw.get("chunk", 0), kw.get("window", 0)
+    assert (ops._hl().lig_paged_attention_prefill_turns(tiles, len(segs), 32, 8, keys, *args) > 0) == dealt
 
 
 def _uneven_weight():
