@@ -109,10 +109,15 @@ extern "C" long lig_gated_delta_scratch(int R, int S, int H) {
 
 #define DI_THREADS 256
 #define DI_ROW 68  // padded fp32 LDS row
-#define DI_WAVES 5  // to a SIMD, at 96 registers; at 80, for six, it spills and gains nothing
+// Waves to a SIMD, of which a workgroup brings one to each.  For five the compiler keeps to 96
+// registers and does without copies in accumulation registers (heads of 192, 8 prompts of 1000, four waves and
+// five, both kernels 215 -> 209 us); at 80, for six, heads of 128 spill and gain nothing.  Heads of 256 take 116
+// for four; asked for five it gave them 130, for three (16 heads with values of 128 128.2 -> 125.4 us, 16 prompts of
+// 500 with values of 64 174 -> 170).
+#define DI_WAVES(DP) ((DP) <= 192 ? 5 : 4)
 
 template <int DP, typename Chunk>
-__global__ __launch_bounds__(DI_THREADS, DI_WAVES) void delta_chunk_prepare_kernel(
+__global__ __launch_bounds__(DI_THREADS, DI_WAVES(DP)) void delta_chunk_prepare_kernel(
     const MsArgs A, Chunk* __restrict__ scratch) {
   constexpr bool WALK = __is_same(Chunk, DeltaWalkChunk);
   constexpr int KB = DP / 32;
@@ -914,6 +919,18 @@ __global__ __launch_bounds__(NW * WAVE_SIZE, 1) void delta_chunk_walk_kernel(con
       }
     }
   }
+}
+
+// Workgroups of the first kernel that a CU holds, of heads of that many key entries; 0: unknown.
+extern "C" int lig_gated_delta_prepare_workgroups(int D) {
+  int n = 0;
+  const void* f = D <= 32    ? (const void*)delta_chunk_prepare_kernel<32, DeltaChunk>
+                  : D <= 64  ? (const void*)delta_chunk_prepare_kernel<64, DeltaChunk>
+                  : D == 128 ? (const void*)delta_chunk_prepare_kernel<128, DeltaWalkChunk>
+                  : D < 128  ? (const void*)delta_chunk_prepare_kernel<128, DeltaChunk>
+                  : D <= 192 ? (const void*)delta_chunk_prepare_kernel<192, DeltaChunk>
+                             : (const void*)delta_chunk_prepare_kernel<256, DeltaChunk>;
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, DI_THREADS, 0) == hipSuccess ? n : 0;
 }
 
 bool ms_delta_chunks_served(const MsArgs& a) {

@@ -173,6 +173,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     gs = lib.lig_gated_delta_scratch
     gs.argtypes = [i, i, i]
     gs.restype = l
+    gp = lib.lig_gated_delta_prepare_workgroups
+    gp.argtypes = [i]
+    gp.restype = ctypes.c_int
 
 
 def lib() -> ctypes.CDLL:

@@ -93,3 +93,9 @@ def test_value_blocks_in_pairs(dim, vdim):
 @pytest.mark.parametrize("heads,kv,dim", [(8, 4, 128), (16, 16, 64), (24, 12, 128), (9, 3, 128)])
 def test_heads_dealt_to_the_xcds(heads, kv, dim):
     test_delta_chunks([17, 200, 64], heads, kv, dim, 64)
+
+
+@pytest.mark.parametrize("dim,least", [(32, 6), (64, 5), (96, 5), (128, 5), (192, 5), (256, 4)])
+def test_workgroups_to_a_cu(dim, least):
+    """The first kernel is a chain of short steps, which need each other's waves to hide."""
+    assert ops._hl().lig_gated_delta_prepare_workgroups(dim) >= least
