@@ -133,6 +133,7 @@ def test_parts_of_a_walk(D, ctx, nsplits):
     args = (q, k, v, table, torch.tensor([ctx], dtype=torch.int32, device="cuda"), D ** -0.5)
     want = ops.row_product(ops.paged_attention_decode(*args, nsplits=nsplits).view(1, -1), w)
     x, parts = ops.paged_attention_decode_open(*args, nsplits=nsplits)
+    assert (parts is not None) == (nsplits in (2, 4))  # above, a launch merges them
     assert torch.equal(ops.row_product(x, w, parts=parts), want)
 
 
@@ -160,3 +161,45 @@ def test_an_attend_of_its_own_is_called():
     for _ in range(3):
         eng.step()
     assert rows == [33, 1, 1]
+
+
+def test_a_walk_that_grows_into_parts(monkeypatch):
+    """A lone request's steps, replayed from the graph, over the contexts at which its walk is cut in
+    two for the first time, against the same engine with projections of their own."""
+    from dataclasses import replace
+
+    from llm_instance_gateway_amd.engine import EngineConfig, LLMEngine, SamplingParams
+    from llm_instance_gateway_amd.models.config import get_model_config
+    from llm_instance_gateway_amd.models.llama import LlamaForCausalLM
+
+    mc = replace(get_model_config("llama3-8b"), num_layers=3, vocab_size=1024)
+    prompt = torch.randint(1, 1000, (985,), generator=torch.Generator().manual_seed(4)).tolist()
+    outs, opened = [], []
+    walk = ops.paged_attention_decode_open
+
+    def watched(*args):
+        out = walk(*args)
+        opened.append(out[1])
+        return out
+
+    monkeypatch.setattr(ops, "paged_attention_decode_open", watched)
+    for row in (True, False):
+        if not row:
+            monkeypatch.setattr(LlamaForCausalLM, "_row_products", lambda self: False)
+            monkeypatch.setattr(LlamaForCausalLM, "_open_norms", lambda self, rows: False)
+        torch.manual_seed(3)
+        eng = LLMEngine(EngineConfig(model=mc, num_kv_blocks=160, max_num_seqs=2, max_num_batched_tokens=1024,
+                                     max_model_len=2048), device="cuda")
+        s = eng.add_request(prompt, SamplingParams(max_new_tokens=32))
+        logits = []
+        for i in range(16):  # contexts of 986 to 1000 behind the prompt: 32 steps of 32 keys from 993 on
+            eng.step()
+            s.output_token_ids[-1] = 11 + i
+            if i:
+                logits.append(eng.runner.graph_runner.logits[1][:1].float().clone())
+        assert eng.runner.graph_runner._graph_nsplits(1) == 4
+        outs.append(torch.cat(logits))
+        # captured once, with room for parts
+        assert not row or (opened and all(p is not None and p[2] == 4 for p in opened))
+    # two correct orders of bf16 rounding, 3 layers deep
+    assert ((outs[0] - outs[1]).norm(dim=1) <= 0.03 * outs[1].norm(dim=1)).all()
