@@ -292,6 +292,18 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
   // ---- walk ------------------------------------------------------------------
   const int qpos0 = ctx - n + qt;
   const int kv_end = min(ctx, qpos0 + TQ);
+  if (kv_end <= 0) {
+    // a context shorter than its own rows, of which this tile's see no key: nothing to fetch ahead
+    if constexpr (!SPLIT) {
+      const int h0 = kvh * group + (blockIdx.x % per_kv) * GH;
+      for (int i = tid; i < TQ * GH * (D / 4); i += 256) {
+        const int r = qt + i / (GH * (D / 4));
+        uint16_t* op = a.out + ((size_t)(lo + r) * a.num_q_heads + h0) * D + i % (GH * (D / 4)) * 4;
+        if (r < n) *reinterpret_cast<u32x2*>(op) = u32x2{0, 0};
+      }
+    }
+    return;
+  }
   const int first_key = oldest_key<EXTRA>(a, qpos0);
   int kv_begin = first_key & ~(KT - 1), kv_stop = kv_end;
   if constexpr (SPLIT) {

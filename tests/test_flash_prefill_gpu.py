@@ -103,6 +103,24 @@ def test_tiles_without_keys_in_parts(D, H, G, bs):
     _check(got[sees], b, D, D ** -0.5, H)
 
 
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 6, 1, 2), (128, 32, 8, 16), (64, 32, 8, 6)])
+@pytest.mark.parametrize("kw", [{}, {"window": 70}, {"chunk": 96, "softcap": 5.0}, {"weights": "sigmoid"}], ids=range(4))
+def test_tiles_without_keys(D, H, G, bs, kw):
+    """The same of launches in one part, dealt by the lengths of their walks (32 heads) and as listed."""
+    b = _batch([(700, 700), (930, 930), (64, 5), (300, 300), (500, 500)], G, D, bs, H, 11)
+    for i, c in {1: 300, 2: 0, 3: 50}.items():
+        b["ctx"][i] = c
+    run = _in_any_order(b, H, D, 4, **kw)
+    got = run()
+    lens = (b["starts"][1:] - b["starts"][:-1]).long()
+    b["pos"] = torch.cat([torch.arange(int(n), device="cuda") + int(c) - int(n) for c, n in zip(b["ctx"], lens)])
+    sees = b["pos"] >= 0
+    assert (got[~sees] == 0).all() and int((~sees).sum()) == 630 + 5 + 250
+    for k in ("q", "tok_seq", "pos"):
+        b[k] = b[k][sees]
+    _check(got[sees], b, D, D ** -0.5, H, **kw)
+
+
 @pytest.mark.parametrize("D,H,G", [(128, 32, 8), (64, 32, 16)])
 def test_two_heads_per_workgroup(D, H, G):
     # enough tiles for the two-head workgroups, the last portions ragged
