@@ -124,9 +124,10 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_tiles_kernel(
   const int kv_end_tile = min(ctx, ctx - n + qt + PT_TQ);
 
   // chunked visibility: a row at position p sees keys from floor(p / chunk)
-  // * chunk on; the tile's walk starts at its first row's chunk
+  // * chunk on; the tile's walk starts at its first row's chunk (the first key's, where a
+  // context is shorter than its own rows)
   const int qpos0 = ctx - n + qt;
-  int kv_begin = chunk > 0 ? (qpos0 / chunk) * chunk : 0;
+  int kv_begin = chunk > 0 ? max(0, (qpos0 / chunk) * chunk) : 0;
   int key_lo = (chunk > 0 && row_valid) ? (qpos / chunk) * chunk : 0;
   if (window > 0) {
     kv_begin = max(kv_begin, qpos0 - window + 1);

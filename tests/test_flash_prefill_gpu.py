@@ -103,10 +103,12 @@ def test_tiles_without_keys_in_parts(D, H, G, bs):
     _check(got[sees], b, D, D ** -0.5, H)
 
 
-@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 6, 1, 2), (128, 32, 8, 16), (64, 32, 8, 6)])
-@pytest.mark.parametrize("kw", [{}, {"window": 70}, {"chunk": 96, "softcap": 5.0}, {"weights": "sigmoid"}], ids=range(4))
+@pytest.mark.parametrize("D,H,G,bs", [(128, 8, 2, 16), (64, 6, 1, 2), (128, 32, 8, 16), (64, 32, 8, 6), (96, 4, 2, 16)])
+@pytest.mark.parametrize("kw", [{}, {"window": 70}, {"chunk": 96, "softcap": 5.0}, {"weights": "sigmoid"}, {"chunk": 16}],
+                         ids=range(5))
 def test_tiles_without_keys(D, H, G, bs, kw):
-    """The same of launches in one part, dealt by the lengths of their walks (32 heads) and as listed."""
+    """The same of launches in one part, dealt by the lengths of their walks (32 heads) and as listed,
+    and of the kernel for other heads."""
     b = _batch([(700, 700), (930, 930), (64, 5), (300, 300), (500, 500)], G, D, bs, H, 11)
     for i, c in {1: 300, 2: 0, 3: 50}.items():
         b["ctx"][i] = c
