@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_tiles_kernel(
 // Of a launch of heads of 64 or 128 (and of the Llama path's in one part): whether its tiles take
 // their turns by length, then above 0.  keys: what a row of the block table has room for.
 extern "C" int lig_paged_attention_prefill_turns(int ntiles, int num_seqs, int num_q_heads, int num_kv_heads, long keys,
-                                                 int chunk, int window) {
+                                                 int chunk, int window, float softcap) {
   flash_prefill::Args a{};
   a.num_q_heads = num_q_heads;
   a.num_kv_heads = num_kv_heads;
@@ -305,6 +305,7 @@ extern "C" int lig_paged_attention_prefill_turns(int ntiles, int num_seqs, int n
   a.num_seqs = num_seqs;
   a.chunk = chunk;
   a.window = window;
+  a.softcap = softcap;
   return flash_prefill::turns(a, ntiles);
 }
 

@@ -10,7 +10,7 @@
 //   * a workgroup serves a tile of 64 query rows of GH heads of one key/value
 //     head, a wave RB = GH blocks of 16 rows of one of them, so an operand
 //     read from LDS feeds RB matrix instructions.  Two heads where that still
-//     gives every CU two workgroups, else one (see launch());
+//     gives every CU two workgroups, else one (heads_of_workgroup);
 //   * keys are dealt to the rows of the S^T = K Q^T tiles in the order in
 //     which a lane's scores ARE the operand of O^T += V^T P^T (rows g*4+i of
 //     two tiles hold keys g*8+i and g*8+4+i), so the weights never leave the
@@ -32,10 +32,11 @@
 // rows by DMA and their block's row number worked out once per group of keys: 4000
 // rows on 4000 keys 560 -> 441 us (between products), 20 prompts of 200 37 -> 33, one
 // of 202 8.9 -> 7.9, 8 of 1000 with the window and a cap 120 -> 96.
-// A cap's tanh goes into the weight's exponent as it comes.  Weights are summed in fp32, ahead of
-// their rounding; summed as the matrix cores see them, two to an instruction, they took as long
-// (8 of 1000 with the window and a cap 93.3 us, unrounded 92.5; 4000 rows of one prompt 150.7, 152.4; 24
-// of 640 107.5, 107.4; steps level).
+// A cap's tanh goes into the weight's exponent as it comes: 8 of 1000 with the window and a cap,
+// replayed without pauses, 95.8 -> 93.3 us, 3 of 1500 59.3 -> 58.0; results are rounded unlike, 1e-4
+// apart.  Weights are summed in fp32, ahead of their rounding; summed as the matrix cores see them,
+// two to an instruction, they took as long (8 of 1000 with the window and a cap 93.3 us, unrounded 92.5; 4000
+// rows of one prompt 150.7, 152.4; 24 of 640 107.5, 107.4; steps level).
 // Results in 16-byte pieces, a lane's four entries of a block swapped with its neighbour's for
 // eight, instead of 8-byte ones: 20 prompts of 200 28.3 -> 24.4, 24 of 640 118 -> 107, 40 of 400 99.8 ->
 // 87.5; 8 of 1000 with the window and a cap, their tiles in turn by length as well, 94 -> 85.
@@ -123,40 +124,31 @@ LIG_DEVICE int oldest_key(const Args& a, int qpos0) {
   return first;
 }
 
-// A tile of the caller's list and its portion.
-struct Place {
-  int s, qt, lo, n, ctx;
-};
-
 // Which tile of the list is this workgroup's: the longest walks first, so that the last
 // workgroups to begin are the shortest; of equal ones the last in the list first.  Lane i
 // brings portion i's numbers in the round of loads that brings the list.
-constexpr int TURN_TILES = 256, TURN_PORTION = 8;  // at most, and at least for each portion
+constexpr int TURN_TILES = 256, TURN_SEQS = 63;  // at most: a lane for each portion and the end of the last
 template <bool EXTRA>
-LIG_DEVICE Place tile_in_turn(const Args& a) {
+LIG_DEVICE void tile_in_turn(const Args& a, int& seq, int& qt) {
   constexpr int MOST = TURN_TILES / 64;
-  static_assert(TURN_TILES / TURN_PORTION < 64, "a lane for each portion and the end of the last");
   const int lane = threadIdx.x & 63, nt = gridDim.y, longest = a.turns;
   const int first = a.query_start_locs[min(lane, a.num_seqs)], held = a.context_lens[min(lane, a.num_seqs - 1)];
-  Place p[MOST];
-  int key[MOST];
+  int s[MOST], q[MOST], key[MOST];
 #pragma unroll
   for (int j = 0; j < MOST; ++j) {
     if (j * 64 >= nt) continue;
     const int at = max(nt - 1 - (j * 64 + lane), 0);
-    p[j].s = a.tile_seq[at];
-    p[j].qt = a.tile_qstart[at];
+    s[j] = a.tile_seq[at];
+    q[j] = a.tile_qstart[at];
   }
 #pragma unroll
   for (int j = 0; j < MOST; ++j) {
     key[j] = -1;
     if (j * 64 >= nt) continue;
-    p[j].lo = __shfl(first, p[j].s, 64);
-    p[j].n = __shfl(first, p[j].s + 1, 64) - p[j].lo;
-    p[j].ctx = __shfl(held, p[j].s, 64);
-    const int qpos0 = p[j].ctx - p[j].n + p[j].qt;
-    const int steps = (min(p[j].ctx, qpos0 + TQ) + KT - 1) / KT - oldest_key<EXTRA>(a, qpos0) / KT;
-    if (j * 64 + lane < nt) key[j] = p[j].qt < p[j].n ? min(max(steps, 0), longest) : 0;
+    const int n = __shfl(first, s[j] + 1, 64) - __shfl(first, s[j], 64), ctx = __shfl(held, s[j], 64);
+    const int qpos0 = ctx - n + q[j];
+    const int steps = (min(ctx, qpos0 + TQ) + KT - 1) / KT - oldest_key<EXTRA>(a, qpos0) / KT;
+    if (j * 64 + lane < nt) key[j] = q[j] < n ? min(max(steps, 0), longest) : 0;
   }
   auto from = [&](int k) {  // tiles with that key or a higher one
     int c = 0;
@@ -178,12 +170,12 @@ LIG_DEVICE Place tile_in_turn(const Args& a) {
     const uint64_t mine = __ballot(key[j] == k && at == before);
     if (mine) {
       const int l = __builtin_ctzll(mine);
-      return {__builtin_amdgcn_readlane(p[j].s, l), __builtin_amdgcn_readlane(p[j].qt, l), __builtin_amdgcn_readlane(p[j].lo, l),
-              __builtin_amdgcn_readlane(p[j].n, l), __builtin_amdgcn_readlane(p[j].ctx, l)};
+      seq = __builtin_amdgcn_readlane(s[j], l);
+      qt = __builtin_amdgcn_readlane(q[j], l);
+      return;
     }
     before -= __popcll(have);
   }
-  return {0, 0, 0, 0, 0};  // not reached: there are as many turns as tiles
 }
 
 // PB: block size a power of two, at least 4.  CAP: scores bent by softcap * tanh(score / softcap).  SIG: unnormalised
@@ -216,18 +208,17 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const Args a) {
 
   // grid.x runs over the head groups, so that with a multiple of 8 of them
   // every XCD keeps to some heads' keys in its own L2
-  Place own;
+  int s, qt;
   if (!SPLIT && a.turns > 0) {
-    own = tile_in_turn<EXTRA>(a);
+    tile_in_turn<EXTRA>(a, s, qt);
   } else {  // backwards, so that of one prompt the rows with the most keys start first
-    own.s = a.tile_seq[gridDim.y - 1 - blockIdx.y];
-    own.qt = a.tile_qstart[gridDim.y - 1 - blockIdx.y];
-    own.lo = a.query_start_locs[own.s];
-    own.n = a.query_start_locs[own.s + 1] - own.lo;
-    own.ctx = a.context_lens[own.s];
+    s = a.tile_seq[gridDim.y - 1 - blockIdx.y];
+    qt = a.tile_qstart[gridDim.y - 1 - blockIdx.y];
   }
-  const int s = own.s, qt = own.qt, lo = own.lo, n = own.n, ctx = own.ctx;
+  const int lo = a.query_start_locs[s];
+  const int n = a.query_start_locs[s + 1] - lo;
   if (qt >= n || n <= 0) return;
+  const int ctx = a.context_lens[s];
   const int* bt = a.block_tables + (size_t)s * a.max_blocks;
   const int group = a.num_q_heads / a.num_kv_heads;
   const int per_kv = group / GH;
@@ -710,14 +701,14 @@ static inline int heads_of_workgroup(const Args& a, long ntiles) {
 // 500 24.6, 21.6; 6 of 512 to 1000 rows on contexts of 600 to 4000 132.9, 109.1; 2 of 128 on 4000
 // listed ahead of 2 of 1500 130.8, 99.0.  As listed stay 20 of 202 (29.4, 30.7; with one of 600 33.4, 34.1),
 // 16 of 448 (54.4, 57.5), 24 of 640 (134.0, 141.7: 3840 workgroups) and one alone, which is in order (4000 rows
-// 145.5, 146.6).
+// 145.5, 146.6).  With a cap, whose scores take longer, 20 of 202 beside one of 600 gain: 42.1, 40.5.
 static inline int turns(const Args& a, long ntiles) {
   const long wgs = ntiles * (a.num_q_heads / heads_of_workgroup(a, ntiles));
   long seen = (long)a.max_blocks * a.block_size;  // by a tile
   if (a.window > 0) seen = std::min(seen, (long)a.window + TQ);
   if (a.chunk > 0) seen = std::min(seen, (long)a.chunk + TQ);
-  const bool pays = a.num_seqs > 1 && ntiles >= (long)TURN_PORTION * a.num_seqs && ntiles <= TURN_TILES && wgs > 256 &&
-                    wgs <= 2048 && seen >= 512;
+  const bool pays = a.num_seqs > 1 && a.num_seqs <= TURN_SEQS && ntiles >= (a.softcap > 0.f ? 4L : 8L) * a.num_seqs &&
+                    ntiles <= TURN_TILES && wgs > 256 && wgs <= 2048 && seen >= 512;
   return pays ? (int)(seen < 65472 ? seen / KT + 1 : 1023) : 0;
 }
 

@@ -133,7 +133,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     ]
     pt.restype = ctypes.c_int
     tu = lib.lig_paged_attention_prefill_turns
-    tu.argtypes = [i, i, i, i, l, i, i]
+    tu.argtypes = [i, i, i, i, l, i, i, f]
     tu.restype = ctypes.c_int
     hs = lib.lig_hyper_step
     hs.argtypes = [p, p, p, p, f, p, p, f, p, i, i, i, i, p]

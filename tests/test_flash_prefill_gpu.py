@@ -221,10 +221,10 @@ def test_keys_behind_the_last_row_of_the_tile(D, H, G, bs):
     assert torch.equal(got[:64], want[:64]) and got[70:].isnan().all()
 
 
-def _turns(b, H, G, bs, chunk=0, window=0, **_):
+def _turns(b, H, G, bs, chunk=0, window=0, softcap=0.0, **_):
     """Whether tiles are dealt by the lengths of their walks."""
     keys = b["tab"].shape[1] * bs
-    return ops._hl().lig_paged_attention_prefill_turns(len(b["ts"]), len(b["ctx"]), H, G, keys, chunk, window) > 0
+    return ops._hl().lig_paged_attention_prefill_turns(len(b["ts"]), len(b["ctx"]), H, G, keys, chunk, window, softcap) > 0
 
 
 def _in_any_order(b, H, D, seed, **kw):
@@ -263,16 +263,28 @@ def test_turns_with_options(D, H, G, bs, kw):
     _check(run(), b, D, D ** -0.5, H, **kw)
 
 
+def test_turns_of_many_portions():
+    """As many portions as there may be, the last lane's the end of the last."""
+    segs = [(900, 900), *[(n, n) for n in range(129, 191)]]
+    b = _batch(segs, 2, 64, 16, 8, 23)
+    b["ts"], b["tq"] = (torch.cat([b[t], torch.full_like(b[t][:51], x)]) for t, x in (("ts", 5), ("tq", 9000)))
+    run = _in_any_order(b, 8, 64, 6, softcap=5.0)
+    assert len(segs) == 63 and len(b["ts"]) <= 256 and _turns(b, 8, 2, 16, softcap=5.0)
+    _check(run(), b, 64, 64 ** -0.5, 8, softcap=5.0)
+
+
 @pytest.mark.parametrize("segs,kw,dealt", [
     ([(1000, 1000)] * 8, {}, True), ([(202, 202)] * 20, {}, False), ([(202, 202)] * 20 + [(600, 600)], {}, False),
+    ([(202, 202)] * 20 + [(600, 600)], {"softcap": 30.0}, True), ([(200, 200)] * 64, {"softcap": 30.0}, False),
     ([(4000, 4000)], {}, False), ([(400, 400)] * 36, {}, False), ([(1000, 1000)] * 8, {"window": 512}, True),
     ([(1000, 1000)] * 8, {"window": 128}, False), ([(1000, 1000)] * 8, {"chunk": 64}, False),
     ([(2000, 2000)] * 2, {"window": 512}, True), ([(2000, 2000)] * 2, {"window": 2 ** 31 - 1}, True),
 ])
 def test_which_launches_are_dealt(segs, kw, dealt):
-    """Not prompts of a few tiles, also beside a long one, nor one alone, nor walks that chunks or windows cut short."""
+    """Not prompts of a few tiles, also beside a long one (but with a cap), nor one alone, nor walks that
+    chunks or windows cut short."""
     tiles, keys = sum(-(-n // 64) for _, n in segs), max(c for c, _ in segs)
-    args = kw.get("chunk", 0), kw.get("window", 0)
+    args = kw.get("chunk", 0), kw.get("window", 0), kw.get("softcap", 0.0)
     assert (ops._hl().lig_paged_attention_prefill_turns(tiles, len(segs), 32, 8, keys, *args) > 0) == dealt
 
 
