@@ -72,16 +72,26 @@ constexpr int LR_PART_PAD = 4;  // a slice row is Dv values, running max (log2 u
 // Workgroups begin in the order of x, then y, one to each XCD in turn, and one whose
 // XCD is full holds up the others.  Segment for segment, a late one's longest walks
 // began when the others were at their last, and empty workgroups between left XCDs
-// unevenly full.  So the tiles that have rows are dealt by their number in the segment, the
-// highest of all segments first.  Of 4 prompts of 700-1000 with 16 heads 512 workgroups ran for
+// unevenly full.  So the tiles that have rows are dealt by the lengths of their walks, the longest
+// of all segments first: by their number in the segment, counted from the first token of the sequence,
+// of which a window sees so many.  Of 4 prompts of 700-1000 with 16 heads 512 workgroups ran for
 // 60 us and less and less of them for 38 more: 94 -> 83 us, with results in 16-byte pieces and
 // one round of loads ahead of the block table less; 8 of them 197 -> 174, 16 of 70-100 23.1 -> 19.9.
+// By the number in the segment alone the longest walks came last where tokens are cached: 6 of 512-1000 on
+// 600-4000 keys 249 us in their order, 395 so, 232 now; 32 heads, 100 on 4000 keys beside 15 of 200 192, 490, 197.
 // More than 16 segments, whose keys would no longer stay in the L2 (64 prompts of 210-300: 190 us
 // in their order, 249 dealt), and single tiles stay as they are.  False: no tile is left.
 struct Walk {
   int seg, tile, n, start, ctx;
 };
-LIG_DEVICE bool deal(const int* seg_start, const int* seg_len, const int* seg_ctx, int H, int rows, Walk& w) {
+template <typename F>
+LIG_DEVICE int over_row(int v, const F& f) {  // of 16 lanes side by side, in each of them
+  v = f(v, __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true));  // rotated by 8
+  v = f(v, __builtin_amdgcn_mov_dpp(v, 0x124, 0xF, 0xF, true));
+  v = f(v, __builtin_amdgcn_mov_dpp(v, 0x122, 0xF, 0xF, true));
+  return f(v, __builtin_amdgcn_mov_dpp(v, 0x121, 0xF, 0xF, true));
+}
+LIG_DEVICE bool deal(const int* seg_start, const int* seg_len, const int* seg_ctx, int H, int rows, int window, Walk& w) {
   const unsigned segs = gridDim.y, most = gridDim.x;
   if (most == 1 || segs == 1 || segs > 16 || most > 65535) {
     w.seg = blockIdx.y;
@@ -91,31 +101,32 @@ LIG_DEVICE bool deal(const int* seg_start, const int* seg_len, const int* seg_ct
     w.ctx = seg_ctx[w.seg];
     return (long)w.tile * rows < (long)w.n * H;
   }
-  const int lane = threadIdx.x & 63, at = min(lane, (int)segs - 1);
+  // every 16 lanes hold all segments
+  const int lane = threadIdx.x & 63, seg = lane & 15, at = min(seg, (int)segs - 1);
   const int n = seg_len[at], start = seg_start[at], ctx = seg_ctx[at];
-  // of this lane's segment
-  const int tiles = lane < (int)segs && n > 0 ? (int)min((long)most, ((long)n * H + rows - 1) / rows) : 0;
-  auto from = [&](int t) {  // tiles numbered t and higher: under 2^21
-    int c = 0;
-    for (unsigned g = 0; g < segs; ++g) c += max(__builtin_amdgcn_readlane(tiles, g) - t, 0);
-    return c;
-  };
+  const int tiles = seg < (int)segs && n > 0 ? (int)min((long)most, ((long)n * H + rows - 1) / rows) : 0;
+  auto sum = [](int v) { return over_row(v, [](int a, int b) { return a + b; }); };  // under 2^21
   const int i = blockIdx.y * most + blockIdx.x;
-  if (i >= __builtin_amdgcn_readfirstlane(from(0))) return false;
-  // the last number from which on there are more than i tiles: of 64 at a time
+  if (i >= __builtin_amdgcn_readfirstlane(sum(tiles))) return false;
+  // tiles of its tokens before these, or of those that the window's first row sees
+  constexpr long MOST = 1 << 24;
+  long before = min(MOST, (long)max(ctx - n, 0) * H / rows);
+  if (window > 0) before = min(before, ((long)window * H + rows - 1) / rows);
+  const int ahead = tiles > 0 ? (int)before : 0, end = ahead + tiles;
+  auto from = [&](int t) { return sum(min(max(end - t, 0), tiles)); };  // tiles that end at t + 1 and behind
+  // the last number from which on there are more than i tiles: four at a time, one for each 16 lanes
   int lo = 0;
-  for (int width = most; width > 1;) {
-    const int step = (width + 63) / 64, t = lo + lane * step;
-    lo += (__popcll(__ballot(lane * step < width && from(t) > i)) - 1) * step;
+  for (int width = __builtin_amdgcn_readfirstlane(over_row(end, [](int a, int b) { return max(a, b); })); width > 1;) {
+    const int step = (width + 4) / 5;
+    lo += __popcll(__ballot(from(lo + ((lane >> 4) + 1) * step) > i) & 0x0001000100010001) * step;
     width = step;
   }
-  // the segments that have tile lo, in their order
-  const int k = i - __builtin_amdgcn_readfirstlane(from(lo + 1));
-  const uint64_t have = __ballot(tiles > lo);
-  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0));
-  const uint64_t mine = __ballot(tiles > lo && before == k);
-  w.seg = __builtin_ctzll(mine);
-  w.tile = lo;
+  // the segments that have such a tile, in their order
+  const int k = i - __builtin_amdgcn_readfirstlane(from(lo + 1)), tile = lo - ahead;
+  const bool has = lane < 16 && tile >= 0 && tile < tiles;
+  const uint32_t have = (uint32_t)__ballot(has);
+  w.seg = __builtin_ctzll(__ballot(has && (int)__builtin_amdgcn_mbcnt_lo(have, 0) == k));
+  w.tile = __builtin_amdgcn_readlane(tile, w.seg);
   w.n = __builtin_amdgcn_readlane(n, w.seg);
   w.start = __builtin_amdgcn_readlane(start, w.seg);
   w.ctx = __builtin_amdgcn_readlane(ctx, w.seg);
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
   __shared__ __align__(16) uint16_t sm[LDS];
 
   Walk walk;  // the longest first
-  if (!deal(seg_start, seg_len, seg_ctx, H, ROWS, walk)) return;
+  if (!deal(seg_start, seg_len, seg_ctx, H, ROWS, window, walk)) return;
   const int s = walk.seg, n = walk.n, ctx = walk.ctx;
   const long lo = walk.start;
   const long nrows = (long)n * H;

@@ -114,6 +114,13 @@ def test_tiles_are_dealt_over_the_segments(D, Dv, H, count):
     _run([(n + 1 + 37 * i % 200, n) for i, n in enumerate(new)], H, D, Dv, 16, 0, 1 + count % 2, gate=count == 3)
 
 
+@pytest.mark.parametrize("window", [0, 1, 300, 100000])
+@pytest.mark.parametrize("D,Dv,H", [(576, 512, 16), (72, 56, 3), (192, 128, 80)])
+def test_tiles_are_dealt_by_their_walks(D, Dv, H, window):
+    """Few rows on long contexts among longer portions of short ones, and single tokens."""
+    _run([(3000, 33), (200, 200), (40, 0), (1500, 70), (900, 1), (64, 64), (2100, 120)], H, D, Dv, 16, window, 1, gate=False)
+
+
 def test_results_that_lie_8_bytes_off():
     q = torch.randn(100, 16 * 72, device="cuda").to(BF)
     cache = torch.randn(8, 1, 16, 72, device="cuda").to(BF)
