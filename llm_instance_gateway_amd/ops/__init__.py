@@ -213,12 +213,15 @@ def paged_attention_decode(
     return res if out is None else out.copy_(res)
 
 
-# Up to that many parts of a walk are merged by every workgroup of the product behind: attention
-# and a product of 4096 x 4096, 32 heads of 128, merged by a launch and by the product, 381
-# keys of at most 4 parts 17.8 us, 16.2 (in one part: the launch has nothing to do); 1100
-# 21.2, 20.1; 2000 22.9, 22.8; 4000 26.3, 27.2; but 4000 and 8000 of at most 16 24.6, 27.2
-# and 27.7, 37.4.
+# Up to that many parts of a walk are merged by every workgroup of the product behind, of rows up
+# to so wide: attention and a product of 4096 x 4096, 32 heads of 128, at most 4 parts, merged by a
+# launch and by the product, 381 keys (in one part: the launch has nothing to do) 17.2 us,
+# 15.9; 1100 20.4, 19.6; 1600 21.1, 20.7; 2047 20.4, 21.5; 2048 x 2048, 16 heads, 14.2, 12.5; 16.9,
+# 15.6; 17.0, 16.1; 16.5, 16.1.  But 4000 and 8000 keys of at most 16 24.6, 27.2 and 27.7, 37.4, and what
+# a workgroup merges grows with the row: 8192 x 8192, 64 heads, 381 keys 33.4, 32.0; 1100 37.0, 37.6; 2047
+# 36.6, 42.4; 5120 x 5120, 40 heads, 21.5, 20.1; 24.8, 24.8; 24.7, 28.3.
 _OPEN_PARTS = 4
+_OPEN_WIDTH = 4096
 
 
 def paged_attention_decode_open(
@@ -228,7 +231,7 @@ def paged_attention_decode_open(
     row [1, heads * D], whole or not, and what it takes to merge it.  GPU."""
     N, Hq, D = q.shape
     ns = nsplits if nsplits > 0 else decode_nsplits(N, k_cache.shape[1], max_ctx)
-    if ns <= 1 or ns > _OPEN_PARTS:
+    if ns <= 1 or ns > _OPEN_PARTS or Hq * D > _OPEN_WIDTH:
         return paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, nsplits=ns).view(1, -1), None
     out = torch.empty_like(q)
     scratch = split_scratch(q.device, N * Hq * ns * (D + 2))

@@ -137,6 +137,14 @@ def test_parts_of_a_walk(D, ctx, nsplits):
     assert torch.equal(ops.row_product(x, w, parts=parts), want)
 
 
+@pytest.mark.parametrize("heads,opens", [(32, True), (33, False), (64, False)])
+def test_wide_rows_come_merged(heads, opens):
+    q, kv = torch.zeros(1, heads, 128, dtype=BF, device="cuda"), torch.zeros(70, heads, 16, 128, dtype=BF, device="cuda")
+    table, ctx = torch.arange(70, dtype=torch.int32, device="cuda").view(1, -1), torch.tensor([1100], dtype=torch.int32, device="cuda")
+    row, parts = ops.paged_attention_decode_open(q, kv, kv, table, ctx, 1.0, nsplits=4)
+    assert (parts is not None) == opens and row.shape == (1, heads * 128)
+
+
 def test_an_attend_of_its_own_is_called():
     """An instance's own `attend`, which its layer calls at any number of rows, for a single token too."""
     from dataclasses import replace
