@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256, KG == 1 ? 2 : 1) void latent_attention_rows_ke
     load_v(0);
 
     // the other workgroup's products give way to these few instructions, behind which
-    // this wave's own wait: 4 prompts of 700-1000 78.9 -> 75.0 us, one of 4000 298 -> 292
+    // this wave's own wait: 4 prompts of 700-1000 83 -> 79 us, one of 4000 298 -> 292
     if constexpr (KG == 1) __builtin_amdgcn_s_setprio(1);
     // ---- weights of keys k0 + lg*8 + e -----------------------------------------
     const bool masked = k0 + 32 > min(all_end, kv_hi) || k0 < all_lo;

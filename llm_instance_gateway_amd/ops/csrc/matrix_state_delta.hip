@@ -947,9 +947,11 @@ void ms_delta_chunks_launch(const MsArgs& a, int S, int max_seg_len, void* scrat
   const dim3 gi((max_seg_len + MC_T - 1) / MC_T * a.H, S);
   // Two value blocks per workgroup share the staged operands where the
   // registers of eight waves hold the state, and a workgroup each would not
-  // find a CU each.  Both calls, 32 heads of 128 x 128, one block here and two:
-  // 1 prompt of 4000 tokens 244 us, 298; of 1000 78, 95; 2 of these 85, 100;
-  // 4 (256 workgroups) 100, 114; 5 153, 123; 8 183, 151.  That is prompts alone: S counts
+  // find a CU each.  One call, 32 heads of 128 x 128, one block here and two: 1 prompt
+  // of 4000 tokens 192 us, 243; of 1000 62, 77; 2 of these 68, 82; 4 (256 workgroups) 79, 92;
+  // 5 124, 97; 8 156, 131; 64 heads, 2 of 1000 79, 91, 3 134, 107; 16 of 500 354, 283.  The other
+  // walk: values of 96, 4 of 1000 88, 101, 5 145, 106; heads of 64 x 128 66, 80 and 89, 84, but 8
+  // 120, 123; past 128 entries it has no pairs.  That is prompts alone: S counts
   // every segment of a call, also those too short for these kernels, whose workgroups are
   // over at once, so that a prompt beside a few single tokens gets pairs.
   const bool pair = a.NB > 1 && (long)S * a.H * a.NB > 256;

@@ -45,7 +45,9 @@ constexpr int XCD_PHASES = 4;  // starting points in K
 // lanes are in 16 rows and every one of them is an access of its own, 64 to a kilobyte.  So
 // 16 rows at a time go through LDS (`room`, this wave's own) and leave in the order in which
 // they lie in memory: parts of 4096 x 14336 at 202 rows 35.0 -> 33.0 us, 384 46 -> 44.4; of 4096 x
-// 4096 at 786 32.8 -> 31.1; 28672 x 4096 rounded, 786 rows 151 -> 148; to 64 rows level.
+// 4096 at 786 32.8 -> 31.1; 28672 x 4096 rounded, 786 rows 151 -> 148; in the mean of 10 weights 202 rows
+// 2.5 % faster, 100 and 64 1 %, 48 level, 2 to 33 up to 1.7 % slower (a tenth of a us), which blocks of rows past
+// M left out do not mend (1 % at 2 rows, and a branch that costs 0.5 % at 64).
 template <int TN, bool PARTIAL>
 constexpr int ROOM_ROW = TN * 16 * (PARTIAL ? 4 : 2) + 16;  // bytes of a row, for rows to start 4 banks apart
 template <int TM, int TN, bool PARTIAL>
@@ -531,7 +533,9 @@ Plan plan(int M, int N, int K) {
   return best;
 }
 
-// The tile that runs a plan: its own, or TILE_COUNT and more for one of the others.
+// The tile that runs a plan: its own, or TILE_COUNT and more for one of the others.  Its tiles begin at
+// other places in K, so that sums are of the same terms in another order: of 786 x 28672 x 4096 one
+// rounded result in 80000 differs, and the fp32 error against 64 bits stays 3.95e-7.
 int tile_of(const Plan& p, int M, int N, int K) {
   if (p.tile < FEW || M > 1024) return p.tile;  // not measured
   int tile = p.tile;
@@ -588,14 +592,14 @@ extern "C" {
 
 // Sizes that these kernels are for where their reader adds up the parts of K.  Above 256
 // rows, from 3072 columns on, they take 0.6 to 1 of the library's time, of the largest
-// matrices 0.85 to 1.05 (384 rows: 6144 x 4096 29 us here, 35 there; 4096 x 14336 49, 75;
-// 28672 x 4096 77, 79; 960: 181, 175).  With many tiles of fewer columns neither is ahead
-// (16384 x 2048: 288 rows 24, 27; 384 29, 27).
+// matrices 0.9 to 1 (384 rows: 6144 x 4096 27 us here, 37 there; 4096 x 14336 45, 79;
+// 28672 x 4096 75, 82; 786: 150, 172; 960: 177, 183).  With many tiles of fewer columns neither
+// was ahead, on the planned tiles and with results as lanes hold them (16384 x 2048: 288 rows 24, 27; 384 29, 27).
 // Above 1024 rows it is large weights with long rows, to 1792, where all of K in one part
-// fills the chip (here, the library's; 8192 x 28672: 1152 rows 518, 548; 1408 518, 520; 1792
-// 589, 802; 8192 x 16384: 1280 258, 276; 12288 x 28672: 1536 869, 1423; 5120 x 13824: 1792 213,
-// 221).  From 1793 on they lose as often as they win (1920: 644, 647; 373, 363; 16384 x 53248
-// 2438, 2299).  In parts 4096 x 14336 would win too (1216 rows 115, 149), but where a step's
+// fills the chip (here, the library's; 8192 x 28672: 1152 rows 440, 440; 1408 500, 512; 1792
+// 572, 779; 8192 x 16384: 1280 250, 262; 12288 x 28672: 1536 842, 1422; 5120 x 13824: 1792 207,
+// 216).  From 1793 on, measured like 16384 x 2048, they lost as often as they won (1920: 644, 647; 373, 363;
+// 16384 x 53248 2438, 2299).  In parts 4096 x 14336 would win too (1216 rows 115, 149), but where a step's
 // other products are the library's nothing adds them up, and the sum takes what the cut gains.
 bool lig_projection_serves(long M, long N, long K) {
   if (M < 1 || M > 1792 || N < 1 || N > (1 << 24) || K < 64 || K > (1 << 20) || N % 8 || K % 64) return false;
@@ -605,14 +609,14 @@ bool lig_projection_serves(long M, long N, long K) {
 
 // Whether a served product that has to come rounded, its parts added up by a launch
 // of its own, runs here too (us here, the library's):
-//   * to 128 rows it does (100 x 28672 x 4096: 42, 52), not a vocabulary's worth of short
-//     rows of W, 24 x 57344 x 1024;
-//   * to 256 rows where K is cut (202 x 4096 x 14336: 41, 57; 202 x 4096 x 4096: 19, 21, but
-//     256 of these 20, 22 with a launch more) or the weight large (202 x 28672 x 4096: 55, 66;
-//     202 x 57344 x 8192: 179, 215);
-//   * above, large weights do at any row count (384 x 4096 x 14336: 54, 75; 384 x 28672 x
-//     4096: 77, 79) and others where K is cut into many parts.  What is left gains a few us
-//     at most (1000 x 4096 x 4096: 36, 39; 448 x 6144 x 4096: 31, 33).
+//   * to 128 rows it does (100 x 28672 x 4096: 43, 56), but for a vocabulary's worth of short
+//     rows of W, which gain little (24 x 57344 x 1024: 22, 24);
+//   * to 256 rows where K is cut (202 x 4096 x 14336: 41, 57; 202 x 4096 x 4096: 19, 22, but
+//     256 of these 20, 23 with a launch more) or the weight large (202 x 28672 x 4096: 56, 66;
+//     202 x 57344 x 8192: 189, 200);
+//   * above, large weights do at any row count (384 x 4096 x 14336: 53, 79; 384 x 28672 x
+//     4096: 75, 82) and others where K is cut into many parts.  What is left gains a few us
+//     at most (1000 x 4096 x 4096: 38, 42; 786 x 6144 x 4096: 43, 47; 448: 34, 33).
 // Of smaller weights the library's call takes longer on the host than is gained, which steps
 // of narrow models wait for: 300 rows, 16 layers of 2048 columns 2106 us, 2488 with its
 // products.
